@@ -30,7 +30,7 @@
 //   csrc/include/natten/cuda/reference/fna_reference_backward.hpp:60-150, :165-265, :282-380
 //     (P = exp(scale q.k - LSE), dS = P scale (dO.v - dO.o), dQ / dK / dV as sums over the mask)
 //   csrc/include/natten/cuda/fna_blackwell/collective/fna_fusion_bwd.hpp:256-318 (the Q tiles a KV tile meets;
-//     here the query interval is found by bisection on the forward window functions instead)
+//     here the query interval is inverted from the forward's own window functions)
 // Operands are token-permuted sequences whose tiles hold 128 tokens; such a tile splits, along
 // its slowest dimension, into two contiguous 64-token tiles, which is what the other role streams.
 #pragma once
@@ -88,7 +88,37 @@ struct FnaBwdParams {
   int kv_wg_run;
   // Host side only: which launches a call makes (bit 0: the dQ role, bit 1: the dK / dV role; 0 = both).
   int roles;
+  // Derived by set_bwd_divisions(): what the per-workgroup set-up would otherwise divide for (tile
+  // extents are powers of two, the other divisors get multiply-shift pairs).
+  // Dividing and bisecting for the query ranges in the kernel cost every workgroup several
+  // thousand instructions: a training step of 128 x 128 tokens, H 16, D 128 (2 048 key tiles, one
+  // workgroup per CU at a time) 1046 -> 956 us, 29 x 46 x 78 dilated H 24 50.3 -> 48.4 ms.
+  int q_tile_lg[3], kv_tile_lg[3];
+  int ext_base[3], ext_rem[3];  // qkv_shape / dil and qkv_shape % dil
+  NaDiv d_stride[3], d_dil[3], d_num_groups, d_rep, d_kv_wg_run;
+  NaDiv d_q_tiled[3], d_kv_tiled[3], d_num_q, d_num_kv, d_heads_q, d_heads_kv;
 };
+
+inline void set_bwd_divisions(FnaBwdParams& p) {
+  for (int a = 0; a < 3; ++a) {
+    p.q_tile_lg[a] = p.kv_tile_lg[a] = 0;
+    while ((1 << p.q_tile_lg[a]) < p.q_tile[a]) ++p.q_tile_lg[a];
+    while ((1 << p.kv_tile_lg[a]) < p.kv_tile[a]) ++p.kv_tile_lg[a];
+    p.ext_base[a] = p.qkv_shape[a] / p.dil[a];
+    p.ext_rem[a] = p.qkv_shape[a] % p.dil[a];
+    p.d_stride[a] = na_make_div(p.stride[a]);
+    p.d_dil[a] = na_make_div(p.dil[a]);
+    p.d_q_tiled[a] = na_make_div(p.q_tiled[a]);
+    p.d_kv_tiled[a] = na_make_div(p.kv_tiled[a]);
+  }
+  p.d_num_groups = na_make_div(p.num_groups);
+  p.d_rep = na_make_div(p.heads_q / p.heads_kv);
+  p.d_kv_wg_run = na_make_div(p.kv_wg_run > 0 ? p.kv_wg_run : 1);
+  p.d_num_q = na_make_div(p.q_tiled[0] * p.q_tiled[1] * p.q_tiled[2]);
+  p.d_num_kv = na_make_div(p.kv_tiled[0] * p.kv_tiled[1] * p.kv_tiled[2]);
+  p.d_heads_q = na_make_div(p.heads_q);
+  p.d_heads_kv = na_make_div(p.heads_kv);
+}
 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 
@@ -151,13 +181,15 @@ fna_bwd_kernel(const FnaBwdParams p) {
 
   const int* a_tile = KV_STATIONARY ? p.kv_tile : p.q_tile;
   const int* a_tiled = KV_STATIONARY ? p.kv_tiled : p.q_tiled;
+  const int* a_tile_lg = KV_STATIONARY ? p.kv_tile_lg : p.q_tile_lg;
   const int* b_tile = KV_STATIONARY ? p.q_tile : p.kv_tile;
+  const int* b_tile_lg = KV_STATIONARY ? p.q_tile_lg : p.kv_tile_lg;
   const int* b_tiled = KV_STATIONARY ? p.q_tiled : p.kv_tiled;
   const int heads_a = KV_STATIONARY ? p.heads_kv : p.heads_q;
   const int heads_b = KV_STATIONARY ? p.heads_q : p.heads_kv;
   const int seq_a = KV_STATIONARY ? p.seqlen_kv : p.seqlen_q;
   const int seq_b = KV_STATIONARY ? p.seqlen_q : p.seqlen_kv;
-  const int rep = p.heads_q / p.heads_kv;
+  const int rep = na_div(p.heads_q, p.d_heads_kv);
   const int split_dim = KV_STATIONARY ? p.q_split : p.kv_split;  // of the streamed side
 
   // ---- workgroup -> (batch * group, head, stationary tile) --------------------------------------
@@ -172,7 +204,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
   int lin;
   if (wg_run > 0) {
     const int local = int(blockIdx.x) / kNumXcd;
-    lin = ((local / wg_run) * kNumXcd + int(blockIdx.x) % kNumXcd) * wg_run + local % wg_run;
+    const int round = na_div(local, p.d_kv_wg_run);
+    lin = (round * kNumXcd + int(blockIdx.x) % kNumXcd) * wg_run + local - round * wg_run;
   } else {
     const int chunk = (total_wg + kNumXcd - 1) / kNumXcd;
     lin = (int(blockIdx.x) % kNumXcd) * chunk + int(blockIdx.x) / kNumXcd;
@@ -181,19 +214,22 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // Within a head the tiles are taken with dimension 0 slowest: the workgroups running side by
   // side are then neighbours in the faster dimensions at the same dimension-0 position and
   // walk the same streamed tiles at about the same time.
+  const int bh = na_div(lin, KV_STATIONARY ? p.d_num_kv : p.d_num_q);
   int tc[3];
   {
-    const int rm = lin % num_a;
-    tc[2] = rm % a_tiled[2];
-    tc[1] = (rm / a_tiled[2]) % a_tiled[1];
-    tc[0] = rm / (a_tiled[2] * a_tiled[1]);
+    const int rm = lin - bh * num_a;
+    const int t01 = na_div(rm, KV_STATIONARY ? p.d_kv_tiled[2] : p.d_q_tiled[2]);
+    tc[2] = rm - t01 * a_tiled[2];
+    tc[0] = na_div(t01, KV_STATIONARY ? p.d_kv_tiled[1] : p.d_q_tiled[1]);
+    tc[1] = t01 - tc[0] * a_tiled[1];
     // a causal dimension 0: the query tiles with the longest key ranges are the last ones;
     // they start first (key tiles are already in that order)
     if (!KV_STATIONARY && p.causal[0]) tc[0] = a_tiled[0] - 1 - tc[0];
   }
   const int at = tc[0] + a_tiled[0] * (tc[1] + a_tiled[1] * tc[2]);  // position in the permuted sequence
-  const int head_a = (lin / num_a) % heads_a;
-  const int bg = lin / (num_a * heads_a);
+  const int bg = na_div(bh, KV_STATIONARY ? p.d_heads_kv : p.d_heads_q);
+  const int head_a = bh - bg * heads_a;
+  const int b_orig = na_div(bg, p.d_num_groups);  // batch entry before the dilation groups were folded in
 
   // first rows of this batch entry's sequences, its lse / delta values of head 0, and the
   // parameters a packed sequence overrides
@@ -201,7 +237,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   int64_t stat_row_q = int64_t(bg) * p.heads_q * p.seqlen_q;
   int64_t stat_head_stride = p.seqlen_q;
   int ksz[3] = {p.ksize[0], p.ksize[1], p.ksize[2]};
-  int keys0 = p.qkv_shape[0], queries0 = p.q_extent0;
+  int keys0 = p.ext_base[0], queries0 = p.q_extent0;  // (extents of dimension 0 before the uneven dilation groups)
   bool empty = false;
   if constexpr (VARLEN) {
     const int q0 = p.cu_q[bg], kv0 = p.cu_kv[bg], pq0 = p.pcu_q[bg], pkv0 = p.pcu_kv[bg];
@@ -220,48 +256,51 @@ fna_bwd_kernel(const FnaBwdParams p) {
     empty = len_q == 0 || len_kv == 0;  // nothing attends, or attends to nothing: zero gradients
   }
 
-  int extent[3], q_extent[3], a_first[3], b_sub[3], box_tile0[3], box_n[3], full_t0[3], full_t1[3];
+  int extent[3], q_extent[3], a_first[3], b_sub[3], b_sub_lg[3], box_tile0[3], box_n[3], full_t0[3], full_t1[3];
   int tok_step[3];    // original layout: tokens per unit step of a coordinate inside a dilation group
   int group_tok = 0;  // original layout: token of the dilation group's first element
   {
-    int gl = bg % p.num_groups;
+    int gl = bg - b_orig * p.num_groups;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int gi = gl % p.dil[a];
-      gl /= p.dil[a];
+      const int rest = na_div(gl, p.d_dil[a]);
+      const int gi = gl - rest * p.dil[a];
+      gl = rest;
       tok_step[a] = p.dil[a] * p.tok_stride[a];
       group_tok += gi * p.tok_stride[a];
-      extent[a] = na_group_extent(a == 0 ? keys0 : p.qkv_shape[a], p.dil[a], gi);
+      // (as in the forward kernel: the first groups hold one token more when the dilation does not divide the extent)
+      extent[a] = (a == 0 ? keys0 : p.ext_base[a]) + (gi < p.ext_rem[a] ? 1 : 0);
       q_extent[a] = (a == 0 && queries0 > 0) ? queries0 : extent[a];
-      a_first[a] = tc[a] * a_tile[a];
-      b_sub[a] = (a == split_dim) ? b_tile[a] / 2 : b_tile[a];
+      a_first[a] = tc[a] << a_tile_lg[a];
+      b_sub_lg[a] = b_tile_lg[a] - (a == split_dim ? 1 : 0);
+      b_sub[a] = 1 << b_sub_lg[a];
       const bool c = p.causal[a] != 0;
       int lo, hi;  // first and last streamed coordinate this tile meets
       if constexpr (!KV_STATIONARY) {
         const int qf = a_first[a], ql = na_min(qf + a_tile[a], q_extent[a]) - 1;
         if (qf >= q_extent[a]) empty = true;
-        lo = na_window_start(qf, ksz[a], p.stride[a], extent[a], c);
-        const int st_l = na_window_start(na_max(ql, 0), ksz[a], p.stride[a], extent[a], c);
+        lo = na_window_start(qf, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
+        const int st_l = na_window_start(na_max(ql, 0), ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
         hi = na_window_end(na_max(ql, 0), st_l, ksz[a], extent[a], c) - 1;
       } else {
         const int j0 = a_first[a], j1 = na_min(j0 + a_tile[a], extent[a]) - 1;
         if (j0 >= extent[a]) empty = true;
-        lo = na_first_query_attending(j0, ksz[a], p.stride[a], extent[a], q_extent[a], c);
-        hi = na_last_query_attending(na_max(j1, 0), ksz[a], p.stride[a], extent[a], q_extent[a], c);
+        lo = na_first_query_attending(j0, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
+        hi = na_last_query_attending(na_max(j1, 0), ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
         if (lo > hi) empty = true;
       }
       lo = na_max(lo, 0);
       hi = na_max(hi, lo);
-      box_tile0[a] = lo / b_sub[a];
-      box_n[a] = hi / b_sub[a] + 1 - box_tile0[a];
+      box_tile0[a] = lo >> b_sub_lg[a];
+      box_n[a] = (hi >> b_sub_lg[a]) + 1 - box_tile0[a];
       // Streamed tiles every row of which pairs with every row of the stationary tile (no mask
       // needed) form an interval of tile coordinates per dimension, again by monotonicity:
       // streamed coordinates flo .. fhi pair with all stationary ones.
       int flo, fhi;
       if constexpr (!KV_STATIONARY) {
         const int qf = a_first[a], ql = qf + a_tile[a] - 1;  // rows past the extent use the last window
-        const int st_l = na_window_start(ql, ksz[a], p.stride[a], extent[a], c);
-        const int st_f = na_window_start(qf, ksz[a], p.stride[a], extent[a], c);
+        const int st_l = na_window_start(ql, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
+        const int st_f = na_window_start(qf, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
         flo = st_l;
         fhi = na_window_end(qf, st_f, ksz[a], extent[a], c) - 1;
       } else {
@@ -270,12 +309,12 @@ fna_bwd_kernel(const FnaBwdParams p) {
           flo = 1;  // the tile holds padding keys: never whole
           fhi = 0;
         } else {
-          flo = na_first_query_attending(j1, ksz[a], p.stride[a], extent[a], q_extent[a], c);
-          fhi = na_last_query_attending(j0, ksz[a], p.stride[a], extent[a], q_extent[a], c);
+          flo = na_first_query_attending(j1, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
+          fhi = na_last_query_attending(j0, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
         }
       }
-      full_t0[a] = na_max(na_ceil_div(na_max(flo, 0), b_sub[a]), box_tile0[a]);
-      full_t1[a] = na_min((fhi + 1) / b_sub[a], box_tile0[a] + box_n[a]);  // one past the last whole tile
+      full_t0[a] = na_max((na_max(flo, 0) + b_sub[a] - 1) >> b_sub_lg[a], box_tile0[a]);
+      full_t1[a] = na_min((fhi + 1) >> b_sub_lg[a], box_tile0[a] + box_n[a]);  // one past the last whole tile
       if (fhi < 0 || full_t1[a] < full_t0[a]) full_t1[a] = full_t0[a];
     }
   }
@@ -283,9 +322,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // ---- this lane's stationary row -----------------------------------------------------------------
   const int r_in = rw * 32 + l32;  // row inside the tile: dimension 0 fastest
   int a_off[3];
-  a_off[0] = r_in % a_tile[0];
-  a_off[1] = (r_in / a_tile[0]) % a_tile[1];
-  a_off[2] = r_in / (a_tile[0] * a_tile[1]);
+  a_off[0] = r_in & (a_tile[0] - 1);
+  a_off[1] = (r_in >> a_tile_lg[0]) & (a_tile[1] - 1);
+  a_off[2] = r_in >> (a_tile_lg[0] + a_tile_lg[1]);
   // Row of the tensors / index into lse and delta: position in the permuted sequence, or the
   // token of the lane's coordinate in the original layout.
   // (original layout: a row past the end of its dilation group works on the group's last row and stores nothing)
@@ -299,7 +338,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
     a_crd[a] = p.fused ? na_min(c, e - 1) : c;
   }
   const int a_tok = group_tok + a_crd[0] * tok_step[0] + a_crd[1] * tok_step[1] + a_crd[2] * tok_step[2];
-  const int64_t batch_row0 = p.fused ? int64_t(bg / p.num_groups) * p.tokens : 0;  // first row of the batch entry (original layout)
+  const int64_t batch_row0 = p.fused ? int64_t(b_orig) * p.tokens : 0;  // first row of the batch entry (original layout)
   const int64_t a_row = p.fused ? batch_row0 + a_tok : (seq_row_a + int64_t(at) * AT + r_in);
   const int64_t a_stride = int64_t(heads_a) * D;
   const int64_t b_stride = int64_t(heads_b) * D;
@@ -363,18 +402,18 @@ fna_bwd_kernel(const FnaBwdParams p) {
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const int c = a_crd[a];
-      wst[a] = na_window_start(c, ksz[a], p.stride[a], extent[a], p.causal[a] != 0);
+      wst[a] = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
       wen[a] = na_window_end(c, wst[a], ksz[a], extent[a], p.causal[a] != 0);
     }
-    const int64_t stat_idx = p.fused ? (int64_t(bg / p.num_groups) * p.heads_q + head_a) * p.tokens + a_tok
+    const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
                                      : stat_row_q + head_a * stat_head_stride + int64_t(at) * AT + r_in;
     lse_l = p.lse[stat_idx] * kLog2e;
     delta_l = p.delta[stat_idx];
     // in-tile coordinates of every streamed position, packed in 10-bit fields
     for (int i = tid; i < BT; i += NT) {
-      const int t0 = i % b_sub[0];
-      const int t1 = (i / b_sub[0]) % b_sub[1];
-      const int t2 = i / (b_sub[0] * b_sub[1]);
+      const int t0 = i & (b_sub[0] - 1);
+      const int t1 = (i >> b_sub_lg[0]) & (b_sub[1] - 1);
+      const int t2 = i >> (b_sub_lg[0] + b_sub_lg[1]);
       sTabA[i] = uint32_t(t0) | (uint32_t(t1) << 10) | (uint32_t(t2) << 20);
     }
   } else {
@@ -388,9 +427,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // row (permuted) or token offset (original layout) of position r (dimension 0 fastest) of a streamed tile
   auto sub_pos = [&](int r) {
     if (!p.fused) return r;
-    const int t0 = r % b_sub[0];
-    r /= b_sub[0];
-    return t0 * tok_step[0] + (r % b_sub[1]) * tok_step[1] + (r / b_sub[1]) * tok_step[2];
+    const int t0 = r & (b_sub[0] - 1);
+    r >>= b_sub_lg[0];
+    return t0 * tok_step[0] + (r & (b_sub[1] - 1)) * tok_step[1] + (r >> b_sub_lg[1]) * tok_step[2];
   };
   // copy i of a thread moves chunk P = i * NT + tid of the tile (row P / CPR, LDS slot P % CPR)
   uint32_t off_u[PER];
@@ -413,7 +452,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // whole tiles, see full_t0), then the whole ones (the inner box itself).
   const int total = box_n[0] * box_n[1] * box_n[2];
   const int n_whole = (full_t1[0] - full_t0[0]) * (full_t1[1] - full_t0[1]) * (full_t1[2] - full_t0[2]);
-  const int head_b0 = KV_STATIONARY ? head_a * rep : head_a / rep;
+  const int head_b0 = KV_STATIONARY ? head_a * rep : na_div(head_a, p.d_rep);
   int wc[3], walk_head = 0;  // position of the walk in absolute tile coordinates
   // one step inside the box of the pass (WHOLE: the inner box, else the whole box)
   auto step = [&](auto whole_tag) {
@@ -454,7 +493,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
     int cc[3], half = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      t.origin[a] = wc[a] * b_sub[a];
+      t.origin[a] = wc[a] << b_sub_lg[a];
       t.lead[a] = 0;
       if (p.edge) {
         const int moved = na_min(t.origin[a], (KV_STATIONARY ? q_extent[a] : extent[a]) - b_sub[a]);
@@ -477,9 +516,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
 
   // in-tile coordinates of streamed position `lane` (the window tables below are built by wave 0)
   int qo[3];
-  qo[0] = lane % b_sub[0];
-  qo[1] = (lane / b_sub[0]) % b_sub[1];
-  qo[2] = lane / (b_sub[0] * b_sub[1]);
+  qo[0] = lane & (b_sub[0] - 1);
+  qo[1] = (lane >> b_sub_lg[0]) & (b_sub[1] - 1);
+  qo[2] = lane >> (b_sub_lg[0] + b_sub_lg[1]);
 
   const uint32_t lds_y1 = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sY1))));
   const uint32_t lds_y2 = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sY2))));
@@ -495,7 +534,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
         for (int a = 0; a < 3; ++a) {
           const int qc = t.origin[a] + qo[a];
           valid = valid && (qc < q_extent[a]) && (qo[a] >= t.lead[a]);
-          const int st = na_window_start(qc, ksz[a], p.stride[a], extent[a], p.causal[a] != 0);
+          const int st = na_window_start(qc, ksz[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
           const int en = na_window_end(qc, st, ksz[a], extent[a], p.causal[a] != 0);
           const int lo = na_min(na_max(st - a_first[a], 0), a_tile[a]);
           const int hi = na_min(na_max(en - a_first[a], 0), a_tile[a]);
@@ -514,7 +553,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       // LSE / delta of the tile's 64 queries: one asynchronous 4-byte-per-lane copy each
       // (wave 1, wave 2; the other waves but wave 0 make the same number of copies into a
       // spare row so that every wave counts the same number of outstanding copies per tile)
-      const int64_t stat_row0 = p.fused ? (int64_t(bg / p.num_groups) * p.heads_q + t.head_b) * p.tokens + t.row0
+      const int64_t stat_row0 = p.fused ? (int64_t(b_orig) * p.heads_q + t.head_b) * p.tokens + t.row0
                                         : stat_row_q + t.head_b * stat_head_stride + t.row0;
       const float* src = (wave == 2 ? p.delta : p.lse) + stat_row0;
       float* dst = (wave == 1) ? &sLse[stage * BT] : (wave == 2) ? &sDelta[stage * BT] : &sSpare[0];

@@ -115,27 +115,26 @@ NA_HD int na_group_extent(int X, int d, int g) { return X / d + 1 - ((g + (d - X
 // The queries that attend key coordinates j0 .. j1 of a dimension form an interval, because
 // window start and end are non-decreasing in the query coordinate: its first element is the
 // first query whose window ends past j0, its last the last query whose window starts at or
-// before j1 (queries 0 .. Lq-1, keys of extent L).  Both by bisection.  An empty interval comes
-// back as first > last.
-NA_HD int na_first_query_attending(int j0, int k, int s, int L, int Lq, bool causal) {
-  int lo = 0, hi = Lq;  // answer in [lo, hi]; hi == Lq: none
-  while (lo < hi) {
-    const int mid = (lo + hi) / 2;
-    const int st = na_window_start(mid, k, s, L, causal);
-    if (na_window_end(mid, st, k, L, causal) > j0) hi = mid;
-    else lo = mid + 1;
-  }
-  return lo;
+// before j1 (queries 0 .. Lq-1, keys of extent L, s_div = na_make_div(s)).  In closed form, one
+// division each: a window's start is its leader less the left reach, clamped to 0 .. L - k, and
+// the leaders are one per stride group.  An empty interval comes back as first > last.
+NA_HD int na_first_query_attending(int j0, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
+  if (causal) return na_min(j0, Lq);  // a causal window ends at its query
+  // start >= j0 - k + 1, that is leader >= j0 - k + 1 + left reach; without the clamp at 0 nothing to do
+  const int start = j0 - k + 1;
+  if (start <= 0) return 0;
+  const int past = start + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
+  return past <= 0 ? 0 : na_min(na_div(past + s - 1, s_div) * s, Lq);
 }
 
-NA_HD int na_last_query_attending(int j1, int k, int s, int L, int Lq, bool causal) {
-  int lo = -1, hi = Lq - 1;  // answer in [lo, hi]; lo == -1: none
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) / 2;
-    if (na_window_start(mid, k, s, L, causal) <= j1) lo = mid;
-    else hi = mid - 1;
+NA_HD int na_last_query_attending(int j1, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
+  if (causal) {
+    if (j1 + k >= L) return Lq - 1;
+    return na_min(na_div(j1 + k - s, s_div) * s + s - 1, Lq - 1);  // (s <= k)
   }
-  return lo;
+  if (j1 >= L - k) return Lq - 1;
+  const int reach = j1 + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
+  return reach < 0 ? -1 : na_min(na_div(reach, s_div) * s + s - 1, Lq - 1);
 }
 
 }  // namespace natten_amd

@@ -809,6 +809,7 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
     const long long runs = ((long long)p.batch * p.heads_kv * prod3(p.kv_tiled) + run - 1) / run;
     wg_kv = (runs + kNumXcd - 1) / kNumXcd * kNumXcd * run;
   }
+  set_bwd_divisions(p);
   if (wg_q > 0x7fffffffLL || wg_kv > 0x7fffffffLL) return fail("fna_backward: problem needs more than 2^31 workgroups");
   const int roles = p.roles ? p.roles : 3;
   if (roles & 2) {
@@ -1145,8 +1146,8 @@ int natten_amd_query_range(int key_first, int key_last, int kernel_size, int str
   if (kernel_size < 1 || stride < 1 || extent < 1 || num_queries < 1 || kernel_size > extent || stride > kernel_size ||
       key_first < 0 || key_last < key_first || key_last >= extent)
     return fail("query_range: invalid argument");
-  *first_query = na_first_query_attending(key_first, kernel_size, stride, extent, num_queries, is_causal != 0);
-  *last_query = na_last_query_attending(key_last, kernel_size, stride, extent, num_queries, is_causal != 0);
+  *first_query = na_first_query_attending(key_first, kernel_size, stride, na_make_div(stride), extent, num_queries, is_causal != 0);
+  *last_query = na_last_query_attending(key_last, kernel_size, stride, na_make_div(stride), extent, num_queries, is_causal != 0);
   return 0;
 }
 
