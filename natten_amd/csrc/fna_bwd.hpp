@@ -122,8 +122,18 @@ inline void set_bwd_divisions(FnaBwdParams& p) {
 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 
+// Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to):
+// what each instance's registers allow without spilling (head dim 128: 212 and 254; 64: 230 and 167;
+// 32: 153 and 122 of the SIMD's 512 per lane).  With two waves throughout, head dim 32 on 4 x 56 x 56
+// tokens, 7 x 7 windows took 82 (dK, dV) and 52 us (dQ); with three and four 59 and 39 us (the set-up
+// without divisions included).
+constexpr int bwd_waves_per_simd(int head_dim, int role) {
+  return head_dim == 128 ? 2 : head_dim == 64 ? (role == kBwdDQ ? 3 : 2) : (role == kBwdDQ ? 4 : 3);
+}
+
 template <typename T, int D, int ROLE, bool VARLEN = false>
-__global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256)
+__attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D, ROLE), bwd_waves_per_simd(D, ROLE))))
 fna_bwd_kernel(const FnaBwdParams p) {
   constexpr bool KV_STATIONARY = ROLE != kBwdDQ;
   constexpr bool PAIR = ROLE == kBwdPair;
