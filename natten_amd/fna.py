@@ -308,24 +308,29 @@ class AmdFnaFunction(torch.autograd.Function):
         )
         delta = torch_ops.compute_delta(output, d_output)
         na_dim = len(kernel_size)
-        fusable = _lib.backward_fused_layout_supported(query.shape[1 : 1 + na_dim], dilation, q_tile, kv_tile,
-                                                       row_bytes=query.shape[-2] * query.shape[-1] * 2)
-        if fusable and ctx.fused is not False:
-            # the kernels gather and scatter their tiles themselves: no permuted copies; each launch
-            # with the tile shapes that visit the fewest tiles for its role
-            kv_role = (None, None)
+        layout, row_bytes = tuple(int(x) for x in query.shape[1 : 1 + na_dim]), query.shape[-2] * query.shape[-1] * 2
+
+        def fits(qt, kt):
+            return _lib.backward_fused_layout_supported(layout, dilation, qt, kt, row_bytes=row_bytes)
+
+        # On the original tensors (the kernels gather and scatter their tiles themselves: no permuted
+        # copies) each launch takes the tile shapes that visit the fewest tiles for its role.  They are
+        # chosen among those that fit the dilation groups, so a problem whose one common pair of shapes
+        # does not fit stays off the permuted route too.
+        fused, kv_role = False, (None, None)
+        if ctx.fused is not False:
+            roles = None
             if ctx.role_tiles:
                 from .tile_config import choose_backward_role_tile_shapes
 
-                roles = choose_backward_role_tile_shapes(
-                    tuple(int(x) for x in query.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride),
-                    tuple(dilation), tuple(is_causal))
-                row_bytes = query.shape[-2] * query.shape[-1] * 2
-                if roles is not None and all(
-                    _lib.backward_fused_layout_supported(query.shape[1 : 1 + na_dim], dilation, qt, kt, row_bytes=row_bytes)
-                    for qt, kt in roles
-                ):
-                    (q_tile, kv_tile), kv_role = roles
+                roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation),
+                                                         tuple(is_causal))
+            if roles is not None and all(fits(qt, kt) for qt, kt in roles):
+                (q_tile, kv_tile), kv_role = roles
+                fused = True
+            else:
+                fused = fits(q_tile, kv_tile)
+        if fused:
             dq, dk, dv = torch_ops.fna_backward_fused(
                 query, key, value, d_output, lse.contiguous(), delta, kernel_size, stride, dilation, is_causal, scale,
                 q_tile, kv_tile, *kv_role,
