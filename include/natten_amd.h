@@ -307,6 +307,16 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
                              int64_t items, int head_dim, void* stream);
 
 /*
+ * What the backward entry points take besides the operands, in one pass: from q, out, d_out
+ * [batch, tokens, heads, head_dim] and lse [batch, tokens, heads] (the forward's) it writes q_scaled
+ * (q's shape: the logit operand described below), delta = rowsum(out * d_out) and a copy of lse, both
+ * head-major [batch, heads, tokens] float32.  natten_amd_fna_backward_fused then takes `roles` + 4.
+ */
+int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse,
+                                void* q_scaled, float* delta, float* lse_heads, int dtype, int batch,
+                                int tokens, int heads, int head_dim, float scale, void* stream);
+
+/*
  * Fused neighborhood attention backward on token-permuted operands.
  *   q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv [batch, seqlen_kv, heads_kv,
  *   head_dim], permuted like the forward operands (dimension 0 fastest inside a tile, dilation

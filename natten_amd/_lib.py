@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 16
+ABI_VERSION = 17
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -84,6 +84,10 @@ _SIGNATURES = {
     "natten_amd_compute_delta": (
         ctypes.c_int,
         [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p],
+    ),
+    "natten_amd_backward_prepare": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 7 + [ctypes.c_int] * 5 + [ctypes.c_float, ctypes.c_void_p],
     ),
     "natten_amd_fna_backward": (
         ctypes.c_int,
@@ -540,6 +544,26 @@ def compute_delta(out: Tensor, d_out: Tensor) -> Tensor:
     return delta
 
 
+def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: float, q_scaled: Tensor) -> Tuple[Tensor, Tensor]:
+    """q, out, d_out [B, *X, H, D], lse [B, *X, H] -> head-major float32 [B, H, prod(X)] delta =
+    rowsum(out * d_out) and lse; fills q_scaled (like q) with the logit operand of the dk / dv launch."""
+    _require_gpu(q, out, d_out, lse, q_scaled)
+    if out.dtype != q.dtype or d_out.dtype != q.dtype or out.shape != q.shape or d_out.shape != q.shape:
+        raise ValueError("out and d_out must be of q's shape and dtype.")
+    if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
+        raise ValueError("lse must be float32 of q's shape without the last dimension.")
+    B, H = q.shape[0], q.shape[-2]
+    tokens = lse.numel() // (B * H)
+    delta, lse_heads = torch.empty((2, B, H, tokens), dtype=torch.float32, device=q.device)
+    with _on_device(q):
+        rc = lib().natten_amd_backward_prepare(
+            q.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), q_scaled.data_ptr(), delta.data_ptr(),
+            lse_heads.data_ptr(), DTYPE_CODES[q.dtype], B, tokens, H, q.shape[-1], float(scale), _stream(q),
+        )
+    _check(rc)
+    return delta, lse_heads
+
+
 def fna_backward(
     q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, kernel_size, stride, dilation,
     is_causal, scale: float, q_shape, kv_shape, qkv_shape, q_tile_shape, kv_tile_shape,
@@ -580,32 +604,40 @@ def backward_fused_layout_supported(token_layout, dilation, q_tile_shape, kv_til
 
 
 def fna_backward_fused(
-    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, kernel_size, stride, dilation,
+    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Optional[Tensor], kernel_size, stride, dilation,
     is_causal, scale: float, q_tile_shape, kv_tile_shape, kv_role_q_tile_shape=None, kv_role_kv_tile_shape=None,
+    out: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    """Backward on the original tensors [B, *X, H, D] (lse, delta [B, *X, H]) -> (dq, dk, dv).
+    """Backward on the original tensors [B, *X, H, D] (lse, delta [B, *X, H]) -> (dq, dk, dv).  With
+    `out` (the forward's output) instead of delta, one pass forms delta and what else the launches read.
     kv_role_*_tile_shape: tile shapes of the launch that forms dk and dv, when they differ from those
     of the dq launch (q_tile_shape, kv_tile_shape)."""
     L = lib()
     na_dim = len(kernel_size)
     B, H = q.shape[0], q.shape[-2]
-    lse = lse.reshape(B, -1, H).transpose(1, 2).contiguous()
-    delta = delta.reshape(B, -1, H).transpose(1, 2).contiguous()
-    _require_gpu(q, k, v, d_out, lse, delta)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd fna_backward_fused does not support {q.dtype}.")
-    if lse.dtype != torch.float32 or delta.dtype != torch.float32:
-        raise ValueError("lse and delta must be float32.")
+    if (out is None) == (delta is None):
+        raise ValueError("fna_backward_fused takes either delta or the forward's output.")
     if (kv_role_q_tile_shape is None) != (kv_role_kv_tile_shape is None):
         raise ValueError("kv_role_q_tile_shape and kv_role_kv_tile_shape must be given together.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    if out is not None:
+        delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
+    else:
+        lse = lse.reshape(B, -1, H).transpose(1, 2).contiguous()
+        delta = delta.reshape(B, -1, H).transpose(1, 2).contiguous()
+    _require_gpu(q, k, v, d_out, lse, delta)
+    if lse.dtype != torch.float32 or delta.dtype != torch.float32:
+        raise ValueError("lse and delta must be float32.")
+    filled = 4 if out is not None else 0
     same = kv_role_q_tile_shape is None or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
     # The dk / dv launch streams the queries as the forward kernel multiplied them (scaled, rounded
     # once) from a workspace of q's size that the call fills first; dq serves as that workspace, so
     # the launch that writes dq comes last.
-    launches = [(3, q_tile_shape, kv_tile_shape)] if same else [
-        (2, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
+    launches = [(3 + filled, q_tile_shape, kv_tile_shape)] if same else [
+        (2 + filled, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
     with _on_device(q):
         for roles, qt, kt in launches:
             rc = L.natten_amd_fna_backward_fused(

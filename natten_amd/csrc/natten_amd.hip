@@ -320,7 +320,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
 
 extern "C" {
 
-int natten_amd_abi_version(void) { return 16; }
+int natten_amd_abi_version(void) { return 17; }
 
 uint64_t natten_amd_fna_forward_workspace_bytes(void) { return uint64_t(kQueueWords) * 4; }
 
@@ -812,7 +812,7 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   set_bwd_divisions(p);
   if (wg_q > 0x7fffffffLL || wg_kv > 0x7fffffffLL) return fail("fna_backward: problem needs more than 2^31 workgroups");
   const int roles = p.roles ? p.roles : 3;
-  if (roles & 2) {
+  if ((roles & 2) && !(roles & 4)) {
     // The key-stationary launch streams the queries as the forward kernel multiplied them: scaled
     // and rounded once, into the workspace.  It runs before the dQ launch, so that the workspace
     // may be the dq buffer.
@@ -824,6 +824,8 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
     hipLaunchKernelGGL((scale_queries_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<const T*>(p.q),
                        static_cast<T*>(const_cast<void*>(p.qs)), (int64_t)chunks, p.scale * 1.4426950408889634f);
     if (int rc = check_launch("fna_backward (scaled queries)")) return rc;
+  }
+  if (roles & 2) {
     if constexpr (D == 128) {
       // dK and dV by wave pairs (eight waves per workgroup): one wave's registers cannot hold the
       // accumulators, fragments and products of both
@@ -955,7 +957,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                   float scale, int roles, void* stream) {
   g_error[0] = 0;
   const char* what = "fna_backward_fused";
-  if (roles < 1 || roles > 3) return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), got %d", what, roles);
+  if (roles < 1 || roles > 7 || (roles & 3) == 0)
+    return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 where q_scaled is filled already, got %d", what, roles);
   if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, roles)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape || !kv_tile_shape)
@@ -1182,6 +1185,44 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
 #undef NA_DELTA_DTYPE
 #undef NA_DELTA_LAUNCH
   return check_launch("compute_delta");
+}
+
+int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse, void* q_scaled,
+                                float* delta, float* lse_heads, int dtype, int batch, int tokens, int heads, int head_dim,
+                                float scale, void* stream) {
+  g_error[0] = 0;
+  const char* what = "backward_prepare";
+  if (!q || !out || !d_out || !lse || !q_scaled || !delta || !lse_heads) return fail("%s: null pointer argument", what);
+  if (batch < 1 || tokens < 1 || heads < 1) return fail("%s: batch, tokens and heads must be positive", what);
+  if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(d_out) |
+       reinterpret_cast<uintptr_t>(q_scaled)) & 15)
+    return fail("%s: q, out, d_out and q_scaled must be 16-byte aligned", what);
+  int hb_lg = 0;
+  while (hb_lg < 3 && heads % (2 << hb_lg) == 0) ++hb_lg;
+  const int token_blocks = (tokens + (256 >> hb_lg) - 1) / (256 >> hb_lg), head_blocks = heads >> hb_lg;
+  const long long blocks = (long long)token_blocks * head_blocks * batch;
+  if (blocks > 0x7fffffffLL) return fail("%s: problem needs more than 2^31 workgroups", what);
+  const float c_log2 = scale * 1.4426950408889634f;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+#define NA_PREPARE_LAUNCH(TYPE, DD)                                                                                        \
+  hipLaunchKernelGGL((bwd_prepare_kernel<TYPE, DD>), dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const TYPE*>(q),                     \
+                     static_cast<const TYPE*>(out), static_cast<const TYPE*>(d_out), lse, static_cast<TYPE*>(q_scaled), delta, \
+                     lse_heads, tokens, heads, hb_lg, na_make_div(head_blocks), na_make_div(token_blocks), c_log2)
+#define NA_PREPARE_DTYPE(DD)                                             \
+  do {                                                                   \
+    if (dtype == NATTEN_AMD_F16) NA_PREPARE_LAUNCH(_Float16, DD);        \
+    else if (dtype == NATTEN_AMD_BF16) NA_PREPARE_LAUNCH(__bf16, DD);    \
+    else return fail("%s: unsupported dtype code %d", what, dtype);      \
+  } while (0)
+  switch (head_dim) {
+    case 32: NA_PREPARE_DTYPE(32); break;
+    case 64: NA_PREPARE_DTYPE(64); break;
+    case 128: NA_PREPARE_DTYPE(128); break;
+    default: return fail("%s: head_dim must be 32, 64 or 128, got %d", what, head_dim);
+  }
+#undef NA_PREPARE_DTYPE
+#undef NA_PREPARE_LAUNCH
+  return check_launch(what);
 }
 
 // widen: 0 = copy the payload, NATTEN_AMD_F8E4M3 / NATTEN_AMD_F8E5M2 = 8-bit float source, bf16 destination

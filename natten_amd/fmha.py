@@ -110,10 +110,13 @@ class AmdFmhaFunction(torch.autograd.Function):
         ctx.save_for_backward(query, key, value, out, lse)
         ctx.args = (is_causal, scale)
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)
         return out, lse
 
     @staticmethod
     def backward(ctx, d_out, d_lse):
+        if d_out is None:
+            return (None,) * 5
         query, key, value, out, lse = ctx.saved_tensors
         is_causal, scale = ctx.args
         head_dim = query.shape[-1]
@@ -179,10 +182,13 @@ class AmdFmhaVarlenFunction(torch.autograd.Function):
         ctx.args = (is_causal, scale)
         ctx.max_seqlens = (int(max_q), int(max_kv))
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)
         return out, lse
 
     @staticmethod
     def backward(ctx, d_out, d_lse):
+        if d_out is None:
+            return (None,) * 9
         query, key, value, out, lse, cu_q, cu_kv = ctx.saved_tensors
         is_causal, scale = ctx.args
         head_dim = query.shape[-1]

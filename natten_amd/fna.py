@@ -294,10 +294,13 @@ class AmdFnaFunction(torch.autograd.Function):
         # other route's bits (anchored_tiles=False promises those of the permuted route)
         ctx.role_tiles = bool(anchored_tiles) and not bwd_tiles_given
         ctx.mark_non_differentiable(lse)
+        ctx.set_materialize_grads(False)  # (no zeros for the gradient of lse, which is not read)
         return output, lse
 
     @staticmethod
     def backward(ctx, d_output, d_lse):
+        if d_output is None:
+            return (None,) * 16
         query, key, value, output, lse = ctx.saved_tensors
         kernel_size, stride, dilation, is_causal, scale, q_tile, kv_tile = ctx.na_args
         head_dim = query.shape[-1]
@@ -306,7 +309,6 @@ class AmdFnaFunction(torch.autograd.Function):
         query, key, value, output, d_output = (
             pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, output, d_output)
         )
-        delta = torch_ops.compute_delta(output, d_output)
         na_dim = len(kernel_size)
         layout, row_bytes = tuple(int(x) for x in query.shape[1 : 1 + na_dim]), query.shape[-2] * query.shape[-1] * 2
 
@@ -332,8 +334,8 @@ class AmdFnaFunction(torch.autograd.Function):
                 fused = fits(q_tile, kv_tile)
         if fused:
             dq, dk, dv = torch_ops.fna_backward_fused(
-                query, key, value, d_output, lse.contiguous(), delta, kernel_size, stride, dilation, is_causal, scale,
-                q_tile, kv_tile, *kv_role,
+                query, key, value, d_output, lse.contiguous(), None, kernel_size, stride, dilation, is_causal, scale,
+                q_tile, kv_tile, *kv_role, out=output,
             )
             if d_pad != head_dim:
                 dq, dk, dv = (t[..., :head_dim].contiguous() for t in (dq, dk, dv))
@@ -342,6 +344,7 @@ class AmdFnaFunction(torch.autograd.Function):
         def perm(x, tile):
             return token_permute_operation(x.contiguous(), tile, dilation, flip_tiled_dims=True)
 
+        delta = torch_ops.compute_delta(output, d_output)
         q_perm, qkv_shape, q_shape = perm(query, q_tile)
         do_perm, _, _ = perm(d_output, q_tile)
         lse_perm, _, _ = perm(lse.unsqueeze(-1), q_tile)
