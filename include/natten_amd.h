@@ -379,39 +379,34 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                   float scale, int roles, void* stream);
 
 /*
- * Dense attention backward (optional top-left causal mask).  Operands as above (lse and delta
- * head-major) with sequences zero-padded to padded_seqlen_q / padded_seqlen_kv rows (multiples
- * of 128); seqlen_q / seqlen_kv are the true lengths.
+ * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
+ * [batch, seqlen_kv, heads_kv, head_dim]; lse, delta head-major [batch, heads_q, seqlen_q].
+ * q_scaled as above; q_scaled_filled != 0: it is filled already (natten_amd_backward_prepare).
+ * Any sequence lengths: rows past the end of a sequence are gathered from its last row and masked.
  */
 int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out,
                                   const float* lse, const float* delta, void* dq, void* dk,
-                                  void* dv, void* q_scaled, int dtype, int batch, int seqlen_q, int seqlen_kv,
-                                  int padded_seqlen_q, int padded_seqlen_kv, int heads_q,
-                                  int heads_kv, int head_dim, int is_causal, float scale,
-                                  void* stream);
+                                  void* dv, void* q_scaled, int q_scaled_filled, int dtype, int batch,
+                                  int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                  int is_causal, float scale, void* stream);
 
 /*
  * Dense attention backward of a sequence-packed batch, one set of launches for all sequences.
- * The operands hold the `num_seqs` sequences back to back, each zero-padded to a multiple of
- * 128 rows: q, d_out, dq [1, rows_q, heads_q, head_dim], k, v, dk, dv [1, rows_kv, heads_kv,
- * head_dim], lse and delta head-major [1, heads_q, rows_q]; rows_q and rows_kv are multiples
- * of 128.  All four cumulative arrays are device int32 [num_seqs + 1]: sequence b has
- * cu_seqlens_q[b+1] - cu_seqlens_q[b] queries, which are rows padded_cu_seqlens_q[b] ... of the
- * operands (padded_cu_seqlens_* count padded lengths: multiples of 128, each covering the
- * sequence); keys likewise.  max_seqlen_q / max_seqlen_kv bound the sequence lengths (they size
- * the grid; rows of longer sequences would be left out).  Rows of dq, dk, dv outside every
- * sequence's padded range are not written.  A sequence whose offsets do not fit the row counts
- * is skipped by the kernels (the host cannot see the device arrays).  No host synchronisation.
+ * The operands hold the `num_seqs` sequences back to back: q, d_out, dq [1, rows_q, heads_q,
+ * head_dim], k, v, dk, dv [1, rows_kv, heads_kv, head_dim], lse and delta head-major
+ * [1, heads_q, rows_q].  Both cumulative arrays are device int32 [num_seqs + 1]: sequence b owns
+ * rows cu_seqlens_q[b] .. cu_seqlens_q[b+1] - 1 of the queries, keys likewise.  dq, dk and dv are
+ * written completely: rows of no sequence get zeros, and so do the rows of a sequence whose
+ * offsets do not fit the row counts of the other side (the host cannot see the device arrays).
+ * No host synchronisation.
  */
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v,
                                          const void* d_out, const float* lse, const float* delta,
-                                         void* dq, void* dk, void* dv, void* q_scaled, int dtype, int num_seqs,
-                                         int rows_q, int rows_kv, const int32_t* cu_seqlens_q,
-                                         const int32_t* cu_seqlens_kv,
-                                         const int32_t* padded_cu_seqlens_q,
-                                         const int32_t* padded_cu_seqlens_kv, int max_seqlen_q,
-                                         int max_seqlen_kv, int heads_q, int heads_kv,
-                                         int head_dim, int is_causal, float scale, void* stream);
+                                         void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
+                                         int dtype, int num_seqs, int rows_q, int rows_kv,
+                                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
+                                         int heads_q, int heads_kv, int head_dim, int is_causal,
+                                         float scale, void* stream);
 
 /*
  * Token permute: src [batch, *token_layout, heads, head_dim] -> dst

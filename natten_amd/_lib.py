@@ -100,11 +100,11 @@ _SIGNATURES = {
     ),
     "natten_amd_attention_backward": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 10 + [ctypes.c_float, ctypes.c_void_p],
+        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 9 + [ctypes.c_float, ctypes.c_void_p],
     ),
     "natten_amd_attention_backward_varlen": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 4 + [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6
+        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 2 + [ctypes.c_int] * 4
         + [ctypes.c_float, ctypes.c_void_p],
     ),
     "natten_amd_token_permute_widen": (
@@ -651,54 +651,48 @@ def fna_backward_fused(
 
 
 def attention_backward(
-    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, seqlen_q: int, seqlen_kv: int,
-    is_causal: bool, scale: float,
+    q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, is_causal: bool, scale: float,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    """Dense attention backward on operands zero-padded to multiples of 128 rows -> (dq, dk, dv), padded alike.
-    lse, delta: [batch, padded seqlen_q, heads_q]; the kernels take them head-major."""
+    """Dense attention backward, q, out, d_out [B, S, H, D], k / v [B, Skv, Hkv, D], lse [B, S, H] -> (dq, dk, dv)."""
     L = lib()
-    lse, delta = lse.transpose(1, 2).contiguous(), delta.transpose(1, 2).contiguous()
-    _require_gpu(q, k, v, d_out, lse, delta)
+    _require_gpu(q, k, v)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_backward does not support {q.dtype}.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
     with _on_device(q):
         rc = L.natten_amd_attention_backward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], q.shape[0], int(seqlen_q),
-            int(seqlen_kv), q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,
-            float(scale), _stream(q),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], q.shape[0], q.shape[1],
+            k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)
     return dq, dk, dv
 
 
 def attention_backward_varlen(
-    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, cu_q: Tensor, cu_kv: Tensor,
-    padded_cu_q: Tensor, padded_cu_kv: Tensor, max_seqlen_q: int, max_seqlen_kv: int, is_causal: bool, scale: float,
+    q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, cu_q: Tensor, cu_kv: Tensor,
+    is_causal: bool, scale: float,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    """Dense attention backward of a sequence-packed batch whose sequences are each zero-padded to
-    a multiple of 128 rows -> (dq, dk, dv) in the same padded packing.  q, d_out [1, rows_q, H, D];
-    k, v [1, rows_kv, Hkv, D]; lse, delta [1, rows_q, H] (the kernels take them head-major); the
-    four cumulative arrays are device int32 [sequences + 1].  Rows outside every sequence's padded
-    range are left unwritten."""
+    """Dense attention backward of a sequence-packed batch: q, out, d_out [1, rows_q, H, D], k, v [1, rows_kv,
+    Hkv, D], lse [1, rows_q, H], device int32 cumulative lengths [sequences + 1] -> (dq, dk, dv); rows
+    of no sequence come back as zeros."""
     L = lib()
-    lse, delta = lse.transpose(1, 2).contiguous(), delta.transpose(1, 2).contiguous()
-    _require_gpu(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv)
+    _require_gpu(q, k, v, cu_q, cu_kv)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_backward_varlen does not support {q.dtype}.")
-    cums = (cu_q, cu_kv, padded_cu_q, padded_cu_kv)
-    if any(c.dtype != torch.int32 or c.dim() != 1 or c.numel() != cu_q.numel() or not c.is_contiguous() for c in cums):
+    if any(c.dtype != torch.int32 or c.dim() != 1 or c.numel() != cu_q.numel() for c in (cu_q, cu_kv)):
         raise ValueError("cumulative sequence lengths must be contiguous int32 vectors of one length.")
     if cu_q.numel() < 2 or q.shape[0] != 1 or k.shape[0] != 1:
         raise ValueError("sequence-packed operands have batch 1 and at least one sequence.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
     with _on_device(q):
         rc = L.natten_amd_attention_backward_varlen(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], cu_q.numel() - 1, q.shape[1], k.shape[1],
-            cu_q.data_ptr(), cu_kv.data_ptr(), padded_cu_q.data_ptr(), padded_cu_kv.data_ptr(), int(max_seqlen_q),
-            int(max_seqlen_kv), q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], cu_q.numel() - 1, q.shape[1],
+            k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,
+            float(scale), _stream(q),
         )
     _check(rc)
     return dq, dk, dv

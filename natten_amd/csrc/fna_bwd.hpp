@@ -73,15 +73,13 @@ struct FnaBwdParams {
   int edge;
   int tok_stride[3];  // tokens per unit step of an original coordinate: X1*X2, X2, 1
   int tokens;         // X0 * X1 * X2
-  // Sequence-packed dense attention (VARLEN instances only; null otherwise).  `batch` sequences
-  // lie back to back in one row range (the tensors have batch 1; seqlen_q / seqlen_kv count all
-  // their rows), each padded to a multiple of 128 rows: sequence b owns query rows
-  // pcu_q[b] .. pcu_q[b+1]-1 of which the first cu_q[b+1] - cu_q[b] are real, keys likewise;
-  // q_tiled[0] / kv_tiled[0] count the tiles of the longest sequence.
-  const int32_t* cu_q;    // [batch + 1] cumulative real lengths
+  // Sequence-packed dense attention (RAGGED instances only; null otherwise): num_seqs sequences lie
+  // back to back in one row range (the tensors have batch 1; seqlen_q / seqlen_kv count all their
+  // rows), sequence b owns query rows cu_q[b] .. cu_q[b+1]-1 and key rows cu_kv[b] .. cu_kv[b+1]-1;
+  // q_tiled[0] / kv_tiled[0] count the tiles that any such batch has at most (locate_packed_tile).
+  const int32_t* cu_q;    // [num_seqs + 1]
   const int32_t* cu_kv;
-  const int32_t* pcu_q;   // [batch + 1] cumulative padded lengths (row offsets into the tensors)
-  const int32_t* pcu_kv;
+  int num_seqs;
   // Workgroup order of the key-stationary launch.  0: every XCD takes one contiguous eighth of
   // the (batch, head, tile) space.  > 0: runs of this many consecutive tiles are dealt round-robin
   // to the XCDs (the grid is then a whole number of rounds of 8 runs).
@@ -131,7 +129,11 @@ constexpr int bwd_waves_per_simd(int head_dim, int role) {
   return head_dim == 128 ? 2 : head_dim == 64 ? (role == kBwdDQ ? 3 : 2) : (role == kBwdDQ ? 4 : 3);
 }
 
-template <typename T, int D, int ROLE, bool VARLEN = false>
+// RAGGED: dense attention whose sequences end inside a tile, packed ones among them.  Rows past the end
+// of a sequence are gathered from its last row; stationary ones store nothing, streamed ones are masked.
+// (Padding the sequences into copies first made 67 launches of a packed training step, of index arithmetic
+// and copies most of them: 10 sequences of 1 .. 2048, H 16 / 4, D 128 919 us, now 6 launches and 462 us.)
+template <typename T, int D, int ROLE, bool RAGGED = false>
 __global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256)
 __attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D, ROLE), bwd_waves_per_simd(D, ROLE))))
 fna_bwd_kernel(const FnaBwdParams p) {
@@ -220,25 +222,40 @@ fna_bwd_kernel(const FnaBwdParams p) {
     const int chunk = (total_wg + kNumXcd - 1) / kNumXcd;
     lin = (int(blockIdx.x) % kNumXcd) * chunk + int(blockIdx.x) / kNumXcd;
   }
+  // Ragged dense attention: heads fastest, so that the long tiles of a head's sequences (the first key
+  // tiles and the last query tiles where causal) are spread over all XCDs, and with as many heads
+  // as XCDs, or a divisor of them, every XCD still streams one head's tiles.  Runs of 32 tiles put a whole
+  // 2048-token sequence of a head on one XCD: packed training step of 10 sequences of 1 .. 2048, H 16 /
+  // 4, D 128: dK / dV launch 326 -> 254 us.
+  if constexpr (RAGGED) lin = int(blockIdx.x);
   if (lin >= total_wg) return;
   // Within a head the tiles are taken with dimension 0 slowest: the workgroups running side by
   // side are then neighbours in the faster dimensions at the same dimension-0 position and
   // walk the same streamed tiles at about the same time.
-  const int bh = na_div(lin, KV_STATIONARY ? p.d_num_kv : p.d_num_q);
+  const NaDiv d_num_a = KV_STATIONARY ? p.d_num_kv : p.d_num_q, d_heads_a = KV_STATIONARY ? p.d_heads_kv : p.d_heads_q;
+  int bg, head_a, rm;
+  if constexpr (RAGGED) {
+    const int bt = na_div(lin, d_heads_a);
+    head_a = lin - bt * heads_a;
+    bg = na_div(bt, d_num_a);
+    rm = bt - bg * num_a;
+  } else {
+    const int bh = na_div(lin, d_num_a);
+    rm = lin - bh * num_a;
+    bg = na_div(bh, d_heads_a);
+    head_a = bh - bg * heads_a;
+  }
   int tc[3];
   {
-    const int rm = lin - bh * num_a;
     const int t01 = na_div(rm, KV_STATIONARY ? p.d_kv_tiled[2] : p.d_q_tiled[2]);
     tc[2] = rm - t01 * a_tiled[2];
     tc[0] = na_div(t01, KV_STATIONARY ? p.d_kv_tiled[1] : p.d_q_tiled[1]);
     tc[1] = t01 - tc[0] * a_tiled[1];
     // a causal dimension 0: the query tiles with the longest key ranges are the last ones;
     // they start first (key tiles are already in that order)
-    if (!KV_STATIONARY && p.causal[0]) tc[0] = a_tiled[0] - 1 - tc[0];
+    if (!KV_STATIONARY && p.causal[0] && !(RAGGED && p.cu_q)) tc[0] = a_tiled[0] - 1 - tc[0];
   }
   const int at = tc[0] + a_tiled[0] * (tc[1] + a_tiled[1] * tc[2]);  // position in the permuted sequence
-  const int bg = na_div(bh, KV_STATIONARY ? p.d_heads_kv : p.d_heads_q);
-  const int head_a = bh - bg * heads_a;
   const int b_orig = na_div(bg, p.d_num_groups);  // batch entry before the dilation groups were folded in
 
   // first rows of this batch entry's sequences, its lse / delta values of head 0, and the
@@ -249,21 +266,27 @@ fna_bwd_kernel(const FnaBwdParams p) {
   int ksz[3] = {p.ksize[0], p.ksize[1], p.ksize[2]};
   int keys0 = p.ext_base[0], queries0 = p.q_extent0;  // (extents of dimension 0 before the uneven dilation groups)
   bool empty = false;
-  if constexpr (VARLEN) {
-    const int q0 = p.cu_q[bg], kv0 = p.cu_kv[bg], pq0 = p.pcu_q[bg], pkv0 = p.pcu_kv[bg];
-    const int len_q = p.cu_q[bg + 1] - q0, len_kv = p.cu_kv[bg + 1] - kv0;
-    const int pad_q = p.pcu_q[bg + 1] - pq0, pad_kv = p.pcu_kv[bg + 1] - pkv0;
-    // offsets the tensors cannot hold are not followed
-    if (len_q < 0 || len_kv < 0 || pq0 < 0 || pkv0 < 0 || pad_q < len_q || pad_kv < len_kv ||
-        ((pq0 | pkv0 | pad_q | pad_kv) & 127) != 0 || pq0 + pad_q > p.seqlen_q || pkv0 + pad_kv > p.seqlen_kv)
-      return;
-    if (tc[0] * AT >= (KV_STATIONARY ? pad_kv : pad_q)) return;  // the longest sequence has more tiles than this one
-    seq_row_a = KV_STATIONARY ? pkv0 : pq0;
-    seq_row_b = KV_STATIONARY ? pq0 : pkv0;
-    stat_row_q = pq0;
-    keys0 = ksz[0] = na_max(len_kv, 1);
-    queries0 = na_max(len_q, 1);
-    empty = len_q == 0 || len_kv == 0;  // nothing attends, or attends to nothing: zero gradients
+  if constexpr (RAGGED) {
+    if (p.cu_q) {
+      PackedTile t;
+      if (!locate_packed_tile(KV_STATIONARY ? p.cu_kv : p.cu_q, p.num_seqs, seq_a, 7, tc[0], lane, t)) return;
+      tc[0] = t.tile;
+      seq_row_a = t.row0;
+      int other0 = 0, other = 0;  // the sequence's rows on the streamed side
+      if (!t.gap) {
+        const int32_t* cu = KV_STATIONARY ? p.cu_q : p.cu_kv;
+        other0 = cu[t.seq];
+        other = cu[t.seq + 1] - other0;
+        if (other0 < 0 || other < 0 || other0 > seq_b - other) other0 = other = 0;  // offsets the tensors cannot hold are not followed
+        // (the query tiles with the longest key ranges first, as above)
+        if (!KV_STATIONARY && p.causal[0]) tc[0] = ((t.rows + AT - 1) / AT) - 1 - tc[0];
+      }
+      empty = other == 0;  // nothing attends, or attends to nothing: zero gradients
+      seq_row_b = other0;
+      stat_row_q = KV_STATIONARY ? other0 : t.row0;
+      keys0 = ksz[0] = na_max(KV_STATIONARY ? t.rows : other, 1);
+      queries0 = na_max(KV_STATIONARY ? other : t.rows, 1);
+    }
   }
 
   int extent[3], q_extent[3], a_first[3], b_sub[3], b_sub_lg[3], box_tile0[3], box_n[3], full_t0[3], full_t1[3];
@@ -314,7 +337,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
         flo = st_l;
         fhi = na_window_end(qf, st_f, ksz[a], extent[a], c) - 1;
       } else {
-        const int j0 = a_first[a], j1 = j0 + a_tile[a] - 1;
+        // (rows past the end that are not stored may take part: only zero-padded sequences need their mask)
+        const int j0 = a_first[a];
+        const int j1 = (RAGGED || p.fused) ? na_min(j0 + a_tile[a], extent[a]) - 1 : j0 + a_tile[a] - 1;
         if (j1 >= extent[a]) {
           flo = 1;  // the tile holds padding keys: never whole
           fhi = 0;
@@ -344,12 +369,13 @@ fna_bwd_kernel(const FnaBwdParams p) {
   for (int a = 0; a < 3; ++a) {
     const int c = a_first[a] + a_off[a];
     const int e = KV_STATIONARY ? extent[a] : q_extent[a];
-    a_valid = a_valid && (c < e || !p.fused);
-    a_crd[a] = p.fused ? na_min(c, e - 1) : c;
+    a_valid = a_valid && (c < e || !(RAGGED || p.fused));
+    a_crd[a] = (RAGGED || p.fused) ? na_min(c, e - 1) : c;
   }
   const int a_tok = group_tok + a_crd[0] * tok_step[0] + a_crd[1] * tok_step[1] + a_crd[2] * tok_step[2];
   const int64_t batch_row0 = p.fused ? int64_t(b_orig) * p.tokens : 0;  // first row of the batch entry (original layout)
-  const int64_t a_row = p.fused ? batch_row0 + a_tok : (seq_row_a + int64_t(at) * AT + r_in);
+  const int a_seq_row = RAGGED ? a_crd[0] : at * AT + r_in;  // its row of the permuted / ragged sequence
+  const int64_t a_row = p.fused ? batch_row0 + a_tok : seq_row_a + a_seq_row;
   const int64_t a_stride = int64_t(heads_a) * D;
   const int64_t b_stride = int64_t(heads_b) * D;
   const float kLog2e = 1.4426950408889634f;
@@ -416,7 +442,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       wen[a] = na_window_end(c, wst[a], ksz[a], extent[a], p.causal[a] != 0);
     }
     const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
-                                     : stat_row_q + head_a * stat_head_stride + int64_t(at) * AT + r_in;
+                                     : stat_row_q + head_a * stat_head_stride + a_seq_row;
     lse_l = p.lse[stat_idx] * kLog2e;
     delta_l = p.delta[stat_idx];
     // in-tile coordinates of every streamed position, packed in 10-bit fields
@@ -559,6 +585,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // the asynchronous copies of a streamed tile (and of its LSE / delta values) into a stage
   auto issue_copies = [&](const Tile& t, int stage, int stage2) {
     const int64_t row = p.fused ? batch_row0 + t.row0 : seq_row_b + t.row0;
+    // a tile that ends past its sequence: the rows from `last` on are the sequence's last one
+    const int last = (KV_STATIONARY ? q_extent[0] : extent[0]) - 1 - t.origin[0];
+    const bool partial = RAGGED && last < BT - 1;
     if constexpr (KV_STATIONARY) {
       // LSE / delta of the tile's 64 queries: one asynchronous 4-byte-per-lane copy each
       // (wave 1, wave 2; the other waves but wave 0 make the same number of copies into a
@@ -567,7 +596,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
                                         : stat_row_q + t.head_b * stat_head_stride + t.row0;
       const float* src = (wave == 2 ? p.delta : p.lse) + stat_row0;
       float* dst = (wave == 1) ? &sLse[stage * BT] : (wave == 2) ? &sDelta[stage * BT] : &sSpare[0];
-      if (wave != 0) async_copy4_asm(src, stat_off, lds_address(dst));
+      const uint32_t off = partial ? uint32_t(na_min(lane, last)) * 4u : stat_off;
+      if (wave != 0) async_copy4_asm(src, off, lds_address(dst));
     }
     const int64_t elem = row * b_stride + int64_t(t.head_b) * D;
     const uint64_t y1 = uniform64(y1_all + elem), y2 = uniform64(y2_all + elem);
@@ -575,8 +605,12 @@ fna_bwd_kernel(const FnaBwdParams p) {
     const uint32_t dst2 = uint32_t(__builtin_amdgcn_readfirstlane(stage2 * TILE_BYTES + wave * 1024));
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      async_copy16_uniform(y1, off_u[i], lds_y1 + dst + uint32_t(i * NT * 16));
-      async_copy16_uniform(y2, off_u[i], lds_y2 + dst2 + uint32_t(i * NT * 16));
+      uint32_t off = off_u[i];
+      if constexpr (RAGGED) {
+        if (partial) off -= uint32_t(na_max((i * NT + tid) / CPR - last, 0)) * uint32_t(b_stride * 2);
+      }
+      async_copy16_uniform(y1, off, lds_y1 + dst + uint32_t(i * NT * 16));
+      async_copy16_uniform(y2, off, lds_y2 + dst2 + uint32_t(i * NT * 16));
     }
   };
   auto issue = [&](const Tile& t, int stage, bool masked) {

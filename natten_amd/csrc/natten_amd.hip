@@ -785,7 +785,7 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
 // ---- backward ---------------------------------------------------------------------------------
 
 extern "C++" {
-template <typename T, int D, bool VARLEN>
+template <typename T, int D, bool RAGGED>
 static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   FnaBwdParams p = params;
   // grids are padded to a multiple of the 8 XCDs: each XCD takes a contiguous eighth of the tiles
@@ -829,34 +829,34 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
     if constexpr (D == 128) {
       // dK and dV by wave pairs (eight waves per workgroup): one wave's registers cannot hold the
       // accumulators, fragments and products of both
-      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdPair, VARLEN>), dim3((unsigned)wg_kv), dim3(512), 0, stream, p);
+      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdPair, RAGGED>), dim3((unsigned)wg_kv), dim3(512), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDKV, VARLEN>), dim3((unsigned)wg_kv), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDKV, RAGGED>), dim3((unsigned)wg_kv), dim3(256), 0, stream, p);
     }
     if (int rc = check_launch("fna_backward (dK, dV)")) return rc;
   }
   if (roles & 1) {
-    hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDQ, VARLEN>), dim3((unsigned)wg_q), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDQ, RAGGED>), dim3((unsigned)wg_q), dim3(256), 0, stream, p);
     if (int rc = check_launch("fna_backward (dQ)")) return rc;
   }
   return 0;
 }
 
 template <typename T>
-static int dispatch_bwd_head_dim(const FnaBwdParams& p, int head_dim, hipStream_t stream) {
-  const bool varlen = p.cu_q != nullptr;  // sequence-packed dense attention
+static int dispatch_bwd_head_dim(const FnaBwdParams& p, int head_dim, hipStream_t stream, bool ragged) {
   switch (head_dim) {
-    case 32: return varlen ? launch_bwd<T, 32, true>(p, stream) : launch_bwd<T, 32, false>(p, stream);
-    case 64: return varlen ? launch_bwd<T, 64, true>(p, stream) : launch_bwd<T, 64, false>(p, stream);
-    case 128: return varlen ? launch_bwd<T, 128, true>(p, stream) : launch_bwd<T, 128, false>(p, stream);
+    case 32: return ragged ? launch_bwd<T, 32, true>(p, stream) : launch_bwd<T, 32, false>(p, stream);
+    case 64: return ragged ? launch_bwd<T, 64, true>(p, stream) : launch_bwd<T, 64, false>(p, stream);
+    case 128: return ragged ? launch_bwd<T, 128, true>(p, stream) : launch_bwd<T, 128, false>(p, stream);
   }
   return fail("fna_backward: head_dim must be 32, 64 or 128, got %d", head_dim);
 }
 
-static int dispatch_bwd(const FnaBwdParams& p, int dtype, int head_dim, hipStream_t stream) {
+// ragged: dense attention on sequences that end inside a tile
+static int dispatch_bwd(const FnaBwdParams& p, int dtype, int head_dim, hipStream_t stream, bool ragged = false) {
   switch (dtype) {
-    case NATTEN_AMD_F16: return dispatch_bwd_head_dim<_Float16>(p, head_dim, stream);
-    case NATTEN_AMD_BF16: return dispatch_bwd_head_dim<__bf16>(p, head_dim, stream);
+    case NATTEN_AMD_F16: return dispatch_bwd_head_dim<_Float16>(p, head_dim, stream, ragged);
+    case NATTEN_AMD_BF16: return dispatch_bwd_head_dim<__bf16>(p, head_dim, stream, ragged);
   }
   return fail("fna_backward: only 16-bit float operands are supported, got dtype code %d", dtype);
 }
@@ -1043,31 +1043,21 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
 }
 
-int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int batch,
-                                  int seqlen_q, int seqlen_kv, int padded_seqlen_q, int padded_seqlen_kv, int heads_q,
-                                  int heads_kv, int head_dim, int is_causal, float scale, void* stream) {
-  g_error[0] = 0;
-  const char* what = "attention_backward";
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
-  if (int rc = check_common(what, q, k, v, dq, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
-  if (padded_seqlen_q % 128 != 0 || padded_seqlen_kv % 128 != 0 || padded_seqlen_q < seqlen_q ||
-      padded_seqlen_kv < seqlen_kv)
-    return fail("%s: padded sequence lengths (%d, %d) must be multiples of 128 that cover (%d, %d)", what,
-                padded_seqlen_q, padded_seqlen_kv, seqlen_q, seqlen_kv);
-  // the 1-D neighborhood problem whose window is the whole key sequence, with its own query count
-  FnaBwdParams p;
+namespace {
+// dense attention backward as the 1-D neighborhood problem whose window is the whole key sequence
+void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v, const void* d_out, const float* lse,
+                    const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int batch, int seqlen_q, int seqlen_kv,
+                    int heads_q, int heads_kv, int is_causal, float scale, int filled) {
   memset(&p, 0, sizeof(p));
   for (int a = 0; a < 3; ++a) {
     p.qkv_shape[a] = p.ksize[a] = p.stride[a] = p.dil[a] = p.q_tile[a] = p.kv_tile[a] = p.q_tiled[a] = p.kv_tiled[a] = 1;
   }
-  p.qkv_shape[0] = seqlen_kv;
-  p.ksize[0] = seqlen_kv;
+  p.qkv_shape[0] = p.ksize[0] = seqlen_kv;
+  p.q_extent0 = seqlen_q;
   p.causal[0] = is_causal != 0;
   p.q_tile[0] = p.kv_tile[0] = 128;
-  p.q_tiled[0] = padded_seqlen_q / 128;
-  p.kv_tiled[0] = padded_seqlen_kv / 128;
-  p.q_extent0 = seqlen_q;
+  p.q_tiled[0] = na_ceil_div(seqlen_q, 128);
+  p.kv_tiled[0] = na_ceil_div(seqlen_kv, 128);
   p.q = q;
   p.qs = q_scaled;
   p.k = k;
@@ -1081,65 +1071,49 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
   p.batch = batch;
   p.heads_q = heads_q;
   p.heads_kv = heads_kv;
-  p.seqlen_q = padded_seqlen_q;
-  p.seqlen_kv = padded_seqlen_kv;
+  p.seqlen_q = seqlen_q;
+  p.seqlen_kv = seqlen_kv;
   p.num_groups = 1;
   p.scale = scale;
-  return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
+  p.roles = 3 + (filled ? 4 : 0);
+}
+}  // namespace
+
+int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
+                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
+                                  int dtype, int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                  int is_causal, float scale, void* stream) {
+  g_error[0] = 0;
+  const char* what = "attention_backward";
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
+  FnaBwdParams p;
+  fill_dense_bwd(p, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal,
+                 scale, q_scaled_filled);
+  // (sequences of whole tiles need no clamping: the instances of neighborhood attention)
+  return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), seqlen_q % 128 != 0 || seqlen_kv % 128 != 0);
 }
 
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v, const void* d_out,
                                          const float* lse, const float* delta, void* dq, void* dk, void* dv,
-                                         void* q_scaled, int dtype, int num_seqs, int rows_q, int rows_kv, const int32_t* cu_seqlens_q,
-                                         const int32_t* cu_seqlens_kv, const int32_t* padded_cu_seqlens_q,
-                                         const int32_t* padded_cu_seqlens_kv, int max_seqlen_q, int max_seqlen_kv,
-                                         int heads_q, int heads_kv, int head_dim, int is_causal, float scale,
-                                         void* stream) {
+                                         void* q_scaled, int q_scaled_filled, int dtype, int num_seqs, int rows_q, int rows_kv,
+                                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv, int heads_q,
+                                         int heads_kv, int head_dim, int is_causal, float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "attention_backward_varlen";
   if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
   if (int rc = check_common(what, q, k, v, dq, lse, num_seqs, rows_q, rows_kv, heads_q, heads_kv, head_dim)) return rc;
-  if (!cu_seqlens_q || !cu_seqlens_kv || !padded_cu_seqlens_q || !padded_cu_seqlens_kv)
-    return fail("%s: null cumulative length argument", what);
-  if (rows_q % 128 != 0 || rows_kv % 128 != 0)
-    return fail("%s: the padded row counts (%d, %d) must be multiples of 128", what, rows_q, rows_kv);
-  if (max_seqlen_q < 1 || max_seqlen_kv < 1 || max_seqlen_q > rows_q || max_seqlen_kv > rows_kv)
-    return fail("%s: max_seqlen_q / max_seqlen_kv (%d, %d) must lie in 1 .. the row counts (%d, %d)", what,
-                max_seqlen_q, max_seqlen_kv, rows_q, rows_kv);
-  // per sequence: the 1-D neighborhood problem whose window is the whole key sequence
+  if (!cu_seqlens_q || !cu_seqlens_kv) return fail("%s: null cumulative length argument", what);
   FnaBwdParams p;
-  memset(&p, 0, sizeof(p));
-  for (int a = 0; a < 3; ++a) {
-    p.qkv_shape[a] = p.ksize[a] = p.stride[a] = p.dil[a] = p.q_tile[a] = p.kv_tile[a] = p.q_tiled[a] = p.kv_tiled[a] = 1;
-  }
-  p.qkv_shape[0] = p.ksize[0] = max_seqlen_kv;  // replaced per sequence inside the kernel
-  p.q_extent0 = max_seqlen_q;
-  p.causal[0] = is_causal != 0;
-  p.q_tile[0] = p.kv_tile[0] = 128;
-  p.q_tiled[0] = (max_seqlen_q + 127) / 128;
-  p.kv_tiled[0] = (max_seqlen_kv + 127) / 128;
-  p.q = q;
-  p.qs = q_scaled;
-  p.k = k;
-  p.v = v;
-  p.d_out = d_out;
-  p.lse = lse;
-  p.delta = delta;
-  p.dq = dq;
-  p.dk = dk;
-  p.dv = dv;
-  p.batch = num_seqs;
-  p.heads_q = heads_q;
-  p.heads_kv = heads_kv;
-  p.seqlen_q = rows_q;
-  p.seqlen_kv = rows_kv;
-  p.num_groups = 1;
-  p.scale = scale;
+  fill_dense_bwd(p, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
+                 q_scaled_filled);
+  // lengths and windows are replaced per sequence inside the kernel
+  p.q_tiled[0] = rows_q / 128 + 2 * (num_seqs + 1);
+  p.kv_tiled[0] = rows_kv / 128 + 2 * (num_seqs + 1);
   p.cu_q = cu_seqlens_q;
   p.cu_kv = cu_seqlens_kv;
-  p.pcu_q = padded_cu_seqlens_q;
-  p.pcu_kv = padded_cu_seqlens_kv;
-  return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
+  p.num_seqs = num_seqs;
+  return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), true);
 }
 
 int natten_amd_query_range(int key_first, int key_last, int kernel_size, int stride, int extent, int num_queries,

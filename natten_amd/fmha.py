@@ -88,18 +88,10 @@ def amd_fmha(
     return out
 
 
-def _pad_rows(x: Tensor, rows: int) -> Tensor:
-    """Zero-pads dimension 1 to `rows`."""
-    if x.shape[1] == rows:
-        return x.contiguous()
-    pad = [0, 0] * (x.dim() - 2) + [0, rows - x.shape[1]]
-    return torch.nn.functional.pad(x, pad).contiguous()
-
-
 class AmdFmhaFunction(torch.autograd.Function):
     """Dense attention with a backward pass (fp16 / bf16, fixed-length batches): the backward
-    kernels of neighborhood attention on the 1-D problem whose window is the whole key sequence,
-    sequences zero-padded to multiples of 128 rows.  Counterpart of the reference's
+    kernels of neighborhood attention on the 1-D problem whose window is the whole key sequence.
+    Counterpart of the reference's
     src/natten/backends/blackwell_fmha.py:52-170; the gradient of LSE is not propagated.  The saved
     output and LSE are the returned tensors themselves (see AmdFnaFunction)."""
 
@@ -124,53 +116,16 @@ class AmdFmhaFunction(torch.autograd.Function):
         query, key, value, out, d_out = (
             pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, out, d_out)
         )
-        delta = torch_ops.compute_delta(out, d_out)
-        sq, skv = query.shape[1], key.shape[1]
-        pq, pkv = -(-sq // 128) * 128, -(-skv // 128) * 128
-        dq, dk, dv = torch_ops.attention_backward(
-            _pad_rows(query, pq), _pad_rows(key, pkv), _pad_rows(value, pkv), _pad_rows(d_out, pq),
-            _pad_rows(lse, pq), _pad_rows(delta, pq), sq, skv, is_causal, scale,
-        )
-        return dq[:, :sq, :, :head_dim], dk[:, :skv, :, :head_dim], dv[:, :skv, :, :head_dim], None, None
-
-
-def _padded_packing(cu: Tensor, rows: int) -> Tuple[Tensor, Tensor, Tensor, int]:
-    """A packing of the same sequences with every sequence padded to a multiple of 128 rows, from
-    device arithmetic only (no copy to the host): (padded cumulative lengths [sequences + 1] int32,
-    padded row of every packed row [rows] int64, which packed rows belong to a sequence [rows]
-    bool, row count of the padded packing).  The row count is an upper bound the host can know:
-    rows + 127 per sequence, rounded up to 128."""
-    num_seqs = cu.numel() - 1
-    cu = cu.to(torch.int32)
-    padded_len = (cu[1:] - cu[:-1] + 127) // 128 * 128
-    padded_cu = torch.cat([cu.new_zeros(1), torch.cumsum(padded_len, 0).to(torch.int32)])
-    row = torch.arange(rows, device=cu.device, dtype=torch.int32)
-    # the sequence of a packed row (empty sequences own no row; rows past the last sequence belong
-    # to none: they count to the last one, which keeps them inside the bound, and their gradients
-    # are set to zero afterwards)
-    seq = torch.searchsorted(cu[1:].contiguous(), row, right=True).clamp_(max=num_seqs - 1)
-    dest = (padded_cu[seq] + (row - cu[seq])).long()
-    return padded_cu, dest, row < cu[-1], -(-(rows + 127 * num_seqs) // 128) * 128
-
-
-def _from_padded_packing(x: Tensor, dest: Tensor, owned: Tensor) -> Tensor:
-    """The rows of the packed layout back from the padded packing; rows of no sequence are zero."""
-    rows = x.index_select(1, dest)
-    return torch.where(owned.view(1, -1, *([1] * (x.dim() - 2))), rows, torch.zeros_like(rows))
-
-
-def _to_padded_packing(x: Tensor, dest: Tensor, padded_rows: int) -> Tensor:
-    out = x.new_zeros((x.shape[0], padded_rows) + tuple(x.shape[2:]))
-    return out.index_copy_(1, dest, x)
+        dq, dk, dv = torch_ops.attention_backward(query, key, value, out, d_out, lse.contiguous(), is_causal, scale)
+        if d_pad != head_dim:
+            dq, dk, dv = (t[..., :head_dim] for t in (dq, dk, dv))
+        return dq, dk, dv, None, None
 
 
 class AmdFmhaVarlenFunction(torch.autograd.Function):
-    """Variable-length dense attention with a backward pass.  The forward is the sequence-packed
-    kernel.  The backward kernels work on 128-row tiles that must not straddle two sequences, so
-    the backward first copies the operands into a packing whose sequences are padded to multiples
-    of 128 rows (index arithmetic on the device, no copy of the lengths to the host), runs one
-    set of launches for all sequences, and gathers the gradient rows back.  Counterpart of the
-    varlen arguments of src/natten/backends/blackwell_fmha.py:52-170."""
+    """Variable-length dense attention with a backward pass, both on the packed operands as they are: one
+    set of launches for all sequences.  Counterpart of the varlen arguments of
+    src/natten/backends/blackwell_fmha.py:52-170."""
 
     @staticmethod
     def forward(ctx, query, key, value, is_causal, scale, cu_q, cu_kv, max_q, max_kv):
@@ -198,16 +153,10 @@ class AmdFmhaVarlenFunction(torch.autograd.Function):
         if max_q == 0 or max_kv == 0 or q.shape[1] == 0 or k.shape[1] == 0:
             # no sequence has both queries and keys: the output does not depend on the operands
             return (torch.zeros_like(query), torch.zeros_like(key), torch.zeros_like(value)) + (None,) * 6
-        delta = torch_ops.compute_delta(o, do)
-        pcu_q, dest_q, owned_q, rows_q = _padded_packing(cu_q, q.shape[1])
-        pcu_kv, dest_kv, owned_kv, rows_kv = _padded_packing(cu_kv, k.shape[1])
         dq, dk, dv = torch_ops.attention_backward_varlen(
-            _to_padded_packing(q, dest_q, rows_q), _to_padded_packing(k, dest_kv, rows_kv),
-            _to_padded_packing(v, dest_kv, rows_kv), _to_padded_packing(do, dest_q, rows_q),
-            _to_padded_packing(lse, dest_q, rows_q), _to_padded_packing(delta, dest_q, rows_q),
-            cu_q.to(torch.int32).contiguous(), cu_kv.to(torch.int32).contiguous(), pcu_q, pcu_kv, max_q, max_kv,
-            is_causal, scale,
+            q, k, v, o, do, lse.contiguous(), cu_q.to(torch.int32).contiguous(), cu_kv.to(torch.int32).contiguous(), is_causal,
+            scale,
         )
-        dq = _from_padded_packing(dq, dest_q, owned_q)
-        dk, dv = _from_padded_packing(dk, dest_kv, owned_kv), _from_padded_packing(dv, dest_kv, owned_kv)
-        return (dq[..., :head_dim], dk[..., :head_dim], dv[..., :head_dim]) + (None,) * 6
+        if d_pad != head_dim:
+            dq, dk, dv = (t[..., :head_dim] for t in (dq, dk, dv))
+        return (dq, dk, dv) + (None,) * 6

@@ -134,28 +134,26 @@ def _(q, k, v, d_out, lse, delta, kernel_size, stride, dilation, is_causal, scal
 
 @torch.library.custom_op("natten_amd::attention_backward", mutates_args=(), device_types="cuda")
 def _attention_backward_op(
-    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, seqlen_q: int, seqlen_kv: int,
-    is_causal: bool, scale: float,
+    q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, is_causal: bool, scale: float,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    return _lib.attention_backward(q, k, v, d_out, lse, delta, seqlen_q, seqlen_kv, is_causal, scale)
+    return _lib.attention_backward(q, k, v, out, d_out, lse, is_causal, scale)
 
 
 @_attention_backward_op.register_fake
-def _(q, k, v, d_out, lse, delta, seqlen_q, seqlen_kv, is_causal, scale):
+def _(q, k, v, out, d_out, lse, is_causal, scale):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
 
 
 @torch.library.custom_op("natten_amd::attention_backward_varlen", mutates_args=(), device_types="cuda")
 def _attention_backward_varlen_op(
-    q: Tensor, k: Tensor, v: Tensor, d_out: Tensor, lse: Tensor, delta: Tensor, cu_q: Tensor, cu_kv: Tensor,
-    padded_cu_q: Tensor, padded_cu_kv: Tensor, max_seqlen_q: int, max_seqlen_kv: int, is_causal: bool, scale: float,
+    q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, cu_q: Tensor, cu_kv: Tensor,
+    is_causal: bool, scale: float,
 ) -> Tuple[Tensor, Tensor, Tensor]:
-    return _lib.attention_backward_varlen(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv,
-                                          max_seqlen_q, max_seqlen_kv, is_causal, scale)
+    return _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale)
 
 
 @_attention_backward_varlen_op.register_fake
-def _(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv, max_seqlen_q, max_seqlen_kv, is_causal, scale):
+def _(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale):
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
 
 
@@ -282,20 +280,16 @@ def fna_backward_fused(q, k, v, d_out, lse, delta, kernel_size, stride, dilation
                                    q_tile_shape, kv_tile_shape, kv_role_q_tile_shape, kv_role_kv_tile_shape, out=out)
 
 
-def attention_backward(q, k, v, d_out, lse, delta, seqlen_q, seqlen_kv, is_causal, scale):
+def attention_backward(q, k, v, out, d_out, lse, is_causal, scale):
     if _tracing():
-        return _attention_backward_op(q, k, v, d_out, lse, delta, int(seqlen_q), int(seqlen_kv), bool(is_causal),
-                                      float(scale))
-    return _lib.attention_backward(q, k, v, d_out, lse, delta, seqlen_q, seqlen_kv, is_causal, scale)
+        return _attention_backward_op(q, k, v, out, d_out, lse, bool(is_causal), float(scale))
+    return _lib.attention_backward(q, k, v, out, d_out, lse, is_causal, scale)
 
 
-def attention_backward_varlen(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv, max_seqlen_q,
-                              max_seqlen_kv, is_causal, scale):
+def attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale):
     if _tracing():
-        return _attention_backward_varlen_op(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv,
-                                             int(max_seqlen_q), int(max_seqlen_kv), bool(is_causal), float(scale))
-    return _lib.attention_backward_varlen(q, k, v, d_out, lse, delta, cu_q, cu_kv, padded_cu_q, padded_cu_kv,
-                                          max_seqlen_q, max_seqlen_kv, is_causal, scale)
+        return _attention_backward_varlen_op(q, k, v, out, d_out, lse, cu_q, cu_kv, bool(is_causal), float(scale))
+    return _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale)
 
 
 def token_permute(x, tile_shape, dilation, flip_tiled_dims, widen=False):

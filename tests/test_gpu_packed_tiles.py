@@ -1,0 +1,46 @@
+"""The tile walk of sequence-packed attention (backward kernels): sequence counts around the 64 that one
+step of the walk takes, empty sequences, lengths around the 128-row tile, rows in front of and behind
+the sequences.  Gradients against the float64 oracle at the tolerance of the backward tests (bf16 2e-2:
+P and dS are rounded to bf16 before the second product)."""
+
+import numpy as np
+import pytest
+import torch
+
+import natten_amd
+from oracle import na_oracle as O
+from tests.gpu_utils import assert_close, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("num_seqs,head,tail", [(1, 0, 5), (63, 3, 0), (64, 0, 0), (65, 130, 257), (130, 1, 1)])
+def test_every_row_is_covered_once(num_seqs, head, tail):
+    rng = np.random.default_rng(num_seqs)
+    lens = rng.choice([0, 1, 5, 63, 64, 127, 128, 129], size=num_seqs)
+    lens[0], lens[-1] = 129, 128
+    cu_list = head + np.concatenate([[0], np.cumsum(lens)])
+    total = int(cu_list[-1]) + tail
+    gen = torch.Generator().manual_seed(num_seqs)
+    q, d_out = (torch.randn((1, total, 2, 32), generator=gen).bfloat16().cuda() for _ in range(2))
+    k, v = (torch.randn((1, total, 1, 32), generator=gen).bfloat16().cuda() for _ in range(2))
+    cu = torch.tensor(cu_list, dtype=torch.int32, device="cuda")
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    causal = num_seqs % 2 == 1
+    out = natten_amd.attention(q, k, v, is_causal=causal, cumulative_seqlen_Q=cu, cumulative_seqlen_KV=cu, max_seqlen_Q=129,
+                               max_seqlen_KV=129)
+    out.backward(d_out)
+    grads = [to_np(t.grad) for t in (q, k, v)]
+    owned = np.zeros(total, dtype=bool)
+    for a, b in zip(cu_list[:-1], cu_list[1:]):
+        owned[a:b] = True
+    for g in grads + [to_np(out)]:
+        assert np.isfinite(g).all() and not g[:, ~owned].any()
+    for i in list(range(min(num_seqs, 8))) + list(range(max(num_seqs - 8, 0), num_seqs)):
+        a, b = int(cu_list[i]), int(cu_list[i + 1])
+        if a == b:
+            continue
+        ref = O.attention_backward(*(to_np(t[:, a:b]) for t in (q, k, v, d_out)), is_causal=causal)
+        for name, g, r in zip(("dq", "dk", "dv"), grads, ref):
+            assert_close(f"{name} of sequence {i} of {num_seqs}, {b - a} rows", g[:, a:b], r, atol=2e-2, rtol=2e-2)
