@@ -309,20 +309,21 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
 /*
  * What the backward entry points take besides the operands, in one pass: from q, out, d_out
  * [batch, tokens, heads, head_dim] and lse [batch, tokens, heads] (the forward's) it writes q_scaled
- * (q's shape: the logit operand described below), delta = rowsum(out * d_out) and a copy of lse, both
- * head-major [batch, heads, tokens] float32.  natten_amd_fna_backward_fused then takes `roles` + 4.
+ * (q's shape: the logit operand described below), neg_delta = -rowsum(out * d_out) and neg_lse2 =
+ * -log2(e) lse, both head-major [batch, heads, tokens] float32: what the kernels' accumulators start
+ * from.  natten_amd_fna_backward_fused then takes `roles` + 4.
  */
 int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse,
-                                void* q_scaled, float* delta, float* lse_heads, int dtype, int batch,
+                                void* q_scaled, float* neg_delta, float* neg_lse2, int dtype, int batch,
                                 int tokens, int heads, int head_dim, float scale, void* stream);
 
 /*
  * Fused neighborhood attention backward on token-permuted operands.
  *   q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv [batch, seqlen_kv, heads_kv,
  *   head_dim], permuted like the forward operands (dimension 0 fastest inside a tile, dilation
- *   groups folded into batch); lse, delta float32, permuted the same way and then stored
+ *   groups folded into batch); neg_lse2, neg_delta float32, permuted the same way and then stored
  *   head-major, [batch, heads_q, seqlen_q] (the kernels read 64 consecutive rows of one head at
- *   a time); lse from the forward pass (natural log), delta from natten_amd_compute_delta.
+ *   a time): -log2(e) times the forward's lse, minus natten_amd_compute_delta's result.
  *   Both tile shapes must hold 128 tokens and their last extent above 1 must be even; q_shape /
  *   kv_shape are the padded per-group layouts (multiples of the tiles), seqlen = their product.
  * dq, dk, dv are written completely (padding rows get zeros); nothing is accumulated through
@@ -340,7 +341,7 @@ int natten_amd_backward_prepare(const void* q, const void* out, const void* d_ou
  * afterwards); it must not be q.  May be null for a call that only makes the dq launch.
  */
 int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out,
-                            const float* lse, const float* delta, void* dq, void* dk, void* dv,
+                            const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv,
                             void* q_scaled, int dtype, int na_dim, int batch, int seqlen_q, int seqlen_kv,
                             int heads_q, int heads_kv, int head_dim, const int32_t* q_shape,
                             const int32_t* kv_shape, const int32_t* qkv_shape,
@@ -351,7 +352,7 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
 
 /*
  * The same backward on the original tensors: q, d_out, dq [batch, *qkv_shape, heads_q, head_dim],
- * k, v, dk, dv [batch, *qkv_shape, heads_kv, head_dim], lse and delta head-major
+ * k, v, dk, dv [batch, *qkv_shape, heads_kv, head_dim], neg_lse2 and neg_delta head-major
  * [batch, heads_q, prod(qkv_shape)].  The kernels gather and scatter the rows of their tiles
  * themselves, which replaces the six token permutes and three unpermutes of the reference's
  * backward driver (src/natten/backends/blackwell_fna.py:205-297).  Where every extent is a
@@ -370,7 +371,7 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
  * (a caller makes one call per role, each with that role's shapes).
  */
 int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out,
-                                  const float* lse, const float* delta, void* dq, void* dk,
+                                  const float* neg_lse2, const float* neg_delta, void* dq, void* dk,
                                   void* dv, void* q_scaled, int dtype, int na_dim, int batch, int heads_q,
                                   int heads_kv, int head_dim, const int32_t* qkv_shape,
                                   const int32_t* kernel_size, const int32_t* stride,
@@ -380,12 +381,12 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
 
 /*
  * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
- * [batch, seqlen_kv, heads_kv, head_dim]; lse, delta head-major [batch, heads_q, seqlen_q].
+ * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2, neg_delta head-major [batch, heads_q, seqlen_q].
  * q_scaled as above; q_scaled_filled != 0: it is filled already (natten_amd_backward_prepare).
  * Any sequence lengths: rows past the end of a sequence are gathered from its last row and masked.
  */
 int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out,
-                                  const float* lse, const float* delta, void* dq, void* dk,
+                                  const float* neg_lse2, const float* neg_delta, void* dq, void* dk,
                                   void* dv, void* q_scaled, int q_scaled_filled, int dtype, int batch,
                                   int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
                                   int is_causal, float scale, void* stream);
@@ -393,7 +394,7 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
 /*
  * Dense attention backward of a sequence-packed batch, one set of launches for all sequences.
  * The operands hold the `num_seqs` sequences back to back: q, d_out, dq [1, rows_q, heads_q,
- * head_dim], k, v, dk, dv [1, rows_kv, heads_kv, head_dim], lse and delta head-major
+ * head_dim], k, v, dk, dv [1, rows_kv, heads_kv, head_dim], neg_lse2 and neg_delta head-major
  * [1, heads_q, rows_q].  Both cumulative arrays are device int32 [num_seqs + 1]: sequence b owns
  * rows cu_seqlens_q[b] .. cu_seqlens_q[b+1] - 1 of the queries, keys likewise.  dq, dk and dv are
  * written completely: rows of no sequence get zeros, and so do the rows of a sequence whose
@@ -401,7 +402,7 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
  * No host synchronisation.
  */
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v,
-                                         const void* d_out, const float* lse, const float* delta,
+                                         const void* d_out, const float* neg_lse2, const float* neg_delta,
                                          void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
                                          int dtype, int num_seqs, int rows_q, int rows_kv,
                                          const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,

@@ -545,8 +545,8 @@ def compute_delta(out: Tensor, d_out: Tensor) -> Tensor:
 
 
 def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: float, q_scaled: Tensor) -> Tuple[Tensor, Tensor]:
-    """q, out, d_out [B, *X, H, D], lse [B, *X, H] -> head-major float32 [B, H, prod(X)] delta =
-    rowsum(out * d_out) and lse; fills q_scaled (like q) with the logit operand of the dk / dv launch."""
+    """q, out, d_out [B, *X, H, D], lse [B, *X, H] -> head-major float32 [B, H, prod(X)] -rowsum(out * d_out)
+    and -log2(e) lse; fills q_scaled (like q) with the logit operand of the dk / dv launch."""
     _require_gpu(q, out, d_out, lse, q_scaled)
     if out.dtype != q.dtype or d_out.dtype != q.dtype or out.shape != q.shape or d_out.shape != q.shape:
         raise ValueError("out and d_out must be of q's shape and dtype.")
@@ -554,14 +554,22 @@ def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: 
         raise ValueError("lse must be float32 of q's shape without the last dimension.")
     B, H = q.shape[0], q.shape[-2]
     tokens = lse.numel() // (B * H)
-    delta, lse_heads = torch.empty((2, B, H, tokens), dtype=torch.float32, device=q.device)
+    neg_delta, neg_lse2 = torch.empty((2, B, H, tokens), dtype=torch.float32, device=q.device)
     with _on_device(q):
         rc = lib().natten_amd_backward_prepare(
-            q.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), q_scaled.data_ptr(), delta.data_ptr(),
-            lse_heads.data_ptr(), DTYPE_CODES[q.dtype], B, tokens, H, q.shape[-1], float(scale), _stream(q),
+            q.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), q_scaled.data_ptr(), neg_delta.data_ptr(),
+            neg_lse2.data_ptr(), DTYPE_CODES[q.dtype], B, tokens, H, q.shape[-1], float(scale), _stream(q),
         )
     _check(rc)
-    return delta, lse_heads
+    return neg_delta, neg_lse2
+
+
+def _head_major(lse: Tensor, delta: Tensor) -> Tuple[Tensor, Tensor]:
+    """lse, delta [B, *X, H] as the backward kernels take them: -log2(e) lse and -delta, [B, H, prod(X)]."""
+    if lse.dtype != torch.float32 or delta.dtype != torch.float32:
+        raise ValueError("lse and delta must be float32.")
+    B, H = lse.shape[0], lse.shape[-1]
+    return tuple((t.reshape(B, -1, H).transpose(1, 2) * c).contiguous() for t, c in ((lse, -1.4426950408889634), (delta, -1.0)))
 
 
 def fna_backward(
@@ -571,17 +579,15 @@ def fna_backward(
     """Backward on token-permuted operands (128-token tiles on both sides) -> (dq, dk, dv).
     lse, delta: [batch, seqlen_q, heads_q] as the permute gives them; the kernels take them head-major."""
     L = lib()
-    lse, delta = lse.transpose(1, 2).contiguous(), delta.transpose(1, 2).contiguous()
-    _require_gpu(q, k, v, d_out, lse, delta)
+    neg_lse2, neg_delta = _head_major(lse, delta)
+    _require_gpu(q, k, v, d_out, neg_lse2, neg_delta)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd fna_backward does not support {q.dtype}.")
-    if lse.dtype != torch.float32 or delta.dtype != torch.float32:
-        raise ValueError("lse and delta must be float32.")
     na_dim = len(kernel_size)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     with _on_device(q):
         rc = L.natten_amd_fna_backward(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, q.shape[0], q.shape[1],
             k.shape[1], q.shape[2], k.shape[2], q.shape[3], _i32(q_shape), _i32(kv_shape), _i32(qkv_shape),
             _i32(kernel_size), _i32(stride), _i32(dilation), _i32([1 if c else 0 for c in is_causal]),
@@ -623,13 +629,10 @@ def fna_backward_fused(
         raise ValueError("kv_role_q_tile_shape and kv_role_kv_tile_shape must be given together.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     if out is not None:
-        delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
+        neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
     else:
-        lse = lse.reshape(B, -1, H).transpose(1, 2).contiguous()
-        delta = delta.reshape(B, -1, H).transpose(1, 2).contiguous()
-    _require_gpu(q, k, v, d_out, lse, delta)
-    if lse.dtype != torch.float32 or delta.dtype != torch.float32:
-        raise ValueError("lse and delta must be float32.")
+        neg_lse2, neg_delta = _head_major(lse, delta)
+    _require_gpu(q, k, v, d_out, neg_lse2, neg_delta)
     filled = 4 if out is not None else 0
     same = kv_role_q_tile_shape is None or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
@@ -641,7 +644,7 @@ def fna_backward_fused(
     with _on_device(q):
         for roles, qt, kt in launches:
             rc = L.natten_amd_fna_backward_fused(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2],
                 q.shape[-1], _i32(q.shape[1 : 1 + na_dim]), _i32(kernel_size), _i32(stride), _i32(dilation),
                 _i32([1 if c else 0 for c in is_causal]), _i32(qt), _i32(kt), float(scale), roles, _stream(q),
@@ -659,10 +662,10 @@ def attention_backward(
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_backward does not support {q.dtype}.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
     with _on_device(q):
         rc = L.natten_amd_attention_backward(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], q.shape[0], q.shape[1],
             k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
         )
@@ -686,10 +689,10 @@ def attention_backward_varlen(
     if cu_q.numel() < 2 or q.shape[0] != 1 or k.shape[0] != 1:
         raise ValueError("sequence-packed operands have batch 1 and at least one sequence.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
     with _on_device(q):
         rc = L.natten_amd_attention_backward_varlen(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], cu_q.numel() - 1, q.shape[1],
             k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,
             float(scale), _stream(q),

@@ -7,7 +7,8 @@
 //   dKV, paired role : stationary = keys    (operands K, V; results dK and dV), streamed = queries (Q, dO)
 // Per streamed tile, with Y1/Y2 the streamed and X1/X2 the stationary operands:
 //   S^T  = Y1 X1^T,  dP^T = Y2 X2^T                     (32x32x16 MFMA, the lane owns a stationary row)
-//   P    = exp2(S - log2e LSE) on unmasked pairs, 0 elsewhere;  dS = P (dP - delta)
+//   P    = exp2(S - log2e LSE) on unmasked pairs, 0 elsewhere;  dS = P (dP - delta)   (both differences
+//          are the products' accumulator inputs)
 //   acc1^T += Y1^T dS^T   (dQ = scale * sum_k dS k  /  dK = ln 2 * sum_q dS q')
 // The logits are formed from the same operand as in the forward kernel, q' = round(q * scale *
 // log2(e)) in the operand type, so that S is the forward's logit to the last bit of its operands
@@ -25,6 +26,15 @@
 // and forms dS and dK.  LSE and delta = rowsum(dO * O) belong to the
 // query: per-lane scalars in the dQ role, a small per-tile LDS table in the others.  Nothing
 // is accumulated through memory, so the results are deterministic.
+//
+// What bounds it is the instruction issue of two waves per SIMD next to the matrix pipe: per wave and tile of
+// head dim 128 the paired role's P waves issue 49 vector instructions and 32 exponentials beside 32
+// matrix instructions (115 under the mask), its dS waves 66.  That took: products that start from
+// -log2e LSE and -delta (no subtraction per pair), the mask as one bit per pair (two instructions
+// where the comparison of packed coordinates took five), dS from the half-precision probabilities by
+// mixed multiply-adds, tile descriptors formed 64 at a time.  Before it the counts were 82 / 244 / 131 and
+// the dK / dV launch took 25.2 ms on 29 x 46 x 78 tokens, window 9 x 24 x 24, H 24 (now 20.7), 569 us on
+// 128 x 128, window 32 x 32, stride 16, H 16 (433); head dim 32, 4 x 56 x 56, window 7 x 7, H 8: 59 (43).
 //
 // What it restates (not the code): SHI-Labs/NATTEN
 //   csrc/include/natten/cuda/reference/fna_reference_backward.hpp:60-150, :165-265, :282-380
@@ -45,8 +55,10 @@ struct FnaBwdParams {
   const void* k;      // [batch, seqlen_kv, heads_kv, D]
   const void* v;
   const void* d_out;  // like q
-  const float* lse;   // [batch, heads_q, seqlen_q] (head-major: a tile's values are contiguous), natural log
-  const float* delta; // [batch, heads_q, seqlen_q], rowsum(d_out * out)
+  // [batch, heads_q, seqlen_q] (head-major: a tile's values are contiguous), as the kernels' accumulators
+  // start from them: -log2(e) LSE and -rowsum(d_out * out)
+  const float* neg_lse2;
+  const float* neg_delta;
   void* dq;
   void* dk;
   void* dv;
@@ -118,15 +130,37 @@ inline void set_bwd_divisions(FnaBwdParams& p) {
   p.d_heads_kv = na_make_div(p.heads_kv);
 }
 
+// Stores a lane's row of a transposed result (32 DB columns; register 4 j + i of block db is column
+// 32 db + 8 j + 4 g + i): the lanes of a row's two wave halves trade four columns of every sixteen, so
+// that each stores sixteen bytes at a time.
+template <typename T, int DB>
+static __device__ __forceinline__ void store_row_blocks(T* orow, const f32x16_t (&acc)[DB], float mul, int g, bool valid) {
+  using vec2 = typename Mma<T>::vec2;
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int j = 0; j < 4; j += 2) {
+      uint32_t w[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * (j + i / 2) + 2 * (i % 2);
+        const vec2 v = {static_cast<T>(acc[db][r] * mul), static_cast<T>(acc[db][r + 1] * mul)};
+        w[i] = __builtin_bit_cast(uint32_t, v);
+      }
+      asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
+                   : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
+      if (valid) *reinterpret_cast<u32x4_t*>(orow + db * 32 + 8 * (j + g)) = u32x4_t{w[0], w[1], w[2], w[3]};
+    }
+}
+
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 
 // Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to):
-// what each instance's registers allow without spilling (head dim 128: 212 and 254; 64: 230 and 167;
-// 32: 153 and 122 of the SIMD's 512 per lane).  With two waves throughout, head dim 32 on 4 x 56 x 56
-// tokens, 7 x 7 windows took 82 (dK, dV) and 52 us (dQ); with three and four 59 and 39 us (the set-up
-// without divisions included).
+// what each instance's registers allow without spilling (head dim 128: 222 and 256 of the SIMD's 512 per
+// lane; 64: 229 and 210; 32: 168 and 167).  Head dim 32 on 4 x 56 x 56 tokens, 7 x 7 windows with two
+// waves throughout: 82 (dK, dV) and 52 us (dQ).
 constexpr int bwd_waves_per_simd(int head_dim, int role) {
-  return head_dim == 128 ? 2 : head_dim == 64 ? (role == kBwdDQ ? 3 : 2) : (role == kBwdDQ ? 4 : 3);
+  return head_dim == 128 ? 2 : head_dim == 64 ? 2 : 3;
 }
 
 // RAGGED: dense attention whose sequences end inside a tile, packed ones among them.  Rows past the end
@@ -174,8 +208,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   static_assert(!PAIR || D == 128, "the paired role is for head dim 128 (smaller ones fit the combined role)");
   __shared__ __attribute__((aligned(1024))) char sY1[NS1 * TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char sY2[NS * TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) uint32_t sTabA[NS1 * BT];
-  __shared__ __attribute__((aligned(16))) uint32_t sTabB[NS1 * BT];
+  // sRows[a][g][x]: the rows of a streamed tile whose coordinate along dimension a is >= x, one bit per
+  // row: the 32 bits that the lanes of wave half g hold logits for (as sKeys of the forward kernel)
+  __shared__ __attribute__((aligned(16))) uint32_t sRows[3][2][BT + 1];
   __shared__ __attribute__((aligned(16))) float sLse[NS1 * BT];
   __shared__ __attribute__((aligned(16))) float sDelta[NS1 * BT];
   __shared__ __attribute__((aligned(16))) float sSpare[BT];
@@ -380,19 +415,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   const int64_t b_stride = int64_t(heads_b) * D;
   const float kLog2e = 1.4426950408889634f;
 
-  typedef T tx4 __attribute__((ext_vector_type(4)));
   auto store_rows = [&](void* dst, const f32x16_t (&acc)[DB], float mul) {
-    if (!a_valid) return;
     T* orow = reinterpret_cast<T*>(dst) + a_row * a_stride + int64_t(head_a) * D;
-#pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        tx4 o4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o4[i] = static_cast<T>(acc[db][4 * j + i] * mul);
-        *reinterpret_cast<tx4*>(orow + db * 32 + 8 * j + 4 * g) = o4;
-      }
+    store_row_blocks<T, DB>(orow, acc, mul, g, a_valid);
   };
   auto store_results = [&](const f32x16_t (&a1)[DB], const f32x16_t (&a2)[DB], float scale1) {
     if constexpr (ROLE == kBwdDQ) store_rows(p.dq, a1, scale1);
@@ -430,30 +455,51 @@ fna_bwd_kernel(const FnaBwdParams p) {
     if constexpr (HAS_DS) x2f[ks] = *reinterpret_cast<const vec8*>(x2 + ks * 16);
   }
 
-  // mask state of the lane
-  int wst[3] = {0, 0, 0}, wen[3] = {0, 0, 0};  // dQ role: window of the lane's query
-  uint32_t key_packed = 0;                     // other roles: in-tile coordinates of the lane's key
+  // Mask state of the lane: along every dimension the streamed rows that pair with its stationary row are
+  // an interval (the window of a query; the queries whose windows hold a key), so that the pairs of
+  // a tile are the AND of two rows of sRows per dimension.
+  int win_lo[3], win_hi[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int c = a_crd[a];
+    const bool cs = p.causal[a] != 0;
+    if constexpr (!KV_STATIONARY) {
+      win_lo[a] = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
+      win_hi[a] = na_window_end(c, win_lo[a], ksz[a], extent[a], cs);
+    } else {
+      win_lo[a] = na_first_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs);
+      win_hi[a] = na_last_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs) + 1;
+      if (c >= extent[a]) win_hi[a] = win_lo[a];  // a padding key of a permuted sequence: nothing attends it
+    }
+  }
+  if (wave < 3) {
+    // one row per lane and, by wave, one dimension (the row past the extent holds nothing)
+    const int lg_stride = wave == 0 ? 0 : wave == 1 ? b_sub_lg[0] : b_sub_lg[0] + b_sub_lg[1];
+    const int lg = wave == 0 ? b_sub_lg[0] : wave == 1 ? b_sub_lg[1] : b_sub_lg[2];
+    const uint64_t rows = na_keys_at_or_after(na_min(lane, 1 << lg), lg_stride, lg);
+    sRows[wave][0][lane] = na_lane_half_bits(rows, 0);
+    sRows[wave][1][lane] = na_lane_half_bits(rows, 1);
+    if (lane == 0) sRows[wave][0][BT] = sRows[wave][1][BT] = 0;
+  }
+  // Accumulator inputs of the first matrix instruction of a logit / dP block: -log2e LSE and -delta of
+  // the block's queries, so that P = exp2(S) and dS = P dP are what the matrix pipe returns.  In the
+  // key-stationary roles they differ by row and come from the tile's table in LDS; in the dQ role they
+  // are the lane's own, sixteen copies of them where the registers allow (head dims below 128).
+  constexpr bool INIT_REGS = !KV_STATIONARY && D < 128;
   float lse_l = 0.f, delta_l = 0.f;
   if constexpr (!KV_STATIONARY) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const int c = a_crd[a];
-      wst[a] = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
-      wen[a] = na_window_end(c, wst[a], ksz[a], extent[a], p.causal[a] != 0);
-    }
     const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
                                      : stat_row_q + head_a * stat_head_stride + a_seq_row;
-    lse_l = p.lse[stat_idx] * kLog2e;
-    delta_l = p.delta[stat_idx];
-    // in-tile coordinates of every streamed position, packed in 10-bit fields
-    for (int i = tid; i < BT; i += NT) {
-      const int t0 = i & (b_sub[0] - 1);
-      const int t1 = (i >> b_sub_lg[0]) & (b_sub[1] - 1);
-      const int t2 = i >> (b_sub_lg[0] + b_sub_lg[1]);
-      sTabA[i] = uint32_t(t0) | (uint32_t(t1) << 10) | (uint32_t(t2) << 20);
+    lse_l = p.neg_lse2[stat_idx];
+    delta_l = p.neg_delta[stat_idx];
+  }
+  f32x16_t lse_init, delta_init;
+  if constexpr (INIT_REGS) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      lse_init[r] = lse_l;
+      delta_init[r] = delta_l;
     }
-  } else {
-    key_packed = uint32_t(a_off[0]) | (uint32_t(a_off[1]) << 10) | (uint32_t(a_off[2]) << 20);
   }
 
   // ---- streamed tiles ---------------------------------------------------------------------------
@@ -476,112 +522,106 @@ fna_bwd_kernel(const FnaBwdParams p) {
     off_u[i] = uint32_t(sub_pos(row)) * uint32_t(b_stride * 2) + uint32_t(L::u_slot(row, slot) * 16);
   }
 
+  // The streamed tiles in visiting order: the box of tiles the stationary tile meets, dimension 2 fastest,
+  // dimension 0 slowest; the key-stationary roles walk it once per query head of the key head's group.
+  // First the tiles that need the element mask (the box minus the inner box of whole tiles, see
+  // full_t0), then the whole ones: one sequence, but each kind has a loop body of its own.
+  // Descriptors are formed 64 box positions at a time, one per lane, and read back by lane number: a
+  // tile costs the wave a handful of scalar instructions (a scalar walk of the box with its edge cases
+  // took some seventy, every one an issue slot of a wave that also feeds the matrix pipe).
   struct Tile {
-    int origin[3];  // coordinate of the tile's first token (a tile moved back from the group's edge: of the first one gathered)
-    int lead[3];    // ... whose first lead[a] positions along dimension a belong to the tile before it
-    int row0;       // its first row in the streamed side's permuted sequence
+    int row0;       // its first row in the streamed side's sequence / its token in the dilation group's batch entry
     int head_b;
+    int origin[3];  // coordinate of its first row (a tile moved back from the group's edge: of the first one gathered)
+    int lead;       // ... whose first (lead >> 8 a) & 255 positions along dimension a belong to the tile before it
   };
-  // The streamed tiles in visiting order: dimension 2 fastest, dimension 0 slowest; the
-  // key-stationary roles walk the box once per query head of the key head's group.  The box is
-  // walked twice: first the tiles that need the element mask (the box minus the inner box of
-  // whole tiles, see full_t0), then the whole ones (the inner box itself).
   const int total = box_n[0] * box_n[1] * box_n[2];
+  const int heads_walked = KV_STATIONARY ? rep : 1;
   const int n_whole = (full_t1[0] - full_t0[0]) * (full_t1[1] - full_t0[1]) * (full_t1[2] - full_t0[2]);
+  const int n_masked = (total - n_whole) * heads_walked;  // the first n_masked of the n_iter tiles need the mask
+  const int n_iter = total * heads_walked;
   const int head_b0 = KV_STATIONARY ? head_a * rep : na_div(head_a, p.d_rep);
-  int wc[3], walk_head = 0;  // position of the walk in absolute tile coordinates
-  // one step inside the box of the pass (WHOLE: the inner box, else the whole box)
-  auto step = [&](auto whole_tag) {
-    constexpr bool WHOLE = decltype(whole_tag)::value;
-    auto lo = [&](int a) { return WHOLE ? full_t0[a] : box_tile0[a]; };
-    auto hi = [&](int a) { return WHOLE ? full_t1[a] : box_tile0[a] + box_n[a]; };
-    if (++wc[2] == hi(2)) {
-      wc[2] = lo(2);
-      if (++wc[1] == hi(1)) {
-        wc[1] = lo(1);
-        if (++wc[0] == hi(0)) {
-          wc[0] = lo(0);
-          ++walk_head;
-        }
+  const float inv_n1 = 1.f / float(box_n[1]), inv_n2 = 1.f / float(box_n[2]);
+  int walk = -64, walk_head = -1;  // first of the 64 positions described, query head of the group
+  bool walk_whole = n_masked == 0;
+  int r_row0 = 0, r_origin[3] = {0, 0, 0}, r_lead = 0;
+  uint64_t whole_bits = 0, todo = 0;  // of the positions described: the whole tiles, the tiles still to visit
+  auto load_descriptors = [&]() __attribute__((always_inline)) {
+    // quotient by a rounded reciprocal, then put right (positions are far below 2^24)
+    auto divide = [](int n, int d, float inv, int& rem) __attribute__((always_inline)) {
+      int q = int(float(n) * inv);
+      rem = n - q * d;
+      if (rem < 0) {
+        --q;
+        rem += d;
+      } else if (rem >= d) {
+        ++q;
+        rem -= d;
       }
-    }
-  };
-  // masked pass: a position at the start of a run of whole tiles jumps to the run's end
-  auto skip_whole = [&]() {
-    while (n_whole > 0 && wc[2] == full_t0[2] && wc[1] >= full_t0[1] && wc[1] < full_t1[1] && wc[0] >= full_t0[0] &&
-           wc[0] < full_t1[0]) {
-      wc[2] = full_t1[2] - 1;
-      step(std::false_type{});
-    }
-  };
-  auto start_walk = [&](auto whole_tag) {
-    constexpr bool WHOLE = decltype(whole_tag)::value;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) wc[a] = WHOLE ? full_t0[a] : box_tile0[a];
-    walk_head = 0;
-    if constexpr (!WHOLE) skip_whole();
-  };
-  // descriptor of the current position, then on to the next one; `more` = tiles of this pass still
-  // to come after this one (past the last one the position is never used)
-  auto next_tile = [&](auto whole_tag, bool more) {
-    constexpr bool WHOLE = decltype(whole_tag)::value;
-    Tile t;
+      return q;
+    };
+    int t[3];
+    const int rest = divide(na_min(walk + lane, total - 1), box_n[2], inv_n2, t[2]);
+    t[0] = divide(rest, box_n[1], inv_n1, t[1]);
+    bool whole = true;
     int cc[3], half = 0;
+    r_lead = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      t.origin[a] = wc[a] << b_sub_lg[a];
-      t.lead[a] = 0;
-      if (p.edge) {
-        const int moved = na_min(t.origin[a], (KV_STATIONARY ? q_extent[a] : extent[a]) - b_sub[a]);
-        t.lead[a] = t.origin[a] - moved;
-        t.origin[a] = moved;
-      }
+      t[a] += box_tile0[a];
+      whole = whole && t[a] >= full_t0[a] && t[a] < full_t1[a];
+      const int org = t[a] << b_sub_lg[a];
+      r_origin[a] = p.edge ? na_min(org, (KV_STATIONARY ? q_extent[a] : extent[a]) - b_sub[a]) : org;
+      r_lead |= (org - r_origin[a]) << (8 * a);
       const bool split = (a == split_dim);
-      half |= split ? (wc[a] & 1) : 0;
-      cc[a] = split ? (wc[a] >> 1) : wc[a];
+      half |= split ? (t[a] & 1) : 0;
+      cc[a] = split ? (t[a] >> 1) : t[a];
     }
-    t.row0 = p.fused ? group_tok + t.origin[0] * tok_step[0] + t.origin[1] * tok_step[1] + t.origin[2] * tok_step[2]
+    r_row0 = p.fused ? group_tok + r_origin[0] * tok_step[0] + r_origin[1] * tok_step[1] + r_origin[2] * tok_step[2]
                      : (cc[0] + b_tiled[0] * (cc[1] + b_tiled[1] * cc[2])) * AT + half * BT;
-    t.head_b = KV_STATIONARY ? head_b0 + walk_head : head_b0;
-    if (more) {
-      step(whole_tag);
-      if constexpr (!WHOLE) skip_whole();
+    whole_bits = __ballot(whole);
+  };
+  auto next_tile = [&]() __attribute__((always_inline)) {
+    while (todo == 0) {  // (called while tiles remain: some position ahead has one)
+      walk += 64;
+      if (walk_head < 0 || walk >= total) {
+        walk = 0;
+        if (++walk_head == heads_walked) {
+          walk_head = 0;
+          walk_whole = true;
+        }
+        if (total > 64 || whole_bits == 0) load_descriptors();
+      } else {
+        load_descriptors();
+      }
+      todo = walk_whole ? whole_bits : ~whole_bits;
+      if (total - walk < 64) todo &= (uint64_t(1) << (total - walk)) - 1;
     }
+    const int l = __builtin_ctzll(todo);
+    todo &= todo - 1;
+    Tile t;
+    t.row0 = __builtin_amdgcn_readlane(r_row0, l);
+    t.head_b = head_b0 + walk_head;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) t.origin[a] = __builtin_amdgcn_readlane(r_origin[a], l);
+    t.lead = __builtin_amdgcn_readlane(r_lead, l);
     return t;
   };
-
-  // in-tile coordinates of streamed position `lane` (the window tables below are built by wave 0)
-  int qo[3];
-  qo[0] = lane & (b_sub[0] - 1);
-  qo[1] = (lane >> b_sub_lg[0]) & (b_sub[1] - 1);
-  qo[2] = lane >> (b_sub_lg[0] + b_sub_lg[1]);
+  // bit 16 sb + r: the lane's logit r of sub-block sb belongs to an attended pair
+  auto pair_bits = [&](const Tile& t) __attribute__((always_inline)) {
+    uint32_t from[3], upto[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const int lead = (t.lead >> (8 * a)) & 255;
+      from[a] = sRows[a][g][na_min(na_max(win_lo[a] - t.origin[a], lead), b_sub[a])];
+      upto[a] = sRows[a][g][na_min(na_max(win_hi[a] - t.origin[a], 0), b_sub[a])];
+    }
+    return from[0] & ~upto[0] & from[1] & ~upto[1] & from[2] & ~upto[2];
+  };
 
   const uint32_t lds_y1 = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sY1))));
   const uint32_t lds_y2 = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sY2))));
   const uint32_t stat_off = uint32_t(sub_pos(lane)) * 4u;  // byte offset of streamed row `lane` in lse / delta (head-major)
-  // the window tables of a masked streamed tile (key-stationary roles, wave 0)
-  auto build_tables = [&](const Tile& t, int stage, bool masked) {
-    if constexpr (KV_STATIONARY) {
-      if (wave == 0 && masked) {
-        // per streamed query: its window relative to this workgroup's key tile
-        uint32_t addc = 0, subc = 0;
-        bool valid = true;
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int qc = t.origin[a] + qo[a];
-          valid = valid && (qc < q_extent[a]) && (qo[a] >= t.lead[a]);
-          const int st = na_window_start(qc, ksz[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
-          const int en = na_window_end(qc, st, ksz[a], extent[a], p.causal[a] != 0);
-          const int lo = na_min(na_max(st - a_first[a], 0), a_tile[a]);
-          const int hi = na_min(na_max(en - a_first[a], 0), a_tile[a]);
-          addc |= uint32_t(512 - lo) << (10 * a);
-          subc |= uint32_t(511 + hi) << (10 * a);
-        }
-        sTabA[stage * BT + lane] = valid ? addc : 0u;  // no guard bit survives a zero addend
-        sTabB[stage * BT + lane] = valid ? subc : 0u;
-      }
-    }
-  };
   // the asynchronous copies of a streamed tile (and of its LSE / delta values) into a stage
   auto issue_copies = [&](const Tile& t, int stage, int stage2) {
     const int64_t row = p.fused ? batch_row0 + t.row0 : seq_row_b + t.row0;
@@ -594,7 +634,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       // spare row so that every wave counts the same number of outstanding copies per tile)
       const int64_t stat_row0 = p.fused ? (int64_t(b_orig) * p.heads_q + t.head_b) * p.tokens + t.row0
                                         : stat_row_q + t.head_b * stat_head_stride + t.row0;
-      const float* src = (wave == 2 ? p.delta : p.lse) + stat_row0;
+      const float* src = (wave == 2 ? p.neg_delta : p.neg_lse2) + stat_row0;
       float* dst = (wave == 1) ? &sLse[stage * BT] : (wave == 2) ? &sDelta[stage * BT] : &sSpare[0];
       const uint32_t off = partial ? uint32_t(na_min(lane, last)) * 4u : stat_off;
       if (wave != 0) async_copy4_asm(src, off, lds_address(dst));
@@ -613,11 +653,6 @@ fna_bwd_kernel(const FnaBwdParams p) {
       async_copy16_uniform(y2, off, lds_y2 + dst2 + uint32_t(i * NT * 16));
     }
   };
-  auto issue = [&](const Tile& t, int stage, bool masked) {
-    build_tables(t, stage, masked);
-    issue_copies(t, stage, stage);
-  };
-
   // lane-constant LDS read offsets (same fragment layouts as the forward kernel)
   int k_off[KSTEPS];
 #pragma unroll
@@ -658,7 +693,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // of sub-block 0), so that the wave's vector work runs while the matrix pipe does.
   constexpr bool SPREAD = PAIR;
   static_assert(!SPREAD || (NP == 8 && NC == 8), "two of a sub-block's 16 probabilities per slot");
-  auto tile_body = [&](auto masked_tag, int stage, int stage2, uint32_t addc, uint32_t subc, int exch, auto&& after_slot) __attribute__((always_inline)) {
+  auto tile_body = [&](auto masked_tag, int stage, int stage2, uint32_t bits, int exch, auto&& after_slot) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
     (void)exch;  // paired role: which of the two probability buffers this tile writes
     const char* y1 = sY1 + stage * TILE_BYTES;
@@ -693,46 +728,37 @@ fna_bwd_kernel(const FnaBwdParams p) {
 
     f32x16_t S[NSB], dP[NSB];
     vec8 pf[NSB][2], dsf[NSB][2];
-    // tables of the streamed rows, four rows (8*jj + 4*g + i of a sub-block) at a time, read
-    // when they are needed (the other wave covers the wait)
-    u32x4_t ta, tb;
-    f32x4_t ls4, dl4;
-    auto load_group = [&](auto gi_tag) {
-      constexpr int gi = decltype(gi_tag)::value;  // sub-block * 4 + jj
-      if constexpr (gi < 2 * 4) {
-        const int e0 = (gi / 4) * 32 + 8 * (gi % 4) + 4 * g;
-        if constexpr (KV_STATIONARY) {
-          if constexpr (MASKED) {
-            ta = *reinterpret_cast<const u32x4_t*>(&sTabA[stage * BT + e0]);
-            tb = *reinterpret_cast<const u32x4_t*>(&sTabB[stage * BT + e0]);
-          }
-          ls4 = *reinterpret_cast<const f32x4_t*>(&sLse[stage * BT + e0]) * kLog2e;
-          if constexpr (HAS_DS) dl4 = *reinterpret_cast<const f32x4_t*>(&sDelta[stage * BT + e0]);
-        } else if constexpr (MASKED) {
-          ta = *reinterpret_cast<const u32x4_t*>(&sTabA[e0]);
-        }
+    // the rows 8*jj + 4*g + i of sub-block sb (logit r = 4 jj + i) of a per-row table
+    auto init_from = [&](const float* table, int sb) __attribute__((always_inline)) {
+      f32x16_t c;
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&table[stage * BT + sb * 32 + 8 * jj + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[4 * jj + i] = v[i];
+      }
+      return c;
+    };
+    auto load_inits = [&](auto sb_tag) __attribute__((always_inline)) {
+      constexpr int sb = decltype(sb_tag)::value;
+      if constexpr (KV_STATIONARY && sb < NSB) {
+        S[sb] = init_from(sLse, sb);
+        if constexpr (HAS_DS) dP[sb] = init_from(sDelta, sb);
       }
     };
     float held_p = 0.f, held_ds = 0.f;
     uint32_t px[PAIR ? 8 : 1];  // paired role: the sub-block's probabilities as fp16 pairs
     auto elem = [&](auto sb_tag, auto r_tag) {
       constexpr int sb = decltype(sb_tag)::value, r = decltype(r_tag)::value;
-      constexpr int i = r % 4;
-      if constexpr (i == 0) load_group(std::integral_constant<int, sb * 4 + r / 4>{});
-      float x;
-      if constexpr (KV_STATIONARY) x = fast_exp2(S[sb][r] - ls4[i]);
-      else x = fast_exp2(S[sb][r] - lse_l);
+      float x = fast_exp2((KV_STATIONARY || INIT_REGS) ? S[sb][r] : S[sb][r] + lse_l);
       if constexpr (MASKED) {
-        uint32_t ok;
-        if constexpr (KV_STATIONARY) ok = (key_packed + ta[i]) & (tb[i] - key_packed) & kGuardBits;
-        else ok = (ta[i] + addc) & (subc - ta[i]) & kGuardBits;
-        x = (ok == kGuardBits) ? x : 0.f;
+        // 0 or ~0 (as assembly: from the builtin the compiler forms a test of the bit and a select)
+        uint32_t keep;
+        asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(keep) : "v"(bits), "n"(16 * sb + r));
+        x = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, x) & keep);
       }
       float ds = 0.f;
-      if constexpr (HAS_DS) {
-        if constexpr (KV_STATIONARY) ds = x * (dP[sb][r] - dl4[i]);
-        else ds = x * (dP[sb][r] - delta_l);
-      }
+      if constexpr (HAS_DS) ds = x * ((KV_STATIONARY || INIT_REGS) ? dP[sb][r] : dP[sb][r] + delta_l);
       if constexpr (r % 2 == 0) {
         pin(x);
         held_p = x;
@@ -770,6 +796,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
     };
 
     vec8 fr[G];
+    load_inits(std::integral_constant<int, 0>{});
     for_range<0, PF>([&](auto x_tag) { fr[decltype(x_tag)::value] = frag(x_tag); });
     for_range<0, G>([&](auto x_tag) __attribute__((always_inline)) {
       constexpr int x = decltype(x_tag)::value;
@@ -778,11 +805,23 @@ fna_bwd_kernel(const FnaBwdParams p) {
       if constexpr (x + PF < G) fr[x + PF] = frag(std::integral_constant<int, x + PF>{});
       if constexpr (sl.prod) {
         constexpr int ks = sl.i / WP, which = sl.i % WP;
-        f32x16_t zero;
+        if constexpr (ks == 0 && !KV_STATIONARY) {
+          if constexpr (INIT_REGS) {
+            if constexpr (which == 0) S[sb] = M::run_from(fr[x], x1f[ks], lse_init);
+            else dP[sb] = M::run_from(fr[x], x2f[ks], delta_init);
+          } else {
+            f32x16_t zero;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-        if constexpr (which == 0) S[sb] = M::run(fr[x], x1f[ks], ks == 0 ? zero : S[sb]);
-        else dP[sb] = M::run(fr[x], x2f[ks], ks == 0 ? zero : dP[sb]);
+            for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+            if constexpr (which == 0) S[sb] = M::run(fr[x], x1f[ks], zero);
+            else dP[sb] = M::run(fr[x], x2f[ks], zero);
+          }
+        } else {
+          if constexpr (which == 0) S[sb] = M::run(fr[x], x1f[ks], S[sb]);
+          else dP[sb] = M::run(fr[x], x2f[ks], dP[sb]);
+        }
+        // the accumulator inputs of the other sub-block's products, a few slots before these begin
+        if constexpr (SPREAD && sb == 0 && sl.i == NP - 3) load_inits(std::integral_constant<int, 1>{});
         // all probabilities of the sub-block once its products are complete
         if constexpr (!SPREAD && sl.i == NP - 1) for_range<0, 16>([&](auto r_tag) { elem(std::integral_constant<int, sb>{}, r_tag); });
       } else {
@@ -790,6 +829,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
         constexpr bool to_acc1 = HAS_DS && (sl.i % W == 0);
         if constexpr (to_acc1) acc1[db] = M::run(fr[x], dsf[sb][h], acc1[db]);
         else acc2[db] = M::run(fr[x], pf[sb][h], acc2[db]);
+        if constexpr (!SPREAD && sb == 0 && sl.i == NC - 3) load_inits(std::integral_constant<int, 1>{});
       }
       if constexpr (SPREAD && x >= NP && x < 2 * NP + NC) {
         // two probabilities per slot, between the matrix instructions of the other sub-block
@@ -807,10 +847,19 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // consume: dS of the previous tile from its dP^T, its delta and the P waves' probabilities,
   // then dK += dS^T Q with that tile's Q (still in its stage).
   f32x16_t held_dp[NSB];
-  auto pair_produce = [&](int stage) __attribute__((always_inline)) {
+  auto pair_produce = [&](int stage1, int stage) __attribute__((always_inline)) {
     const char* y2 = sY2 + stage * TILE_BYTES;
     constexpr int N = NSB * KSTEPS;
     vec8 fr[N];
+    // the products start from -delta of the tile's queries (tables live in the stages of Y1)
+#pragma unroll
+    for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj) {
+        const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sDelta[stage1 * BT + sb * 32 + 8 * jj + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) held_dp[sb][4 * jj + i] = v[i];
+      }
     for_range<0, PF>([&](auto x_tag) {
       constexpr int x = decltype(x_tag)::value;
       fr[x] = row_frag(y2, x / KSTEPS, x % KSTEPS);
@@ -819,10 +868,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       constexpr int x = decltype(x_tag)::value;
       constexpr int sb = x / KSTEPS, ks = x % KSTEPS;
       if constexpr (x + PF < N) fr[x + PF] = row_frag(y2, (x + PF) / KSTEPS, (x + PF) % KSTEPS);
-      f32x16_t zero;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-      held_dp[sb] = M::run(fr[x], x1f[ks], ks == 0 ? zero : held_dp[sb]);
+      held_dp[sb] = M::run(fr[x], x1f[ks], held_dp[sb]);
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -836,17 +882,14 @@ fna_bwd_kernel(const FnaBwdParams p) {
       plo[sb] = *reinterpret_cast<const u32x4_t*>(src);
       phi[sb] = *reinterpret_cast<const u32x4_t*>(src + 64 * 16);
     }
-    // dS values 4 jj + 2 i2 and + 1 of a sub-block (k = 2 jj + i2)
-    f32x4_t dl4;
+    // dS values 2 k and 2 k + 1 of a sub-block: the probabilities as they lie in the word, times dP
     auto ds_pair = [&](auto sb_tag, auto k_tag) {
-      constexpr int sb = decltype(sb_tag)::value, k = decltype(k_tag)::value;
-      constexpr int jj = k / 2, i2 = k % 2, r = 4 * jj + 2 * i2;
-      if constexpr (i2 == 0) dl4 = *reinterpret_cast<const f32x4_t*>(&sDelta[stage * BT + sb * 32 + 8 * jj + 4 * g]);
+      constexpr int sb = decltype(sb_tag)::value, r = 2 * decltype(k_tag)::value;
       const uint32_t pw = (r < 8) ? plo[sb][r / 2] : phi[sb][r / 2 - 4];
+      // (as multiply-adds: one mixed-precision instruction each instead of a conversion and a product)
       const h16x2_t h2 = __builtin_bit_cast(h16x2_t, pw);
-      const float d0 = float(h2[0]) * (held_dp[sb][r] - dl4[2 * i2]);
-      const float d1 = float(h2[1]) * (held_dp[sb][r + 1] - dl4[2 * i2 + 1]);
-      vec2 d2 = {static_cast<T>(d0), static_cast<T>(d1)};
+      const vec2 d2 = {static_cast<T>(__builtin_fmaf(float(h2[0]), held_dp[sb][r], 0.f)),
+                       static_cast<T>(__builtin_fmaf(float(h2[1]), held_dp[sb][r + 1], 0.f))};
       dsf[sb][r / 8][r % 8] = d2[0];
       dsf[sb][r / 8][r % 8 + 1] = d2[1];
     };
@@ -873,29 +916,33 @@ fna_bwd_kernel(const FnaBwdParams p) {
     });
   };
   constexpr int CPT = 2 * PER;  // tile copies per thread and tile
-  // One pass of the paired role over n_iter tiles: step `it` has the P waves on tile `it` and the
-  // dS waves forming dP of tile `it` after finishing tile it - 1; one more step drains the dS
-  // waves.  Tiles are copied two steps ahead: tile it + 2 during step `it`, into the Y2 stage of
-  // tile it - 1 and the Y1 / table stage of tile it - 2, both last read in step it - 1.  The
-  // barrier at the top of a step makes tile `it` and the probabilities of tile it - 1 visible and
-  // separates those last reads from the copies that overwrite them.
-  auto run_pass_pair = [&](auto masked_tag, auto ds_wave_tag, int n_iter) __attribute__((always_inline)) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
+  workgroup_sync();  // sRows is written
+  // The paired role over n_iter tiles: step `it` has the P waves on tile `it` and the dS waves forming
+  // dP of tile `it` after finishing tile it - 1; one more step drains the dS waves.  Tiles are copied
+  // two steps ahead: tile it + 2 during step `it`, into the Y2 stage of tile it - 1 and the Y1 / table
+  // stage of tile it - 2, both last read in step it - 1.  The barrier at the top of a step makes tile
+  // `it` and the probabilities of tile it - 1 visible and separates those last reads from the
+  // copies that overwrite them.
+  auto run_pair = [&](auto ds_wave_tag) __attribute__((always_inline)) {
     constexpr bool DS_WAVE = decltype(ds_wave_tag)::value;
-    if (n_iter <= 0) return;
-    start_walk(std::integral_constant<bool, !MASKED>{});
-    Tile tn = next_tile(std::integral_constant<bool, !MASKED>{}, 1 < n_iter);
-    issue(tn, 0, MASKED && !DS_WAVE);  // wave 0, which builds the window tables, is a P wave
+    uint32_t bits0 = 0, bits1 = 0, bits2 = 0;  // P waves: attended pairs of the tiles it, it + 1, it + 2 (while masked)
+    {
+      const Tile t = next_tile();
+      issue_copies(t, 0, 0);
+      if constexpr (!DS_WAVE) bits0 = pair_bits(t);
+    }
     if (1 < n_iter) {
-      tn = next_tile(std::integral_constant<bool, !MASKED>{}, 2 < n_iter);
-      issue(tn, 1, MASKED && !DS_WAVE);
+      const Tile t = next_tile();
+      issue_copies(t, 1, 1);
+      if constexpr (!DS_WAVE) bits1 = pair_bits(t);
     }
     // A wave walks to tile it + 2 and issues its share of the copies where it has vector or
     // scalar work anyway: the dS waves between their two matrix phases, the P waves after the
     // products of their first sub-block; the eight waves then do not queue on the CU's address
     // path together while the matrix pipe idles.
     int s2 = 0;  // it % 3
-    for (int it = 0; it <= n_iter; ++it) {
+    auto step = [&](auto masked_tag, int it) __attribute__((always_inline)) {
+      constexpr bool MASKED = decltype(masked_tag)::value;
       // this thread's copies of tile `it` have landed once only those of tile it + 1 are
       // outstanding (wave 0 makes one copy less per tile)
       if (it + 1 < n_iter) {
@@ -908,64 +955,49 @@ fna_bwd_kernel(const FnaBwdParams p) {
       const int s2_ahead = s2 == 0 ? 2 : s2 - 1;  // (it + 2) % 3
       auto ahead = [&]() __attribute__((always_inline)) {
         if (it + 2 < n_iter) {
-          tn = next_tile(std::integral_constant<bool, !MASKED>{}, it + 3 < n_iter);
-          build_tables(tn, (it + 2) & 3, MASKED && !DS_WAVE);
-          issue_copies(tn, (it + 2) & 3, s2_ahead);
+          const Tile t = next_tile();
+          issue_copies(t, (it + 2) & 3, s2_ahead);
+          if constexpr (MASKED && !DS_WAVE) bits2 = pair_bits(t);
         }
       };
       if constexpr (DS_WAVE) {
         if (it > 0) pair_consume((it - 1) & 3, (it - 1) & 1);
         ahead();
-        if (it < n_iter) pair_produce(s2);
+        if (it < n_iter) pair_produce(it & 3, s2);
       } else {
-        if (it < n_iter) {
-          tile_body(masked_tag, it & 3, s2, 0u, 0u, it & 1, [&](auto x_tag) __attribute__((always_inline)) {
-            if constexpr (decltype(x_tag)::value == NP - 1) ahead();
-          });
+        tile_body(masked_tag, it & 3, s2, bits0, it & 1, [&](auto x_tag) __attribute__((always_inline)) {
+          if constexpr (decltype(x_tag)::value == NP - 1) ahead();
+        });
+        if constexpr (MASKED) {
+          bits0 = bits1;
+          bits1 = bits2;
         }
       }
       s2 = s2 == 2 ? 0 : s2 + 1;
+    };
+    if constexpr (DS_WAVE) {
+      for (int it = 0; it <= n_iter; ++it) step(std::false_type{}, it);
+    } else {
+      int it = 0;
+      for (; it < n_masked; ++it) step(std::true_type{}, it);
+      for (; it < n_iter; ++it) step(std::false_type{}, it);
+      workgroup_sync();  // the step in which the dS waves finish the last tile
     }
-    wait_vmcnt<0>();
-    workgroup_sync();  // stages and probability buffers are free for the next pass
   };
 
-  // ---- pipeline: tile `it` is multiplied while tiles it+1 .. it+NS-1 are in flight ----------------
-  // Descriptor queue: d[0] = tile `it`, d[k] = tile it + k.
-  auto run_pass = [&](auto masked_tag, int n_iter) __attribute__((always_inline)) {
-    constexpr bool MASKED = decltype(masked_tag)::value;
-    if (n_iter <= 0) return;
-    start_walk(std::integral_constant<bool, !MASKED>{});
-    // dQ role, masked pass: origins of the tiles in flight (the lane's mask constants need the
-    // origin of the tile being multiplied); og<k> = origin of tile it + k
-    constexpr bool NEED_ORIGIN = MASKED && !KV_STATIONARY;
-    int og0[3] = {0, 0, 0}, og1[3] = {0, 0, 0}, og2[3] = {0, 0, 0};
-    int ld0[3] = {0, 0, 0}, ld1[3] = {0, 0, 0}, ld2[3] = {0, 0, 0};  // ... and their leads
-    if (0 < n_iter && NS > 1) {
-      const Tile t = next_tile(std::integral_constant<bool, !MASKED>{}, 1 < n_iter);
-      issue(t, 0, MASKED);
-      if constexpr (NEED_ORIGIN) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          og0[a] = t.origin[a];
-          ld0[a] = t.lead[a];
-        }
-      }
-    }
-    if (1 < n_iter && NS > 2) {
-      const Tile t = next_tile(std::integral_constant<bool, !MASKED>{}, 2 < n_iter);
-      issue(t, 1, MASKED);
-      if constexpr (NEED_ORIGIN) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          og1[a] = t.origin[a];
-          ld1[a] = t.lead[a];
-        }
-      }
-    }
-
-    for (int it = 0; it < n_iter; ++it) {
-      const int stage = it % NS;
+  // ---- the other roles: tile `it` is multiplied while tiles it+1 .. it+NS-1 are in flight ----------
+  auto run_tiles = [&]() __attribute__((always_inline)) {
+    uint32_t bits0 = 0, bits1 = 0, bits2 = 0;  // attended pairs of the tiles it, it + 1, it + 2 (while masked)
+    auto issue_next = [&](int stage) __attribute__((always_inline)) {
+      const Tile t = next_tile();
+      issue_copies(t, stage, stage);
+      return t;
+    };
+    bits0 = pair_bits(issue_next(0));
+    if (NS > 2 && 1 < n_iter) bits1 = pair_bits(issue_next(1));
+    int stage = 0;  // it % NS
+    auto step = [&](auto masked_tag, int it) __attribute__((always_inline)) {
+      constexpr bool MASKED = decltype(masked_tag)::value;
       // this thread's copies of tile `it` have landed once at most those of the later tiles in
       // flight (one tile with three stages, none with two) are outstanding; wave 0 makes one
       // copy less per tile in the key-stationary roles
@@ -977,56 +1009,29 @@ fna_bwd_kernel(const FnaBwdParams p) {
       }
       workgroup_sync();  // tile `it` and its tables are in LDS; everyone is done with the stage of tile it - 1
       if (it + NS - 1 < n_iter) {
-        const Tile t = next_tile(std::integral_constant<bool, !MASKED>{}, it + NS < n_iter);
-        issue(t, (it + NS - 1) % NS, MASKED);
-        if constexpr (NEED_ORIGIN) {
-#pragma unroll
-          for (int a = 0; a < 3; ++a) {
-            (NS == 3 ? og2[a] : og1[a]) = t.origin[a];
-            (NS == 3 ? ld2[a] : ld1[a]) = t.lead[a];
-          }
-        }
+        const Tile t = issue_next(stage == 0 ? NS - 1 : stage - 1);  // stage (it + NS - 1) % NS
+        if constexpr (MASKED) (NS == 3 ? bits2 : bits1) = pair_bits(t);
       }
-
-      uint32_t addc = 0, subc = 0;
-      if constexpr (NEED_ORIGIN) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int lo = na_min(na_max(wst[a] - og0[a], ld0[a]), b_sub[a]);
-          const int hi = na_min(na_max(wen[a] - og0[a], 0), b_sub[a]);
-          addc |= uint32_t(512 - lo) << (10 * a);
-          subc |= uint32_t(511 + hi) << (10 * a);
-        }
+      tile_body(masked_tag, stage, stage, bits0, 0, [](auto) {});
+      if constexpr (MASKED) {
+        bits0 = bits1;
+        bits1 = bits2;
       }
-      tile_body(masked_tag, stage, stage, addc, subc, 0, [](auto) {});
-      if constexpr (NEED_ORIGIN) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          og0[a] = og1[a];
-          og1[a] = og2[a];
-          ld0[a] = ld1[a];
-          ld1[a] = ld2[a];
-        }
-      }
-    }
-    wait_vmcnt<0>();
-    workgroup_sync();  // the stages are free for the next pass
+      stage = stage == NS - 1 ? 0 : stage + 1;
+    };
+    int it = 0;
+    for (; it < n_masked; ++it) step(std::true_type{}, it);
+    for (; it < n_iter; ++it) step(std::false_type{}, it);
   };
-  const int heads_walked = KV_STATIONARY ? rep : 1;
   if constexpr (PAIR) {
-    // the two kinds of wave run separate copies of the passes (the same barriers in both), so
+    // the two kinds of wave run separate copies of the loop (the same barriers in both), so
     // that neither carries the other's registers
-    if (part == 0) {
-      run_pass_pair(std::true_type{}, std::false_type{}, (total - n_whole) * heads_walked);
-      run_pass_pair(std::false_type{}, std::false_type{}, n_whole * heads_walked);
-    } else {
-      run_pass_pair(std::true_type{}, std::true_type{}, (total - n_whole) * heads_walked);
-      run_pass_pair(std::false_type{}, std::true_type{}, n_whole * heads_walked);
-    }
+    if (part == 0) run_pair(std::false_type{});
+    else run_pair(std::true_type{});
   } else {
-    run_pass(std::true_type{}, (total - n_whole) * heads_walked);
-    run_pass(std::false_type{}, n_whole * heads_walked);
+    run_tiles();
   }
+  wait_vmcnt<0>();
 
   // dQ = scale * sum_k dS k;  dK = scale * sum_q dS q = ln 2 * sum_q dS q'
   store_results(acc1, acc2, KV_STATIONARY ? 0.6931471805599453f : p.scale);
@@ -1044,7 +1049,7 @@ __global__ void __launch_bounds__(256) scale_queries_kernel(const T* q, T* qs, i
 
 // What the backward launches read besides the operands, in one pass over q, out and d_out
 // [batch, tokens, heads, D]: q' (as scale_queries_kernel), and head-major [batch, heads, tokens]
-// delta = rowsum(d_out * out) and a copy of lse [batch, tokens, heads].  HBM-bound (three reads and
+// -rowsum(d_out * out) and -log2(e) lse (lse [batch, tokens, heads]).  HBM-bound (three reads and
 // one write of q's size; the reads are non-temporal, 5-10 % faster here).  Against separate launches
 // (delta, scaled queries, two transposes): 17.9 -> 6.3 us on 4 x 56 x 56 tokens, H 8, D 32; 52.5 -> 42.8
 // on 128 x 128, H 16, D 128 (6.3 TB/s); 450 -> 480 on 29 x 46 x 78, H 24, D 128 (5.3 TB/s).
@@ -1054,8 +1059,8 @@ __global__ void __launch_bounds__(256) scale_queries_kernel(const T* q, T* qs, i
 template <typename T, int D>
 __global__ void __launch_bounds__(256) bwd_prepare_kernel(const T* __restrict__ q, const T* __restrict__ out,
                                                           const T* __restrict__ d_out, const float* __restrict__ lse,
-                                                          T* __restrict__ qs, float* __restrict__ delta,
-                                                          float* __restrict__ lse_heads, int tokens, int heads, int hb_lg,
+                                                          T* __restrict__ qs, float* __restrict__ neg_delta,
+                                                          float* __restrict__ neg_lse2, int tokens, int heads, int hb_lg,
                                                           NaDiv d_head_blocks, NaDiv d_token_blocks, float c_log2) {
   using vec8 = typename Mma<T>::vec8;
   constexpr int LPI = D / 8;     // lanes per row
@@ -1092,8 +1097,8 @@ __global__ void __launch_bounds__(256) bwd_prepare_kernel(const T* __restrict__ 
   workgroup_sync();
   if (tt < tokens) {
     const int64_t at = (int64_t(b) * heads + h0 + ht) * tokens + tt;
-    delta[at] = s_delta[tid];
-    lse_heads[at] = my_lse;
+    neg_delta[at] = -s_delta[tid];
+    neg_lse2[at] = -1.4426950408889634f * my_lse;
   }
 }
 

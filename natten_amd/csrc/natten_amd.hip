@@ -871,9 +871,9 @@ static int split_dim_of(const int* tile) {
 }
 
 static int check_bwd_pointers(const char* what, const void* q, const void* k, const void* v, const void* d_out,
-                              const float* lse, const float* delta, void* dq, void* dk, void* dv, void* q_scaled,
+                              const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled,
                               int roles) {
-  if (!q || !k || !v || !d_out || !lse || !delta || !dq || !dk || !dv) return fail("%s: null pointer argument", what);
+  if (!q || !k || !v || !d_out || !neg_lse2 || !neg_delta || !dq || !dk || !dv) return fail("%s: null pointer argument", what);
   if ((roles & 2) && !q_scaled) return fail("%s: the dk / dv launch needs the q_scaled workspace", what);
   if (q_scaled == q) return fail("%s: q_scaled must not be q itself (the dq launch reads the unscaled queries)", what);
   if (reinterpret_cast<uintptr_t>(q_scaled) & 15) return fail("%s: q_scaled must be 16-byte aligned", what);
@@ -884,8 +884,8 @@ static int check_bwd_pointers(const char* what, const void* q, const void* k, co
   return 0;
 }
 
-int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                            const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
+int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
+                            const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
                             int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
                             const int32_t* q_shape, const int32_t* kv_shape, const int32_t* qkv_shape,
                             const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
@@ -893,8 +893,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
                             float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "fna_backward";
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
-  if (int rc = check_common(what, q, k, v, dq, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 3)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!q_shape || !kv_shape || !qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape ||
       !kv_tile_shape)
@@ -933,8 +933,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.lse = lse;
-  p.delta = delta;
+  p.neg_lse2 = neg_lse2;
+  p.neg_delta = neg_delta;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
@@ -949,8 +949,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
 }
 
-int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
+int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
+                                  const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
                                   int batch, int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
                                   const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
                                   const int32_t* is_causal, const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
@@ -959,7 +959,7 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   const char* what = "fna_backward_fused";
   if (roles < 1 || roles > 7 || (roles & 3) == 0)
     return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 where q_scaled is filled already, got %d", what, roles);
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, roles)) return rc;
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, roles)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape || !kv_tile_shape)
     return fail("%s: null shape argument", what);
@@ -987,7 +987,7 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                is_causal, q_tile_shape, kv_tile_shape))
     return rc;
   if (!fna_tiles_are_powers_of_two(f)) return fail("%s: tile extents must be powers of two", what);
-  if (int rc = check_common(what, q, k, v, dq, lse, batch, int(tokens), int(tokens), heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, int(tokens), int(tokens), heads_q, heads_kv, head_dim)) return rc;
   // per-lane byte offsets inside a tile are 32-bit
   long long span_q = 0, span_kv = 0;
   for (int a = 0; a < 3; ++a) {
@@ -1023,8 +1023,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.lse = lse;
-  p.delta = delta;
+  p.neg_lse2 = neg_lse2;
+  p.neg_delta = neg_delta;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
@@ -1045,8 +1045,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
 
 namespace {
 // dense attention backward as the 1-D neighborhood problem whose window is the whole key sequence
-void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                    const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int batch, int seqlen_q, int seqlen_kv,
+void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
+                    const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int batch, int seqlen_q, int seqlen_kv,
                     int heads_q, int heads_kv, int is_causal, float scale, int filled) {
   memset(&p, 0, sizeof(p));
   for (int a = 0; a < 3; ++a) {
@@ -1063,8 +1063,8 @@ void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.lse = lse;
-  p.delta = delta;
+  p.neg_lse2 = neg_lse2;
+  p.neg_delta = neg_delta;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
@@ -1079,33 +1079,33 @@ void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v
 }
 }  // namespace
 
-int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
+int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
+                                  const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
                                   int dtype, int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
                                   int is_causal, float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "attention_backward";
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
-  if (int rc = check_common(what, q, k, v, dq, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 3)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
   FnaBwdParams p;
-  fill_dense_bwd(p, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal,
+  fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal,
                  scale, q_scaled_filled);
   // (sequences of whole tiles need no clamping: the instances of neighborhood attention)
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), seqlen_q % 128 != 0 || seqlen_kv % 128 != 0);
 }
 
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v, const void* d_out,
-                                         const float* lse, const float* delta, void* dq, void* dk, void* dv,
+                                         const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv,
                                          void* q_scaled, int q_scaled_filled, int dtype, int num_seqs, int rows_q, int rows_kv,
                                          const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv, int heads_q,
                                          int heads_kv, int head_dim, int is_causal, float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "attention_backward_varlen";
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
-  if (int rc = check_common(what, q, k, v, dq, lse, num_seqs, rows_q, rows_kv, heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 3)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, neg_lse2, num_seqs, rows_q, rows_kv, heads_q, heads_kv, head_dim)) return rc;
   if (!cu_seqlens_q || !cu_seqlens_kv) return fail("%s: null cumulative length argument", what);
   FnaBwdParams p;
-  fill_dense_bwd(p, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
+  fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
                  q_scaled_filled);
   // lengths and windows are replaced per sequence inside the kernel
   p.q_tiled[0] = rows_q / 128 + 2 * (num_seqs + 1);
@@ -1162,11 +1162,11 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
 }
 
 int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse, void* q_scaled,
-                                float* delta, float* lse_heads, int dtype, int batch, int tokens, int heads, int head_dim,
+                                float* neg_delta, float* neg_lse2, int dtype, int batch, int tokens, int heads, int head_dim,
                                 float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "backward_prepare";
-  if (!q || !out || !d_out || !lse || !q_scaled || !delta || !lse_heads) return fail("%s: null pointer argument", what);
+  if (!q || !out || !d_out || !lse || !q_scaled || !neg_delta || !neg_lse2) return fail("%s: null pointer argument", what);
   if (batch < 1 || tokens < 1 || heads < 1) return fail("%s: batch, tokens and heads must be positive", what);
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(d_out) |
        reinterpret_cast<uintptr_t>(q_scaled)) & 15)
@@ -1180,8 +1180,8 @@ int natten_amd_backward_prepare(const void* q, const void* out, const void* d_ou
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define NA_PREPARE_LAUNCH(TYPE, DD)                                                                                        \
   hipLaunchKernelGGL((bwd_prepare_kernel<TYPE, DD>), dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const TYPE*>(q),                     \
-                     static_cast<const TYPE*>(out), static_cast<const TYPE*>(d_out), lse, static_cast<TYPE*>(q_scaled), delta, \
-                     lse_heads, tokens, heads, hb_lg, na_make_div(head_blocks), na_make_div(token_blocks), c_log2)
+                     static_cast<const TYPE*>(out), static_cast<const TYPE*>(d_out), lse, static_cast<TYPE*>(q_scaled),       \
+                     neg_delta, neg_lse2, tokens, heads, hb_lg, na_make_div(head_blocks), na_make_div(token_blocks), c_log2)
 #define NA_PREPARE_DTYPE(DD)                                             \
   do {                                                                   \
     if (dtype == NATTEN_AMD_F16) NA_PREPARE_LAUNCH(_Float16, DD);        \
