@@ -86,8 +86,8 @@ const char* natten_amd_last_error(void);
  *
  * float32 operands (dtype F32; the reference's tests run float32 at atol 1e-4,
  * tests/test_fna.py:107-131): tiles of 128 x 64 tokens, head_dim 32, 64 or 128, no scales; products,
- * sums and softmax in float32 (P not rounded), output float32.  This entry point only (no one-launch
- * form, no backward).
+ * sums and softmax in float32 (P not rounded), output float32.  The one-launch form is
+ * natten_amd_fna_forward_f32; there is no backward.
  *
  * run_persistent (the reference's `run_persistent` argument, blackwell_fna.h:52, scheduler
  * csrc/include/natten/cuda/fmha_blackwell/kernel/fmha_tile_scheduler.hpp:146-149): non-zero
@@ -155,6 +155,19 @@ int natten_amd_fna_forward_fused(const void* q, const void* k, const void* v, vo
                                  float scale, const float* q_scale, const float* k_scale,
                                  const float* v_scale, int anchor_kv_tiles, int run_persistent,
                                  void* workspace, uint64_t workspace_bytes, void* stream);
+
+/*
+ * float32 operands in the original layout, one launch: q, out [batch, *qkv_shape, heads_q, head_dim],
+ * k, v [batch, *qkv_shape, heads_kv, head_dim], lse [batch, *qkv_shape, heads_q], head_dim any multiple
+ * of 8 up to 128, pointers 16-byte aligned, any extents.  The operation of
+ * blackwell_na{1,2,3}d_forward (csrc/include/natten/blackwell_fna.h:36-52) with products, sums and
+ * softmax in float32; the kernel picks its own boxes of 16 queries and blocks of 16 keys.
+ */
+int natten_amd_fna_forward_f32(const void* q, const void* k, const void* v, void* out, float* lse,
+                               int na_dim, int batch, int heads_q, int heads_kv, int head_dim,
+                               const int32_t* qkv_shape, const int32_t* kernel_size,
+                               const int32_t* stride, const int32_t* dilation,
+                               const int32_t* is_causal, float scale, void* stream);
 
 /*
  * natten_amd_fna_forward_fused for problems with fewer Q tiles than the chip keeps workgroups

@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -61,6 +61,10 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_void_p] * 5 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 7 + [ctypes.c_float] + [ctypes.c_void_p] * 3
         + [ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p],
+    ),
+    "natten_amd_fna_forward_f32": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 5 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 5 + [ctypes.c_float, ctypes.c_void_p],
     ),
     "natten_amd_fna_forward_fused_split": (
         ctypes.c_int,
@@ -359,6 +363,30 @@ def fna_forward_fused(
             _i32(qkv_shape), _i32(kernel_size), _i32(stride), _i32(dilation),
             _i32([1 if c else 0 for c in is_causal]), _i32(q_tile_shape), _i32(kv_tile_shape),
             float(scale), *scales, 1 if anchored_tiles else 0, *_queue_workspace(q, run_persistent), _stream(q),
+        )
+    _check(rc)
+    return out, lse
+
+
+def fna_forward_f32(
+    q: Tensor, k: Tensor, v: Tensor, kernel_size, stride, dilation, is_causal, scale: float,
+) -> Tuple[Tensor, Tensor]:
+    """Float32 operands in the original layout, q [B, *X, H, D], k/v [B, *X, Hkv, D], any D that is a
+    multiple of 8 up to 128 -> (out like q, lse float32 [B, *X, H]), one launch."""
+    L = lib()
+    _require_gpu(q, k, v)
+    if not q.dtype == k.dtype == v.dtype == torch.float32:
+        raise NotImplementedError(f"natten_amd fna_forward_f32 does not support {q.dtype}.")
+    # (the kernel reads and writes sixteen bytes per lane)
+    q, k, v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
+    na_dim = len(kernel_size)
+    out = torch.empty_like(q)
+    lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
+    with _on_device(q):
+        rc = L.natten_amd_fna_forward_f32(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), na_dim, q.shape[0], q.shape[-2],
+            k.shape[-2], q.shape[-1], _i32(q.shape[1 : 1 + na_dim]), _i32(kernel_size), _i32(stride), _i32(dilation),
+            _i32([1 if c else 0 for c in is_causal]), float(scale), _stream(q),
         )
     _check(rc)
     return out, lse

@@ -1,11 +1,12 @@
-// Fused neighborhood attention forward for float32 operands on gfx950, on token-permuted sequences.
+// Neighborhood attention forward for float32 operands on gfx950: fna_fwd_f32_direct_kernel on the
+// original tensors (the default), fna_fwd_f32_kernel on token-permuted sequences (for callers that fix
+// tile shapes or ask for that route).
 // The reference runs float32 through its CUTLASS 2.x kernels and, on CPU, through flex attention
 // (SHI-Labs/NATTEN tests/test_fna.py:107-131 states the tolerance: 1e-4 on the output); here it is a
 // plain kernel of its own: S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x2_f32 (IEEE float32
 // products and sums), exact online softmax in float32 (no lazy rescale, P not rounded), every logit
 // tested against its query's window (no whole-tile classification).  One workgroup per Q tile of
-// 128 rows, 64-key tiles staged through LDS with ordinary loads; built for correctness at the
-// stated dtype, not tuned like fna_fwd_kernel.
+// 128 rows, 64-key tiles staged through LDS with ordinary loads.
 #pragma once
 
 #include "fna_fwd.hpp"
@@ -203,6 +204,316 @@ __global__ void __launch_bounds__(256) fna_fwd_f32_kernel(const FnaParams p) {
       *reinterpret_cast<f32x4_t*>(orow + db * 32 + 8 * j + 4 * g) = o4;
     }
   if (g == 0) p.lse[q_row * p.heads_q + head] = (l > 0.f) ? (m_run * 0.6931471805599453f + logf(l)) : -INFINITY;
+}
+
+// ---- on the original tensors ----------------------------------------------------------------------
+struct FnaF32Params {
+  const float *q, *k, *v;
+  float *o, *lse;
+  int heads_q, heads_kv, head_dim;  // head_dim: elements of a row, a multiple of 4, at most the instance's D
+  int dims;                         // dimensions that can mask anything: 1, 2 or 3 (the rest have extent 1)
+  int ksize[3], stride[3], dil[3], causal[3];
+  int ext_base[3], ext_rem[3];      // extent of dilation group g along a dimension = base + (g < rem)
+  int tok_stride[3], tokens;
+  int q_lg[3], kv_lg[3];            // log2 extents of a wave's box of 16 queries / of a block of 16 keys (sums 4)
+  int q_boxes[3];                   // boxes per dimension
+  NaDiv d_stride[3], d_dil[3], d_q_boxes[3], d_boxes, d_heads_q, d_q_per_kv, d_num_groups;
+  int num_boxes, num_groups;
+  int waves, wgs_per_xcd;           // one wave per (batch, dilation group, head, box)
+  float scale;
+};
+
+// Boxes of 16 queries and blocks of 16 keys that let the fewest (query, key) pairs be multiplied: along a
+// dimension a box of tq queries spans the window plus the distance its stride groups' leaders cover,
+// rounded up to whole blocks.  Ties go to boxes that are long in the last dimension.
+inline void choose_f32_boxes(FnaF32Params& p) {
+  long long cost[3][5][5];
+  for (int a = 0; a < 3; ++a) {
+    const int ext = p.ext_base[a] + (p.ext_rem[a] > 0);
+    for (int lq = 0; lq < 5; ++lq)
+      for (int lk = 0; lk < 5; ++lk) {
+        const int tq = 1 << lq, s = p.stride[a];
+        const int reach = s % tq == 0 ? 0 : ((tq - 1 + s - 1) / s) * s;
+        const int span = na_min(ext, p.ksize[a] + (p.causal[a] ? tq - 1 : reach));
+        cost[a][lq][lk] = (long long)(((ext + tq - 1) >> lq) << lq) * (((span + (1 << lk) - 1) >> lk) << lk);
+      }
+  }
+  // (dimensions from p.dims on have extent 1: boxes and blocks stay inside it, the element mask skips them)
+  double best = -1;
+  for (int q0 = 0; q0 <= 4; ++q0)
+    for (int q1 = 0; q0 + q1 <= 4; ++q1)
+      for (int k0 = 0; k0 <= 4; ++k0)
+        for (int k1 = 0; k0 + k1 <= 4; ++k1) {
+          const int q2 = 4 - q0 - q1, k2 = 4 - k0 - k1;
+          if ((p.dims < 2 && (q1 | k1)) || (p.dims < 3 && (q2 | k2))) continue;
+          const double c = double(cost[0][q0][k0]) * double(cost[1][q1][k1]) * double(cost[2][q2][k2]);
+          if (best >= 0 && c >= best) continue;
+          best = c;
+          p.q_lg[0] = q0, p.q_lg[1] = q1, p.q_lg[2] = q2;
+          p.kv_lg[0] = k0, p.kv_lg[1] = k1, p.kv_lg[2] = k2;
+        }
+}
+
+// One wave per box of 16 queries; no LDS and no barriers.  What bounds the float32 path is the matrix rate
+// (1/16 of bf16's), so what counts is how few pairs outside the windows are multiplied: with boxes of
+// 16 queries and blocks of 16 keys laid out from the first key of the wave's own windows a 13 x 13
+// window costs 256 keys a query, where a 128-query tile over 64-key tiles at multiples of their extent
+// costs 1024.  Each 16 x D block of K and of V goes straight from memory (mostly L1 / L2: neighbouring waves read
+// nearly the same keys) to the registers the matrix instruction reads, 8 D bytes per lane group against
+// 16 D matrix cycles, one block ahead of its use.
+//
+// v_mfma_f32_16x16x4_f32: with i = lane % 16, g = lane / 16 the A operand holds row i, the B operand
+// column i, k-index g; the result's register r is row 4 g + r, column i.  S^T = K Q^T: which head-dim
+// element k-index g of a step stands for is free as long as both operands agree: step (j, e) uses
+// element 16 j + 4 g + e, so that a lane's operands are float4 loads of its row.  The result holds the
+// logits of keys 4 g + r of query i, which is the B operand of O^T += V^T P^T step r (k-index g = key
+// 4 g + r) as it stands; row i of result block (h, c) is head-dim element VEC (16 h + i) + c, so that
+// V operands and results are VEC-wide loads and stores of whole rows.
+// Softmax in float32; a row's maximum is followed once it grew by more than 2^8 (exact: the sums are
+// normalised by the same maximum).
+// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 62 us (45 TFLOP/s of window pairs, 69 of pairs
+// multiplied; the card's float32 matrix products reach 154), 300 us as permutes, 128-query kernel and
+// unpermutes; 256 tokens, H 2, D 32, window 7: 23 us, all of it the call, from 83.
+template <int D, bool PAD>
+__global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32Params p) {
+  constexpr int KJ = D / 16;
+  constexpr int VEC = KJ < 4 ? KJ : 4;
+  constexpr int NH = D / (16 * VEC);
+  typedef float fvec __attribute__((ext_vector_type(VEC)));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int i16 = lane & 15, g = lane >> 4;
+
+  // waves are numbered box fastest, then head, then batch entry; every XCD takes a contiguous run of them
+  const int w = (int(blockIdx.x % kNumXcd) * p.wgs_per_xcd + int(blockIdx.x / kNumXcd)) * 4 + wave;
+  if (w >= p.waves) return;
+  const int bh = na_div(w, p.d_boxes);
+  int box = w - bh * p.num_boxes;
+  const int bg = na_div(bh, p.d_heads_q);
+  const int head = bh - bg * p.heads_q;
+  const int head_kv = na_div(head, p.d_q_per_kv);
+  const int b = na_div(bg, p.d_num_groups);
+  int gl = bg - b * p.num_groups;
+
+  int extent[3], step[3], org0[3], nblk[3], full_lo[3], full_hi[3];
+  int ws[3], width[3];  // this lane's query: window start and length
+  int kc[3], vc[3][4];  // in-block coordinates of the lane's key row (K) and of its four logits' keys (V)
+  int q_tok = 0, group_tok = 0;
+  bool valid = true;
+  {
+    int q_in = i16, k_in = i16;
+    int bc[3];
+    const int t01 = na_div(box, p.d_q_boxes[2]);
+    bc[2] = box - t01 * p.q_boxes[2];
+    bc[0] = na_div(t01, p.d_q_boxes[1]);
+    bc[1] = t01 - bc[0] * p.q_boxes[1];
+    bool empty = false;
+    int v_in = 4 * g;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) vc[0][r] = v_in + r;
+#pragma unroll
+    for (int a = 2; a >= 0; --a) {
+      const int off = q_in & ((1 << p.q_lg[a]) - 1);
+      q_in >>= p.q_lg[a];
+      kc[a] = k_in & ((1 << p.kv_lg[a]) - 1);
+      k_in >>= p.kv_lg[a];
+      if (a > 0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          vc[a][r] = vc[0][r] & ((1 << p.kv_lg[a]) - 1);
+          vc[0][r] >>= p.kv_lg[a];
+        }
+      }
+      bc[a] = (bc[a] << p.q_lg[a]);
+      ws[a] = off;
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const int rest = na_div(gl, p.d_dil[a]);
+      const int gi = gl - rest * p.dil[a];
+      gl = rest;
+      extent[a] = p.ext_base[a] + (gi < p.ext_rem[a] ? 1 : 0);
+      step[a] = p.dil[a] * p.tok_stride[a];
+      group_tok += gi * p.tok_stride[a];
+      empty = empty || bc[a] >= extent[a];  // (groups may be one shorter than the boxes were counted for)
+      const bool c = p.causal[a] != 0;
+      const int qf = na_min(bc[a], extent[a] - 1);
+      const int ql = na_min(bc[a] + (1 << p.q_lg[a]) - 1, extent[a] - 1);
+      const int st_f = na_window_start(qf, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
+      const int st_l = na_window_start(ql, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
+      org0[a] = st_f;
+      full_lo[a] = st_l;
+      full_hi[a] = na_window_end(qf, st_f, p.ksize[a], extent[a], c);
+      nblk[a] = (na_window_end(ql, st_l, p.ksize[a], extent[a], c) - st_f + (1 << p.kv_lg[a]) - 1) >> p.kv_lg[a];
+      const int qc = bc[a] + ws[a];
+      valid = valid && qc < extent[a];
+      const int q = na_min(qc, extent[a] - 1);  // queries past the group act as its last one and are not stored
+      ws[a] = na_window_start(q, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
+      width[a] = na_window_end(q, ws[a], p.ksize[a], extent[a], c) - ws[a];
+      q_tok += q * step[a];
+    }
+    if (empty) return;
+  }
+  const int64_t token0 = int64_t(b) * p.tokens + group_tok;
+  const int64_t q_row = (token0 + q_tok) * p.heads_q + head;
+  const int kv_row = p.heads_kv * p.head_dim;
+  const float* kbase = p.k + (token0 * p.heads_kv + head_kv) * p.head_dim;
+  const float* vbase = p.v + (token0 * p.heads_kv + head_kv) * p.head_dim;
+  const float c_log2 = p.scale * 1.4426950408889634f;
+
+  f32x4_t qf[KJ];
+#pragma unroll
+  for (int j = 0; j < KJ; ++j) {
+    qf[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if (!PAD || 16 * j + 4 * g < p.head_dim)
+      qf[j] = *reinterpret_cast<const f32x4_t*>(p.q + q_row * p.head_dim + 16 * j + 4 * g) * c_log2;
+  }
+
+  f32x4_t acc[NH][VEC];
+#pragma unroll
+  for (int h = 0; h < NH; ++h)
+#pragma unroll
+    for (int c = 0; c < VEC; ++c) acc[h][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+
+  // a lane's rows of a block that lies inside the group: fixed distances from the block's first token
+  int64_t k_off = 0, v_off[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    k_off += int64_t(kc[a] * step[a]) * kv_row;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v_off[r] += int64_t(vc[a][r] * step[a]) * kv_row;
+  }
+
+  struct Block {
+    f32x4_t k[KJ];
+    fvec v[4][NH];
+    int org[3];
+    bool full;
+  };
+  int it[3] = {0, 0, 0};
+  auto load = [&](Block& t) {
+    bool inside = true;
+    t.full = true;
+    int64_t row0 = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      t.org[a] = org0[a] + (it[a] << p.kv_lg[a]);
+      const int end = t.org[a] + (1 << p.kv_lg[a]);
+      inside = inside && end <= extent[a];
+      t.full = t.full && t.org[a] >= full_lo[a] && end <= full_hi[a];
+      row0 += int64_t(t.org[a]) * step[a];
+    }
+    int64_t ko = row0 * kv_row + k_off, vo[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) vo[r] = row0 * kv_row + v_off[r];
+    if (!inside) {
+      // keys past the group are masked: read its last ones in their place
+      int kt = 0, vt[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        kt += na_min(t.org[a] + kc[a], extent[a] - 1) * step[a];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) vt[r] += na_min(t.org[a] + vc[a][r], extent[a] - 1) * step[a];
+      }
+      ko = int64_t(kt) * kv_row;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) vo[r] = int64_t(vt[r]) * kv_row;
+    }
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      if constexpr (PAD) t.k[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (!PAD || 16 * j + 4 * g < p.head_dim) t.k[j] = *reinterpret_cast<const f32x4_t*>(kbase + ko + 16 * j + 4 * g);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        const int d = VEC * (16 * h + i16);
+        if constexpr (PAD) t.v[r][h] = fvec(0.f);
+        if (!PAD || d < p.head_dim) t.v[r][h] = *reinterpret_cast<const fvec*>(vbase + vo[r] + d);
+      }
+    if (++it[2] == nblk[2]) {
+      it[2] = 0;
+      if (++it[1] == nblk[1]) {
+        it[1] = 0;
+        ++it[0];
+      }
+    }
+  };
+  auto multiply = [&](const Block& t) {
+    f32x4_t S = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+      if (PAD && 16 * j >= p.head_dim) break;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) S = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[j][e], qf[j][e], S, 0, 0, 0);
+    }
+    if (!t.full) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        if (a < p.dims) {
+          const int lo = ws[a] - t.org[a];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[r] = uint32_t(vc[a][r] - lo) < uint32_t(width[a]) ? S[r] : -INFINITY;
+        }
+      }
+    }
+    const float mx_own = fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]));
+    if (__ballot(mx_own > m_run + kLazyRescaleLog2) != 0) {
+      float mx = fmaxf(mx_own, __shfl_xor(mx_own, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = fast_exp2(m_run - (m_new == -INFINITY ? 0.f : m_new));  // 0 while m_run is -inf
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) acc[h][c] *= alpha;
+    }
+    const float m_use = m_run == -INFINITY ? 0.f : m_run;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = fast_exp2(S[r] - m_use);
+    l_run += (S[0] + S[1]) + (S[2] + S[3]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) acc[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.v[r][h][c], S[r], acc[h][c], 0, 0, 0);
+  };
+
+  // two blocks in registers: while one is multiplied the other is on its way
+  Block A, B;
+  const int total = nblk[0] * nblk[1] * nblk[2];
+  load(A);
+  for (int n = 0; n < total; n += 2) {
+    if (n + 1 < total) load(B);
+    multiply(A);
+    if (n + 1 < total) {
+      if (n + 2 < total) load(A);
+      multiply(B);
+    }
+  }
+
+  float l = l_run + __shfl_xor(l_run, 16);
+  l += __shfl_xor(l, 32);
+  const float inv = (l > 0.f) ? 1.f / l : 0.f;
+  if (valid) {
+    float* orow = p.o + q_row * p.head_dim;
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int d = VEC * (16 * h + 4 * g + r);
+        fvec o;
+#pragma unroll
+        for (int c = 0; c < VEC; ++c) o[c] = acc[h][c][r] * inv;
+        if (!PAD || d < p.head_dim) *reinterpret_cast<fvec*>(orow + d) = o;
+      }
+    if (g == 0) p.lse[q_row] = (l > 0.f) ? (m_run * 0.6931471805599453f + logf(l)) : -INFINITY;
+  }
 }
 
 }  // namespace natten_amd

@@ -320,7 +320,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
 
 extern "C" {
 
-int natten_amd_abi_version(void) { return 17; }
+int natten_amd_abi_version(void) { return 18; }
 
 uint64_t natten_amd_fna_forward_workspace_bytes(void) { return uint64_t(kQueueWords) * 4; }
 
@@ -588,6 +588,92 @@ int natten_amd_fna_forward_fused(const void* q, const void* k, const void* v, vo
   return fna_forward_fused_impl(q, k, v, out, lse, dtype, na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape,
                                 kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape, scale, q_scale,
                                 k_scale, v_scale, anchor_kv_tiles, queues, stream);
+}
+
+int natten_amd_fna_forward_f32(const void* q, const void* k, const void* v, void* out, float* lse, int na_dim, int batch,
+                               int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
+                               const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
+                               const int32_t* is_causal, float scale, void* stream) {
+  g_error[0] = 0;
+  const char* what = "fna_forward_f32";
+  if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
+  if (!qkv_shape || !kernel_size || !stride || !dilation || !is_causal) return fail("%s: null shape argument", what);
+  if (head_dim < 8 || head_dim > 128 || head_dim % 8 != 0)
+    return fail("%s: head_dim must be a multiple of 8 from 8 to 128, got %d", what, head_dim);
+  if (int rc = check_common(what, q, k, v, out, lse, batch, 1, 1, heads_q, heads_kv, 32)) return rc;
+  FnaF32Params p;
+  memset(&p, 0, sizeof(p));
+  p.num_groups = 1;
+  p.dims = na_dim;
+  long long tokens = 1;
+  for (int a = 0; a < 3; ++a) {
+    const bool used = a < na_dim;
+    const int X = used ? qkv_shape[a] : 1;
+    p.ksize[a] = used ? kernel_size[a] : 1;
+    p.stride[a] = used ? stride[a] : 1;
+    p.dil[a] = used ? dilation[a] : 1;
+    p.causal[a] = used ? (is_causal[a] != 0) : 0;
+    if (X < 1 || p.dil[a] < 1 || p.stride[a] < 1 || (used && p.ksize[a] < 2))
+      return fail("%s: invalid parameter along dimension %d", what, a);
+    if ((long long)p.ksize[a] * p.dil[a] > X)
+      return fail("%s: kernel_size * dilation exceeds the input along dimension %d (%d * %d > %d)", what, a, p.ksize[a],
+                  p.dil[a], X);
+    if (p.stride[a] > p.ksize[a])
+      return fail("%s: stride exceeds kernel_size along dimension %d (%d > %d)", what, a, p.stride[a], p.ksize[a]);
+    p.ext_base[a] = X / p.dil[a];
+    p.ext_rem[a] = X % p.dil[a];
+    p.num_groups *= p.dil[a];
+    tokens *= X;
+    if (tokens > 0x7fffffffLL) return fail("%s: more than 2^31 tokens per batch", what);
+    p.d_stride[a] = na_make_div(p.stride[a]);
+    p.d_dil[a] = na_make_div(p.dil[a]);
+  }
+  p.tok_stride[2] = 1;
+  p.tok_stride[1] = na_dim > 2 ? qkv_shape[2] : 1;
+  p.tok_stride[0] = (na_dim > 1 ? qkv_shape[1] : 1) * p.tok_stride[1];
+  p.tokens = int(tokens);
+  p.q = static_cast<const float*>(q);
+  p.k = static_cast<const float*>(k);
+  p.v = static_cast<const float*>(v);
+  p.o = static_cast<float*>(out);
+  p.lse = lse;
+  p.heads_q = heads_q;
+  p.heads_kv = heads_kv;
+  p.head_dim = head_dim;
+  p.scale = scale;
+  choose_f32_boxes(p);
+  long long waves = (long long)batch * heads_q * p.num_groups;
+  p.num_boxes = 1;
+  for (int a = 0; a < 3; ++a) {
+    const int ext = p.ext_base[a] + (p.ext_rem[a] > 0);
+    p.q_boxes[a] = (ext + (1 << p.q_lg[a]) - 1) >> p.q_lg[a];
+    p.d_q_boxes[a] = na_make_div(p.q_boxes[a]);
+    p.num_boxes *= p.q_boxes[a];  // (at most the tokens of a batch entry)
+  }
+  waves *= p.num_boxes;
+  const long long wgs_per_xcd = (waves + 4 * kNumXcd - 1) / (4 * kNumXcd);
+  if (waves > 0x7fffff00LL) return fail("%s: problem needs more than 2^31 waves", what);
+  p.waves = int(waves);
+  p.wgs_per_xcd = int(wgs_per_xcd);
+  p.d_boxes = na_make_div(p.num_boxes);
+  p.d_heads_q = na_make_div(heads_q);
+  p.d_q_per_kv = na_make_div(heads_q / heads_kv);
+  p.d_num_groups = na_make_div(p.num_groups);
+  const dim3 grid((unsigned)(wgs_per_xcd * kNumXcd));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (head_dim) {
+    case 32: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, false>), grid, dim3(256), 0, s, p); break;
+    case 64: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, false>), grid, dim3(256), 0, s, p); break;
+    case 128: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, false>), grid, dim3(256), 0, s, p); break;
+    default:
+      if (head_dim < 32)
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, true>), grid, dim3(256), 0, s, p);
+      else if (head_dim < 64)
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, true>), grid, dim3(256), 0, s, p);
+      else
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, true>), grid, dim3(256), 0, s, p);
+  }
+  return check_launch(what);
 }
 
 int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void* v, void* out_parts, float* lse_parts,

@@ -145,6 +145,10 @@ def amd_fna_generic(
         kernel_size, stride, dilation, is_causal = check_all_args(na_dim, kernel_size, stride, dilation, is_causal)
         check_args_against_input(query, kernel_size, stride, dilation, is_causal)
     can_run_amd_fna(query, key, value, raise_error=True)
+    # float32 on the original tensors, in one launch with boxes of its own: unless the caller fixed tile
+    # shapes or a route, which the kernel on permuted sequences serves (2x64x64 tokens, H 8, D 64,
+    # 13 x 13 windows: 62 us here, 300 us there; 256 tokens, H 2, D 32, window 7: 23 and 83 us)
+    f32_direct = query.dtype == torch.float32 and fused is None and anchored_tiles and q_tile_shape is None
     q_tile_shape, kv_tile_shape = check_fna_forward_config(
         query, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape
     )
@@ -169,7 +173,7 @@ def amd_fna_generic(
         if out_dtype is not None and output.dtype != out_dtype:
             output = output.to(out_dtype)
         return (output, lse) if return_lse else output
-    if d_pad != head_dim:
+    if d_pad != head_dim and not f32_direct:
         # zero columns change neither q.k nor the first head_dim output columns
         query, key, value = (_pad_head_dim(t, d_pad) for t in (query, key, value))
 
@@ -215,6 +219,12 @@ def amd_fna_generic(
             "natten_amd: kv_splits > 1 needs the one-launch path, fp16 / bf16 operands without dequantisation scales "
             f"and tiles of 128 x 64 tokens (and no graph tracing); got {in_dtype}, {q_tile_shape=}, {kv_tile_shape=}, {fused=}."
         )
+    if f32_direct:
+        output, lse = torch_ops.fna_forward_f32(
+            query.contiguous(), key.contiguous(), value.contiguous(), kernel_size, stride, dilation, is_causal, scale)
+        if out_dtype is not None and out_dtype != in_dtype:
+            output = output.to(out_dtype)
+        return (output, lse) if return_lse else output
     if fusable and fused is not False:
         if kv_splits > 1:
             out_parts, lse_parts = _lib.fna_forward_fused_split(

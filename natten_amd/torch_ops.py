@@ -59,6 +59,19 @@ def _(q, k, v, kernel_size, stride, dilation, is_causal, scale, q_tile_shape, kv
     return q.new_empty(q.shape, dtype=_out_dtype(q)), q.new_empty(q.shape[:-1], dtype=torch.float32)
 
 
+@torch.library.custom_op("natten_amd::fna_forward_f32", mutates_args=(), device_types="cuda")
+def _fna_forward_f32_op(
+    q: Tensor, k: Tensor, v: Tensor, kernel_size: List[int], stride: List[int], dilation: List[int],
+    is_causal: List[bool], scale: float,
+) -> Tuple[Tensor, Tensor]:
+    return _lib.fna_forward_f32(q, k, v, kernel_size, stride, dilation, is_causal, scale)
+
+
+@_fna_forward_f32_op.register_fake
+def _(q, k, v, kernel_size, stride, dilation, is_causal, scale):
+    return torch.empty_like(q), q.new_empty(q.shape[:-1], dtype=torch.float32)
+
+
 @torch.library.custom_op("natten_amd::attention_forward", mutates_args=(), device_types="cuda")
 def _attention_forward_op(
     q: Tensor, k: Tensor, v: Tensor, is_causal: bool, scale: float, q_scale: Optional[Tensor],
@@ -233,6 +246,13 @@ def fna_forward_fused(q, k, v, kernel_size, stride, dilation, is_causal, scale, 
     return _lib.fna_forward_fused(q, k, v, kernel_size, stride, dilation, is_causal, scale, q_tile_shape, kv_tile_shape,
                                   q_scale=q_scale, k_scale=k_scale, v_scale=v_scale, run_persistent=run_persistent,
                                   anchored_tiles=anchored_tiles)
+
+
+def fna_forward_f32(q, k, v, kernel_size, stride, dilation, is_causal, scale):
+    if _tracing():
+        return _fna_forward_f32_op(q, k, v, _ints(kernel_size), _ints(stride), _ints(dilation),
+                                   [bool(c) for c in is_causal], float(scale))
+    return _lib.fna_forward_f32(q, k, v, kernel_size, stride, dilation, is_causal, scale)
 
 
 def attention_forward(q, k, v, is_causal, scale, q_scale=None, k_scale=None, v_scale=None):
