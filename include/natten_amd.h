@@ -136,7 +136,9 @@ int natten_amd_fna_forward(const void* q, const void* k, const void* v, void* ou
  *     of 128 x 64 tokens only (the instance that clamps its gathers).
  * Anything else returns an error that says which rule was missed, and the caller uses the
  * permuted path.  A KV tile must span less than 2^31 bytes of the input.  dtype, tiles, head_dim,
- * scales, run_persistent and workspace as in natten_amd_fna_forward.
+ * scales, run_persistent and workspace as in natten_amd_fna_forward; fp16 / bf16 operands with tiles of
+ * 128 x 64 tokens and run_persistent == 0 also take the multiples of 8 between 32 and 128 as head_dim
+ * (the bits are those of rows padded with zeros to 64 or 128).
  *
  * anchor_kv_tiles != 0: the KV tiles of a Q tile are laid out from the first key of its window
  * box (per dimension) instead of from multiples of the KV tile extent -- there is no permuted
@@ -273,6 +275,7 @@ int natten_amd_fna_supported_tiles(int dtype, int head_dim, int32_t* q_sizes, in
  * Dense attention forward (optional top-left causal mask) on unpermuted operands.
  *   q [batch, seqlen_q, heads_q, head_dim], k/v [batch, seqlen_kv, heads_kv, head_dim],
  *   out like q, lse [batch, seqlen_q, heads_q] float32.  Any seqlen >= 1.
+ * head_dim 32, 64, 128 or a multiple of 8 between 32 and 128.
  * q_scale / k_scale / v_scale as in natten_amd_fna_forward.
  */
 int natten_amd_attention_forward(const void* q, const void* k, const void* v, void* out,

@@ -338,6 +338,14 @@ def fused_layout_supported(qkv_shape, dilation, kv_tile_shape, row_bytes: int = 
     return q_tokens == 128 and kv_tokens == 64
 
 
+def _aligned_narrow_rows(q: Tensor, k: Tensor, v: Tensor):
+    """Operands of a head dim between the native ones, on sixteen-byte boundaries (at native head dims the
+    library refuses operands that are not; these used to be padded, which aligned them)."""
+    if q.shape[-1] in (32, 64, 128):
+        return q, k, v
+    return tuple(t if t.data_ptr() % 16 == 0 else t.clone() for t in (q, k, v))
+
+
 def fna_forward_fused(
     q: Tensor, k: Tensor, v: Tensor,
     kernel_size, stride, dilation, is_causal, scale: float, q_tile_shape, kv_tile_shape,
@@ -351,6 +359,7 @@ def fna_forward_fused(
     _require_gpu(q, k, v)
     if q.dtype not in (torch.float16, torch.bfloat16) + FP8_DTYPES:
         raise NotImplementedError(f"natten_amd fna_forward_fused does not support {q.dtype}.")
+    q, k, v = _aligned_narrow_rows(q, k, v)
     na_dim = len(kernel_size)
     qkv_shape = [int(x) for x in q.shape[1 : 1 + na_dim]]
     scales = _scale_ptrs(q, k, q_scale, k_scale, v_scale)
@@ -459,6 +468,7 @@ def attention_forward(
     _require_gpu(q, k, v)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_forward does not support {q.dtype}.")
+    q, k, v = _aligned_narrow_rows(q, k, v)
     scales = _scale_ptrs(q, k, q_scale, k_scale, v_scale)
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)

@@ -37,6 +37,7 @@ struct FnaParams {
   void* o;
   float* lse;
   int batch, heads_q, heads_kv;
+  int row_dim;              // instances for narrow rows (DC != 0): elements of an operand row in memory
   int seqlen_q, seqlen_kv;  // rows of the (permuted) sequences
   int num_groups;           // prod(dilation)
   int qkv_shape[3];         // original token layout
@@ -406,16 +407,25 @@ struct FnaSmem {
 // NOMASK: the launch is fully block-sparse (the host has checked that every KV tile a Q tile visits is
 // attended in full by every query of that Q tile: reference fna_fusion.hpp:503-593); the instance then
 // holds no mask code, tables or per-wave windows at all.
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, typename Hook>
+// DC != 0: the operands' rows hold row_dim <= DC <= D elements (a multiple of 8) instead of D, and DC (a
+// multiple of 32) of the D columns that the tiles have room for are multiplied: head dims between
+// the native ones on the tensors as they are, where padded copies of q, k and v and a slice of the
+// result cost more than the attention itself (2x64x64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context
+// tokens: the call takes 76 us instead of 139 with its ten copies and fills).  The chunks past a row are not
+// fetched: their places in the tiles are zeroed once, before the first copy.
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
+          typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
   const int split = SPLIT ? pid_in / p.split_grid : 0;
   const int pid = SPLIT ? pid_in - split * p.split_grid : pid_in;
   constexpr int NT = NWAVES * 64;
   constexpr int QT = NWAVES * MQ * 32;
-  constexpr int KSTEPS = D / 16;
-  constexpr int DB = D / 32;
+  constexpr bool NARROW = DC != 0;
+  constexpr int KSTEPS = (NARROW ? DC : D) / 16;
+  constexpr int DB = (NARROW ? DC : D) / 32;
   constexpr int NSB = KVT / 32;
+  const int row_dim = NARROW ? p.row_dim : D;
   using L = FnaSmem<D, KVT>;
   constexpr int ROWB = L::ROWB;
   constexpr int CPR = L::CPR;
@@ -625,15 +635,26 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
   }
 
-  const int64_t q_row_stride = int64_t(p.heads_q) * D;
-  const int64_t kv_row_stride = int64_t(p.heads_kv) * D;
+  const int64_t q_row_stride = int64_t(p.heads_q) * row_dim;
+  const int64_t kv_row_stride = int64_t(p.heads_kv) * row_dim;
   // first row of this (batch, dilation group): rows are then addressed by permuted row index
   // (permuted layout) or by token offset inside the group (fused layout)
   const int64_t q_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : q_seq_row0;
   const int64_t kv_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : kv_seq_row0;
-  const T* qbase = reinterpret_cast<const T*>(p.q) + q_row_base * q_row_stride + int64_t(head) * D;
-  const T* kbase = reinterpret_cast<const T*>(p.k) + kv_row_base * kv_row_stride + int64_t(head_kv) * D;
-  const T* vbase = reinterpret_cast<const T*>(p.v) + kv_row_base * kv_row_stride + int64_t(head_kv) * D;
+  const T* qbase = reinterpret_cast<const T*>(p.q) + q_row_base * q_row_stride + int64_t(head) * row_dim;
+  const T* kbase = reinterpret_cast<const T*>(p.k) + kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim;
+  const T* vbase = reinterpret_cast<const T*>(p.v) + kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim;
+  if constexpr (NARROW) {
+    // (every copy leaves out the same places, so this is needed once)
+    for (int i = tid; i < TILE_BYTES / 16; i += NT) {
+      const u32x4_t zero = {0, 0, 0, 0};
+      reinterpret_cast<u32x4_t*>(sK0)[i] = zero;
+      reinterpret_cast<u32x4_t*>(sV0)[i] = zero;
+      reinterpret_cast<u32x4_t*>(sK1)[i] = zero;
+      reinterpret_cast<u32x4_t*>(sV1)[i] = zero;
+    }
+    workgroup_sync();
+  }
   // row (permuted) or token offset (fused) of position `r` (dimension 0 fastest) of a KV tile
   auto kv_tile_pos = [&](int r) {
     if (!p.fused) return r;
@@ -741,7 +762,15 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           // off the uniform base instead
           src -= IMM;
         }
-        async_copy16_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096));
+        if constexpr (NARROW) {
+          // lanes whose chunk lies past the row sit out (a copy covers whole tile rows, so every wave
+          // still issues it and the counted waits hold); a lane's place in LDS follows from its number
+          const int P = (wave * PER + I) * 64 + lane;
+          const int chunk = V_LAYOUT ? L::v_slot(P / CPR, P % CPR) : L::k_slot(P / CPR, P % CPR);
+          if (chunk * 8 < row_dim) async_copy16_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096));
+        } else {
+          async_copy16_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096));
+        }
       }
     }
   };
@@ -872,7 +901,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const T* qrow = qbase + int64_t(row_c) * q_row_stride + g * 8;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      const vec8 raw = *reinterpret_cast<const vec8*>(qrow + ks * 16);
+      vec8 raw = {};
+      if (!NARROW || ks * 16 + g * 8 < row_dim) raw = *reinterpret_cast<const vec8*>(qrow + ks * 16);
       // The query row carries the softmax scale (in the exp2 domain) into the matrix product, so
       // that the logits leave the matrix pipe ready for exp2: q' = round(q * scale * log2(e)).
       // Rounding q' to the operand type moves a logit by about 2^-9 (bf16) / 2^-12 (fp16) of
@@ -1285,7 +1315,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   before_stores();
 
   // ---- epilogue: O = acc / rowsum, LSE = ln(rowsum) + scale * rowmax -------------------------
-  T* obase = reinterpret_cast<T*>(p.o) + q_row_base * q_row_stride + int64_t(head) * D;
+  T* obase = reinterpret_cast<T*>(p.o) + q_row_base * q_row_stride + int64_t(head) * row_dim;
   float* lse_base = p.lse;
   if constexpr (SPLIT) {
     obase += split * p.o_split_stride;
@@ -1306,7 +1336,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           tx4 o4;
 #pragma unroll
           for (int i = 0; i < 4; ++i) o4[i] = static_cast<T>(acc[mb][db][4 * j + i] * inv);
-          *reinterpret_cast<tx4*>(orow + db * 32 + 8 * j + 4 * g) = o4;
+          if (!NARROW || db * 32 + 8 * j < row_dim) *reinterpret_cast<tx4*>(orow + db * 32 + 8 * j + 4 * g) = o4;
         }
       if (g == 0) {
         const float lse = (l > 0.f) ? (m_run[mb] * 0.6931471805599453f + __logf(l)) : -INFINITY;
@@ -1316,10 +1346,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
 }
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false>
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
 __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
 fna_fwd_kernel(const FnaParams p) {
-  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC>(p, int(blockIdx.x), []() {});
 }
 
 // Split launch: kv_splits workgroups per Q tile, each on a contiguous run of the tile's KV tiles,

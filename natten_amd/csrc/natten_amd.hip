@@ -77,6 +77,9 @@ int resident_workgroups() {
   return n;
 }
 
+// Head dims whose rows the 128 x 64 forward instances take as they are, besides 32, 64 and 128
+bool narrow_rows(int head_dim) { return head_dim > 32 && head_dim < 128 && head_dim != 64 && head_dim % 8 == 0; }
+
 // The counters of a work-queue launch (null: one workgroup per Q tile).  Every work-queue kernel
 // leaves the counters at zero when its last workgroup ends; `clear_first` clears them by a kernel
 // before the launch, for memory whose contents are not known.
@@ -85,37 +88,44 @@ struct WorkQueue {
   bool clear_first = true;
 };
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false>
+// DC != 0: rows of p.row_dim elements, DC columns multiplied (a workgroup per Q tile only)
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
 int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   constexpr int QT = NWAVES * MQ * 32;
   if (!fna_tiles_are_powers_of_two(p)) return fail("fna_forward: tile extents must be powers of two");
   if ((p.seqlen_q + QT - 1) / QT != p.num_q_tiles) return fail("fna_forward: internal tile count mismatch");
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
   if (wgs > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
-  if (queues.counters != nullptr) {
-    const long long resident = resident_workgroups();
-    if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
-    hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>),
-                       dim3((unsigned)(wgs < resident ? wgs : resident)), dim3(NWAVES * 64), 0, stream, p, queues.counters,
-                       int(wgs / kNumXcd));
-    return check_launch("fna_forward (work queue)");
-  }
-  if (p.kv_splits > 1) {
-    // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
-    if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64) {
-      if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
-      FnaParams ps = p;
-      ps.split_grid = int(wgs);
-      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT>), dim3((unsigned)(wgs * p.kv_splits)),
-                         dim3(NWAVES * 64), 0, stream, ps);
-      return check_launch("fna_forward (split)");
-    } else {
-      return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
+  if constexpr (DC != 0) {
+    hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
+                       stream, p);
+    return check_launch("fna_forward (narrow rows)");
+  } else {
+    if (queues.counters != nullptr) {
+      const long long resident = resident_workgroups();
+      if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
+      hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>),
+                         dim3((unsigned)(wgs < resident ? wgs : resident)), dim3(NWAVES * 64), 0, stream, p, queues.counters,
+                         int(wgs / kNumXcd));
+      return check_launch("fna_forward (work queue)");
     }
+    if (p.kv_splits > 1) {
+      // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
+      if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64) {
+        if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
+        FnaParams ps = p;
+        ps.split_grid = int(wgs);
+        hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT>), dim3((unsigned)(wgs * p.kv_splits)),
+                           dim3(NWAVES * 64), 0, stream, ps);
+        return check_launch("fna_forward (split)");
+      } else {
+        return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
+      }
+    }
+    hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0, stream,
+                       p);
+    return check_launch("fna_forward");
   }
-  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0, stream,
-                     p);
-  return check_launch("fna_forward");
 }
 
 // Whether the launch is fully block-sparse: every Q tile is whole (no padding queries), all its
@@ -188,6 +198,15 @@ int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, Work
   return fail("fna_forward: no kernel for Q tile of %d and KV tile of %d tokens", qt, kvt);
 }
 
+// Head dims between the native ones (multiples of 8 above 32).  Up to 96 of 128 columns are multiplied as
+// 96: a quarter of the matrix work and of the LDS reads less.
+template <typename T, bool RAGGED>
+int dispatch_narrow_rows(const FnaParams& p, int head_dim, hipStream_t stream) {
+  if (head_dim < 64) return launch_fna<T, 64, 4, 1, RAGGED, 64, false, 64>(p, stream);
+  if (head_dim <= 96) return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 96>(p, stream);
+  return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 128>(p, stream);
+}
+
 template <typename T>
 int dispatch_head_dim(const FnaParams& p, int head_dim, int qt, int kvt, hipStream_t stream, WorkQueue queues) {
   switch (head_dim) {
@@ -195,7 +214,11 @@ int dispatch_head_dim(const FnaParams& p, int head_dim, int qt, int kvt, hipStre
     case 64: return dispatch_tiles<T, 64>(p, qt, kvt, stream, queues);
     case 128: return dispatch_tiles<T, 128>(p, qt, kvt, stream, queues);
   }
-  return fail("fna_forward: head_dim must be 32, 64 or 128, got %d", head_dim);
+  if (!narrow_rows(head_dim)) return fail("fna_forward: head_dim must be 32, 64 or 128, got %d", head_dim);
+  if (qt != 128 || kvt != 64 || queues.counters != nullptr || p.kv_splits > 1 || p.cu_q != nullptr || p.row_dim != head_dim)
+    return fail("fna_forward: head_dim %d needs tiles of 128 x 64 tokens and a workgroup per Q tile", head_dim);
+  if (p.seqlen_kv % kvt != 0 || p.edge == 2) return dispatch_narrow_rows<T, true>(p, head_dim, stream);
+  return dispatch_narrow_rows<T, false>(p, head_dim, stream);
 }
 
 int dispatch_dtype(const FnaParams& p, int dtype, int head_dim, int qt, int kvt, hipStream_t stream,
@@ -242,13 +265,13 @@ int dispatch_dtype(const FnaParams& p, int dtype, int head_dim, int qt, int kvt,
 }
 
 int check_common(const char* what, const void* q, const void* k, const void* v, const void* out, const float* lse,
-                 int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim) {
+                 int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim, bool narrow_ok = false) {
   if (!q || !k || !v || !out || !lse) return fail("%s: null pointer argument", what);
   if (batch < 1 || seqlen_q < 1 || seqlen_kv < 1 || heads_q < 1 || heads_kv < 1)
     return fail("%s: batch, sequence lengths and head counts must be positive", what);
   if (heads_q % heads_kv != 0)
     return fail("%s: heads_kv (%d) must divide heads_q (%d)", what, heads_kv, heads_q);
-  if (head_dim != 32 && head_dim != 64 && head_dim != 128)
+  if (head_dim != 32 && head_dim != 64 && head_dim != 128 && !(narrow_ok && narrow_rows(head_dim)))
     return fail("%s: head_dim must be 32, 64 or 128, got %d", what, head_dim);
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v) |
        reinterpret_cast<uintptr_t>(out)) & 15)
@@ -549,7 +572,7 @@ int fna_forward_fused_impl(const void* q, const void* k, const void* v, void* ou
                               anchor_kv_tiles, &tokens))
     return rc;
   if (int rc = check_common("fna_forward_fused", q, k, v, out, lse, batch, p.seqlen_q, p.seqlen_kv, heads_q, heads_kv,
-                            head_dim))
+                            head_dim, dtype == NATTEN_AMD_F16 || dtype == NATTEN_AMD_BF16))
     return rc;
   p.q = q;
   p.k = k;
@@ -559,6 +582,7 @@ int fna_forward_fused_impl(const void* q, const void* k, const void* v, void* ou
   p.batch = batch * p.num_groups;
   p.heads_q = heads_q;
   p.heads_kv = heads_kv;
+  p.row_dim = head_dim;
   p.scale = scale;
   p.q_scale = q_scale;
   p.k_scale = k_scale;
@@ -772,7 +796,7 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
                                  const float* v_scale, void* stream) {
   g_error[0] = 0;
   if (int rc = check_common("attention_forward", q, k, v, out, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv,
-                            head_dim))
+                            head_dim, dtype == NATTEN_AMD_F16 || dtype == NATTEN_AMD_BF16))
     return rc;
   // Dense attention is the 1-D neighborhood problem whose window is the whole key sequence:
   // non-causal windows are [0, seqlen_kv), causal ones [0, min(i + 1, seqlen_kv)).
@@ -802,6 +826,7 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
   p.lse = lse;
   p.batch = batch;
   p.heads_q = heads_q;
+  p.row_dim = head_dim;
   p.heads_kv = heads_kv;
   p.seqlen_q = seqlen_q;
   p.seqlen_kv = seqlen_kv;

@@ -12,7 +12,7 @@ from torch import Tensor
 from . import _lib, torch_ops
 from .checks import fmha_tensor_checks
 from .fna import SUPPORTED_DTYPES, is_fp8, pad_head_dim, resolve_scale
-from .tile_config import padded_head_dim
+from .tile_config import padded_head_dim, takes_narrow_rows
 
 
 def amd_fmha(
@@ -57,6 +57,8 @@ def amd_fmha(
         if out_dtype is not None and out.dtype != out_dtype:
             out = out.to(out_dtype)
         return (out, lse) if return_lse else out
+    if cumulative_seqlen_Q is None and takes_narrow_rows(head_dim, query.dtype):
+        d_pad = head_dim
     q, k, v = (pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value))
     if is_fp8(query.dtype):
         # a one-token tile with no dilation is the identity permutation: a plain widening copy

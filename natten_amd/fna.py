@@ -15,7 +15,7 @@ from torch import Tensor
 
 from . import _lib, torch_ops
 from .checks import check_all_args, check_args_against_input, na_tensor_checks
-from .tile_config import check_fna_backward_config, check_fna_forward_config, padded_head_dim
+from .tile_config import check_fna_backward_config, check_fna_forward_config, padded_head_dim, takes_narrow_rows
 from .token_permute import token_permute_operation, token_unpermute_operation
 
 SUPPORTED_DTYPES = (torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.float8_e5m2)
@@ -155,7 +155,11 @@ def amd_fna_generic(
     head_dim = query.shape[-1]
     scale = scale or head_dim**-0.5
     d_pad = padded_head_dim(head_dim)
-    if run_persistent_kernel is None:
+    # rows narrower than the kernels' are read as they are by a workgroup per Q tile of the default tiles; a
+    # work-queue or split launch that the caller asks for takes padded copies
+    narrow = (takes_narrow_rows(head_dim, query.dtype) and fused is not False and not run_persistent_kernel
+              and kv_splits in (None, 1) and _prod(q_tile_shape) == 128 and _prod(kv_tile_shape) == 64)
+    if run_persistent_kernel is None and not narrow:
         from .functional import work_queue_default
 
         run_persistent_kernel = work_queue_default(
@@ -173,10 +177,6 @@ def amd_fna_generic(
         if out_dtype is not None and output.dtype != out_dtype:
             output = output.to(out_dtype)
         return (output, lse) if return_lse else output
-    if d_pad != head_dim and not f32_direct:
-        # zero columns change neither q.k nor the first head_dim output columns
-        query, key, value = (_pad_head_dim(t, d_pad) for t in (query, key, value))
-
     in_dtype = query.dtype
     if in_dtype == torch.float32 and not (q_scale is None and k_scale is None and v_scale is None):
         raise ValueError("natten_amd: dequantisation scales belong to 8- and 16-bit operands; float32 operands take none.")
@@ -206,12 +206,13 @@ def amd_fna_generic(
         and q_scale is None and k_scale is None and v_scale is None
         and _prod(q_tile_shape) == 128 and _prod(kv_tile_shape) == 64 and not torch_ops._tracing()
     )
+    narrow = narrow and fusable
     if kv_splits is None:
         from .functional import kv_splits_default
 
         kv_splits = kv_splits_default(
             query.shape[0], query.shape[-2], query.shape[1 : 1 + na_dim], kernel_size, stride, dilation, is_causal,
-            q_tile_shape, kv_tile_shape) if (splittable and anchored_tiles and not run_persistent_kernel) else 1
+            q_tile_shape, kv_tile_shape) if (splittable and anchored_tiles and not run_persistent_kernel and not narrow) else 1
     if not isinstance(kv_splits, int) or not 1 <= kv_splits <= 8:
         raise ValueError(f"natten_amd: kv_splits must be an integer from 1 to 8, got {kv_splits!r}.")
     if kv_splits > 1 and not splittable:
@@ -219,6 +220,9 @@ def amd_fna_generic(
             "natten_amd: kv_splits > 1 needs the one-launch path, fp16 / bf16 operands without dequantisation scales "
             f"and tiles of 128 x 64 tokens (and no graph tracing); got {in_dtype}, {q_tile_shape=}, {kv_tile_shape=}, {fused=}."
         )
+    if d_pad != head_dim and not f32_direct and not narrow:
+        # zero columns change neither q.k nor the first head_dim output columns
+        query, key, value = (_pad_head_dim(t, d_pad) for t in (query, key, value))
     if f32_direct:
         output, lse = torch_ops.fna_forward_f32(
             query.contiguous(), key.contiguous(), value.contiguous(), kernel_size, stride, dilation, is_causal, scale)
@@ -241,7 +245,7 @@ def amd_fna_generic(
                 v_scale=resolve_scale(v_scale, key.shape[-2], query.device, "v_scale"),
                 run_persistent=bool(run_persistent_kernel), anchored_tiles=bool(anchored_tiles),
             )
-        if d_pad != head_dim:
+        if output.shape[-1] != head_dim:
             output = output[..., :head_dim].contiguous()
         out_dtype = out_dtype or in_dtype
         if output.dtype != out_dtype:

@@ -23,6 +23,12 @@ TILE_SIZES: List[Tuple[int, int]] = [(128, 64), (256, 64), (64, 64)]
 SUPPORTED_HEAD_DIMS = (32, 64, 128)
 
 
+def takes_narrow_rows(head_dim: int, dtype: torch.dtype) -> bool:
+    """Head dims between the native ones that the 128 x 64 forward kernels take as they are (below 32 a
+    quarter of a tile row and less would be data: those are padded)."""
+    return dtype in (torch.float16, torch.bfloat16) and 32 < head_dim < 128 and head_dim != 64 and head_dim % 8 == 0
+
+
 def padded_head_dim(head_dim: int) -> int:
     for d in SUPPORTED_HEAD_DIMS:
         if head_dim <= d:
