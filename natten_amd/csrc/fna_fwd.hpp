@@ -65,6 +65,8 @@ struct FnaParams {
   // dimension; such a tile is then gathered from where it ends at the group's last position, and its
   // leading keys (which the tile before it already delivered) are masked.  2: the RAGGED instance,
   // which gathers the tile where it is and clamps the rows that fall outside the group.
+  // fused == 0: 1 for dense attention on a sequence of at least a KV tile that no KV tile divides, whose
+  // last tile is moved back the same way; 0 otherwise.
   int edge;
   // fused == 1 only: KV tiles are laid out from the first key of the Q tile's window box (per
   // dimension) instead of from multiples of the tile extent, which saves the part of a tile that
@@ -825,7 +827,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const int row0_permuted = (((box_org[0] >> p.kv_tile_lg[0]) + itc[0]) +
                                p.kv_tiled[0] * (((box_org[1] >> p.kv_tile_lg[1]) + itc[1]) +
                                                 p.kv_tiled[1] * ((box_org[2] >> p.kv_tile_lg[2]) + itc[2]))) * KVT;
-    t.row0 = p.fused ? row0_fused : row0_permuted;
+    t.row0 = p.fused ? row0_fused : row0_permuted - t.lead[0];  // (only a dense sequence's last tile is moved back there)
     if (++itc[2] == box_n[2]) {
       itc[2] = 0;
       if (++itc[1] == box_n[1]) {
