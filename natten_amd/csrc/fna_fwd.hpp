@@ -799,6 +799,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     bool skip;      // no key of the tile is attended by any query of this wave
     int lead[3];    // a tile moved back from the group's edge: its first lead[a] positions belong to the tile before it
   };
+  // (a packed sequence sums in the order in which a dense call on it alone does)
+  const bool move_back = p.edge == 1 || p.anchor || (RAGGED && p.cu_q != nullptr && seqlen_kv >= KVT);
   int itc[3] = {0, 0, 0};
   if constexpr (SPLIT) {
     itc[2] = first_tile % box_n[2];
@@ -819,7 +821,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
         t.skip = t.skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
       }
       // a tile that would reach past the group is moved back to end at the group's last position
-      t.origin[a] = (p.edge == 1 || p.anchor) ? na_min(org, extent[a] - p.kv_tile[a]) : org;
+      t.origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
       t.lead[a] = org - t.origin[a];
     }
     // (both forms are a handful of scalar operations: computed side by side and selected, a branch costs more)
