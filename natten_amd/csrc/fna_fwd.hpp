@@ -1570,6 +1570,39 @@ inline void choose_wave_box(FnaParams& p) {
   for (int a = 0; a < 3; ++a) last_box[a] = p.wave_box_lg[a];
 }
 
+// Few groups: the XCDs' shares differ by whole groups, and a short last group per (batch, head) pair can
+// meet the same XCDs every time (8 heads of 65 + 20 tiles: 130 on every other XCD, 40 on the rest).
+// Equal groups, and as many of them per pair as even the shares out: the fewest within a twentieth of
+// the best, at most four times as many (smaller groups share less of their keys in an L2).  From 16 groups an
+// XCD on the shares differ by less than that and the groups stay as they are.
+inline void balance_wg_groups(FnaParams& p, int units, long long bh) {
+  auto largest_share = [&](int per_pair, int size) {
+    long long share[kNumXcd] = {}, most = 0;
+    for (long long g = 0; g < bh * per_pair; ++g)
+      share[g % kNumXcd] += na_min(size, units - int(g % per_pair) * size);
+    for (long long s : share) most = s > most ? s : most;
+    return most;
+  };
+  const int now = (units + p.wg_group - 1) / p.wg_group;
+  if (bh * now >= 16 * kNumXcd) return;
+  const double even = double(bh) * units / kNumXcd;
+  if (largest_share(now, p.wg_group) <= 1.05 * even) return;
+  int size[4 * 16 * kNumXcd + 1];  // by groups per pair
+  long long best = -1;
+  const int most = na_min(4 * now, units);
+  long long share[4 * 16 * kNumXcd + 1];
+  for (int n = now; n <= most; ++n) {
+    size[n] = (units + n - 1) / n;
+    share[n] = (units + size[n] - 1) / size[n] == n ? largest_share(n, size[n]) : -1;
+    if (share[n] >= 0 && (best < 0 || share[n] < best)) best = share[n];
+  }
+  for (int n = now; n <= most; ++n)
+    if (share[n] >= 0 && share[n] <= 1.05 * best) {
+      if (share[n] < largest_share(now, p.wg_group)) p.wg_group = size[n];
+      return;
+    }
+}
+
 inline void set_wg_layout(FnaParams& p, int tiles_per_wg = 1) {
   p.num_q_tiles = p.q_tiled[0] * p.q_tiled[1] * p.q_tiled[2];
   const int slab = p.q_tiled[1] * p.q_tiled[2];
@@ -1587,6 +1620,7 @@ inline void set_wg_layout(FnaParams& p, int tiles_per_wg = 1) {
     if (want > units) want = units;
     p.wg_group = (units + want - 1) / want;
   }
+  balance_wg_groups(p, units, bh);
   p.groups_per_bh = (units + p.wg_group - 1) / p.wg_group;
   p.total_groups = p.batch * p.heads_q * p.groups_per_bh;
   // what the kernels' set-up would otherwise divide for (every forward launch comes through here)
