@@ -1350,8 +1350,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
 }
 
+// Head dim 32 needs 153 registers: three waves per SIMD, which an upper bound of two would keep it from.
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
+__global__ void __launch_bounds__(NWAVES * 64)
+    __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? (D == 32 ? 3 : 2) : 1)))
 fna_fwd_kernel(const FnaParams p) {
   fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC>(p, int(blockIdx.x), []() {});
 }

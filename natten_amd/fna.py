@@ -15,7 +15,13 @@ from torch import Tensor
 
 from . import _lib, torch_ops
 from .checks import check_all_args, check_args_against_input, na_tensor_checks
-from .tile_config import check_fna_backward_config, check_fna_forward_config, padded_head_dim, takes_narrow_rows
+from .tile_config import (
+    check_fna_backward_config,
+    check_fna_forward_config,
+    choose_small_forward_tiles,
+    padded_head_dim,
+    takes_narrow_rows,
+)
 from .token_permute import token_permute_operation, token_unpermute_operation
 
 SUPPORTED_DTYPES = (torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.float8_e5m2)
@@ -148,7 +154,8 @@ def amd_fna_generic(
     # float32 on the original tensors, in one launch with boxes of its own: unless the caller fixed tile
     # shapes or a route, which the kernel on permuted sequences serves (2x64x64 tokens, H 8, D 64,
     # 13 x 13 windows: 62 us here, 300 us there; 256 tokens, H 2, D 32, window 7: 23 and 83 us)
-    f32_direct = query.dtype == torch.float32 and fused is None and anchored_tiles and q_tile_shape is None
+    own_tiles = q_tile_shape is None
+    f32_direct = query.dtype == torch.float32 and fused is None and anchored_tiles and own_tiles
     q_tile_shape, kv_tile_shape = check_fna_forward_config(
         query, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape
     )
@@ -159,12 +166,21 @@ def amd_fna_generic(
     # work-queue or split launch that the caller asks for takes padded copies
     narrow = (takes_narrow_rows(head_dim, query.dtype) and fused is not False and not run_persistent_kernel
               and kv_splits in (None, 1) and _prod(q_tile_shape) == 128 and _prod(kv_tile_shape) == 64)
-    if run_persistent_kernel is None and not narrow:
+    launch_left_open = run_persistent_kernel is None  # (the launch kinds promise each other's bits, hence tiles)
+    if launch_left_open and not narrow:
         from .functional import work_queue_default
 
         run_persistent_kernel = work_queue_default(
             query.shape[0], query.shape[-2], query.shape[1 : 1 + na_dim], kernel_size, stride, dilation, is_causal,
             q_tile_shape, kv_tile_shape)
+    if (own_tiles and launch_left_open and d_pad <= 64 and not narrow and not run_persistent_kernel and fused is None
+            and anchored_tiles and kv_splits is None and query.dtype in (torch.float16, torch.bfloat16)):
+        from .functional import kv_splits_default
+
+        problem = (query.shape[1 : 1 + na_dim], kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape)
+        small = choose_small_forward_tiles(*problem)
+        if small is not None and kv_splits_default(query.shape[0], query.shape[-2], *problem) == 1:
+            q_tile_shape, kv_tile_shape = small
     if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad):
         bwd_q_tile, bwd_kv_tile = check_fna_backward_config(
             query, kernel_size, stride, dilation, is_causal, backward_q_tile_shape, backward_kv_tile_shape

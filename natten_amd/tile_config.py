@@ -21,6 +21,7 @@ DimensionType = Tuple[int, ...]
 # (Q tile tokens, KV tile tokens) with a kernel instance; first entry = default.
 TILE_SIZES: List[Tuple[int, int]] = [(128, 64), (256, 64), (64, 64)]
 SUPPORTED_HEAD_DIMS = (32, 64, 128)
+SMALL_TILE_GAIN = 0.2
 
 
 def takes_narrow_rows(head_dim: int, dtype: torch.dtype) -> bool:
@@ -128,6 +129,37 @@ def _choose_tile_shapes(
                 best, best_cost = (qt, kt), key
     assert best is not None
     return best
+
+
+@torch.compiler.assume_constant_result
+def choose_small_forward_tiles(
+    token_layout: DimensionType, kernel_size: DimensionType, stride: DimensionType, dilation: DimensionType,
+    is_causal: Tuple[bool, ...], q_tile_shape: DimensionType, kv_tile_shape: DimensionType,
+) -> Optional[Tuple[DimensionType, DimensionType]]:
+    return _choose_small_forward_tiles(tuple(token_layout), tuple(kernel_size), tuple(stride), tuple(dilation),
+                                       tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape))
+
+
+@functools.lru_cache(maxsize=1024)
+def _choose_small_forward_tiles(token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape):
+    """Shapes of a 64 x 64 tile pair for the one-launch forward of head dims up to 64, where they beat the
+    128 x 64 pair given; None where they do not.  Small windows: half the queries span a smaller box, so
+    fewer pairs outside the windows are multiplied.  They have to be at least SMALL_TILE_GAIN fewer, because a
+    workgroup of half the queries fetches every key tile for half the work, and three tiles a workgroup, because
+    shorter loops are all set-up.  Measured (bf16, us, 128 x 64 against 64 x 64; pairs as a share):
+    2x64x64 H 8 D 64, 13x13: 27.7 / 21.4 (.70); 4x56x56 H 8 D 32, 7x7: 29.9 / 24.5 (.65); 128x128 H 8 D 64, 25x25:
+    73.1 / 71.5 (.84); 4096 tokens, 33: 10.7 / 11.5 (two tiles); 57 random problems up to .80: .61 to 1.17 of the
+    time, .84 at the median, 16 from there to .86: .86 to 1.11, .92 at the median (not worth the losses).  At head dim 128 the larger
+    pair wins throughout (2x64x64, 13x13: 33.5 / 37.1).  No group may be narrower than
+    a key tile (only the 128 x 64 instance clamps its gathers)."""
+    qt, kt = _choose_tile_shapes(token_layout, kernel_size, stride, dilation, is_causal, 64, 64, True)
+    if any(x // d < t for x, d, t in zip(token_layout, dilation, kt)):
+        return None
+    small = visited_pairs(token_layout, kernel_size, stride, dilation, is_causal, qt, kt)
+    large = visited_pairs(token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape)
+    if small > (1 - SMALL_TILE_GAIN) * large or small < 3 * 64 * math.prod(token_layout):
+        return None
+    return qt, kt
 
 
 def check_fna_forward_config(
