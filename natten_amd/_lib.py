@@ -187,6 +187,13 @@ def _i32(values: Sequence[int]):
     return _i32_array(tuple(int(v) for v in values))
 
 
+@functools.lru_cache(maxsize=4096)
+def _problem_arrays(qkv_shape, kernel_size, stride, dilation, is_causal, *tile_shapes):
+    """The int32 arrays of a problem's geometry, in the order the entry points take them: one look-up per
+    call for what would be seven conversions."""
+    return tuple(_i32(x) for x in (qkv_shape, kernel_size, stride, dilation, [1 if c else 0 for c in is_causal], *tile_shapes))
+
+
 def _check(rc: int):
     if rc != 0:
         raise RuntimeError(lib().natten_amd_last_error().decode())
@@ -361,7 +368,6 @@ def fna_forward_fused(
         raise NotImplementedError(f"natten_amd fna_forward_fused does not support {q.dtype}.")
     q, k, v = _aligned_narrow_rows(q, k, v)
     na_dim = len(kernel_size)
-    qkv_shape = [int(x) for x in q.shape[1 : 1 + na_dim]]
     scales = _scale_ptrs(q, k, q_scale, k_scale, v_scale)
     out = torch.empty(q.shape, dtype=torch.bfloat16 if q.dtype in FP8_DTYPES else q.dtype, device=q.device)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
@@ -369,8 +375,8 @@ def fna_forward_fused(
         rc = L.natten_amd_fna_forward_fused(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
             DTYPE_CODES[q.dtype], na_dim, q.shape[0], q.shape[-2], k.shape[-2], q.shape[-1],
-            _i32(qkv_shape), _i32(kernel_size), _i32(stride), _i32(dilation),
-            _i32([1 if c else 0 for c in is_causal]), _i32(q_tile_shape), _i32(kv_tile_shape),
+            *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
+                             tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
             float(scale), *scales, 1 if anchored_tiles else 0, *_queue_workspace(q, run_persistent), _stream(q),
         )
     _check(rc)
@@ -394,8 +400,9 @@ def fna_forward_f32(
     with _on_device(q):
         rc = L.natten_amd_fna_forward_f32(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), na_dim, q.shape[0], q.shape[-2],
-            k.shape[-2], q.shape[-1], _i32(q.shape[1 : 1 + na_dim]), _i32(kernel_size), _i32(stride), _i32(dilation),
-            _i32([1 if c else 0 for c in is_causal]), float(scale), _stream(q),
+            k.shape[-2], q.shape[-1],
+            *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation), tuple(is_causal)),
+            float(scale), _stream(q),
         )
     _check(rc)
     return out, lse

@@ -121,7 +121,13 @@ def additional_kv_tensor_checks(
 
 def _dim_arg(name: str, na_dim: int, value: Any, minimum: int, default: Optional[int]) -> DimensionType:
     if value is None and default is not None:
-        return tuple([default] * na_dim)
+        return (default,) * na_dim
+    if type(value) is tuple and len(value) == na_dim:
+        for x in value:
+            if type(x) is not int or x < minimum:
+                break
+        else:
+            return value
     if (
         isinstance(value, Sequence)
         and len(value) == na_dim
@@ -150,7 +156,13 @@ def check_dilation_arg(na_dim: int, dilation: Any) -> DimensionType:
 
 def check_causal_arg(na_dim: int, is_causal: Any) -> CausalArgType:
     if is_causal is None:
-        return tuple([False] * na_dim)
+        return (False,) * na_dim
+    if type(is_causal) is tuple and len(is_causal) == na_dim:
+        for c in is_causal:
+            if type(c) is not bool:
+                break
+        else:
+            return is_causal
     if isinstance(is_causal, Sequence) and len(is_causal) == na_dim and all(isinstance(c, bool) for c in is_causal):
         return tuple(bool(c) for c in is_causal)
     if isinstance(is_causal, bool):
@@ -174,6 +186,11 @@ def check_all_args(na_dim: int, kernel_size: Any, stride: Any, dilation: Any, is
 def check_args_against_input(input_tensor: Tensor, kernel_size, stride, dilation, is_causal):
     na_dim = input_tensor.dim() - 3
     input_size = tuple(input_tensor.shape[1 : 1 + na_dim])
+    for x, k, d, s in zip(input_size, kernel_size, dilation, stride):
+        if k * d > x or s > k:
+            break
+    else:
+        return
     if any(k * d > x for x, k, d in zip(input_size, kernel_size, dilation)):
         raise ValueError(
             "The product of kernel size and dilation cannot be larger than input size along any dimension, "

@@ -1573,34 +1573,26 @@ inline void choose_wave_box(FnaParams& p) {
 }
 
 // Few groups: the XCDs' shares differ by whole groups, and a short last group per (batch, head) pair can
-// meet the same XCDs every time (8 heads of 65 + 20 tiles: 130 on every other XCD, 40 on the rest).
-// Equal groups, and as many of them per pair as even the shares out: the fewest within a twentieth of
-// the best, at most four times as many (smaller groups share less of their keys in an L2).  From 16 groups an
-// XCD on the shares differ by less than that and the groups stay as they are.
+// meet the same XCDs every time (8 heads of 65 + 20 tiles: 130 on every other XCD, 40 on the rest; 66 x 66
+// tokens, H 8, D 64, 4 x 36 windows, 64 x 64 tiles: 25.3 us like that, 19.5 with two groups of 43).  Equal
+// groups, and as many of them per pair as even the shares out: the fewest within a twentieth of the best, at
+// most four times as many (smaller groups share less of their keys in an L2).  From 16 groups an XCD on
+// the shares differ by less than that and the groups stay as they are.
 inline void balance_wg_groups(FnaParams& p, int units, long long bh) {
-  auto largest_share = [&](int per_pair, int size) {
-    long long share[kNumXcd] = {}, most = 0;
-    for (long long g = 0; g < bh * per_pair; ++g)
-      share[g % kNumXcd] += na_min(size, units - int(g % per_pair) * size);
-    for (long long s : share) most = s > most ? s : most;
-    return most;
-  };
   const int now = (units + p.wg_group - 1) / p.wg_group;
   if (bh * now >= 16 * kNumXcd) return;
-  const double even = double(bh) * units / kNumXcd;
-  if (largest_share(now, p.wg_group) <= 1.05 * even) return;
-  int size[4 * 16 * kNumXcd + 1];  // by groups per pair
-  long long best = -1;
+  // tiles of the XCD that gets the most, with n groups of `size` per pair
+  auto share = [&](int n, int size) { return ((bh * n + kNumXcd - 1) / kNumXcd) * size; };
+  auto equal = [&](int n) { return (units + n - 1) / n; };
+  const long long start = share(now, p.wg_group);
+  if (start * kNumXcd * 20 <= bh * units * 21) return;
   const int most = na_min(4 * now, units);
-  long long share[4 * 16 * kNumXcd + 1];
-  for (int n = now; n <= most; ++n) {
-    size[n] = (units + n - 1) / n;
-    share[n] = (units + size[n] - 1) / size[n] == n ? largest_share(n, size[n]) : -1;
-    if (share[n] >= 0 && (best < 0 || share[n] < best)) best = share[n];
-  }
+  long long best = start;
+  for (int n = now; n <= most; ++n) best = share(n, equal(n)) < best ? share(n, equal(n)) : best;
+  if (best == start) return;
   for (int n = now; n <= most; ++n)
-    if (share[n] >= 0 && share[n] <= 1.05 * best) {
-      if (share[n] < largest_share(now, p.wg_group)) p.wg_group = size[n];
+    if (share(n, equal(n)) * 20 <= best * 21) {
+      p.wg_group = equal(n);
       return;
     }
 }

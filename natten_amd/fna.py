@@ -8,6 +8,7 @@ and :332-407 (driver).
 
 from __future__ import annotations
 
+import functools
 from typing import Optional, Tuple, Union
 
 import torch
@@ -16,9 +17,11 @@ from torch import Tensor
 from . import _lib, torch_ops
 from .checks import check_all_args, check_args_against_input, na_tensor_checks
 from .tile_config import (
+    TILE_SIZES,
     check_fna_backward_config,
     check_fna_forward_config,
     choose_small_forward_tiles,
+    choose_tile_shapes,
     padded_head_dim,
     takes_narrow_rows,
 )
@@ -96,6 +99,38 @@ def _prod(t) -> int:
     return out
 
 
+@functools.lru_cache(maxsize=1024)
+def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
+    """What amd_fna_generic comes to for a forward call on checked arguments that fixes neither tiles nor route
+    nor splits and has no scales, where that is a single launch on the operands as they are: its tile shapes
+    and launch kind, or "float32"; None for everything else.  A small call is bound by the time it
+    takes to get to its launch (256 tokens, float32: 23 us a call for 5 us of kernel), and the choices are a
+    third of that time.  Plain values in and out: nothing here knows a tensor."""
+    if dtype == torch.float32:
+        return "float32"
+    head_dim, layout = shape[-1], shape[1:-2]
+    narrow = takes_narrow_rows(head_dim, dtype) and not run_persistent_kernel
+    if dtype not in (torch.float16, torch.bfloat16) or (head_dim != padded_head_dim(head_dim) and not narrow):
+        return None
+    from .functional import kv_splits_default, work_queue_default
+
+    problem = (layout, kernel_size, stride, dilation, is_causal)
+    tiles = choose_tile_shapes(*problem, *TILE_SIZES[0], anchored=True)
+    launch_left_open = run_persistent_kernel is None
+    persistent = bool(run_persistent_kernel)
+    if launch_left_open and not narrow:
+        persistent = work_queue_default(shape[0], shape[-2], *problem, *tiles)
+    if not persistent and not narrow:
+        if kv_splits_default(shape[0], shape[-2], *problem, *tiles) != 1:
+            return None
+        if launch_left_open and head_dim <= 64:
+            tiles = choose_small_forward_tiles(*problem, *tiles) or tiles
+    if not _lib.fused_layout_supported(layout, dilation, tiles[1], row_bytes=heads_kv * padded_head_dim(head_dim) * 2,
+                                       q_tile_shape=tiles[0], dtype=dtype):
+        return None
+    return (*tiles, persistent)
+
+
 def amd_fna_generic(
     query: Tensor,
     key: Tensor,
@@ -151,6 +186,19 @@ def amd_fna_generic(
         kernel_size, stride, dilation, is_causal = check_all_args(na_dim, kernel_size, stride, dilation, is_causal)
         check_args_against_input(query, kernel_size, stride, dilation, is_causal)
     can_run_amd_fna(query, key, value, raise_error=True)
+    if (q_tile_shape is None and kv_tile_shape is None and fused is None and anchored_tiles and kv_splits is None
+            and fp8_matmul is None and q_scale is None and k_scale is None and v_scale is None and not torch_ops._tracing()
+            and not (torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad))):
+        plan = _open_call_plan(query.dtype, tuple(query.shape), key.shape[-2], kernel_size, stride, dilation, is_causal,
+                               run_persistent_kernel)
+        if plan is not None:
+            operands = (query.contiguous(), key.contiguous(), value.contiguous(), kernel_size, stride, dilation, is_causal,
+                        scale or query.shape[-1] ** -0.5)
+            output, lse = (_lib.fna_forward_f32(*operands) if plan == "float32" else
+                           _lib.fna_forward_fused(*operands, plan[0], plan[1], run_persistent=plan[2]))
+            if out_dtype is not None and out_dtype != output.dtype:
+                output = output.to(out_dtype)
+            return (output, lse) if return_lse else output
     # float32 on the original tensors, in one launch with boxes of its own: unless the caller fixed tile
     # shapes or a route, which the kernel on permuted sequences serves (2x64x64 tokens, H 8, D 64,
     # 13 x 13 windows: 62 us here, 300 us there; 256 tokens, H 2, D 32, window 7: 23 and 83 us)
