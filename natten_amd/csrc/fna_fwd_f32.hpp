@@ -271,9 +271,9 @@ inline void choose_f32_boxes(FnaF32Params& p) {
 // V operands and results are VEC-wide loads and stores of whole rows.
 // Softmax in float32; a row's maximum is followed once it grew by more than 2^8 (exact: the sums are
 // normalised by the same maximum).
-// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 62 us (45 TFLOP/s of window pairs, 69 of pairs
+// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 54 us (53 TFLOP/s of window pairs, 80 of pairs
 // multiplied; the card's float32 matrix products reach 154), 300 us as permutes, 128-query kernel and
-// unpermutes; 256 tokens, H 2, D 32, window 7: 23 us, all of it the call, from 83.
+// unpermutes; 256 tokens, H 2, D 32, window 7: 17 us, all of it the call, from 83.
 template <int D, bool PAD>
 __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32Params p) {
   constexpr int KJ = D / 16;
@@ -484,17 +484,19 @@ __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32
         for (int c = 0; c < VEC; ++c) acc[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.v[r][h][c], S[r], acc[h][c], 0, 0, 0);
   };
 
-  // two blocks in registers: while one is multiplied the other is on its way
+  // Two blocks in registers: while one is multiplied the other is on its way.  The loads are not
+  // conditional (past the last block they fetch clamped rows that nothing reads): behind a branch the wait for
+  // a block becomes a wait for everything outstanding, the next block included (62.6 us instead of 54.0).
   Block A, B;
   const int total = nblk[0] * nblk[1] * nblk[2];
   load(A);
-  for (int n = 0; n < total; n += 2) {
-    if (n + 1 < total) load(B);
+  for (int n = 0;; n += 2) {
+    load(B);
     multiply(A);
-    if (n + 1 < total) {
-      if (n + 2 < total) load(A);
-      multiply(B);
-    }
+    if (n + 1 >= total) break;
+    load(A);
+    multiply(B);
+    if (n + 2 >= total) break;
   }
 
   float l = l_run + __shfl_xor(l_run, 16);

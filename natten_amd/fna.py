@@ -201,7 +201,7 @@ def amd_fna_generic(
             return (output, lse) if return_lse else output
     # float32 on the original tensors, in one launch with boxes of its own: unless the caller fixed tile
     # shapes or a route, which the kernel on permuted sequences serves (2x64x64 tokens, H 8, D 64,
-    # 13 x 13 windows: 62 us here, 300 us there; 256 tokens, H 2, D 32, window 7: 23 and 83 us)
+    # 13 x 13 windows: 54 us here, 300 us there; 256 tokens, H 2, D 32, window 7: 17 and 83 us)
     own_tiles = q_tile_shape is None
     f32_direct = query.dtype == torch.float32 and fused is None and anchored_tiles and own_tiles
     q_tile_shape, kv_tile_shape = check_fna_forward_config(
