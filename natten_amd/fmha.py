@@ -57,9 +57,11 @@ def amd_fmha(
         if out_dtype is not None and out.dtype != out_dtype:
             out = out.to(out_dtype)
         return (out, lse) if return_lse else out
-    if cumulative_seqlen_Q is None and takes_narrow_rows(head_dim, query.dtype):
+    if d_pad != head_dim and cumulative_seqlen_Q is None and takes_narrow_rows(head_dim, query.dtype):
         d_pad = head_dim
-    q, k, v = (pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value))
+    q, k, v = query.contiguous(), key.contiguous(), value.contiguous()
+    if d_pad != head_dim:
+        q, k, v = (pad_head_dim(t, d_pad).contiguous() for t in (q, k, v))
     if is_fp8(query.dtype):
         # a one-token tile with no dilation is the identity permutation: a plain widening copy
         q, k, v = (torch_ops.token_permute(t, (1,), (1,), True, widen=True) for t in (q, k, v))
