@@ -327,7 +327,8 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
  * [batch, tokens, heads, head_dim] and lse [batch, tokens, heads] (the forward's) it writes q_scaled
  * (q's shape: the logit operand described below), neg_delta = -rowsum(out * d_out) and neg_lse2 =
  * -log2(e) lse, both head-major [batch, heads, tokens] float32: what the kernels' accumulators start
- * from.  natten_amd_fna_backward_fused then takes `roles` + 4.
+ * from.  natten_amd_fna_backward_fused takes the three in place of an unfilled q_scaled, delta and lse
+ * when `roles` + 4 says so; the dense attention entry points take neg_lse2 and neg_delta always.
  */
 int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse,
                                 void* q_scaled, float* neg_delta, float* neg_lse2, int dtype, int batch,
@@ -337,9 +338,9 @@ int natten_amd_backward_prepare(const void* q, const void* out, const void* d_ou
  * Fused neighborhood attention backward on token-permuted operands.
  *   q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv [batch, seqlen_kv, heads_kv,
  *   head_dim], permuted like the forward operands (dimension 0 fastest inside a tile, dilation
- *   groups folded into batch); neg_lse2, neg_delta float32, permuted the same way and then stored
- *   head-major, [batch, heads_q, seqlen_q] (the kernels read 64 consecutive rows of one head at
- *   a time): -log2(e) times the forward's lse, minus natten_amd_compute_delta's result.
+ *   groups folded into batch); lse (the forward's) and delta (natten_amd_compute_delta's) float32,
+ *   permuted the same way and then stored head-major, [batch, heads_q, seqlen_q] (the kernels read 64
+ *   consecutive rows of one head at a time).
  *   Both tile shapes must hold 128 tokens and their last extent above 1 must be even; q_shape /
  *   kv_shape are the padded per-group layouts (multiples of the tiles), seqlen = their product.
  * dq, dk, dv are written completely (padding rows get zeros); nothing is accumulated through
@@ -352,12 +353,13 @@ int natten_amd_backward_prepare(const void* q, const void* out, const void* d_ou
  * q', which makes its probabilities exp(logit - LSE) those the forward normalised (they sum to
  * one over a query's window).  The launch that writes dq scales the query rows it holds in
  * registers; the launch that writes dk and dv streams q' and first writes it to q_scaled with
- * one pass over q.  The call makes the dk / dv launch first and the dq launch last, so q_scaled
+ * one pass over q, unless the caller says that q_scaled is filled already (`roles` + 4, or
+ * q_scaled_filled).  The call makes the dk / dv launch first and the dq launch last, so q_scaled
  * may be the dq buffer itself (for a call that only makes the dk / dv launch: if dq is written
  * afterwards); it must not be q.  May be null for a call that only makes the dq launch.
  */
 int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out,
-                            const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv,
+                            const float* lse, const float* delta, void* dq, void* dk, void* dv,
                             void* q_scaled, int dtype, int na_dim, int batch, int seqlen_q, int seqlen_kv,
                             int heads_q, int heads_kv, int head_dim, const int32_t* q_shape,
                             const int32_t* kv_shape, const int32_t* qkv_shape,
@@ -368,7 +370,7 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
 
 /*
  * The same backward on the original tensors: q, d_out, dq [batch, *qkv_shape, heads_q, head_dim],
- * k, v, dk, dv [batch, *qkv_shape, heads_kv, head_dim], neg_lse2 and neg_delta head-major
+ * k, v, dk, dv [batch, *qkv_shape, heads_kv, head_dim], lse and delta head-major
  * [batch, heads_q, prod(qkv_shape)].  The kernels gather and scatter the rows of their tiles
  * themselves, which replaces the six token permutes and three unpermutes of the reference's
  * backward driver (src/natten/backends/blackwell_fna.py:205-297).  Where every extent is a
@@ -384,10 +386,12 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
  * dv (the other results are left untouched).  With no permuted layout to share, the two launches
  * need not use the same tile shapes: the dq launch streams half KV tiles past a Q tile, the
  * dk / dv launch half Q tiles past a KV tile, and the shapes that visit the fewest tiles differ
- * (a caller makes one call per role, each with that role's shapes).
+ * (a caller makes one call per role, each with that role's shapes).  Plus 4 (5, 6 or 7): lse, delta
+ * and q_scaled hold what natten_amd_backward_prepare wrote (neg_lse2, neg_delta, q_scaled), which
+ * saves the call its own pass over q and the kernels the scaling of the two arrays.
  */
 int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out,
-                                  const float* neg_lse2, const float* neg_delta, void* dq, void* dk,
+                                  const float* lse, const float* delta, void* dq, void* dk,
                                   void* dv, void* q_scaled, int dtype, int na_dim, int batch, int heads_q,
                                   int heads_kv, int head_dim, const int32_t* qkv_shape,
                                   const int32_t* kernel_size, const int32_t* stride,
@@ -397,8 +401,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
 
 /*
  * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
- * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2, neg_delta head-major [batch, heads_q, seqlen_q].
- * q_scaled as above; q_scaled_filled != 0: it is filled already (natten_amd_backward_prepare).
+ * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2 = -log2(e) lse and neg_delta = -delta head-major
+ * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above; q_scaled_filled != 0: it is filled already (natten_amd_backward_prepare).
  * Any sequence lengths: rows past the end of a sequence are gathered from its last row and masked.
  */
 int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out,

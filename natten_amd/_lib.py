@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -610,11 +610,11 @@ def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: 
 
 
 def _head_major(lse: Tensor, delta: Tensor) -> Tuple[Tensor, Tensor]:
-    """lse, delta [B, *X, H] as the backward kernels take them: -log2(e) lse and -delta, [B, H, prod(X)]."""
+    """lse, delta [B, *X, H] as the backward kernels take them, [B, H, prod(X)]: a copy each and no more."""
     if lse.dtype != torch.float32 or delta.dtype != torch.float32:
         raise ValueError("lse and delta must be float32.")
     B, H = lse.shape[0], lse.shape[-1]
-    return tuple((t.reshape(B, -1, H).transpose(1, 2) * c).contiguous() for t, c in ((lse, -1.4426950408889634), (delta, -1.0)))
+    return tuple(t.reshape(B, -1, H).transpose(1, 2).contiguous() for t in (lse, delta))
 
 
 def fna_backward(
@@ -624,15 +624,15 @@ def fna_backward(
     """Backward on token-permuted operands (128-token tiles on both sides) -> (dq, dk, dv).
     lse, delta: [batch, seqlen_q, heads_q] as the permute gives them; the kernels take them head-major."""
     L = lib()
-    neg_lse2, neg_delta = _head_major(lse, delta)
-    _require_gpu(q, k, v, d_out, neg_lse2, neg_delta)
+    lse, delta = _head_major(lse, delta)
+    _require_gpu(q, k, v, d_out, lse, delta)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd fna_backward does not support {q.dtype}.")
     na_dim = len(kernel_size)
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     with _on_device(q):
         rc = L.natten_amd_fna_backward(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, q.shape[0], q.shape[1],
             k.shape[1], q.shape[2], k.shape[2], q.shape[3], _i32(q_shape), _i32(kv_shape), _i32(qkv_shape),
             _i32(kernel_size), _i32(stride), _i32(dilation), _i32([1 if c else 0 for c in is_causal]),
@@ -674,25 +674,25 @@ def fna_backward_fused(
         raise ValueError("kv_role_q_tile_shape and kv_role_kv_tile_shape must be given together.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     if out is not None:
-        neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
+        delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
     else:
-        neg_lse2, neg_delta = _head_major(lse, delta)
-    _require_gpu(q, k, v, d_out, neg_lse2, neg_delta)
-    filled = 4 if out is not None else 0
+        lse, delta = _head_major(lse, delta)
+    _require_gpu(q, k, v, d_out, lse, delta)
+    prepared = 4 if out is not None else 0
     same = kv_role_q_tile_shape is None or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
     # The dk / dv launch streams the queries as the forward kernel multiplied them (scaled, rounded
     # once) from a workspace of q's size that the call fills first; dq serves as that workspace, so
     # the launch that writes dq comes last.
-    launches = [(3 + filled, q_tile_shape, kv_tile_shape)] if same else [
-        (2 + filled, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
+    launches = [(3, q_tile_shape, kv_tile_shape)] if same else [
+        (2, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
     with _on_device(q):
         for roles, qt, kt in launches:
             rc = L.natten_amd_fna_backward_fused(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2],
                 q.shape[-1], _i32(q.shape[1 : 1 + na_dim]), _i32(kernel_size), _i32(stride), _i32(dilation),
-                _i32([1 if c else 0 for c in is_causal]), _i32(qt), _i32(kt), float(scale), roles, _stream(q),
+                _i32([1 if c else 0 for c in is_causal]), _i32(qt), _i32(kt), float(scale), roles + prepared, _stream(q),
             )
             _check(rc)
     return dq, dk, dv

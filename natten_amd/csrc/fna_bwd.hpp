@@ -55,10 +55,14 @@ struct FnaBwdParams {
   const void* k;      // [batch, seqlen_kv, heads_kv, D]
   const void* v;
   const void* d_out;  // like q
-  // [batch, heads_q, seqlen_q] (head-major: a tile's values are contiguous), as the kernels' accumulators
-  // start from them: -log2(e) LSE and -rowsum(d_out * out)
-  const float* neg_lse2;
-  const float* neg_delta;
+  // [batch, heads_q, seqlen_q] (head-major: a tile's values are contiguous).  The kernels' accumulators
+  // start from lse_mul times `lse` and delta_mul times `delta`, that is from -log2(e) LSE and -rowsum(d_out *
+  // out).  prepared != 0: the arrays hold these values already (both factors are 1; bwd_prepare_kernel);
+  // 0: the forward's LSE and the row sums themselves, which the RAW instances scale as they read a tile's.
+  const float* lse;
+  const float* delta;
+  int prepared;
+  float lse_mul, delta_mul;
   void* dq;
   void* dk;
   void* dv;
@@ -110,6 +114,8 @@ struct FnaBwdParams {
 };
 
 inline void set_bwd_divisions(FnaBwdParams& p) {
+  p.lse_mul = p.prepared ? 1.f : -1.4426950408889634f;
+  p.delta_mul = p.prepared ? 1.f : -1.f;
   for (int a = 0; a < 3; ++a) {
     p.q_tile_lg[a] = p.kv_tile_lg[a] = 0;
     while ((1 << p.q_tile_lg[a]) < p.q_tile[a]) ++p.q_tile_lg[a];
@@ -167,7 +173,9 @@ constexpr int bwd_waves_per_simd(int head_dim, int role) {
 // of a sequence are gathered from its last row; stationary ones store nothing, streamed ones are masked.
 // (Padding the sequences into copies first made 67 launches of a packed training step, of index arithmetic
 // and copies most of them: 10 sequences of 1 .. 2048, H 16 / 4, D 128 919 us, now 6 launches and 462 us.)
-template <typename T, int D, int ROLE, bool RAGGED = false>
+// RAW (key-stationary roles): LSE and delta as they are, scaled on the way from LDS to the accumulators
+// (the dQ role scales its two values per lane in every instance).
+template <typename T, int D, int ROLE, bool RAGGED = false, bool RAW = false>
 __global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256)
 __attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D, ROLE), bwd_waves_per_simd(D, ROLE))))
 fna_bwd_kernel(const FnaBwdParams p) {
@@ -490,8 +498,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
   if constexpr (!KV_STATIONARY) {
     const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
                                      : stat_row_q + head_a * stat_head_stride + a_seq_row;
-    lse_l = p.neg_lse2[stat_idx];
-    delta_l = p.neg_delta[stat_idx];
+    lse_l = p.lse[stat_idx] * p.lse_mul;
+    delta_l = p.delta[stat_idx] * p.delta_mul;
   }
   f32x16_t lse_init, delta_init;
   if constexpr (INIT_REGS) {
@@ -634,7 +642,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       // spare row so that every wave counts the same number of outstanding copies per tile)
       const int64_t stat_row0 = p.fused ? (int64_t(b_orig) * p.heads_q + t.head_b) * p.tokens + t.row0
                                         : stat_row_q + t.head_b * stat_head_stride + t.row0;
-      const float* src = (wave == 2 ? p.neg_delta : p.neg_lse2) + stat_row0;
+      const float* src = (wave == 2 ? p.delta : p.lse) + stat_row0;
       float* dst = (wave == 1) ? &sLse[stage * BT] : (wave == 2) ? &sDelta[stage * BT] : &sSpare[0];
       const uint32_t off = partial ? uint32_t(na_min(lane, last)) * 4u : stat_off;
       if (wave != 0) async_copy4_asm(src, off, lds_address(dst));
@@ -729,21 +737,21 @@ fna_bwd_kernel(const FnaBwdParams p) {
     f32x16_t S[NSB], dP[NSB];
     vec8 pf[NSB][2], dsf[NSB][2];
     // the rows 8*jj + 4*g + i of sub-block sb (logit r = 4 jj + i) of a per-row table
-    auto init_from = [&](const float* table, int sb) __attribute__((always_inline)) {
+    auto init_from = [&](const float* table, float mul, int sb) __attribute__((always_inline)) {
       f32x16_t c;
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&table[stage * BT + sb * 32 + 8 * jj + 4 * g]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) c[4 * jj + i] = v[i];
+        for (int i = 0; i < 4; ++i) c[4 * jj + i] = RAW ? v[i] * mul : v[i];
       }
       return c;
     };
     auto load_inits = [&](auto sb_tag) __attribute__((always_inline)) {
       constexpr int sb = decltype(sb_tag)::value;
       if constexpr (KV_STATIONARY && sb < NSB) {
-        S[sb] = init_from(sLse, sb);
-        if constexpr (HAS_DS) dP[sb] = init_from(sDelta, sb);
+        S[sb] = init_from(sLse, -kLog2e, sb);
+        if constexpr (HAS_DS) dP[sb] = init_from(sDelta, -1.f, sb);
       }
     };
     float held_p = 0.f, held_ds = 0.f;
@@ -858,7 +866,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       for (int jj = 0; jj < 4; ++jj) {
         const f32x4_t v = *reinterpret_cast<const f32x4_t*>(&sDelta[stage1 * BT + sb * 32 + 8 * jj + 4 * g]);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) held_dp[sb][4 * jj + i] = v[i];
+        for (int i = 0; i < 4; ++i) held_dp[sb][4 * jj + i] = RAW ? -v[i] : v[i];
       }
     for_range<0, PF>([&](auto x_tag) {
       constexpr int x = decltype(x_tag)::value;

@@ -350,7 +350,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
 
 extern "C" {
 
-int natten_amd_abi_version(void) { return 18; }
+int natten_amd_abi_version(void) { return 19; }
 
 uint64_t natten_amd_fna_forward_workspace_bytes(void) { return uint64_t(kQueueWords) * 4; }
 
@@ -904,7 +904,7 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
 // ---- backward ---------------------------------------------------------------------------------
 
 extern "C++" {
-template <typename T, int D, bool RAGGED>
+template <typename T, int D, bool RAGGED, bool RAW>
 static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   FnaBwdParams p = params;
   // grids are padded to a multiple of the 8 XCDs: each XCD takes a contiguous eighth of the tiles
@@ -948,9 +948,9 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
     if constexpr (D == 128) {
       // dK and dV by wave pairs (eight waves per workgroup): one wave's registers cannot hold the
       // accumulators, fragments and products of both
-      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdPair, RAGGED>), dim3((unsigned)wg_kv), dim3(512), 0, stream, p);
+      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdPair, RAGGED, RAW>), dim3((unsigned)wg_kv), dim3(512), 0, stream, p);
     } else {
-      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDKV, RAGGED>), dim3((unsigned)wg_kv), dim3(256), 0, stream, p);
+      hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDKV, RAGGED, RAW>), dim3((unsigned)wg_kv), dim3(256), 0, stream, p);
     }
     if (int rc = check_launch("fna_backward (dK, dV)")) return rc;
   }
@@ -961,12 +961,18 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   return 0;
 }
 
+template <typename T, int D>
+static int dispatch_bwd_form(const FnaBwdParams& p, hipStream_t stream, bool ragged) {
+  if (ragged) return launch_bwd<T, D, true, false>(p, stream);  // (dense attention: prepared arrays only)
+  return p.prepared ? launch_bwd<T, D, false, false>(p, stream) : launch_bwd<T, D, false, true>(p, stream);
+}
+
 template <typename T>
 static int dispatch_bwd_head_dim(const FnaBwdParams& p, int head_dim, hipStream_t stream, bool ragged) {
   switch (head_dim) {
-    case 32: return ragged ? launch_bwd<T, 32, true>(p, stream) : launch_bwd<T, 32, false>(p, stream);
-    case 64: return ragged ? launch_bwd<T, 64, true>(p, stream) : launch_bwd<T, 64, false>(p, stream);
-    case 128: return ragged ? launch_bwd<T, 128, true>(p, stream) : launch_bwd<T, 128, false>(p, stream);
+    case 32: return dispatch_bwd_form<T, 32>(p, stream, ragged);
+    case 64: return dispatch_bwd_form<T, 64>(p, stream, ragged);
+    case 128: return dispatch_bwd_form<T, 128>(p, stream, ragged);
   }
   return fail("fna_backward: head_dim must be 32, 64 or 128, got %d", head_dim);
 }
@@ -990,9 +996,9 @@ static int split_dim_of(const int* tile) {
 }
 
 static int check_bwd_pointers(const char* what, const void* q, const void* k, const void* v, const void* d_out,
-                              const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled,
+                              const float* lse, const float* delta, void* dq, void* dk, void* dv, void* q_scaled,
                               int roles) {
-  if (!q || !k || !v || !d_out || !neg_lse2 || !neg_delta || !dq || !dk || !dv) return fail("%s: null pointer argument", what);
+  if (!q || !k || !v || !d_out || !lse || !delta || !dq || !dk || !dv) return fail("%s: null pointer argument", what);
   if ((roles & 2) && !q_scaled) return fail("%s: the dk / dv launch needs the q_scaled workspace", what);
   if (q_scaled == q) return fail("%s: q_scaled must not be q itself (the dq launch reads the unscaled queries)", what);
   if (reinterpret_cast<uintptr_t>(q_scaled) & 15) return fail("%s: q_scaled must be 16-byte aligned", what);
@@ -1003,8 +1009,8 @@ static int check_bwd_pointers(const char* what, const void* q, const void* k, co
   return 0;
 }
 
-int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
-                            const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
+int natten_amd_fna_backward(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
+                            const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
                             int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
                             const int32_t* q_shape, const int32_t* kv_shape, const int32_t* qkv_shape,
                             const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
@@ -1012,8 +1018,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
                             float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "fna_backward";
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 3)) return rc;
-  if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, 3)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!q_shape || !kv_shape || !qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape ||
       !kv_tile_shape)
@@ -1052,8 +1058,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.neg_lse2 = neg_lse2;
-  p.neg_delta = neg_delta;
+  p.lse = lse;
+  p.delta = delta;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
@@ -1068,8 +1074,8 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
 }
 
-int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* neg_lse2,
-                                  const float* neg_delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
+int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
+                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
                                   int batch, int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
                                   const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
                                   const int32_t* is_causal, const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
@@ -1077,8 +1083,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   g_error[0] = 0;
   const char* what = "fna_backward_fused";
   if (roles < 1 || roles > 7 || (roles & 3) == 0)
-    return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 where q_scaled is filled already, got %d", what, roles);
-  if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, roles)) return rc;
+    return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 for prepared arrays, got %d", what, roles);
+  if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, roles)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape || !kv_tile_shape)
     return fail("%s: null shape argument", what);
@@ -1106,7 +1112,7 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                is_causal, q_tile_shape, kv_tile_shape))
     return rc;
   if (!fna_tiles_are_powers_of_two(f)) return fail("%s: tile extents must be powers of two", what);
-  if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, int(tokens), int(tokens), heads_q, heads_kv, head_dim)) return rc;
+  if (int rc = check_common(what, q, k, v, dq, lse, batch, int(tokens), int(tokens), heads_q, heads_kv, head_dim)) return rc;
   // per-lane byte offsets inside a tile are 32-bit
   long long span_q = 0, span_kv = 0;
   for (int a = 0; a < 3; ++a) {
@@ -1142,8 +1148,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.neg_lse2 = neg_lse2;
-  p.neg_delta = neg_delta;
+  p.lse = lse;
+  p.delta = delta;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
@@ -1159,6 +1165,7 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   p.edge = edge;
   p.tokens = int(tokens);
   p.roles = roles;
+  p.prepared = (roles & 4) != 0;
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
 }
 
@@ -1182,8 +1189,9 @@ void fill_dense_bwd(FnaBwdParams& p, const void* q, const void* k, const void* v
   p.k = k;
   p.v = v;
   p.d_out = d_out;
-  p.neg_lse2 = neg_lse2;
-  p.neg_delta = neg_delta;
+  p.lse = neg_lse2;
+  p.delta = neg_delta;
+  p.prepared = 1;
   p.dq = dq;
   p.dk = dk;
   p.dv = dv;
