@@ -329,10 +329,16 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
  * -log2(e) lse, both head-major [batch, heads, tokens] float32: what the kernels' accumulators start
  * from.  natten_amd_fna_backward_fused takes the three in place of an unfilled q_scaled, delta and lse
  * when `roles` + 4 says so; the dense attention entry points take neg_lse2 and neg_delta always.
+ *
+ * packed_tiles (null otherwise, with the four arguments before it null or zero): for a sequence-packed
+ * batch (batch = 1, tokens = rows_q) the call also counts the tiles of both sides' sequences, for
+ * natten_amd_attention_backward_varlen: device memory of 4 (num_seqs + 2) int32, 8-byte aligned.
  */
 int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse,
                                 void* q_scaled, float* neg_delta, float* neg_lse2, int dtype, int batch,
-                                int tokens, int heads, int head_dim, float scale, void* stream);
+                                int tokens, int heads, int head_dim, float scale,
+                                const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv, int num_seqs,
+                                int rows_kv, int32_t* packed_tiles, void* stream);
 
 /*
  * Fused neighborhood attention backward on token-permuted operands.
@@ -419,6 +425,7 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
  * rows cu_seqlens_q[b] .. cu_seqlens_q[b+1] - 1 of the queries, keys likewise.  dq, dk and dv are
  * written completely: rows of no sequence get zeros, and so do the rows of a sequence whose
  * offsets do not fit the row counts of the other side (the host cannot see the device arrays).
+ * packed_tiles: what natten_amd_backward_prepare counted for the same two arrays and row counts.
  * No host synchronisation.
  */
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v,
@@ -426,8 +433,8 @@ int natten_amd_attention_backward_varlen(const void* q, const void* k, const voi
                                          void* dq, void* dk, void* dv, void* q_scaled, int q_scaled_filled,
                                          int dtype, int num_seqs, int rows_q, int rows_kv,
                                          const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
-                                         int heads_q, int heads_kv, int head_dim, int is_causal,
-                                         float scale, void* stream);
+                                         const int32_t* packed_tiles, int heads_q, int heads_kv,
+                                         int head_dim, int is_causal, float scale, void* stream);
 
 /*
  * Token permute: src [batch, *token_layout, heads, head_dim] -> dst

@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -91,7 +91,8 @@ _SIGNATURES = {
     ),
     "natten_amd_backward_prepare": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 7 + [ctypes.c_int] * 5 + [ctypes.c_float, ctypes.c_void_p],
+        [ctypes.c_void_p] * 7 + [ctypes.c_int] * 5 + [ctypes.c_float] + [ctypes.c_void_p] * 2 + [ctypes.c_int] * 2
+        + [ctypes.c_void_p] * 2,
     ),
     "natten_amd_fna_backward": (
         ctypes.c_int,
@@ -108,7 +109,7 @@ _SIGNATURES = {
     ),
     "natten_amd_attention_backward_varlen": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 2 + [ctypes.c_int] * 4
+        [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4
         + [ctypes.c_float, ctypes.c_void_p],
     ),
     "natten_amd_token_permute_widen": (
@@ -589,9 +590,13 @@ def compute_delta(out: Tensor, d_out: Tensor) -> Tensor:
     return delta
 
 
-def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: float, q_scaled: Tensor) -> Tuple[Tensor, Tensor]:
+def backward_prepare(
+    q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: float, q_scaled: Tensor,
+    packed: Optional[Tuple[Tensor, Tensor, int, Tensor]] = None,
+) -> Tuple[Tensor, Tensor]:
     """q, out, d_out [B, *X, H, D], lse [B, *X, H] -> head-major float32 [B, H, prod(X)] -rowsum(out * d_out)
-    and -log2(e) lse; fills q_scaled (like q) with the logit operand of the dk / dv launch."""
+    and -log2(e) lse; fills q_scaled (like q) with the logit operand of the dk / dv launch.  packed: the
+    cumulative lengths, the key rows and the [2, sequences + 2, 2] int32 tile counts to fill."""
     _require_gpu(q, out, d_out, lse, q_scaled)
     if out.dtype != q.dtype or d_out.dtype != q.dtype or out.shape != q.shape or d_out.shape != q.shape:
         raise ValueError("out and d_out must be of q's shape and dtype.")
@@ -600,10 +605,14 @@ def backward_prepare(q: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, scale: 
     B, H = q.shape[0], q.shape[-2]
     tokens = lse.numel() // (B * H)
     neg_delta, neg_lse2 = torch.empty((2, B, H, tokens), dtype=torch.float32, device=q.device)
+    packed_args = (None, None, 0, 0, None)
+    if packed is not None:
+        cu_q, cu_kv, rows_kv, tiles = packed
+        packed_args = (cu_q.data_ptr(), cu_kv.data_ptr(), cu_q.numel() - 1, int(rows_kv), tiles.data_ptr())
     with _on_device(q):
         rc = lib().natten_amd_backward_prepare(
             q.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), q_scaled.data_ptr(), neg_delta.data_ptr(),
-            neg_lse2.data_ptr(), DTYPE_CODES[q.dtype], B, tokens, H, q.shape[-1], float(scale), _stream(q),
+            neg_lse2.data_ptr(), DTYPE_CODES[q.dtype], B, tokens, H, q.shape[-1], float(scale), *packed_args, _stream(q),
         )
     _check(rc)
     return neg_delta, neg_lse2
@@ -734,13 +743,14 @@ def attention_backward_varlen(
     if cu_q.numel() < 2 or q.shape[0] != 1 or k.shape[0] != 1:
         raise ValueError("sequence-packed operands have batch 1 and at least one sequence.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
+    tiles = torch.empty((2, cu_q.numel() + 1, 2), dtype=torch.int32, device=q.device)
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq, (cu_q, cu_kv, k.shape[1], tiles))
     with _on_device(q):
         rc = L.natten_amd_attention_backward_varlen(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], cu_q.numel() - 1, q.shape[1],
-            k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,
-            float(scale), _stream(q),
+            k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), tiles.data_ptr(), q.shape[2], k.shape[2], q.shape[3],
+            1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)
     return dq, dk, dv

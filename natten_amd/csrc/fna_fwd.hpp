@@ -307,67 +307,6 @@ static __device__ __forceinline__ float cross_half_max(float x) {
   return fmaxf(fmaxf(a, b), x);
 }
 
-// Where tile `x` of a sequence-packed batch lies.  The rows 0 .. total - 1 of one side are the
-// sequences cu[i] .. cu[i + 1] - 1 (those whose offsets the rows can hold) and the gaps in front of and
-// behind them, whose rows belong to no sequence; tiles of 2^tile_lg rows are counted through both, a
-// sequence's gap first, the rows behind the last sequence as the gap of sequence num_seqs.  All 64
-// lanes of a wave call it together and take 64 sequences a step; false: there are fewer tiles than x.
-// So a launch of total / tile + 2 (num_seqs + 1) tiles per head covers any lengths, where one sized for
-// the longest sequence starts a workgroup per sequence and tile of that one (10 sequences of 1 .. 2048:
-// 160 tiles a head instead of 72, of which 87 find nothing to do).
-struct PackedTile {
-  int seq;
-  bool gap;        // rows of no sequence
-  int row0, rows;  // first row and row count of the sequence (or the gap)
-  int tile;        // position of the tile inside it
-};
-static __device__ __forceinline__ bool locate_packed_tile(const int32_t* __restrict__ cu, const int num_seqs, const int total,
-                                                          const int tile_lg, int x, const int lane, PackedTile& t) {
-  int covered = 0;  // rows below it lie in a sequence or gap already counted
-  for (int s0 = 0; s0 <= num_seqs; s0 += 64) {
-    const int i = s0 + lane;
-    int beg = 0, end = 0;
-    if (i < num_seqs) {
-      beg = cu[i];
-      end = cu[i + 1];
-    }
-    const bool valid = i < num_seqs && beg >= 0 && end >= beg && end <= total;
-    int upto = valid ? end : 0;  // inclusive prefix maximum of the ends
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(upto, o);
-      if (lane >= o) upto = na_max(upto, y);
-    }
-    const int before = __shfl_up(upto, 1);
-    const int gap0 = na_max(lane > 0 ? before : 0, covered);
-    const int gap_rows = na_max((i == num_seqs ? total : valid ? beg : 0) - gap0, 0);
-    const int rows = valid ? end - beg : 0;
-    const int gap_tiles = (gap_rows + (1 << tile_lg) - 1) >> tile_lg;
-    const int tiles = gap_tiles + ((rows + (1 << tile_lg) - 1) >> tile_lg);
-    int sum = tiles;  // inclusive prefix sum
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int y = __shfl_up(sum, o);
-      if (lane >= o) sum += y;
-    }
-    const uint64_t past = __ballot(sum > x);
-    if (past != 0) {
-      const int l = __ffsll((unsigned long long)past) - 1;
-      auto of = [&](int v) { return __builtin_amdgcn_readlane(v, l); };
-      const int local = x - (of(sum) - of(tiles));
-      t.seq = s0 + l;
-      t.gap = local < of(gap_tiles);
-      t.tile = t.gap ? local : local - of(gap_tiles);
-      t.row0 = t.gap ? of(gap0) : of(beg);
-      t.rows = t.gap ? of(gap_rows) : of(rows);
-      return true;
-    }
-    x -= __builtin_amdgcn_readlane(sum, 63);
-    covered = na_max(covered, __builtin_amdgcn_readlane(upto, 63));
-  }
-  return false;
-}
-
 constexpr uint32_t kGuardBits = (1u << 9) | (1u << 19) | (1u << 29);
 // a row's running maximum may lag the true one by up to this many powers of two
 constexpr float kLazyRescaleLog2 = 8.0f;

@@ -350,7 +350,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
 
 extern "C" {
 
-int natten_amd_abi_version(void) { return 19; }
+int natten_amd_abi_version(void) { return 20; }
 
 uint64_t natten_amd_fna_forward_workspace_bytes(void) { return uint64_t(kQueueWords) * 4; }
 
@@ -1224,13 +1224,16 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
 int natten_amd_attention_backward_varlen(const void* q, const void* k, const void* v, const void* d_out,
                                          const float* neg_lse2, const float* neg_delta, void* dq, void* dk, void* dv,
                                          void* q_scaled, int q_scaled_filled, int dtype, int num_seqs, int rows_q, int rows_kv,
-                                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv, int heads_q,
-                                         int heads_kv, int head_dim, int is_causal, float scale, void* stream) {
+                                         const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv,
+                                         const int32_t* packed_tiles, int heads_q, int heads_kv, int head_dim, int is_causal,
+                                         float scale, void* stream) {
   g_error[0] = 0;
   const char* what = "attention_backward_varlen";
   if (int rc = check_bwd_pointers(what, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 3)) return rc;
   if (int rc = check_common(what, q, k, v, dq, neg_lse2, num_seqs, rows_q, rows_kv, heads_q, heads_kv, head_dim)) return rc;
-  if (!cu_seqlens_q || !cu_seqlens_kv) return fail("%s: null cumulative length argument", what);
+  if (!cu_seqlens_q || !cu_seqlens_kv || !packed_tiles) return fail("%s: null cumulative length or packed_tiles argument", what);
+  if (reinterpret_cast<uintptr_t>(packed_tiles) & 7) return fail("%s: packed_tiles must be 8-byte aligned", what);
+  if (num_seqs > (1 << 28)) return fail("%s: more than 2^28 sequences", what);
   FnaBwdParams p;
   fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
                  q_scaled_filled);
@@ -1239,6 +1242,8 @@ int natten_amd_attention_backward_varlen(const void* q, const void* k, const voi
   p.kv_tiled[0] = rows_kv / 128 + 2 * (num_seqs + 1);
   p.cu_q = cu_seqlens_q;
   p.cu_kv = cu_seqlens_kv;
+  p.packed_q = reinterpret_cast<const int2*>(packed_tiles);
+  p.packed_kv = p.packed_q + (num_seqs + 2);
   p.num_seqs = num_seqs;
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), true);
 }
@@ -1290,7 +1295,8 @@ int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, i
 
 int natten_amd_backward_prepare(const void* q, const void* out, const void* d_out, const float* lse, void* q_scaled,
                                 float* neg_delta, float* neg_lse2, int dtype, int batch, int tokens, int heads, int head_dim,
-                                float scale, void* stream) {
+                                float scale, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_kv, int num_seqs,
+                                int rows_kv, int32_t* packed_tiles, void* stream) {
   g_error[0] = 0;
   const char* what = "backward_prepare";
   if (!q || !out || !d_out || !lse || !q_scaled || !neg_delta || !neg_lse2) return fail("%s: null pointer argument", what);
@@ -1298,17 +1304,31 @@ int natten_amd_backward_prepare(const void* q, const void* out, const void* d_ou
   if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(d_out) |
        reinterpret_cast<uintptr_t>(q_scaled)) & 15)
     return fail("%s: q, out, d_out and q_scaled must be 16-byte aligned", what);
+  PackedCounts packed;
+  memset(&packed, 0, sizeof(packed));
+  if (packed_tiles) {
+    if (!cu_seqlens_q || !cu_seqlens_kv || num_seqs < 1 || num_seqs > (1 << 28) || rows_kv < 1 || batch != 1)
+      return fail("%s: a packed batch needs both cumulative length arrays, its sequence and key row counts and batch 1", what);
+    if (reinterpret_cast<uintptr_t>(packed_tiles) & 7) return fail("%s: packed_tiles must be 8-byte aligned", what);
+    packed.cu_q = cu_seqlens_q;
+    packed.cu_kv = cu_seqlens_kv;
+    packed.q = reinterpret_cast<int2*>(packed_tiles);
+    packed.kv = packed.q + (num_seqs + 2);
+    packed.num_seqs = num_seqs;
+    packed.rows_q = tokens;
+    packed.rows_kv = rows_kv;
+  }
   int hb_lg = 0;
   while (hb_lg < 3 && heads % (2 << hb_lg) == 0) ++hb_lg;
   const int token_blocks = (tokens + (256 >> hb_lg) - 1) / (256 >> hb_lg), head_blocks = heads >> hb_lg;
-  const long long blocks = (long long)token_blocks * head_blocks * batch;
+  const long long blocks = (long long)token_blocks * head_blocks * batch + (packed_tiles ? 2 : 0);
   if (blocks > 0x7fffffffLL) return fail("%s: problem needs more than 2^31 workgroups", what);
   const float c_log2 = scale * 1.4426950408889634f;
   hipStream_t s = static_cast<hipStream_t>(stream);
 #define NA_PREPARE_LAUNCH(TYPE, DD)                                                                                        \
   hipLaunchKernelGGL((bwd_prepare_kernel<TYPE, DD>), dim3((unsigned)blocks), dim3(256), 0, s, static_cast<const TYPE*>(q),                     \
                      static_cast<const TYPE*>(out), static_cast<const TYPE*>(d_out), lse, static_cast<TYPE*>(q_scaled),       \
-                     neg_delta, neg_lse2, tokens, heads, hb_lg, na_make_div(head_blocks), na_make_div(token_blocks), c_log2)
+                     neg_delta, neg_lse2, tokens, heads, hb_lg, na_make_div(head_blocks), na_make_div(token_blocks), c_log2, packed)
 #define NA_PREPARE_DTYPE(DD)                                             \
   do {                                                                   \
     if (dtype == NATTEN_AMD_F16) NA_PREPARE_LAUNCH(_Float16, DD);        \

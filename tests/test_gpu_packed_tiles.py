@@ -44,3 +44,24 @@ def test_every_row_is_covered_once(num_seqs, head, tail):
         ref = O.attention_backward(*(to_np(t[:, a:b]) for t in (q, k, v, d_out)), is_causal=causal)
         for name, g, r in zip(("dq", "dk", "dv"), grads, ref):
             assert_close(f"{name} of sequence {i} of {num_seqs}, {b - a} rows", g[:, a:b], r, atol=2e-2, rtol=2e-2)
+
+
+def test_time_grows_with_the_sequences_not_with_their_square():
+    # 16 rows a sequence: eight times the sequences are eight times the tiles.  Finding a tile's sequence by
+    # counting through all lengths in every workgroup made it 64 times the counting (52 times the time; now 6.4).
+    def step(num_seqs):
+        cu = torch.arange(num_seqs + 1, dtype=torch.int32, device="cuda") * 16
+        q, k, v = (torch.randn((1, 16 * num_seqs, 4, 64), device="cuda", dtype=torch.bfloat16).requires_grad_(True) for _ in range(3))
+        out = natten_amd.attention(q, k, v, cumulative_seqlen_Q=cu, cumulative_seqlen_KV=cu, max_seqlen_Q=16, max_seqlen_KV=16)
+        d_out = torch.randn_like(out)
+        best = float("inf")
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            torch.autograd.grad(out, (q, k, v), d_out, retain_graph=True)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, start.elapsed_time(end))
+        return best
+
+    assert step(16384) < 16 * step(2048)
