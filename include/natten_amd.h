@@ -424,7 +424,8 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
  * [1, heads_q, rows_q].  Both cumulative arrays are device int32 [num_seqs + 1]: sequence b owns
  * rows cu_seqlens_q[b] .. cu_seqlens_q[b+1] - 1 of the queries, keys likewise.  dq, dk and dv are
  * written completely: rows of no sequence get zeros, and so do the rows of a sequence whose
- * offsets do not fit the row counts of the other side (the host cannot see the device arrays).
+ * offsets do not fit the row counts of either side or that reaches back over rows of an earlier
+ * sequence (the host cannot see the device arrays).
  * packed_tiles: what natten_amd_backward_prepare counted for the same two arrays and row counts.
  * No host synchronisation.
  */

@@ -164,12 +164,14 @@ static __device__ __forceinline__ void store_row_blocks(T* orow, const f32x16_t 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 
 // Tiles of a sequence-packed batch.  The rows 0 .. total - 1 of one side are the sequences cu[i] ..
-// cu[i + 1] - 1 (those whose offsets the rows can hold) and the gaps in front of and behind them, whose
-// rows belong to no sequence; tiles of 2^tile_lg rows are counted through both, a sequence's gap first,
-// the rows behind the last sequence as the gap of sequence num_seqs.  So a launch of total / tile + 2 (num_seqs
-// + 1) tiles per head covers any lengths, where one sized for the longest sequence starts a workgroup
-// per sequence and tile of that one (10 sequences of 1 .. 2048: 160 tiles a head instead of 72, of which
-// 87 find nothing to do).
+// cu[i + 1] - 1 (those whose offsets the rows can hold and that do not reach back over rows of an earlier
+// one) and the gaps around them, whose rows belong to no sequence; tiles of 2^tile_lg rows are counted
+// through both, a sequence's gap first, the rows behind the last sequence as the gap of sequence num_seqs.
+// Every row is in one sequence or gap, whatever the offsets: a launch leaves none unwritten.  There are at
+// most num_seqs + 2 of them (where a sequence follows one that counts, it begins where that ends: a gap takes
+// a sequence that does not count, or is the first or the last), so a launch of total / tile + num_seqs + 3
+// tiles per head covers any lengths, where one sized for the longest sequence starts a workgroup per sequence
+// and tile of that one (10 sequences of 1 .. 2048: 160 tiles a head, of which 87 find nothing to do).
 // One workgroup of the pass before counts (count_packed_tiles), and a tile finds its sequence in the
 // counts (locate_packed_tile): 64 places looked at per step, one step up to 64 sequences, three up to
 // 262144.  Counting through the lengths in every workgroup instead is quadratic in their number: 10000
@@ -187,11 +189,12 @@ static __device__ __forceinline__ PackedSeq packed_seq(const int32_t* cu, int i,
     end = cu[i + 1];
   }
   const bool valid = i < num_seqs && beg >= 0 && end >= beg && end <= total;
+  const bool counts = valid && beg >= covered;
   PackedSeq s;
   s.gap0 = covered;
-  s.gap_rows = na_max((i == num_seqs ? total : valid ? beg : 0) - covered, 0);
+  s.gap_rows = na_max((i == num_seqs ? total : counts ? beg : valid ? end : 0) - covered, 0);
   s.row0 = beg;
-  s.rows = valid ? end - beg : 0;
+  s.rows = counts ? end - beg : 0;
   s.end = valid ? end : 0;
   return s;
 }

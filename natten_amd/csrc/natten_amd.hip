@@ -1238,8 +1238,8 @@ int natten_amd_attention_backward_varlen(const void* q, const void* k, const voi
   fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
                  q_scaled_filled);
   // lengths and windows are replaced per sequence inside the kernel
-  p.q_tiled[0] = rows_q / 128 + 2 * (num_seqs + 1);
-  p.kv_tiled[0] = rows_kv / 128 + 2 * (num_seqs + 1);
+  p.q_tiled[0] = rows_q / 128 + num_seqs + 3;
+  p.kv_tiled[0] = rows_kv / 128 + num_seqs + 3;
   p.cu_q = cu_seqlens_q;
   p.cu_kv = cu_seqlens_kv;
   p.packed_q = reinterpret_cast<const int2*>(packed_tiles);

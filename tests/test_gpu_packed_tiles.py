@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import natten_amd
+from natten_amd import _lib
 from oracle import na_oracle as O
 from tests.gpu_utils import assert_close, to_np
 
@@ -65,3 +66,41 @@ def test_time_grows_with_the_sequences_not_with_their_square():
         return best
 
     assert step(16384) < 16 * step(2048)
+
+
+def _packed_backward(cu_q, cu_kv, rows, D):
+    """Gradients of the library's packed backward for any cumulative lengths, from made-up saved tensors."""
+    gen = torch.Generator().manual_seed(D)
+    q, d_out, out = (torch.randn((1, rows, 2, D), generator=gen).bfloat16().cuda() for _ in range(3))
+    k, v = (torch.randn((1, rows, 1, D), generator=gen).bfloat16().cuda() for _ in range(2))
+    lse = (torch.randn((1, rows, 2), generator=gen) + 6).cuda()
+    cus = [torch.tensor(cu, dtype=torch.int32, device="cuda") for cu in (cu_q, cu_kv)]
+    return _lib.attention_backward_varlen(q, k, v, out, d_out, lse, *cus, False, D**-0.5)
+
+
+@pytest.mark.parametrize("D", [32, 128])
+def test_malformed_lengths_are_not_followed(D):
+    # the first sequence is well-formed on both sides; the second's end lies past the rows, before them, or before its start
+    ref = _packed_backward([0, 40], [0, 40], 200, D)
+    for g in ref:
+        assert g[:, :40].any() and not g[:, 40:].any()
+    for tail in (5000, -7, 20):
+        for a, b in (([0, 40, tail], [0, 40, 200]), ([0, 40, 200], [0, 40, tail])):
+            for name, g, r in zip(("dq", "dk", "dv"), _packed_backward(a, b, 200, D), ref):
+                assert torch.equal(g, r), (name, a, b)
+
+
+@pytest.mark.parametrize("D", [32, 128])
+def test_rows_behind_overlapping_sequences_are_written(D):
+    # lengths that run back and forth over the same rows: the rows behind them belong to no sequence and get
+    # zeros (dq doubles as the workspace of the scaled queries: a row that no tile visits would keep those)
+    ref = _packed_backward([0, 1024], [0, 1024], 1300, D)
+    cu = [0, 1024] * 20
+    for name, g, r in zip(("dq", "dk", "dv"), _packed_backward(cu, cu, 1300, D), ref):
+        assert torch.equal(g, r), name
+    # one overlap on one side: the rows that only the overlapping sequence holds get zeros
+    dq, dk, dv = _packed_backward([0, 60, 40, 100], [0, 50, 80, 120], 300, D)
+    rq, rk, rv = _packed_backward([0, 60], [0, 50], 300, D)
+    assert torch.equal(dq, rq)
+    for g, r in ((dk, rk), (dv, rv)):
+        assert torch.equal(g[:, :50], r[:, :50]) and not g[:, 50:80].any() and not g[:, 120:].any() and g[:, 80:120].any()
