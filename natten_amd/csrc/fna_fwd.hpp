@@ -73,6 +73,7 @@ struct FnaParams {
   // would lie before the window; a tile that then reaches past the group is moved back as under
   // edge == 1 (every dilation group must be at least one KV tile wide in every dimension).
   int anchor;
+  int token_rows;     // a KV tile's first row is counted in tokens: the original layout, dense sequences (tok_stride 1, 0, 0)
   int tok_stride[3];  // tokens per unit step of an original coordinate: X1*X2, X2, 1
   int tokens;         // X0 * X1 * X2
   // Sequence-packed dense attention (RAGGED instances only; null otherwise): `batch` sequences
@@ -738,8 +739,14 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     bool skip;      // no key of the tile is attended by any query of this wave
     int lead[3];    // a tile moved back from the group's edge: its first lead[a] positions belong to the tile before it
   };
-  // (a packed sequence sums in the order in which a dense call on it alone does)
-  const bool move_back = p.edge == 1 || p.anchor || (RAGGED && p.cu_q != nullptr && seqlen_kv >= KVT);
+  // A tile that would reach past the group is moved back to end at the group's last position.  In the
+  // instances that clamp rows only the last tile of a packed sequence is (which then sums in the order in
+  // which a dense call on it alone does): one bound along dimension 0, and nothing the other dimensions and the
+  // token-permuted rows would pay for; a dense sequence's rows are counted by token like those of the original
+  // layout.  Against moving tiles in all dimensions there, and taking the distance off every permuted row:
+  // @@
+  const bool move_back = p.edge == 1 || p.anchor;
+  const int last_origin0 = (RAGGED && !p.fused && seqlen_kv >= KVT) ? seqlen_kv - KVT : 0x7fffffff;
   int itc[3] = {0, 0, 0};
   if constexpr (SPLIT) {
     itc[2] = first_tile % box_n[2];
@@ -759,16 +766,16 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
         t.full = t.full && (org >= wave_full_lo[a]) && (end <= wave_full_hi[a]);  // never when end > extent
         t.skip = t.skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
       }
-      // a tile that would reach past the group is moved back to end at the group's last position
-      t.origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
+      if constexpr (RAGGED) t.origin[a] = a == 0 ? na_min(org, last_origin0) : org;
+      else t.origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
       t.lead[a] = org - t.origin[a];
     }
     // (both forms are a handful of scalar operations: computed side by side and selected, a branch costs more)
-    const int row0_fused = t.origin[0] * tok_step[0] + t.origin[1] * tok_step[1] + t.origin[2] * tok_step[2];
+    const int row0_tokens = t.origin[0] * tok_step[0] + t.origin[1] * tok_step[1] + t.origin[2] * tok_step[2];
     const int row0_permuted = (((box_org[0] >> p.kv_tile_lg[0]) + itc[0]) +
                                p.kv_tiled[0] * (((box_org[1] >> p.kv_tile_lg[1]) + itc[1]) +
                                                 p.kv_tiled[1] * ((box_org[2] >> p.kv_tile_lg[2]) + itc[2]))) * KVT;
-    t.row0 = p.fused ? row0_fused : row0_permuted - t.lead[0];  // (only a dense sequence's last tile is moved back there)
+    t.row0 = (RAGGED || p.token_rows) ? row0_tokens : row0_permuted;  // (the clamping instances see no permuted rows)
     if (++itc[2] == box_n[2]) {
       itc[2] = 0;
       if (++itc[1] == box_n[1]) {

@@ -553,7 +553,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
     return fail("%s: a KV tile spans more than 2^31 bytes of the input; use the token-permuted entry point", what);
   p.seqlen_q = prod3(qs);
   p.seqlen_kv = prod3(ks);
-  p.fused = 1;
+  p.fused = p.token_rows = 1;
   p.edge = edge;
   // tiles laid out from the window's first key: needs every dilation group at least a KV tile wide
   p.anchor = (anchor_kv_tiles != 0 && edge != 2) ? 1 : 0;
@@ -826,6 +826,7 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
   p.q_tiled[0] = na_ceil_div(seqlen_q, QT);
   p.kv_tiled[0] = na_ceil_div(seqlen_kv, KVT);
   p.edge = (seqlen_kv % KVT != 0 && seqlen_kv >= KVT) ? 1 : 0;
+  p.token_rows = p.tok_stride[0] = 1;
   p.num_groups = 1;
   p.q = q;
   p.k = k;
@@ -878,6 +879,7 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
   p.kv_tile[0] = KVT;
   p.q_tiled[0] = na_ceil_div(max_seqlen_q, QT);
   p.kv_tiled[0] = na_ceil_div(max_seqlen_kv, KVT);
+  p.token_rows = p.tok_stride[0] = 1;
   p.num_groups = 1;
   p.q = q;
   p.k = k;
