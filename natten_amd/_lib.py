@@ -422,16 +422,16 @@ def fna_forward_fused_split(
     _require_gpu(q, k, v)
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd fna_forward_fused_split does not support {q.dtype}.")
+    q, k, v = _aligned_narrow_rows(q, k, v)
     na_dim = len(kernel_size)
-    qkv_shape = [int(x) for x in q.shape[1 : 1 + na_dim]]
     out = torch.empty((kv_splits, *q.shape), dtype=q.dtype, device=q.device)
     lse = torch.empty((kv_splits, *q.shape[:-1]), dtype=torch.float32, device=q.device)
     with _on_device(q):
         rc = L.natten_amd_fna_forward_fused_split(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
             DTYPE_CODES[q.dtype], na_dim, q.shape[0], q.shape[-2], k.shape[-2], q.shape[-1],
-            _i32(qkv_shape), _i32(kernel_size), _i32(stride), _i32(dilation),
-            _i32([1 if c else 0 for c in is_causal]), _i32(q_tile_shape), _i32(kv_tile_shape),
+            *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
+                             tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
             float(scale), 1 if anchored_tiles else 0, int(kv_splits), _stream(q),
         )
     _check(rc)

@@ -1309,10 +1309,10 @@ fna_fwd_kernel(const FnaParams p) {
 // fewer Q tiles than the chip keeps workgroups resident: a lone workgroup's tile loop is bound by
 // its own instruction issue, not by anything it shares, so two on half the tiles each take about
 // half the time.
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT>
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, int DC = 0>
 __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
 fna_fwd_split_kernel(const FnaParams p) {
-  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, true>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
 }
 
 // Work-queue launch: as many workgroups as the chip keeps resident, each taking Q tiles until

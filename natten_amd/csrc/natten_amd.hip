@@ -88,7 +88,7 @@ struct WorkQueue {
   bool clear_first = true;
 };
 
-// DC != 0: rows of p.row_dim elements, DC columns multiplied (a workgroup per Q tile only)
+// DC != 0: rows of p.row_dim elements, DC columns multiplied (no work-queue launch)
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
 int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   constexpr int QT = NWAVES * MQ * 32;
@@ -96,11 +96,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   if ((p.seqlen_q + QT - 1) / QT != p.num_q_tiles) return fail("fna_forward: internal tile count mismatch");
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
   if (wgs > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
-  if constexpr (DC != 0) {
-    hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
-                       stream, p);
-    return check_launch("fna_forward (narrow rows)");
-  } else {
+  if constexpr (DC == 0) {
     if (queues.counters != nullptr) {
       const long long resident = resident_workgroups();
       if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
@@ -109,23 +105,23 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
                          int(wgs / kNumXcd));
       return check_launch("fna_forward (work queue)");
     }
-    if (p.kv_splits > 1) {
-      // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
-      if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64) {
-        if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
-        FnaParams ps = p;
-        ps.split_grid = int(wgs);
-        hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT>), dim3((unsigned)(wgs * p.kv_splits)),
-                           dim3(NWAVES * 64), 0, stream, ps);
-        return check_launch("fna_forward (split)");
-      } else {
-        return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
-      }
-    }
-    hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0, stream,
-                       p);
-    return check_launch("fna_forward");
   }
+  if (p.kv_splits > 1) {
+    // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
+    if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64) {
+      if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
+      FnaParams ps = p;
+      ps.split_grid = int(wgs);
+      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>), dim3((unsigned)(wgs * p.kv_splits)),
+                         dim3(NWAVES * 64), 0, stream, ps);
+      return check_launch("fna_forward (split)");
+    } else {
+      return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
+    }
+  }
+  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
+                     stream, p);
+  return check_launch("fna_forward");
 }
 
 // Whether the launch is fully block-sparse: every Q tile is whole (no padding queries), all its
@@ -222,8 +218,8 @@ int dispatch_head_dim(const FnaParams& p, int head_dim, int qt, int kvt, hipStre
     case 128: return dispatch_tiles<T, 128>(p, qt, kvt, stream, queues);
   }
   if (!narrow_rows(head_dim)) return fail("fna_forward: head_dim must be 32, 64 or 128, got %d", head_dim);
-  if (qt != 128 || kvt != 64 || queues.counters != nullptr || p.kv_splits > 1 || p.cu_q != nullptr || p.row_dim != head_dim)
-    return fail("fna_forward: head_dim %d needs tiles of 128 x 64 tokens and a workgroup per Q tile", head_dim);
+  if (qt != 128 || kvt != 64 || queues.counters != nullptr || p.cu_q != nullptr || p.row_dim != head_dim)
+    return fail("fna_forward: head_dim %d needs tiles of 128 x 64 tokens and no work queue", head_dim);
   if (needs_clamped_rows(p, kvt)) return dispatch_narrow_rows<T, true>(p, head_dim, stream);
   return dispatch_narrow_rows<T, false>(p, head_dim, stream);
 }

@@ -102,8 +102,8 @@ def _prod(t) -> int:
 @functools.lru_cache(maxsize=1024)
 def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
     """What amd_fna_generic comes to for a forward call on checked arguments that fixes neither tiles nor route
-    nor splits and has no scales, where that is a single launch on the operands as they are: its tile shapes
-    and launch kind, or "float32"; None for everything else.  A small call is bound by the time it
+    nor splits and has no scales, where that runs on the operands as they are: its tile shapes,
+    launch kind and KV splits, or "float32"; None for everything else.  A small call is bound by the time it
     takes to get to its launch (256 tokens, float32: 23 us a call for 5 us of kernel), and the choices are a
     third of that time.  Plain values in and out: nothing here knows a tensor."""
     if dtype == torch.float32:
@@ -112,7 +112,7 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
     narrow = takes_narrow_rows(head_dim, dtype) and not run_persistent_kernel
     if dtype not in (torch.float16, torch.bfloat16) or (head_dim != padded_head_dim(head_dim) and not narrow):
         return None
-    from .functional import kv_splits_default, work_queue_default
+    from .functional import kv_splits_default, narrow_kv_splits_default, work_queue_default
 
     problem = (layout, kernel_size, stride, dilation, is_causal)
     tiles = choose_tile_shapes(*problem, *TILE_SIZES[0], anchored=True)
@@ -120,15 +120,15 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
     persistent = bool(run_persistent_kernel)
     if launch_left_open and not narrow:
         persistent = work_queue_default(shape[0], shape[-2], *problem, *tiles)
-    if not persistent and not narrow:
-        if kv_splits_default(shape[0], shape[-2], *problem, *tiles) != 1:
-            return None
-        if launch_left_open and head_dim <= 64:
+    splits = 1
+    if not persistent:
+        splits = (narrow_kv_splits_default if narrow else kv_splits_default)(shape[0], shape[-2], *problem, *tiles)
+        if splits == 1 and launch_left_open and not narrow and head_dim <= 64:
             tiles = choose_small_forward_tiles(*problem, *tiles) or tiles
     if not _lib.fused_layout_supported(layout, dilation, tiles[1], row_bytes=heads_kv * padded_head_dim(head_dim) * 2,
                                        q_tile_shape=tiles[0], dtype=dtype):
         return None
-    return (*tiles, persistent)
+    return (*tiles, persistent, splits)
 
 
 def amd_fna_generic(
@@ -194,8 +194,12 @@ def amd_fna_generic(
         if plan is not None:
             operands = (query.contiguous(), key.contiguous(), value.contiguous(), kernel_size, stride, dilation, is_causal,
                         scale or query.shape[-1] ** -0.5)
-            output, lse = (_lib.fna_forward_f32(*operands) if plan == "float32" else
-                           _lib.fna_forward_fused(*operands, plan[0], plan[1], run_persistent=plan[2]))
+            if plan == "float32":
+                output, lse = _lib.fna_forward_f32(*operands)
+            elif plan[3] > 1:
+                output, lse = _lib.merge_parts(*_lib.fna_forward_fused_split(*operands, plan[0], plan[1], plan[3]))
+            else:
+                output, lse = _lib.fna_forward_fused(*operands, plan[0], plan[1], run_persistent=plan[2])
             if out_dtype is not None and out_dtype != output.dtype:
                 output = output.to(out_dtype)
             return (output, lse) if return_lse else output
@@ -210,10 +214,10 @@ def amd_fna_generic(
     head_dim = query.shape[-1]
     scale = scale or head_dim**-0.5
     d_pad = padded_head_dim(head_dim)
-    # rows narrower than the kernels' are read as they are by a workgroup per Q tile of the default tiles; a
-    # work-queue or split launch that the caller asks for takes padded copies
+    # rows narrower than the kernels' are read as they are by workgroups on Q tiles of the default size; a
+    # work-queue launch that the caller asks for takes padded copies
     narrow = (takes_narrow_rows(head_dim, query.dtype) and fused is not False and not run_persistent_kernel
-              and kv_splits in (None, 1) and _prod(q_tile_shape) == 128 and _prod(kv_tile_shape) == 64)
+              and _prod(q_tile_shape) == 128 and _prod(kv_tile_shape) == 64)
     launch_left_open = run_persistent_kernel is None  # (the launch kinds promise each other's bits, hence tiles)
     if launch_left_open and not narrow:
         from .functional import work_queue_default
@@ -272,11 +276,11 @@ def amd_fna_generic(
     )
     narrow = narrow and fusable
     if kv_splits is None:
-        from .functional import kv_splits_default
+        from .functional import kv_splits_default, narrow_kv_splits_default
 
-        kv_splits = kv_splits_default(
+        kv_splits = (narrow_kv_splits_default if narrow else kv_splits_default)(
             query.shape[0], query.shape[-2], query.shape[1 : 1 + na_dim], kernel_size, stride, dilation, is_causal,
-            q_tile_shape, kv_tile_shape) if (splittable and anchored_tiles and not run_persistent_kernel and not narrow) else 1
+            q_tile_shape, kv_tile_shape) if (splittable and anchored_tiles and not run_persistent_kernel) else 1
     if not isinstance(kv_splits, int) or not 1 <= kv_splits <= 8:
         raise ValueError(f"natten_amd: kv_splits must be an integer from 1 to 8, got {kv_splits!r}.")
     if kv_splits > 1 and not splittable:

@@ -218,14 +218,20 @@ def work_queue_default(batch: int, heads: int, token_layout, kernel_size, stride
 
 @functools.lru_cache(maxsize=1024)
 def _work_queue_default(batch, heads, token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape):
-    tiles, visits = batch * heads, 1
+    tiles = batch * heads
+    for X, d, qt in zip(token_layout, dilation, q_tile_shape):
+        tiles *= -(-(-(-X // d)) // qt) * d
+    return _use_work_queue(None, is_causal, tiles, _kv_tiles_per_q_tile(
+        token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape))
+
+
+def _kv_tiles_per_q_tile(token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape) -> int:
+    """KV tiles a Q tile visits at most (causal masks and borders visit fewer)."""
+    visits = 1
     for X, k, s, d, qt, kt in zip(token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape):
-        extent = -(-X // d)
-        tiles *= -(-extent // qt) * d
         # keys the queries of one Q tile attend along this dimension: a window per stride group the tile spans
-        box = min(extent, k + (-(-qt // s) - 1) * s)
-        visits *= -(-box // kt)
-    return _use_work_queue(None, is_causal, tiles, visits)
+        visits *= -(-min(-(-X // d), k + (-(-qt // s) - 1) * s) // kt)
+    return visits
 
 
 @torch.compiler.assume_constant_result
@@ -240,6 +246,20 @@ def kv_splits_default(batch: int, heads: int, token_layout, kernel_size, stride,
     53 (no gain: the loop only shortens in proportion while a workgroup does not share its SIMDs)."""
     return _kv_splits_default(int(batch), int(heads), *(tuple(x) for x in (
         token_layout, kernel_size, dilation, is_causal, q_tile_shape, kv_tile_shape)))
+
+
+@torch.compiler.assume_constant_result
+def narrow_kv_splits_default(batch: int, heads: int, token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape,
+                             kv_tile_shape) -> int:
+    """kv_splits_default for rows between the native head dims, whose single launch has no padded copies beside it:
+    split from 24 KV tiles a Q tile on.  The device is faster split at any length (60 random problems), but a call
+    takes the host 30 us split and 20 in one launch, and up to there the one launch is over by then.  Measured
+    (one launch / split and merged, device us, bf16): 10 tiles, 4096 tokens, D 48 17.2 / 16.3; 18 tiles, 2048 tokens,
+    H 8, D 96 29.8 / 26.6; 27 tiles, 9 x 27 x 12, D 56 36.5 / 27.2; 34 tiles, 8192 tokens, D 96 44.3 / 26.4; 81 tiles, 16 x
+    32 x 32, D 96 114.6 / 68.6."""
+    if _kv_tiles_per_q_tile(token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape) < 24:
+        return 1
+    return kv_splits_default(batch, heads, token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape)
 
 
 @functools.lru_cache(maxsize=1024)

@@ -85,3 +85,27 @@ def test_launches_without_a_narrow_form_take_padded_copies():
     with pytest.raises(RuntimeError):
         torch_ops.fna_forward(q.flatten(1, 2), k.flatten(1, 2), v.flatten(1, 2), (7, 7), (1, 1), (1, 1), (False, False), 0.1,
                               (32, 32), (32, 32), (32, 32), (8, 16), (8, 8))
+
+
+@pytest.mark.parametrize("D", [40, 96, 120])
+def test_few_heads_share_the_key_tiles_of_a_query_tile(D):
+    # 16 query tiles of 26 key tiles: left open, the call splits the key tiles as it does at native head dims
+    q, k, v = make(1, (2048,), 1, 1, D, torch.bfloat16)
+    args = ((1500,), (1,), (1,), (False,), D**-0.5)
+    out, lse = amd_fna_generic(q, k, v, *args, return_lse=True)
+    ref, ref_lse = amd_fna_generic(padded(q), padded(k), padded(v), *args, return_lse=True, kv_splits=4)
+    assert torch.equal(out, ref[..., :D]) and torch.equal(lse, ref_lse)
+    one, _ = amd_fna_generic(q, k, v, *args, return_lse=True, kv_splits=1)
+    assert not torch.equal(out, one)
+    assert_close("split against unsplit", to_np(out), to_np(one))
+
+
+@pytest.mark.parametrize("case", CASES)
+@pytest.mark.parametrize("D", [56, 72, 104])
+def test_split_rows_as_they_are(case, D):
+    shape, kernel, stride, dilation, causal = case
+    q, k, v = make(2, shape, 4, 2, D, torch.float16)
+    args = (kernel, stride, dilation, causal, D**-0.5)
+    out, lse = amd_fna_generic(q, k, v, *args, return_lse=True, kv_splits=3)
+    ref, ref_lse = amd_fna_generic(padded(q), padded(k), padded(v), *args, return_lse=True, kv_splits=3)
+    assert torch.equal(out, ref[..., :D]) and torch.equal(lse, ref_lse)
