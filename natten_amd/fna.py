@@ -381,8 +381,6 @@ class AmdFnaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_output, d_lse):
-        if d_output is None:
-            return (None,) * 16
         query, key, value, output, lse = ctx.saved_tensors
         kernel_size, stride, dilation, is_causal, scale, q_tile, kv_tile = ctx.na_args
         head_dim = query.shape[-1]
@@ -410,6 +408,8 @@ class AmdFnaFunction(torch.autograd.Function):
                 roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation),
                                                          tuple(is_causal))
             if roles is not None and all(fits(qt, kt) for qt, kt in roles):
+        if d_output is None:  # (what came after the output passed no gradient on)
+            return tuple(torch.zeros_like(t) for t in (query, key, value)) + (None,) * 13
                 (q_tile, kv_tile), kv_role = roles
                 fused = True
             else:
