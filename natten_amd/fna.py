@@ -163,8 +163,10 @@ def amd_fna_generic(
     route); 1: never.  Results differ from the unsplit launch by the rounding of the partial outputs.
 
     `run_persistent_kernel`: work-queue launch of the forward kernel (resident workgroups pull
-    Q tiles from per-XCD queues) instead of a workgroup per Q tile; bit-identical results.  None:
-    whichever was measured faster for this kind of problem (`functional.work_queue_default`).
+    Q tiles from per-XCD queues) instead of a workgroup per Q tile; True gives the bits of an unsplit
+    False.  None: whichever was measured faster for this kind of problem (`functional.work_queue_default`);
+    the tiles are then open too (`choose_small_forward_tiles`, when `kv_splits` is None as well), and with
+    them the order of summation.
 
     `anchored_tiles` (one-launch path only): KV tiles are laid out from the first key of a Q tile's
     window instead of from multiples of the tile extent, so that no tile lies partly before the
@@ -173,7 +175,8 @@ def amd_fna_generic(
 
     `fused` selects the one-launch path that gathers tiles from the original tensors (None:
     whenever the problem allows it); otherwise tokens are permuted, multiplied and unpermuted
-    by separate kernels, as the reference does.  Both give bit-identical results.
+    by separate kernels, as the reference does.  Both give the same bits on the same tiles with `anchored_tiles`
+    False and no KV splits.
 
     8-bit float operands (e4m3fn / e5m2): `q_scale`, `k_scale`, `v_scale` (number or per-head
     tensor) are their dequantisation scales; `out_dtype` defaults to the dtype of `query`, as in
@@ -348,9 +351,6 @@ def amd_fna_generic(
     return output
 
 
-class AmdFnaFunction(torch.autograd.Function):
-    """Neighborhood attention with a backward pass (fp16 / bf16, head dims the kernels take).
-
 def backward_route(layout, kernel_size, stride, dilation, is_causal, row_bytes, q_tile, kv_tile, role_tiles=True, fused=None):
     """Whether a backward pass runs on the original tensors (the kernels gather and scatter their tiles themselves:
     no permuted copies), the tile shapes of its dq launch and those of its dk / dv launch where they differ from
@@ -373,6 +373,9 @@ def backward_route(layout, kernel_size, stride, dilation, is_causal, row_bytes, 
             return True, roles[0], roles[1]
     return fits(q_tile, kv_tile), (q_tile, kv_tile), (None, None)
 
+
+class AmdFnaFunction(torch.autograd.Function):
+    """Neighborhood attention with a backward pass (fp16 / bf16, head dims the kernels take).
 
     Mirrors the reference's autograd function (src/natten/backends/blackwell_fna.py:72-318):
     the forward saves q, k, v, out and LSE; the backward computes delta = rowsum(dO * O), permutes
@@ -405,11 +408,11 @@ def backward_route(layout, kernel_size, stride, dilation, is_causal, row_bytes, 
     @staticmethod
     def backward(ctx, d_output, d_lse):
         query, key, value, output, lse = ctx.saved_tensors
+        if d_output is None:  # (what came after the output passed no gradient on)
+            return tuple(torch.zeros_like(t) for t in (query, key, value)) + (None,) * 13
         kernel_size, stride, dilation, is_causal, scale, q_tile, kv_tile = ctx.na_args
         head_dim = query.shape[-1]
         d_pad = padded_head_dim(head_dim)
-        if d_output is None:  # (what came after the output passed no gradient on)
-            return tuple(torch.zeros_like(t) for t in (query, key, value)) + (None,) * 13
         # zero columns add nothing to q.k, dO.v or rowsum(dO * O); their gradients are dropped
         query, key, value, output, d_output = (
             pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, output, d_output)
