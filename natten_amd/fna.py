@@ -163,10 +163,8 @@ def amd_fna_generic(
     route); 1: never.  Results differ from the unsplit launch by the rounding of the partial outputs.
 
     `run_persistent_kernel`: work-queue launch of the forward kernel (resident workgroups pull
-    Q tiles from per-XCD queues) instead of a workgroup per Q tile; True gives the bits of an unsplit
-    False.  None: whichever was measured faster for this kind of problem (`functional.work_queue_default`);
-    the tiles are then open too (`choose_small_forward_tiles`, when `kv_splits` is None as well), and with
-    them the order of summation.
+    Q tiles from per-XCD queues) instead of a workgroup per Q tile; bit-identical results.  None:
+    whichever was measured faster for this kind of problem (`functional.work_queue_default`).
 
     `anchored_tiles` (one-launch path only): KV tiles are laid out from the first key of a Q tile's
     window instead of from multiples of the tile extent, so that no tile lies partly before the
@@ -175,8 +173,7 @@ def amd_fna_generic(
 
     `fused` selects the one-launch path that gathers tiles from the original tensors (None:
     whenever the problem allows it); otherwise tokens are permuted, multiplied and unpermuted
-    by separate kernels, as the reference does.  Both give the same bits on the same tiles with `anchored_tiles`
-    False and no KV splits.
+    by separate kernels, as the reference does.  Both give bit-identical results.
 
     8-bit float operands (e4m3fn / e5m2): `q_scale`, `k_scale`, `v_scale` (number or per-head
     tensor) are their dequantisation scales; `out_dtype` defaults to the dtype of `query`, as in
@@ -351,29 +348,6 @@ def amd_fna_generic(
     return output
 
 
-def backward_route(layout, kernel_size, stride, dilation, is_causal, row_bytes, q_tile, kv_tile, role_tiles=True, fused=None):
-    """Whether a backward pass runs on the original tensors (the kernels gather and scatter their tiles themselves:
-    no permuted copies), the tile shapes of its dq launch and those of its dk / dv launch where they differ from
-    them: (bool, (q tile, kv tile), (q tile, kv tile) or (None, None)).  `q_tile`, `kv_tile`: the problem's
-    common pair.
-
-    With `role_tiles` each launch takes the tile shapes that visit the fewest tiles for its role.  They are
-    chosen among those that fit the dilation groups, so a problem whose one common pair of shapes does not
-    fit stays off the permuted route too."""
-    def fits(qt, kt):
-        return _lib.backward_fused_layout_supported(layout, dilation, qt, kt, row_bytes=row_bytes)
-
-    if fused is False:
-        return False, (q_tile, kv_tile), (None, None)
-    if role_tiles:
-        from .tile_config import choose_backward_role_tile_shapes
-
-        roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation), tuple(is_causal))
-        if roles is not None and all(fits(qt, kt) for qt, kt in roles):
-            return True, roles[0], roles[1]
-    return fits(q_tile, kv_tile), (q_tile, kv_tile), (None, None)
-
-
 class AmdFnaFunction(torch.autograd.Function):
     """Neighborhood attention with a backward pass (fp16 / bf16, head dims the kernels take).
 
@@ -407,9 +381,9 @@ class AmdFnaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_output, d_lse):
+        if d_output is None:
+            return (None,) * 16
         query, key, value, output, lse = ctx.saved_tensors
-        if d_output is None:  # (what came after the output passed no gradient on)
-            return tuple(torch.zeros_like(t) for t in (query, key, value)) + (None,) * 13
         kernel_size, stride, dilation, is_causal, scale, q_tile, kv_tile = ctx.na_args
         head_dim = query.shape[-1]
         d_pad = padded_head_dim(head_dim)
@@ -418,10 +392,28 @@ class AmdFnaFunction(torch.autograd.Function):
             pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, output, d_output)
         )
         na_dim = len(kernel_size)
-        layout = tuple(int(x) for x in query.shape[1 : 1 + na_dim])
-        fused, (q_tile, kv_tile), kv_role = backward_route(
-            layout, kernel_size, stride, dilation, is_causal, query.shape[-2] * query.shape[-1] * 2, q_tile, kv_tile,
-            ctx.role_tiles, ctx.fused)
+        layout, row_bytes = tuple(int(x) for x in query.shape[1 : 1 + na_dim]), query.shape[-2] * query.shape[-1] * 2
+
+        def fits(qt, kt):
+            return _lib.backward_fused_layout_supported(layout, dilation, qt, kt, row_bytes=row_bytes)
+
+        # On the original tensors (the kernels gather and scatter their tiles themselves: no permuted
+        # copies) each launch takes the tile shapes that visit the fewest tiles for its role.  They are
+        # chosen among those that fit the dilation groups, so a problem whose one common pair of shapes
+        # does not fit stays off the permuted route too.
+        fused, kv_role = False, (None, None)
+        if ctx.fused is not False:
+            roles = None
+            if ctx.role_tiles:
+                from .tile_config import choose_backward_role_tile_shapes
+
+                roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation),
+                                                         tuple(is_causal))
+            if roles is not None and all(fits(qt, kt) for qt, kt in roles):
+                (q_tile, kv_tile), kv_role = roles
+                fused = True
+            else:
+                fused = fits(q_tile, kv_tile)
         if fused:
             dq, dk, dv = torch_ops.fna_backward_fused(
                 query, key, value, d_output, lse.contiguous(), None, kernel_size, stride, dilation, is_causal, scale,
