@@ -111,9 +111,9 @@ class AmdFmhaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_out, d_lse):
-        if d_out is None:
-            return (None,) * 5
         query, key, value, out, lse = ctx.saved_tensors
+        if d_out is None:  # (what came after the output passed no gradient on)
+            return (torch.zeros_like(query), torch.zeros_like(key), torch.zeros_like(value)) + (None,) * 2
         is_causal, scale = ctx.args
         head_dim = query.shape[-1]
         d_pad = padded_head_dim(head_dim)
@@ -146,17 +146,16 @@ class AmdFmhaVarlenFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_out, d_lse):
-        if d_out is None:
-            return (None,) * 9
         query, key, value, out, lse, cu_q, cu_kv = ctx.saved_tensors
         is_causal, scale = ctx.args
         head_dim = query.shape[-1]
+        max_q, max_kv = ctx.max_seqlens
+        if d_out is None or max_q == 0 or max_kv == 0 or query.shape[1] == 0 or key.shape[1] == 0:
+            # what came after the output passed no gradient on, or no sequence has both queries and keys: the
+            # output does not depend on the operands
+            return (torch.zeros_like(query), torch.zeros_like(key), torch.zeros_like(value)) + (None,) * 6
         d_pad = padded_head_dim(head_dim)
         q, k, v, o, do = (pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, out, d_out))
-        max_q, max_kv = ctx.max_seqlens
-        if max_q == 0 or max_kv == 0 or q.shape[1] == 0 or k.shape[1] == 0:
-            # no sequence has both queries and keys: the output does not depend on the operands
-            return (torch.zeros_like(query), torch.zeros_like(key), torch.zeros_like(value)) + (None,) * 6
         dq, dk, dv = torch_ops.attention_backward_varlen(
             q, k, v, o, do, lse.contiguous(), cu_q.to(torch.int32).contiguous(), cu_kv.to(torch.int32).contiguous(), is_causal,
             scale,

@@ -381,9 +381,9 @@ class AmdFnaFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_output, d_lse):
-        if d_output is None:
-            return (None,) * 16
         query, key, value, output, lse = ctx.saved_tensors
+        if d_output is None:  # (what came after the output passed no gradient on)
+            return tuple(torch.zeros_like(t) for t in (query, key, value)) + (None,) * 13
         kernel_size, stride, dilation, is_causal, scale, q_tile, kv_tile = ctx.na_args
         head_dim = query.shape[-1]
         d_pad = padded_head_dim(head_dim)

@@ -382,3 +382,28 @@ def test_backward_tile_shapes_per_launch_match_oracle_and_common_tiles():
         only_kv = _lib.fna_backward_fused(q, kk, v, d_out, lse, delta, k, s, d, causal, D ** -0.5, *roles[1])
     assert torch.equal(both[0], only_dq[0])                                   # dq: the dq launch's shapes
     assert torch.equal(both[1], only_kv[1]) and torch.equal(both[2], only_kv[2])  # dk, dv: the other launch's
+
+
+class PassesNoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x.sum()
+
+    @staticmethod
+    def backward(ctx, grad):
+        return None
+
+
+@pytest.mark.parametrize("form", ["neighborhood", "dense", "packed"])
+def test_output_whose_consumer_passes_no_gradient(form):
+    # the gradients are zeros, not "unused": torch.autograd.grad refuses the latter
+    if form == "neighborhood":
+        q, k, v = (t.requires_grad_(True) for t in make_qkv(1, (12, 14), 2, 2, 32, torch.bfloat16))
+        out = natten_amd.na2d(q, k, v, 5)
+    else:
+        q, k, v = (t.requires_grad_(True) for t in make_qkv(1, (150,), 2, 2, 64, torch.bfloat16))
+        cu = torch.tensor([0, 40, 150], dtype=torch.int32, device="cuda")
+        lengths = dict(cumulative_seqlen_Q=cu, cumulative_seqlen_KV=cu, max_seqlen_Q=110, max_seqlen_KV=110)
+        out = natten_amd.attention(q, k, v, **(lengths if form == "packed" else {}))
+    for t, g in zip((q, k, v), torch.autograd.grad(PassesNoGradient.apply(out), (q, k, v))):
+        assert g.shape == t.shape and g.dtype == t.dtype and not g.any()
