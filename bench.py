@@ -293,6 +293,7 @@ def bench_backward(args, q, k, v, kernel, stride, dilation, causal, dt_name):
 
     import natten_amd
     from natten_amd import _lib
+    from natten_amd.fna import backward_route
     from natten_amd.tile_config import check_fna_backward_config
     from natten_amd.token_permute import token_permute_operation
 
@@ -337,30 +338,20 @@ def bench_backward(args, q, k, v, kernel, stride, dilation, causal, dt_name):
         kp, _, kv_shape = perm(k, kv_tile)
         vp = perm(v, kv_tile)[0]
 
-        fused = _lib.backward_fused_layout_supported(layout, dilation, q_tile, kv_tile)
         qd, kd, vd = q.detach(), k.detach(), v.detach()
-        # left to itself the op gives each launch on the original tensors the tile shapes that suit its role
-        kv_role = (None, None)
-        if fused and not tiles_given:
-            from natten_amd.tile_config import choose_backward_role_tile_shapes
-
-            roles = choose_backward_role_tile_shapes(layout, tuple(kernel), tuple(stride), tuple(dilation), tuple(causal))
-            if roles is not None and all(_lib.backward_fused_layout_supported(layout, dilation, a, b) for a, b in roles):
-                (q_tile_dq, kv_tile_dq), kv_role = roles
-            else:
-                q_tile_dq, kv_tile_dq = q_tile, kv_tile
-        else:
-            q_tile_dq, kv_tile_dq = q_tile, kv_tile
+        # the route and the tile shapes per launch that the step above takes
+        fused, (q_tile_dq, kv_tile_dq), kv_role = backward_route(
+            layout, kernel, stride, dilation, causal, H * D * 2, q_tile, kv_tile, role_tiles=not tiles_given)
 
         def kern_permuted():
             return _lib.fna_backward(qp, kp, vp, dop, lp, dp, kernel, stride, dilation, causal, D**-0.5, q_shape,
                                      kv_shape, qkv_shape, q_tile, kv_tile)
 
         def kern():
-            # the launches the step above makes
+            # the launches of the step's backward
             if fused:
-                return _lib.fna_backward_fused(qd, kd, vd, d_out, lse, delta, kernel, stride, dilation, causal,
-                                               D**-0.5, q_tile_dq, kv_tile_dq, *kv_role)
+                return _lib.fna_backward_fused(qd, kd, vd, d_out, lse, None, kernel, stride, dilation, causal,
+                                               D**-0.5, q_tile_dq, kv_tile_dq, *kv_role, out=out)
             return kern_permuted()
 
         def timed(fn):

@@ -348,6 +348,29 @@ def amd_fna_generic(
     return output
 
 
+def backward_route(layout, kernel_size, stride, dilation, is_causal, row_bytes, q_tile, kv_tile, role_tiles=True, fused=None):
+    """Whether a backward pass runs on the original tensors (the kernels gather and scatter their tiles themselves:
+    no permuted copies), the tile shapes of its dq launch and those of its dk / dv launch where they differ from
+    them: (bool, (q tile, kv tile), (q tile, kv tile) or (None, None)).  `q_tile`, `kv_tile`: the problem's
+    common pair.
+
+    With `role_tiles` each launch takes the tile shapes that visit the fewest tiles for its role.  They are
+    chosen among those that fit the dilation groups, so a problem whose one common pair of shapes does not
+    fit stays off the permuted route too."""
+    def fits(qt, kt):
+        return _lib.backward_fused_layout_supported(layout, dilation, qt, kt, row_bytes=row_bytes)
+
+    if fused is False:
+        return False, (q_tile, kv_tile), (None, None)
+    if role_tiles:
+        from .tile_config import choose_backward_role_tile_shapes
+
+        roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation), tuple(is_causal))
+        if roles is not None and all(fits(qt, kt) for qt, kt in roles):
+            return True, roles[0], roles[1]
+    return fits(q_tile, kv_tile), (q_tile, kv_tile), (None, None)
+
+
 class AmdFnaFunction(torch.autograd.Function):
     """Neighborhood attention with a backward pass (fp16 / bf16, head dims the kernels take).
 
@@ -392,28 +415,10 @@ class AmdFnaFunction(torch.autograd.Function):
             pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, output, d_output)
         )
         na_dim = len(kernel_size)
-        layout, row_bytes = tuple(int(x) for x in query.shape[1 : 1 + na_dim]), query.shape[-2] * query.shape[-1] * 2
-
-        def fits(qt, kt):
-            return _lib.backward_fused_layout_supported(layout, dilation, qt, kt, row_bytes=row_bytes)
-
-        # On the original tensors (the kernels gather and scatter their tiles themselves: no permuted
-        # copies) each launch takes the tile shapes that visit the fewest tiles for its role.  They are
-        # chosen among those that fit the dilation groups, so a problem whose one common pair of shapes
-        # does not fit stays off the permuted route too.
-        fused, kv_role = False, (None, None)
-        if ctx.fused is not False:
-            roles = None
-            if ctx.role_tiles:
-                from .tile_config import choose_backward_role_tile_shapes
-
-                roles = choose_backward_role_tile_shapes(layout, tuple(kernel_size), tuple(stride), tuple(dilation),
-                                                         tuple(is_causal))
-            if roles is not None and all(fits(qt, kt) for qt, kt in roles):
-                (q_tile, kv_tile), kv_role = roles
-                fused = True
-            else:
-                fused = fits(q_tile, kv_tile)
+        layout = tuple(int(x) for x in query.shape[1 : 1 + na_dim])
+        fused, (q_tile, kv_tile), kv_role = backward_route(
+            layout, kernel_size, stride, dilation, is_causal, query.shape[-2] * query.shape[-1] * 2, q_tile, kv_tile,
+            ctx.role_tiles, ctx.fused)
         if fused:
             dq, dk, dv = torch_ops.fna_backward_fused(
                 query, key, value, d_output, lse.contiguous(), None, kernel_size, stride, dilation, is_causal, scale,

@@ -153,6 +153,20 @@ def test_route_predicates_keep_32_bit_tile_offsets():
     assert not _lib.fused_layout_supported((20, 24), (1, 1), (8, 8), row_bytes=1024)
 
 
+def test_backward_route_takes_role_tiles_where_the_common_pair_does_not_fit():
+    """4 x 56 x 56 tokens, 7 x 7 windows, head dim 32: what the autograd function and the benchmark both ask."""
+    from natten_amd.fna import backward_route
+
+    problem = ((56, 56), (7, 7), (1, 1), (1, 1), (False, False))
+    qt, kt = tile_config.choose_tile_shapes(*problem, 128, 128, anchored=False)
+    row_bytes = 8 * 32 * 2
+    assert not _lib.backward_fused_layout_supported(problem[0], problem[3], qt, kt, row_bytes=row_bytes)
+    fused, dq_tiles, kv_role = backward_route(*problem, row_bytes, qt, kt)
+    assert fused and (dq_tiles, kv_role) == tile_config.choose_backward_role_tile_shapes(*problem)
+    assert backward_route(*problem, row_bytes, qt, kt, role_tiles=False) == (False, (qt, kt), (None, None))
+    assert backward_route(*problem, row_bytes, qt, kt, fused=False) == (False, (qt, kt), (None, None))
+
+
 def test_backward_entry_point_rejects_tiles_beyond_32_bit_offsets():
     # argument validation happens before anything touches a device: fake (aligned, non-null)
     # pointers are never dereferenced on this path
