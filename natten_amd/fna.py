@@ -163,8 +163,10 @@ def amd_fna_generic(
     route); 1: never.  Results differ from the unsplit launch by the rounding of the partial outputs.
 
     `run_persistent_kernel`: work-queue launch of the forward kernel (resident workgroups pull
-    Q tiles from per-XCD queues) instead of a workgroup per Q tile; bit-identical results.  None:
-    whichever was measured faster for this kind of problem (`functional.work_queue_default`).
+    Q tiles from per-XCD queues) instead of a workgroup per Q tile; True gives the bits of an unsplit
+    False.  None: whichever was measured faster for this kind of problem (`functional.work_queue_default`);
+    the tiles are then open too (`choose_small_forward_tiles`, when `kv_splits` is None as well), and with
+    them the order of summation.
 
     `anchored_tiles` (one-launch path only): KV tiles are laid out from the first key of a Q tile's
     window instead of from multiples of the tile extent, so that no tile lies partly before the
@@ -173,7 +175,8 @@ def amd_fna_generic(
 
     `fused` selects the one-launch path that gathers tiles from the original tensors (None:
     whenever the problem allows it); otherwise tokens are permuted, multiplied and unpermuted
-    by separate kernels, as the reference does.  Both give bit-identical results.
+    by separate kernels, as the reference does.  Both give the same bits on the same tiles with `anchored_tiles`
+    False and no KV splits.
 
     8-bit float operands (e4m3fn / e5m2): `q_scale`, `k_scale`, `v_scale` (number or per-head
     tensor) are their dequantisation scales; `out_dtype` defaults to the dtype of `query`, as in

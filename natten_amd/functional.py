@@ -201,8 +201,8 @@ def _use_work_queue(run_persistent_kernel: Optional[bool], is_causal, num_q_tile
     one-workgroup-per-tile launch: 2.5-10 % on the large shapes measured, causal or not; on 2 048 Q
     tiles x 16 KV tiles (c3) the two are within 2 % of each other either way, and below that the queue's
     bookkeeping costs more than it saves.  `num_q_tiles`: Q tiles over all batch entries, dilation
-    groups and heads; `kv_tiles_per_q_tile`: KV tiles a Q tile visits (an estimate).  Results are
-    bit-identical either way."""
+    groups and heads; `kv_tiles_per_q_tile`: KV tiles a Q tile visits (an estimate).  True
+    and False give the same bits (without KV splits); None leaves the tile shapes open as well."""
     if run_persistent_kernel is not None:
         return bool(run_persistent_kernel)
     return num_q_tiles >= 2048 and num_q_tiles * kv_tiles_per_q_tile >= 65536
