@@ -408,7 +408,8 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
 /*
  * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
  * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2 = -log2(e) lse and neg_delta = -delta head-major
- * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above; q_scaled_filled != 0: it is filled already (natten_amd_backward_prepare).
+ * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above; q_scaled_filled != 0: it
+ * is filled already (by the same call).
  * Any sequence lengths: rows past the end of a sequence are gathered from its last row and masked.
  */
 int natten_amd_attention_backward(const void* q, const void* k, const void* v, const void* d_out,

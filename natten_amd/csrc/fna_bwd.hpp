@@ -297,23 +297,25 @@ static __device__ __forceinline__ bool locate_packed_tile(const int2* __restrict
   return true;
 }
 
-// Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to):
-// what each instance's registers allow without spilling (head dim 128: 222 and 256 of the SIMD's 512 per
-// lane; 64: 229 and 210; 32: 168 and 167).  Head dim 32 on 4 x 56 x 56 tokens, 7 x 7 windows with two
-// waves throughout: 82 (dK, dV) and 52 us (dQ).
-constexpr int bwd_waves_per_simd(int head_dim, int role) {
-  return head_dim == 128 ? 2 : head_dim == 64 ? 2 : 3;
-}
+// Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to).  Of the
+// SIMD's 512 registers a lane, the key-stationary and the dQ instance take 224 and 256 at head dim 128, 229 and
+// 210 at 64, 168 and 167 at 32; the dQ instance at 128 spills 9 more (11 where sequences end inside a tile).  One wave
+// more for the dQ role at 64 and 32 needs its LSE and delta in a register each instead of sixteen copies that
+// the accumulators start from, and two additions a logit: dQ launch in us, copies / one wave more, D 64: 48 x 48
+// tokens, H 6, 11 x 11 18.5 / 20.3; 4 x 56 x 56, H 8, 7 x 7 39.5 / 41.9; 16 x 40 x 40, H 12, 7 x 15 x 15 409 / 424; D 32: 24 x
+// 32 x 32, H 8, 9 x 9 x 9 105 / 115; 2 x 40 x 40, H 16, 25 x 25 31.9 / 36.2; 4 x 56 x 56, H 8, 7 x 7 33.3 / 32.1.
+// Head dim 32 with two waves instead of three on the last: 52, and dK and dV 82 instead of 59.
+constexpr int bwd_waves_per_simd(int head_dim) { return head_dim > 32 ? 2 : 3; }
 
 // RAGGED: dense attention whose sequences end inside a tile, packed ones among them.  Rows past the end
 // of a sequence are gathered from its last row; stationary ones store nothing, streamed ones are masked.
 // (Padding the sequences into copies first made 67 launches of a packed training step, of index arithmetic
-// and copies most of them: 10 sequences of 1 .. 2048, H 16 / 4, D 128 919 us, now 6 launches and 462 us.)
+// and copies most of them: 10 sequences of 1 .. 2048, H 16 / 4, D 128 919 us, now 6 launches and 424 us.)
 // RAW (key-stationary roles): LSE and delta as they are, scaled on the way from LDS to the accumulators
 // (the dQ role scales its two values per lane in every instance).
 template <typename T, int D, int ROLE, bool RAGGED = false, bool RAW = false>
 __global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256)
-__attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D, ROLE), bwd_waves_per_simd(D, ROLE))))
+__attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D), bwd_waves_per_simd(D))))
 fna_bwd_kernel(const FnaBwdParams p) {
   constexpr bool KV_STATIONARY = ROLE != kBwdDQ;
   constexpr bool PAIR = ROLE == kBwdPair;

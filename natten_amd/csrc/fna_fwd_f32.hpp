@@ -1,11 +1,11 @@
-// Neighborhood attention forward for float32 operands on gfx950: fna_fwd_f32_direct_kernel on the
-// original tensors (the default), fna_fwd_f32_kernel on token-permuted sequences (for callers that fix
-// tile shapes or ask for that route).
+// Neighborhood attention forward for float32 operands on gfx950, two kernels: fna_fwd_f32_direct_kernel on the
+// original tensors (the default; described where it stands), and fna_fwd_f32_kernel on token-permuted
+// sequences, for callers that fix tile shapes or ask for that route.
 // The reference runs float32 through its CUTLASS 2.x kernels and, on CPU, through flex attention
-// (SHI-Labs/NATTEN tests/test_fna.py:107-131 states the tolerance: 1e-4 on the output); here it is a
-// plain kernel of its own: S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x2_f32 (IEEE float32
-// products and sums), exact online softmax in float32 (no lazy rescale, P not rounded), every logit
-// tested against its query's window (no whole-tile classification).  One workgroup per Q tile of
+// (SHI-Labs/NATTEN tests/test_fna.py:107-131 states the tolerance: 1e-4 on the output).  Both kernels keep
+// products, sums and softmax in IEEE float32, P unrounded.  The permuted one: S^T = K Q^T and O^T += V^T P^T on
+// v_mfma_f32_32x32x2_f32, exact online softmax (its maximum is followed at once, the direct kernel's lags),
+// every logit tested against its query's window (no whole-tile classification), one workgroup per Q tile of
 // 128 rows, 64-key tiles staged through LDS with ordinary loads.
 #pragma once
 

@@ -1,6 +1,6 @@
-"""Driver of the MI355X fused neighborhood attention:
-forward = token permute -> fused kernel -> token unpermute (output and LSE), or one launch on
-the original tensors; backward = delta, token permutes, the dQ and dK/dV kernels, unpermutes.
+"""Driver of the MI355X fused neighborhood attention: forward and backward on the original tensors (the
+kernels gather their tiles themselves), or token permute -> kernels -> token unpermute where a caller fixes that
+route or a layout does not allow the other.
 
 Counterpart of the reference's src/natten/backends/blackwell_fna.py:72-318 (autograd function)
 and :332-407 (driver).
@@ -28,7 +28,7 @@ from .tile_config import (
 from .token_permute import token_permute_operation, token_unpermute_operation
 
 SUPPORTED_DTYPES = (torch.float16, torch.bfloat16, torch.float8_e4m3fn, torch.float8_e5m2)
-# neighborhood attention also takes float32 (forward only, token-permuted route, a kernel of its own)
+# neighborhood attention also takes float32 (forward only, kernels of its own)
 FNA_DTYPES = SUPPORTED_DTYPES + (torch.float32,)
 FP8_DTYPES = _lib.FP8_DTYPES
 

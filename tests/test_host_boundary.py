@@ -115,7 +115,7 @@ def test_cpu_tensors_are_rejected_not_emulated():
 
 def test_query_range_matches_brute_force():
     """The interval of queries whose window meets a run of keys (what the dK/dV kernel iterates
-    over): the library's bisection against an exhaustive scan with the oracle's window functions."""
+    over): the library's closed form against an exhaustive scan with the oracle's window functions."""
     from natten_amd import _lib
     from oracle import na_oracle as O
 
