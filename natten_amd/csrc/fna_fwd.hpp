@@ -341,6 +341,21 @@ struct FnaSmem {
   }
 };
 
+// Coordinates of KV tile i of a box of n[0] x n[1] x n[2] tiles, dimension 2 fastest: quotients by a rounded
+// reciprocal, then put right (boxes of several dimensions hold far fewer than 2^24 tiles).
+static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], int (&t)[3]) {
+#pragma unroll
+  for (int a = 2; a > 0; --a) {
+    const int d = n[a];
+    const int q = int(float(i) * __builtin_amdgcn_rcpf(float(d)));
+    const int rem = i - q * d;
+    const int off = rem < 0 ? -1 : (rem >= d ? 1 : 0);
+    t[a] = d == 1 ? 0 : rem - off * d;
+    i = d == 1 ? i : q + off;
+  }
+  t[0] = i;
+}
+
 // MQ 32-row query blocks per wave.  MQ = 1 runs two waves per SIMD (256 registers each);
 // MQ = 2 one wave per SIMD (512 registers: accumulators and Q fragments can sit in the
 // accumulation registers) and reads every K / V fragment from LDS once for two MFMAs.
@@ -401,6 +416,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   constexpr int MASK_ROWS = NOMASK ? 1 : KVT + 1;
   __shared__ __attribute__((aligned(16))) uint32_t sKeys[NOMASK ? 1 : 3][2][MASK_ROWS];
   __shared__ __attribute__((aligned(16))) int sWin[NOMASK ? 1 : NWAVES * MQ * 32][8];
+  //   sTile[wave * 64 + i]  the i-th described KV tile (see describe)
+  __shared__ __attribute__((aligned(16))) int sTile[NOMASK ? 1 : NWAVES * 64][4];
   __shared__ __attribute__((aligned(16))) int sGeo[4];
   static_assert(NOMASK || KVT == 64, "the element mask holds one bit per key of a 64-key tile");
 
@@ -589,8 +606,11 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const int64_t q_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : q_seq_row0;
   const int64_t kv_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : kv_seq_row0;
   const T* qbase = reinterpret_cast<const T*>(p.q) + q_row_base * q_row_stride + int64_t(head) * row_dim;
-  const T* kbase = reinterpret_cast<const T*>(p.k) + kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim;
-  const T* vbase = reinterpret_cast<const T*>(p.v) + kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim;
+  // (less the bias of the copies' per-lane offsets, see below)
+  constexpr int kImmBias = RAGGED ? 0 : 3 * 1024;  // largest immediate offset of a copy
+  const int64_t kv_base = (kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim) * 2 - kImmBias;
+  const char* kbase = static_cast<const char*>(p.k) + kv_base;
+  const char* vbase = static_cast<const char*>(p.v) + kv_base;
   if constexpr (NARROW) {
     // (every copy leaves out the same places, so this is needed once)
     for (int i = tid; i < TILE_BYTES / 16; i += NT) {
@@ -619,7 +639,6 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // the per-lane offset again), and copy i + 4 lies a whole number of swizzle periods (16 rows
   // or more) below copy i, so it reuses that copy's per-lane offset on a shifted base.
   constexpr int NOFF = PER < 4 ? PER : 4;
-  constexpr int kImmBias = 3 * 1024;  // largest immediate offset of a copy
   constexpr int ROWS_PER_4 = 256 / CPR;  // rows between copy i and copy i + 4
   // Copy i + 4 (only waves with eight copies have one) sets one more bit of the tile position;
   // tile extents are powers of two, so that bit moves one coordinate by a fixed amount and the
@@ -643,6 +662,74 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       ld_voff[i] += uint32_t(kImmBias - i * 1024);
     }
   }
+  // KV tile stream: dimension 2 fastest, dimension 0 slowest.  The tiles are described 64 at a time, one
+  // per lane, and a tile's description is read back by lane number: its first row, and whether all keys
+  // are attended by all queries of this wave (no mask) or none by any.  Forming it tile by tile on the
+  // scalar unit took some ninety of the 120-140 scalar instructions that an iteration had, each an issue
+  // slot of a wave that also has to keep the matrix pipe fed (2 x 4097 tokens, dense, H 16, D 64: 200 -> 177 us; 32768
+  // tokens, window 2048, H 1, D 128: 47.3 -> 44.6; 30 x 48 x 80, window 18 x 24 x 24, H 24, D 128: 9.38 -> 9.11 ms;
+  // the D 64 and D 128 instances no longer spill scalars).  The load stream runs two tiles ahead of the
+  // softmax, so the lanes are moved on by 32 tiles when it reaches their end, which leaves the tiles still
+  // in use described.
+  // A tile that would reach past the group is moved back to end at the group's last position.  In the
+  // instances that clamp rows only the last tile of a packed sequence is (which then sums in the order in
+  // which a dense call on it alone does): one bound along dimension 0, and nothing the other dimensions and the
+  // token-permuted rows would pay for; a dense sequence's rows are counted by token like those of the original
+  // layout.  Against moving tiles in all dimensions there, and taking the distance off every permuted row:
+  // 31 x 25 x 17 tokens, dilation 2 x 1 x 3, H 8, D 128: 126 -> 116 us; 8 spilled scalars -> 2 at D 64 and D 128.
+  const bool move_back = p.edge == 1 || p.anchor;
+  const int last_origin0 = (RAGGED && !p.fused && seqlen_kv >= KVT) ? seqlen_kv - KVT : 0x7fffffff;
+  int d_first = 0;           // number of the tile that lane 0 describes
+  int d_row0 = 0;            // first row of the lane's tile in the permuted KV sequence / token offset of its origin (fused)
+  // What only some tiles ask for, kept in LDS (in registers the instances of head dim 128 spill): the coordinate of
+  // the tile's first token (a tile moved back from the group's edge: of the first one gathered), whose first
+  // (lead >> 8 a) & 255 positions along dimension a belong to the tile before it.
+  int d_origin[3] = {0, 0, 0};  // (RAGGED instances, whose copies look at it)
+  uint64_t d_plain = ~uint64_t(0);  // by lane: every key of the tile is attended by every query of this wave
+  uint64_t d_skip = 0;              // ... no key of the tile is attended by any query of this wave
+  auto describe = [&](int first) __attribute__((always_inline)) {
+    d_first = first;
+    // lanes past the last tile describe that one again: copies past the end re-read it into a free stage (never used)
+    int t[3];
+    kv_tile_of_box(first_tile + na_min(first + lane, total_tiles - 1), box_n, t);
+    bool full = true, skip = false;
+    int lead = 0;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const int org = box_org[a] + (t[a] << p.kv_tile_lg[a]);
+      const int end = org + p.kv_tile[a];
+      if constexpr (!NOMASK) {
+        full = full && (org >= wave_full_lo[a]) && (end <= wave_full_hi[a]);  // never when end > extent
+        skip = skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
+      }
+      if constexpr (RAGGED) d_origin[a] = a == 0 ? na_min(org, last_origin0) : org;
+      else d_origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
+      lead |= (org - d_origin[a]) << (8 * a);
+    }
+    if constexpr (!NOMASK) {
+      typedef int i32x4 __attribute__((ext_vector_type(4)));
+      *reinterpret_cast<i32x4*>(&sTile[wave * 64 + lane][0]) = i32x4{d_origin[0], d_origin[1], d_origin[2], lead};
+    }
+    // (the clamping instances see no permuted rows, and hold tok_step anyway)
+    const int* row_step = RAGGED ? tok_step : p.kv_row_step;
+    d_row0 = d_origin[0] * row_step[0] + d_origin[1] * row_step[1] + d_origin[2] * row_step[2];
+    if constexpr (!NOMASK && (kAblate & kAblateMask) == 0) {
+      d_plain = __ballot(full && !skip);
+      d_skip = __ballot(skip);
+    }
+  };
+  // where the rows of a described tile lie
+  struct TileRows {
+    int row0;
+    uint64_t bytes;  // row0 in bytes
+  };
+  auto tile_rows = [&](int l) __attribute__((always_inline)) {
+    TileRows t;
+    t.row0 = __builtin_amdgcn_readlane(d_row0, l);
+    t.bytes = uint64_t(uint32_t(t.row0)) * uint32_t(kv_row_stride * 2);
+    return t;
+  };
+
   // One operand tile in flight: uniform source base, LDS destination of this wave's share.
   struct TileCopy {
     const char* src;  // first row of the tile (this head)
@@ -651,18 +738,20 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     int lim[3];       // original layout: positions of the tile that lie inside the dilation group, per dimension
     bool inside;      // the whole tile lies inside the sequence / the dilation group
   };
-  auto make_copy = [&](const T* base, char* dst, int kv_row0, const int (&origin)[3]) {
+  // `l`: place of the tile among the described ones (RAGGED instances, which look at its origin)
+  auto make_copy = [&](const char* base, char* dst, const TileRows& t, int l) {
     TileCopy c;
-    kv_row0 = __builtin_amdgcn_readfirstlane(kv_row0);  // uniform by construction; keeps the base in scalar registers
-    c.src = reinterpret_cast<const char*>(base) + int64_t(kv_row0) * kv_row_stride * 2 - (RAGGED ? 0 : kImmBias);
+    c.src = base + t.bytes;
     c.lds0 = lds_address(dst) + uint32_t(wave * PER * 1024);
-    c.row0 = kv_row0;
     c.inside = true;
     if constexpr (RAGGED) {
+      const int kv_row0 = t.row0;
+      c.row0 = kv_row0;
       if (p.fused) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-          c.lim[a] = na_min(extent[a] - origin[a], p.kv_tile[a]);
+          const int origin = __builtin_amdgcn_readlane(d_origin[a], l);
+          c.lim[a] = na_min(extent[a] - origin, p.kv_tile[a]);
           c.inside = c.inside && (c.lim[a] == p.kv_tile[a]);
         }
       } else {
@@ -722,9 +811,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
   };
   static_assert(PER <= 8, "tile copy is written for at most eight copies per thread");
-  auto issue_tile_load = [&](const T* base, const uint32_t (&off)[NOFF], char* dst, int kv_row0, const int (&origin)[3],
-                             auto v_tag) {
-    const TileCopy c = make_copy(base, dst, kv_row0, origin);
+  auto issue_tile_load = [&](const char* base, const uint32_t (&off)[NOFF], char* dst, const TileRows& t, int l, auto v_tag) {
+    const TileCopy c = make_copy(base, dst, t, l);
     copy_one(std::integral_constant<int, 0>{}, c, off, v_tag);
     copy_one(std::integral_constant<int, 1>{}, c, off, v_tag);
     copy_one(std::integral_constant<int, 2>{}, c, off, v_tag);
@@ -735,70 +823,16 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     copy_one(std::integral_constant<int, 7>{}, c, off, v_tag);
   };
 
-  // KV tile stream: dimension 2 fastest, dimension 0 slowest.  The load stream runs up to two
-  // tiles ahead of the softmax, so tile descriptors are produced in order and handed down.
-  struct TileInfo {
-    int row0;       // first row of the tile in the permuted KV sequence / token offset of its origin (fused)
-    int origin[3];  // coordinate of its first token (a tile moved back from the group's edge: of the first one gathered)
-    bool full;      // every key of the tile is attended by every query of this wave
-    bool skip;      // no key of the tile is attended by any query of this wave
-    int lead[3];    // a tile moved back from the group's edge: its first lead[a] positions belong to the tile before it
-  };
-  // A tile that would reach past the group is moved back to end at the group's last position.  In the
-  // instances that clamp rows only the last tile of a packed sequence is (which then sums in the order in
-  // which a dense call on it alone does): one bound along dimension 0, and nothing the other dimensions and the
-  // token-permuted rows would pay for; a dense sequence's rows are counted by token like those of the original
-  // layout.  Against moving tiles in all dimensions there, and taking the distance off every permuted row:
-  // 31 x 25 x 17 tokens, dilation 2 x 1 x 3, H 8, D 128: 126 -> 116 us; 8 spilled scalars -> 2 at D 64 and D 128.
-  const bool move_back = p.edge == 1 || p.anchor;
-  const int last_origin0 = (RAGGED && !p.fused && seqlen_kv >= KVT) ? seqlen_kv - KVT : 0x7fffffff;
-  int itc[3] = {0, 0, 0};
-  if constexpr (SPLIT) {
-    itc[2] = first_tile % box_n[2];
-    const int rest = first_tile / box_n[2];
-    itc[1] = rest % box_n[1];
-    itc[0] = rest / box_n[1];
-  }
-  auto next_tile = [&]() {
-    TileInfo t;
-    t.full = true;
-    t.skip = false;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const int org = box_org[a] + (itc[a] << p.kv_tile_lg[a]);
-      const int end = org + p.kv_tile[a];
-      if constexpr (!NOMASK) {
-        t.full = t.full && (org >= wave_full_lo[a]) && (end <= wave_full_hi[a]);  // never when end > extent
-        t.skip = t.skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
-      }
-      if constexpr (RAGGED) t.origin[a] = a == 0 ? na_min(org, last_origin0) : org;
-      else t.origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
-      t.lead[a] = org - t.origin[a];
-    }
-    // (the clamping instances see no permuted rows, and hold tok_step anyway)
-    const int* row_step = RAGGED ? tok_step : p.kv_row_step;
-    t.row0 = t.origin[0] * row_step[0] + t.origin[1] * row_step[1] + t.origin[2] * row_step[2];
-    if (++itc[2] == box_n[2]) {
-      itc[2] = 0;
-      if (++itc[1] == box_n[1]) {
-        itc[1] = 0;
-        ++itc[0];
-      }
-    }
-    if constexpr (NOMASK || (kAblate & kAblateMask) != 0) {
-      t.full = true;
-      t.skip = false;
-    }
-    return t;
-  };
-
   using Stage0 = std::integral_constant<int, 0>;
   using Stage1 = std::integral_constant<int, 1>;
-  TileInfo cur = next_tile();  // tile 0
   using KLayout = std::false_type;
   using VLayout = std::true_type;
-  issue_tile_load(kbase, ld_koff, sK0, cur.row0, cur.origin, KLayout{});
-  issue_tile_load(vbase, ld_voff, sV0, cur.row0, cur.origin, VLayout{});
+  describe(0);
+  {
+    const TileRows rows = tile_rows(0);
+    issue_tile_load(kbase, ld_koff, sK0, rows, 0, KLayout{});
+    issue_tile_load(vbase, ld_voff, sV0, rows, 0, VLayout{});
+  }
 
   float sm_scale = p.scale, out_scale = 1.f;
   if (p.q_scale) sm_scale *= p.q_scale[head];
@@ -1050,16 +1084,17 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     asm volatile("" : "+v"(c_init[mb]));
   };
   // masks (PARTIAL tiles) and maxima of a whole tile of logits, outside the slots
-  auto finish_logits = [&](f32x16_t (&S)[MQ][NSB], const TileInfo& t, bool have_max, const float (&mx_in)[MQ]) __attribute__((always_inline)) {
+  // (`l`: place of the tile among the described ones)
+  auto finish_logits = [&](f32x16_t (&S)[MQ][NSB], int l, bool have_max, const float (&mx_in)[MQ]) __attribute__((always_inline)) {
     // One test on the way of a tile that needs nothing (attended in full, maxima at hand): every
     // wave-uniform branch in the tile loop costs about a hundredth of its time.
-    const bool t_full = t.full, t_skip = t.skip;
-    const bool plain = t_full && !t_skip && have_max;
+    const bool full = (d_plain >> l) & 1;
+    const bool plain = full && have_max;
 #pragma unroll
     for (int mb = 0; mb < MQ; ++mb) {
       float mx = mx_in[mb];
       if (__builtin_expect(!plain, 0)) {
-        if (t_skip) {
+        if ((d_skip >> l) & 1) {
           // none of this wave's queries attends the tile: every logit is masked
           mx = -INFINITY;
 #pragma unroll
@@ -1067,7 +1102,17 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 #pragma unroll
             for (int r = 0; r < 16; ++r) S[mb][sb][r] = -INFINITY;
         } else {
-          if (!t_full) apply_mask(S[mb], mb, t.origin, t.lead);
+          if (!full) {
+            int origin[3], lead[3];
+            typedef int i32x4 __attribute__((ext_vector_type(4)));
+            const i32x4 tile = *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+              origin[a] = tile[a];
+              lead[a] = (tile[3] >> (8 * a)) & 255;
+            }
+            apply_mask(S[mb], mb, origin, lead);
+          }
           mx = -INFINITY;
 #pragma unroll
           for (int sb = 0; sb < NSB; ++sb)
@@ -1084,10 +1129,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // and V(j+1); (G2, G3) the slots of O += P(j) V(j), the second half with the row maxima of
   // S(j+1).  The exponentials of S(j) are spread evenly over all of them.
   // LDS: K(j) and V(j) live in stage j % 2.
-  TileInfo nxt = next_tile();  // tile 1 (a descriptor past the box is never used)
+  TileRows nxt = tile_rows(1);  // tile 1
   wait_vmcnt<0>();
   workgroup_sync();  // K(0), V(0), the mask tables and the queries' windows are in LDS
-  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt.row0, nxt.origin, KLayout{});
+  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, 1, KLayout{});
 #pragma unroll
   for (int mb = 0; mb < MQ; ++mb)
 #pragma unroll
@@ -1106,7 +1151,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       for (int mb = 0; mb < MQ; ++mb) S_a[mb][s / KSTEPS] = M::run(kf, qf[mb][s % KSTEPS], S_a[mb][s / KSTEPS]);
     }
     const float none[MQ] = {};
-    finish_logits(S_a, cur, false, none);
+    finish_logits(S_a, 0, false, none);
   }
 
   // CUR / NXT: this wave attends keys of tile j / tile j + 1; an inactive tile only takes part
@@ -1122,18 +1167,21 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     char* sV_cur = st ? sV1 : sV0;  // holds V(j)
     char* sV_nxt = st ? sV0 : sV1;  // held V(j-1): free, receives V(j+1)
 
+    if constexpr (st == 0) {  // (64 and the first tile described are even)
+      if (j + 2 - d_first == 64) describe(d_first + 32);
+    }
     wait_vmcnt<0>();   // this thread's copies of K(j+1) and V(j) have landed
     if constexpr ((kAblate & kAblateBarrier) == 0)
       workgroup_sync();   // ... and everyone's; everyone is done reading K(j) and V(j-1)
-    const TileInfo t2 = next_tile();
-    // Past the end of the box the spread copies re-read the current tile into the free stage
+    // Past the end of the box the spread copies re-read its last tile into the free stage
     // (never used), which keeps the slots below free of control flow.
-    // (the spread copies only exist without RAGGED, where a tile's origin is not looked at)
-    const TileCopy ck = make_copy(kbase, sK_cur, (j + 2 < total_tiles) ? t2.row0 : cur.row0, cur.origin);
-    const TileCopy cv = make_copy(vbase, sV_nxt, (j + 1 < total_tiles) ? nxt.row0 : cur.row0, cur.origin);
+    const int l2 = j + 2 - d_first;
+    const TileRows t2 = tile_rows(l2);
+    const TileCopy ck = make_copy(kbase, sK_cur, t2, l2);
+    const TileCopy cv = make_copy(vbase, sV_nxt, nxt, l2 - 1);
     if constexpr (!SPREAD && (kAblate & kAblateCopies) == 0) {
-      if (j + 2 < total_tiles) issue_tile_load(kbase, ld_koff, sK_cur, t2.row0, t2.origin, KLayout{});
-      if (j + 1 < total_tiles) issue_tile_load(vbase, ld_voff, sV_nxt, nxt.row0, nxt.origin, VLayout{});
+      if (j + 2 < total_tiles) issue_tile_load(kbase, ld_koff, sK_cur, t2, l2, KLayout{});
+      if (j + 1 < total_tiles) issue_tile_load(vbase, ld_voff, sV_nxt, nxt, l2 - 1, VLayout{});
     }
 
     // -- G1 ------------------------------------------------------------------------------------
@@ -1251,9 +1299,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       float mxs[MQ];
 #pragma unroll
       for (int mb = 0; mb < MQ; ++mb) mxs[mb] = fmaxf(mx[mb][0], mx[mb][1]);
-      finish_logits(S_nxt, nxt, true, mxs);
+      finish_logits(S_nxt, j + 1 - d_first, true, mxs);
     }
-    cur = nxt;
     nxt = t2;
   };
   // A tile this wave has no use for (skip) is still multiplied and then masked entirely:
