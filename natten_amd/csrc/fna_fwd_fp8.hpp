@@ -31,7 +31,11 @@ static __device__ __forceinline__ i32x2_t lds_read_tr8(const char* p) {
 constexpr float kFp8ProbLog2Scale = 6.0f;   // P is stored as 2^6 * exp(...)
 constexpr float kFp8LazyRescaleLog2 = 2.0f; // so that 2^6 * 2^2 = 256 stays below e4m3's 448
 
-// One 32-row query block per wave, 64-key tiles, two waves per SIMD.  D = 64 or 128.
+// Waves per SIMD: a lane takes 225 to 234 of the SIMD's 512 registers at head dim 128, 161 at 64 (16 x 64 x 64 tokens,
+// window 8 x 16 x 16, H 16, D 64: 1487 us with two waves, 1331 with three; 8 x 32 x 40, 4 x 9 x 11, H 8: 67.3 and 52.4).
+constexpr int fp8_waves_per_simd(int head_dim) { return head_dim > 64 ? 2 : 3; }
+
+// One 32-row query block per wave, 64-key tiles.  D = 64 or 128.
 // LDS tile: 64 rows of D bytes, 16-byte chunks XOR-swizzled by (row / rows-per-256-bytes); the
 // rows of a V tile are stored in the order the P fragment holds its keys (see v_key_of_lds_row).
 // `pid`: the launch position (the workgroup id of a launch with one workgroup per Q tile).
@@ -63,6 +67,8 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   __shared__ __attribute__((aligned(1024))) char sK1[TILE_BYTES];
   __shared__ __attribute__((aligned(1024))) char sV1[TILE_BYTES];
   __shared__ __attribute__((aligned(16))) uint32_t sTab[NOMASK ? 1 : KVT];
+  __shared__ __attribute__((aligned(16))) int sTile[NOMASK ? 1 : NT][4];  // origins of the described KV tiles
+  __shared__ __attribute__((aligned(16))) int sWin[NOMASK ? 1 : QT][8];   // windows of the Q tile's queries (row-major): start and end per dimension
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -185,8 +191,11 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   const int64_t q_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : int64_t(bg) * p.seqlen_q;
   const int64_t kv_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : int64_t(bg) * p.seqlen_kv;
   const uint8_t* qbase = static_cast<const uint8_t*>(p.q) + q_row_base * q_row_stride + int64_t(head) * D;
-  const uint8_t* kbase = static_cast<const uint8_t*>(p.k) + kv_row_base * kv_row_stride + int64_t(head_kv) * D;
-  const uint8_t* vbase = static_cast<const uint8_t*>(p.v) + kv_row_base * kv_row_stride + int64_t(head_kv) * D;
+  // (less the bias of the copies' per-lane offsets, see below)
+  constexpr int kImmBias = 3 * 1024;
+  const int64_t kv_base = kv_row_base * kv_row_stride + int64_t(head_kv) * D - kImmBias;
+  const char* kbase = static_cast<const char*>(p.k) + kv_base;
+  const char* vbase = static_cast<const char*>(p.v) + kv_base;
   // row (permuted) or token offset (fused) of position `r` (dimension 0 fastest) of a KV tile
   auto kv_tile_pos = [&](int r) {
     if (!p.fused) return r;
@@ -195,9 +204,7 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
     return t0 * tok_step[0] + (r & (p.kv_tile[1] - 1)) * tok_step[1] + (r >> p.kv_tile_lg[1]) * tok_step[2];
   };
 
-
   // ---- async tile loads (see fna_fwd_kernel): copy i of wave w fills LDS chunks (w*PER + i)*64 .. +63
-  constexpr int kImmBias = 3 * 1024;
   uint32_t ld_koff[PER], ld_voff[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
@@ -211,10 +218,9 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
     const char* src;
     uint32_t lds0;
   };
-  auto make_copy = [&](const uint8_t* base, char* dst, int kv_row0) {
+  auto make_copy = [&](const char* base, char* dst, uint64_t row_bytes) {
     TileCopy c;
-    kv_row0 = __builtin_amdgcn_readfirstlane(kv_row0);
-    c.src = reinterpret_cast<const char*>(base) + int64_t(kv_row0) * kv_row_stride - kImmBias;
+    c.src = base + row_bytes;
     c.lds0 = lds_address(dst) + uint32_t(wave * PER * 1024);
     return c;
   };
@@ -222,61 +228,54 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
     constexpr int I = decltype(i_tag)::value;
     if constexpr (I < PER) async_copy16_asm<I * 1024>(c.src, off[I], c.lds0);
   };
-  auto issue_tile_load = [&](const uint8_t* base, const uint32_t (&off)[PER], char* dst, int kv_row0) {
-    const TileCopy c = make_copy(base, dst, kv_row0);
+  auto issue_tile_load = [&](const char* base, const uint32_t (&off)[PER], char* dst, uint64_t row_bytes) {
+    const TileCopy c = make_copy(base, dst, row_bytes);
     copy_one(std::integral_constant<int, 0>{}, c, off);
     copy_one(std::integral_constant<int, 1>{}, c, off);
     copy_one(std::integral_constant<int, 2>{}, c, off);
     copy_one(std::integral_constant<int, 3>{}, c, off);
   };
 
-  // KV tile stream: dimension 2 fastest, dimension 0 slowest.  The load stream runs up to two
-  // tiles ahead of the softmax, so tile descriptors are produced in order and handed down.
-  struct TileInfo {
-    int row0;       // first row of the tile in the permuted KV sequence / token offset of its origin (fused)
-    int origin[3];  // coordinate of its first token
-    bool full;      // every key of the tile is attended by every query of this wave
-    bool skip;      // no key of the tile is attended by any query of this wave
-  };
-  int itc[3] = {0, 0, 0};
-  auto next_tile = [&]() {
-    TileInfo t;
-    t.full = true;
-    t.skip = false;
+  // KV tile stream: dimension 2 fastest, dimension 0 slowest, described 64 tiles at a time, one per lane, and moved
+  // on by 32 (as in fna_fwd_tile).
+  int d_first = 0;  // number of the tile that lane 0 describes
+  int d_row0 = 0;   // first row of the lane's tile in the permuted KV sequence / token offset of its origin (fused)
+  uint64_t d_full = ~uint64_t(0);  // by lane: every key of the tile is attended by every query of this wave
+  uint64_t d_skip = 0;             // ... no key of the tile is attended by any query of this wave
+  auto describe = [&](int first) __attribute__((always_inline)) {
+    d_first = first;
+    int t[3], origin[3];
+    kv_tile_of_box(na_min(first + lane, total_tiles - 1), box_n, t);
+    bool full = true, skip = false;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int org = box_org[a] + (itc[a] << p.kv_tile_lg[a]);
+      const int org = box_org[a] + (t[a] << p.kv_tile_lg[a]);
       const int end = org + p.kv_tile[a];
       if constexpr (!NOMASK) {
-        t.full = t.full && (org >= wave_full_lo[a]) && (end <= wave_full_hi[a]);  // never when end > extent
-        t.skip = t.skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
+        full = full && (org >= wave_full_lo[a]) && (end <= wave_full_hi[a]);  // never when end > extent
+        skip = skip || (end <= wave_lo[a]) || (org >= wave_hi[a]);
       }
       // a tile that would reach past the group is moved back to end at the group's last position
-      t.origin[a] = (p.edge == 1 || p.anchor) ? na_min(org, extent[a] - p.kv_tile[a]) : org;
+      origin[a] = (p.edge == 1 || p.anchor) ? na_min(org, extent[a] - p.kv_tile[a]) : org;
     }
-    t.row0 = p.fused ? t.origin[0] * tok_step[0] + t.origin[1] * tok_step[1] + t.origin[2] * tok_step[2]
-                     : (((box_org[0] >> p.kv_tile_lg[0]) + itc[0]) +
-                        p.kv_tiled[0] * (((box_org[1] >> p.kv_tile_lg[1]) + itc[1]) +
-                                         p.kv_tiled[1] * ((box_org[2] >> p.kv_tile_lg[2]) + itc[2]))) * KVT;
-    if (++itc[2] == box_n[2]) {
-      itc[2] = 0;
-      if (++itc[1] == box_n[1]) {
-        itc[1] = 0;
-        ++itc[0];
-      }
+    d_row0 = origin[0] * p.kv_row_step[0] + origin[1] * p.kv_row_step[1] + origin[2] * p.kv_row_step[2];
+    if constexpr (!NOMASK) {
+      d_full = __ballot(full);
+      d_skip = __ballot(skip);
+      *reinterpret_cast<i32x4_t*>(&sTile[tid][0]) = i32x4_t{origin[0], origin[1], origin[2], 0};
     }
-    return t;
+  };
+  // distance of a described tile's first row from the first one of the sequence / the dilation group, in bytes
+  auto row_bytes = [&](int l) __attribute__((always_inline)) {
+    return uint64_t(uint32_t(__builtin_amdgcn_readlane(d_row0, l))) * uint32_t(kv_row_stride);
   };
 
   using Stage0 = std::integral_constant<int, 0>;
   using Stage1 = std::integral_constant<int, 1>;
-  TileInfo cur = next_tile();  // tile 0
-  issue_tile_load(kbase, ld_koff, sK0, cur.row0);
-  issue_tile_load(vbase, ld_voff, sV0, cur.row0);
-
+  describe(0);
+  issue_tile_load(kbase, ld_koff, sK0, row_bytes(0));
 
   // ---- per-lane setup: this lane's query row, its window, Q fragments ------------------------
-  int wst[3], wen[3];
   int q_row;  // row of the permuted sequence / token offset in the group (fused), or -1 for padding
   i32x8_t qf[KSTEPS];
   {
@@ -298,8 +297,11 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
     for (int a = 0; a < 3; ++a) {
       const int c = q_first[a] + off[a];
       if constexpr (!NOMASK) {
-        wst[a] = na_window_start(c, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
-        wen[a] = na_window_end(c, wst[a], p.ksize[a], extent[a], p.causal[a] != 0);
+        if (g == 0) {
+          const int ws = na_window_start(c, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], p.causal[a] != 0);
+          sWin[wave * 32 + l32][2 * a] = ws;
+          sWin[wave * 32 + l32][2 * a + 1] = na_window_end(c, ws, p.ksize[a], extent[a], p.causal[a] != 0);
+        }
       }
       if (p.fused) {
         valid = valid && (c < extent[a]);
@@ -334,22 +336,35 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   // A operand of S^T: lane (key row l32 of sub-block sb, half g) holds head-dim bytes
   // 64*ks + 32*g .. +31 of its key: two 16-byte LDS reads.  Both operands use the same byte ->
   // k-index map, which is all the instruction needs.
+  // The swizzle works on chunk numbers by exclusive or: where the bits it touches do not depend on the lane the
+  // result is a constant distance, which goes into the instruction, so that few lane offsets serve all fragments
+  // (a register per fragment and stage otherwise: 36 of them, or an addition for each).
+  uint32_t k_off[KSTEPS][2];
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks)
+#pragma unroll
+    for (int i = 0; i < 2; ++i) k_off[ks][i] = uint32_t(l32 * ROWB + slot_of(l32, ks * 4 + 2 * g + i) * 16);
   auto k_frag = [&](const char* sK, int s) {  // slot s: sub-block s / KSTEPS, k-step s % KSTEPS
-    const int row = (s / KSTEPS) * 32 + l32, c0 = (s % KSTEPS) * 4 + 2 * g;
-    const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(sK + row * ROWB + slot_of(row, c0) * 16);
-    const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(sK + row * ROWB + slot_of(row, c0 + 1) * 16);
+    const char* rows = sK + (s / KSTEPS) * 32 * ROWB;  // (32 rows are a whole number of swizzle periods)
+    const i32x4_t lo = *reinterpret_cast<const i32x4_t*>(rows + k_off[s % KSTEPS][0]);
+    const i32x4_t hi = *reinterpret_cast<const i32x4_t*>(rows + k_off[s % KSTEPS][1]);
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
   // A operand of O^T += V^T P^T for the 32 columns of block db: lane (column l32, half g) needs
   // its column of LDS rows 32*g .. 32*g + 31: four transpose reads of 8 rows x 16 columns.
+  // Read m is of row 32 g + 8 m + (l16 >> 1), chunk 2 db + (l32 >> 4): of the swizzle's pattern (row / RPL) % CPR the
+  // highest bit is m & 1 and the others belong to the lane, and of the chunk number's bits the lane has the lowest.
   const int l16 = lane & 15;
+  constexpr int V_PAR = CPR / 4;  // chunk numbers of the blocks differ in this many ways below their highest bit
+  uint32_t v_off[V_PAR];
+#pragma unroll
+  for (int b = 0; b < V_PAR; ++b)
+    v_off[b] = uint32_t((32 * g + (l16 >> 1)) * ROWB + slot_of(l16 >> 1, 2 * b + (l32 >> 4)) * 16 + 8 * (l16 & 1));
   auto v_frag = [&](const char* sV, int db) {
     i32x8_t out;
 #pragma unroll
     for (int m = 0; m < 4; ++m) {
-      const int row = 32 * g + 8 * m + (l16 >> 1);
-      const int chunk = 2 * db + (l32 >> 4);
-      const i32x2_t t = lds_read_tr8(sV + row * ROWB + slot_of(row, chunk) * 16 + 8 * (l16 & 1));
+      const i32x2_t t = lds_read_tr8(sV + v_off[db % V_PAR] + 8 * m * ROWB + ((db / V_PAR) ^ (m & 1)) * (CPR / 2) * 16);
       out[2 * m] = t[0];
       out[2 * m + 1] = t[1];
     }
@@ -357,7 +372,11 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   };
 
   f32x16_t S_a[NSB], S_b[NSB];
-  uint32_t pfw[8];    // P fragment: byte 16*sb + r of the lane = its probability for logit (sb, r)
+  // P fragments of the tile before (operand of this iteration's O += P V) and of the current one, swapping roles
+  // every iteration: byte 16*sb + r of the lane = its probability for logit (sb, r)
+  i32x8_t P_a, P_b;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) P_a[i] = P_b[i] = 0;
   float msc = 0.f;    // running maximum in the exp2 domain minus the probability scale
   // Row sums are taken from the unrounded probabilities (in float): summing the rounded ones
   // with one more MFMA was measured to be no faster and costs two digits of the LSE.
@@ -365,17 +384,17 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   float held[3];
 
   // probability of logit v (sub-block v / 16, register v % 16) of the current tile
-  auto exp_elem = [&](const f32x16_t (&S_cur)[NSB], int v) {
+  auto exp_elem = [&](const f32x16_t (&S_cur)[NSB], i32x8_t& P, int v) {
     const int sb = v / 16, r = v % 16;
     float x = fast_exp2(S_cur[sb][r] * c_log2 - msc);
-    psum[r & 1] += x;
+    if (v < 2) psum[v] = x;
+    else psum[r & 1] += x;
     pin(x);
-    if (r % 4 == 1) {
-      pfw[4 * sb + r / 4] = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(held[0], x, 0, false));
-      pin(pfw[4 * sb + r / 4]);
-    } else if (r % 4 == 3) {
-      pfw[4 * sb + r / 4] = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(held[2], x, int(pfw[4 * sb + r / 4]), true));
-      pin(pfw[4 * sb + r / 4]);
+    if (r % 4 == 1 || r % 4 == 3) {
+      uint32_t w = r % 4 == 1 ? uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(held[0], x, P[4 * sb + r / 4], false))
+                              : uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(held[2], x, P[4 * sb + r / 4], true));
+      pin(w);
+      P[4 * sb + r / 4] = int(w);
     } else {
       held[r % 4] = x;
     }
@@ -383,6 +402,9 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
 
   auto apply_mask = [&](f32x16_t (&S)[NSB], const int (&origin)[3]) {
     if constexpr (NOMASK) return;
+    const i32x4_t w01 = *reinterpret_cast<const i32x4_t*>(&sWin[NOMASK ? 0 : wave * 32 + l32][0]);
+    const i32x2_t w2 = *reinterpret_cast<const i32x2_t*>(&sWin[NOMASK ? 0 : wave * 32 + l32][4]);
+    const int wst[3] = {w01[0], w01[2], w2[0]}, wen[3] = {w01[1], w01[3], w2[1]};
     uint32_t addc = 0, subc = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -408,32 +430,49 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
         }
       }
   };
+  // O trails the maxima by one tile: what it holds when an iteration ends was formed with the maxima of the tile
+  // before, so a new maximum scales the row sum at once and O an iteration later (behind the products of
+  // the probabilities that were formed with the old one).
+  float o_alpha = 1.f;     // what O is still to be multiplied by
+  bool o_pending = false;  // ... in some lane of the wave
+  auto rescale_o = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[db][r] *= o_alpha;
+    o_alpha = 1.f;
+  };
   auto update_max = [&](float mx) {
     mx = cross_half_max(mx);
-    const bool grow = (mx - m_run) * c_log2 > kFp8LazyRescaleLog2;
-    if (__any(grow)) {
-      const float m_new = fmaxf(m_run, mx);
-      const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
-      const float alpha = fast_exp2((m_run - m_use) * c_log2);
-      m_run = m_new;
-      l_run *= alpha;
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
+    const bool grow = __any((mx - m_run) * c_log2 > kFp8LazyRescaleLog2);
+    if (__builtin_expect(grow || o_pending, 0)) {
+      if (o_pending) rescale_o();
+      o_pending = grow;
+      if (grow) {
+        const float m_new = fmaxf(m_run, mx);
+        const float m_use = (m_new == -INFINITY) ? 0.f : m_new;
+        o_alpha = fast_exp2((m_run - m_use) * c_log2);
+        m_run = m_new;
+        l_run *= o_alpha;
+        msc = m_use * c_log2 - kFp8ProbLog2Scale;
+      }
     }
-    msc = ((m_run == -INFINITY) ? 0.f : m_run) * c_log2 - kFp8ProbLog2Scale;
   };
-  auto finish_logits = [&](f32x16_t (&S)[NSB], const bool t_full, const bool t_skip, const int (&t_origin)[3],
-                           bool have_max, float mx) {
-    if (t_skip) {
+  // (`l`: place of the tile among the described ones)
+  auto finish_logits = [&](f32x16_t (&S)[NSB], int l, bool have_max, float mx) {
+    const bool full = (d_full >> l) & 1, skip = (d_skip >> l) & 1;
+    if (skip) {
       mx = -INFINITY;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[sb][r] = -INFINITY;
-    } else if (!t_full || !have_max) {
-      if (!t_full) apply_mask(S, t_origin);
+    } else if (!full || !have_max) {
+      if (!full) {
+        const i32x4_t tile = *reinterpret_cast<const i32x4_t*>(&sTile[wave * 64 + l][0]);
+        const int origin[3] = {tile[0], tile[1], tile[2]};
+        apply_mask(S, origin);
+      }
       mx = -INFINITY;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
@@ -448,17 +487,34 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
   using FmtIn = std::integral_constant<int, FMT_IN>;
   using FmtP = std::integral_constant<int, 0>;
 
-  // ---- software pipeline (as in fna_fwd_kernel): iteration j = slots of S(j+1) = K(j+1) Q^T,
-  // carrying the exponentials of S(j) and the tile copies, then slots of O += P(j) V(j),
-  // carrying the row maximum of S(j+1).  The matrix instruction is twice as fast here and the
-  // vector work per key the same, so the vector units set the pace.
+  // ---- software pipeline: iteration j forms S(j+1) = K(j+1) Q^T and O += P(j-1) V(j-1) on the matrix pipe,
+  // and the probabilities of S(j) and the maxima of S(j+1) beside them.  The P fragment of a 64-key
+  // matrix instruction is complete only with a tile's last exponential, so that the tile's own O += P V
+  // cannot begin before; with O a tile behind, the exponentials spread over all of an iteration's matrix
+  // instructions instead of the first half (where the vector unit held the matrix pipe up, which
+  // then held up nothing in the second).  K tiles are copied two ahead, V tiles in the iteration of their
+  // own exponentials: both keep two stages.
+  // us with O += P V of tile j in iteration j / as it is: 16 x 64 x 64, 8 x 16 x 16, stride 4 x 8 x 8, dilation 1 x 2 x 2, H 16,
+  // D 128 735 / 693; the same without stride and dilation 1890 / 1725; 30 x 48 x 80, 18 x 24 x 24, H 24 16600 / 15420,
+  // stride 1 x 8 x 8 and causal 6570 / 6490 (power-limited); 8 x 32 x 40, 4 x 9 x 11, H 8 82 / 77.
   constexpr int N_QK = NSB * KSTEPS;
   constexpr int N_PV = DB;
   constexpr int N_ELEMS = NSB * 16;
-  TileInfo nxt = next_tile();
+  constexpr int N_SLOTS = N_QK + N_PV;
+  // Half of O += P V, the products of the coming tile, the other half: the coming logits need registers only
+  // when a part of the current ones is done with, and there is matrix work left beside their maxima.
+  constexpr int PV_FIRST = N_PV / 2;
+  auto is_qk = [](int x) constexpr { return x >= PV_FIRST && x < PV_FIRST + N_QK; };
+  auto elems_done = [](int x) constexpr {  // exponentials up to and with slot x: fewer in the last ones, which take the maxima
+    const int n = (N_ELEMS * (x + 1) * 16 + N_SLOTS * 13 - 1) / (N_SLOTS * 13);
+    return n > N_ELEMS ? N_ELEMS : n;
+  };
+  uint64_t cur = row_bytes(0), nxt = row_bytes(1);  // of the tiles j and j + 1
+  // the V stage that iteration 0 reads (with probabilities of zero)
+  for (int i = tid; i < TILE_BYTES / 16; i += NT) reinterpret_cast<i32x4_t*>(sV1)[i] = i32x4_t{0, 0, 0, 0};
   wait_vmcnt<0>();
   workgroup_sync();
-  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt.row0);
+  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt);
   msc = -kFp8ProbLog2Scale;
   {
 #pragma unroll
@@ -468,82 +524,91 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
 #pragma unroll
     for (int s = 0; s < N_QK; ++s)
       S_a[s / KSTEPS] = mfma8(k_frag(sK0, s), qf[s % KSTEPS], S_a[s / KSTEPS], FmtIn{}, FmtIn{});
-    finish_logits(S_a, cur.full, cur.skip, cur.origin, false, 0.f);
+    finish_logits(S_a, 0, false, 0.f);
+    o_pending = false;  // (O holds nothing yet)
+    o_alpha = 1.f;
   }
 
   auto iteration = [&](auto stage_tag, int j) __attribute__((always_inline)) {
     constexpr int st = decltype(stage_tag)::value;
     f32x16_t (&S_cur)[NSB] = st ? S_b : S_a;
     f32x16_t (&S_nxt)[NSB] = st ? S_a : S_b;
-    char* sK_cur = st ? sK1 : sK0;
-    char* sK_nxt = st ? sK0 : sK1;
-    char* sV_cur = st ? sV1 : sV0;
-    char* sV_nxt = st ? sV0 : sV1;
+    i32x8_t& P_cur = st ? P_b : P_a;
+    const i32x8_t& P_prev = st ? P_a : P_b;
+    char* sK_cur = st ? sK1 : sK0;   // held K(j): free, receives K(j+2)
+    char* sK_nxt = st ? sK0 : sK1;   // holds K(j+1)
+    char* sV_cur = st ? sV1 : sV0;   // held V(j-2): free, receives V(j)
+    char* sV_prev = st ? sV0 : sV1;  // holds V(j-1)
 
+    if constexpr (st == 0) {
+      if (j + 2 - d_first == 64) describe(d_first + 32);
+    }
     wait_vmcnt<0>();
     workgroup_sync();
-    const TileInfo t2 = next_tile();
-    const TileCopy ck = make_copy(kbase, sK_cur, (j + 2 < total_tiles) ? t2.row0 : cur.row0);
-    const TileCopy cv = make_copy(vbase, sV_nxt, (j + 1 < total_tiles) ? nxt.row0 : cur.row0);
+    const uint64_t t2 = row_bytes(j + 2 - d_first);
+    // (past the end of the box the last tile is read again into a free stage, never used)
+    const TileCopy ck = make_copy(kbase, sK_cur, t2);
+    const TileCopy cv = make_copy(vbase, sV_cur, cur);
 
-    i32x8_t kf[N_QK];
-    kf[0] = k_frag(sK_nxt, 0);
-    psum[0] = psum[1] = 0.f;
-    auto g1_slot = [&](auto s_tag) __attribute__((always_inline)) {
-      constexpr int s = decltype(s_tag)::value;
-      if constexpr (s + 1 < N_QK) kf[s + 1] = k_frag(sK_nxt, s + 1);
-      if constexpr (s % KSTEPS == 0) {
-        f32x16_t zero;
+    i32x8_t fr[N_SLOTS];
+    auto frag = [&](auto x_tag) __attribute__((always_inline)) {
+      constexpr int x = decltype(x_tag)::value;
+      if constexpr (is_qk(x)) return k_frag(sK_nxt, x - PV_FIRST);
+      else return v_frag(sV_prev, x < PV_FIRST ? x : x - N_QK);
+    };
+    fr[0] = frag(std::integral_constant<int, 0>{});
+    float mx0 = -INFINITY, mx1 = -INFINITY;
+    auto slot = [&](auto x_tag) __attribute__((always_inline)) {
+      constexpr int x = decltype(x_tag)::value;
+      if constexpr (x + 1 < N_SLOTS) fr[x + 1] = frag(std::integral_constant<int, x + 1>{});
+      if constexpr (is_qk(x)) {
+        constexpr int s = x - PV_FIRST;
+        if constexpr (s % KSTEPS == 0) {
+          f32x16_t zero;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) zero[r] = 0.f;
-        S_nxt[s / KSTEPS] = mfma8(kf[s], qf[s % KSTEPS], zero, FmtIn{}, FmtIn{});
+          for (int r = 0; r < 16; ++r) zero[r] = 0.f;
+          S_nxt[s / KSTEPS] = mfma8(fr[x], qf[s % KSTEPS], zero, FmtIn{}, FmtIn{});
+        } else {
+          S_nxt[s / KSTEPS] = mfma8(fr[x], qf[s % KSTEPS], S_nxt[s / KSTEPS], FmtIn{}, FmtIn{});
+        }
       } else {
-        S_nxt[s / KSTEPS] = mfma8(kf[s], qf[s % KSTEPS], S_nxt[s / KSTEPS], FmtIn{}, FmtIn{});
+        constexpr int t = x < PV_FIRST ? x : x - N_QK;
+        acc[t] = mfma8(fr[x], P_prev, acc[t], FmtIn{}, FmtP{});
       }
-      constexpr int e_lo = (s * N_ELEMS) / N_QK, e_hi = ((s + 1) * N_ELEMS) / N_QK;
-#pragma unroll
-      for (int e = e_lo; e < e_hi; ++e) exp_elem(S_cur, e);
-      pin(psum[0]);
-      pin(psum[1]);
-      // 2 * PER copies over the slots, K first
-      constexpr int c_lo = (s * 2 * PER) / N_QK, c_hi = ((s + 1) * 2 * PER) / N_QK;
+      // 2 * PER copies over the first half of the slots, K first
+      constexpr int c_lo = (x * 4 * PER) / N_SLOTS, c_hi = ((x + 1) * 4 * PER) / N_SLOTS;
       for_range<c_lo, c_hi - c_lo>([&](auto c_tag) {
         constexpr int c = decltype(c_tag)::value;
         if constexpr (c < PER) copy_one(std::integral_constant<int, c>{}, ck, ld_koff);
-        else copy_one(std::integral_constant<int, c - PER>{}, cv, ld_voff);
+        else if constexpr (c < 2 * PER) copy_one(std::integral_constant<int, c - PER>{}, cv, ld_voff);
       });
-      __builtin_amdgcn_sched_barrier(0);
-    };
-    __builtin_amdgcn_s_setprio(1);  // as in the 16-bit kernel: the QK slots run at raised wave priority
-    for_range<0, N_QK>(g1_slot);
-    __builtin_amdgcn_s_setprio(0);
-
-    i32x8_t pf;
+      if constexpr (x >= PV_FIRST + N_QK) {
+        constexpr int NV = NSB * 16, t = x - PV_FIRST - N_QK, n = N_PV - PV_FIRST;
+        constexpr int e_lo = (t * NV) / n, e_hi = ((t + 1) * NV) / n;
+        static_assert((e_hi - e_lo) % 4 == 0, "row maxima are taken two logits per instruction, on two chains");
 #pragma unroll
-    for (int i = 0; i < 8; ++i) pf[i] = int(pfw[i]);
-    i32x8_t vf[N_PV];
-    vf[0] = v_frag(sV_cur, 0);
-    float mx0 = -INFINITY, mx1 = -INFINITY;
-    auto pv_slot = [&](auto t_tag) __attribute__((always_inline)) {
-      constexpr int t = decltype(t_tag)::value;
-      if constexpr (t + 1 < N_PV) vf[t + 1] = v_frag(sV_cur, t + 1);
-      acc[t] = mfma8(vf[t], pf, acc[t], FmtIn{}, FmtP{});
-      constexpr int NV = NSB * 16;
-      constexpr int e_lo = (t * NV) / N_PV, e_hi = ((t + 1) * NV) / N_PV;
-      static_assert((e_hi - e_lo) % 4 == 0, "row maxima are taken two logits per instruction, on two chains");
-#pragma unroll
-      for (int e = e_lo; e < e_hi; e += 4) {
-        mx0 = fmaxf(fmaxf(mx0, S_nxt[e / 16][e % 16]), S_nxt[(e + 1) / 16][(e + 1) % 16]);
-        mx1 = fmaxf(fmaxf(mx1, S_nxt[(e + 2) / 16][(e + 2) % 16]), S_nxt[(e + 3) / 16][(e + 3) % 16]);
+        for (int e = e_lo; e < e_hi; e += 4) {
+          mx0 = fmaxf(fmaxf(mx0, S_nxt[e / 16][e % 16]), S_nxt[(e + 1) / 16][(e + 1) % 16]);
+          mx1 = fmaxf(fmaxf(mx1, S_nxt[(e + 2) / 16][(e + 2) % 16]), S_nxt[(e + 3) / 16][(e + 3) % 16]);
+        }
+        pin(mx0);
+        pin(mx1);
       }
-      pin(mx0);
-      pin(mx1);
+#pragma unroll
+      for (int e = elems_done(x - 1); e < elems_done(x); ++e) exp_elem(S_cur, P_cur, e);
+      pin(psum[0]);
+      pin(psum[1]);
       __builtin_amdgcn_sched_barrier(0);
     };
-    for_range<0, N_PV>(pv_slot);
+    // (raised priority as in the 16-bit kernel; 30 x 48 x 80, stride 1 x 8 x 8 as above: 7090 us without, 6790 over half the
+    // slots, 6490 over three quarters)
+    __builtin_amdgcn_s_setprio(1);
+    for_range<0, N_SLOTS * 3 / 4>(slot);
+    __builtin_amdgcn_s_setprio(0);
+    for_range<N_SLOTS * 3 / 4, N_SLOTS - N_SLOTS * 3 / 4>(slot);
     l_run += psum[0] + psum[1];
 
-    if (j + 1 < total_tiles) finish_logits(S_nxt, nxt.full, nxt.skip, nxt.origin, true, fmaxf(mx0, mx1));
+    if (j + 1 < total_tiles) finish_logits(S_nxt, j + 1 - d_first, true, fmaxf(mx0, mx1));
     cur = nxt;
     nxt = t2;
   };
@@ -551,7 +616,16 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
     iteration(Stage0{}, j);
     if (j + 1 < total_tiles) iteration(Stage1{}, j + 1);
   }
-  wait_vmcnt<0>();  // copies into the unused stage must land before the LDS is released
+  // O += P V of the last tile
+  wait_vmcnt<0>();
+  workgroup_sync();
+  if (o_pending) rescale_o();
+  {
+    const char* sV_last = (total_tiles & 1) ? sV0 : sV1;
+    const i32x8_t P = (total_tiles & 1) ? P_a : P_b;
+#pragma unroll
+    for (int t = 0; t < N_PV; ++t) acc[t] = mfma8(v_frag(sV_last, t), P, acc[t], FmtIn{}, FmtP{});
+  }
   before_stores();  // (see fna_fwd_tile)
 
   // ---- epilogue: O = acc / rowsum (bf16), LSE = ln(rowsum) + scale * rowmax - ln(2^6) ----------
@@ -581,14 +655,14 @@ static __device__ __forceinline__ void fna_fwd_fp8_tile(const FnaParams& p, cons
 }
 
 template <bool E5M2, int D, int NWAVES, bool NOMASK = false>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(fp8_waves_per_simd(D), fp8_waves_per_simd(D))))
 fna_fwd_fp8_kernel(const FnaParams p) {
   fna_fwd_fp8_tile<E5M2, D, NWAVES, NOMASK>(p, blockIdx.x, []() {});
 }
 
 // Work-queue form (see fna_fwd_queue_kernel).
 template <bool E5M2, int D, int NWAVES, bool NOMASK = false>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(fp8_waves_per_simd(D), fp8_waves_per_simd(D))))
 fna_fwd_fp8_queue_kernel(const FnaParams p, uint32_t* __restrict__ queues, const int per_xcd) {
   FnaKernargPtr args = fna_kernarg_params();
   fna_queue_loop(queues, per_xcd, [&](int pid, auto& fetch) __attribute__((always_inline)) {

@@ -60,21 +60,21 @@ struct TileConfig {
 const TileConfig kTileConfigs[] = {{128, 64}, {256, 64}, {64, 64}};
 constexpr int kNumTileConfigs = sizeof(kTileConfigs) / sizeof(kTileConfigs[0]);
 
-// Workgroups a work-queue launch starts: two per compute unit (what the kernel's LDS and register
+// Workgroups a work-queue launch starts: `per_cu` per compute unit (what the kernel's LDS and register
 // use keep resident), a multiple of the XCD count; the device's figure is read once.
-int resident_workgroups() {
+int resident_workgroups(int per_cu = 2) {
   static std::atomic<int> cached[64] = {};  // (threads that race here compute the same value)
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 512;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256 * per_cu;
   int n = cached[dev].load(std::memory_order_relaxed);
   if (n == 0) {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    n = (2 * cus / kNumXcd) * kNumXcd;
-    if (n < kNumXcd) n = kNumXcd;
+    n = cus;
     cached[dev].store(n, std::memory_order_relaxed);
   }
-  return n;
+  n = (per_cu * n / kNumXcd) * kNumXcd;
+  return n < kNumXcd ? kNumXcd : n;
 }
 
 // Head dims whose rows the 128 x 64 forward instances take as they are, besides 32, 64 and 128
@@ -161,7 +161,7 @@ int launch_fna_fp8_instance(const FnaParams& p, hipStream_t stream, WorkQueue qu
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
   if (wgs > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
   if (queues.counters != nullptr) {
-    const long long resident = resident_workgroups();
+    const long long resident = resident_workgroups(fp8_waves_per_simd(D));
     if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
     hipLaunchKernelGGL((fna_fwd_fp8_queue_kernel<E5M2, D, 4, NOMASK>), dim3((unsigned)(wgs < resident ? wgs : resident)),
                        dim3(256), 0, stream, p, queues.counters, int(wgs / kNumXcd));
