@@ -738,11 +738,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     int lim[3];       // original layout: positions of the tile that lie inside the dilation group, per dimension
     bool inside;      // the whole tile lies inside the sequence / the dilation group
   };
+  const uint32_t lds_wave = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sK0) + uint32_t(wave * PER * 1024))));
   // `l`: place of the tile among the described ones (RAGGED instances, which look at its origin)
   auto make_copy = [&](const char* base, char* dst, const TileRows& t, int l) {
     TileCopy c;
     c.src = base + t.bytes;
-    c.lds0 = lds_address(dst) + uint32_t(wave * PER * 1024);
+    c.lds0 = lds_wave + (lds_address(dst) - lds_address(sK0));
     c.inside = true;
     if constexpr (RAGGED) {
       const int kv_row0 = t.row0;
@@ -919,6 +920,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const int v_row = 4 * g + v_e;
   const int v_chunk = (l32 >> 4) * 2 + (v_j4 >> 1);  // 16-byte chunk inside the 64-byte column block
   const int v_sub = (v_j4 & 1) * 8;
+  uint32_t v_off[DB];  // (8 rows are a whole number of the V swizzle's periods)
+  static_assert(8 % (L::RPL * CPR / 2) == 0, "the transpose reads of a fragment lie 8 rows apart");
+#pragma unroll
+  for (int db = 0; db < DB; ++db) v_off[db] = uint32_t(v_row * ROWB + v_sub + L::v_slot(v_row, db * 4 + v_chunk) * 16);
 
   // ---- building blocks ---------------------------------------------------------------------------
   // The lane owns query row l32 of each of its wave's MQ row blocks and, per 32-key sub-block,
@@ -939,10 +944,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   };
   // PV slot t: sub-block t / (2*DB), 16-key half (t / DB) % 2, 32-column block t % DB
   auto v_frag = [&](const char* sV, int t) {
-    const int r0 = (t / (2 * DB)) * 32 + ((t / DB) % 2) * 16 + v_row;
-    const int c = (t % DB) * 4 + v_chunk;
-    const s16x4_t lo = lds_read_tr16(sV + r0 * ROWB + v_sub + L::v_slot(r0, c) * 16);
-    const s16x4_t hi = lds_read_tr16(sV + (r0 + 8) * ROWB + v_sub + L::v_slot(r0 + 8, c) * 16);
+    const char* rows = sV + ((t / (2 * DB)) * 32 + ((t / DB) % 2) * 16) * ROWB;
+    const s16x4_t lo = lds_read_tr16(rows + v_off[t % DB]);
+    const s16x4_t hi = lds_read_tr16(rows + v_off[t % DB] + 8 * ROWB);
     return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
@@ -1345,10 +1349,17 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
 }
 
-// Head dim 32 needs 153 registers: three waves per SIMD, which an upper bound of two would keep it from.
+// Waves per SIMD the compiler makes room for, at least and at most.  Head dim 32 takes 153 registers: three waves, which an
+// upper bound of two would keep it from.  Head dim 64 without masks is held to the 168 that three waves leave (five
+// values of the set-up go to scratch, none in the loop): 96 x 96 tokens, window 32 x 32, stride 16, H 8: 35.1 us with
+// two, 31.1 with three; dense 2 x 2048, H 24: 67.7 and 64.3; 2 x 4096, H 16: 158.6 and 155.9.  With masks it would
+// reload in every iteration (2 x 128 x 128, 25 x 25: 124 and 175).
+constexpr int fwd_min_waves(int d, bool nomask) { return d == 64 && nomask ? 3 : 2; }
+constexpr int fwd_max_waves(int d, bool nomask) { return d == 32 || (d == 64 && nomask) ? 3 : 2; }
+
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
 __global__ void __launch_bounds__(NWAVES * 64)
-    __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? (D == 32 ? 3 : 2) : 1)))
+    __attribute__((amdgpu_waves_per_eu(MQ == 1 ? fwd_min_waves(D, NOMASK) : 1, MQ == 1 ? fwd_max_waves(D, NOMASK) : 1)))
 fna_fwd_kernel(const FnaParams p) {
   fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC>(p, int(blockIdx.x), []() {});
 }
