@@ -138,29 +138,6 @@ inline void set_bwd_divisions(FnaBwdParams& p) {
   p.d_heads_kv = na_make_div(p.heads_kv);
 }
 
-// Stores a lane's row of a transposed result (32 DB columns; register 4 j + i of block db is column
-// 32 db + 8 j + 4 g + i): the lanes of a row's two wave halves trade four columns of every sixteen, so
-// that each stores sixteen bytes at a time.
-template <typename T, int DB>
-static __device__ __forceinline__ void store_row_blocks(T* orow, const f32x16_t (&acc)[DB], float mul, int g, bool valid) {
-  using vec2 = typename Mma<T>::vec2;
-#pragma unroll
-  for (int db = 0; db < DB; ++db)
-#pragma unroll
-    for (int j = 0; j < 4; j += 2) {
-      uint32_t w[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * (j + i / 2) + 2 * (i % 2);
-        const vec2 v = {static_cast<T>(acc[db][r] * mul), static_cast<T>(acc[db][r + 1] * mul)};
-        w[i] = __builtin_bit_cast(uint32_t, v);
-      }
-      asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %2\n\tv_permlane32_swap_b32 %1, %3\n\ts_nop 1"
-                   : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]));
-      if (valid) *reinterpret_cast<u32x4_t*>(orow + db * 32 + 8 * (j + g)) = u32x4_t{w[0], w[1], w[2], w[3]};
-    }
-}
-
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 
 // Tiles of a sequence-packed batch.  The rows 0 .. total - 1 of one side are the sequences cu[i] ..
@@ -565,7 +542,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
 
   auto store_rows = [&](void* dst, const f32x16_t (&acc)[DB], float mul) {
     T* orow = reinterpret_cast<T*>(dst) + a_row * a_stride + int64_t(head_a) * D;
-    store_row_blocks<T, DB>(orow, acc, mul, g, a_valid);
+    store_row_blocks<T, DB>(orow, acc, mul, g, a_valid, D);
   };
   auto store_results = [&](const f32x16_t (&a1)[DB], const f32x16_t (&a2)[DB], float scale1) {
     if constexpr (ROLE == kBwdDQ) store_rows(p.dq, a1, scale1);

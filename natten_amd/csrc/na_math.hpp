@@ -70,6 +70,15 @@ NA_HD int na_window_start(int i, int k, int s, NaDiv s_div, int L, bool causal) 
   return na_max(leader - wl, 0) + ((leader + wr >= L) ? (L - wr - leader - 1) : 0);
 }
 
+// The same without a branch on `causal`, for vector code.
+NA_HD int na_window_start_flat(int i, int k, int s, NaDiv s_div, int L, bool causal) {
+  const int wl = int(uint32_t(k) >> 1);
+  const int wr = wl + int(uint32_t(k) & 1u) - 1;
+  const int leader = na_min(na_div(i, s_div) * s + (causal ? s - 1 : int(uint32_t(s) >> 1)), L - 1);
+  const int start = na_max(leader - (causal ? wl + wr : wl), 0);
+  return start + (causal ? 0 : na_min(L - wr - 1 - leader, 0));
+}
+
 // Keys of a 64-key KV tile are numbered with dimension 0 fastest and all tile extents are powers of
 // two, so a key's coordinate along one dimension is a bit field of its number: (i >> lg_stride) &
 // (2^lg_extent - 1).  Bit i of the result is set when that coordinate of key i is >= x
