@@ -341,6 +341,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // [sub-block][half of the 16 values][lane] x 16 bytes
   __shared__ __attribute__((aligned(16))) char sX[PAIR ? 2 * 4 * NSB * 2 * 64 * 16 : 16];
 
+  touch_launch_params<sizeof(FnaBwdParams)>();
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -449,7 +450,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
     }
   }
 
-  int extent[3], q_extent[3], a_first[3], b_sub[3], b_sub_lg[3], box_tile0[3], box_n[3], full_t0[3], full_t1[3];
+  int extent[3], q_extent[3], a_first[3], b_sub[3], b_sub_lg[3];
   int tok_step[3];    // original layout: tokens per unit step of a coordinate inside a dilation group
   int group_tok = 0;  // original layout: token of the dilation group's first element
   {
@@ -467,50 +468,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       a_first[a] = tc[a] << a_tile_lg[a];
       b_sub_lg[a] = b_tile_lg[a] - (a == split_dim ? 1 : 0);
       b_sub[a] = 1 << b_sub_lg[a];
-      const bool c = p.causal[a] != 0;
-      int lo, hi;  // first and last streamed coordinate this tile meets
-      if constexpr (!KV_STATIONARY) {
-        const int qf = a_first[a], ql = na_min(qf + a_tile[a], q_extent[a]) - 1;
-        if (qf >= q_extent[a]) empty = true;
-        lo = na_window_start(qf, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
-        const int st_l = na_window_start(na_max(ql, 0), ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
-        hi = na_window_end(na_max(ql, 0), st_l, ksz[a], extent[a], c) - 1;
-      } else {
-        const int j0 = a_first[a], j1 = na_min(j0 + a_tile[a], extent[a]) - 1;
-        if (j0 >= extent[a]) empty = true;
-        lo = na_first_query_attending(j0, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
-        hi = na_last_query_attending(na_max(j1, 0), ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
-        if (lo > hi) empty = true;
-      }
-      lo = na_max(lo, 0);
-      hi = na_max(hi, lo);
-      box_tile0[a] = lo >> b_sub_lg[a];
-      box_n[a] = (hi >> b_sub_lg[a]) + 1 - box_tile0[a];
-      // Streamed tiles every row of which pairs with every row of the stationary tile (no mask
-      // needed) form an interval of tile coordinates per dimension, again by monotonicity:
-      // streamed coordinates flo .. fhi pair with all stationary ones.
-      int flo, fhi;
-      if constexpr (!KV_STATIONARY) {
-        const int qf = a_first[a], ql = qf + a_tile[a] - 1;  // rows past the extent use the last window
-        const int st_l = na_window_start(ql, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
-        const int st_f = na_window_start(qf, ksz[a], p.stride[a], p.d_stride[a], extent[a], c);
-        flo = st_l;
-        fhi = na_window_end(qf, st_f, ksz[a], extent[a], c) - 1;
-      } else {
-        // (rows past the end that are not stored may take part: only zero-padded sequences need their mask)
-        const int j0 = a_first[a];
-        const int j1 = (RAGGED || p.fused) ? na_min(j0 + a_tile[a], extent[a]) - 1 : j0 + a_tile[a] - 1;
-        if (j1 >= extent[a]) {
-          flo = 1;  // the tile holds padding keys: never whole
-          fhi = 0;
-        } else {
-          flo = na_first_query_attending(j1, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
-          fhi = na_last_query_attending(j0, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], c);
-        }
-      }
-      full_t0[a] = na_max((na_max(flo, 0) + b_sub[a] - 1) >> b_sub_lg[a], box_tile0[a]);
-      full_t1[a] = na_min((fhi + 1) >> b_sub_lg[a], box_tile0[a] + box_n[a]);  // one past the last whole tile
-      if (fhi < 0 || full_t1[a] < full_t0[a]) full_t1[a] = full_t0[a];
+      if (a_first[a] >= (KV_STATIONARY ? extent[a] : q_extent[a])) empty = true;
     }
   }
 
@@ -540,6 +498,70 @@ fna_bwd_kernel(const FnaBwdParams p) {
   const int64_t b_stride = int64_t(heads_b) * D;
   const float kLog2e = 1.4426950408889634f;
 
+  // Stationary operand fragments: row r_in, elements 16*ks + 8*g .. +7 (paired role: K for the P waves, V
+  // for the dS waves).  On their way from here on, and scaled (dQ role) once everything else is set up.
+  const T* x1 = reinterpret_cast<const T*>(KV_STATIONARY ? ((PAIR && part) ? p.v : p.k) : p.q) + a_row * a_stride +
+                int64_t(head_a) * D + g * 8;
+  const T* x2 = reinterpret_cast<const T*>(KV_STATIONARY ? p.v : p.d_out) + a_row * a_stride + int64_t(head_a) * D + g * 8;
+  vec8 x1f[KSTEPS], x2f[HAS_DS ? KSTEPS : 1];
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    x1f[ks] = *reinterpret_cast<const vec8*>(x1 + ks * 16);
+    if constexpr (HAS_DS) x2f[ks] = *reinterpret_cast<const vec8*>(x2 + ks * 16);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  // ---- which streamed rows meet -----------------------------------------------------------------------
+  // Along every dimension the streamed rows that pair with a stationary row are an interval (the window of a
+  // query; the queries whose windows hold a key), monotone in the row, so that the tile's first and last
+  // rows give the box of streamed tiles it meets, and the inner box of those every row of which pairs with
+  // every row of the tile (no mask needed).  One evaluation per dimension serves all of it: the lower half of
+  // the wave takes its lanes' rows (the lanes of the upper half, which hold the same ones, get the results
+  // from there), lane 32 the tile's first row, lane 33 its last one inside the extent, lane 34 its last one.
+  // A workgroup's first step began after 10000 cycles: the loads of the launch parameters one behind the other, 18
+  // evaluations of which 12 on the scalar unit, and the tables before the first copies.  dK / dV and dQ launches,
+  // us before / after: 4 x 56 x 56, 7 x 7, H 8, D 32 41.4 / 39.0 and 32.4 / 31.3; 56 x 56, H 32, D 64 56.2 / 53.7 and 43.2 / 42.7;
+  // 96 x 96, 24 x 24, stride 8, H 8, D 64 51.0 / 48.8 and 37.4 / 36.6; dense 2 x 1000, H 8, D 128 33.6 / 32.4 and 30.5 / 29.0.  Large
+  // launches of head dim 128 run at the card's power limit and take as long as before.
+  int win_lo[3], win_hi[3];  // the rows win_lo .. win_hi - 1 pair with the lane's
+  int box_tile0[3], box_n[3], full_t0[3], full_t1[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int e = KV_STATIONARY ? extent[a] : q_extent[a];
+    const int last = a_first[a] + a_tile[a] - 1, last_in = na_max(na_min(last, e - 1), 0);
+    const int c = g == 0 ? a_crd[a] : l32 == 0 ? a_first[a] : l32 == 1 ? last_in : last;
+    const bool cs = p.causal[a] != 0;
+    int from, upto;
+    if constexpr (!KV_STATIONARY) {
+      from = na_window_start_flat(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
+      upto = na_window_end(c, from, ksz[a], extent[a], cs);
+    } else {
+      from = na_first_query_attending_flat(c, ksz[a], p.stride[a], p.d_stride[a], q_extent[a], cs);
+      upto = na_last_query_attending_flat(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs) + 1;
+      if (c >= extent[a]) upto = from;  // a padding key of a permuted sequence: nothing attends it
+    }
+    win_lo[a] = lower_half(from);
+    win_hi[a] = lower_half(upto);
+    const int first_from = __builtin_amdgcn_readlane(from, 32), first_upto = __builtin_amdgcn_readlane(upto, 32);
+    int hi = __builtin_amdgcn_readlane(upto, 33) - 1;
+    if (KV_STATIONARY && first_from > hi) empty = true;
+    const int lo = na_max(first_from, 0);
+    hi = na_max(hi, lo);
+    box_tile0[a] = lo >> b_sub_lg[a];
+    box_n[a] = (hi >> b_sub_lg[a]) + 1 - box_tile0[a];
+    // Whole tiles: streamed coordinates flo .. fhi pair with all stationary ones.  dQ: rows past the extent use the
+    // last window.  Key-stationary: rows past the end that are not stored may take part, only zero-padded
+    // sequences need their mask.
+    int flo = __builtin_amdgcn_readlane(from, (KV_STATIONARY && (RAGGED || p.fused)) ? 33 : 34), fhi = first_upto - 1;
+    if (KV_STATIONARY && !(RAGGED || p.fused) && last >= e) {
+      flo = 1;  // the tile holds padding keys: never whole
+      fhi = 0;
+    }
+    full_t0[a] = na_max((na_max(flo, 0) + b_sub[a] - 1) >> b_sub_lg[a], box_tile0[a]);
+    full_t1[a] = na_min((fhi + 1) >> b_sub_lg[a], box_tile0[a] + box_n[a]);  // one past the last whole tile
+    if (fhi < 0 || full_t1[a] < full_t0[a]) full_t1[a] = full_t0[a];
+  }
+
   auto store_rows = [&](void* dst, const f32x16_t (&acc)[DB], float mul) {
     T* orow = reinterpret_cast<T*>(dst) + a_row * a_stride + int64_t(head_a) * D;
     store_row_blocks<T, DB>(orow, acc, mul, g, a_valid, D);
@@ -565,66 +587,6 @@ fna_bwd_kernel(const FnaBwdParams p) {
     // padding rows, or rows nothing attends: their gradients are zero
     store_results(acc1, acc2, 0.f);
     return;
-  }
-
-  // stationary operand fragments: row r_in, elements 16*ks + 8*g .. +7
-  // (paired role: K for the P waves, V for the dS waves)
-  const T* x1 = reinterpret_cast<const T*>(KV_STATIONARY ? ((PAIR && part) ? p.v : p.k) : p.q) + a_row * a_stride +
-                int64_t(head_a) * D + g * 8;
-  const T* x2 = reinterpret_cast<const T*>(KV_STATIONARY ? p.v : p.d_out) + a_row * a_stride + int64_t(head_a) * D + g * 8;
-  vec8 x1f[KSTEPS], x2f[HAS_DS ? KSTEPS : 1];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    x1f[ks] = *reinterpret_cast<const vec8*>(x1 + ks * 16);
-    if constexpr (!KV_STATIONARY) x1f[ks] = scale_query_fragment<T>(x1f[ks], p.scale * kLog2e);
-    if constexpr (HAS_DS) x2f[ks] = *reinterpret_cast<const vec8*>(x2 + ks * 16);
-  }
-
-  // Mask state of the lane: along every dimension the streamed rows that pair with its stationary row are
-  // an interval (the window of a query; the queries whose windows hold a key), so that the pairs of
-  // a tile are the AND of two rows of sRows per dimension.
-  int win_lo[3], win_hi[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    const int c = a_crd[a];
-    const bool cs = p.causal[a] != 0;
-    if constexpr (!KV_STATIONARY) {
-      win_lo[a] = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
-      win_hi[a] = na_window_end(c, win_lo[a], ksz[a], extent[a], cs);
-    } else {
-      win_lo[a] = na_first_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs);
-      win_hi[a] = na_last_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs) + 1;
-      if (c >= extent[a]) win_hi[a] = win_lo[a];  // a padding key of a permuted sequence: nothing attends it
-    }
-  }
-  if (wave < 3) {
-    // one row per lane and, by wave, one dimension (the row past the extent holds nothing)
-    const int lg_stride = wave == 0 ? 0 : wave == 1 ? b_sub_lg[0] : b_sub_lg[0] + b_sub_lg[1];
-    const int lg = wave == 0 ? b_sub_lg[0] : wave == 1 ? b_sub_lg[1] : b_sub_lg[2];
-    const uint64_t rows = na_keys_at_or_after(na_min(lane, 1 << lg), lg_stride, lg);
-    sRows[wave][0][lane] = na_lane_half_bits(rows, 0);
-    sRows[wave][1][lane] = na_lane_half_bits(rows, 1);
-    if (lane == 0) sRows[wave][0][BT] = sRows[wave][1][BT] = 0;
-  }
-  // Accumulator inputs of the first matrix instruction of a logit / dP block: -log2e LSE and -delta of
-  // the block's queries, so that P = exp2(S) and dS = P dP are what the matrix pipe returns.  In the
-  // key-stationary roles they differ by row and come from the tile's table in LDS; in the dQ role they
-  // are the lane's own, sixteen copies of them where the registers allow (head dims below 128).
-  constexpr bool INIT_REGS = !KV_STATIONARY && D < 128;
-  float lse_l = 0.f, delta_l = 0.f;
-  if constexpr (!KV_STATIONARY) {
-    const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
-                                     : stat_row_q + head_a * stat_head_stride + a_seq_row;
-    lse_l = p.lse[stat_idx] * p.lse_mul;
-    delta_l = p.delta[stat_idx] * p.delta_mul;
-  }
-  f32x16_t lse_init, delta_init;
-  if constexpr (INIT_REGS) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      lse_init[r] = lse_l;
-      delta_init[r] = delta_l;
-    }
   }
 
   // ---- streamed tiles ---------------------------------------------------------------------------
@@ -798,6 +760,50 @@ fna_bwd_kernel(const FnaBwdParams p) {
     const s16x4_t hi = lds_read_tr16(s + (r0 + 8) * ROWB + v_sub + L::u_slot(r0 + 8, c) * 16);
     return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
+
+  // The first tiles' copies are on their way while the rest is set up: two tiles ahead in the paired role and with
+  // three stages, one with two.
+  constexpr int CPT = 2 * PER;  // tile copies per thread and tile
+  constexpr int AHEAD = NS == 3 ? 2 : 1;
+  const Tile tile0 = next_tile();
+  issue_copies(tile0, 0, 0);
+  Tile tile1 = tile0;
+  if (AHEAD > 1 && 1 < n_iter) {
+    tile1 = next_tile();
+    issue_copies(tile1, 1, 1);
+  }
+  if (wave < 3) {
+    // one row per lane and, by wave, one dimension (the row past the extent holds nothing)
+    const int lg_stride = wave == 0 ? 0 : wave == 1 ? b_sub_lg[0] : b_sub_lg[0] + b_sub_lg[1];
+    const int lg = wave == 0 ? b_sub_lg[0] : wave == 1 ? b_sub_lg[1] : b_sub_lg[2];
+    const uint64_t rows = na_keys_at_or_after(na_min(lane, 1 << lg), lg_stride, lg);
+    sRows[wave][0][lane] = na_lane_half_bits(rows, 0);
+    sRows[wave][1][lane] = na_lane_half_bits(rows, 1);
+    if (lane == 0) sRows[wave][0][BT] = sRows[wave][1][BT] = 0;
+  }
+  // Accumulator inputs of the first matrix instruction of a logit / dP block: -log2e LSE and -delta of
+  // the block's queries, so that P = exp2(S) and dS = P dP are what the matrix pipe returns.  In the
+  // key-stationary roles they differ by row and come from the tile's table in LDS; in the dQ role they
+  // are the lane's own, sixteen copies of them where the registers allow (head dims below 128).
+  constexpr bool INIT_REGS = !KV_STATIONARY && D < 128;
+  float lse_l = 0.f, delta_l = 0.f;
+  if constexpr (!KV_STATIONARY) {
+    const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
+                                     : stat_row_q + head_a * stat_head_stride + a_seq_row;
+    lse_l = p.lse[stat_idx] * p.lse_mul;
+    delta_l = p.delta[stat_idx] * p.delta_mul;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) x1f[ks] = scale_query_fragment<T>(x1f[ks], p.scale * kLog2e);
+  }
+  f32x16_t lse_init, delta_init;
+  if constexpr (INIT_REGS) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      lse_init[r] = lse_l;
+      delta_init[r] = delta_l;
+    }
+  }
+
 
   // One streamed tile: its two 32-row sub-blocks one after the other, each as products (S, dP),
   // probabilities, accumulations.  Only one sub-block's products are live at a time, which keeps
@@ -1040,7 +1046,6 @@ fna_bwd_kernel(const FnaBwdParams p) {
       __builtin_amdgcn_sched_barrier(0);
     });
   };
-  constexpr int CPT = 2 * PER;  // tile copies per thread and tile
   workgroup_sync();  // sRows is written
   // The paired role over n_iter tiles: step `it` has the P waves on tile `it` and the dS waves forming
   // dP of tile `it` after finishing tile it - 1; one more step drains the dS waves.  Tiles are copied
@@ -1051,15 +1056,9 @@ fna_bwd_kernel(const FnaBwdParams p) {
   auto run_pair = [&](auto ds_wave_tag) __attribute__((always_inline)) {
     constexpr bool DS_WAVE = decltype(ds_wave_tag)::value;
     uint32_t bits0 = 0, bits1 = 0, bits2 = 0;  // P waves: attended pairs of the tiles it, it + 1, it + 2 (while masked)
-    {
-      const Tile t = next_tile();
-      issue_copies(t, 0, 0);
-      if constexpr (!DS_WAVE) bits0 = pair_bits(t);
-    }
-    if (1 < n_iter) {
-      const Tile t = next_tile();
-      issue_copies(t, 1, 1);
-      if constexpr (!DS_WAVE) bits1 = pair_bits(t);
+    if constexpr (!DS_WAVE) {
+      bits0 = pair_bits(tile0);
+      bits1 = pair_bits(tile1);  // (of tile 0 again, never used, where it is the only one)
     }
     // A wave walks to tile it + 2 and issues its share of the copies where it has vector or
     // scalar work anyway: the dS waves between their two matrix phases, the P waves after the
@@ -1118,8 +1117,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
       issue_copies(t, stage, stage);
       return t;
     };
-    bits0 = pair_bits(issue_next(0));
-    if (NS > 2 && 1 < n_iter) bits1 = pair_bits(issue_next(1));
+    bits0 = pair_bits(tile0);
+    if (NS > 2) bits1 = pair_bits(tile1);
     int stage = 0;  // it % NS
     auto step = [&](auto masked_tag, int it) __attribute__((always_inline)) {
       constexpr bool MASKED = decltype(masked_tag)::value;

@@ -254,6 +254,30 @@ static __device__ __forceinline__ void async_copy16_uniform(uint64_t base, uint3
       : "memory", "m0");
 }
 
+// Brings the first BYTES of a kernel's launch parameters into the scalar cache: the set-up reads them where it needs
+// them, line after line, each a trip of its own to memory for the first workgroup of a compute unit (2 x 64 x 64
+// tokens, 13 x 13, forward: the first product of a workgroup after 9900 cycles instead of 12600).
+template <int FIRST, int LINES>
+static __device__ __forceinline__ void touch_eight_lines(uint64_t args) {
+  constexpr auto at = [](int i) { return 64 * (FIRST + i < LINES ? FIRST + i : LINES - 1); };
+  uint32_t x[8];
+  asm volatile(
+      "s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
+      "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
+      : "s"(args), "n"(at(0)), "n"(at(1)), "n"(at(2)), "n"(at(3)), "n"(at(4)), "n"(at(5)), "n"(at(6)), "n"(at(7)));
+  asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]));
+}
+template <int BYTES>
+static __device__ __forceinline__ void touch_launch_params() {
+  constexpr int LINES = (BYTES + 63) / 64;
+  static_assert(LINES >= 8 && LINES <= 16, "two batches of eight loads at most, spare ones of the last line");
+  const uint64_t args = uint64_t(reinterpret_cast<uintptr_t>((const void*)__builtin_amdgcn_kernarg_segment_ptr()));
+  touch_eight_lines<0, LINES>(args);
+  if constexpr (LINES > 8) touch_eight_lines<8, LINES>(args);
+}
+
 static __device__ __forceinline__ uint64_t uniform64(const void* p) {
   const uint64_t b = reinterpret_cast<uint64_t>(p);
   return (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(b >> 32)))) << 32) |
@@ -336,6 +360,13 @@ static __device__ __forceinline__ void store_row_blocks(T* orow, const f32x16_t 
       if (valid && db * 32 + 8 * (j + g) < row_dim)
         *reinterpret_cast<u32x4_t*>(orow + db * 32 + 8 * (j + g)) = u32x4_t{w[0], w[1], w[2], w[3]};
     }
+}
+
+// x of the lane with the same number in the wave's lower half
+static __device__ __forceinline__ int lower_half(int x) {
+  int a = x, b = x;
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return a;
 }
 
 constexpr uint32_t kGuardBits = (1u << 9) | (1u << 19) | (1u << 29);
@@ -1350,27 +1381,11 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 constexpr int fwd_min_waves(int d, bool nomask) { return d == 64 && nomask ? 3 : 2; }
 constexpr int fwd_max_waves(int d, bool nomask) { return d == 32 || (d == 64 && nomask) ? 3 : 2; }
 
-// Brings the launch parameters into the scalar cache: the set-up reads them where it needs them, line after line,
-// each a trip of its own to memory for the first workgroup of a compute unit (2 x 64 x 64 tokens, 13 x 13: the first
-// product of a workgroup after 9900 cycles instead of 12600).
-static __device__ __forceinline__ void touch_launch_params() {
-  static_assert(sizeof(FnaParams) > 7 * 64 && sizeof(FnaParams) <= 8 * 64, "one load per 64 bytes");
-  const uint64_t args = uint64_t(reinterpret_cast<uintptr_t>((const void*)__builtin_amdgcn_kernarg_segment_ptr()));
-  uint32_t x[8];
-  asm volatile(
-      "s_load_dword %0, %8, 0x0\n\ts_load_dword %1, %8, 0x40\n\ts_load_dword %2, %8, 0x80\n\t"
-      "s_load_dword %3, %8, 0xc0\n\ts_load_dword %4, %8, 0x100\n\ts_load_dword %5, %8, 0x140\n\t"
-      "s_load_dword %6, %8, 0x180\n\ts_load_dword %7, %8, 0x1c0\n\ts_waitcnt lgkmcnt(0)"
-      : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
-      : "s"(args));
-  asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]));
-}
-
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
 __global__ void __launch_bounds__(NWAVES * 64)
     __attribute__((amdgpu_waves_per_eu(MQ == 1 ? fwd_min_waves(D, NOMASK) : 1, MQ == 1 ? fwd_max_waves(D, NOMASK) : 1)))
 fna_fwd_kernel(const FnaParams p) {
-  touch_launch_params();
+  touch_launch_params<sizeof(FnaParams)>();
   fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC>(p, int(blockIdx.x), []() {});
 }
 
@@ -1382,7 +1397,7 @@ fna_fwd_kernel(const FnaParams p) {
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, int DC = 0>
 __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
 fna_fwd_split_kernel(const FnaParams p) {
-  touch_launch_params();
+  touch_launch_params<sizeof(FnaParams)>();
   fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
 }
 

@@ -146,4 +146,17 @@ NA_HD int na_last_query_attending(int j1, int k, int s, NaDiv s_div, int L, int 
   return reach < 0 ? -1 : na_min(na_div(reach, s_div) * s + s - 1, Lq - 1);
 }
 
+// The two without branches, for vector code.
+NA_HD int na_first_query_attending_flat(int j0, int k, int s, NaDiv s_div, int Lq, bool causal) {
+  const int start = j0 - k + 1;
+  const int past = start + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
+  const int group = na_div(na_max(past, 0) + s - 1, s_div) * s;
+  return na_min(causal ? j0 : (start <= 0 || past <= 0) ? 0 : group, Lq);
+}
+NA_HD int na_last_query_attending_flat(int j1, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
+  const int reach = causal ? j1 + k - s : j1 + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
+  const int group = na_min(na_div(na_max(reach, 0), s_div) * s + s - 1, Lq - 1);
+  return (j1 + k >= L) ? Lq - 1 : (!causal && reach < 0) ? -1 : group;
+}
+
 }  // namespace natten_amd
