@@ -316,6 +316,14 @@ int natten_amd_query_range(int key_first, int key_last, int kernel_size, int str
                            int32_t* last_query);
 
 /*
+ * How many keys before the first one the key tiles of the dk / dv launch begin along one dimension when
+ * natten_amd_fna_backward_fused lays them out by the windows (`roles` + 8): key_tile is the key tile's
+ * extent there, query_tile that of the streamed half query tiles.  Host arithmetic only.
+ */
+int natten_amd_key_tile_shift(int extent, int kernel_size, int stride, int is_causal, int key_tile,
+                              int query_tile, int32_t* shift);
+
+/*
  * delta[i] = sum_d out[i, d] * d_out[i, d] for `items` rows of head_dim contiguous elements
  * (any layout whose last dimension is head_dim: items = batch * tokens * heads).  float32 result.
  */
@@ -394,7 +402,9 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
  * dk / dv launch half Q tiles past a KV tile, and the shapes that visit the fewest tiles differ
  * (a caller makes one call per role, each with that role's shapes).  Plus 4 (5, 6 or 7): lse, delta
  * and q_scaled hold what natten_amd_backward_prepare wrote (neg_lse2, neg_delta, q_scaled), which
- * saves the call its own pass over q and the kernels the scaling of the two arrays.
+ * saves the call its own pass over q and the kernels the scaling of the two arrays.  Plus 8: the key
+ * tiles of the dk / dv launch may begin before the first key, where the windows make that meet fewer
+ * query tiles (the sums over queries then run in another order).
  */
 int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out,
                                   const float* lse, const float* delta, void* dq, void* dk,

@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 20
+ABI_VERSION = 21
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -85,6 +85,7 @@ _SIGNATURES = {
         + [ctypes.c_void_p] * 4,
     ),
     "natten_amd_query_range": (ctypes.c_int, [ctypes.c_int] * 7 + [ctypes.c_void_p] * 2),
+    "natten_amd_key_tile_shift": (ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_void_p]),
     "natten_amd_compute_delta": (
         ctypes.c_int,
         [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_void_p],
@@ -576,6 +577,14 @@ def query_range(key_first: int, key_last: int, kernel_size: int, stride: int, ex
     return first.value, last.value
 
 
+def key_tile_shift(extent: int, kernel_size: int, stride: int, is_causal: bool, key_tile: int, query_tile: int) -> int:
+    """How many keys before the first one the key tiles of the dk / dv launch begin along a dimension (host arithmetic only)."""
+    shift = ctypes.c_int32()
+    _check(lib().natten_amd_key_tile_shift(int(extent), int(kernel_size), int(stride), 1 if is_causal else 0, int(key_tile),
+                                           int(query_tile), ctypes.byref(shift)))
+    return shift.value
+
+
 def compute_delta(out: Tensor, d_out: Tensor) -> Tensor:
     """rowsum(out * d_out) over the last dimension, float32, shape out.shape[:-1]."""
     L = lib()
@@ -670,8 +679,9 @@ def fna_backward_fused(
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """Backward on the original tensors [B, *X, H, D] (lse, delta [B, *X, H]) -> (dq, dk, dv).  With
     `out` (the forward's output) instead of delta, one pass forms delta and what else the launches read.
-    kv_role_*_tile_shape: tile shapes of the launch that forms dk and dv, when they differ from those
-    of the dq launch (q_tile_shape, kv_tile_shape)."""
+    kv_role_*_tile_shape: tile shapes of the launch that forms dk and dv, whose key tiles are then also laid out
+    by the windows; without them it has those of the dq launch (q_tile_shape, kv_tile_shape) and its key tiles lie at
+    multiples of their extents."""
     L = lib()
     na_dim = len(kernel_size)
     B, H = q.shape[0], q.shape[-2]
@@ -687,7 +697,7 @@ def fna_backward_fused(
     else:
         lse, delta = _head_major(lse, delta)
     _require_gpu(q, k, v, d_out, lse, delta)
-    prepared = 4 if out is not None else 0
+    prepared = (4 if out is not None else 0) + (8 if kv_role_q_tile_shape is not None else 0)
     same = kv_role_q_tile_shape is None or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
     # The dk / dv launch streams the queries as the forward kernel multiplied them (scaled, rounded

@@ -74,6 +74,7 @@ struct FnaBwdParams {
   int ksize[3], stride[3], dil[3], causal[3];
   int q_tile[3], kv_tile[3];    // 128-token tiles of the two permuted layouts
   int q_tiled[3], kv_tiled[3];  // tiles per dimension
+  int kv_shift[3];              // fused == 1, key-stationary launches: key tile t holds the keys from t kv_tile - kv_shift on (choose_kv_shift)
   int q_split, kv_split;        // the dimension along which a 128-token tile of either side halves
                                 // (its last dimension of extent > 1, so that the halves are contiguous)
   float scale;
@@ -136,6 +137,50 @@ inline void set_bwd_divisions(FnaBwdParams& p) {
   p.d_num_kv = na_make_div(p.kv_tiled[0] * p.kv_tiled[1] * p.kv_tiled[2]);
   p.d_heads_q = na_make_div(p.heads_q);
   p.d_heads_kv = na_make_div(p.heads_kv);
+}
+
+// Where the key tiles of the key-stationary launch begin (original layout).  With strided windows the queries that
+// attend a key change at the keys where a stride group's window begins or ends; tiles that begin there meet fewer
+// query tiles than tiles at multiples of their extent, which cross such a key in the middle (128 x 128 tokens, window
+// 32 x 32, stride 16 x 16, H 16, D 128, key tiles of 8 x 16: the launch takes 430 us with tiles at multiples of 16 and 362
+// with the first tile beginning 8 keys early).  Per dimension, the choice that meets the fewest among: multiples of
+// the extent, the first keys of windows, their ends, the last tile ending with the keys -- and at least a
+// twentieth fewer than the first, since other choices may take a tile more.  Tiles are counted from both
+// ends where there are many: what lies between repeats.
+inline int choose_kv_shift(int L, int k, int s, bool causal, int tile, int q_sub) {
+  if (s <= 1 || tile <= 1 || L <= tile) return 0;
+  const NaDiv d = na_make_div(s);
+  const int begin = causal ? s - k : s / 2 - k / 2;  // windows of whole groups begin at begin + i s
+  auto place = [&](int x) { return ((-x) % tile + tile) % tile; };
+  const int candidate[4] = {0, place(begin), place(begin + k), place(L)};
+  auto met = [&](int shift) {
+    const int n = (L + shift + tile - 1) / tile;
+    double sum = 0;
+    int counted = 0;
+    for (int t = 0; t < n; ++t) {
+      if (n > 64 && t == 32) t = n - 32;
+      const int j0 = na_max(t * tile - shift, 0), j1 = na_min((t + 1) * tile - shift, L) - 1;
+      const int lo = na_first_query_attending(j0, k, s, d, L, causal), hi = na_last_query_attending(j1, k, s, d, L, L, causal);
+      const int flo = na_first_query_attending(j1, k, s, d, L, causal), fhi = na_last_query_attending(j0, k, s, d, L, L, causal);
+      ++counted;
+      if (lo > hi) continue;
+      const int tiles = hi / q_sub - lo / q_sub + 1;
+      const int whole = na_max((fhi + 1) / q_sub - (flo + q_sub - 1) / q_sub, 0);
+      sum += tiles + 0.3 * (tiles - whole);
+    }
+    return sum * n / counted;
+  };
+  const double plain = met(0);
+  double least = plain * 0.95;
+  int best = 0;
+  for (int i = 1; i < 4; ++i) {
+    const double m = candidate[i] ? met(candidate[i]) : plain;
+    if (m < least) {
+      least = m;
+      best = candidate[i];
+    }
+  }
+  return best;
 }
 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
@@ -465,7 +510,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
       // (as in the forward kernel: the first groups hold one token more when the dilation does not divide the extent)
       extent[a] = (a == 0 ? keys0 : p.ext_base[a]) + (gi < p.ext_rem[a] ? 1 : 0);
       q_extent[a] = (a == 0 && queries0 > 0) ? queries0 : extent[a];
-      a_first[a] = tc[a] << a_tile_lg[a];
+      a_first[a] = (tc[a] << a_tile_lg[a]) - (KV_STATIONARY && !RAGGED ? p.kv_shift[a] : 0);
       b_sub_lg[a] = b_tile_lg[a] - (a == split_dim ? 1 : 0);
       b_sub[a] = 1 << b_sub_lg[a];
       if (a_first[a] >= (KV_STATIONARY ? extent[a] : q_extent[a])) empty = true;
@@ -480,15 +525,15 @@ fna_bwd_kernel(const FnaBwdParams p) {
   a_off[2] = r_in >> (a_tile_lg[0] + a_tile_lg[1]);
   // Row of the tensors / index into lse and delta: position in the permuted sequence, or the
   // token of the lane's coordinate in the original layout.
-  // (original layout: a row past the end of its dilation group works on the group's last row and stores nothing)
+  // (original layout: a row past an end of its dilation group works on the group's first or last row and stores nothing)
   int a_crd[3];
   bool a_valid = true;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
     const int c = a_first[a] + a_off[a];
     const int e = KV_STATIONARY ? extent[a] : q_extent[a];
-    a_valid = a_valid && (c < e || !(RAGGED || p.fused));
-    a_crd[a] = (RAGGED || p.fused) ? na_min(c, e - 1) : c;
+    a_valid = a_valid && ((c >= 0 && c < e) || !(RAGGED || p.fused));
+    a_crd[a] = (RAGGED || p.fused) ? na_max(na_min(c, e - 1), 0) : c;
   }
   const int a_tok = group_tok + a_crd[0] * tok_step[0] + a_crd[1] * tok_step[1] + a_crd[2] * tok_step[2];
   const int64_t batch_row0 = p.fused ? int64_t(b_orig) * p.tokens : 0;  // first row of the batch entry (original layout)
@@ -517,7 +562,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // rows give the box of streamed tiles it meets, and the inner box of those every row of which pairs with
   // every row of the tile (no mask needed).  One evaluation per dimension serves all of it: the lower half of
   // the wave takes its lanes' rows (the lanes of the upper half, which hold the same ones, get the results
-  // from there), lane 32 the tile's first row, lane 33 its last one inside the extent, lane 34 its last one.
+  // from there), lane 32 the tile's first row inside the extent, lane 33 its last one inside the extent, lane 34 its last one.
   // A workgroup's first step began after 10000 cycles: the loads of the launch parameters one behind the other, 18
   // evaluations of which 12 on the scalar unit, and the tables before the first copies.  dK / dV and dQ launches,
   // us before / after: 4 x 56 x 56, 7 x 7, H 8, D 32 41.4 / 39.0 and 32.4 / 31.3; 56 x 56, H 32, D 64 56.2 / 53.7 and 43.2 / 42.7;
@@ -529,15 +574,15 @@ fna_bwd_kernel(const FnaBwdParams p) {
   for (int a = 0; a < 3; ++a) {
     const int e = KV_STATIONARY ? extent[a] : q_extent[a];
     const int last = a_first[a] + a_tile[a] - 1, last_in = na_max(na_min(last, e - 1), 0);
-    const int c = g == 0 ? a_crd[a] : l32 == 0 ? a_first[a] : l32 == 1 ? last_in : last;
+    const int c = g == 0 ? a_crd[a] : l32 == 0 ? na_max(a_first[a], 0) : l32 == 1 ? last_in : last;
     const bool cs = p.causal[a] != 0;
     int from, upto;
     if constexpr (!KV_STATIONARY) {
-      from = na_window_start_flat(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
+      from = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
       upto = na_window_end(c, from, ksz[a], extent[a], cs);
     } else {
-      from = na_first_query_attending_flat(c, ksz[a], p.stride[a], p.d_stride[a], q_extent[a], cs);
-      upto = na_last_query_attending_flat(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs) + 1;
+      from = na_first_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], q_extent[a], cs);
+      upto = na_last_query_attending(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], q_extent[a], cs) + 1;
       if (c >= extent[a]) upto = from;  // a padding key of a permuted sequence: nothing attends it
     }
     win_lo[a] = lower_half(from);

@@ -606,7 +606,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       const int edge = (l32 & 2) ? ((l32 & 1) ? o[a] + (1 << p.wave_box_lg[a]) - 1 : o[a]) : ((l32 & 1) ? p.q_tile[a] - 1 : 0);
       const int c = g == 0 ? own : q_first[a] + edge;
       const bool cs = p.causal[a] != 0;
-      const int ws = na_window_start_flat(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
+      const int ws = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
       const int we = na_window_end(c, ws, ksz[a], extent[a], cs);
       if constexpr (!NOMASK) {
         if (g == 0) {

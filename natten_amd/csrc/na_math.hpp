@@ -57,21 +57,9 @@ inline NaDiv na_make_div(int d) {
 
 NA_HD int na_div(int n, NaDiv f) { return int((uint64_t(f.mul) * uint64_t(uint32_t(n))) >> f.shift); }
 
-// na_window_start with the stride's division precomputed (s_div = na_make_div(s))
+// na_window_start with the stride's division precomputed (s_div = na_make_div(s)), without a branch on `causal`: the
+// kernels evaluate it for a query per lane.
 NA_HD int na_window_start(int i, int k, int s, NaDiv s_div, int L, bool causal) {
-  const int wl = int(uint32_t(k) >> 1);
-  const int wr = wl + int(uint32_t(k) & 1u) - 1;
-  const int group_first = na_div(i, s_div) * s;
-  if (causal) {
-    const int leader = na_min(group_first + s - 1, L - 1);
-    return na_max(leader - wl - wr, 0);
-  }
-  const int leader = na_min(group_first + int(uint32_t(s) >> 1), L - 1);
-  return na_max(leader - wl, 0) + ((leader + wr >= L) ? (L - wr - leader - 1) : 0);
-}
-
-// The same without a branch on `causal`, for vector code.
-NA_HD int na_window_start_flat(int i, int k, int s, NaDiv s_div, int L, bool causal) {
   const int wl = int(uint32_t(k) >> 1);
   const int wr = wl + int(uint32_t(k) & 1u) - 1;
   const int leader = na_min(na_div(i, s_div) * s + (causal ? s - 1 : int(uint32_t(s) >> 1)), L - 1);
@@ -127,36 +115,20 @@ NA_HD int na_group_extent(int X, int d, int g) { return X / d + 1 - ((g + (d - X
 // before j1 (queries 0 .. Lq-1, keys of extent L, s_div = na_make_div(s)).  In closed form, one
 // division each: a window's start is its leader less the left reach, clamped to 0 .. L - k, and
 // the leaders are one per stride group.  An empty interval comes back as first > last.
-NA_HD int na_first_query_attending(int j0, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
-  if (causal) return na_min(j0, Lq);  // a causal window ends at its query
-  // start >= j0 - k + 1, that is leader >= j0 - k + 1 + left reach; without the clamp at 0 nothing to do
-  const int start = j0 - k + 1;
-  if (start <= 0) return 0;
-  const int past = start + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
-  return past <= 0 ? 0 : na_min(na_div(past + s - 1, s_div) * s, Lq);
-}
-
-NA_HD int na_last_query_attending(int j1, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
-  if (causal) {
-    if (j1 + k >= L) return Lq - 1;
-    return na_min(na_div(j1 + k - s, s_div) * s + s - 1, Lq - 1);  // (s <= k)
-  }
-  if (j1 >= L - k) return Lq - 1;
-  const int reach = j1 + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
-  return reach < 0 ? -1 : na_min(na_div(reach, s_div) * s + s - 1, Lq - 1);
-}
-
-// The two without branches, for vector code.
-NA_HD int na_first_query_attending_flat(int j0, int k, int s, NaDiv s_div, int Lq, bool causal) {
+// (Without branches, as above.)
+NA_HD int na_first_query_attending(int j0, int k, int s, NaDiv s_div, int Lq, bool causal) {
+  // causal: a window ends at its query.  Else: start >= j0 - k + 1, that is leader >= j0 - k + 1 + left reach; without
+  // the clamp at 0 nothing to do.
   const int start = j0 - k + 1;
   const int past = start + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
   const int group = na_div(na_max(past, 0) + s - 1, s_div) * s;
   return na_min(causal ? j0 : (start <= 0 || past <= 0) ? 0 : group, Lq);
 }
-NA_HD int na_last_query_attending_flat(int j1, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
-  const int reach = causal ? j1 + k - s : j1 + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);
+
+NA_HD int na_last_query_attending(int j1, int k, int s, NaDiv s_div, int L, int Lq, bool causal) {
+  const int reach = causal ? j1 + k - s : j1 + int(uint32_t(k) >> 1) - int(uint32_t(s) >> 1);  // (s <= k)
   const int group = na_min(na_div(na_max(reach, 0), s_div) * s + s - 1, Lq - 1);
-  return (j1 + k >= L) ? Lq - 1 : (!causal && reach < 0) ? -1 : group;
+  return (j1 >= L - k) ? Lq - 1 : (!causal && reach < 0) ? -1 : group;
 }
 
 }  // namespace natten_amd

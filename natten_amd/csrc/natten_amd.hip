@@ -346,7 +346,7 @@ int fused_geometry(const char* what, FnaParams& p, bool sixteen_bit, int na_dim,
 
 extern "C" {
 
-int natten_amd_abi_version(void) { return 20; }
+int natten_amd_abi_version(void) { return 21; }
 
 uint64_t natten_amd_fna_forward_workspace_bytes(void) { return uint64_t(kQueueWords) * 4; }
 
@@ -1080,8 +1080,12 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                   float scale, int roles, void* stream) {
   g_error[0] = 0;
   const char* what = "fna_backward_fused";
-  if (roles < 1 || roles > 7 || (roles & 3) == 0)
-    return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 for prepared arrays, got %d", what, roles);
+  if (roles < 1 || roles > 15 || (roles & 3) == 0)
+    return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 for prepared arrays, plus 8 for key tiles laid out "
+                "by the windows, got %d",
+                what, roles);
+  const bool lay_out_keys = (roles & 8) != 0;
+  roles &= 7;
   if (int rc = check_bwd_pointers(what, q, k, v, d_out, lse, delta, dq, dk, dv, q_scaled, roles)) return rc;
   if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
   if (!qkv_shape || !kernel_size || !stride || !dilation || !is_causal || !q_tile_shape || !kv_tile_shape)
@@ -1138,6 +1142,11 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
     p.kv_tile[a] = f.kv_tile[a];
     p.q_tiled[a] = f.q_tiled[a];
     p.kv_tiled[a] = f.kv_tiled[a];
+    if (lay_out_keys && (roles & 2)) {
+      const int ext = na_ceil_div(f.qkv_shape[a], f.dil[a]), q_sub = f.q_tile[a] >> (a == p.q_split ? 1 : 0);
+      p.kv_shift[a] = choose_kv_shift(ext, f.ksize[a], f.stride[a], f.causal[a] != 0, f.kv_tile[a], q_sub);
+      p.kv_tiled[a] = na_ceil_div(ext + p.kv_shift[a], f.kv_tile[a]);
+    }
     p.tok_stride[a] = f.tok_stride[a];
     groups *= f.dil[a];
   }
@@ -1253,8 +1262,17 @@ int natten_amd_query_range(int key_first, int key_last, int kernel_size, int str
   if (kernel_size < 1 || stride < 1 || extent < 1 || num_queries < 1 || kernel_size > extent || stride > kernel_size ||
       key_first < 0 || key_last < key_first || key_last >= extent)
     return fail("query_range: invalid argument");
-  *first_query = na_first_query_attending(key_first, kernel_size, stride, na_make_div(stride), extent, num_queries, is_causal != 0);
+  *first_query = na_first_query_attending(key_first, kernel_size, stride, na_make_div(stride), num_queries, is_causal != 0);
   *last_query = na_last_query_attending(key_last, kernel_size, stride, na_make_div(stride), extent, num_queries, is_causal != 0);
+  return 0;
+}
+
+int natten_amd_key_tile_shift(int extent, int kernel_size, int stride, int is_causal, int key_tile, int query_tile, int32_t* shift) {
+  g_error[0] = 0;
+  if (!shift) return fail("key_tile_shift: null pointer argument");
+  if (extent < 1 || kernel_size < 1 || kernel_size > extent || stride < 1 || stride > kernel_size || key_tile < 1 || query_tile < 1)
+    return fail("key_tile_shift: 1 <= stride <= kernel_size <= extent and positive tile extents expected");
+  *shift = choose_kv_shift(extent, kernel_size, stride, is_causal != 0, key_tile, query_tile);
   return 0;
 }
 

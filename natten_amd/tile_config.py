@@ -52,16 +52,16 @@ def _win(i: int, k: int, s: int, L: int, causal: bool) -> Tuple[int, int]:
 
 
 @functools.lru_cache(maxsize=4096)
-def _dim_cost(L: int, k: int, s: int, causal: bool, tq: int, tk: int, anchored: bool = False) -> Tuple[int, int]:
+def _dim_cost(L: int, k: int, s: int, causal: bool, tq: int, tk: int, anchored: bool = False, shift: int = 0) -> Tuple[int, int]:
     """(visited pairs, fully-unmasked pairs) along one dimension of extent L for Q tile extent tq
     and KV tile extent tk; the totals of a multi-dimensional problem are products of these.
     `anchored`: the KV tiles of a Q tile start at its window's first key (the one-launch forward
-    on the original tensors) instead of at multiples of tk."""
+    on the original tensors) instead of at multiples of tk.  `shift`: multiples of tk less that many keys."""
     visited = full = 0
     for q0 in range(0, _ceil_div(L, tq) * tq, tq):
         st_f, en_f = _win(q0, k, s, L, causal)
         st_l, en_l = _win(q0 + tq - 1, k, s, L, causal)
-        org = st_f if anchored and L >= tk else (st_f // tk) * tk
+        org = st_f if anchored and L >= tk else ((st_f + shift) // tk) * tk - shift
         n = _ceil_div(en_l - org, tk)
         visited += n * tk * tq
         for t in range(n):
@@ -238,6 +238,20 @@ def choose_backward_role_tile_shapes(
                                              tuple(is_causal))
 
 
+@functools.lru_cache(maxsize=4096)
+def _key_tile_dim_cost(L: int, k: int, s: int, causal: bool, tq: int, tk: int) -> Tuple[int, int]:
+    """_dim_cost of the dk / dv launch, whose key tiles may begin before the first key (choose_kv_shift in
+    csrc/fna_bwd.hpp, which has the last word on where)."""
+    plain = best = _dim_cost(L, k, s, causal, tq, tk)
+    if s > 1 and 1 < tk < L:
+        begin = s - k if causal else s // 2 - k // 2
+        for shift in {-begin % tk, -(begin + k) % tk, -L % tk}:
+            cost = _dim_cost(L, k, s, causal, tq, tk, False, shift)
+            if 1.3 * cost[0] - 0.3 * cost[1] < min(1.3 * best[0] - 0.3 * best[1], 0.95 * (1.3 * plain[0] - 0.3 * plain[1])):
+                best = cost
+    return best
+
+
 @functools.lru_cache(maxsize=1024)
 def _choose_backward_role_tile_shapes(
     token_layout: DimensionType, kernel_size: DimensionType, stride: DimensionType, dilation: DimensionType,
@@ -258,10 +272,11 @@ def _choose_backward_role_tile_shapes(
         return None
     ext = tuple(_ceil_div(x, d) for x, d in zip(token_layout, dilation))
 
-    def cost(q_ext: DimensionType, kv_ext: DimensionType) -> float:
+    def cost(q_ext: DimensionType, kv_ext: DimensionType, role: int) -> float:
+        dim_cost = _key_tile_dim_cost if role else _dim_cost
         visited = full = 1
         for a in range(n):
-            v, f = _dim_cost(ext[a], kernel_size[a], stride[a], is_causal[a], q_ext[a], kv_ext[a])
+            v, f = dim_cost(ext[a], kernel_size[a], stride[a], is_causal[a], q_ext[a], kv_ext[a])
             visited *= v
             full *= f
         return visited + 0.3 * (visited - full)
@@ -271,7 +286,7 @@ def _choose_backward_role_tile_shapes(
         keyed = []
         for qt in shapes:
             for kt in shapes:
-                c = cost(qt, _half_tile(kt)) if role == 0 else cost(_half_tile(qt), kt)
+                c = cost(qt, _half_tile(kt), 0) if role == 0 else cost(_half_tile(qt), kt, 1)
                 keyed.append(((c, tuple(-x for x in reversed(qt)), tuple(-x for x in reversed(kt))), (qt, kt)))
         best.append(min(keyed)[1])
     return best[0], best[1]
