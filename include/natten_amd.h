@@ -194,6 +194,23 @@ int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void*
                                        int anchor_kv_tiles, int kv_splits, void* stream);
 
 /*
+ * natten_amd_fna_forward_fused (anchored KV tiles, fp16 / bf16) whose queries also
+ * attend to context_len >= 64 more keys per batch entry, context_k / context_v [batch, context_len, heads_kv,
+ * head_dim]: out and lse are those of attention over the window and the context together (the role of the
+ * reference's additional keys / values, src/natten/functional.py:354-564, without a merge).  Every dilation
+ * group at least a KV tile wide in every dimension; Q tiles of 128 or, at head dims 32 and 64 and without
+ * run_persistent, of 64 tokens.
+ */
+int natten_amd_fna_forward_fused_context(const void* q, const void* k, const void* v, const void* context_k,
+                                         const void* context_v, void* out, float* lse, int dtype, int na_dim,
+                                         int batch, int context_len, int heads_q, int heads_kv, int head_dim,
+                                         const int32_t* qkv_shape, const int32_t* kernel_size,
+                                         const int32_t* stride, const int32_t* dilation,
+                                         const int32_t* is_causal, const int32_t* q_tile_shape,
+                                         const int32_t* kv_tile_shape, float scale, int run_persistent,
+                                         void* workspace, uint64_t workspace_bytes, void* stream);
+
+/*
  * natten_amd_fna_forward_fused with run_persistent = 1 for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc):
  * it has no counterpart in the reference.  The queue counters live in a 512-byte array inside

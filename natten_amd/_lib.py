@@ -84,6 +84,11 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 5 + [ctypes.c_int] * 9 + [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_float]
         + [ctypes.c_void_p] * 4,
     ),
+    "natten_amd_fna_forward_fused_context": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 7 + [ctypes.c_int] * 7 + [ctypes.c_void_p] * 7
+        + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p],
+    ),
     "natten_amd_query_range": (ctypes.c_int, [ctypes.c_int] * 7 + [ctypes.c_void_p] * 2),
     "natten_amd_key_tile_shift": (ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_void_p]),
     "natten_amd_compute_delta": (
@@ -380,6 +385,34 @@ def fna_forward_fused(
             *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
                              tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
             float(scale), *scales, 1 if anchored_tiles else 0, *_queue_workspace(q, run_persistent), _stream(q),
+        )
+    _check(rc)
+    return out, lse
+
+
+def fna_forward_fused_context(
+    q: Tensor, k: Tensor, v: Tensor, context_k: Tensor, context_v: Tensor,
+    kernel_size, stride, dilation, is_causal, scale: float, q_tile_shape, kv_tile_shape, run_persistent: bool = False,
+) -> Tuple[Tensor, Tensor]:
+    """fna_forward_fused whose queries also attend to context_k / context_v [B, N >= 64, Hkv, D]: (out like q, lse float32
+    [B, *X, H]) of attention over both together, in one launch."""
+    L = lib()
+    _require_gpu(q, k, v, context_k, context_v)
+    if q.dtype not in (torch.float16, torch.bfloat16):
+        raise NotImplementedError(f"natten_amd fna_forward_fused_context does not support {q.dtype}.")
+    q, k, v = _aligned_narrow_rows(q, k, v)
+    if q.shape[-1] not in (32, 64, 128):  # (as _aligned_narrow_rows)
+        context_k, context_v = (t if t.data_ptr() % 16 == 0 else t.clone() for t in (context_k, context_v))
+    na_dim = len(kernel_size)
+    out = torch.empty_like(q)
+    lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
+    with _on_device(q):
+        rc = L.natten_amd_fna_forward_fused_context(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), context_k.data_ptr(), context_v.data_ptr(), out.data_ptr(), lse.data_ptr(),
+            DTYPE_CODES[q.dtype], na_dim, q.shape[0], context_k.shape[1], q.shape[-2], k.shape[-2], q.shape[-1],
+            *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
+                             tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
+            float(scale), *_queue_workspace(q, run_persistent), _stream(q),
         )
     _check(rc)
     return out, lse

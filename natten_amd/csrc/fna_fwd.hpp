@@ -101,8 +101,22 @@ struct FnaParams {
   // to `kv_splits` workgroups in contiguous runs; workgroup `pid` of the grid works on Q-tile
   // position pid % split_grid for split pid / split_grid and stores its partial result (normalised
   // over its own keys, with their LSE) `split` strides into o and lse.
-  int kv_splits, split_grid;
-  int64_t o_split_stride, lse_split_stride;  // elements of the output type / floats
+  // CTX instances only (no splits): ctx_len >= 64 more keys and values per batch entry, [batch, ctx_len, heads_kv, row],
+  // that every query attends to besides its window.  (In one place: the block stays under 512 bytes, which a launch copies.)
+  int kv_splits;
+  union {
+    int split_grid;
+    int ctx_len;
+  };
+  union {
+    int64_t o_split_stride;  // elements of the output type
+    const void* ctx_k;
+  };
+  union {
+    int64_t lse_split_stride;  // floats
+    const void* ctx_v;
+  };
+  __host__ bool has_context() const { return kv_splits <= 1 && ctx_len > 0; }
 };
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -257,25 +271,27 @@ static __device__ __forceinline__ void async_copy16_uniform(uint64_t base, uint3
 // Brings the first BYTES of a kernel's launch parameters into the scalar cache: the set-up reads them where it needs
 // them, line after line, each a trip of its own to memory for the first workgroup of a compute unit (2 x 64 x 64
 // tokens, 13 x 13, forward: the first product of a workgroup after 9900 cycles instead of 12600).
-template <int FIRST, int LINES>
-static __device__ __forceinline__ void touch_eight_lines(uint64_t args) {
-  constexpr auto at = [](int i) { return 64 * (FIRST + i < LINES ? FIRST + i : LINES - 1); };
-  uint32_t x[8];
-  asm volatile(
-      "s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
-      "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
-      : "s"(args), "n"(at(0)), "n"(at(1)), "n"(at(2)), "n"(at(3)), "n"(at(4)), "n"(at(5)), "n"(at(6)), "n"(at(7)));
-  asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]));
-}
 template <int BYTES>
 static __device__ __forceinline__ void touch_launch_params() {
   constexpr int LINES = (BYTES + 63) / 64;
-  static_assert(LINES >= 8 && LINES <= 16, "two batches of eight loads at most, spare ones of the last line");
+  static_assert(LINES >= 8 && LINES <= 12, "eight loads, or four more");
+  constexpr auto at = [](int i) { return 64 * (i < LINES ? i : LINES - 1); };
   const uint64_t args = uint64_t(reinterpret_cast<uintptr_t>((const void*)__builtin_amdgcn_kernarg_segment_ptr()));
-  touch_eight_lines<0, LINES>(args);
-  if constexpr (LINES > 8) touch_eight_lines<8, LINES>(args);
+  uint32_t x[8], y[4] = {0, 0, 0, 0};
+  asm volatile(
+      "s_load_dword %0, %8, 0x0\n\ts_load_dword %1, %8, 0x40\n\ts_load_dword %2, %8, 0x80\n\ts_load_dword %3, %8, 0xc0\n\t"
+      "s_load_dword %4, %8, 0x100\n\ts_load_dword %5, %8, 0x140\n\ts_load_dword %6, %8, 0x180\n\ts_load_dword %7, %8, 0x1c0\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
+      : "s"(args));
+  if constexpr (LINES > 8)
+    asm volatile(
+        "s_load_dword %0, %4, %5\n\ts_load_dword %1, %4, %6\n\ts_load_dword %2, %4, %7\n\ts_load_dword %3, %4, %8\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&s"(y[0]), "=&s"(y[1]), "=&s"(y[2]), "=&s"(y[3])
+        : "s"(args), "n"(at(8)), "n"(at(9)), "n"(at(10)), "n"(at(11)));
+  asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]), "s"(y[0]), "s"(y[1]),
+               "s"(y[2]), "s"(y[3]));
 }
 
 static __device__ __forceinline__ uint64_t uniform64(const void* p) {
@@ -369,6 +385,8 @@ static __device__ __forceinline__ int lower_half(int x) {
   return a;
 }
 
+constexpr int kCtxTile = -(1 << 30);  // in place of the first coordinate of a tile of context keys
+
 constexpr uint32_t kGuardBits = (1u << 9) | (1u << 19) | (1u << 29);
 // a row's running maximum may lag the true one by up to this many powers of two
 constexpr float kLazyRescaleLog2 = 8.0f;
@@ -431,8 +449,11 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // result cost more than the attention itself (2x64x64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context
 // tokens: the call takes 76 us instead of 139 with its ten copies and fills).  The chunks past a row are not
 // fetched: their places in the tiles are zeroed once, before the first copy.
+// CTX: every query also attends to the ctx_len keys of its batch entry's context, whose tiles come behind those of the
+// window box, in the same walk.  Context as a launch of dense attention of its own and a merge write and read both
+// results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a call 62 -> 31; 4 x 96 x 96, 24 x 24, H 16, D 128, 256 tokens: 665 -> 476).
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
-          typename Hook>
+          bool CTX = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
   const int split = SPLIT ? pid_in / p.split_grid : 0;
@@ -627,8 +648,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // The tiles this workgroup visits: all of the box, or run `split` of its kv_splits runs.  A run
   // that is empty (a box of fewer tiles than splits) still walks one tile, for the sake of one code
   // path, and stores the result of no keys at all: zeros and an LSE of -inf.
+  static_assert(!CTX || (!SPLIT && !NOMASK && !RAGGED && KVT == 64), "context tiles: masked instances that hold whole tiles");
   const int box_tiles = box_n[0] * box_n[1] * box_n[2];
-  int first_tile = 0, total_tiles = box_tiles;
+  const int ctx_len = CTX ? p.ctx_len : 0;
+  int first_tile = 0, total_tiles = box_tiles + (ctx_len + KVT - 1) / KVT;
   bool empty_split = false;
   if constexpr (SPLIT) {
     first_tile = int(int64_t(split) * box_tiles / p.kv_splits);
@@ -652,6 +675,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const int64_t kv_base = (kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim) * 2 - kImmBias;
   const char* kbase = static_cast<const char*>(p.k) + kv_base;
   const char* vbase = static_cast<const char*>(p.v) + kv_base;
+  const int64_t ctx_base = CTX ? (int64_t(b_orig) * ctx_len * kv_row_stride + int64_t(head_kv) * row_dim) * 2 - kImmBias : 0;
   if constexpr (NARROW) {
     // (every copy leaves out the same places, so this is needed once)
     for (int i = tid; i < TILE_BYTES / 16; i += NT) {
@@ -685,24 +709,35 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // tile extents are powers of two, so that bit moves one coordinate by a fixed amount and the
   // row (permuted) or token (fused) distance to copy i is the same for every lane.
   const int64_t bytes_per_4 = int64_t(kv_tile_pos(ROWS_PER_4 % KVT)) * (kv_row_stride * 2);
+  static_assert(!CTX || PER <= 4, "the distance between the copies i and i + 4 is the window's");
   int ld_row[NOFF];
   uint32_t ld_koff[NOFF], ld_voff[NOFF];
+  auto copy_offset = [&](int i, auto v_tag, auto&& pos_of) __attribute__((always_inline)) {
+    constexpr bool V_LAYOUT = decltype(v_tag)::value;
+    const int P = (wave * PER + i) * 64 + lane;
+    const int row = P / CPR, slot = P % CPR;
+    // XOR swizzles are involutions: slot -> source chunk uses the same function
+    const int chunk = V_LAYOUT ? L::v_slot(row, slot) : L::k_slot(row, slot);
+    // the instruction adds its immediate i * 1024 to the global address as well (RAGGED: taken off the base): take it
+    // off here, on top of a bias that keeps the offset non-negative and is taken off the tile base
+    return uint32_t(pos_of(row)) * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16) + (RAGGED ? 0u : uint32_t(kImmBias - i * 1024));
+  };
 #pragma unroll
   for (int i = 0; i < NOFF; ++i) {
-    const int P = (wave * PER + i) * 64 + lane;
-    ld_row[i] = P / CPR;
-    const int slot = P % CPR;
-    // XOR swizzles are involutions: slot -> source chunk uses the same function
-    const uint32_t pos = uint32_t(kv_tile_pos(ld_row[i]));
-    ld_koff[i] = pos * uint32_t(kv_row_stride * 2) + uint32_t(L::k_slot(ld_row[i], slot) * 16);
-    ld_voff[i] = pos * uint32_t(kv_row_stride * 2) + uint32_t(L::v_slot(ld_row[i], slot) * 16);
-    if constexpr (!RAGGED) {
-      // the instruction adds its immediate i * 1024 to the global address as well: take it off
-      // here, on top of a bias that keeps the offset non-negative and is taken off the tile base
-      ld_koff[i] += uint32_t(kImmBias - i * 1024);
-      ld_voff[i] += uint32_t(kImmBias - i * 1024);
-    }
+    ld_row[i] = ((wave * PER + i) * 64 + lane) / CPR;
+    ld_koff[i] = copy_offset(i, std::false_type{}, kv_tile_pos);
+    ld_voff[i] = copy_offset(i, std::true_type{}, kv_tile_pos);
   }
+  // CTX: from the first context tile on (number box_tiles) the copies are of consecutive rows of the context
+  auto at_tile = [&](int tile, const char*& base, uint32_t (&off)[NOFF], const void* ctx, auto v_tag) __attribute__((always_inline)) {
+    if constexpr (CTX) {
+      if (tile == box_tiles) {
+        base = static_cast<const char*>(ctx) + ctx_base;
+#pragma unroll
+        for (int i = 0; i < NOFF; ++i) off[i] = copy_offset(i, v_tag, [](int row) { return row; });
+      }
+    }
+  };
   // KV tile stream: dimension 2 fastest, dimension 0 slowest.  The tiles are described 64 at a time, one
   // per lane, and a tile's description is read back by lane number: its first row, and whether all keys
   // are attended by all queries of this wave (no mask) or none by any.  Forming it tile by tile on the
@@ -732,7 +767,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     d_first = first;
     // lanes past the last tile describe that one again: copies past the end re-read it into a free stage (never used)
     int t[3];
-    kv_tile_of_box(first_tile + na_min(first + lane, total_tiles - 1), box_n, t);
+    const int number = na_min(first + lane, total_tiles - 1);
+    kv_tile_of_box(first_tile + (CTX ? na_min(number, box_tiles - 1) : number), box_n, t);
     bool full = true, skip = false;
     int lead = 0;
 #pragma unroll
@@ -747,13 +783,24 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       else d_origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
       lead |= (org - d_origin[a]) << (8 * a);
     }
+    // (the clamping instances see no permuted rows, and hold tok_step anyway)
+    const int* row_step = RAGGED ? tok_step : p.kv_row_step;
+    d_row0 = d_origin[0] * row_step[0] + d_origin[1] * row_step[1] + d_origin[2] * row_step[2];
+    if constexpr (CTX) {
+      // the last context tile is moved back to end with the context; no coordinates: its first one is marked
+      const int org = (number - box_tiles) * KVT;
+      if (number >= box_tiles) {
+        d_row0 = na_min(org, ctx_len - KVT);
+        lead = org - d_row0;
+        d_origin[0] = kCtxTile;
+        full = lead == 0;
+        skip = false;
+      }
+    }
     if constexpr (!NOMASK) {
       typedef int i32x4 __attribute__((ext_vector_type(4)));
       *reinterpret_cast<i32x4*>(&sTile[wave * 64 + lane][0]) = i32x4{d_origin[0], d_origin[1], d_origin[2], lead};
     }
-    // (the clamping instances see no permuted rows, and hold tok_step anyway)
-    const int* row_step = RAGGED ? tok_step : p.kv_row_step;
-    d_row0 = d_origin[0] * row_step[0] + d_origin[1] * row_step[1] + d_origin[2] * row_step[2];
     if constexpr (!NOMASK && (kAblate & kAblateMask) == 0) {
       d_plain = __ballot(full && !skip);
       d_skip = __ballot(skip);
@@ -1082,7 +1129,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   };
   auto apply_mask = [&](f32x16_t (&S)[NSB], int mb, const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
     if constexpr (!NOMASK) {
-      const uint32_t lane_bits = mask_bits(mb, origin, lead);
+      uint32_t lane_bits = mask_bits(mb, origin, lead);
+      // (a context tile holds no coordinates: what the line above made of its row is replaced)
+      if constexpr (CTX) lane_bits = origin[0] == kCtxTile ? na_lane_half_bits(~na_ones64(lead[0]), g) : lane_bits;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
@@ -1170,6 +1219,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   TileRows nxt = tile_rows(1);  // tile 1
   wait_vmcnt<0>();
   workgroup_sync();  // K(0), V(0), the mask tables and the queries' windows are in LDS
+  at_tile(1, kbase, ld_koff, p.ctx_k, KLayout{});
   if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, 1, KLayout{});
 #pragma unroll
   for (int mb = 0; mb < MQ; ++mb)
@@ -1215,6 +1265,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     // (never used), which keeps the slots below free of control flow.
     const int l2 = j + 2 - d_first;
     const TileRows t2 = tile_rows(l2);
+    at_tile(j + 2, kbase, ld_koff, p.ctx_k, KLayout{});
+    at_tile(j + 1, vbase, ld_voff, p.ctx_v, VLayout{});
     const TileCopy ck = make_copy(kbase, sK_cur, t2, l2);
     const TileCopy cv = make_copy(vbase, sV_nxt, nxt, l2 - 1);
     if constexpr (!SPREAD && (kAblate & kAblateCopies) == 0) {
@@ -1381,12 +1433,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 constexpr int fwd_min_waves(int d, bool nomask) { return d == 64 && nomask ? 3 : 2; }
 constexpr int fwd_max_waves(int d, bool nomask) { return d == 32 || (d == 64 && nomask) ? 3 : 2; }
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
 __global__ void __launch_bounds__(NWAVES * 64)
     __attribute__((amdgpu_waves_per_eu(MQ == 1 ? fwd_min_waves(D, NOMASK) : 1, MQ == 1 ? fwd_max_waves(D, NOMASK) : 1)))
 fna_fwd_kernel(const FnaParams p) {
   touch_launch_params<sizeof(FnaParams)>();
-  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC, CTX>(p, int(blockIdx.x), []() {});
 }
 
 // Split launch: kv_splits workgroups per Q tile, each on a contiguous run of the tile's KV tiles,
@@ -1487,12 +1539,12 @@ static __device__ __forceinline__ void fna_queue_loop(uint32_t* __restrict__ que
   }
 }
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false>
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, bool CTX = false>
 __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
 fna_fwd_queue_kernel(const FnaParams p, uint32_t* __restrict__ queues, const int per_xcd) {
   FnaKernargPtr args = fna_kernarg_params();
   fna_queue_loop(queues, per_xcd, [&](int pid, auto& fetch) __attribute__((always_inline)) {
-    fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK>(fna_params_for_this_tile(args), pid, fetch);
+    fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, 0, CTX>(fna_params_for_this_tile(args), pid, fetch);
   });
   (void)p;
 }

@@ -89,18 +89,18 @@ struct WorkQueue {
 };
 
 // DC != 0: rows of p.row_dim elements, DC columns multiplied (no work-queue launch)
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0>
+template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
 int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   constexpr int QT = NWAVES * MQ * 32;
   if (!fna_tiles_are_powers_of_two(p)) return fail("fna_forward: tile extents must be powers of two");
   if ((p.seqlen_q + QT - 1) / QT != p.num_q_tiles) return fail("fna_forward: internal tile count mismatch");
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
   if (wgs > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
-  if constexpr (DC == 0) {
+  if constexpr (DC == 0 && (NWAVES == 4 || !CTX)) {
     if (queues.counters != nullptr) {
       const long long resident = resident_workgroups();
       if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
-      hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK>),
+      hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, CTX>),
                          dim3((unsigned)(wgs < resident ? wgs : resident)), dim3(NWAVES * 64), 0, stream, p, queues.counters,
                          int(wgs / kNumXcd));
       return check_launch("fna_forward (work queue)");
@@ -108,7 +108,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   }
   if (p.kv_splits > 1) {
     // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
-    if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64) {
+    if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64 && !CTX) {
       if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
       FnaParams ps = p;
       ps.split_grid = int(wgs);
@@ -119,7 +119,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
       return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
     }
   }
-  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
+  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
                      stream, p);
   return check_launch("fna_forward");
 }
@@ -185,8 +185,20 @@ bool needs_clamped_rows(const FnaParams& p, int kvt) {
   return p.cu_q != nullptr || p.edge == 2 || (p.seqlen_kv % kvt != 0 && p.edge != 1);
 }
 
+// Launches whose queries also attend to a context: masked instances.
+bool context_launch_fits(const FnaParams& p, int kvt) { return kvt == 64 && !needs_clamped_rows(p, kvt); }
+
 template <typename T, int D>
 int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, WorkQueue queues) {
+  if (p.has_context()) {
+    if (context_launch_fits(p, kvt)) {
+      if (qt == 128) return launch_fna<T, D, 4, 1, false, 64, false, 0, true>(p, stream, queues);
+      if constexpr (D <= 64) {
+        if (qt == 64 && queues.counters == nullptr) return launch_fna<T, D, 2, 1, false, 64, false, 0, true>(p, stream);
+      }
+    }
+    return fail("fna_forward: no kernel with a context for these tiles and extents (Q tile %d, KV tile %d, head_dim %d)", qt, kvt, D);
+  }
   if (needs_clamped_rows(p, kvt)) {
     if (qt == 128 && kvt == 64) return launch_fna<T, D, 4, 1, true, 64>(p, stream);
     return fail("fna_forward: seqlen_kv (%d) must be a multiple of the KV tile (%d tokens)", p.seqlen_kv, kvt);
@@ -203,11 +215,11 @@ int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, Work
 
 // Head dims between the native ones (multiples of 8 above 32).  Up to 96 of 128 columns are multiplied as
 // 96: a quarter of the matrix work and of the LDS reads less.
-template <typename T, bool RAGGED>
+template <typename T, bool RAGGED, bool CTX = false>
 int dispatch_narrow_rows(const FnaParams& p, int head_dim, hipStream_t stream) {
-  if (head_dim < 64) return launch_fna<T, 64, 4, 1, RAGGED, 64, false, 64>(p, stream);
-  if (head_dim <= 96) return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 96>(p, stream);
-  return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 128>(p, stream);
+  if (head_dim < 64) return launch_fna<T, 64, 4, 1, RAGGED, 64, false, 64, CTX>(p, stream);
+  if (head_dim <= 96) return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 96, CTX>(p, stream);
+  return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 128, CTX>(p, stream);
 }
 
 template <typename T>
@@ -220,6 +232,10 @@ int dispatch_head_dim(const FnaParams& p, int head_dim, int qt, int kvt, hipStre
   if (!narrow_rows(head_dim)) return fail("fna_forward: head_dim must be 32, 64 or 128, got %d", head_dim);
   if (qt != 128 || kvt != 64 || queues.counters != nullptr || p.cu_q != nullptr || p.row_dim != head_dim)
     return fail("fna_forward: head_dim %d needs tiles of 128 x 64 tokens and no work queue", head_dim);
+  if (p.has_context()) {
+    if (!context_launch_fits(p, kvt)) return fail("fna_forward: no kernel with a context for these extents (head_dim %d)", head_dim);
+    return dispatch_narrow_rows<T, false, true>(p, head_dim, stream);
+  }
   if (needs_clamped_rows(p, kvt)) return dispatch_narrow_rows<T, true>(p, head_dim, stream);
   return dispatch_narrow_rows<T, false>(p, head_dim, stream);
 }
@@ -566,7 +582,8 @@ int fna_forward_fused_impl(const void* q, const void* k, const void* v, void* ou
                            const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
                            const int32_t* is_causal, const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
                            float scale, const float* q_scale, const float* k_scale, const float* v_scale,
-                           int anchor_kv_tiles, WorkQueue queues, void* stream, int kv_splits = 1) {
+                           int anchor_kv_tiles, WorkQueue queues, void* stream, int kv_splits = 1,
+                           const void* ctx_k = nullptr, const void* ctx_v = nullptr, int ctx_len = 0) {
   FnaParams p;
   long long tokens = 0;
   if (heads_kv < 1 || head_dim < 1) return fail("fna_forward_fused: head counts and head_dim must be positive");
@@ -590,6 +607,11 @@ int fna_forward_fused_impl(const void* q, const void* k, const void* v, void* ou
   p.q_scale = q_scale;
   p.k_scale = k_scale;
   p.v_scale = v_scale;
+  if (ctx_len > 0) {
+    p.ctx_k = ctx_k;
+    p.ctx_v = ctx_v;
+    p.ctx_len = ctx_len;
+  }
   if (kv_splits > 1) {
     // out and lse hold kv_splits results of the full shape, one after the other
     p.kv_splits = kv_splits;
@@ -726,6 +748,29 @@ int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void*
   return fna_forward_fused_impl(q, k, v, out_parts, lse_parts, dtype, na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape,
                                 kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape, scale, nullptr,
                                 nullptr, nullptr, anchor_kv_tiles, WorkQueue{}, stream, kv_splits);
+}
+
+int natten_amd_fna_forward_fused_context(const void* q, const void* k, const void* v, const void* context_k,
+                                         const void* context_v, void* out, float* lse, int dtype, int na_dim, int batch,
+                                         int context_len, int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
+                                         const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
+                                         const int32_t* is_causal, const int32_t* q_tile_shape,
+                                         const int32_t* kv_tile_shape, float scale, int run_persistent, void* workspace,
+                                         uint64_t workspace_bytes, void* stream) {
+  g_error[0] = 0;
+  const char* what = "fna_forward_fused_context";
+  if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
+  WorkQueue queues;
+  if (int rc = queue_workspace(what, run_persistent, workspace, workspace_bytes, &queues)) return rc;
+  if (!context_k || !context_v) return fail("%s: null pointer argument", what);
+  if ((reinterpret_cast<uintptr_t>(context_k) | reinterpret_cast<uintptr_t>(context_v)) & 15)
+    return fail("%s: context_k and context_v must be 16-byte aligned", what);
+  if (context_len < 64) return fail("%s: the context must hold at least a KV tile (64 keys), got %d", what, context_len);
+  if (dtype != NATTEN_AMD_F16 && dtype != NATTEN_AMD_BF16)
+    return fail("%s: fp16 / bf16 operands expected, got dtype code %d", what, dtype);
+  return fna_forward_fused_impl(q, k, v, out, lse, dtype, na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape,
+                                kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape, scale, nullptr,
+                                nullptr, nullptr, /*anchor_kv_tiles=*/1, queues, stream, 1, context_k, context_v, context_len);
 }
 
 namespace {

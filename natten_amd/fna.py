@@ -20,6 +20,7 @@ from .tile_config import (
     TILE_SIZES,
     check_fna_backward_config,
     check_fna_forward_config,
+    choose_fitting_forward_tiles,
     choose_small_forward_tiles,
     choose_tile_shapes,
     padded_head_dim,
@@ -129,6 +130,46 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
                                        q_tile_shape=tiles[0], dtype=dtype):
         return None
     return (*tiles, persistent, splits)
+
+
+@functools.lru_cache(maxsize=1024)
+def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
+    """Tile shapes and kind of the launch over windows and context, or None.  Where the windows alone would be a split launch it is
+    taken for up to 48 KV tiles a Q tile: a split launch, dense attention and two merges take the host 68 us and the device
+    17 beside the split walk, the whole walk in one launch 1.05 us a tile (head dim 128; 2 x 30 x 40, 21 x 21, H 4 and 128
+    context tokens: 68 us so, 23 in one launch)."""
+    plan = _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel)
+    if plan is None:
+        return None
+    layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2], plan[3]
+    if any(x // d < t for x, d, t in zip(layout, dilation, tiles[1])):
+        tiles = choose_fitting_forward_tiles(layout, kernel_size, stride, dilation, is_causal)
+        if tiles is None:
+            return None
+    if splits > 1:
+        from .functional import _kv_tiles_per_q_tile
+
+        if _kv_tiles_per_q_tile(layout, kernel_size, stride, dilation, *tiles) > 48:
+            return None
+    return (*tiles, persistent)
+
+
+def amd_fna_with_context(query: Tensor, key: Tensor, value: Tensor, context_key: Tensor, context_value: Tensor, kernel_size,
+                         stride, dilation, is_causal, scale: float, run_persistent_kernel: Optional[bool] = None):
+    """Neighborhood attention whose queries also attend to context_key / context_value [B, N, Hkv, D] in one launch,
+    forward only, on checked arguments that leave tiles and route open: (output, lse), or None where
+    there is no such launch (contexts shorter than a KV tile, long split walks, dilation groups narrower than any KV
+    tile): the callers then merge two attentions."""
+    if context_key.shape[1] < 64 or query.dtype not in (torch.float16, torch.bfloat16) or torch_ops._tracing():
+        return None
+    plan = _context_call_plan(query.dtype, tuple(query.shape), key.shape[-2], kernel_size, stride, dilation, is_causal,
+                              run_persistent_kernel)
+    if plan is None:
+        return None
+    can_run_amd_fna(query, key, value, raise_error=True)
+    return _lib.fna_forward_fused_context(
+        query.contiguous(), key.contiguous(), value.contiguous(), context_key.contiguous(), context_value.contiguous(),
+        kernel_size, stride, dilation, is_causal, scale, *plan)
 
 
 def amd_fna_generic(

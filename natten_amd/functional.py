@@ -25,7 +25,7 @@ from .checks import (
     na_tensor_checks,
 )
 from .fmha import amd_fmha
-from .fna import amd_fna_generic, is_fp8
+from .fna import amd_fna_generic, amd_fna_with_context, is_fp8
 from .utils.varlen import varlen_tensor_checks
 
 _BACKEND_FNA = "amd-fna"
@@ -165,6 +165,14 @@ def neighborhood_attention_generic(
     needs_grad = torch.is_grad_enabled() and any(
         t is not None and t.requires_grad for t in (query, key, value, additional_keys, additional_values)
     )
+    if (has_additional_attention and not needs_grad and not attn_kwargs and q_tile_shape is None and kv_tile_shape is None
+            and q_scale is None and k_scale is None and v_scale is None):
+        # one launch over the window and the context, where there is one
+        joint = amd_fna_with_context(query, key, value, additional_keys, additional_values, kernel_size, stride, dilation,
+                                     is_causal, scale, run_persistent_kernel)
+        if joint is not None:
+            output = joint[0].to(final_dtype)
+            return (output, joint[1]) if return_lse else output
     if is_fp8(query.dtype):
         work_dtype = torch.bfloat16
     else:

@@ -131,6 +131,19 @@ def _choose_tile_shapes(
     return best
 
 
+def choose_fitting_forward_tiles(
+    token_layout: DimensionType, kernel_size: DimensionType, stride: DimensionType, dilation: DimensionType,
+    is_causal: Tuple[bool, ...],
+) -> Optional[Tuple[DimensionType, DimensionType]]:
+    """Shapes of the default tile pair that visit the fewest pairs among those whose KV tile no dilation group is narrower
+    than; None where there are none."""
+    n = len(token_layout)
+    problem = (token_layout, kernel_size, stride, dilation, is_causal)
+    fitting = [kt for kt in _factorisations(TILE_SIZES[0][1], n) if all(x // d >= t for x, d, t in zip(token_layout, dilation, kt))]
+    pairs = [(visited_pairs(*problem, qt, kt), (qt, kt)) for qt in _factorisations(TILE_SIZES[0][0], n) for kt in fitting]
+    return min(pairs)[1] if pairs else None
+
+
 @torch.compiler.assume_constant_result
 def choose_small_forward_tiles(
     token_layout: DimensionType, kernel_size: DimensionType, stride: DimensionType, dilation: DimensionType,
