@@ -302,6 +302,27 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
                                  const float* v_scale, void* stream);
 
 /*
+ * What natten_amd_attention_forward_split is to be given for a problem on the current device, where it was
+ * measured to be faster than natten_amd_attention_forward; *kv_splits = 1 elsewhere.
+ */
+int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int heads_q, int head_dim,
+                                    int is_causal, int32_t* split_positions, int32_t* kv_splits);
+
+/*
+ * natten_amd_attention_forward with the KV tiles of the Q tiles of the last `split_positions` launch positions
+ * (a multiple of 8; a grid position per Q tile of 128 queries and head, rounded up over the 8 XCDs) dealt to
+ * kv_splits (2 .. 16) workgroups each, and their float results merged in a second launch: for the last,
+ * nearly empty round of workgroups, and for problems of few Q tiles.  parts: a 16-byte aligned workspace of
+ * split_positions * kv_splits * 128 * (head_dim + 1) floats, not read before it is written.  At least 64 keys.
+ */
+int natten_amd_attention_forward_split(const void* q, const void* k, const void* v, void* out, float* lse,
+                                       float* parts, uint64_t parts_floats, int split_positions,
+                                       int kv_splits, int dtype, int batch, int seqlen_q, int seqlen_kv,
+                                       int heads_q, int heads_kv, int head_dim, int is_causal, float scale,
+                                       const float* q_scale, const float* k_scale, const float* v_scale,
+                                       void* stream);
+
+/*
  * Dense attention forward on sequence-packed operands (variable-length batches).
  *   q / out [total_seqlen_q, heads_q, head_dim], k / v [total_seqlen_kv, heads_kv, head_dim],
  *   lse [total_seqlen_q, heads_q] float32.  Sequence b (0 <= b < num_seqs) owns query rows

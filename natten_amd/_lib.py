@@ -89,6 +89,11 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 7 + [ctypes.c_int] * 7 + [ctypes.c_void_p] * 7
         + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_void_p],
     ),
+    "natten_amd_attention_split_plan": (ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_void_p] * 2),
+    "natten_amd_attention_forward_split": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 6 + [ctypes.c_uint64] + [ctypes.c_int] * 10 + [ctypes.c_float] + [ctypes.c_void_p] * 4,
+    ),
     "natten_amd_query_range": (ctypes.c_int, [ctypes.c_int] * 7 + [ctypes.c_void_p] * 2),
     "natten_amd_key_tile_shift": (ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.c_void_p]),
     "natten_amd_compute_delta": (
@@ -501,6 +506,16 @@ def fna_forward_fused_static(
     _check(rc)
 
 
+@functools.lru_cache(maxsize=1024)
+def attention_split_plan(device_index: int, batch: int, seqlen_q: int, seqlen_kv: int, heads: int, head_dim: int,
+                         is_causal: bool) -> Tuple[int, int]:
+    """(launch positions whose Q tiles are split, workgroups each): (0, 1) where dense attention is one launch."""
+    positions, splits = ctypes.c_int32(), ctypes.c_int32()
+    _check(lib().natten_amd_attention_split_plan(batch, seqlen_q, seqlen_kv, heads, head_dim, 1 if is_causal else 0,
+                                                 ctypes.byref(positions), ctypes.byref(splits)))
+    return positions.value, splits.value
+
+
 def attention_forward(
     q: Tensor, k: Tensor, v: Tensor, is_causal: bool, scale: float,
     q_scale: Optional[Tensor] = None, k_scale: Optional[Tensor] = None, v_scale: Optional[Tensor] = None,
@@ -515,6 +530,15 @@ def attention_forward(
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     with _on_device(q):
+        positions, splits = attention_split_plan(q.device.index, q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3], bool(is_causal))
+        if splits > 1:
+            parts = torch.empty(positions * splits * 128 * (q.shape[3] + 1), dtype=torch.float32, device=q.device)
+            _check(L.natten_amd_attention_forward_split(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), parts.data_ptr(), parts.numel(), positions,
+                splits, DTYPE_CODES[q.dtype], q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3],
+                1 if is_causal else 0, float(scale), *scales, _stream(q),
+            ))
+            return out, lse
         rc = L.natten_amd_attention_forward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), DTYPE_CODES[q.dtype],
             q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,

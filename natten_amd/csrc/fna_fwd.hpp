@@ -97,23 +97,28 @@ struct FnaParams {
   int ext_base[3], ext_rem[3];  // qkv_shape / dil and qkv_shape % dil: extent of dilation group g = base + (g < rem)
   NaDiv d_stride[3], d_dil[3], d_q_tiled[3];
   NaDiv d_wg_group, d_groups_per_bh, d_heads_q, d_q_per_kv, d_num_groups;
-  // Split launches only (fna_fwd_split_kernel; 0 otherwise): the KV tiles of every Q tile are dealt
-  // to `kv_splits` workgroups in contiguous runs; workgroup `pid` of the grid works on Q-tile
-  // position pid % split_grid for split pid / split_grid and stores its partial result (normalised
-  // over its own keys, with their LSE) `split` strides into o and lse.
+  // Split launches only (fna_fwd_split_kernel; 0 otherwise): the KV tiles of a Q tile are dealt to
+  // `kv_splits` workgroups in contiguous runs, each of which stores a partial result (normalised over its own
+  // keys, with their LSE).  Neighborhood attention splits every Q tile: workgroup `pid` of the grid works on
+  // position pid % split_grid for split pid / split_grid and stores `split` strides into o and lse, in the output
+  // type (split_first < 0).  Dense attention splits the positions from split_first on: the workgroups before
+  // take a Q tile each, as in any launch, the others store float rows [position - split_first][split][128][row] and
+  // their LSE, which merge_tail_kernel combines.
   // CTX instances only (no splits): ctx_len >= 64 more keys and values per batch entry, [batch, ctx_len, heads_kv, row],
-  // that every query attends to besides its window.  (In one place: the block stays under 512 bytes, which a launch copies.)
-  int kv_splits;
+  // that every query attends to besides its window.  (In one place: a block of more than 512 bytes takes a launch 0.3 us.)
+  int kv_splits, split_first;
   union {
     int split_grid;
     int ctx_len;
   };
   union {
     int64_t o_split_stride;  // elements of the output type
+    float* split_parts;
     const void* ctx_k;
   };
   union {
     int64_t lse_split_stride;  // floats
+    float* split_lse;
     const void* ctx_v;
   };
   __host__ bool has_context() const { return kv_splits <= 1 && ctx_len > 0; }
@@ -456,8 +461,14 @@ template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLI
           bool CTX = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
-  const int split = SPLIT ? pid_in / p.split_grid : 0;
-  const int pid = SPLIT ? pid_in - split * p.split_grid : pid_in;
+  int split = 0, splits = 1, pid = pid_in;
+  if constexpr (SPLIT) {
+    if (pid_in >= p.split_first) {
+      splits = p.kv_splits;
+      split = (pid_in - na_max(p.split_first, 0)) / p.split_grid;
+      pid = pid_in - split * p.split_grid;
+    }
+  }
   constexpr int NT = NWAVES * 64;
   constexpr int QT = NWAVES * MQ * 32;
   constexpr bool NARROW = DC != 0;
@@ -654,8 +665,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   int first_tile = 0, total_tiles = box_tiles + (ctx_len + KVT - 1) / KVT;
   bool empty_split = false;
   if constexpr (SPLIT) {
-    first_tile = int(int64_t(split) * box_tiles / p.kv_splits);
-    total_tiles = int(int64_t(split + 1) * box_tiles / p.kv_splits) - first_tile;
+    first_tile = int(int64_t(split) * box_tiles / splits);
+    total_tiles = int(int64_t(split + 1) * box_tiles / splits) - first_tile;
     if (total_tiles == 0) {
       empty_split = true;
       first_tile = 0;
@@ -1407,8 +1418,26 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   T* obase = reinterpret_cast<T*>(p.o) + q_row_base * q_row_stride + int64_t(head) * row_dim;
   float* lse_base = p.lse;
   if constexpr (SPLIT) {
-    obase += split * p.o_split_stride;
-    lse_base += split * p.lse_split_stride;
+    if (p.split_first < 0) {
+      obase += split * p.o_split_stride;
+      lse_base += split * p.lse_split_stride;
+    } else if (splits > 1) {
+      const int64_t row = (int64_t(pid - p.split_first) * splits + split) * QT + wave * 32 + l32;
+      const float l = empty_split ? 0.f : l_run[0] + __shfl_xor(l_run[0], 32);
+      const float inv = (l > 0.f) ? out_scale / l : 0.f;
+      float* part = p.split_parts + row * row_dim + 4 * g;
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          f32x4_t o4;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o4[i] = acc[0][db][4 * j + i] * inv;
+          if (!NARROW || db * 32 + 8 * j < row_dim) *reinterpret_cast<f32x4_t*>(part + db * 32 + 8 * j) = o4;
+        }
+      if (g == 0) p.split_lse[row] = (l > 0.f) ? (m_run[0] * 0.6931471805599453f + __logf(l)) : -INFINITY;
+      return;
+    }
   }
 #pragma unroll
   for (int mb = 0; mb < MQ; ++mb) {
@@ -1451,6 +1480,56 @@ __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_e
 fna_fwd_split_kernel(const FnaParams p) {
   touch_launch_params<sizeof(FnaParams)>();
   fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
+}
+
+// Combines the partial results of a dense split launch, sixteen rows of a Q tile per workgroup, four columns per lane:
+// out = sum_i w_i part_i with w_i = exp(lse_i - lse), in float, rounded once.  Bound by the trips to memory
+// (the parts come from other XCDs' workgroups), so that loads of several parts are in flight.
+template <typename T>
+__global__ void __launch_bounds__(256) merge_tail_kernel(const FnaParams p) {
+  constexpr int QT = 128, ROWS = 16;
+  const int pos = p.split_first + int(blockIdx.x) / (QT / ROWS), row0 = int(blockIdx.x) % (QT / ROWS) * ROWS;
+  // (position -> Q tile as in fna_fwd_tile; one dimension)
+  const int local = pos / kNumXcd, run = na_div(local, p.d_wg_group);
+  const int group = run * kNumXcd + pos % kNumXcd;
+  if (group >= p.total_groups) return;
+  const int bh = na_div(group, p.d_groups_per_bh);
+  int tile = (group - bh * p.groups_per_bh) * p.wg_group + local - run * p.wg_group;
+  if (tile >= p.num_q_tiles) return;
+  if (p.causal[0]) tile = p.q_tiled[0] - 1 - tile;
+  const int b = na_div(bh, p.d_heads_q), head = bh - b * p.heads_q;
+  const int slices = p.row_dim / 4;
+  const int64_t part0 = int64_t(pos - p.split_first) * p.kv_splits * QT + row0;
+  for (int i = threadIdx.x; i < ROWS * slices; i += 256) {
+    const int r = i / slices, c = (i - r * slices) * 4;
+    const int q_row = tile * QT + row0 + r;
+    if (q_row >= p.seqlen_q) continue;
+    const float* lses = p.split_lse + part0 + r;
+    const float* part = p.split_parts + (part0 + r) * p.row_dim + c;
+    const int64_t part_stride = int64_t(QT) * p.row_dim;
+    float mx = -INFINITY;
+#pragma unroll 8
+    for (int s = 0; s < p.kv_splits; ++s) mx = fmaxf(mx, lses[s * QT]);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    float sum = 0.f;
+    const float ref = mx == -INFINITY ? 0.f : mx;  // (no keys at all: every weight is 0)
+#pragma unroll 8
+    for (int s = 0; s < p.kv_splits; ++s) {
+      const f32x4_t x = *reinterpret_cast<const f32x4_t*>(part + s * part_stride);
+      const float w = __expf(lses[s * QT] - ref);
+      sum += w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] += w * x[e];
+    }
+    const float inv = sum > 0.f ? 1.f / sum : 0.f;
+    typedef T tx4 __attribute__((ext_vector_type(4)));
+    tx4 out;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) out[e] = static_cast<T>(acc[e] * inv);
+    const int64_t row = (int64_t(b) * p.seqlen_q + q_row) * p.heads_q + head;
+    *reinterpret_cast<tx4*>(reinterpret_cast<T*>(p.o) + row * p.row_dim + c) = out;
+    if (c == 0) p.lse[row] = sum > 0.f ? mx + __logf(sum) : -INFINITY;
+  }
 }
 
 // Work-queue launch: as many workgroups as the chip keeps resident, each taking Q tiles until

@@ -111,10 +111,21 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
     if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64 && !CTX) {
       if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
       FnaParams ps = p;
-      ps.split_grid = int(wgs);
-      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>), dim3((unsigned)(wgs * p.kv_splits)),
-                         dim3(NWAVES * 64), 0, stream, ps);
-      return check_launch("fna_forward (split)");
+      if (p.split_first < 0) {
+        ps.split_grid = int(wgs);
+        hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>), dim3((unsigned)(wgs * p.kv_splits)),
+                           dim3(NWAVES * 64), 0, stream, ps);
+        return check_launch("fna_forward (split)");
+      }
+      // the last split_grid positions (a multiple of 8: positions keep their XCDs)
+      if (p.split_grid < kNumXcd || p.split_grid % kNumXcd != 0 || p.split_grid > wgs)
+        return fail("fna_forward: the split positions must be a multiple of %d up to %lld, got %d", kNumXcd, wgs, p.split_grid);
+      ps.split_first = int(wgs) - p.split_grid;
+      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>),
+                         dim3((unsigned)(ps.split_first + p.split_grid * p.kv_splits)), dim3(NWAVES * 64), 0, stream, ps);
+      if (int rc = check_launch("fna_forward (split)")) return rc;
+      hipLaunchKernelGGL((merge_tail_kernel<T>), dim3((unsigned)p.split_grid * 8), dim3(256), 0, stream, ps);
+      return check_launch("fna_forward (merge)");
     } else {
       return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
     }
@@ -615,6 +626,7 @@ int fna_forward_fused_impl(const void* q, const void* k, const void* v, void* ou
   if (kv_splits > 1) {
     // out and lse hold kv_splits results of the full shape, one after the other
     p.kv_splits = kv_splits;
+    p.split_first = -1;
     p.o_split_stride = (int64_t)batch * tokens * heads_q * head_dim;
     p.lse_split_stride = (int64_t)batch * tokens * heads_q;
   }
@@ -838,10 +850,10 @@ int natten_amd_fna_forward_fused_static(const void* q, const void* k, const void
                                 k_scale, v_scale, /*anchor_kv_tiles=*/1, queues, stream);
 }
 
-int natten_amd_attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
-                                 int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
-                                 int is_causal, float scale, const float* q_scale, const float* k_scale,
-                                 const float* v_scale, void* stream) {
+static int attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int batch,
+                             int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim, int is_causal, float scale,
+                             const float* q_scale, const float* k_scale, const float* v_scale, void* stream, int split_positions,
+                             int kv_splits, float* parts, float* lse_parts) {
   g_error[0] = 0;
   if (int rc = check_common("attention_forward", q, k, v, out, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv,
                             head_dim, dtype == NATTEN_AMD_F16 || dtype == NATTEN_AMD_BF16))
@@ -884,8 +896,100 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
   p.q_scale = q_scale;
   p.k_scale = k_scale;
   p.v_scale = v_scale;
+  if (kv_splits > 1) {
+    p.kv_splits = kv_splits;
+    p.split_grid = split_positions;
+    p.split_parts = parts;
+    p.split_lse = lse_parts;
+  }
   set_wg_layout(p, 1);
   return dispatch_dtype(p, dtype, head_dim, QT, KVT, static_cast<hipStream_t>(stream));
+}
+
+int natten_amd_attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                                 int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                 int is_causal, float scale, const float* q_scale, const float* k_scale,
+                                 const float* v_scale, void* stream) {
+  return attention_forward(q, k, v, out, lse, dtype, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim, is_causal, scale,
+                           q_scale, k_scale, v_scale, stream, 0, 1, nullptr, nullptr);
+}
+
+int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int heads_q, int head_dim, int is_causal,
+                                    int32_t* split_positions, int32_t* kv_splits) {
+  g_error[0] = 0;
+  const char* what = "attention_split_plan";
+  if (!split_positions || !kv_splits) return fail("%s: null pointer argument", what);
+  if (batch < 1 || seqlen_q < 1 || seqlen_kv < 1 || heads_q < 1 || head_dim < 1)
+    return fail("%s: batch, sequence lengths, heads and head_dim must be positive", what);
+  *split_positions = 0;
+  *kv_splits = 1;
+  const int kv_tiles = na_ceil_div(seqlen_kv, 64);
+  const long long q_tiles = na_ceil_div(seqlen_q, 128), n = q_tiles * heads_q * batch;
+  // The chip takes `slots` workgroups at a time.  What does not fill a last round is split so that it does, where
+  // that saves a twelfth of the whole and more than the merge takes (2 x 4097 tokens, H 16, D 64, a third round of 32 Q
+  // tiles: 185 us, 170 with them split 13 ways; 2 x 9000, H 4, D 64: 232 and 187; 2 x 5000, H 8, D 128: 211 and 199).  In KV tiles of a workgroup that shares its
+  // compute unit (0.62 us at head dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch
+  // and the parts' way through memory eight.  The second launch and the workspace also take the host 5 us: launches under
+  // 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.  Causal: rounds even out by themselves (the longest walks
+  // start first), and only a single round is split.  One batch entry is never split: a packed call promises the
+  // bits of a dense call on each of its sequences alone.
+  const int slots = resident_workgroups(head_dim <= 32 ? 3 : 2), cus = resident_workgroups(1);
+  const long long full = n / slots, rem = n % slots;
+  if (batch < 2 || kv_tiles < 16 || rem == 0 || full > 12 || (is_causal && full > 0)) return 0;
+  const double round = rem <= cus ? 0.75 * kv_tiles : kv_tiles;
+  double least = 1e30;
+  int best = 1;
+  for (int s = 2; s <= 16 && rem * s <= slots && kv_tiles / s >= 3; ++s) {
+    const double t = (rem * s <= cus ? 0.75 : 1.0) * na_ceil_div(kv_tiles, s) + 8;
+    if (t < least) {
+      least = t;
+      best = s;
+    }
+  }
+  if (best == 1 || full * kv_tiles + round < 40 || least > round - (full * kv_tiles + round) / 12) return 0;
+  // the launch positions that hold the last `rem` Q tiles
+  FnaParams p;
+  memset(&p, 0, sizeof(p));
+  p.batch = batch;
+  p.heads_q = p.heads_kv = heads_q;
+  for (int a = 0; a < 3; ++a) p.qkv_shape[a] = p.ksize[a] = p.stride[a] = p.dil[a] = p.q_tile[a] = p.kv_tile[a] = p.q_tiled[a] = p.kv_tiled[a] = 1;
+  p.q_tile[0] = 128;
+  p.kv_tile[0] = 64;
+  p.q_tiled[0] = int(q_tiles);
+  p.num_groups = 1;
+  set_wg_layout(p, 1);
+  const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
+  long long first = wgs;
+  for (long long left = rem; first > 0 && left > 0;) {
+    --first;
+    const int local = int(first / kNumXcd), run = local / p.wg_group, group = run * kNumXcd + int(first % kNumXcd);
+    if (group < p.total_groups && group % p.groups_per_bh * p.wg_group + local - run * p.wg_group < p.num_q_tiles) --left;
+  }
+  first = first / kNumXcd * kNumXcd;
+  *split_positions = int(wgs - first);
+  *kv_splits = best;
+  return 0;
+}
+
+int natten_amd_attention_forward_split(const void* q, const void* k, const void* v, void* out, float* lse, float* parts,
+                                       uint64_t parts_floats, int split_positions, int kv_splits, int dtype, int batch,
+                                       int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim, int is_causal,
+                                       float scale, const float* q_scale, const float* k_scale, const float* v_scale,
+                                       void* stream) {
+  g_error[0] = 0;
+  const char* what = "attention_forward_split";
+  if (!parts || (reinterpret_cast<uintptr_t>(parts) & 15)) return fail("%s: parts must be a 16-byte aligned workspace", what);
+  if (kv_splits < 2 || kv_splits > 16) return fail("%s: kv_splits must be 2 .. 16, got %d", what, kv_splits);
+  if (split_positions < kNumXcd || split_positions % kNumXcd != 0)
+    return fail("%s: split_positions must be a multiple of %d, got %d", what, kNumXcd, split_positions);
+  if (seqlen_kv < 64) return fail("%s: at least 64 keys expected, got %d", what, seqlen_kv);
+  if (dtype != NATTEN_AMD_F16 && dtype != NATTEN_AMD_BF16) return fail("%s: fp16 / bf16 operands expected, got dtype code %d", what, dtype);
+  const uint64_t rows = uint64_t(split_positions) * uint64_t(kv_splits) * 128;
+  if (head_dim < 1 || parts_floats < rows * (uint64_t(head_dim) + 1))
+    return fail("%s: parts must hold split_positions * kv_splits * 128 rows of head_dim + 1 floats, got %llu floats", what,
+                (unsigned long long)parts_floats);
+  return attention_forward(q, k, v, out, lse, dtype, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim, is_causal, scale,
+                           q_scale, k_scale, v_scale, stream, split_positions, kv_splits, parts, parts + rows * uint64_t(head_dim));
 }
 
 int natten_amd_attention_forward_varlen(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,

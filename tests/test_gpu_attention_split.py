@@ -1,0 +1,83 @@
+"""Dense attention whose last round of workgroups, or only one, is split over the keys: query and key counts around tiles, all
+head dims, GQA, causal; against the CPU oracle and the unsplit launch.  What the plan splits (CPU)."""
+
+import numpy as np
+import pytest
+import torch
+
+import natten_amd
+from natten_amd import _lib
+from oracle import na_oracle as O
+from tests.gpu_utils import assert_close, to_np
+
+
+def rand(shape, dtype, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+
+
+def test_plan():
+    plan = lambda *a: _lib.attention_split_plan(0, *a)
+    assert plan(2, 1000, 4000, 4, 128, False)[1] > 1          # 64 Q tiles on the whole chip
+    assert plan(2, 1000, 1000, 4, 128, False) == (0, 1)        # over before a second launch is made
+    assert plan(1, 1000, 4000, 8, 128, False) == (0, 1)        # one sequence: the bits of a packed call
+    assert plan(2, 4096, 4096, 16, 64, False) == (0, 1)        # whole rounds
+    assert plan(2, 8200, 512, 16, 64, False) == (0, 1)         # too few keys
+    assert plan(2, 9000, 9000, 24, 64, True) == (0, 1)         # causal: rounds even out
+    positions, splits = plan(2, 4097, 4097, 16, 64, False)     # a third round of 32 Q tiles
+    assert positions % 8 == 0 and 32 <= positions < 64 and 2 <= splits <= 16
+    for args in ((2, 1000, 4000, 4, 128, False), (3, 1700, 5000, 5, 64, False), (2, 3600, 3600, 2, 96, True)):
+        positions, splits = plan(*args)
+        tiles = -(-args[1] // 128) * args[0] * args[3]
+        assert splits > 1 and positions >= tiles % 512 and tiles % 512 * splits <= 512
+
+
+CASES = [
+    # B, Sq, Skv, H, Hkv, D, causal
+    (2, 300, 3500, 2, 1, 128, False),
+    (2, 3600, 3600, 2, 2, 64, True),
+    (3, 129, 3500, 5, 1, 32, False),
+    (2, 70, 3470, 6, 3, 96, False),
+    (2, 1500, 3537, 3, 3, 40, True),
+    (2, 8321, 2600, 4, 2, 64, False),       # a whole round, then 16 Q tiles more
+]
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_the_cases_below_are_split(case):
+    B, Sq, Skv, H, Hkv, D, causal = case
+    assert _lib.attention_split_plan(0, B, Sq, Skv, H, D, causal)[1] > 1
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES)
+def test_matches_oracle(case, dtype):
+    B, Sq, Skv, H, Hkv, D, causal = case
+    q, k, v = rand((B, Sq, H, D), dtype, 1), rand((B, Skv, Hkv, D), dtype, 2), rand((B, Skv, Hkv, D), dtype, 3)
+    assert _lib.attention_split_plan(q.device.index, B, Sq, Skv, H, D, causal)[1] > 1
+    with torch.no_grad():
+        out, lse = natten_amd.attention(q, k, v, is_causal=causal, return_lse=True)
+    ref_o, ref_l = O.attention_forward(to_np(q), to_np(k), to_np(v), is_causal=causal)
+    assert_close("out", to_np(out), ref_o)
+    assert_close("lse", to_np(lse), ref_l)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 64, 96, 128])
+@pytest.mark.parametrize("positions,splits", [(8, 2), (16, 16), (48, 5)])
+def test_any_number_of_positions(positions, splits, D):
+    # 48 positions of which 45 hold a Q tile; rows of the others are never written and never read
+    q, k, v = rand((3, 600, 3, D), torch.bfloat16, 1), rand((3, 200, 3, D), torch.bfloat16, 2), rand((3, 200, 3, D), torch.bfloat16, 3)
+    out, lse = torch.full_like(q, float("nan")), torch.full(q.shape[:-1], float("nan"), device="cuda")
+    parts = torch.full((positions * splits * 128 * (D + 1),), float("nan"), device="cuda")
+    L = _lib.lib()
+    args = lambda p, n, pos: (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), p.data_ptr(), n, pos, splits,
+                              _lib.DTYPE_CODES[q.dtype], 3, 600, 200, 3, 3, D, 1, D**-0.5, None, None, None,
+                              torch.cuda.current_stream().cuda_stream)
+    assert L.natten_amd_attention_forward_split(*args(parts, parts.numel(), positions)) == 0, L.natten_amd_last_error()
+    ref_o, ref_l = O.attention_forward(to_np(q), to_np(k), to_np(v), is_causal=True)
+    assert_close("out", to_np(out), ref_o)
+    assert_close("lse", to_np(lse), ref_l)
+    for p, n, pos in ((parts, parts.numel() - 1, positions), (parts[1:], parts.numel(), positions), (parts, 1 << 40, positions + 1),
+                      (parts, 1 << 40, 512)):
+        assert L.natten_amd_attention_forward_split(*args(p, n, pos)) != 0
