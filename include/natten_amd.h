@@ -330,7 +330,8 @@ int natten_amd_attention_forward_split(const void* q, const void* k, const void*
  *   arrays of num_seqs + 1 entries live in device memory.  max_seqlen_* bound the sequence
  *   lengths (the launch is sized from them; rows of a longer sequence would not be computed).
  *   The causal mask is top-left aligned per sequence.  A sequence without keys gets
- *   out = 0 and lse = -inf.  Rows that belong to no sequence are not written.
+ *   out = 0 and lse = -inf.  Rows that belong to no sequence are not written; ..._all_rows
+ *   sets them to zeros (out and lse).
  *   16-bit float operands only.
  */
 int natten_amd_attention_forward_varlen(const void* q, const void* k, const void* v, void* out,
@@ -341,6 +342,14 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
                                         const int32_t* cumulative_seqlen_kv, int is_causal,
                                         float scale, const float* q_scale, const float* k_scale,
                                         const float* v_scale, void* stream);
+int natten_amd_attention_forward_varlen_all_rows(const void* q, const void* k, const void* v, void* out,
+                                                 float* lse, int dtype, int num_seqs, int total_seqlen_q,
+                                                 int total_seqlen_kv, int max_seqlen_q, int max_seqlen_kv,
+                                                 int heads_q, int heads_kv, int head_dim,
+                                                 const int32_t* cumulative_seqlen_q,
+                                                 const int32_t* cumulative_seqlen_kv, int is_causal,
+                                                 float scale, const float* q_scale, const float* k_scale,
+                                                 const float* v_scale, void* stream);
 
 /*
  * Host-only helper (no GPU work): the interval of query coordinates 0 .. num_queries-1 whose

@@ -84,6 +84,11 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 5 + [ctypes.c_int] * 9 + [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_float]
         + [ctypes.c_void_p] * 4,
     ),
+    "natten_amd_attention_forward_varlen_all_rows": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 5 + [ctypes.c_int] * 9 + [ctypes.c_void_p] * 2 + [ctypes.c_int, ctypes.c_float]
+        + [ctypes.c_void_p] * 4,
+    ),
     "natten_amd_fna_forward_fused_context": (
         ctypes.c_int,
         [ctypes.c_void_p] * 7 + [ctypes.c_int] * 7 + [ctypes.c_void_p] * 7
@@ -568,10 +573,10 @@ def attention_forward_varlen(
     if cumulative_seqlen_q.shape[0] != cumulative_seqlen_kv.shape[0] or cumulative_seqlen_q.shape[0] < 2:
         raise ValueError("cumulative sequence lengths must match in size and hold at least 2 entries.")
     scales = _scale_ptrs(q, k, q_scale, k_scale, v_scale)
-    out = torch.zeros_like(q)
-    lse = torch.zeros(q.shape[:-1], dtype=torch.float32, device=q.device)
+    out = torch.empty_like(q)
+    lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     with _on_device(q):
-        rc = L.natten_amd_attention_forward_varlen(
+        rc = L.natten_amd_attention_forward_varlen_all_rows(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), DTYPE_CODES[q.dtype],
             cumulative_seqlen_q.shape[0] - 1, q.shape[1], k.shape[1], int(max_seqlen_q), int(max_seqlen_kv),
             q.shape[2], k.shape[2], q.shape[3], cumulative_seqlen_q.data_ptr(), cumulative_seqlen_kv.data_ptr(),

@@ -130,8 +130,15 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
       return fail("fna_forward: KV splits exist for Q tiles of 128 and KV tiles of 64 tokens");
     }
   }
-  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)wgs), dim3(NWAVES * 64), 0,
-                     stream, p);
+  FnaParams pk = p;
+  long long clearing = 0;
+  if (RAGGED && p.cu_q != nullptr) {
+    clearing = p.split_first != 0 ? na_ceil_div(p.total_q, packed_clear_rows(p.batch)) : 0;
+    pk.split_first = int(wgs);
+    if (wgs + clearing > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
+  }
+  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)(wgs + clearing)),
+                     dim3(NWAVES * 64), 0, stream, pk);
   return check_launch("fna_forward");
 }
 
@@ -992,12 +999,13 @@ int natten_amd_attention_forward_split(const void* q, const void* k, const void*
                            q_scale, k_scale, v_scale, stream, split_positions, kv_splits, parts, parts + rows * uint64_t(head_dim));
 }
 
-int natten_amd_attention_forward_varlen(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
-                                        int num_seqs, int total_seqlen_q, int total_seqlen_kv, int max_seqlen_q,
-                                        int max_seqlen_kv, int heads_q, int heads_kv, int head_dim,
-                                        const int32_t* cumulative_seqlen_q, const int32_t* cumulative_seqlen_kv,
-                                        int is_causal, float scale, const float* q_scale, const float* k_scale,
-                                        const float* v_scale, void* stream) {
+// clear: rows that belong to no sequence become zeros
+static int attention_forward_varlen(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                                    int num_seqs, int total_seqlen_q, int total_seqlen_kv, int max_seqlen_q,
+                                    int max_seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                    const int32_t* cumulative_seqlen_q, const int32_t* cumulative_seqlen_kv,
+                                    int is_causal, float scale, const float* q_scale, const float* k_scale,
+                                    const float* v_scale, void* stream, int clear) {
   g_error[0] = 0;
   const char* what = "attention_forward_varlen";
   if (int rc = check_common(what, q, k, v, out, lse, num_seqs, total_seqlen_q, total_seqlen_kv, heads_q, heads_kv,
@@ -1025,6 +1033,7 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
   p.q_tiled[0] = na_ceil_div(max_seqlen_q, QT);
   p.kv_tiled[0] = na_ceil_div(max_seqlen_kv, KVT);
   p.token_rows = p.tok_stride[0] = 1;
+  p.split_first = clear;
   p.num_groups = 1;
   p.q = q;
   p.k = k;
@@ -1046,6 +1055,28 @@ int natten_amd_attention_forward_varlen(const void* q, const void* k, const void
   p.total_kv = total_seqlen_kv;
   set_wg_layout(p, 1);
   return dispatch_dtype(p, dtype, head_dim, QT, KVT, static_cast<hipStream_t>(stream));
+}
+
+int natten_amd_attention_forward_varlen(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                                        int num_seqs, int total_seqlen_q, int total_seqlen_kv, int max_seqlen_q,
+                                        int max_seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                        const int32_t* cumulative_seqlen_q, const int32_t* cumulative_seqlen_kv,
+                                        int is_causal, float scale, const float* q_scale, const float* k_scale,
+                                        const float* v_scale, void* stream) {
+  return attention_forward_varlen(q, k, v, out, lse, dtype, num_seqs, total_seqlen_q, total_seqlen_kv, max_seqlen_q, max_seqlen_kv,
+                                  heads_q, heads_kv, head_dim, cumulative_seqlen_q, cumulative_seqlen_kv, is_causal, scale,
+                                  q_scale, k_scale, v_scale, stream, 0);
+}
+
+int natten_amd_attention_forward_varlen_all_rows(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                                                 int num_seqs, int total_seqlen_q, int total_seqlen_kv, int max_seqlen_q,
+                                                 int max_seqlen_kv, int heads_q, int heads_kv, int head_dim,
+                                                 const int32_t* cumulative_seqlen_q, const int32_t* cumulative_seqlen_kv,
+                                                 int is_causal, float scale, const float* q_scale, const float* k_scale,
+                                                 const float* v_scale, void* stream) {
+  return attention_forward_varlen(q, k, v, out, lse, dtype, num_seqs, total_seqlen_q, total_seqlen_kv, max_seqlen_q, max_seqlen_kv,
+                                  heads_q, heads_kv, head_dim, cumulative_seqlen_q, cumulative_seqlen_kv, is_causal, scale,
+                                  q_scale, k_scale, v_scale, stream, 1);
 }
 
 // ---- backward ---------------------------------------------------------------------------------
