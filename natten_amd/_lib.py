@@ -779,6 +779,24 @@ def fna_backward_fused(
     return dq, dk, dv
 
 
+def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int, is_causal: bool, equal: bool) -> bool:
+    """Whether the dq launch of dense attention runs beside the dk / dv launch (head dim 128: a workgroup per compute
+    unit), which then has a workspace for the scaled queries besides dq.  `key_tiles` over all heads, `longest_walk`:
+    query tiles of 64 that the longest of them meets, `equal`: sequences of one length.
+    Taken where the compute units stand idle for 20 of those steps (1.6 us) and a tenth of the time or more on the average:
+    the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic.  us of both launches and the pass
+    before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 322 / 259 (62),
+    5 up to 1527, H 4 95 / 75 (20), 16 of 512, H 16 / 4 150 / 157 (16), 7 up to 384, H 8 / 4 58 / 65 (11), 9 up to 176, H 16 37 / 81 (3);
+    1 x 2000 causal, H 16 / 4 248 / 209 (112), 1 x 9000 full, H 8 / 4 1431 / 1067 (251), H 16 2150 / 2095 (79), 2 x 2176 full,
+    H 16 336 / 290 (30), 2 x 4096 full, H 16 / 8 814 / 902 (0), 2 x 3000 causal, H 8 181 / 203 (12), 2 x 3809
+    full, H 24 1146 / 1160 (22 of 360).  Of 39 problems it is taken for 18, which are 1 to 25 % faster."""
+    if head_dim != 128:
+        return False
+    work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / 256
+    span = max(longest_walk, work) if is_causal or not equal else longest_walk * _ceil_div(key_tiles, 256)
+    return span - work >= max(20, span / 10)
+
+
 def attention_backward(
     q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, is_causal: bool, scale: float,
 ) -> Tuple[Tensor, Tensor, Tensor]:
@@ -788,12 +806,15 @@ def attention_backward(
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_backward does not support {q.dtype}.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq)
+    overlap = _backward_launches_overlap(q.shape[3], q.shape[0] * _ceil_div(k.shape[1], 128) * k.shape[2],
+                                         _ceil_div(q.shape[1], 64) * (q.shape[2] // k.shape[2]), is_causal, True)
+    q_scaled = torch.empty_like(q) if overlap else dq
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled)
     with _on_device(q):
         rc = L.natten_amd_attention_backward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], q.shape[0], q.shape[1],
-            k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), q_scaled.data_ptr(), 3 if overlap else 1, DTYPE_CODES[q.dtype],
+            q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)
     return dq, dk, dv
@@ -801,11 +822,11 @@ def attention_backward(
 
 def attention_backward_varlen(
     q: Tensor, k: Tensor, v: Tensor, out: Tensor, d_out: Tensor, lse: Tensor, cu_q: Tensor, cu_kv: Tensor,
-    is_causal: bool, scale: float,
+    is_causal: bool, scale: float, max_seqlen_q: int = 0,
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """Dense attention backward of a sequence-packed batch: q, out, d_out [1, rows_q, H, D], k, v [1, rows_kv,
     Hkv, D], lse [1, rows_q, H], device int32 cumulative lengths [sequences + 1] -> (dq, dk, dv); rows
-    of no sequence come back as zeros."""
+    of no sequence come back as zeros.  max_seqlen_q (0: not known) decides how the launches are made, not what they give."""
     L = lib()
     _require_gpu(q, k, v, cu_q, cu_kv)
     if q.dtype not in (torch.float16, torch.bfloat16):
@@ -816,12 +837,15 @@ def attention_backward_varlen(
         raise ValueError("sequence-packed operands have batch 1 and at least one sequence.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     tiles = torch.empty((2, cu_q.numel() + 1, 2), dtype=torch.int32, device=q.device)
-    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, dq, (cu_q, cu_kv, k.shape[1], tiles))
+    overlap = max_seqlen_q > 0 and _backward_launches_overlap(
+        q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False)
+    q_scaled = torch.empty_like(q) if overlap else dq
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled, (cu_q, cu_kv, k.shape[1], tiles))
     with _on_device(q):
         rc = L.natten_amd_attention_backward_varlen(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), 1, DTYPE_CODES[q.dtype], cu_q.numel() - 1, q.shape[1],
-            k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), tiles.data_ptr(), q.shape[2], k.shape[2], q.shape[3],
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), q_scaled.data_ptr(), 3 if overlap else 1, DTYPE_CODES[q.dtype],
+            cu_q.numel() - 1, q.shape[1], k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), tiles.data_ptr(), q.shape[2], k.shape[2], q.shape[3],
             1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)

@@ -103,7 +103,7 @@ struct FnaBwdParams {
   // the (batch, head, tile) space.  > 0: runs of this many consecutive tiles are dealt round-robin
   // to the XCDs (the grid is then a whole number of rounds of 8 runs).
   int kv_wg_run;
-  // Host side only: which launches a call makes (bit 0: the dQ role, bit 1: the dK / dV role; 0 = both).
+  // Host side only: which launches a call makes (bit 0: the dQ role, bit 1: the dK / dV role; 0 = both), and kBwdOverlap.
   int roles;
   // Derived by set_bwd_divisions(): what the per-workgroup set-up would otherwise divide for (tile
   // extents are powers of two, the other divisors get multiply-shift pairs).
@@ -182,6 +182,12 @@ inline int choose_kv_shift(int L, int k, int s, bool causal, int tile, int q_sub
   }
   return best;
 }
+
+// FnaBwdParams::roles: the dQ launch runs beside the dK / dV launch, on a stream of its own (dq is not the workspace that the
+// other one reads).  That launch lasts as long as its longest workgroup, and while that walks its query tiles most
+// compute units have nothing left to do: both launches of a packed step, 10 sequences of 1 .. 2048, H 16 / 4, D 128, with
+// the pass before, 317 us one behind the other and 256 side by side; the callers know where it pays.
+constexpr int kBwdOverlap = 16;
 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };
 

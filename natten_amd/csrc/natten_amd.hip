@@ -1082,6 +1082,52 @@ int natten_amd_attention_forward_varlen_all_rows(const void* q, const void* k, c
 // ---- backward ---------------------------------------------------------------------------------
 
 extern "C++" {
+// A thread's second stream on a device, and the events that order it behind the caller's stream and that one behind it.
+// Made on first use, given back when the thread ends; work on it is joined before the entry point that put it there returns.
+struct SideStream {
+  hipStream_t stream = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr;
+  void release() {
+    if (join) (void)hipEventDestroy(join);
+    if (fork) (void)hipEventDestroy(fork);
+    if (stream) (void)hipStreamDestroy(stream);
+    stream = nullptr;
+    fork = join = nullptr;
+  }
+};
+struct SideStreams {
+  static constexpr int kDevices = 16;
+  SideStream of[kDevices];
+  ~SideStreams() {
+    for (SideStream& s : of) s.release();
+  }
+};
+// The calling thread's side stream, `stream`'s work so far in front of it; null where there is none: a stream that is
+// being captured (the graph would hold the side stream, which eager calls also use), or any error.
+static SideStream* fork_side_stream(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  int dev = 0;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess ||
+      dev < 0 || dev >= SideStreams::kDevices) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  thread_local SideStreams streams;
+  SideStream& s = streams.of[dev];
+  if (!s.stream && (hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking) != hipSuccess ||
+                    hipEventCreateWithFlags(&s.fork, hipEventDisableTiming) != hipSuccess ||
+                    hipEventCreateWithFlags(&s.join, hipEventDisableTiming) != hipSuccess)) {
+    (void)hipGetLastError();
+    s.release();
+    return nullptr;
+  }
+  if (hipEventRecord(s.fork, stream) != hipSuccess || hipStreamWaitEvent(s.stream, s.fork, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return &s;
+}
+
 template <typename T, int D, bool RAGGED, bool RAW>
 static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   FnaBwdParams p = params;
@@ -1122,6 +1168,8 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
                        static_cast<T*>(const_cast<void*>(p.qs)), (int64_t)chunks, p.scale * 1.4426950408889634f);
     if (int rc = check_launch("fna_backward (scaled queries)")) return rc;
   }
+  SideStream* side = (roles & kBwdOverlap) ? fork_side_stream(stream) : nullptr;
+  int rc_kv = 0, rc_q = 0;
   if (roles & 2) {
     if constexpr (D == 128) {
       // dK and dV by wave pairs (eight waves per workgroup): one wave's registers cannot hold the
@@ -1130,13 +1178,17 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
     } else {
       hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDKV, RAGGED, RAW>), dim3((unsigned)wg_kv), dim3(256), 0, stream, p);
     }
-    if (int rc = check_launch("fna_backward (dK, dV)")) return rc;
+    rc_kv = check_launch("fna_backward (dK, dV)");
   }
-  if (roles & 1) {
-    hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDQ, RAGGED>), dim3((unsigned)wg_q), dim3(256), 0, stream, p);
-    if (int rc = check_launch("fna_backward (dQ)")) return rc;
+  if ((roles & 1) && rc_kv == 0) {
+    hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDQ, RAGGED>), dim3((unsigned)wg_q), dim3(256), 0, side ? side->stream : stream, p);
+    rc_q = check_launch("fna_backward (dQ)");
   }
-  return 0;
+  if (side && (hipEventRecord(side->join, side->stream) != hipSuccess || hipStreamWaitEvent(stream, side->join, 0) != hipSuccess)) {
+    (void)hipStreamSynchronize(side->stream);  // (the caller may reuse its memory once its own stream is past this call)
+    return fail("fna_backward: the dQ launch could not be joined");
+  }
+  return rc_kv ? rc_kv : rc_q;
 }
 
 template <typename T, int D>
@@ -1404,6 +1456,7 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
   FnaBwdParams p;
   fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal,
                  scale, q_scaled_filled);
+  if ((q_scaled_filled & 2) && q_scaled != dq && head_dim == 128) p.roles |= kBwdOverlap;
   // (sequences of whole tiles need no clamping: the instances of neighborhood attention)
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), seqlen_q % 128 != 0 || seqlen_kv % 128 != 0);
 }
@@ -1432,6 +1485,7 @@ int natten_amd_attention_backward_varlen(const void* q, const void* k, const voi
   p.packed_q = reinterpret_cast<const int2*>(packed_tiles);
   p.packed_kv = p.packed_q + (num_seqs + 2);
   p.num_seqs = num_seqs;
+  if ((q_scaled_filled & 2) && q_scaled != dq && head_dim == 128) p.roles |= kBwdOverlap;
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), true);
 }
 

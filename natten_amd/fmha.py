@@ -158,7 +158,7 @@ class AmdFmhaVarlenFunction(torch.autograd.Function):
         q, k, v, o, do = (pad_head_dim(t.contiguous(), d_pad).contiguous() for t in (query, key, value, out, d_out))
         dq, dk, dv = torch_ops.attention_backward_varlen(
             q, k, v, o, do, lse.contiguous(), cu_q.to(torch.int32).contiguous(), cu_kv.to(torch.int32).contiguous(), is_causal,
-            scale,
+            scale, max_q,
         )
         if d_pad != head_dim:
             dq, dk, dv = (t[..., :head_dim] for t in (dq, dk, dv))

@@ -306,10 +306,10 @@ def attention_backward(q, k, v, out, d_out, lse, is_causal, scale):
     return _lib.attention_backward(q, k, v, out, d_out, lse, is_causal, scale)
 
 
-def attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale):
+def attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale, max_seqlen_q=0):
     if _tracing():
         return _attention_backward_varlen_op(q, k, v, out, d_out, lse, cu_q, cu_kv, bool(is_causal), float(scale))
-    return _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale)
+    return _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu_q, cu_kv, is_causal, scale, max_seqlen_q)
 
 
 def token_permute(x, tile_shape, dilation, flip_tiled_dims, widen=False):

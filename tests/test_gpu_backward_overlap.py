@@ -1,0 +1,99 @@
+"""Dense and packed backward whose dq launch runs beside the dk / dv launch: the bits of one behind the other, on several
+streams and threads and where memory is reused at once; a captured call makes its launches one behind the other.  Where it is done (CPU)."""
+
+import threading
+
+import pytest
+import torch
+
+from natten_amd import _lib
+
+
+def test_rule():
+    rule = _lib._backward_launches_overlap
+    assert rule(128, 264, 128, True, False)       # packed, sequences up to 2048, four query heads a key head
+    assert rule(128, 284, 282, False, True)       # a second round of 28 key tiles
+    assert not rule(128, 256, 64, False, True)    # one full round
+    assert not rule(128, 512, 128, False, True)
+    assert not rule(128, 1440, 60, False, True)   # a last round of 160 of six
+    assert not rule(128, 24, 5, False, True)      # over before a second stream has begun
+    assert not rule(64, 264, 128, True, False)
+
+
+def problem(packed, seed, H=8, Hkv=2, D=128):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda", dtype=torch.bfloat16)
+    B, S = (1, 1300) if packed else (2, 600)
+    q, out, d_out, k, v = rand(B, S, H, D), rand(B, S, H, D), rand(B, S, H, D), rand(B, S, Hkv, D), rand(B, S, Hkv, D)
+    lse = torch.rand((B, S, H), generator=gen, device="cuda") + 7
+    if not packed:
+        return lambda: _lib.attention_backward(q, k, v, out, d_out, lse, True, 0.088)
+    cu = torch.tensor([0, 700, 701, 1100, 1290], dtype=torch.int32, device="cuda")
+    return lambda: _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu, cu, True, 0.088, 700)
+
+
+def both_ways(monkeypatch, call):
+    monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: False)
+    serial = call()
+    torch.cuda.synchronize()
+    monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: True)
+    return serial
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_same_bits(monkeypatch, packed):
+    call = problem(packed, 1)
+    serial = both_ways(monkeypatch, call)
+    for _ in range(5):  # (the workspace of one call is memory of the next)
+        copies = [t * 1 for t in call()]  # read on the caller's stream at once
+        for got, want in zip(copies, serial):
+            assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_streams_and_threads(monkeypatch, packed):
+    calls = [problem(packed, s) for s in (1, 2)]
+    serial = [both_ways(monkeypatch, c) for c in calls]
+    torch.cuda.synchronize()
+    wrong = []
+
+    def work(i):
+        for stream in (torch.cuda.Stream(), torch.cuda.Stream()):
+            with torch.cuda.stream(stream):
+                for _ in range(3):
+                    got = [t * 1 for t in calls[i]()]
+                    if not all(torch.equal(a, b) for a, b in zip(got, serial[i])):
+                        wrong.append(i)
+            stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_captured(monkeypatch, packed):
+    call = problem(packed, 1)
+    serial = both_ways(monkeypatch, call)
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        call()
+    torch.cuda.current_stream().wait_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = call()
+    for _ in range(3):
+        for t in got:
+            t.zero_()
+        eager = call()  # (the side stream, between replays)
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b, want in zip(got, eager, serial):
+            assert torch.equal(a, want) and torch.equal(b, want)
