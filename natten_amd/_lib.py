@@ -535,7 +535,10 @@ def attention_forward(
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
     with _on_device(q):
-        positions, splits = attention_split_plan(q.device.index, q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3], bool(is_causal))
+        splits = 1
+        if q.shape[0] > 1 and k.shape[1] > 960:  # (one sequence or under 16 key tiles: never split, and asking takes a small call 0.8 us)
+            positions, splits = attention_split_plan(
+                q.device.index, q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3], bool(is_causal))
         if splits > 1:
             parts = torch.empty(positions * splits * 128 * (q.shape[3] + 1), dtype=torch.float32, device=q.device)
             _check(L.natten_amd_attention_forward_split(
