@@ -458,7 +458,8 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // fetched: their places in the tiles are zeroed once, before the first copy.
 // CTX: every query also attends to the ctx_len keys of its batch entry's context, whose tiles come behind those of the
 // window box, in the same walk.  Context as a launch of dense attention of its own and a merge write and read both
-// results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a call 62 -> 31; 4 x 96 x 96, 24 x 24, H 16, D 128, 256 tokens: 665 -> 476).
+// results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a
+// call 62 -> 31; 4 x 96 x 96, 24 x 24, H 16, D 128, 256 tokens: 665 -> 476).
 template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
           bool CTX = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {

@@ -934,10 +934,11 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   const long long q_tiles = na_ceil_div(seqlen_q, 128), n = q_tiles * heads_q * batch;
   // The chip takes `slots` workgroups at a time.  What does not fill a last round is split so that it does, where
   // that saves a twelfth of the whole and more than the merge takes (2 x 4097 tokens, H 16, D 64, a third round of 32 Q
-  // tiles: 185 us, 170 with them split 13 ways; 2 x 9000, H 4, D 64: 232 and 187; 2 x 5000, H 8, D 128: 211 and 199).  In KV tiles of a workgroup that shares its
-  // compute unit (0.62 us at head dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch
-  // and the parts' way through memory eight.  The second launch and the workspace also take the host 5 us: launches under
-  // 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.  Causal: rounds even out by themselves (the longest walks
+  // tiles: 185 us, 170 with them split 13 ways; 2 x 9000, H 4, D 64: 232 and 187; 2 x 5000, H 8, D 128: 211 and 199).  In
+  // KV tiles of a workgroup that shares its compute unit (0.62 us at head dim 64, 1.05 at 128): a workgroup alone on one
+  // takes three quarters, the second launch and the parts' way through memory eight.  The second launch and the
+  // workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split 23.9;
+  // 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.  Causal: rounds even out by themselves (the longest walks
   // start first), and only a single round is split.  One batch entry is never split: a packed call promises the
   // bits of a dense call on each of its sequences alone.
   const int slots = resident_workgroups(head_dim <= 32 ? 3 : 2), cus = resident_workgroups(1);
