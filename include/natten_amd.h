@@ -465,9 +465,9 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
 /*
  * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
  * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2 = -log2(e) lse and neg_delta = -delta head-major
- * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above; q_scaled_filled != 0: it
- * is filled already (by the same call).
- * q_scaled_filled + 2, head dim 128, q_scaled not dq: the dq launch is made on a second stream of the calling thread and
+ * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above.  q_scaled_filled: two bits, the
+ * others are ignored.  1: q_scaled is filled already (natten_amd_backward_prepare); without it this call fills it.
+ * 2, at head dim 128 and with a q_scaled that is not dq: the dq launch is made on a second stream of the calling thread and
  * runs beside the dk / dv launch, which pays where that leaves the chip idle; `stream` waits for both.  The results are
  * the same.  While `stream` is captured the launches are made one behind the other.
  * Any sequence lengths: rows past the end of a sequence are gathered from its last row and masked.

@@ -1456,7 +1456,7 @@ int natten_amd_attention_backward(const void* q, const void* k, const void* v, c
   if (int rc = check_common(what, q, k, v, dq, neg_lse2, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim)) return rc;
   FnaBwdParams p;
   fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal,
-                 scale, q_scaled_filled);
+                 scale, q_scaled_filled & 1);
   if ((q_scaled_filled & 2) && q_scaled != dq && head_dim == 128) p.roles |= kBwdOverlap;
   // (sequences of whole tiles need no clamping: the instances of neighborhood attention)
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream), seqlen_q % 128 != 0 || seqlen_kv % 128 != 0);
@@ -1477,7 +1477,7 @@ int natten_amd_attention_backward_varlen(const void* q, const void* k, const voi
   if (num_seqs > (1 << 28)) return fail("%s: more than 2^28 sequences", what);
   FnaBwdParams p;
   fill_dense_bwd(p, q, k, v, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, 1, rows_q, rows_kv, heads_q, heads_kv, is_causal, scale,
-                 q_scaled_filled);
+                 q_scaled_filled & 1);
   // lengths and windows are replaced per sequence inside the kernel
   p.q_tiled[0] = rows_q / 128 + num_seqs + 3;
   p.kv_tiled[0] = rows_kv / 128 + num_seqs + 3;

@@ -1,5 +1,6 @@
 """Dense and packed backward whose dq launch runs beside the dk / dv launch: the bits of one behind the other, on several
-streams and threads and where memory is reused at once; a captured call makes its launches one behind the other.  Where it is done (CPU)."""
+streams and threads and where memory is reused at once; a captured call makes its launches one behind the other.  Where it is done
+(CPU).  The two bits of the C interface's q_scaled_filled."""
 
 import threading
 
@@ -97,3 +98,35 @@ def test_captured(monkeypatch, packed):
         torch.cuda.synchronize()
         for a, b, want in zip(got, eager, serial):
             assert torch.equal(a, want) and torch.equal(b, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("filled", [1, 2, 3])
+@pytest.mark.parametrize("packed", [False, True])
+def test_workspace_filled_or_not(packed, filled):
+    """q_scaled_filled: bit 0 says whether the workspace holds the scaled queries, bit 1 asks for the second stream."""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda", dtype=torch.bfloat16)
+    S, H, Hkv, D = 400, 4, 2, 128
+    q, out, d_out, k, v = rand(1, S, H, D), rand(1, S, H, D), rand(1, S, H, D), rand(1, S, Hkv, D), rand(1, S, Hkv, D)
+    lse = torch.rand((1, S, H), generator=gen, device="cuda") + 6
+    cu = torch.tensor([0, 250, 251, 400], dtype=torch.int32, device="cuda")
+    tiles = torch.empty((2, cu.numel() + 1, 2), dtype=torch.int32, device="cuda")
+    scaled = torch.empty_like(q)
+    neg_delta, neg_lse2 = _lib.backward_prepare(q, out, d_out, lse, D**-0.5, scaled, (cu, cu, S, tiles))
+
+    def grads(filled):
+        q_scaled = scaled if filled & 1 else torch.full_like(q, float("nan"))
+        got = [torch.full_like(t, float("nan")) for t in (q, k, v)]
+        head = (q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
+                *(g.data_ptr() for g in got), q_scaled.data_ptr(), filled, _lib.DTYPE_CODES[q.dtype])
+        tail = (H, Hkv, D, 1, D**-0.5, torch.cuda.current_stream().cuda_stream)
+        if packed:
+            rc = _lib.lib().natten_amd_attention_backward_varlen(*head, cu.numel() - 1, S, S, cu.data_ptr(), cu.data_ptr(), tiles.data_ptr(), *tail)
+        else:
+            rc = _lib.lib().natten_amd_attention_backward(*head, 1, S, S, *tail)
+        assert rc == 0, _lib.lib().natten_amd_last_error()
+        return got
+
+    for got, want in zip(grads(filled), grads(0)):
+        assert torch.isfinite(want).all() and torch.equal(got, want)
