@@ -1421,12 +1421,23 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   T* obase = reinterpret_cast<T*>(p.o) + q_row_base * q_row_stride + int64_t(head) * row_dim;
   float* lse_base = p.lse;
   if constexpr (SPLIT) {
+    if (empty_split) {
+      // (not by a factor of 0, which would leave NaN where the tile walked holds infinities)
+#pragma unroll
+      for (int mb = 0; mb < MQ; ++mb) {
+        l_run[mb] = 0.f;
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[mb][db][r] = 0.f;
+      }
+    }
     if (p.split_first < 0) {
       obase += split * p.o_split_stride;
       lse_base += split * p.lse_split_stride;
     } else if (splits > 1) {
       const int64_t row = (int64_t(pid - p.split_first) * splits + split) * QT + wave * 32 + l32;
-      const float l = empty_split ? 0.f : l_run[0] + __shfl_xor(l_run[0], 32);
+      const float l = l_run[0] + __shfl_xor(l_run[0], 32);
       const float inv = (l > 0.f) ? out_scale / l : 0.f;
       float* part = p.split_parts + row * row_dim + 4 * g;
 #pragma unroll
@@ -1444,7 +1455,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
 #pragma unroll
   for (int mb = 0; mb < MQ; ++mb) {
-    const float l = empty_split ? 0.f : l_run[mb] + __shfl_xor(l_run[mb], 32);
+    const float l = l_run[mb] + __shfl_xor(l_run[mb], 32);
     const float inv = (l > 0.f) ? out_scale / l : 0.f;
     const int row = q_row[mb];
     store_row_blocks<T, DB>(obase + int64_t(na_max(row, 0)) * q_row_stride, acc[mb], inv, g, row >= 0, row_dim);

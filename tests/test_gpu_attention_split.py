@@ -81,3 +81,20 @@ def test_any_number_of_positions(positions, splits, D):
     for p, n, pos in ((parts, parts.numel() - 1, positions), (parts[1:], parts.numel(), positions), (parts, 1 << 40, positions + 1),
                       (parts, 1 << 40, 512)):
         assert L.natten_amd_attention_forward_split(*args(p, n, pos)) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_infinite_values(D):
+    """Causal Q tiles with fewer key tiles than splits: a split without keys adds nothing, also where the tile that it walks
+    instead holds infinities.  By rows, as in the unsplit launch (batch 1)."""
+    q, k, v = (rand((2, 3600, 2, D), torch.bfloat16, seed) for seed in (1, 2, 3))
+    assert _lib.attention_split_plan(q.device.index, 2, 3600, 3600, 2, D, True)[1] > 3  # more than the first Q tile has key tiles
+    v[:, 5, :, 3], v[:, 40, :, 7], v[:, 3000, :, 9] = float("inf"), -float("inf"), float("inf")
+    with torch.no_grad():
+        out, lse = natten_amd.attention(q, k, v, is_causal=True, return_lse=True)
+        alone = [natten_amd.attention(q[i : i + 1], k[i : i + 1], v[i : i + 1], is_causal=True, return_lse=True) for i in range(2)]
+    want, want_lse = (torch.cat(t) for t in zip(*alone))
+    assert torch.isinf(want[:, 64:, :, 3]).all() and torch.isfinite(want[..., 0]).all()
+    torch.testing.assert_close(out.float(), want.float(), atol=2.0**-7, rtol=2.0**-7, equal_nan=True)  # (infinities and NaN: where they are)
+    torch.testing.assert_close(lse, want_lse, atol=1e-5, rtol=1e-5)

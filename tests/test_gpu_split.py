@@ -141,3 +141,14 @@ def test_split_random_sweep(n):
         eps = 2.0 ** -7 if dtype == torch.bfloat16 else 2.0 ** -10
         assert_close("out vs unsplit " + tag, to_np(out), to_np(whole_o), atol=eps, rtol=eps)
         assert_close("lse vs unsplit " + tag, to_np(lse), to_np(whole_l), atol=1e-5, rtol=1e-5)
+
+
+def test_infinite_values_in_the_tile_of_an_empty_run():
+    """A run without KV tiles adds nothing, also where the tile that it walks instead holds infinities."""
+    q, k, v = make_qkv(1, (1024,), 2, 1, 64, torch.bfloat16, seed=6)
+    v[:, 5, :, 3], v[:, 40, :, 7] = float("inf"), -float("inf")
+    whole, whole_lse = amd_fna_generic(q, k, v, (512,), (64,), (1,), (True,), return_lse=True, kv_splits=1)
+    out, lse = amd_fna_generic(q, k, v, (512,), (64,), (1,), (True,), return_lse=True, kv_splits=8)
+    assert torch.isinf(whole[:, 64:448, :, 3]).all() and torch.isfinite(whole[..., 0]).all()
+    torch.testing.assert_close(out.float(), whole.float(), atol=2.0**-7, rtol=2.0**-7, equal_nan=True)
+    torch.testing.assert_close(lse, whole_lse, atol=1e-5, rtol=1e-5)
