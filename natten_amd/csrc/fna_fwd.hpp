@@ -1449,7 +1449,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           for (int i = 0; i < 4; ++i) o4[i] = acc[0][db][4 * j + i] * inv;
           if (!NARROW || db * 32 + 8 * j < row_dim) *reinterpret_cast<f32x4_t*>(part + db * 32 + 8 * j) = o4;
         }
-      if (g == 0) p.split_lse[row] = (l > 0.f) ? (m_run[0] * 0.6931471805599453f + __logf(l)) : -INFINITY;
+      // (a sum that is NaN reaches the merge as such: a part of weight 0 would leave the row the LSE of the other parts)
+      if (g == 0) p.split_lse[row] = (l > 0.f) ? (m_run[0] * 0.6931471805599453f + __logf(l)) : (l == 0.f) ? -INFINITY : l;
       return;
     }
   }

@@ -98,3 +98,19 @@ def test_infinite_values(D):
     assert torch.isinf(want[:, 64:, :, 3]).all() and torch.isfinite(want[..., 0]).all()
     torch.testing.assert_close(out.float(), want.float(), atol=2.0**-7, rtol=2.0**-7, equal_nan=True)  # (infinities and NaN: where they are)
     torch.testing.assert_close(lse, want_lse, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 96, 128])
+def test_rows_of_nan(D):
+    """A key or a query of NaN: the rows that it reaches are NaN with an LSE of -inf, as in the unsplit launch (batch 1)."""
+    q, k, v = (rand((2, 3600, 2, D), torch.bfloat16, seed) for seed in (1, 2, 3))
+    q[1, 77], k[0, 3000, 1] = float("nan"), float("nan")
+    with torch.no_grad():
+        out, lse = natten_amd.attention(q, k, v, return_lse=True)
+        alone = [natten_amd.attention(q[i : i + 1], k[i : i + 1], v[i : i + 1], return_lse=True) for i in range(2)]
+    want, want_lse = (torch.cat(t) for t in zip(*alone))
+    assert _lib.attention_split_plan(q.device.index, 2, 3600, 3600, 2, D, False)[1] > 1
+    assert torch.isnan(want[0, :, 1]).all() and torch.isnan(want[1, 77]).all() and torch.isfinite(want[0, :, 0]).all()
+    torch.testing.assert_close(out.float(), want.float(), atol=2.0**-7, rtol=2.0**-7, equal_nan=True)
+    torch.testing.assert_close(lse, want_lse, atol=1e-5, rtol=1e-5)
