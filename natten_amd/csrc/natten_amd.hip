@@ -857,28 +857,15 @@ int natten_amd_fna_forward_fused_static(const void* q, const void* k, const void
                                 k_scale, v_scale, /*anchor_kv_tiles=*/1, queues, stream);
 }
 
-static int attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int batch,
-                             int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim, int is_causal, float scale,
-                             const float* q_scale, const float* k_scale, const float* v_scale, void* stream, int split_positions,
-                             int kv_splits, float* parts, float* lse_parts) {
-  g_error[0] = 0;
-  if (int rc = check_common("attention_forward", q, k, v, out, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv,
-                            head_dim, dtype == NATTEN_AMD_F16 || dtype == NATTEN_AMD_BF16))
-    return rc;
-  // Dense attention is the 1-D neighborhood problem whose window is the whole key sequence:
-  // non-causal windows are [0, seqlen_kv), causal ones [0, min(i + 1, seqlen_kv)).
+// Dense attention is the 1-D neighborhood problem whose window is the whole key sequence:
+// non-causal windows are [0, seqlen_kv), causal ones [0, min(i + 1, seqlen_kv)).
+static void fill_dense_fwd(FnaParams& p, int batch, int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int is_causal) {
   constexpr int QT = 128, KVT = 64;
-  FnaParams p;
   memset(&p, 0, sizeof(p));
   for (int a = 0; a < 3; ++a) {
     p.qkv_shape[a] = p.ksize[a] = p.stride[a] = p.dil[a] = p.q_tile[a] = p.kv_tile[a] = p.q_tiled[a] = p.kv_tiled[a] = 1;
   }
-  if (seqlen_kv < 2) {
-    // a one-key window is the unused-dimension case of the window arithmetic (k = 1)
-    p.ksize[0] = 1;
-  } else {
-    p.ksize[0] = seqlen_kv;
-  }
+  p.ksize[0] = seqlen_kv;  // (a one-key window is the unused-dimension case of the window arithmetic)
   p.qkv_shape[0] = seqlen_kv;
   p.causal[0] = is_causal != 0;
   p.q_tile[0] = QT;
@@ -888,17 +875,30 @@ static int attention_forward(const void* q, const void* k, const void* v, void* 
   p.edge = (seqlen_kv % KVT != 0 && seqlen_kv >= KVT) ? 1 : 0;
   p.token_rows = p.tok_stride[0] = 1;
   p.num_groups = 1;
+  p.batch = batch;
+  p.heads_q = heads_q;
+  p.heads_kv = heads_kv;
+  p.seqlen_q = seqlen_q;
+  p.seqlen_kv = seqlen_kv;
+  set_wg_layout(p, 1);
+}
+
+static int attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype, int batch,
+                             int seqlen_q, int seqlen_kv, int heads_q, int heads_kv, int head_dim, int is_causal, float scale,
+                             const float* q_scale, const float* k_scale, const float* v_scale, void* stream, int split_positions,
+                             int kv_splits, float* parts, float* lse_parts) {
+  g_error[0] = 0;
+  if (int rc = check_common("attention_forward", q, k, v, out, lse, batch, seqlen_q, seqlen_kv, heads_q, heads_kv,
+                            head_dim, dtype == NATTEN_AMD_F16 || dtype == NATTEN_AMD_BF16))
+    return rc;
+  FnaParams p;
+  fill_dense_fwd(p, batch, seqlen_q, seqlen_kv, heads_q, heads_kv, is_causal);
   p.q = q;
   p.k = k;
   p.v = v;
   p.o = out;
   p.lse = lse;
-  p.batch = batch;
-  p.heads_q = heads_q;
   p.row_dim = head_dim;
-  p.heads_kv = heads_kv;
-  p.seqlen_q = seqlen_q;
-  p.seqlen_kv = seqlen_kv;
   p.scale = scale;
   p.q_scale = q_scale;
   p.k_scale = k_scale;
@@ -909,8 +909,7 @@ static int attention_forward(const void* q, const void* k, const void* v, void* 
     p.split_parts = parts;
     p.split_lse = lse_parts;
   }
-  set_wg_layout(p, 1);
-  return dispatch_dtype(p, dtype, head_dim, QT, KVT, static_cast<hipStream_t>(stream));
+  return dispatch_dtype(p, dtype, head_dim, 128, 64, static_cast<hipStream_t>(stream));
 }
 
 int natten_amd_attention_forward(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
@@ -932,18 +931,38 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   *kv_splits = 1;
   const int kv_tiles = na_ceil_div(seqlen_kv, 64);
   const long long q_tiles = na_ceil_div(seqlen_q, 128), n = q_tiles * heads_q * batch;
-  // The chip takes `slots` workgroups at a time.  What does not fill a last round is split so that it does, where
-  // that saves a twelfth of the whole and more than the merge takes (2 x 4097 tokens, H 16, D 64, a third round of 32 Q
-  // tiles: 185 us, 170 with them split 13 ways; 2 x 9000, H 4, D 64: 232 and 187; 2 x 5000, H 8, D 128: 211 and 199).  In
-  // KV tiles of a workgroup that shares its compute unit (0.62 us at head dim 64, 1.05 at 128): a workgroup alone on one
-  // takes three quarters, the second launch and the parts' way through memory eight.  The second launch and the
-  // workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split 23.9;
-  // 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.  Causal: rounds even out by themselves (the longest walks
-  // start first), and only a single round is split.  One batch entry is never split: a packed call promises the
-  // bits of a dense call on each of its sequences alone.
-  const int slots = resident_workgroups(head_dim <= 32 ? 3 : 2), cus = resident_workgroups(1);
-  const long long full = n / slots, rem = n % slots;
-  if (batch < 2 || kv_tiles < 16 || rem == 0 || full > 12 || (is_causal && full > 0)) return 0;
+  const int slots = resident_workgroups(2), cus = resident_workgroups(1);
+  // One batch entry is never split: a packed call promises the bits of a dense call on each of its sequences alone.
+  // Causal: rounds even out by themselves (the longest walks start first), and only a single round is split.
+  if (batch < 2 || kv_tiles < 16 || n / slots > 12 || (is_causal && n > slots)) return 0;
+  FnaParams p;
+  fill_dense_fwd(p, batch, seqlen_q, seqlen_kv, heads_q, heads_q, is_causal);
+  // The chip takes `slots` workgroups of the split launch at a time (two waves per SIMD at every head dim).  What does not
+  // fill a last round is split so that it does, where that saves a twelfth of the whole and more than the merge takes
+  // (2 x 4097 tokens, H 16, D 64, a third round of 32 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
+  // and 180; 2 x 5000, H 8, D 128: 204 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
+  // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch and the parts' way through memory
+  // eight.  The second launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4,
+  // D 128: 19.6 us, split 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
+  long long full = n / slots, rem = n % slots;
+  if (n > slots && fwd_max_waves(head_dim <= 32 ? 32 : head_dim, fully_block_sparse(p)) > 2) {
+    // The one launch holds three waves per SIMD, and whatever is split, every Q tile loses the third.
+    const int held = resident_workgroups(3);
+    if (head_dim <= 32) {
+      // Rounds are those of the one launch.  One and up to an eighth: faster split from some 96 KV tiles on (us, one launch / split:
+      // 792 Q tiles of 65 KV tiles 97.5 / 99.5, of 125 179 / 174, of 197 279 / 266; 840 of 125 180 / 172; 888 of 65 99 / 100, of
+      // 125 181 / 180); more rounds lose more (1562 of 141 340 / 374).
+      full = n / held;
+      rem = n % held;
+      if (full != 1 || rem * 8 > held || kv_tiles < 96) return 0;
+    } else if (n > held || rem * 4 > slots || kv_tiles < 40 + 256 * rem / slots) {
+      // One round there, two here: the walk has to be long for what is left over to be worth the third wave (528 Q tiles of 48 KV
+      // tiles 69.8 / 65.4; 544 of 48 69.8 / 71.0, of 72 101.9 / 98.5; 576 of 48 71.7 / 73.8, of 72 103.3 / 99.1, of 144 200 / 183;
+      // 640 of 40 64 / 68, of 72 106.2 / 108.6, of 100 145.7 / 144.7; 704 of 176 258 / 272; 1056 of 64 156 / 164).
+      return 0;
+    }
+  }
+  if (rem == 0) return 0;
   const double round = rem <= cus ? 0.75 * kv_tiles : kv_tiles;
   double least = 1e30;
   int best = 1;
@@ -956,16 +975,6 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   }
   if (best == 1 || full * kv_tiles + round < 40 || least > round - (full * kv_tiles + round) / 12) return 0;
   // the launch positions that hold the last `rem` Q tiles
-  FnaParams p;
-  memset(&p, 0, sizeof(p));
-  p.batch = batch;
-  p.heads_q = p.heads_kv = heads_q;
-  for (int a = 0; a < 3; ++a) p.qkv_shape[a] = p.ksize[a] = p.stride[a] = p.dil[a] = p.q_tile[a] = p.kv_tile[a] = p.q_tiled[a] = p.kv_tiled[a] = 1;
-  p.q_tile[0] = 128;
-  p.kv_tile[0] = 64;
-  p.q_tiled[0] = int(q_tiles);
-  p.num_groups = 1;
-  set_wg_layout(p, 1);
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
   long long first = wgs;
   for (long long left = rem; first > 0 && left > 0;) {

@@ -31,6 +31,21 @@ def test_plan():
         assert splits > 1 and positions >= tiles % 512 and tiles % 512 * splits <= 512
 
 
+def test_plan_where_the_one_launch_holds_three_waves():
+    """Head dim 32, and head dim 64 without masks: the split launch holds two waves per SIMD at either."""
+    plan = lambda *a: _lib.attention_split_plan(0, *a)
+    for S, H in ((2560, 16), (3072, 12), (5120, 8), (4096, 17)):    # 576 .. 1088 Q tiles: 768 fit one round
+        assert plan(2, S, S, H, 64, False) == (0, 1)
+    assert plan(2, 8448, 3072, 4, 64, False)[1] > 1 and plan(2, 9216, 9216, 4, 64, False)[1] > 1   # long walks, few left over
+    assert plan(2, 2560, 2561, 16, 64, False)[1] > 1                # masks: two waves either way
+    for S, H in ((4097, 16), (3500, 16), (4097, 12), (10000, 10)):
+        assert plan(2, S, S, H, 32, False) == (0, 1)
+    assert plan(2, 12547, 12547, 4, 32, False)[1] > 1
+    for S, H in ((4000, 4), (8000, 2), (4000, 3), (4000, 2)):       # one round
+        positions, splits = plan(2, S, S, H, 32, False)
+        assert splits > 1 and 2 * H * -(-S // 128) * splits <= 512
+
+
 CASES = [
     # B, Sq, Skv, H, Hkv, D, causal
     (2, 300, 3500, 2, 1, 128, False),
