@@ -931,59 +931,80 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   *kv_splits = 1;
   const int kv_tiles = na_ceil_div(seqlen_kv, 64);
   const long long q_tiles = na_ceil_div(seqlen_q, 128), n = q_tiles * heads_q * batch;
-  const int slots = resident_workgroups(2), cus = resident_workgroups(1);
   // One batch entry is never split: a packed call promises the bits of a dense call on each of its sequences alone.
-  // Causal: rounds even out by themselves (the longest walks start first), and only a single round is split.
-  if (batch < 2 || kv_tiles < 16 || n / slots > 12 || (is_causal && n > slots)) return 0;
+  const int slots = resident_workgroups(2) / kNumXcd, cus = resident_workgroups(1) / kNumXcd;
+  if (batch < 2 || kv_tiles < 16 || n / (slots * kNumXcd) > 12) return 0;
   FnaParams p;
   fill_dense_fwd(p, batch, seqlen_q, seqlen_kv, heads_q, heads_q, is_causal);
-  // The chip takes `slots` workgroups of the split launch at a time (two waves per SIMD at every head dim).  What does not
+  // Every XCD works off its own launch positions (see fna_fwd_tile): the one with the most Q tiles sets the time.  In an
+  // XCD's tiles, where the shares are uneven (5 x 3100 tokens, H 5, D 128: 131 us in one launch; counted over the chip, 113 of 625
+  // Q tiles were split four ways, and the fullest XCD still began another round: 149).
+  auto tiles_at = [&](int xcd, int local) {  // 1 where the position holds a Q tile
+    const int run = local / p.wg_group, group = run * kNumXcd + xcd;
+    return group < p.total_groups && group % p.groups_per_bh * p.wg_group + local - run * p.wg_group < p.num_q_tiles ? 1 : 0;
+  };
+  const int positions = na_ceil_div(p.total_groups, kNumXcd) * p.wg_group;  // of an XCD
+  int tiles[kNumXcd] = {}, most = 0;
+  for (int x = 0; x < kNumXcd; ++x) {
+    for (int i = 0; i < positions; ++i) tiles[x] += tiles_at(x, i);
+    most = na_max(most, tiles[x]);
+  }
+  // An XCD takes `slots` workgroups of the split launch at a time (two waves per SIMD at every head dim).  What does not
   // fill a last round is split so that it does, where that saves a twelfth of the whole and more than the merge takes
-  // (2 x 4097 tokens, H 16, D 64, a third round of 32 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
+  // (2 x 4097 tokens, H 16, D 64, a third round of 4 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
   // and 180; 2 x 5000, H 8, D 128: 204 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
   // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch and the parts' way through memory
   // eight.  The second launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4,
   // D 128: 19.6 us, split 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
-  long long full = n / slots, rem = n % slots;
-  if (n > slots && fwd_max_waves(head_dim <= 32 ? 32 : head_dim, fully_block_sparse(p)) > 2) {
-    // The one launch holds three waves per SIMD, and whatever is split, every Q tile loses the third.
-    const int held = resident_workgroups(3);
-    if (head_dim <= 32) {
-      // Rounds are those of the one launch.  One and up to an eighth: faster split from some 96 KV tiles on (us, one launch / split:
-      // 792 Q tiles of 65 KV tiles 97.5 / 99.5, of 125 179 / 174, of 197 279 / 266; 840 of 125 180 / 172; 888 of 65 99 / 100, of
-      // 125 181 / 180); more rounds lose more (1562 of 141 340 / 374).
-      full = n / held;
-      rem = n % held;
-      if (full != 1 || rem * 8 > held || kv_tiles < 96) return 0;
-    } else if (n > held || rem * 4 > slots || kv_tiles < 40 + 256 * rem / slots) {
-      // One round there, two here: the walk has to be long for what is left over to be worth the third wave (528 Q tiles of 48 KV
-      // tiles 69.8 / 65.4; 544 of 48 69.8 / 71.0, of 72 101.9 / 98.5; 576 of 48 71.7 / 73.8, of 72 103.3 / 99.1, of 144 200 / 183;
-      // 640 of 40 64 / 68, of 72 106.2 / 108.6, of 100 145.7 / 144.7; 704 of 176 258 / 272; 1056 of 64 156 / 164).
-      return 0;
+  int round_slots = slots;
+  if (most > slots) {
+    if (is_causal) return 0;  // rounds even out by themselves: the longest walks start first
+    if (fwd_max_waves(head_dim <= 32 ? 32 : head_dim, fully_block_sparse(p)) > 2) {
+      // The one launch holds three waves per SIMD, and whatever is split, every Q tile loses the third.
+      const int held = resident_workgroups(3) / kNumXcd;
+      const int left = most % slots;
+      if (head_dim <= 32) {
+        // Rounds are those of the one launch.  One and up to an eighth: faster split from some 128 KV tiles on (us, one launch /
+        // split: 792 Q tiles of 65 KV tiles 97.5 / 99.5, of 125 179 / 174, of 197 279 / 266; 840 of 80 119 / 119, of 125 180 / 172;
+        // 888 of 125 181 / 180); more rounds lose more (1562 of 141 340 / 374).
+        if (most / held != 1 || most % held * 8 > held || kv_tiles < 128) return 0;
+        round_slots = held;
+      } else if (most > held) {
+        // Two or three rounds and a sixteenth or less: 1040 Q tiles of 100 KV tiles 238 / 237, of 140 330 / 317, of 200 467 / 441; 1568
+        // of 140 482 / 465; 1088 of 100 244 / 242, of 140 337 / 332; 2080 of 140 617 / 615; 2600 of 200 1073 / 1080.
+        if (left * 16 > slots || most > 4 * slots || kv_tiles < 128) return 0;
+      } else if (left * 4 > slots || kv_tiles < 40 + 256 * left / slots) {
+        // One round there, two here: the walk has to be long for what is left over to be worth the third wave (528 Q tiles of 48
+        // KV tiles 69.8 / 65.4; 544 of 48 69.8 / 71.0, of 72 101.9 / 98.5; 576 of 48 71.7 / 73.8, of 72 103.3 / 99.1, of 144
+        // 200 / 183; 640 of 40 64 / 68, of 72 106.2 / 108.6, of 100 145.7 / 144.7; 704 of 176 258 / 272).
+        return 0;
+      }
     }
   }
-  if (rem == 0) return 0;
-  const double round = rem <= cus ? 0.75 * kv_tiles : kv_tiles;
+  const int full = most / round_slots;
+  if (most % round_slots == 0) return 0;
+  // the fewest positions at the end of every XCD's that leave no XCD more than whole rounds
+  int last = 0;
+  for (bool over = true; over;) {
+    ++last;
+    over = false;
+    for (int x = 0; x < kNumXcd; ++x) {
+      tiles[x] -= tiles_at(x, positions - last);
+      over = over || tiles[x] > full * round_slots;
+    }
+  }
+  const double round = last <= cus ? 0.75 * kv_tiles : kv_tiles;
   double least = 1e30;
   int best = 1;
-  for (int s = 2; s <= 16 && rem * s <= slots && kv_tiles / s >= 3; ++s) {
-    const double t = (rem * s <= cus ? 0.75 : 1.0) * na_ceil_div(kv_tiles, s) + 8;
+  for (int s = 2; s <= 16 && last * s <= slots && kv_tiles / s >= 3; ++s) {
+    const double t = (last * s <= cus ? 0.75 : 1.0) * na_ceil_div(kv_tiles, s) + 8;
     if (t < least) {
       least = t;
       best = s;
     }
   }
   if (best == 1 || full * kv_tiles + round < 40 || least > round - (full * kv_tiles + round) / 12) return 0;
-  // the launch positions that hold the last `rem` Q tiles
-  const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
-  long long first = wgs;
-  for (long long left = rem; first > 0 && left > 0;) {
-    --first;
-    const int local = int(first / kNumXcd), run = local / p.wg_group, group = run * kNumXcd + int(first % kNumXcd);
-    if (group < p.total_groups && group % p.groups_per_bh * p.wg_group + local - run * p.wg_group < p.num_q_tiles) --left;
-  }
-  first = first / kNumXcd * kNumXcd;
-  *split_positions = int(wgs - first);
+  *split_positions = last * kNumXcd;
   *kv_splits = best;
   return 0;
 }

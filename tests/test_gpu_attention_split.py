@@ -46,6 +46,16 @@ def test_plan_where_the_one_launch_holds_three_waves():
         assert splits > 1 and 2 * H * -(-S // 128) * splits <= 512
 
 
+def test_plan_counts_by_xcd():
+    """The XCD with the most Q tiles ends a launch: where the shares are uneven, no XCD keeps more than whole rounds unsplit."""
+    plan = lambda *a: _lib.attention_split_plan(0, *a)
+    assert plan(5, 3100, 3100, 5, 128, False) == (0, 1)     # 91 tiles on some: two halves of the last 27 save too little
+    assert plan(3, 5000, 5000, 9, 128, False) == (96, 5)    # 140 on some: the last 12 of each
+    assert plan(2, 8257, 3001, 8, 128, False)[0] == 32      # 132 on every other one
+    assert plan(2, 6500, 6500, 6, 96, False) == (112, 4)
+    assert plan(3, 3522, 3522, 3, 128, False) == (0, 1)     # 35 of 64: not twice
+
+
 CASES = [
     # B, Sq, Skv, H, Hkv, D, causal
     (2, 300, 3500, 2, 1, 128, False),
