@@ -782,10 +782,16 @@ def fna_backward_fused(
     return dq, dk, dv
 
 
-def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int, is_causal: bool, equal: bool) -> bool:
+@functools.lru_cache(maxsize=64)
+def _compute_units(device_index: int) -> int:
+    return torch.cuda.get_device_properties(device_index).multi_processor_count
+
+
+def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int, is_causal: bool, equal: bool,
+                               compute_units: int = 256) -> bool:
     """Whether the dq launch of dense attention runs beside the dk / dv launch (head dim 128: a workgroup per compute
     unit), which then has a workspace for the scaled queries besides dq.  `key_tiles` over all heads, `longest_walk`:
-    query tiles of 64 that the longest of them meets, `equal`: sequences of one length.
+    query tiles of 64 that the longest of them meets, `equal`: sequences of one length.  Figures with 256 compute units.
     Taken where the compute units stand idle for 20 of those steps (1.6 us) and a tenth of the time or more on the average:
     the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic.  us of both launches and the pass
     before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 322 / 259 (62),
@@ -795,8 +801,8 @@ def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int,
     full, H 24 1146 / 1160 (22 of 360).  Of 39 problems it is taken for 18, which are 1 to 25 % faster."""
     if head_dim != 128:
         return False
-    work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / 256
-    span = max(longest_walk, work) if is_causal or not equal else longest_walk * _ceil_div(key_tiles, 256)
+    work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / compute_units
+    span = max(longest_walk, work) if is_causal or not equal else longest_walk * _ceil_div(key_tiles, compute_units)
     return span - work >= max(20, span / 10)
 
 
@@ -810,7 +816,8 @@ def attention_backward(
         raise NotImplementedError(f"natten_amd attention_backward does not support {q.dtype}.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     overlap = _backward_launches_overlap(q.shape[3], q.shape[0] * _ceil_div(k.shape[1], 128) * k.shape[2],
-                                         _ceil_div(q.shape[1], 64) * (q.shape[2] // k.shape[2]), is_causal, True)
+                                         _ceil_div(q.shape[1], 64) * (q.shape[2] // k.shape[2]), is_causal, True,
+                                         _compute_units(q.device.index))
     q_scaled = torch.empty_like(q) if overlap else dq
     neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled)
     with _on_device(q):
@@ -841,7 +848,8 @@ def attention_backward_varlen(
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     tiles = torch.empty((2, cu_q.numel() + 1, 2), dtype=torch.int32, device=q.device)
     overlap = max_seqlen_q > 0 and _backward_launches_overlap(
-        q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False)
+        q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False,
+        _compute_units(q.device.index))
     q_scaled = torch.empty_like(q) if overlap else dq
     neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled, (cu_q, cu_kv, k.shape[1], tiles))
     with _on_device(q):

@@ -21,6 +21,12 @@ def test_rule():
     assert not rule(64, 264, 128, True, False)
 
 
+def test_rule_counts_the_compute_units_of_the_device():
+    rule = _lib._backward_launches_overlap
+    assert rule(128, 264, 128, True, False, 256) and not rule(128, 264, 128, True, False, 132)   # full with half of them
+    assert not rule(128, 256, 128, False, True, 256) and rule(128, 256, 128, False, True, 304)    # a round that is not full
+
+
 def problem(packed, seed, H=8, Hkv=2, D=128):
     gen = torch.Generator(device="cuda").manual_seed(seed)
     rand = lambda *shape: torch.randn(shape, generator=gen, device="cuda", dtype=torch.bfloat16)
@@ -31,6 +37,16 @@ def problem(packed, seed, H=8, Hkv=2, D=128):
         return lambda: _lib.attention_backward(q, k, v, out, d_out, lse, True, 0.088)
     cu = torch.tensor([0, 700, 701, 1100, 1290], dtype=torch.int32, device="cuda")
     return lambda: _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu, cu, True, 0.088, 700)
+
+
+@pytest.mark.gpu
+def test_the_device_is_asked(monkeypatch):
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    for packed in (False, True):
+        call, asked = problem(packed, 1), []
+        monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: asked.append(a[-1]))
+        call()
+        assert asked == [units]
 
 
 def both_ways(monkeypatch, call):
