@@ -836,7 +836,8 @@ def attention_backward_varlen(
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """Dense attention backward of a sequence-packed batch: q, out, d_out [1, rows_q, H, D], k, v [1, rows_kv,
     Hkv, D], lse [1, rows_q, H], device int32 cumulative lengths [sequences + 1] -> (dq, dk, dv); rows
-    of no sequence come back as zeros.  max_seqlen_q (0: not known) decides how the launches are made, not what they give."""
+    of no sequence come back as zeros.  max_seqlen_q (0: not known) decides how the launches are made, not what they give: a
+    bound far above the longest sequence may choose the second stream where that costs time."""
     L = lib()
     _require_gpu(q, k, v, cu_q, cu_kv)
     if q.dtype not in (torch.float16, torch.bfloat16):
@@ -847,7 +848,11 @@ def attention_backward_varlen(
         raise ValueError("sequence-packed operands have batch 1 and at least one sequence.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     tiles = torch.empty((2, cu_q.numel() + 1, 2), dtype=torch.int32, device=q.device)
-    overlap = max_seqlen_q > 0 and _backward_launches_overlap(
+    # The longest sequence is not known here, only what the caller says bounds it.  All rows, with several sequences, says
+    # nothing; any other bound is taken as the longest (us, one behind the other / side by side: 16 of 128, H 8 / 2 49 / 68;
+    # 9 up to 176, H 16 / 4 58 / 68; 16 of 512, H 16 / 4 declared as 1024 152 / 157).
+    bounded = 0 < max_seqlen_q and (max_seqlen_q < q.shape[1] or cu_q.numel() == 2)
+    overlap = bounded and _backward_launches_overlap(
         q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False,
         _compute_units(q.device.index))
     q_scaled = torch.empty_like(q) if overlap else dq

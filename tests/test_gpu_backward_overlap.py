@@ -49,6 +49,20 @@ def test_the_device_is_asked(monkeypatch):
         assert asked == [units]
 
 
+@pytest.mark.gpu
+def test_a_bound_of_all_rows_says_nothing(monkeypatch):
+    """max_seqlen_Q as large as the batch, with several sequences in it, is no estimate of the longest."""
+    asked = []
+    monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: asked.append(a) or False)
+    q, out, d_out = (torch.randn((1, 640, 4, 128), device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    k, v, lse = (*(torch.randn((1, 640, 2, 128), device="cuda", dtype=torch.bfloat16) for _ in range(2)), torch.rand((1, 640, 4), device="cuda"))
+    for lengths, bound, asks in (((300, 340), 340, 1), ((300, 340), 640, 0), ((300, 340), 0, 0), ((640,), 640, 1)):
+        cu = torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device="cuda")
+        asked.clear()
+        _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu, cu, True, 0.088, bound)
+        assert len(asked) == asks, (lengths, bound)
+
+
 def both_ways(monkeypatch, call):
     monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: False)
     serial = call()
