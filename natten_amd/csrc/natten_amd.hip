@@ -1115,8 +1115,9 @@ int natten_amd_attention_forward_varlen_all_rows(const void* q, const void* k, c
 extern "C++" {
 // A thread's second stream on a device, and the events that order it behind the caller's stream and that one behind it.
 // Made on first use, given back when the thread ends; work on it is joined before the entry point that put it there returns.
+// One caller's stream uses it at a time: the work of another one would wait behind the first one's, and with it that stream.
 struct SideStream {
-  hipStream_t stream = nullptr;
+  hipStream_t stream = nullptr, user = nullptr;  // user: the stream that forked it last
   hipEvent_t fork = nullptr, join = nullptr;
   void release() {
     if (join) (void)hipEventDestroy(join);
@@ -1134,7 +1135,8 @@ struct SideStreams {
   }
 };
 // The calling thread's side stream, `stream`'s work so far in front of it; null where there is none: a stream that is
-// being captured (the graph would hold the side stream, which eager calls also use), or any error.
+// being captured (the graph would hold the side stream, which eager calls also use), work of another stream on it that is
+// not done, or any error.
 static SideStream* fork_side_stream(hipStream_t stream) {
   hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
   int dev = 0;
@@ -1152,10 +1154,12 @@ static SideStream* fork_side_stream(hipStream_t stream) {
     s.release();
     return nullptr;
   }
-  if (hipEventRecord(s.fork, stream) != hipSuccess || hipStreamWaitEvent(s.stream, s.fork, 0) != hipSuccess) {
+  if ((s.user != stream && hipStreamQuery(s.stream) != hipSuccess) || hipEventRecord(s.fork, stream) != hipSuccess ||
+      hipStreamWaitEvent(s.stream, s.fork, 0) != hipSuccess) {
     (void)hipGetLastError();
     return nullptr;
   }
+  s.user = stream;
   return &s;
 }
 

@@ -3,6 +3,7 @@ streams and threads and where memory is reused at once; a captured call makes it
 (CPU).  The two bits of the C interface's q_scaled_filled."""
 
 import threading
+import time
 
 import pytest
 import torch
@@ -105,6 +106,44 @@ def test_streams_and_threads(monkeypatch, packed):
     for t in threads:
         t.join()
     assert not wrong
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_streams_of_a_thread_do_not_wait_for_each_other(monkeypatch, packed):
+    """A call on one stream ends while the call before it, on another stream of the thread, still waits for its turn."""
+    calls = [problem(packed, s) for s in (1, 2)]
+    serial = [both_ways(monkeypatch, c) for c in calls]
+    torch.cuda.synchronize()
+    busy = torch.cuda.Stream()
+    done = torch.cuda.Event()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(10**9)  # (half a second: a spin that ends by itself)
+        first = calls[0]()
+        done.record()
+    free = None
+    for _ in range(3):  # streams share a few hardware queues: one whose own work is not behind the spin
+        other = torch.cuda.Stream()
+        with torch.cuda.stream(other):
+            torch.zeros(1, device="cuda")
+        for _ in range(200):
+            if other.query():
+                break
+            time.sleep(1e-4)
+        if other.query() and not done.query():
+            free = other
+            break
+    if free is None:
+        busy.synchronize()
+        pytest.skip("no stream with a hardware queue of its own")
+    with torch.cuda.stream(free):
+        second = calls[1]()
+    free.synchronize()
+    waited = done.query()
+    busy.synchronize()
+    assert not waited, "the second call waited for the first one's stream"
+    for got, want in zip((first, second), serial):
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
 
 
 @pytest.mark.gpu
