@@ -144,7 +144,9 @@ def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is
     layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2], plan[3]
     if any(x // d < t for x, d, t in zip(layout, dilation, tiles[1])):
         tiles = choose_fitting_forward_tiles(layout, kernel_size, stride, dilation, is_causal)
-        if tiles is None:
+        # (other tiles than the plan looked at: their rows have to lie within the kernels' 32-bit offsets as well)
+        if tiles is None or not _lib.fused_layout_supported(layout, dilation, tiles[1], row_bytes=heads_kv * padded_head_dim(shape[-1]) * 2,
+                                                            q_tile_shape=tiles[0], dtype=dtype):
             return None
     if splits > 1:
         from .functional import _kv_tiles_per_q_tile

@@ -9,6 +9,7 @@ import torch
 from natten_amd import _lib
 from natten_amd.fna import _context_call_plan, amd_fna_with_context
 from natten_amd.functional import na1d, na2d, na3d
+from natten_amd.tile_config import choose_fitting_forward_tiles
 from oracle import c_oracle
 from oracle import na_oracle as O
 from tests.gpu_utils import assert_close, to_np
@@ -50,6 +51,16 @@ def reference(case, q, k, v, ck, cv):
 def test_the_cases_below_have_the_launch(case):
     shape, kernel, stride, dilation, causal, H, Hkv, D = case
     assert _context_call_plan(torch.bfloat16, (2, *shape, H, D), Hkv, kernel, stride, dilation, causal, None) is not None
+
+
+@pytest.mark.parametrize("shape,kernel,dilation", [((64, 7, 1000), (8, 5, 2), (2, 1, 1)), ((64, 5, 3000), (8, 5, 2), (2, 1, 1)),
+                                                   ((64, 7, 3000), (8, 3, 2), (1, 1, 1))])
+def test_tiles_that_span_too_much_merge_two(shape, kernel, dilation):
+    """Groups narrower than the cheapest KV tile, and the fitting one spans more than the launch addresses: no joint launch."""
+    ones, causal = (1, 1, 1), (False,) * 3
+    assert choose_fitting_forward_tiles(shape, kernel, ones, dilation, causal) is not None
+    assert _context_call_plan(torch.bfloat16, (1, *shape, 32, 128), 32, kernel, ones, dilation, causal, None) is None
+    assert _context_call_plan(torch.bfloat16, (1, *shape, 2, 128), 2, kernel, ones, dilation, causal, None) is not None
 
 
 @pytest.mark.gpu
