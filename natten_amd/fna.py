@@ -133,11 +133,11 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
 
 
 @functools.lru_cache(maxsize=1024)
-def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
+def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel, context: int = 64):
     """Tile shapes and kind of the launch over windows and context, or None.  Where the windows alone would be a split launch it is
     taken for up to 48 KV tiles a Q tile: a split launch, dense attention and two merges take the host 68 us and the device
     17 beside the split walk, the whole walk in one launch 1.05 us a tile (head dim 128; 2 x 30 x 40, 21 x 21, H 4 and 128
-    context tokens: 68 us so, 23 in one launch)."""
+    context tokens: 68 us so, 23 in one launch).  `context`: its tokens (see _joint_walk_pays)."""
     plan = _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel)
     if plan is None:
         return None
@@ -153,7 +153,33 @@ def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is
 
         if _kv_tiles_per_q_tile(layout, kernel_size, stride, dilation, *tiles) > 48:
             return None
+    if not _joint_walk_pays(shape, kernel_size, stride, dilation, tiles, context):
+        return None
     return (*tiles, persistent)
+
+
+def _joint_walk_pays(shape, kernel_size, stride, dilation, tiles, context: int) -> bool:
+    """Whether Q tiles of windows walk a context faster than a launch of dense attention and a merge take for it.  A joint walk
+    meets the context's tiles once per Q tile of the windows, padding queries included, and at Q tiles of 64 tokens a
+    quarter slower; what it saves are the launches, the merge and the way of one result through memory.  us of a call, two
+    launches / one: 2 x 17 x 33 x 9, H 16 (twice the Q tiles), D 64, 128 tokens 88 / 63, 512 105 / 98, 1024 124 / 153, 3072 201
+    / 344, D 128 1024 187 / 219; 2 x 13 x 37 x 21, H 16, D 128 (a third more) 1024 373 / 341, 2048 498 / 494, 3072 621 / 672; 2 x
+    64 x 64, H 16, D 64 (Q tiles of 64) 1024 79 / 71, 1536 95 / 92, 3072 143 / 158; 2 x 10000, H 16, D 128 3072 437 / 354.
+    Calls of under 55 us in one launch take the host longer than that in two."""
+    from .functional import _kv_tiles_per_q_tile
+
+    batch, layout, heads, head_dim = shape[0], shape[1:-2], shape[-2], shape[-1]
+    context_tiles = -(-context // 64)
+    q_tiles = batch * heads * (_prod(tiles[0]) / 128)
+    for x, d, t in zip(layout, dilation, tiles[0]):
+        q_tiles *= -(-(-(-x // d)) // t) * d
+    q_tiles *= 1.25 if _prod(tiles[0]) == 64 else 1.05
+    dense_q_tiles = batch * heads * -(-_prod(layout) // 128)
+    step = 0.35 + 0.0108 * head_dim  # us of a round of 512 Q tiles on a KV tile
+    walk = context_tiles + _kv_tiles_per_q_tile(layout, kernel_size, stride, dilation, *tiles)
+    if max(q_tiles / 512, 0.5) * step * walk + 5 <= 55:
+        return True
+    return context_tiles * step / 512 * (q_tiles - dense_q_tiles) <= 10 + 0.00022 * head_dim * dense_q_tiles
 
 
 def amd_fna_with_context(query: Tensor, key: Tensor, value: Tensor, context_key: Tensor, context_value: Tensor, kernel_size,
@@ -161,11 +187,11 @@ def amd_fna_with_context(query: Tensor, key: Tensor, value: Tensor, context_key:
     """Neighborhood attention whose queries also attend to context_key / context_value [B, N, Hkv, D] in one launch,
     forward only, on checked arguments that leave tiles and route open: (output, lse), or None where
     there is no such launch (contexts shorter than a KV tile, long split walks, dilation groups narrower than any KV
-    tile): the callers then merge two attentions."""
+    tile) or it is the slower way (long contexts): the callers then merge two attentions."""
     if context_key.shape[1] < 64 or query.dtype not in (torch.float16, torch.bfloat16) or torch_ops._tracing():
         return None
     plan = _context_call_plan(query.dtype, tuple(query.shape), key.shape[-2], kernel_size, stride, dilation, is_causal,
-                              run_persistent_kernel)
+                              run_persistent_kernel, context_key.shape[1])
     if plan is None:
         return None
     can_run_amd_fna(query, key, value, raise_error=True)

@@ -63,6 +63,21 @@ def test_tiles_that_span_too_much_merge_two(shape, kernel, dilation):
     assert _context_call_plan(torch.bfloat16, (1, *shape, 2, 128), 2, kernel, ones, dilation, causal, None) is not None
 
 
+def test_long_contexts_of_padded_q_tiles_merge_two():
+    """A joint walk meets the context once per Q tile of the windows: not where those are many more than dense attention's."""
+    def joint(batch, shape, heads, head_dim, kernel, context):
+        n = len(shape)
+        return _context_call_plan(torch.bfloat16, (batch, *shape, heads, head_dim), heads, kernel, (1,) * n, (1,) * n, (False,) * n,
+                                  None, context) is not None
+
+    for D in (32, 64, 96, 128):
+        for shape in ((17, 33, 9), (5, 5, 300), (13, 37, 21)):
+            assert joint(2, shape, 16, D, (3, 5, 5), 128) and not joint(2, shape, 16, D, (3, 5, 5), 3072)
+        assert joint(2, (10000,), 16, D, (200,), 3072) and joint(1, (30, 48, 40), 4, D, (3, 5, 5), 2048)
+        assert joint(2, (64, 64), 8, D, (13, 13), 128) and joint(2, (128, 128), 16, D, (7, 9), 1024)
+    assert not joint(2, (17, 33, 9), 16, 64, (3, 5, 5), 1024) and not joint(2, (64, 64), 16, 64, (7, 9), 4096)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("context", [64, 65, 77, 127, 128, 256, 4100])
