@@ -253,16 +253,10 @@ def choose_backward_role_tile_shapes(
 
 @functools.lru_cache(maxsize=4096)
 def _key_tile_dim_cost(L: int, k: int, s: int, causal: bool, tq: int, tk: int) -> Tuple[int, int]:
-    """_dim_cost of the dk / dv launch, whose key tiles may begin before the first key (choose_kv_shift in
-    csrc/fna_bwd.hpp, which has the last word on where)."""
-    plain = best = _dim_cost(L, k, s, causal, tq, tk)
-    if s > 1 and 1 < tk < L:
-        begin = s - k if causal else s // 2 - k // 2
-        for shift in {-begin % tk, -(begin + k) % tk, -L % tk}:
-            cost = _dim_cost(L, k, s, causal, tq, tk, False, shift)
-            if 1.3 * cost[0] - 0.3 * cost[1] < min(1.3 * best[0] - 0.3 * best[1], 0.95 * (1.3 * plain[0] - 0.3 * plain[1])):
-                best = cost
-    return best
+    """_dim_cost of the dk / dv launch, whose key tiles may begin before the first key: where the library lays them."""
+    from . import _lib
+
+    return _dim_cost(L, k, s, causal, tq, tk, False, _lib.key_tile_shift(L, k, s, causal, tk, tq) if s > 1 and tk > 1 else 0)
 
 
 @functools.lru_cache(maxsize=1024)
