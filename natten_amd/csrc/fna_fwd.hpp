@@ -437,9 +437,7 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
   t[0] = i;
 }
 
-// MQ 32-row query blocks per wave.  MQ = 1 runs two waves per SIMD (256 registers each);
-// MQ = 2 one wave per SIMD (512 registers: accumulators and Q fragments can sit in the
-// accumulation registers) and reads every K / V fragment from LDS once for two MFMAs.
+// One 32-row query block per wave, two or three waves per SIMD (fwd_max_waves).
 // RAGGED: seqlen_kv is not a multiple of KVT (dense attention on unpadded sequences); the tile
 // copies then clamp their rows and are issued at the top of an iteration instead of one per slot.
 // The work of one workgroup on one Q tile; `pid` is the position of that tile in the launch order
@@ -460,7 +458,7 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // window box, in the same walk.  Context as a launch of dense attention of its own and a merge write and read both
 // results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a
 // call 62 -> 31; 4 x 96 x 96, 24 x 24, H 16, D 128, 256 tokens: 665 -> 476).
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
           bool CTX = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
@@ -473,7 +471,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
   }
   constexpr int NT = NWAVES * 64;
-  constexpr int QT = NWAVES * MQ * 32;
+  constexpr int QT = NWAVES * 32;
   constexpr bool NARROW = DC != 0;
   constexpr int KSTEPS = (NARROW ? DC : D) / 16;
   constexpr int DB = (NARROW ? DC : D) / 32;
@@ -506,7 +504,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   //   sGeo[a]      KV tile extent along dimension a
   constexpr int MASK_ROWS = NOMASK ? 1 : KVT + 1;
   __shared__ __attribute__((aligned(16))) uint32_t sKeys[NOMASK ? 1 : 3][2][MASK_ROWS];
-  __shared__ __attribute__((aligned(16))) int sWin[NOMASK ? 1 : NWAVES * MQ * 32][8];
+  __shared__ __attribute__((aligned(16))) int sWin[NOMASK ? 1 : NWAVES * 32][8];
   //   sTile[wave * 64 + i]  the i-th described KV tile (see describe)
   __shared__ __attribute__((aligned(16))) int sTile[NOMASK ? 1 : NWAVES * 64][4];
   __shared__ __attribute__((aligned(16))) int sGeo[4];
@@ -620,7 +618,6 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // parameters one behind the other most of the 10000 cycles before a masked workgroup's first product.  With
   // touch_launch_params and results stored sixteen bytes per lane, us before / after: 4 x 128 x 128, 7 x 7, H 8, D 64 95.8 /
   // 87.0; 128 x 128, 32 x 32, stride 16, H 16, D 128 166 / 158; 32768 tokens, window 2048, H 1, D 128 48.7 / 46.4.
-  static_assert(MQ == 1, "a wave holds one box of queries");
   int box_org[3], box_n[3];  // box_org: coordinate of the box's first KV tile
   int wave_lo[3], wave_hi[3], wave_full_lo[3], wave_full_hi[3];
   int q_off[3];  // the lane's query inside the tile: its box's origin plus its place in the box
@@ -938,8 +935,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
 
   // ---- this lane's query row, on its way while the tables below are formed ---------------------------
-  int q_row[MQ];     // this lane's row of the permuted sequence / token offset in the group (fused), or -1
-  vec8 qf[MQ][KSTEPS];
+  int q_row;  // this lane's row of the permuted sequence / token offset in the group (fused), or -1
+  vec8 qf[KSTEPS];
   {
     int row = qtile_idx * QT + q_off[0] + p.q_tile[0] * (q_off[1] + p.q_tile[1] * q_off[2]);
     bool valid = row < seqlen_q;
@@ -957,12 +954,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
         row_c += na_min(c, extent[a] - 1) * tok_step[a];
       }
     }
-    q_row[0] = valid ? row : -1;
+    q_row = valid ? row : -1;
     const T* qrow = qbase + int64_t(row_c) * q_row_stride + g * 8;
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) {
-      qf[0][ks] = vec8{};
-      if (!NARROW || ks * 16 + g * 8 < row_dim) qf[0][ks] = *reinterpret_cast<const vec8*>(qrow + ks * 16);
+      qf[ks] = vec8{};
+      if (!NARROW || ks * 16 + g * 8 < row_dim) qf[ks] = *reinterpret_cast<const vec8*>(qrow + ks * 16);
     }
   }
   __builtin_amdgcn_sched_barrier(0);
@@ -991,19 +988,14 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // Rounding q' to the operand type moves a logit by about 2^-9 (bf16) / 2^-12 (fp16) of
   // |q||k| scale / sqrt(D) -- the size of the operands' own rounding.
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) qf[0][ks] = scale_query_fragment<T>(qf[0][ks], c_log2);
+  for (int ks = 0; ks < KSTEPS; ++ks) qf[ks] = scale_query_fragment<T>(qf[ks], c_log2);
 
-  f32x16_t acc[MQ][DB];
-  float m_run[MQ], l_run[MQ];
+  f32x16_t acc[DB];
+  float m_run = -INFINITY, l_run = 0.f;
 #pragma unroll
-  for (int mb = 0; mb < MQ; ++mb) {
-    m_run[mb] = -INFINITY;
-    l_run[mb] = 0.f;
+  for (int db = 0; db < DB; ++db)
 #pragma unroll
-    for (int db = 0; db < DB; ++db)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[mb][db][r] = 0.f;
-  }
+    for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
 
   // lane-constant LDS read offsets
   int k_off[KSTEPS];  // K operand: row l32 (+32*sb), chunk 2*ks+g
@@ -1021,9 +1013,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   for (int db = 0; db < DB; ++db) v_off[db] = uint32_t(v_row * ROWB + v_sub + L::v_slot(v_row, db * 4 + v_chunk) * 16);
 
   // ---- building blocks ---------------------------------------------------------------------------
-  // The lane owns query row l32 of each of its wave's MQ row blocks and, per 32-key sub-block,
+  // The lane owns query row l32 of its wave's row block and, per 32-key sub-block,
   // the 16 key rows 8*(r/4) + 4*g + r%4.  One "slot" below is one operand fragment read from
-  // LDS, the MQ MFMAs that use it, and the vector work that is to run in their shadow; slots are
+  // LDS, the MFMA that uses it, and the vector work that is to run in their shadow; slots are
   // fenced so that the compiler keeps that interleaving (a 32x32x16 MFMA occupies the matrix pipe
   // for 32 cycles but only one issue cycle, and up to six ordinary vector instructions of the
   // same wave issue behind it for free).
@@ -1048,70 +1040,66 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // Logits are kept in the exp2 domain and relative to the row's running maximum: the matrix
   // product starts from the accumulator value -m (sixteen registers per row block that only
   // change when the maximum moves), so the probabilities are exp2 of what the matrix pipe returns.
-  f32x16_t S_a[MQ][NSB], S_b[MQ][NSB];  // logits of the current / coming tile, swapping roles every iteration
-  vec8 pf[MQ][NSB][2];
-  f32x16_t c_init[MQ];          // -(running maximum), 0 while it is -inf: accumulator input of S = K Q^T
-  float psum[MQ][2];
+  f32x16_t S_a[NSB], S_b[NSB];  // logits of the current / coming tile, swapping roles every iteration
+  vec8 pf[NSB][2];
+  f32x16_t c_init;                // -(running maximum), 0 while it is -inf: accumulator input of S = K Q^T
+  float psum[2];
   if constexpr ((kAblate & kAblateSoftmax) != 0) {
     // probability-like operands (values in (0, 1]) in place of the ones the loop would form
 #pragma unroll
-    for (int mb = 0; mb < MQ; ++mb)
+    for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
-      for (int sb = 0; sb < NSB; ++sb)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int e = 0; e < 8; ++e)
-            pf[mb][sb][h][e] = static_cast<T>(fast_exp2(-fabsf(float(qf[mb][(sb * 2 + h) % KSTEPS][e]))));
+        for (int e = 0; e < 8; ++e)
+          pf[sb][h][e] = static_cast<T>(fast_exp2(-fabsf(float(qf[(sb * 2 + h) % KSTEPS][e]))));
   }
 
-  // Element e of the current tile's probabilities: row block e % MQ, logit v = e / MQ of the lane
-  // (sub-block v / 16, register v % 16): exp2(c*s - c*m), summed in float; every second
-  // element of a row block rounds its pair to T.
-  float held[MQ];
-  auto exp_elem = [&](const f32x16_t (&S_cur)[MQ][NSB], int e) {
+  // Element v of the current tile's probabilities: logit v of the lane (sub-block v / 16, register v % 16):
+  // exp2(c*s - c*m), summed in float; every second element rounds its pair to T.
+  float held;
+  auto exp_elem = [&](const f32x16_t (&S_cur)[NSB], int v) {
     if constexpr ((kAblate & kAblateSoftmax) != 0) {
-      asm volatile("" ::"v"(S_cur[e % MQ][(e / MQ) / 16][(e / MQ) % 16]));  // the logits stay in use
+      asm volatile("" ::"v"(S_cur[v / 16][v % 16]));  // the logits stay in use
       return;
     }
-    const int mb = e % MQ, v = e / MQ;
     const int sb = v / 16, r = v % 16;
-    float x = fast_exp2(S_cur[mb][sb][r]);
-    psum[mb][r & 1] += x;
+    float x = fast_exp2(S_cur[sb][r]);
+    psum[r & 1] += x;
     if (r % 2 == 0) {
       pin(x);
-      held[mb] = x;
+      held = x;
     } else {
-      vec2 p2 = {static_cast<T>(held[mb]), static_cast<T>(x)};
+      vec2 p2 = {static_cast<T>(held), static_cast<T>(x)};
       uint32_t bits = __builtin_bit_cast(uint32_t, p2);
       pin(bits);
       p2 = __builtin_bit_cast(vec2, bits);
-      pf[mb][sb][r / 8][r % 8 - 1] = p2[0];
-      pf[mb][sb][r / 8][r % 8] = p2[1];
+      pf[sb][r / 8][r % 8 - 1] = p2[0];
+      pf[sb][r / 8][r % 8] = p2[1];
     }
   };
   // Elements are spread evenly over the slots that precede the last 16-key block of O += P V
   // (whose P fragment is the last to be completed): cumulative count after global slot x.
-  constexpr int N_ELEMS = MQ * NSB * 16;
+  constexpr int N_ELEMS = NSB * 16;
   constexpr int EXP_SLOTS = N_QK + N_PV - DB;
   auto elems_done = [](int x) constexpr {
     const int n = (N_ELEMS * (x + 1) + EXP_SLOTS - 1) / EXP_SLOTS;
     return x < 0 ? 0 : (n > N_ELEMS ? N_ELEMS : n);
   };
 
-  // Element mask of a PARTIAL tile for row block mb.  Per dimension the lane's window, relative to the
+  // Element mask of a PARTIAL tile.  Per dimension the lane's window, relative to the
   // tile origin and clamped to the tile, selects two rows of sKeys (keys at or after its start, keys at
   // or after its end); the AND over the dimensions has one bit per logit of the lane: bit 16 sb + r
   // for logit r of sub-block sb.  A tile moved back from the group's edge starts before its place in
   // the tiling (the box origin plus a multiple of the tile extent): the keys up to there (`lead`)
   // belong to the tile before it.  All six rows are read at once (one register each), so that a
   // masked tile waits for LDS twice -- the windows, then the rows -- and not once per dimension.
-  auto mask_bits = [&](int mb, const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
+  auto mask_bits = [&](const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
     uint32_t bits = ~uint32_t(0);
     if constexpr (!NOMASK) {
       typedef int i32x4 __attribute__((ext_vector_type(4)));
       typedef int i32x2 __attribute__((ext_vector_type(2)));
-      const int row = (wave * MQ + mb) * 32 + l32;
+      const int row = wave * 32 + l32;
       const i32x4 w01 = *reinterpret_cast<const i32x4*>(&sWin[row][0]);
       const i32x2 w2 = *reinterpret_cast<const i32x2*>(&sWin[row][4]);
       const int ws[3] = {w01[0], w01[2], w2[0]}, we[3] = {w01[1], w01[3], w2[1]};
@@ -1141,9 +1129,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const uint32_t bits = __builtin_bit_cast(uint32_t, logit);
     S[sb][r] = __builtin_bit_cast(float, (bits & keep) | (~keep & 0xff800000u));
   };
-  auto apply_mask = [&](f32x16_t (&S)[NSB], int mb, const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
+  auto apply_mask = [&](f32x16_t (&S)[NSB], const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
     if constexpr (!NOMASK) {
-      uint32_t lane_bits = mask_bits(mb, origin, lead);
+      uint32_t lane_bits = mask_bits(origin, lead);
       // (a context tile holds no coordinates: what the line above made of its row is replaced)
       if constexpr (CTX) lane_bits = origin[0] == kCtxTile ? na_lane_half_bits(~na_ones64(lead[0]), g) : lane_bits;
 #pragma unroll
@@ -1156,73 +1144,69 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // adopts the maximum `mx` of the lane's half row of the coming tile (relative to the running
   // maximum, like the logits `S` themselves): the running maximum is only moved (and the logits of
   // that tile, O and the row sum shifted / rescaled) when some row of the wave outgrew it by 2^8
-  auto update_max = [&](int mb, float mx, f32x16_t (&S)[NSB]) __attribute__((always_inline)) {
+  auto update_max = [&](float mx, f32x16_t (&S)[NSB]) __attribute__((always_inline)) {
     mx = cross_half_max(mx);
-    const bool first = (m_run[mb] == -INFINITY) && (mx != -INFINITY);
+    const bool first = (m_run == -INFINITY) && (mx != -INFINITY);
     const bool grow = first || (mx > kLazyRescaleLog2);
     if (__builtin_expect(__any(grow), 0)) {
       // rows still at -inf take their first maximum as it is (it may be negative) and have
       // nothing accumulated yet; the others only grow
-      const bool was_inf = m_run[mb] == -INFINITY;
+      const bool was_inf = m_run == -INFINITY;
       const float shift = was_inf ? ((mx == -INFINITY) ? 0.f : mx) : fmaxf(mx, 0.f);
       const float alpha = was_inf ? 1.f : fast_exp2(-shift);
-      if (mx != -INFINITY) m_run[mb] = (was_inf ? 0.f : m_run[mb]) + shift;
-      l_run[mb] *= alpha;
+      if (mx != -INFINITY) m_run = (was_inf ? 0.f : m_run) + shift;
+      l_run *= alpha;
 #pragma unroll
       for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[mb][db][r] *= alpha;
+        for (int r = 0; r < 16; ++r) acc[db][r] *= alpha;
 #pragma unroll
       for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) S[sb][r] -= shift;
-      const float c = (m_run[mb] == -INFINITY) ? 0.f : -m_run[mb];
+      const float c = (m_run == -INFINITY) ? 0.f : -m_run;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) c_init[mb][r] = c;
+      for (int r = 0; r < 16; ++r) c_init[r] = c;
     }
     // one home for the sixteen registers on both paths (otherwise the compiler keeps a second
     // copy of them alive and copies one to the other in every iteration)
-    asm volatile("" : "+v"(c_init[mb]));
+    asm volatile("" : "+v"(c_init));
   };
   // masks (PARTIAL tiles) and maxima of a whole tile of logits, outside the slots
   // (`l`: place of the tile among the described ones)
-  auto finish_logits = [&](f32x16_t (&S)[MQ][NSB], int l, bool have_max, const float (&mx_in)[MQ]) __attribute__((always_inline)) {
+  auto finish_logits = [&](f32x16_t (&S)[NSB], int l, bool have_max, float mx) __attribute__((always_inline)) {
     // One test on the way of a tile that needs nothing (attended in full, maxima at hand): every
     // wave-uniform branch in the tile loop costs about a hundredth of its time.
     const bool full = (d_plain >> l) & 1;
     const bool plain = full && have_max;
+    if (__builtin_expect(!plain, 0)) {
+      if ((d_skip >> l) & 1) {
+        // none of this wave's queries attends the tile: every logit is masked
+        mx = -INFINITY;
 #pragma unroll
-    for (int mb = 0; mb < MQ; ++mb) {
-      float mx = mx_in[mb];
-      if (__builtin_expect(!plain, 0)) {
-        if ((d_skip >> l) & 1) {
-          // none of this wave's queries attends the tile: every logit is masked
-          mx = -INFINITY;
+        for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
-          for (int sb = 0; sb < NSB; ++sb)
+          for (int r = 0; r < 16; ++r) S[sb][r] = -INFINITY;
+      } else {
+        if (!full) {
+          int origin[3], lead[3];
+          typedef int i32x4 __attribute__((ext_vector_type(4)));
+          const i32x4 tile = *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) S[mb][sb][r] = -INFINITY;
-        } else {
-          if (!full) {
-            int origin[3], lead[3];
-            typedef int i32x4 __attribute__((ext_vector_type(4)));
-            const i32x4 tile = *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-              origin[a] = tile[a];
-              lead[a] = (tile[3] >> (8 * a)) & 255;
-            }
-            apply_mask(S[mb], mb, origin, lead);
+          for (int a = 0; a < 3; ++a) {
+            origin[a] = tile[a];
+            lead[a] = (tile[3] >> (8 * a)) & 255;
           }
-          mx = -INFINITY;
-#pragma unroll
-          for (int sb = 0; sb < NSB; ++sb)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[mb][sb][r]);
+          apply_mask(S, origin, lead);
         }
+        mx = -INFINITY;
+#pragma unroll
+        for (int sb = 0; sb < NSB; ++sb)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, S[sb][r]);
       }
-      update_max(mb, mx, S[mb]);
     }
+    update_max(mx, S);
   };
 
   // ---- software pipeline --------------------------------------------------------------------
@@ -1236,24 +1220,18 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   at_tile(1, kbase, ld_koff, p.ctx_k, KLayout{});
   if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, 1, KLayout{});
 #pragma unroll
-  for (int mb = 0; mb < MQ; ++mb)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) c_init[mb][r] = 0.f;
+  for (int r = 0; r < 16; ++r) c_init[r] = 0.f;
   {
 #pragma unroll
-    for (int mb = 0; mb < MQ; ++mb)
+    for (int sb = 0; sb < NSB; ++sb)
 #pragma unroll
-      for (int sb = 0; sb < NSB; ++sb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) S_a[mb][sb][r] = 0.f;
+      for (int r = 0; r < 16; ++r) S_a[sb][r] = 0.f;
 #pragma unroll
     for (int s = 0; s < N_QK; ++s) {
       const vec8 kf = k_frag(sK0, s);
-#pragma unroll
-      for (int mb = 0; mb < MQ; ++mb) S_a[mb][s / KSTEPS] = M::run(kf, qf[mb][s % KSTEPS], S_a[mb][s / KSTEPS]);
+      S_a[s / KSTEPS] = M::run(kf, qf[s % KSTEPS], S_a[s / KSTEPS]);
     }
-    const float none[MQ] = {};
-    finish_logits(S_a, 0, false, none);
+    finish_logits(S_a, 0, false, 0.f);
   }
 
   // CUR / NXT: this wave attends keys of tile j / tile j + 1; an inactive tile only takes part
@@ -1262,8 +1240,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     constexpr int st = decltype(stage_tag)::value;
     constexpr bool CUR = decltype(cur_tag)::value, NXT = decltype(nxt_tag)::value;
     constexpr bool SPREAD = !RAGGED;
-    f32x16_t (&S_cur)[MQ][NSB] = st ? S_b : S_a;
-    f32x16_t (&S_nxt)[MQ][NSB] = st ? S_a : S_b;
+    f32x16_t (&S_cur)[NSB] = st ? S_b : S_a;
+    f32x16_t (&S_nxt)[NSB] = st ? S_a : S_b;
     char* sK_cur = st ? sK1 : sK0;  // held K(j): free, receives K(j+2)
     char* sK_nxt = st ? sK0 : sK1;  // holds K(j+1)
     char* sV_cur = st ? sV1 : sV0;  // holds V(j)
@@ -1294,8 +1272,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 #pragma unroll
       for (int s = 0; s < PF_K; ++s) kf[s] = k_frag(sK_nxt, s);
     }
-#pragma unroll
-    for (int mb = 0; mb < MQ; ++mb) psum[mb][0] = psum[mb][1] = 0.f;
+    psum[0] = psum[1] = 0.f;
     auto g1_slot = [&](auto s_tag) __attribute__((always_inline)) {
       constexpr int s = decltype(s_tag)::value;
       if constexpr (NXT) {
@@ -1303,24 +1280,18 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           if constexpr ((kAblate & kAblateLdsReads) == 0 || s + PF_K < 4) kf[s + PF_K] = k_frag(sK_nxt, s + PF_K);
           else kf[s + PF_K] = kf[(s + PF_K) % 4];
         }
-#pragma unroll
-        for (int mb = 0; mb < MQ; ++mb) {
-          if constexpr (s % KSTEPS == 0) {
-            S_nxt[mb][s / KSTEPS] = M::run_from(kf[s], qf[mb][s % KSTEPS], c_init[mb]);
-          } else {
-            S_nxt[mb][s / KSTEPS] = M::run(kf[s], qf[mb][s % KSTEPS], S_nxt[mb][s / KSTEPS]);
-          }
+        if constexpr (s % KSTEPS == 0) {
+          S_nxt[s / KSTEPS] = M::run_from(kf[s], qf[s % KSTEPS], c_init);
+        } else {
+          S_nxt[s / KSTEPS] = M::run(kf[s], qf[s % KSTEPS], S_nxt[s / KSTEPS]);
         }
       }
       constexpr int e_lo = elems_done(s - 1), e_hi = elems_done(s);
       if constexpr (CUR && e_hi > e_lo) {
 #pragma unroll
         for (int e = e_lo; e < e_hi; ++e) exp_elem(S_cur, e);
-#pragma unroll
-        for (int mb = 0; mb < MQ; ++mb) {
-          pin(psum[mb][0]);
-          pin(psum[mb][1]);
-        }
+        pin(psum[0]);
+        pin(psum[1]);
       }
       if constexpr (SPREAD && (kAblate & kAblateCopies) == 0) {
         // 2 * PER copies spread over the first half of the slots, K first
@@ -1347,63 +1318,46 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 #pragma unroll
       for (int t = 0; t < PF_V; ++t) vf[t] = v_frag(sV_cur, t);
     }
-    float mx[MQ][2];
-#pragma unroll
-    for (int mb = 0; mb < MQ; ++mb) mx[mb][0] = mx[mb][1] = -INFINITY;
+    float mx[2] = {-INFINITY, -INFINITY};
     auto pv_slot = [&](auto t_tag) __attribute__((always_inline)) {
       constexpr int t = decltype(t_tag)::value;
       // the P fragment of this slot's 16-key block is complete
-      static_assert(elems_done(N_QK + (t / DB) * DB - 1) >= MQ * 8 * (t / DB + 1), "exponentials scheduled too late");
+      static_assert(elems_done(N_QK + (t / DB) * DB - 1) >= 8 * (t / DB + 1), "exponentials scheduled too late");
       constexpr int x_lo = elems_done(N_QK + t - 1), x_hi = elems_done(N_QK + t);
       if constexpr (CUR) {
         if constexpr (t + PF_V < N_PV) {
           if constexpr ((kAblate & kAblateLdsReads) == 0 || t + PF_V < 4) vf[t + PF_V] = v_frag(sV_cur, t + PF_V);
           else vf[t + PF_V] = vf[(t + PF_V) % 4];
         }
-#pragma unroll
-        for (int mb = 0; mb < MQ; ++mb)
-          acc[mb][t % DB] = M::run(vf[t], pf[mb][t / (2 * DB)][(t / DB) % 2], acc[mb][t % DB]);
+        acc[t % DB] = M::run(vf[t], pf[t / (2 * DB)][(t / DB) % 2], acc[t % DB]);
         if constexpr (x_hi > x_lo) {
 #pragma unroll
           for (int e = x_lo; e < x_hi; ++e) exp_elem(S_cur, e);
-#pragma unroll
-          for (int mb = 0; mb < MQ; ++mb) {
-            pin(psum[mb][0]);
-            pin(psum[mb][1]);
-          }
+          pin(psum[0]);
+          pin(psum[1]);
         }
       }
       if constexpr (NXT && t >= N_PV / 2 && (kAblate & kAblateMax) == 0) {
-        // row maxima of the coming tile (as if unmasked), MQ * NSB * 16 values over N_PV / 2 slots
+        // row maxima of the coming tile (as if unmasked), NSB * 16 values over N_PV / 2 slots
         constexpr int t3 = t - N_PV / 2;
-        constexpr int NV = MQ * NSB * 16;
+        constexpr int NV = NSB * 16;
         constexpr int e_lo = (t3 * NV) / (N_PV / 2), e_hi = ((t3 + 1) * NV) / (N_PV / 2);
 #pragma unroll
         for (int e = e_lo; e < e_hi; ++e) {
-          const int mb = e / (NSB * 16), i = e % (NSB * 16);
-          mx[mb][i % 2] = fmaxf(mx[mb][i % 2], S_nxt[mb][i / 16][i % 16]);
+          mx[e % 2] = fmaxf(mx[e % 2], S_nxt[e / 16][e % 16]);
         }
         if constexpr (e_hi > e_lo) {
-#pragma unroll
-          for (int mb = 0; mb < MQ; ++mb) {
-            pin(mx[mb][0]);
-            pin(mx[mb][1]);
-          }
+          pin(mx[0]);
+          pin(mx[1]);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
     };
     if constexpr (CUR || NXT) for_range<0, N_PV>(pv_slot);
-    if constexpr (CUR) {
-#pragma unroll
-      for (int mb = 0; mb < MQ; ++mb) l_run[mb] += psum[mb][0] + psum[mb][1];
-    }
+    if constexpr (CUR) l_run += psum[0] + psum[1];
 
     if ((kAblate & kAblateMax) == 0 && NXT && j + 1 < total_tiles) {
-      float mxs[MQ];
-#pragma unroll
-      for (int mb = 0; mb < MQ; ++mb) mxs[mb] = fmaxf(mx[mb][0], mx[mb][1]);
-      finish_logits(S_nxt, j + 1 - d_first, true, mxs);
+      finish_logits(S_nxt, j + 1 - d_first, true, fmaxf(mx[0], mx[1]));
     }
     nxt = t2;
   };
@@ -1423,21 +1377,18 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   if constexpr (SPLIT) {
     if (empty_split) {
       // (not by a factor of 0, which would leave NaN where the tile walked holds infinities)
+      l_run = 0.f;
 #pragma unroll
-      for (int mb = 0; mb < MQ; ++mb) {
-        l_run[mb] = 0.f;
+      for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[mb][db][r] = 0.f;
-      }
+        for (int r = 0; r < 16; ++r) acc[db][r] = 0.f;
     }
     if (p.split_first < 0) {
       obase += split * p.o_split_stride;
       lse_base += split * p.lse_split_stride;
     } else if (splits > 1) {
       const int64_t row = (int64_t(pid - p.split_first) * splits + split) * QT + wave * 32 + l32;
-      const float l = l_run[0] + __shfl_xor(l_run[0], 32);
+      const float l = l_run + __shfl_xor(l_run, 32);
       const float inv = (l > 0.f) ? out_scale / l : 0.f;
       float* part = p.split_parts + row * row_dim + 4 * g;
 #pragma unroll
@@ -1446,26 +1397,20 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
         for (int j = 0; j < 4; ++j) {
           f32x4_t o4;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o4[i] = acc[0][db][4 * j + i] * inv;
+          for (int i = 0; i < 4; ++i) o4[i] = acc[db][4 * j + i] * inv;
           if (!NARROW || db * 32 + 8 * j < row_dim) *reinterpret_cast<f32x4_t*>(part + db * 32 + 8 * j) = o4;
         }
       // (a sum that is NaN reaches the merge as such: a part of weight 0 would leave the row the LSE of the other parts)
-      if (g == 0) p.split_lse[row] = (l > 0.f) ? (m_run[0] * 0.6931471805599453f + __logf(l)) : (l == 0.f) ? -INFINITY : l;
+      if (g == 0) p.split_lse[row] = (l > 0.f) ? (m_run * 0.6931471805599453f + __logf(l)) : (l == 0.f) ? -INFINITY : l;
       return;
     }
   }
-#pragma unroll
-  for (int mb = 0; mb < MQ; ++mb) {
-    const float l = l_run[mb] + __shfl_xor(l_run[mb], 32);
-    const float inv = (l > 0.f) ? out_scale / l : 0.f;
-    const int row = q_row[mb];
-    store_row_blocks<T, DB>(obase + int64_t(na_max(row, 0)) * q_row_stride, acc[mb], inv, g, row >= 0, row_dim);
-    if (row >= 0) {
-      if (g == 0) {
-        const float lse = (l > 0.f) ? (m_run[mb] * 0.6931471805599453f + __logf(l)) : -INFINITY;
-        lse_base[(q_row_base + row) * p.heads_q + head] = lse;
-      }
-    }
+  const float l = l_run + __shfl_xor(l_run, 32);
+  const float inv = (l > 0.f) ? out_scale / l : 0.f;
+  store_row_blocks<T, DB>(obase + int64_t(na_max(q_row, 0)) * q_row_stride, acc, inv, g, q_row >= 0, row_dim);
+  if (q_row >= 0 && g == 0) {
+    const float lse = (l > 0.f) ? (m_run * 0.6931471805599453f + __logf(l)) : -INFINITY;
+    lse_base[(q_row_base + q_row) * p.heads_q + head] = lse;
   }
 }
 
@@ -1526,9 +1471,9 @@ static __device__ __forceinline__ void clear_uncovered_rows(const FnaParams& p, 
   }
 }
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
 __global__ void __launch_bounds__(NWAVES * 64)
-    __attribute__((amdgpu_waves_per_eu(MQ == 1 ? fwd_min_waves(D, NOMASK) : 1, MQ == 1 ? fwd_max_waves(D, NOMASK) : 1)))
+    __attribute__((amdgpu_waves_per_eu(fwd_min_waves(D, NOMASK), fwd_max_waves(D, NOMASK))))
 fna_fwd_kernel(const FnaParams p) {
   touch_launch_params<sizeof(FnaParams)>();
   if constexpr (RAGGED) {
@@ -1537,7 +1482,7 @@ fna_fwd_kernel(const FnaParams p) {
       return;
     }
   }
-  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, DC, CTX>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, false, NOMASK, DC, CTX>(p, int(blockIdx.x), []() {});
 }
 
 // Split launch: kv_splits workgroups per Q tile, each on a contiguous run of the tile's KV tiles,
@@ -1545,11 +1490,11 @@ fna_fwd_kernel(const FnaParams p) {
 // fewer Q tiles than the chip keeps workgroups resident: a lone workgroup's tile loop is bound by
 // its own instruction issue, not by anything it shares, so two on half the tiles each take about
 // half the time.
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, int DC = 0>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, int DC = 0>
+__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fna_fwd_split_kernel(const FnaParams p) {
   touch_launch_params<sizeof(FnaParams)>();
-  fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
 }
 
 // Combines the partial results of a dense split launch, sixteen rows of a Q tile per workgroup, four columns per lane:
@@ -1688,12 +1633,12 @@ static __device__ __forceinline__ void fna_queue_loop(uint32_t* __restrict__ que
   }
 }
 
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, bool CTX = false>
-__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(MQ == 1 ? 2 : 1, MQ == 1 ? 2 : 1)))
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool NOMASK = false, bool CTX = false>
+__global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 fna_fwd_queue_kernel(const FnaParams p, uint32_t* __restrict__ queues, const int per_xcd) {
   FnaKernargPtr args = fna_kernarg_params();
   fna_queue_loop(queues, per_xcd, [&](int pid, auto& fetch) __attribute__((always_inline)) {
-    fna_fwd_tile<T, D, NWAVES, MQ, RAGGED, KVT, false, NOMASK, 0, CTX>(fna_params_for_this_tile(args), pid, fetch);
+    fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, false, NOMASK, 0, CTX>(fna_params_for_this_tile(args), pid, fetch);
   });
   (void)p;
 }

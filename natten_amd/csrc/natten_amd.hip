@@ -89,9 +89,9 @@ struct WorkQueue {
 };
 
 // DC != 0: rows of p.row_dim elements, DC columns multiplied (no work-queue launch)
-template <typename T, int D, int NWAVES, int MQ, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
 int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
-  constexpr int QT = NWAVES * MQ * 32;
+  constexpr int QT = NWAVES * 32;
   if (!fna_tiles_are_powers_of_two(p)) return fail("fna_forward: tile extents must be powers of two");
   if ((p.seqlen_q + QT - 1) / QT != p.num_q_tiles) return fail("fna_forward: internal tile count mismatch");
   const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
@@ -100,7 +100,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
     if (queues.counters != nullptr) {
       const long long resident = resident_workgroups();
       if (queues.clear_first) hipLaunchKernelGGL(fna_queue_clear_kernel, dim3(1), dim3(kQueueWords), 0, stream, queues.counters);
-      hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, CTX>),
+      hipLaunchKernelGGL((fna_fwd_queue_kernel<T, D, NWAVES, RAGGED, KVT, NOMASK, CTX>),
                          dim3((unsigned)(wgs < resident ? wgs : resident)), dim3(NWAVES * 64), 0, stream, p, queues.counters,
                          int(wgs / kNumXcd));
       return check_launch("fna_forward (work queue)");
@@ -108,12 +108,12 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   }
   if (p.kv_splits > 1) {
     // kv_splits workgroups per Q-tile position, split slowest (positions keep their XCDs: wgs is a multiple of 8)
-    if constexpr (NWAVES == 4 && MQ == 1 && KVT == 64 && !CTX) {
+    if constexpr (NWAVES == 4 && KVT == 64 && !CTX) {
       if (wgs * p.kv_splits > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
       FnaParams ps = p;
       if (p.split_first < 0) {
         ps.split_grid = int(wgs);
-        hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>), dim3((unsigned)(wgs * p.kv_splits)),
+        hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, RAGGED, KVT, DC>), dim3((unsigned)(wgs * p.kv_splits)),
                            dim3(NWAVES * 64), 0, stream, ps);
         return check_launch("fna_forward (split)");
       }
@@ -121,7 +121,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
       if (p.split_grid < kNumXcd || p.split_grid % kNumXcd != 0 || p.split_grid > wgs)
         return fail("fna_forward: the split positions must be a multiple of %d up to %lld, got %d", kNumXcd, wgs, p.split_grid);
       ps.split_first = int(wgs) - p.split_grid;
-      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, MQ, RAGGED, KVT, DC>),
+      hipLaunchKernelGGL((fna_fwd_split_kernel<T, D, NWAVES, RAGGED, KVT, DC>),
                          dim3((unsigned)(ps.split_first + p.split_grid * p.kv_splits)), dim3(NWAVES * 64), 0, stream, ps);
       if (int rc = check_launch("fna_forward (split)")) return rc;
       hipLaunchKernelGGL((merge_tail_kernel<T>), dim3((unsigned)p.split_grid * 8), dim3(256), 0, stream, ps);
@@ -137,7 +137,7 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
     pk.split_first = int(wgs);
     if (wgs + clearing > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
   }
-  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, MQ, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)(wgs + clearing)),
+  hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)(wgs + clearing)),
                      dim3(NWAVES * 64), 0, stream, pk);
   return check_launch("fna_forward");
 }
@@ -210,24 +210,24 @@ template <typename T, int D>
 int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, WorkQueue queues) {
   if (p.has_context()) {
     if (context_launch_fits(p, kvt)) {
-      if (qt == 128) return launch_fna<T, D, 4, 1, false, 64, false, 0, true>(p, stream, queues);
+      if (qt == 128) return launch_fna<T, D, 4, false, 64, false, 0, true>(p, stream, queues);
       if constexpr (D <= 64) {
-        if (qt == 64 && queues.counters == nullptr) return launch_fna<T, D, 2, 1, false, 64, false, 0, true>(p, stream);
+        if (qt == 64 && queues.counters == nullptr) return launch_fna<T, D, 2, false, 64, false, 0, true>(p, stream);
       }
     }
     return fail("fna_forward: no kernel with a context for these tiles and extents (Q tile %d, KV tile %d, head_dim %d)", qt, kvt, D);
   }
   if (needs_clamped_rows(p, kvt)) {
-    if (qt == 128 && kvt == 64) return launch_fna<T, D, 4, 1, true, 64>(p, stream);
+    if (qt == 128 && kvt == 64) return launch_fna<T, D, 4, true, 64>(p, stream);
     return fail("fna_forward: seqlen_kv (%d) must be a multiple of the KV tile (%d tokens)", p.seqlen_kv, kvt);
   }
   // the work-queue launch exists for the default tile pair; the others launch a workgroup per Q tile
   if (qt == 128 && kvt == 64) {
-    if (fully_block_sparse(p)) return launch_fna<T, D, 4, 1, false, 64, true>(p, stream, queues);
-    return launch_fna<T, D, 4, 1, false, 64>(p, stream, queues);
+    if (fully_block_sparse(p)) return launch_fna<T, D, 4, false, 64, true>(p, stream, queues);
+    return launch_fna<T, D, 4, false, 64>(p, stream, queues);
   }
-  if (qt == 256 && kvt == 64) return launch_fna<T, D, 8, 1, false, 64>(p, stream);
-  if (qt == 64 && kvt == 64) return launch_fna<T, D, 2, 1, false, 64>(p, stream);
+  if (qt == 256 && kvt == 64) return launch_fna<T, D, 8, false, 64>(p, stream);
+  if (qt == 64 && kvt == 64) return launch_fna<T, D, 2, false, 64>(p, stream);
   return fail("fna_forward: no kernel for Q tile of %d and KV tile of %d tokens", qt, kvt);
 }
 
@@ -235,9 +235,9 @@ int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, Work
 // 96: a quarter of the matrix work and of the LDS reads less.
 template <typename T, bool RAGGED, bool CTX = false>
 int dispatch_narrow_rows(const FnaParams& p, int head_dim, hipStream_t stream) {
-  if (head_dim < 64) return launch_fna<T, 64, 4, 1, RAGGED, 64, false, 64, CTX>(p, stream);
-  if (head_dim <= 96) return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 96, CTX>(p, stream);
-  return launch_fna<T, 128, 4, 1, RAGGED, 64, false, 128, CTX>(p, stream);
+  if (head_dim < 64) return launch_fna<T, 64, 4, RAGGED, 64, false, 64, CTX>(p, stream);
+  if (head_dim <= 96) return launch_fna<T, 128, 4, RAGGED, 64, false, 96, CTX>(p, stream);
+  return launch_fna<T, 128, 4, RAGGED, 64, false, 128, CTX>(p, stream);
 }
 
 template <typename T>
