@@ -794,11 +794,12 @@ def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int,
     query tiles of 64 that the longest of them meets, `equal`: sequences of one length.  Figures with 256 compute units.
     Taken where the compute units stand idle for 20 of those steps (1.6 us) and a tenth of the time or more on the average:
     the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic.  us of both launches and the pass
-    before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 322 / 259 (62),
-    5 up to 1527, H 4 95 / 75 (20), 16 of 512, H 16 / 4 150 / 157 (16), 7 up to 384, H 8 / 4 58 / 65 (11), 9 up to 176, H 16 37 / 81 (3);
+    before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 310 / 255 (62),
+    5 up to 1527, H 4 97 / 76 (18), 16 of 512, H 16 / 4 152 / 157 (16), 7 up to 384, H 8 / 4 60 / 69 (11), 9 up to 176, H 16 44 / 70 (3);
     1 x 2000 causal, H 16 / 4 248 / 209 (112), 1 x 9000 full, H 8 / 4 1431 / 1067 (251), H 16 2150 / 2095 (79), 2 x 2176 full,
     H 16 336 / 290 (30), 2 x 4096 full, H 16 / 8 814 / 902 (0), 2 x 3000 causal, H 8 181 / 203 (12), 2 x 3809
-    full, H 24 1146 / 1160 (22 of 360).  Of 39 problems it is taken for 18, which are 1 to 25 % faster."""
+    full, H 24 1146 / 1160 (22 of 360).  Of 60 random problems that it is taken for, 59 are 3 to 59 % faster and one 5 % slower (1 x 6051
+    full, H 8 / 4: 541 / 572, 192 key tiles in one round)."""
     if head_dim != 128:
         return False
     work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / compute_units

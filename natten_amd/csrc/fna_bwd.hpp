@@ -186,7 +186,7 @@ inline int choose_kv_shift(int L, int k, int s, bool causal, int tile, int q_sub
 // FnaBwdParams::roles: the dQ launch runs beside the dK / dV launch, on a stream of its own (dq is not the workspace that the
 // other one reads).  That launch lasts as long as its longest workgroup, and while that walks its query tiles most
 // compute units have nothing left to do: both launches of a packed step, 10 sequences of 1 .. 2048, H 16 / 4, D 128, with
-// the pass before, 317 us one behind the other and 256 side by side; the callers know where it pays.
+// the pass before, 310 us one behind the other and 255 side by side; the callers know where it pays.
 constexpr int kBwdOverlap = 16;
 
 enum BwdRole : int { kBwdDQ = 0, kBwdDKV = 1, kBwdPair = 2 };

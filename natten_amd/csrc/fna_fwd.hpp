@@ -91,7 +91,7 @@ struct FnaParams {
   // Tile extents are powers of two (log2 below); the other divisors get multiply-shift pairs.
   int q_tile_lg[3], kv_tile_lg[3];
   // log2 extents of the box of 32 queries that a wave's lanes hold (sum 5, each <= q_tile_lg): the Q
-  // tile is a grid of such boxes, one per wave and row block.  Chosen per launch (choose_wave_box) so
+  // tile is a grid of such boxes, one per wave.  Chosen per launch (choose_wave_box) so
   // that as many (wave, KV tile) pairs as possible need no element mask.
   int wave_box_lg[3];
   int ext_base[3], ext_rem[3];  // qkv_shape / dil and qkv_shape % dil: extent of dilation group g = base + (g < rem)
@@ -1038,7 +1038,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   };
 
   // Logits are kept in the exp2 domain and relative to the row's running maximum: the matrix
-  // product starts from the accumulator value -m (sixteen registers per row block that only
+  // product starts from the accumulator value -m (sixteen registers that only
   // change when the maximum moves), so the probabilities are exp2 of what the matrix pipe returns.
   f32x16_t S_a[NSB], S_b[NSB];  // logits of the current / coming tile, swapping roles every iteration
   vec8 pf[NSB][2];

@@ -73,6 +73,12 @@ def attention(
     `[batch, seqlen, heads]` when `return_lse=True`.  For e4m3 / e5m2 operands `q_scale`, `k_scale`,
     `v_scale` (number or per-head tensor) are the dequantisation scales and `out_dtype` the
     result type (default: the operands' type, as in the reference).
+
+    Results are the same from call to call.  From a batch of two on, where the last workgroups would leave most
+    of the chip idle, their key walks are split and the parts summed in float: the entries of such a batch
+    may then differ from each other, and from a call on one entry alone, in the order of summation (by
+    about one rounding of the result).  Batches of one and packed sequences are never split: those give each
+    other's bits.
     """
     fmha_tensor_checks(query, key, value, must_match_head_dims=True)
     cumulative_seqlen_Q, cumulative_seqlen_KV, max_seqlen_Q, max_seqlen_KV = varlen_tensor_checks(
