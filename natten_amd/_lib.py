@@ -788,10 +788,11 @@ def _compute_units(device_index: int) -> int:
 
 
 def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int, is_causal: bool, equal: bool,
-                               compute_units: int = 256) -> bool:
+                               compute_units: int = 256, longest_query: Optional[int] = None) -> bool:
     """Whether the dq launch of dense attention runs beside the dk / dv launch (head dim 128: a workgroup per compute
     unit), which then has a workspace for the scaled queries besides dq.  `key_tiles` over all heads, `longest_walk`:
-    query tiles of 64 that the longest of them meets, `equal`: sequences of one length.  Figures with 256 compute units.
+    query tiles of 64 that the longest of them meets (over the query heads of a key head), `longest_query`: of one head (None:
+    as many), `equal`: sequences of one length.  Figures with 256 compute units.
     Taken where the compute units stand idle for 20 of those steps (1.6 us) and a tenth of the time or more on the average:
     the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic.  us of both launches and the pass
     before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 310 / 255 (62),
@@ -799,12 +800,17 @@ def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int,
     1 x 2000 causal, H 16 / 4 248 / 209 (112), 1 x 9000 full, H 8 / 4 1431 / 1067 (251), H 16 2150 / 2095 (79), 2 x 2176 full,
     H 16 336 / 290 (30), 2 x 4096 full, H 16 / 8 814 / 902 (0), 2 x 3000 causal, H 8 181 / 203 (12), 2 x 3809
     full, H 24 1146 / 1160 (22 of 360).  Of 60 random problems that it is taken for, 59 are 3 to 59 % faster and one 5 % slower (1 x 6051
-    full, H 8 / 4: 541 / 572, 192 key tiles in one round)."""
+    full, H 8 / 4: 541 / 572, 192 key tiles in one round).
+    The second stream also takes the host 41 us a call, and a training step on one attention takes it 140 to 175 without: steps whose launches
+    are over by then only get longer (us, forward and backward: 2 x 944 full, H 2 / 1 143 / 184; 5 up to 952, H 16 / 4 173 / 219;
+    1 x 2906 causal, H 4 197 / 206; 4 x 2157 full, H 2 / 1 207 / 206; 3 up to 3143, H 4 223 / 198; 2 x 1532 full, H 4 / 1 228 / 209).  So
+    the launches of a step have to add up to 210 us: 1.6 a step of the key-stationary walk, 2.2 a step of the forward's and dQ's."""
     if head_dim != 128:
         return False
     work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / compute_units
     span = max(longest_walk, work) if is_causal or not equal else longest_walk * _ceil_div(key_tiles, compute_units)
-    return span - work >= max(20, span / 10)
+    step_us = 30 + 1.6 * span + 2.2 * (longest_walk if longest_query is None else longest_query)
+    return span - work >= max(20, span / 10) and step_us >= 210
 
 
 def attention_backward(
@@ -818,7 +824,7 @@ def attention_backward(
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     overlap = _backward_launches_overlap(q.shape[3], q.shape[0] * _ceil_div(k.shape[1], 128) * k.shape[2],
                                          _ceil_div(q.shape[1], 64) * (q.shape[2] // k.shape[2]), is_causal, True,
-                                         _compute_units(q.device.index))
+                                         _compute_units(q.device.index), _ceil_div(q.shape[1], 64))
     q_scaled = torch.empty_like(q) if overlap else dq
     neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled)
     with _on_device(q):
@@ -855,7 +861,7 @@ def attention_backward_varlen(
     bounded = 0 < max_seqlen_q and (max_seqlen_q < q.shape[1] or cu_q.numel() == 2)
     overlap = bounded and _backward_launches_overlap(
         q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False,
-        _compute_units(q.device.index))
+        _compute_units(q.device.index), _ceil_div(max_seqlen_q, 64))
     q_scaled = torch.empty_like(q) if overlap else dq
     neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled, (cu_q, cu_kv, k.shape[1], tiles))
     with _on_device(q):

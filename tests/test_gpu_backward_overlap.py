@@ -40,12 +40,21 @@ def problem(packed, seed, H=8, Hkv=2, D=128):
     return lambda: _lib.attention_backward_varlen(q, k, v, out, d_out, lse, cu, cu, True, 0.088, 700)
 
 
+def test_rule_leaves_out_what_the_host_takes_longer_for():
+    """Steps whose launches are over before the host has made them gain nothing from a second stream."""
+    def dense(B, S, H, Hkv, causal):
+        return _lib._backward_launches_overlap(128, B * -(-S // 128) * Hkv, -(-S // 64) * (H // Hkv), causal, True, 256, -(-S // 64))
+
+    assert not dense(2, 944, 2, 1, False) and not dense(1, 1893, 16, 8, True) and not dense(2, 235, 16, 1, False)
+    assert dense(2, 1532, 4, 1, False) and dense(1, 4000, 4, 4, True) and dense(2, 2552, 16, 1, True)
+
+
 @pytest.mark.gpu
 def test_the_device_is_asked(monkeypatch):
     units = torch.cuda.get_device_properties(0).multi_processor_count
     for packed in (False, True):
         call, asked = problem(packed, 1), []
-        monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: asked.append(a[-1]))
+        monkeypatch.setattr(_lib, "_backward_launches_overlap", lambda *a: asked.append(a[5]))
         call()
         assert asked == [units]
 
