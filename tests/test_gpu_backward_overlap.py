@@ -20,6 +20,7 @@ def test_rule():
     assert not rule(128, 1440, 60, False, True)   # a last round of 160 of six
     assert not rule(128, 24, 5, False, True)      # over before a second stream has begun
     assert not rule(64, 264, 128, True, False)
+    assert not rule(128, 456, 228, True, True)    # idle for a ninth of the time
 
 
 def test_rule_counts_the_compute_units_of_the_device():
