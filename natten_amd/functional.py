@@ -172,13 +172,13 @@ def neighborhood_attention_generic(
         t is not None and t.requires_grad for t in (query, key, value, additional_keys, additional_values)
     )
     if (has_additional_attention and not needs_grad and not attn_kwargs and q_tile_shape is None and kv_tile_shape is None
-            and q_scale is None and k_scale is None and v_scale is None):
-        # one launch over the window and the context, where there is one
+            and q_scale is None and k_scale is None and v_scale is None and final_dtype == query.dtype):
+        # one launch over the window and the context, where there is one (it rounds to the operands' type: a caller
+        # who asks for float32 gets the merge's, and one who asks for what the merge does not take its refusal)
         joint = amd_fna_with_context(query, key, value, additional_keys, additional_values, kernel_size, stride, dilation,
                                      is_causal, scale, run_persistent_kernel)
         if joint is not None:
-            output = joint[0].to(final_dtype)
-            return (output, joint[1]) if return_lse else output
+            return joint if return_lse else joint[0]
     if is_fp8(query.dtype):
         work_dtype = torch.bfloat16
     else:

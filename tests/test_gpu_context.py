@@ -8,7 +8,7 @@ import torch
 
 from natten_amd import _lib
 from natten_amd.fna import _context_call_plan, amd_fna_with_context
-from natten_amd.functional import na1d, na2d, na3d
+from natten_amd.functional import attention, merge_attentions, na1d, na2d, na3d
 from natten_amd.tile_config import choose_fitting_forward_tiles
 from oracle import c_oracle
 from oracle import na_oracle as O
@@ -119,6 +119,32 @@ def test_without_the_launch_two_attentions_are_merged():
         ref_o, ref_l = reference(case, q, k, v, ck, cv)
         assert_close("out", to_np(out), ref_o)
         assert_close("lse", to_np(lse), ref_l)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_result_type_that_the_caller_chooses_merges_two(dtype):
+    """The joint launch rounds to the operands' type.  A float32 result is that of the merge in float32; a type that the merge
+    does not take is refused."""
+    case = ((40, 33), (7, 7), (1, 1), (1, 1), (False, False), 4, 2, 64)
+    kernel = case[1]
+    q, k, v, ck, cv = inputs(case, 128, dtype)
+    v, cv = v + 3, cv + 3  # (rounding errors of one sign and size in both parts: the merge averages them)
+    context = dict(additional_keys=ck, additional_values=cv, return_lse=True)
+    with torch.no_grad():
+        out, lse = na2d(q, k, v, kernel, out_dtype=torch.float32, **context)
+        parts = na2d(q, k, v, kernel, out_dtype=torch.float32, return_lse=True), attention(
+            q.flatten(1, 2), ck, cv, out_dtype=torch.float32, return_lse=True)
+        want, want_lse = merge_attentions(*([t.flatten(1, 2) for t in pair] for pair in zip(*(
+            (o.reshape(out.shape), l.reshape(lse.shape)) for o, l in parts))))
+        assert out.dtype == torch.float32 and torch.equal(out, want.reshape(out.shape)) and torch.equal(lse, want_lse.reshape(lse.shape))
+        with pytest.raises(NotImplementedError):
+            na2d(q, k, v, kernel, out_dtype=torch.float64, **context)
+    ref_o, _ = reference(case, q, k, v, ck, cv)
+    error = lambda t: float(np.linalg.norm(to_np(t) - ref_o) / np.linalg.norm(ref_o))
+    joint = amd_fna_with_context(q, k, v, ck, cv, *case[1:5], 0.125)[0]
+    print(f"error of a float32 result {error(out):.3e}, of the joint launch {error(joint):.3e}")
+    assert error(out) < error(joint)
 
 
 @pytest.mark.gpu
