@@ -534,22 +534,23 @@ def attention_forward(
     scales = _scale_ptrs(q, k, q_scale, k_scale, v_scale)
     out = torch.empty_like(q)
     lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
+    batch, seqlen_q, heads_q, head_dim = q.shape
+    _, seqlen_kv, heads_kv, _ = k.shape
     with _on_device(q):
         splits = 1
-        if q.shape[0] > 1 and k.shape[1] > 960:  # (one sequence or under 16 key tiles: never split, and asking takes a small call 0.8 us)
-            positions, splits = attention_split_plan(
-                q.device.index, q.shape[0], q.shape[1], k.shape[1], q.shape[2], q.shape[3], bool(is_causal))
+        if batch > 1 and seqlen_kv > 960:  # (one sequence or under 16 key tiles: never split, and asking takes a small call 0.8 us)
+            positions, splits = attention_split_plan(q.device.index, batch, seqlen_q, seqlen_kv, heads_q, head_dim, bool(is_causal))
         if splits > 1:
-            parts = torch.empty(positions * splits * 128 * (q.shape[3] + 1), dtype=torch.float32, device=q.device)
+            parts = torch.empty(positions * splits * 128 * (head_dim + 1), dtype=torch.float32, device=q.device)
             _check(L.natten_amd_attention_forward_split(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), parts.data_ptr(), parts.numel(), positions,
-                splits, DTYPE_CODES[q.dtype], q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3],
+                splits, DTYPE_CODES[q.dtype], batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim,
                 1 if is_causal else 0, float(scale), *scales, _stream(q),
             ))
             return out, lse
         rc = L.natten_amd_attention_forward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(), DTYPE_CODES[q.dtype],
-            q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0,
+            batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim, 1 if is_causal else 0,
             float(scale), *scales, _stream(q),
         )
     _check(rc)
@@ -787,6 +788,7 @@ def _compute_units(device_index: int) -> int:
     return torch.cuda.get_device_properties(device_index).multi_processor_count
 
 
+@functools.lru_cache(maxsize=1024)
 def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int, is_causal: bool, equal: bool,
                                compute_units: int = 256, longest_query: Optional[int] = None) -> bool:
     """Whether the dq launch of dense attention runs beside the dk / dv launch (head dim 128: a workgroup per compute
@@ -822,16 +824,19 @@ def attention_backward(
     if q.dtype not in (torch.float16, torch.bfloat16):
         raise NotImplementedError(f"natten_amd attention_backward does not support {q.dtype}.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    overlap = _backward_launches_overlap(q.shape[3], q.shape[0] * _ceil_div(k.shape[1], 128) * k.shape[2],
-                                         _ceil_div(q.shape[1], 64) * (q.shape[2] // k.shape[2]), is_causal, True,
-                                         _compute_units(q.device.index), _ceil_div(q.shape[1], 64))
+    # (a short step waits for the host: the rule is not asked where it has one answer, and every extent is read once)
+    batch, seqlen_q, heads_q, head_dim = q.shape
+    _, seqlen_kv, heads_kv, _ = k.shape
+    overlap = head_dim == 128 and _backward_launches_overlap(
+        head_dim, batch * _ceil_div(seqlen_kv, 128) * heads_kv, _ceil_div(seqlen_q, 64) * (heads_q // heads_kv), is_causal, True,
+        _compute_units(q.device.index), _ceil_div(seqlen_q, 64))
     q_scaled = torch.empty_like(q) if overlap else dq
     neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled)
     with _on_device(q):
         rc = L.natten_amd_attention_backward(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), q_scaled.data_ptr(), 3 if overlap else 1, DTYPE_CODES[q.dtype],
-            q.shape[0], q.shape[1], k.shape[1], q.shape[2], k.shape[2], q.shape[3], 1 if is_causal else 0, float(scale), _stream(q),
+            batch, seqlen_q, seqlen_kv, heads_q, heads_kv, head_dim, 1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)
     return dq, dk, dv
@@ -858,17 +863,19 @@ def attention_backward_varlen(
     # The longest sequence is not known here, only what the caller says bounds it.  All rows, with several sequences, says
     # nothing; any other bound is taken as the longest (us, one behind the other / side by side: 16 of 128, H 8 / 2 49 / 68;
     # 9 up to 176, H 16 / 4 58 / 68; 16 of 512, H 16 / 4 declared as 1024 152 / 157).
-    bounded = 0 < max_seqlen_q and (max_seqlen_q < q.shape[1] or cu_q.numel() == 2)
+    _, rows_q, heads_q, head_dim = q.shape
+    _, rows_kv, heads_kv, _ = k.shape
+    bounded = head_dim == 128 and 0 < max_seqlen_q and (max_seqlen_q < rows_q or cu_q.numel() == 2)
     overlap = bounded and _backward_launches_overlap(
-        q.shape[3], _ceil_div(k.shape[1], 128) * k.shape[2], _ceil_div(max_seqlen_q, 64) * (q.shape[2] // k.shape[2]), is_causal, False,
+        head_dim, _ceil_div(rows_kv, 128) * heads_kv, _ceil_div(max_seqlen_q, 64) * (heads_q // heads_kv), is_causal, False,
         _compute_units(q.device.index), _ceil_div(max_seqlen_q, 64))
     q_scaled = torch.empty_like(q) if overlap else dq
-    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled, (cu_q, cu_kv, k.shape[1], tiles))
+    neg_delta, neg_lse2 = backward_prepare(q, out, d_out, lse, scale, q_scaled, (cu_q, cu_kv, rows_kv, tiles))
     with _on_device(q):
         rc = L.natten_amd_attention_backward_varlen(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), neg_lse2.data_ptr(), neg_delta.data_ptr(),
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), q_scaled.data_ptr(), 3 if overlap else 1, DTYPE_CODES[q.dtype],
-            cu_q.numel() - 1, q.shape[1], k.shape[1], cu_q.data_ptr(), cu_kv.data_ptr(), tiles.data_ptr(), q.shape[2], k.shape[2], q.shape[3],
+            cu_q.numel() - 1, rows_q, rows_kv, cu_q.data_ptr(), cu_kv.data_ptr(), tiles.data_ptr(), heads_q, heads_kv, head_dim,
             1 if is_causal else 0, float(scale), _stream(q),
         )
     _check(rc)

@@ -61,6 +61,19 @@ def test_the_device_is_asked(monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("packed", [False, True])
+def test_other_head_dims_do_not_ask(monkeypatch, packed):
+    """Only head dim 128 has the two streams: a short step of another one waits for the host and does not pay for the question."""
+    def asked(*a):
+        raise AssertionError("asked")
+
+    call = problem(packed, 1, D=64)
+    monkeypatch.setattr(_lib, "_backward_launches_overlap", asked)
+    monkeypatch.setattr(_lib, "_compute_units", asked)
+    call()
+
+
+@pytest.mark.gpu
 def test_a_bound_of_all_rows_says_nothing(monkeypatch):
     """max_seqlen_Q as large as the batch, with several sequences in it, is no estimate of the longest."""
     asked = []
