@@ -795,24 +795,25 @@ def _backward_launches_overlap(head_dim: int, key_tiles: int, longest_walk: int,
     unit), which then has a workspace for the scaled queries besides dq.  `key_tiles` over all heads, `longest_walk`:
     query tiles of 64 that the longest of them meets (over the query heads of a key head), `longest_query`: of one head (None:
     as many), `equal`: sequences of one length.  Figures with 256 compute units.
-    Taken where the compute units stand idle for 20 of those steps (1.6 us) and an eighth of the time or more on the average:
-    the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic.  us of both launches and the pass
+    Taken where the compute units stand idle for 20 of those steps (1.6 us) and, causal, an eighth of the time or more, else 0.36 of
+    it: the two streams cost some 15 us, and launches that fill the chip lose to each other's traffic, those without a mask, whose
+    workgroups all last the longest, more.  us of both launches and the pass
     before, one behind the other / side by side (idle steps): packed, causal, 10 sequences of 1 .. 2048, H 16 / 4 310 / 255 (62),
     5 up to 1527, H 4 97 / 76 (18), 16 of 512, H 16 / 4 152 / 157 (16), 7 up to 384, H 8 / 4 60 / 69 (11), 9 up to 176, H 16 44 / 70 (3);
-    1 x 2000 causal, H 16 / 4 248 / 209 (112), 1 x 9000 full, H 8 / 4 1431 / 1067 (251), H 16 2150 / 2095 (79), 2 x 2176 full,
-    H 16 336 / 290 (30), 2 x 4096 full, H 16 / 8 814 / 902 (0), 2 x 3000 causal, H 8 181 / 203 (12), 2 x 3809
-    full, H 24 1146 / 1160 (22 of 360), 2 x 7230 causal, H 8 / 4 a step 903 / 939 (25 of 228).  Of 60 random problems that it is taken for, 59 are 3 to 59 % faster and one 5 % slower (1 x 6051
-    full, H 8 / 4: 541 / 572, 192 key tiles in one round).
-    The second stream also takes the host 41 us a call, and a training step on one attention takes it 140 to 175 without: steps whose launches
-    are over by then only get longer (us, forward and backward: 2 x 944 full, H 2 / 1 143 / 184; 5 up to 952, H 16 / 4 173 / 219;
-    1 x 2906 causal, H 4 197 / 206; 4 x 2157 full, H 2 / 1 207 / 206; 3 up to 3143, H 4 223 / 198; 2 x 1532 full, H 4 / 1 228 / 209).  So
-    the launches of a step have to add up to 210 us: 1.6 a step of the key-stationary walk, 2.2 a step of the forward's and dQ's."""
+    1 x 2000 causal, H 16 / 4 248 / 209 (112), 1 x 9000 full, H 8 / 4 1431 / 1067 (251), 2 x 4096 full, H 16 / 8 814 / 902 (0), 2 x 3000
+    causal, H 8 181 / 203 (12), 1 x 2920 full, H 16 289 / 306 (26 of 92), 4 x 6450 full, H 2 / 1 585 / 594 (41 of 202), 1 x 8938 full,
+    H 2 414 / 354 (63 of 140), 1 x 6842 causal, H 16 / 8 668 / 641 (33 of 214); steps: 2 x 7230 causal, H 8 / 4 903 / 939 (25 of 228),
+    1 x 5690 full, H 8 / 4 629 / 657 (53 of 178), 1 x 6051 541 / 572.
+    The second stream also takes the host 41 us a call, and a training step on one attention takes it up to 180 without: steps whose launches
+    are over by then only get longer, those up to 225 us with a slow host too (us, forward and backward: 2 x 944 full, H 2 / 1 143 /
+    184; 5 up to 952, H 16 / 4 173 / 219; 1 x 2906 causal, H 4 197 / 206; 2 x 2157 causal, H 8 / 4 205 / 225; 5 up to 3046, H 1 218 / 244).  So
+    the launches of a step have to add up to 250 us: 1.6 a step of the key-stationary walk, 2.2 a step of the forward's and dQ's."""
     if head_dim != 128:
         return False
     work = key_tiles * longest_walk * (0.5 if is_causal else 1.0) / compute_units
     span = max(longest_walk, work) if is_causal or not equal else longest_walk * _ceil_div(key_tiles, compute_units)
     step_us = 30 + 1.6 * span + 2.2 * (longest_walk if longest_query is None else longest_query)
-    return span - work >= max(20, span / 8) and step_us >= 210
+    return span - work >= max(20, span / 8 if is_causal else 0.36 * span) and step_us >= 250
 
 
 def attention_backward(

@@ -21,12 +21,13 @@ def test_rule():
     assert not rule(128, 24, 5, False, True)      # over before a second stream has begun
     assert not rule(64, 264, 128, True, False)
     assert not rule(128, 456, 228, True, True)    # idle for a ninth of the time
+    assert not rule(128, 180, 178, False, True) and not rule(128, 180, 178, False, False)  # without a mask: for three tenths
 
 
 def test_rule_counts_the_compute_units_of_the_device():
     rule = _lib._backward_launches_overlap
     assert rule(128, 264, 128, True, False, 256) and not rule(128, 264, 128, True, False, 132)   # full with half of them
-    assert not rule(128, 256, 128, False, True, 256) and rule(128, 256, 128, False, True, 304)    # a round that is not full
+    assert not rule(128, 256, 128, False, True, 256) and rule(128, 256, 128, False, True, 512)    # a round that is half full
 
 
 def problem(packed, seed, H=8, Hkv=2, D=128):
@@ -47,7 +48,8 @@ def test_rule_leaves_out_what_the_host_takes_longer_for():
         return _lib._backward_launches_overlap(128, B * -(-S // 128) * Hkv, -(-S // 64) * (H // Hkv), causal, True, 256, -(-S // 64))
 
     assert not dense(2, 944, 2, 1, False) and not dense(1, 1893, 16, 8, True) and not dense(2, 235, 16, 1, False)
-    assert dense(2, 1532, 4, 1, False) and dense(1, 4000, 4, 4, True) and dense(2, 2552, 16, 1, True)
+    assert not dense(2, 2157, 8, 4, True) and not dense(1, 1418, 4, 1, True) and not dense(1, 1497, 4, 1, False)
+    assert dense(1, 1710, 8, 2, False) and dense(1, 4000, 4, 4, True) and dense(2, 2552, 16, 1, True)
 
 
 @pytest.mark.gpu
