@@ -303,7 +303,8 @@ int natten_amd_attention_forward(const void* q, const void* k, const void* v, vo
 
 /*
  * What natten_amd_attention_forward_split is to be given for a problem on the current device, where it was
- * measured to be faster than natten_amd_attention_forward; *kv_splits = 1 elsewhere.
+ * measured to be faster than natten_amd_attention_forward; *kv_splits = 1 elsewhere.  seqlen_kv: the
+ * keys that some row meets, for a causal problem of fewer queries than keys as many as there are queries.
  */
 int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int heads_q, int head_dim,
                                     int is_causal, int32_t* split_positions, int32_t* kv_splits);

@@ -539,7 +539,9 @@ def attention_forward(
     with _on_device(q):
         splits = 1
         if batch > 1 and seqlen_kv > 960:  # (one sequence or under 16 key tiles: never split, and asking takes a small call 0.8 us)
-            positions, splits = attention_split_plan(q.device.index, batch, seqlen_q, seqlen_kv, heads_q, head_dim, bool(is_causal))
+            # (causal rows meet the keys up to their own number: 4 x 512 queries, 5568 keys, H 2, D 96 20.3 us, 29.2 split 15 ways)
+            keys = min(seqlen_q, seqlen_kv) if is_causal else seqlen_kv
+            positions, splits = attention_split_plan(q.device.index, batch, seqlen_q, keys, heads_q, head_dim, bool(is_causal))
         if splits > 1:
             parts = torch.empty(positions * splits * 128 * (head_dim + 1), dtype=torch.float32, device=q.device)
             _check(L.natten_amd_attention_forward_split(

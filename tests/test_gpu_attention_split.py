@@ -64,6 +64,7 @@ CASES = [
     (2, 70, 3470, 6, 3, 96, False),
     (2, 1500, 3537, 3, 3, 40, True),
     (2, 8321, 2600, 4, 2, 64, False),       # a whole round, then 16 Q tiles more
+    (2, 2700, 3537, 3, 3, 40, True),        # fewer causal queries than keys
 ]
 
 
@@ -139,3 +140,16 @@ def test_rows_of_nan(D):
     assert torch.isnan(want[0, :, 1]).all() and torch.isnan(want[1, 77]).all() and torch.isfinite(want[0, :, 0]).all()
     torch.testing.assert_close(out.float(), want.float(), atol=2.0**-7, rtol=2.0**-7, equal_nan=True)
     torch.testing.assert_close(lse, want_lse, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.gpu
+def test_causal_queries_fewer_than_keys(monkeypatch):
+    """Causal rows meet the keys up to their own number: the plan is asked for those."""
+    asked, plan = [], _lib.attention_split_plan
+    monkeypatch.setattr(_lib, "attention_split_plan", lambda *a: asked.append(a) or plan(*a))
+    with torch.no_grad():
+        for Sq, causal, split in ((1100, True, False), (512, True, False), (1100, False, True)):
+            q, kv = rand((4, Sq, 2, 96), torch.bfloat16, 1), rand((4, 5568, 2, 96), torch.bfloat16, 2)
+            natten_amd.attention(q, kv, kv, is_causal=causal)
+            assert [a[3] for a in asked] == [Sq if causal else 5568]
+            assert (plan(*asked.pop())[1] > 1) == split
