@@ -936,26 +936,28 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   if (batch < 2 || kv_tiles < 16 || n / (slots * kNumXcd) > 12) return 0;
   FnaParams p;
   fill_dense_fwd(p, batch, seqlen_q, seqlen_kv, heads_q, heads_q, is_causal);
-  // Every XCD works off its own launch positions (see fna_fwd_tile): the one with the most Q tiles sets the time.  In an
-  // XCD's tiles, where the shares are uneven (5 x 3100 tokens, H 5, D 128: 131 us in one launch; counted over the chip, 113 of 625
-  // Q tiles were split four ways, and the fullest XCD still began another round: 149).
-  auto tiles_at = [&](int xcd, int local) {  // 1 where the position holds a Q tile
-    const int run = local / p.wg_group, group = run * kNumXcd + xcd;
-    return group < p.total_groups && group % p.groups_per_bh * p.wg_group + local - run * p.wg_group < p.num_q_tiles ? 1 : 0;
+  // Every XCD works off its own launch positions (see fna_fwd_tile): the one with the most sets the time.  In an XCD's
+  // positions, where the shares are uneven (5 x 3100 tokens, H 5, D 128: 131 us in one launch; counted over the chip, 113 of 625
+  // Q tiles were split four ways, and the fullest XCD still began another round: 149).  Positions without a Q tile, at the end
+  // of a short group, count: workgroups go to the compute units in order, and the room that such a one leaves is not
+  // refilled out of turn (3 x 3712 tokens, H 6, D 64, 68 Q tiles in 70 positions: with 4 of them split, so that 64 Q tiles
+  // are left whole, 105 us, with 6 80, in one launch 82).
+  auto position_at = [&](int xcd, int local) {  // 1 where the position belongs to a group
+    return local / p.wg_group * kNumXcd + xcd < p.total_groups ? 1 : 0;
   };
   const int positions = na_ceil_div(p.total_groups, kNumXcd) * p.wg_group;  // of an XCD
-  int tiles[kNumXcd] = {}, most = 0;
+  int share[kNumXcd] = {}, most = 0;
   for (int x = 0; x < kNumXcd; ++x) {
-    for (int i = 0; i < positions; ++i) tiles[x] += tiles_at(x, i);
-    most = na_max(most, tiles[x]);
+    for (int i = 0; i < positions; ++i) share[x] += position_at(x, i);
+    most = na_max(most, share[x]);
   }
   // An XCD takes `slots` workgroups of the split launch at a time (two waves per SIMD at every head dim).  What does not
   // fill a last round is split so that it does, where that saves a twelfth of the whole and more than the merge takes
   // (2 x 4097 tokens, H 16, D 64, a third round of 4 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
   // and 180; 2 x 5000, H 8, D 128: 204 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
-  // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch and the parts' way through memory
-  // eight.  The second launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4,
-  // D 128: 19.6 us, split 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
+  // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch and the parts' way through memory eight.  The second
+  // launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split
+  // 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
   int round_slots = slots;
   if (most > slots) {
     if (is_causal) return 0;  // rounds even out by themselves: the longest walks start first
@@ -989,8 +991,8 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
     ++last;
     over = false;
     for (int x = 0; x < kNumXcd; ++x) {
-      tiles[x] -= tiles_at(x, positions - last);
-      over = over || tiles[x] > full * round_slots;
+      share[x] -= position_at(x, positions - last);
+      over = over || share[x] > full * round_slots;
     }
   }
   const double round = last <= cus ? 0.75 * kv_tiles : kv_tiles;

@@ -56,6 +56,12 @@ def test_plan_counts_by_xcd():
     assert plan(3, 3522, 3522, 3, 128, False) == (0, 1)     # 35 of 64: not twice
 
 
+def test_plan_counts_positions_without_a_q_tile():
+    """29 Q tiles in groups of ten: 70 positions on an XCD, two or three of them empty, keep their places in a round of 64."""
+    assert _lib.attention_split_plan(0, 3, 3712, 3712, 6, 64, False)[0] in (0, 48)
+    assert _lib.attention_split_plan(0, 3, 3712, 3715, 6, 64, False)[0] == 48
+
+
 CASES = [
     # B, Sq, Skv, H, Hkv, D, causal
     (2, 300, 3500, 2, 1, 128, False),
@@ -65,6 +71,7 @@ CASES = [
     (2, 1500, 3537, 3, 3, 40, True),
     (2, 8321, 2600, 4, 2, 64, False),       # a whole round, then 16 Q tiles more
     (2, 2700, 3537, 3, 3, 40, True),        # fewer causal queries than keys
+    (3, 3712, 3715, 6, 6, 64, False),       # groups of Q tiles that do not divide the sequence
 ]
 
 
