@@ -955,7 +955,7 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   // fill a last round is split so that it does, where that saves a twelfth of the whole and more than the merge takes
   // (2 x 4097 tokens, H 16, D 64, a third round of 4 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
   // and 180; 2 x 5000, H 8, D 128: 204 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
-  // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch and the parts' way through memory eight.  The second
+  // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch eight.  The second
   // launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split
   // 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
   int round_slots = slots;
@@ -996,10 +996,15 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
     }
   }
   const double round = last <= cus ? 0.75 * kv_tiles : kv_tiles;
+  // The parts are written and read once, which takes 12 us for 60 of them on every XCD at head dim 128.  Two and three
+  // ways, which fill the chip with parts, lost without this (us, one launch / split: 224 Q tiles of 56 KV tiles, head
+  // dim 128, two ways 57.5 / 65.4, 204 of 72 69.7 / 76.1, 222 of 74 77.8 / 83.1; head dim 64, 240 of 55 38.1 / 43.0; 630 of 42 at
+  // 128, three ways, 117.9 / 125.2).
+  const double part = 0.0015 * (head_dim + 1);
   double least = 1e30;
   int best = 1;
   for (int s = 2; s <= 16 && last * s <= slots && kv_tiles / s >= 3; ++s) {
-    const double t = (last * s <= cus ? 0.75 : 1.0) * na_ceil_div(kv_tiles, s) + 8;
+    const double t = (last * s <= cus ? 0.75 : 1.0) * na_ceil_div(kv_tiles, s) + 8 + part * last * s;
     if (t < least) {
       least = t;
       best = s;

@@ -37,7 +37,7 @@ def test_plan_where_the_one_launch_holds_three_waves():
     for S, H in ((2560, 16), (3072, 12), (5120, 8), (4096, 17)):    # 576 .. 1088 Q tiles: 768 fit one round
         assert plan(2, S, S, H, 64, False) == (0, 1)
     assert plan(2, 8448, 3072, 4, 64, False)[1] > 1 and plan(2, 9216, 9216, 4, 64, False)[1] > 1   # long walks, few left over
-    assert plan(2, 2560, 2561, 16, 64, False)[1] > 1                # masks: two waves either way
+    assert plan(2, 2560, 4001, 16, 64, False)[1] > 1                # masks: two waves either way
     for S, H in ((4097, 16), (3500, 16), (4097, 12), (10000, 10)):
         assert plan(2, S, S, H, 32, False) == (0, 1)
     assert plan(2, 12547, 12547, 4, 32, False)[1] > 1
@@ -60,6 +60,15 @@ def test_plan_counts_positions_without_a_q_tile():
     """29 Q tiles in groups of ten: 70 positions on an XCD, two or three of them empty, keep their places in a round of 64."""
     assert _lib.attention_split_plan(0, 3, 3712, 3712, 6, 64, False)[0] in (0, 48)
     assert _lib.attention_split_plan(0, 3, 3712, 3715, 6, 64, False)[0] == 48
+
+
+def test_plan_counts_the_way_of_the_parts_through_memory():
+    plan = lambda *a: _lib.attention_split_plan(0, *a)
+    for B, Sq, Skv, H, D in ((2, 3526, 3526, 4, 128), (8, 605, 4070, 6, 128), (2, 4352, 4608, 3, 128), (2, 3840, 3520, 4, 64),
+                             (6, 2688, 2688, 5, 128), (2, 3712, 3648, 4, 64), (6, 376, 3464, 12, 128)):
+        assert plan(B, Sq, Skv, H, D, False) == (0, 1)          # two or three ways: as much again as the walks save
+    for B, Sq, Skv, H, D, ways in ((2, 9000, 9000, 1, 128, 3), (4, 800, 6000, 5, 128, 3), (2, 4000, 8000, 2, 64, 4)):
+        assert plan(B, Sq, Skv, H, D, False)[1] >= ways
 
 
 CASES = [
