@@ -953,8 +953,8 @@ int natten_amd_attention_split_plan(int batch, int seqlen_q, int seqlen_kv, int 
   }
   // An XCD takes `slots` workgroups of the split launch at a time (two waves per SIMD at every head dim).  What does not
   // fill a last round is split so that it does, where that saves a twelfth of the whole and more than the merge takes
-  // (2 x 4097 tokens, H 16, D 64, a third round of 4 Q tiles: 176 us, 158 with them split 13 ways; 2 x 9000, H 4, D 64: 226
-  // and 180; 2 x 5000, H 8, D 128: 204 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
+  // (2 x 4097 tokens, H 16, D 64, a third round of 4 Q tiles: 176 us, 153 with them split 8 ways; 2 x 9000, H 4, D 64: 226
+  // and 177; 2 x 5000, H 8, D 128: 205 and 194).  In KV tiles of a workgroup that shares its compute unit (0.62 us at head
   // dim 64, 1.05 at 128): a workgroup alone on one takes three quarters, the second launch eight.  The second
   // launch and the workspace also take the host 5 us: launches under 40 KV tiles (2 x 1000 tokens, H 4, D 128: 19.6 us, split
   // 23.9; 2 x 2000, H 4, D 32: 21.0 and 26.2) are over by then.
