@@ -791,24 +791,26 @@ fna_bwd_kernel(const FnaBwdParams p) {
       async_copy16_uniform(y2, off, lds_y2 + dst2 + uint32_t(i * NT * 16));
     }
   };
-  // lane-constant LDS read offsets (same fragment layouts as the forward kernel)
-  int k_off[KSTEPS];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) k_off[ks] = l32 * ROWB + L::u_slot(l32, ks * 2 + g) * 16;
+  // LDS reads of operand fragments (same fragment layouts as the forward kernel): row l32, chunk 2 ks + g, and transposed
+  // rows 4 g + e [+ 8], chunk 4 db + v_chunk.  The chunk numbers differ by exclusive or as the swizzle does, and stages begin at
+  // multiples of a row of chunks, so that every fragment's address is one lane offset with a few bits turned over: an
+  // instruction each where it is used, as an addition to the stage's base would be, and two registers instead of
+  // sixteen (head dim 128: the paired role 246 -> 216, the dQ role 256 and 9 spilled -> 244).
+  const uint32_t k_lane = uint32_t(l32 * ROWB + L::u_slot(l32, g) * 16);
   const int l16 = lane & 15;
   const int v_e = l16 >> 2, v_j4 = l16 & 3;
   const int v_row = 4 * g + v_e;
   const int v_chunk = (l32 >> 4) * 2 + (v_j4 >> 1);
-  const int v_sub = (v_j4 & 1) * 8;
-  auto row_frag = [&](const char* s, int sb, int ks) {
-    return *reinterpret_cast<const vec8*>(s + sb * 32 * ROWB + k_off[ks]);
+  const uint32_t v_lane = uint32_t(v_row * ROWB + L::u_slot(v_row, v_chunk) * 16 + (v_j4 & 1) * 8);
+  // `s`: LDS address of the stage
+  auto row_frag = [&](uint32_t s, int sb, int ks) __attribute__((always_inline)) {
+    return *lds_pointer<vec8>(((s + k_lane) ^ uint32_t(ks * 32)) + uint32_t(sb * 32 * ROWB));
   };
   // transposed fragment: sub-block sb, 16-row half h, 32-column block db
-  auto tr_frag = [&](const char* s, int sb, int h, int db) {
-    const int r0 = sb * 32 + h * 16 + v_row;
-    const int c = db * 4 + v_chunk;
-    const s16x4_t lo = lds_read_tr16(s + r0 * ROWB + v_sub + L::u_slot(r0, c) * 16);
-    const s16x4_t hi = lds_read_tr16(s + (r0 + 8) * ROWB + v_sub + L::u_slot(r0 + 8, c) * 16);
+  auto tr_frag = [&](uint32_t s, int sb, int h, int db) __attribute__((always_inline)) {
+    const uint32_t at = (s + v_lane) ^ uint32_t(db * 64), row0 = uint32_t((sb * 32 + h * 16) * ROWB);
+    const s16x4_t lo = lds_read_tr16(at + row0);
+    const s16x4_t hi = lds_read_tr16((at ^ 32u) + row0 + 8 * ROWB);
     return __builtin_bit_cast(vec8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
 
@@ -868,7 +870,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
   constexpr int N1 = 2 * NP;
   constexpr int NC = 2 * DB * W;                           // accumulation slots per sub-block
   constexpr int G = N1 + 2 * NC;
-  constexpr int PF = 2;                                    // fragments read ahead
+  // fragments read ahead (dQ at head dim 128, two / three: 29 x 46 x 78, 9 x 24 x 24, H 8 4.36 / 4.30 ms; others level)
+  constexpr int PF = D == 128 && !KV_STATIONARY ? 3 : 2;
   // P waves of the paired role: the products of both sub-blocks first, then the accumulations of
   // both, and the probabilities of a sub-block two per slot between the matrix instructions that
   // follow its products (sub-block 0: the products of sub-block 1; sub-block 1: the accumulations
@@ -878,8 +881,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
   auto tile_body = [&](auto masked_tag, int stage, int stage2, uint32_t bits, int exch, auto&& after_slot) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
     (void)exch;  // paired role: which of the two probability buffers this tile writes
-    const char* y1 = sY1 + stage * TILE_BYTES;
-    const char* y2 = sY2 + stage2 * TILE_BYTES;  // (stage2 differs from stage in the paired role only)
+    const uint32_t y1 = lds_y1 + uint32_t(stage * TILE_BYTES);
+    const uint32_t y2 = lds_y2 + uint32_t(stage2 * TILE_BYTES);  // (stage2 differs from stage in the paired role only)
 
     // slot x of the tile: a product slot (sub-block, index i < NP) or an accumulation slot (i < NC)
     struct Slot {
@@ -1030,7 +1033,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // then dK += dS^T Q with that tile's Q (still in its stage).
   f32x16_t held_dp[NSB];
   auto pair_produce = [&](int stage1, int stage) __attribute__((always_inline)) {
-    const char* y2 = sY2 + stage * TILE_BYTES;
+    const uint32_t y2 = lds_y2 + uint32_t(stage * TILE_BYTES);
     constexpr int N = NSB * KSTEPS;
     vec8 fr[N];
     // the products start from -delta of the tile's queries (tables live in the stages of Y1)
@@ -1055,7 +1058,7 @@ fna_bwd_kernel(const FnaBwdParams p) {
     });
   };
   auto pair_consume = [&](int stage, int exch) __attribute__((always_inline)) {
-    const char* y1 = sY1 + stage * TILE_BYTES;
+    const uint32_t y1 = lds_y1 + uint32_t(stage * TILE_BYTES);
     vec8 dsf[NSB][2];
     u32x4_t plo[NSB], phi[NSB];
 #pragma unroll
@@ -1097,6 +1100,13 @@ fna_bwd_kernel(const FnaBwdParams p) {
       __builtin_amdgcn_sched_barrier(0);
     });
   };
+  // The stationary fragments have landed from here on, as the compiler sees it too: left to the first product of the loop,
+  // the wait for them (a countdown to vmcnt(0)) stands in every step, where it also waits for the tile copies just issued.
+#pragma unroll
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    asm volatile("" : "+v"(x1f[ks]));
+    if constexpr (HAS_DS) asm volatile("" : "+v"(x2f[ks]));
+  }
   workgroup_sync();  // sRows is written
   // The paired role over n_iter tiles: step `it` has the P waves on tile `it` and the dS waves forming
   // dP of tile `it` after finishing tile it - 1; one more step drains the dS waves.  Tiles are copied

@@ -214,9 +214,25 @@ static __device__ __forceinline__ typename Mma<T>::vec8 scale_query_fragment(typ
   return out;
 }
 
+// the value at an LDS address
+template <typename V>
+static __device__ __forceinline__ const NA_LDS V* lds_pointer(uint32_t address) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wold-style-cast"
+  return (const NA_LDS V*)(uintptr_t)(address);
+#pragma clang diagnostic pop
+}
+
 // LDS transpose read: the 16 lanes of a group each point at 4 consecutive 16-bit elements of
 // a row (lane 4e+j -> row e, columns 4j..4j+3 of a 4x16 block); lane c of the group receives
 // column c of the block (rows 0..3).
+static __device__ __forceinline__ s16x4_t lds_read_tr16(uint32_t address) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Wold-style-cast"
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((NA_LDS s16x4_t*)(uintptr_t)(address));
+#pragma clang diagnostic pop
+}
+
 static __device__ __forceinline__ s16x4_t lds_read_tr16(const char* p) {
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Wold-style-cast"
@@ -401,7 +417,7 @@ constexpr float kLazyRescaleLog2 = 8.0f;
 // LDS layout of one K or V tile: KVT rows of D 16-bit elements, unpadded, with the 16-byte
 // chunks of each row XOR-swizzled so that the MFMA operand reads are bank-conflict free:
 //   K: chunk c of row r lives in slot c ^ ((r / RPL) % CPR)            (b128 reads down a column of rows)
-//   V: chunk c of row r lives in slot c ^ (2 * ((r / RPL) % (CPR/2)))  (transpose reads of 4 rows x 32 bytes)
+//   V: chunk c of row r lives in slot c ^ (4 * ((r / RPL) % (CPR/4)))  (transpose reads of 4 rows x 64 bytes)
 // CPR = chunks per row, RPL = rows per 256 bytes.
 template <int D, int KVT>
 struct FnaSmem {
@@ -412,14 +428,15 @@ struct FnaSmem {
   static constexpr int STAGES = 2;
   static constexpr int BYTES = STAGES * 2 * TILE_BYTES + KVT * 4;  // static LDS of the kernel
   static __host__ __device__ constexpr int k_slot(int r, int c) { return c ^ ((r / RPL) % CPR); }
-  static __host__ __device__ constexpr int v_slot(int r, int c) { return c ^ (2 * ((r / RPL) % (CPR / 2))); }
+  // Transpose reads: the 32 lanes of a wave half read four chunks of four consecutive rows in one cycle, so the four rows
+  // take a quarter of the 256-byte line each.  (2.2 cycles a read and compute unit, by a loop of them; with two
+  // rows on the same quarter 4.0.  A wave and tile of the forward at head dim 128 reads for 128 cycles instead of 192;
+  // what it shortens is small, the LDS being no bound: 30 x 48 x 80 causal, H 24 8.78 -> 8.72 ms, smaller problems level.)
+  static __host__ __device__ constexpr int v_slot(int r, int c) { return c ^ (4 * ((r / RPL) % (CPR / 4))); }
   // One layout that serves both kinds of read (the backward kernels read the same tile both
-  // ways): the XOR pattern runs through the even values over the first half of a 16-row period
-  // (what the transpose reads need) and through the odd ones over the second half (so that the
-  // 16 rows of a b128 column read still hit 16 different slots).
-  static __host__ __device__ constexpr int u_slot(int r, int c) {
-    return c ^ ((2 * ((r / RPL) % (CPR / 2))) | (((r / RPL) / (CPR / 2)) & 1));
-  }
+  // ways): a row's quarter as above, and inside the quarter another place for each four rows, so that the
+  // 16 rows of a b128 column read hit 16 different slots.
+  static __host__ __device__ constexpr int u_slot(int r, int c) { return c ^ (4 * ((r / RPL) % (CPR / 4)) | ((r / 4) % 4)); }
 };
 
 // Coordinates of KV tile i of a box of n[0] x n[1] x n[2] tiles, dimension 2 fastest: quotients by a rounded
@@ -1008,7 +1025,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const int v_chunk = (l32 >> 4) * 2 + (v_j4 >> 1);  // 16-byte chunk inside the 64-byte column block
   const int v_sub = (v_j4 & 1) * 8;
   uint32_t v_off[DB];  // (8 rows are a whole number of the V swizzle's periods)
-  static_assert(8 % (L::RPL * CPR / 2) == 0, "the transpose reads of a fragment lie 8 rows apart");
+  static_assert(8 % (L::RPL * CPR / 4) == 0, "the transpose reads of a fragment lie 8 rows apart");
 #pragma unroll
   for (int db = 0; db < DB; ++db) v_off[db] = uint32_t(v_row * ROWB + v_sub + L::v_slot(v_row, db * 4 + v_chunk) * 16);
 
