@@ -22,7 +22,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 # NATTEN_AMD_LIBRARY: another build of the library (the timing-only ones of natten_amd.build --ablate)
 LIB_PATH = os.environ.get("NATTEN_AMD_LIBRARY") or os.path.join(_HERE, "libnatten_amd.so")
 
-ABI_VERSION = 21
+ABI_VERSION = 22
 
 DTYPE_CODES = {
     torch.float16: 0,
@@ -127,6 +127,19 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_void_p] * 10 + [ctypes.c_int] * 5 + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 4
         + [ctypes.c_float, ctypes.c_void_p],
+    ),
+    "natten_amd_linear_forward": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 6 + [ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
+    ),
+    "natten_amd_linear_backward_input": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 5 + [ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
+    ),
+    "natten_amd_linear_backward_weight_workspace": (ctypes.c_int, [ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p]),
+    "natten_amd_linear_backward_weight": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 7 + [ctypes.c_uint64, ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
     ),
     "natten_amd_token_permute_widen": (
         ctypes.c_int,
@@ -695,6 +708,60 @@ def backward_prepare(
     return neg_delta, neg_lse2
 
 
+def _three(tensors) -> Tuple[Optional[int], ...]:
+    return tuple(t.data_ptr() for t in tensors) + (None,) * (3 - len(tensors))
+
+
+def linear_forward(x: Tensor, weight: Tensor, bias: Optional[Tensor], parts: int, shape) -> Tuple[Tensor, ...]:
+    """x (rows of weight.shape[1] elements) weight^T + bias, its columns split into `parts` tensors of `shape`."""
+    n, k = weight.shape
+    _require_gpu(x, weight)
+    outs = tuple(torch.empty(shape, dtype=x.dtype, device=x.device) for _ in range(parts))
+    if outs[0].numel() * parts * k != x.numel() * n:
+        raise ValueError(f"{parts} tensors of {tuple(shape)} do not hold the {n} columns of a map of {tuple(x.shape)}.")
+    with _on_device(x):
+        _check(lib().natten_amd_linear_forward(
+            x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), *_three(outs), DTYPE_CODES[x.dtype],
+            x.numel() // k, n, k, n // parts, _stream(x)))
+    return outs
+
+
+def linear_backward_input(d_outs, weight: Tensor, shape) -> Tensor:
+    """The gradient of a linear map's input, of `shape`, from those of its `len(d_outs)` outputs."""
+    n, k = weight.shape
+    _require_gpu(weight, *d_outs)
+    dx = torch.empty(shape, dtype=weight.dtype, device=weight.device)
+    with _on_device(weight):
+        _check(lib().natten_amd_linear_backward_input(
+            *_three(d_outs), weight.data_ptr(), dx.data_ptr(), DTYPE_CODES[weight.dtype], dx.numel() // k, n, k,
+            n // len(d_outs), _stream(weight)))
+    return dx
+
+
+@functools.lru_cache(maxsize=1024)
+def _linear_workspace(rows: int, n: int, k: int, part: int) -> int:
+    nbytes = ctypes.c_uint64()
+    _check(lib().natten_amd_linear_backward_weight_workspace(rows, n, k, part, ctypes.byref(nbytes)))
+    return nbytes.value
+
+
+def linear_backward_weight(d_outs, x: Tensor, shape, want_bias: bool) -> Tuple[Tensor, Optional[Tensor]]:
+    """The gradients of a linear map's weight [n, k] and bias (None unless wanted)."""
+    n, k = shape
+    L = lib()
+    _require_gpu(x, *d_outs)
+    rows = x.numel() // k
+    dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
+    db = torch.empty((n,), dtype=x.dtype, device=x.device) if want_bias else None
+    nbytes = _linear_workspace(rows, n, k, n // len(d_outs))
+    workspace = torch.empty((nbytes // 4,), dtype=torch.float32, device=x.device)
+    with _on_device(x):
+        _check(L.natten_amd_linear_backward_weight(
+            *_three(d_outs), x.data_ptr(), dw.data_ptr(), None if db is None else db.data_ptr(), workspace.data_ptr(), nbytes,
+            DTYPE_CODES[x.dtype], rows, n, k, n // len(d_outs), _stream(x)))
+    return dw, db
+
+
 def _head_major(lse: Tensor, delta: Tensor) -> Tuple[Tensor, Tensor]:
     """lse, delta [B, *X, H] as the backward kernels take them, [B, H, prod(X)]: a copy each and no more."""
     if lse.dtype != torch.float32 or delta.dtype != torch.float32:
@@ -773,13 +840,14 @@ def fna_backward_fused(
     # the launch that writes dq comes last.
     launches = [(3, q_tile_shape, kv_tile_shape)] if same else [
         (2, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
+    problem = tuple(tuple(x) for x in (kernel_size, stride, dilation, is_causal))
     with _on_device(q):
         for roles, qt, kt in launches:
             rc = L.natten_amd_fna_backward_fused(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2],
-                q.shape[-1], _i32(q.shape[1 : 1 + na_dim]), _i32(kernel_size), _i32(stride), _i32(dilation),
-                _i32([1 if c else 0 for c in is_causal]), _i32(qt), _i32(kt), float(scale), roles + prepared, _stream(q),
+                q.shape[-1], *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), *problem, tuple(qt), tuple(kt)), float(scale),
+                roles + prepared, _stream(q),
             )
             _check(rc)
     return dq, dk, dv

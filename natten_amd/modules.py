@@ -12,6 +12,7 @@ from torch import Tensor, nn
 
 from .checks import check_all_args
 from .functional import neighborhood_attention_generic
+from .linear import layer_step
 
 
 class NeighborhoodAttentionGeneric(nn.Module):
@@ -42,14 +43,15 @@ class NeighborhoodAttentionGeneric(nn.Module):
         batch, *tokens, channels = x.shape
         if channels != self.embed_dim:
             raise ValueError(f"Expected embedding dimension {self.embed_dim}, got {channels} ({x.shape=}).")
-        # [B, *X, 3, heads, head_dim]: q, k, v are strided views that the operation makes contiguous
-        qkv = self.qkv(x).reshape(batch, *tokens, 3, self.num_heads, self.head_dim)
-        q, k, v = qkv.unbind(dim=self.na_dim + 1)
-        out = neighborhood_attention_generic(
-            q, k, v, kernel_size=self.kernel_size, stride=self.stride, dilation=self.dilation,
-            is_causal=self.is_causal, scale=self.scale,
-        )
-        return self.proj_drop(self.proj(out.reshape(batch, *tokens, channels)))
+        problem = (self.kernel_size, self.stride, self.dilation, self.is_causal)
+        out = layer_step(self.qkv, self.proj, x, self.num_heads, problem, self.scale)
+        if out is None:
+            # [B, *X, 3, heads, head_dim]: q, k, v are strided views that the operation makes contiguous
+            qkv = self.qkv(x).reshape(batch, *tokens, 3, self.num_heads, self.head_dim)
+            q, k, v = qkv.unbind(dim=self.na_dim + 1)
+            out = neighborhood_attention_generic(q, k, v, *problem, scale=self.scale)
+            out = self.proj(out.reshape(batch, *tokens, channels))
+        return self.proj_drop(out)
 
     def extra_repr(self) -> str:
         return (f"head_dim={self.head_dim}, num_heads={self.num_heads}, kernel_size={self.kernel_size}, "
