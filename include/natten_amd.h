@@ -464,6 +464,25 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
                                   float scale, int roles, void* stream);
 
 /*
+ * The same from the forward's output, in two launches: the dq launch comes first, forms delta = rowsum(out * d_out) and the scaled
+ * queries itself, and leaves both and -log2(e) lse for the dk / dv launch in q_scaled (q's shape; neither q nor dq), neg_lse2 and
+ * neg_delta (float32 [batch, heads_q, tokens]; contents irrelevant before, those of natten_amd_backward_prepare behind).
+ * lse [batch, tokens, heads_q] is the forward's.  kv_role_*: the tile shapes of the dk / dv launch, whose key tiles are
+ * then laid out by the windows (`roles` + 8 above), or both null: those of the dq launch.
+ */
+int natten_amd_fna_backward_from_output(const void* q, const void* k, const void* v, const void* out,
+                                        const void* d_out, const float* lse, void* dq, void* dk,
+                                        void* dv, void* q_scaled, float* neg_lse2, float* neg_delta,
+                                        int dtype, int na_dim, int batch, int heads_q, int heads_kv,
+                                        int head_dim, const int32_t* qkv_shape,
+                                        const int32_t* kernel_size, const int32_t* stride,
+                                        const int32_t* dilation, const int32_t* is_causal,
+                                        const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
+                                        const int32_t* kv_role_q_tile_shape,
+                                        const int32_t* kv_role_kv_tile_shape, float scale,
+                                        void* stream);
+
+/*
  * Dense attention backward: q, d_out, dq [batch, seqlen_q, heads_q, head_dim]; k, v, dk, dv
  * [batch, seqlen_kv, heads_kv, head_dim]; neg_lse2 = -log2(e) lse and neg_delta = -delta head-major
  * [batch, heads_q, seqlen_q] (natten_amd_backward_prepare).  q_scaled as above.  q_scaled_filled: two bits, the

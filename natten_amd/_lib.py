@@ -119,6 +119,10 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 10 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 7
         + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
     ),
+    "natten_amd_fna_backward_from_output": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 12 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 9 + [ctypes.c_float, ctypes.c_void_p],
+    ),
     "natten_amd_attention_backward": (
         ctypes.c_int,
         [ctypes.c_void_p] * 10 + [ctypes.c_int] * 9 + [ctypes.c_float, ctypes.c_void_p],
@@ -813,7 +817,7 @@ def fna_backward_fused(
     out: Optional[Tensor] = None,
 ) -> Tuple[Tensor, Tensor, Tensor]:
     """Backward on the original tensors [B, *X, H, D] (lse, delta [B, *X, H]) -> (dq, dk, dv).  With
-    `out` (the forward's output) instead of delta, one pass forms delta and what else the launches read.
+    `out` (the forward's output) instead of delta, the dq launch forms delta and what else the other one reads.
     kv_role_*_tile_shape: tile shapes of the launch that forms dk and dv, whose key tiles are then also laid out
     by the windows; without them it has those of the dq launch (q_tile_shape, kv_tile_shape) and its key tiles lie at
     multiples of their extents."""
@@ -827,27 +831,42 @@ def fna_backward_fused(
     if (kv_role_q_tile_shape is None) != (kv_role_kv_tile_shape is None):
         raise ValueError("kv_role_q_tile_shape and kv_role_kv_tile_shape must be given together.")
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    problem = tuple(tuple(x) for x in (kernel_size, stride, dilation, is_causal))
+    layout = tuple(q.shape[1 : 1 + na_dim])
+    role = kv_role_q_tile_shape is not None
     if out is not None:
-        delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
-    else:
-        lse, delta = _head_major(lse, delta)
+        # the dq launch comes first and leaves what the dk / dv launch reads: the scaled queries, LSE and delta
+        _require_gpu(q, k, v, out, d_out, lse)
+        if out.dtype != q.dtype or d_out.dtype != q.dtype or out.shape != q.shape or d_out.shape != q.shape:
+            raise ValueError("out and d_out must be of q's shape and dtype.")
+        if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
+            raise ValueError("lse must be float32 of q's shape without the last dimension.")
+        q_scaled, rows = torch.empty_like(q), torch.empty((2, lse.numel()), dtype=torch.float32, device=q.device)
+        arrays = _problem_arrays(layout, *problem, tuple(q_tile_shape), tuple(kv_tile_shape),
+                                 *((tuple(kv_role_q_tile_shape), tuple(kv_role_kv_tile_shape)) if role else ()))
+        with _on_device(q):
+            _check(L.natten_amd_fna_backward_from_output(
+                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), dq.data_ptr(),
+                dk.data_ptr(), dv.data_ptr(), q_scaled.data_ptr(), rows.data_ptr(), rows.data_ptr() + 4 * lse.numel(),
+                DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2], q.shape[-1], *arrays, *(() if role else (None, None)),
+                float(scale), _stream(q)))
+        return dq, dk, dv
+    lse, delta = _head_major(lse, delta)
     _require_gpu(q, k, v, d_out, lse, delta)
-    prepared = (4 if out is not None else 0) + (8 if kv_role_q_tile_shape is not None else 0)
-    same = kv_role_q_tile_shape is None or (
+    same = not role or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
     # The dk / dv launch streams the queries as the forward kernel multiplied them (scaled, rounded
     # once) from a workspace of q's size that the call fills first; dq serves as that workspace, so
     # the launch that writes dq comes last.
     launches = [(3, q_tile_shape, kv_tile_shape)] if same else [
         (2, kv_role_q_tile_shape, kv_role_kv_tile_shape), (1, q_tile_shape, kv_tile_shape)]
-    problem = tuple(tuple(x) for x in (kernel_size, stride, dilation, is_causal))
     with _on_device(q):
         for roles, qt, kt in launches:
             rc = L.natten_amd_fna_backward_fused(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2],
-                q.shape[-1], *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), *problem, tuple(qt), tuple(kt)), float(scale),
-                roles + prepared, _stream(q),
+                q.shape[-1], *_problem_arrays(layout, *problem, tuple(qt), tuple(kt)), float(scale), roles + (8 if role else 0),
+                _stream(q),
             )
             _check(rc)
     return dq, dk, dv

@@ -63,6 +63,11 @@ struct FnaBwdParams {
   const float* delta;
   int prepared;
   float lse_mul, delta_mul;
+  // dQ launches that come first (RAW instances of that role, original layout): the forward's output and its LSE [batch,
+  // tokens, heads].  The launch forms both values of its rows itself and leaves them, and its scaled queries, in `lse`, `delta`
+  // and `qs` for the launch behind it.
+  const void* out;
+  const float* lse_rows;
   void* dq;
   void* dk;
   void* dv;
@@ -325,6 +330,22 @@ static __device__ __forceinline__ bool locate_packed_tile(const int2* __restrict
   return true;
 }
 
+// sum_e a[e] b[e] of eight elements in order, in float.  (One routine for whoever forms delta: the compiler makes pairwise
+// products of fp16 of some such loops and not of others, and the routes promise each other's bits.)
+template <typename T>
+static __device__ __forceinline__ float dot8(typename Mma<T>::vec8 a, typename Mma<T>::vec8 b) {
+  float s = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    if constexpr (std::is_same<T, _Float16>::value) {
+      s = __builtin_amdgcn_fdot2(typename Mma<T>::vec2{a[e], a[e + 1]}, typename Mma<T>::vec2{b[e], b[e + 1]}, s, false);
+    } else {
+      s = __builtin_fmaf(float(a[e + 1]), float(b[e + 1]), __builtin_fmaf(float(a[e]), float(b[e]), s));
+    }
+  }
+  return s;
+}
+
 // Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to).  Of the
 // SIMD's 512 registers a lane, the key-stationary and the dQ instance take 224 and 256 at head dim 128, 229 and
 // 210 at 64, 168 and 167 at 32; the dQ instance at 128 spills 9 more (11 where sequences end inside a tile).  One wave
@@ -339,8 +360,11 @@ constexpr int bwd_waves_per_simd(int head_dim) { return head_dim > 32 ? 2 : 3; }
 // of a sequence are gathered from its last row; stationary ones store nothing, streamed ones are masked.
 // (Padding the sequences into copies first made 67 launches of a packed training step, of index arithmetic
 // and copies most of them: 10 sequences of 1 .. 2048, H 16 / 4, D 128 919 us, now 6 launches and 424 us.)
-// RAW (key-stationary roles): LSE and delta as they are, scaled on the way from LDS to the accumulators
-// (the dQ role scales its two values per lane in every instance).
+// RAW: in the key-stationary roles LSE and delta as they are, scaled on the way from LDS to the accumulators
+// (the dQ role scales its two values per lane in every instance).  In the dQ role the launch that comes first and prepares the other's
+// arrays (see FnaBwdParams::out): a pass of its own over q, out and d_out reads two of them once more and is waited for
+// (the pass and both launches / both launches, us: 4 x 56 x 56, 7 x 7, H 8, D 32 74.2 / 69.5; 96 x 96, 24 x 24, stride 8, H 8, D 64 91 / 83; 128 x 128,
+// 32 x 32, stride 16, H 16, D 128 594 / 573; 29 x 46 x 78, 9 x 24 x 24, dilated, H 8 12340 / 12270).
 template <typename T, int D, int ROLE, bool RAGGED = false, bool RAW = false>
 __global__ void __launch_bounds__(ROLE == kBwdPair ? 512 : 256)
 __attribute__((amdgpu_waves_per_eu(bwd_waves_per_simd(D), bwd_waves_per_simd(D))))
@@ -554,11 +578,14 @@ fna_bwd_kernel(const FnaBwdParams p) {
   const T* x1 = reinterpret_cast<const T*>(KV_STATIONARY ? ((PAIR && part) ? p.v : p.k) : p.q) + a_row * a_stride +
                 int64_t(head_a) * D + g * 8;
   const T* x2 = reinterpret_cast<const T*>(KV_STATIONARY ? p.v : p.d_out) + a_row * a_stride + int64_t(head_a) * D + g * 8;
-  vec8 x1f[KSTEPS], x2f[HAS_DS ? KSTEPS : 1];
+  constexpr bool FIRST = ROLE == kBwdDQ && RAW;
+  vec8 x1f[KSTEPS], x2f[HAS_DS ? KSTEPS : 1], of[FIRST ? KSTEPS : 1];
 #pragma unroll
   for (int ks = 0; ks < KSTEPS; ++ks) {
     x1f[ks] = *reinterpret_cast<const vec8*>(x1 + ks * 16);
     if constexpr (HAS_DS) x2f[ks] = *reinterpret_cast<const vec8*>(x2 + ks * 16);
+    if constexpr (FIRST)
+      of[ks] = *reinterpret_cast<const vec8*>(reinterpret_cast<const T*>(p.out) + a_row * a_stride + int64_t(head_a) * D + g * 8 + ks * 16);
   }
   __builtin_amdgcn_sched_barrier(0);
 
@@ -843,8 +870,21 @@ fna_bwd_kernel(const FnaBwdParams p) {
   if constexpr (!KV_STATIONARY) {
     const int64_t stat_idx = p.fused ? (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok
                                      : stat_row_q + head_a * stat_head_stride + a_seq_row;
-    lse_l = p.lse[stat_idx] * p.lse_mul;
-    delta_l = p.delta[stat_idx] * p.delta_mul;
+    if constexpr (FIRST) {
+      // (added up as delta_kernel does: eight elements in order, then halves of the row)
+      float sum[KSTEPS];
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) sum[ks] = dot8<T>(of[ks], x2f[ks]);
+#pragma unroll
+      for (int o = KSTEPS / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int ks = 0; ks < o; ++ks) sum[ks] += sum[ks + o];
+      delta_l = -(sum[0] + __shfl_xor(sum[0], 32));
+      lse_l = -kLog2e * p.lse_rows[a_row * heads_a + head_a];
+    } else {
+      lse_l = p.lse[stat_idx] * p.lse_mul;
+      delta_l = p.delta[stat_idx] * p.delta_mul;
+    }
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ++ks) x1f[ks] = scale_query_fragment<T>(x1f[ks], p.scale * kLog2e);
   }
@@ -1218,6 +1258,18 @@ fna_bwd_kernel(const FnaBwdParams p) {
   }
   wait_vmcnt<0>();
 
+  if constexpr (FIRST) {
+    if (a_valid) {
+      T* qs = const_cast<T*>(reinterpret_cast<const T*>(p.qs)) + a_row * a_stride + int64_t(head_a) * D + g * 8;
+#pragma unroll
+      for (int ks = 0; ks < KSTEPS; ++ks) *reinterpret_cast<vec8*>(qs + ks * 16) = x1f[ks];
+      if (g == 0) {
+        const int64_t stat_idx = (int64_t(b_orig) * p.heads_q + head_a) * p.tokens + a_tok;
+        const_cast<float*>(p.lse)[stat_idx] = lse_l;
+        const_cast<float*>(p.delta)[stat_idx] = delta_l;
+      }
+    }
+  }
   // dQ = scale * sum_k dS k;  dK = scale * sum_q dS q = ln 2 * sum_q dS q'
   store_results(acc1, acc2, KV_STATIONARY ? 0.6931471805599453f : p.scale);
 }
@@ -1287,8 +1339,7 @@ __global__ void __launch_bounds__(256) bwd_prepare_kernel(const T* __restrict__ 
       const vec8 x = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(out + at));
       const vec8 y = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(d_out + at));
       const vec8 z = __builtin_nontemporal_load(reinterpret_cast<const vec8*>(q + at));
-#pragma unroll
-      for (int e = 0; e < 8; ++e) s += float(x[e]) * float(y[e]);
+      s = dot8<T>(x, y);
       *reinterpret_cast<vec8*>(qs + at) = scale_query_fragment<T>(z, c_log2);
     }
 #pragma unroll
@@ -1310,16 +1361,13 @@ __global__ void __launch_bounds__(256) bwd_prepare_kernel(const T* __restrict__ 
 template <typename T, int D>
 __global__ void __launch_bounds__(256) delta_kernel(const T* out, const T* d_out, float* delta, int64_t items) {
   constexpr int LPI = D / 8;  // lanes per item
-  typedef T tx8 __attribute__((ext_vector_type(8)));
+  using tx8 = typename Mma<T>::vec8;
   const int64_t gtid = int64_t(blockIdx.x) * 256 + threadIdx.x;
   const int64_t item = gtid / LPI;
   const int part = int(gtid % LPI);
   float s = 0.f;
   if (item < items) {
-    const tx8 a = *reinterpret_cast<const tx8*>(out + item * D + part * 8);
-    const tx8 b = *reinterpret_cast<const tx8*>(d_out + item * D + part * 8);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) s += float(a[i]) * float(b[i]);
+    s = dot8<T>(*reinterpret_cast<const tx8*>(out + item * D + part * 8), *reinterpret_cast<const tx8*>(d_out + item * D + part * 8));
   }
 #pragma unroll
   for (int o = LPI / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);

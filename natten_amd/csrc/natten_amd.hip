@@ -1171,6 +1171,17 @@ static SideStream* fork_side_stream(hipStream_t stream) {
   return &s;
 }
 
+// The dQ launch that comes first (see FnaBwdParams::out)
+template <typename T, int D>
+static int launch_bwd_first(const FnaBwdParams& params, hipStream_t stream) {
+  FnaBwdParams p = params;
+  const long long wgs = ((long long)p.batch * p.heads_q * prod3(p.q_tiled) + kNumXcd - 1) / kNumXcd * kNumXcd;
+  set_bwd_divisions(p);
+  if (wgs > 0x7fffffffLL) return fail("fna_backward: problem needs more than 2^31 workgroups");
+  hipLaunchKernelGGL((fna_bwd_kernel<T, D, kBwdDQ, false, true>), dim3((unsigned)wgs), dim3(256), 0, stream, p);
+  return check_launch("fna_backward (dQ)");
+}
+
 template <typename T, int D, bool RAGGED, bool RAW>
 static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
   FnaBwdParams p = params;
@@ -1236,6 +1247,7 @@ static int launch_bwd(const FnaBwdParams& params, hipStream_t stream) {
 
 template <typename T, int D>
 static int dispatch_bwd_form(const FnaBwdParams& p, hipStream_t stream, bool ragged) {
+  if (p.out != nullptr) return launch_bwd_first<T, D>(p, stream);
   if (ragged) return launch_bwd<T, D, true, false>(p, stream);  // (dense attention: prepared arrays only)
   return p.prepared ? launch_bwd<T, D, false, false>(p, stream) : launch_bwd<T, D, false, true>(p, stream);
 }
@@ -1347,14 +1359,14 @@ int natten_amd_fna_backward(const void* q, const void* k, const void* v, const v
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
 }
 
-int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
-                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
-                                  int batch, int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
-                                  const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
-                                  const int32_t* is_causal, const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
-                                  float scale, int roles, void* stream) {
-  g_error[0] = 0;
-  const char* what = "fna_backward_fused";
+// Launches of the backward on the original tensors.  out, lse_rows: those of the launch that comes first (roles = 1), else null
+static int fna_backward_fused_launches(const char* what, const void* q, const void* k, const void* v, const void* out,
+                                       const float* lse_rows, const void* d_out, const float* lse, const float* delta, void* dq,
+                                       void* dk, void* dv, void* q_scaled, int dtype, int na_dim, int batch, int heads_q,
+                                       int heads_kv, int head_dim, const int32_t* qkv_shape, const int32_t* kernel_size,
+                                       const int32_t* stride, const int32_t* dilation, const int32_t* is_causal,
+                                       const int32_t* q_tile_shape, const int32_t* kv_tile_shape, float scale, int roles,
+                                       void* stream) {
   if (roles < 1 || roles > 15 || (roles & 3) == 0)
     return fail("%s: roles must be 1 (dq), 2 (dk and dv) or 3 (all), plus 4 for prepared arrays, plus 8 for key tiles laid out "
                 "by the windows, got %d",
@@ -1448,7 +1460,46 @@ int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, c
   p.tokens = int(tokens);
   p.roles = roles;
   p.prepared = (roles & 4) != 0;
+  p.out = out;
+  p.lse_rows = lse_rows;
   return dispatch_bwd(p, dtype, head_dim, static_cast<hipStream_t>(stream));
+}
+
+int natten_amd_fna_backward_fused(const void* q, const void* k, const void* v, const void* d_out, const float* lse,
+                                  const float* delta, void* dq, void* dk, void* dv, void* q_scaled, int dtype, int na_dim,
+                                  int batch, int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
+                                  const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
+                                  const int32_t* is_causal, const int32_t* q_tile_shape, const int32_t* kv_tile_shape,
+                                  float scale, int roles, void* stream) {
+  g_error[0] = 0;
+  return fna_backward_fused_launches("fna_backward_fused", q, k, v, nullptr, nullptr, d_out, lse, delta, dq, dk, dv, q_scaled, dtype,
+                                     na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape, kernel_size, stride, dilation, is_causal,
+                                     q_tile_shape, kv_tile_shape, scale, roles, stream);
+}
+
+int natten_amd_fna_backward_from_output(const void* q, const void* k, const void* v, const void* out, const void* d_out,
+                                        const float* lse, void* dq, void* dk, void* dv, void* q_scaled, float* neg_lse2,
+                                        float* neg_delta, int dtype, int na_dim, int batch, int heads_q, int heads_kv,
+                                        int head_dim, const int32_t* qkv_shape, const int32_t* kernel_size, const int32_t* stride,
+                                        const int32_t* dilation, const int32_t* is_causal, const int32_t* q_tile_shape,
+                                        const int32_t* kv_tile_shape, const int32_t* kv_role_q_tile_shape,
+                                        const int32_t* kv_role_kv_tile_shape, float scale, void* stream) {
+  g_error[0] = 0;
+  const char* what = "fna_backward_from_output";
+  if (!out || !lse || !neg_lse2 || !neg_delta || !q_scaled) return fail("%s: null pointer argument", what);
+  if (reinterpret_cast<uintptr_t>(out) & 15) return fail("%s: out must be 16-byte aligned", what);
+  if (q_scaled == dq) return fail("%s: q_scaled must not be dq (the dq launch comes first)", what);
+  if ((kv_role_q_tile_shape == nullptr) != (kv_role_kv_tile_shape == nullptr))
+    return fail("%s: the tile shapes of the dk / dv launch must be given together", what);
+  if (int rc = fna_backward_fused_launches(what, q, k, v, out, lse, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, dtype, na_dim,
+                                           batch, heads_q, heads_kv, head_dim, qkv_shape, kernel_size, stride, dilation, is_causal,
+                                           q_tile_shape, kv_tile_shape, scale, 1 + 4, stream))
+    return rc;
+  const bool own = kv_role_q_tile_shape != nullptr;
+  return fna_backward_fused_launches(what, q, k, v, nullptr, nullptr, d_out, neg_lse2, neg_delta, dq, dk, dv, q_scaled, dtype, na_dim,
+                                     batch, heads_q, heads_kv, head_dim, qkv_shape, kernel_size, stride, dilation, is_causal,
+                                     own ? kv_role_q_tile_shape : q_tile_shape, own ? kv_role_kv_tile_shape : kv_tile_shape, scale,
+                                     2 + 4 + (own ? 8 : 0), stream);
 }
 
 namespace {
