@@ -297,16 +297,16 @@ static __device__ __forceinline__ void async_copy16_uniform(uint64_t base, uint3
 template <int BYTES>
 static __device__ __forceinline__ void touch_launch_params() {
   constexpr int LINES = (BYTES + 63) / 64;
-  static_assert(LINES >= 8 && LINES <= 12, "eight loads, or four more");
+  static_assert(LINES <= 12, "eight loads, or four more");
   constexpr auto at = [](int i) { return 64 * (i < LINES ? i : LINES - 1); };
   const uint64_t args = uint64_t(reinterpret_cast<uintptr_t>((const void*)__builtin_amdgcn_kernarg_segment_ptr()));
   uint32_t x[8], y[4] = {0, 0, 0, 0};
   asm volatile(
-      "s_load_dword %0, %8, 0x0\n\ts_load_dword %1, %8, 0x40\n\ts_load_dword %2, %8, 0x80\n\ts_load_dword %3, %8, 0xc0\n\t"
-      "s_load_dword %4, %8, 0x100\n\ts_load_dword %5, %8, 0x140\n\ts_load_dword %6, %8, 0x180\n\ts_load_dword %7, %8, 0x1c0\n\t"
+      "s_load_dword %0, %8, %9\n\ts_load_dword %1, %8, %10\n\ts_load_dword %2, %8, %11\n\ts_load_dword %3, %8, %12\n\t"
+      "s_load_dword %4, %8, %13\n\ts_load_dword %5, %8, %14\n\ts_load_dword %6, %8, %15\n\ts_load_dword %7, %8, %16\n\t"
       "s_waitcnt lgkmcnt(0)"
       : "=&s"(x[0]), "=&s"(x[1]), "=&s"(x[2]), "=&s"(x[3]), "=&s"(x[4]), "=&s"(x[5]), "=&s"(x[6]), "=&s"(x[7])
-      : "s"(args));
+      : "s"(args), "n"(at(0)), "n"(at(1)), "n"(at(2)), "n"(at(3)), "n"(at(4)), "n"(at(5)), "n"(at(6)), "n"(at(7)));
   if constexpr (LINES > 8)
     asm volatile(
         "s_load_dword %0, %4, %5\n\ts_load_dword %1, %4, %6\n\ts_load_dword %2, %4, %7\n\ts_load_dword %3, %4, %8\n\t"

@@ -260,7 +260,7 @@ inline void choose_f32_boxes(FnaF32Params& p) {
 // window costs 256 keys a query, where a 128-query tile over 64-key tiles at multiples of their extent
 // costs 1024.  Each 16 x D block of K and of V goes straight from memory (mostly L1 / L2: neighbouring waves read
 // nearly the same keys) to the registers the matrix instruction reads, 8 D bytes per lane group against
-// 16 D matrix cycles, one block ahead of its use.
+// 16 D matrix cycles, half a block ahead of its use or more; the loads add a lane's constant distances to a uniform base.
 //
 // v_mfma_f32_16x16x4_f32: with i = lane % 16, g = lane / 16 the A operand holds row i, the B operand
 // column i, k-index g; the result's register r is row 4 g + r, column i.  S^T = K Q^T: which head-dim
@@ -271,15 +271,17 @@ inline void choose_f32_boxes(FnaF32Params& p) {
 // V operands and results are VEC-wide loads and stores of whole rows.
 // Softmax in float32; a row's maximum is followed once it grew by more than 2^8 (exact: the sums are
 // normalised by the same maximum).
-// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 54 us (53 TFLOP/s of window pairs, 80 of pairs
+// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 51 us (56 TFLOP/s of window pairs, 85 of pairs
 // multiplied; the card's float32 matrix products reach 154), 300 us as permutes, 128-query kernel and
-// unpermutes; 256 tokens, H 2, D 32, window 7: 17 us, all of it the call, from 83.
-template <int D, bool PAD>
+// unpermutes.  Of a wave's 81000 cycles there 63000 are its fifteen blocks, the matrix pipe full with four waves a SIMD,
+// and 16000 the set-up and the way of the first block; 256 tokens, H 2, D 32, window 7: 17 us, all of it the call, from 83.
+template <int D, bool PAD, bool WIDE = false, int SETS = (D == 32 ? 2 : 1)>
 __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32Params p) {
   constexpr int KJ = D / 16;
   constexpr int VEC = KJ < 4 ? KJ : 4;
   constexpr int NH = D / (16 * VEC);
   typedef float fvec __attribute__((ext_vector_type(VEC)));
+  touch_launch_params<sizeof(FnaF32Params)>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
   const int i16 = lane & 15, g = lane >> 4;
@@ -297,36 +299,25 @@ __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32
 
   int extent[3], step[3], org0[3], nblk[3], full_lo[3], full_hi[3];
   int ws[3], width[3];  // this lane's query: window start and length
-  int kc[3], vc[3][4];  // in-block coordinates of the lane's key row (K) and of its four logits' keys (V)
   int q_tok = 0, group_tok = 0;
   bool valid = true;
   {
-    int q_in = i16, k_in = i16;
+    int q_in = i16;
     int bc[3];
     const int t01 = na_div(box, p.d_q_boxes[2]);
     bc[2] = box - t01 * p.q_boxes[2];
     bc[0] = na_div(t01, p.d_q_boxes[1]);
     bc[1] = t01 - bc[0] * p.q_boxes[1];
     bool empty = false;
-    int v_in = 4 * g;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) vc[0][r] = v_in + r;
 #pragma unroll
     for (int a = 2; a >= 0; --a) {
       const int off = q_in & ((1 << p.q_lg[a]) - 1);
       q_in >>= p.q_lg[a];
-      kc[a] = k_in & ((1 << p.kv_lg[a]) - 1);
-      k_in >>= p.kv_lg[a];
-      if (a > 0) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          vc[a][r] = vc[0][r] & ((1 << p.kv_lg[a]) - 1);
-          vc[0][r] >>= p.kv_lg[a];
-        }
-      }
       bc[a] = (bc[a] << p.q_lg[a]);
       ws[a] = off;
     }
+    // One window evaluation per dimension: a lane's own query.  The box's first query is lane 0's, its last one lane 15's (queries
+    // past the group act as its last one and are not stored).
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const int rest = na_div(gl, p.d_dil[a]);
@@ -337,19 +328,17 @@ __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32
       group_tok += gi * p.tok_stride[a];
       empty = empty || bc[a] >= extent[a];  // (groups may be one shorter than the boxes were counted for)
       const bool c = p.causal[a] != 0;
-      const int qf = na_min(bc[a], extent[a] - 1);
-      const int ql = na_min(bc[a] + (1 << p.q_lg[a]) - 1, extent[a] - 1);
-      const int st_f = na_window_start(qf, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
-      const int st_l = na_window_start(ql, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
-      org0[a] = st_f;
-      full_lo[a] = st_l;
-      full_hi[a] = na_window_end(qf, st_f, p.ksize[a], extent[a], c);
-      nblk[a] = (na_window_end(ql, st_l, p.ksize[a], extent[a], c) - st_f + (1 << p.kv_lg[a]) - 1) >> p.kv_lg[a];
       const int qc = bc[a] + ws[a];
       valid = valid && qc < extent[a];
-      const int q = na_min(qc, extent[a] - 1);  // queries past the group act as its last one and are not stored
-      ws[a] = na_window_start(q, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
-      width[a] = na_window_end(q, ws[a], p.ksize[a], extent[a], c) - ws[a];
+      const int q = na_min(qc, extent[a] - 1);
+      const int start = na_window_start(q, p.ksize[a], p.stride[a], p.d_stride[a], extent[a], c);
+      const int end = na_window_end(q, start, p.ksize[a], extent[a], c);
+      ws[a] = start;
+      width[a] = end - start;
+      org0[a] = __builtin_amdgcn_readlane(start, 0);
+      full_hi[a] = __builtin_amdgcn_readlane(end, 0);
+      full_lo[a] = __builtin_amdgcn_readlane(start, 15);
+      nblk[a] = (__builtin_amdgcn_readlane(end, 15) - org0[a] + (1 << p.kv_lg[a]) - 1) >> p.kv_lg[a];
       q_tok += q * step[a];
     }
     if (empty) return;
@@ -376,89 +365,156 @@ __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32
     for (int c = 0; c < VEC; ++c) acc[h][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;
 
-  // a lane's rows of a block that lies inside the group: fixed distances from the block's first token
-  int64_t k_off = 0, v_off[4] = {0, 0, 0, 0};
+  // A lane's rows of a block: 32-bit byte distances from the block's first token, which the load instructions add to a uniform
+  // base (the launch takes blocks that span less than 2^32 bytes; WIDE: longer ones, with addresses of their own).
+  using Offset = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+  const uint32_t row_bytes = uint32_t(kv_row) * 4u;
+  // the row with coordinates `c` inside a block that begins at `org` (those past the group are masked: its last ones are
+  // read in their place)
+  auto row_offset = [&](const int (&c)[3], const int (&org)[3], bool clamp) __attribute__((always_inline)) {
+    Offset o = 0;
 #pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    k_off += int64_t(kc[a] * step[a]) * kv_row;
+    for (int a = 0; a < 3; ++a)
+      o += Offset(uint32_t((clamp ? na_min(c[a], extent[a] - 1 - org[a]) : c[a]) * step[a])) * row_bytes;
+    return o;
+  };
+  // coordinates inside a block of key `k` (dimension 2 fastest)
+  auto key_coordinates = [&](int k, int (&c)[3]) __attribute__((always_inline)) {
+    c[2] = k & ((1 << p.kv_lg[2]) - 1);
+    k >>= p.kv_lg[2];
+    c[1] = k & ((1 << p.kv_lg[1]) - 1);
+    c[0] = k >> p.kv_lg[1];
+  };
+  // (at the group's edge formed from the lane number each time: such blocks are few, and fifteen coordinates kept for them are
+  // a wave per SIMD less)
+  auto lane_number = [&]() __attribute__((always_inline)) {
+    uint32_t l = uint32_t(lane);
+    pin(l);
+    return l;
+  };
+  auto k_offset = [&](const int (&org)[3], bool clamp = true) __attribute__((always_inline)) {
+    const uint32_t l = lane_number();
+    int c[3];
+    key_coordinates(int(l & 15), c);
+    return row_offset(c, org, clamp) + (l >> 4) * 16;
+  };
+  auto v_offsets = [&](const int (&org)[3], Offset (&vo)[4], bool clamp = true) __attribute__((always_inline)) {
+    const uint32_t l = lane_number();
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v_off[r] += int64_t(vc[a][r] * step[a]) * kv_row;
+    for (int r = 0; r < 4; ++r) {
+      int c[3];
+      key_coordinates(int(l >> 4) * 4 + r, c);
+      vo[r] = row_offset(c, org, clamp) + (l & 15) * (4 * VEC);
+    }
+  };
+  const Offset k_off = k_offset(org0, false);
+  Offset v_off[4];
+  v_offsets(org0, v_off, false);
+  int v_rel[3][4];  // in-block coordinates of the lane's four keys less its window's start
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    int c[3];
+    key_coordinates(4 * g + r, c);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) v_rel[a][r] = c[a] - ws[a];
   }
 
-  struct Block {
-    f32x4_t k[KJ];
-    fvec v[4][NH];
-    int org[3];
-    bool full;
-  };
-  int it[3] = {0, 0, 0};
-  auto load = [&](Block& t) {
-    bool inside = true;
-    t.full = true;
-    int64_t row0 = 0;
+  // A block's K rows are read by S = K Q^T, its V rows by O += V^T P^T half a block later, and the rows of the block SETS
+  // further on take their registers from then on: one set where the products of half a block are long enough to wait for
+  // memory, and the registers saved are a wave more per SIMD at head dim 64 (2 x 64 x 64, H 8, 13 x 13: 54 us as two sets of whole
+  // blocks, now 51; at 128, 48 x 80, 21 x 17, stride 2 x 4, H 8: 116 and 95; 2 x 8192, 257, stride 8, H 8: 221 and 188), two at head
+  // dim 32 (12 x 24 x 30, 5 x 7 x 9, dilated, H 4: 43.2 us with one set, 41.4 with two; 96 x 96, 25 x 25, H 6: 126 either way, 134 before).
+  // The loads are not conditional (past the last block they fetch it again, which nothing reads): behind a branch the
+  // wait for rows becomes a wait for everything outstanding.
+  // Blocks are described 64 at a time, one per lane, and read back by lane number (a scalar walk with its edge cases took some
+  // hundred of a block's 133 scalar instructions, as long as its matrix instructions at head dim 32).
+  const int total = nblk[0] * nblk[1] * nblk[2];
+  int d_first = 0, d_row0 = 0, d_org[3] = {0, 0, 0};
+  uint64_t d_full = 0, d_inside = 0;  // by lane: no key needs a mask; all keys lie inside the group
+  auto describe = [&](int first) __attribute__((always_inline)) {
+    d_first = first;
+    int t[3];
+    const int number = na_min(first + lane, total - 1);  // past the last block: that one again, which nothing reads
+    if (__builtin_expect(total < (1 << 24), 1)) {
+      kv_tile_of_box(number, nblk, t);
+    } else {
+      t[2] = number % nblk[2];
+      t[1] = number / nblk[2] % nblk[1];
+      t[0] = number / nblk[2] / nblk[1];
+    }
+    bool full = true, inside = true;
+    d_row0 = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      t.org[a] = org0[a] + (it[a] << p.kv_lg[a]);
-      const int end = t.org[a] + (1 << p.kv_lg[a]);
+      d_org[a] = org0[a] + (t[a] << p.kv_lg[a]);
+      const int end = d_org[a] + (1 << p.kv_lg[a]);
       inside = inside && end <= extent[a];
-      t.full = t.full && t.org[a] >= full_lo[a] && end <= full_hi[a];
-      row0 += int64_t(t.org[a]) * step[a];
+      full = full && d_org[a] >= full_lo[a] && end <= full_hi[a];
+      d_row0 += d_org[a] * step[a];
     }
-    int64_t ko = row0 * kv_row + k_off, vo[4];
+    d_full = __ballot(full);
+    d_inside = __ballot(inside);
+  };
+  // what the loads of a block need
+  struct Place {
+    int row0, org[3];
+    bool inside;
+  };
+  auto place = [&](int n) __attribute__((always_inline)) {
+    const int l = n - d_first;
+    Place t;
+    t.row0 = __builtin_amdgcn_readlane(d_row0, l);
+    t.inside = (d_inside >> l) & 1;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) vo[r] = row0 * kv_row + v_off[r];
-    if (!inside) {
-      // keys past the group are masked: read its last ones in their place
-      int kt = 0, vt[4] = {0, 0, 0, 0};
-#pragma unroll
-      for (int a = 0; a < 3; ++a) {
-        kt += na_min(t.org[a] + kc[a], extent[a] - 1) * step[a];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) vt[r] += na_min(t.org[a] + vc[a][r], extent[a] - 1) * step[a];
-      }
-      ko = int64_t(kt) * kv_row;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) vo[r] = int64_t(vt[r]) * kv_row;
-    }
+    for (int a = 0; a < 3; ++a) t.org[a] = __builtin_amdgcn_readlane(d_org[a], l);
+    return t;
+  };
+  f32x4_t kf[SETS][KJ];
+  fvec vf[SETS][4][NH];
+  auto load_k = [&](int set, const Place& t) __attribute__((always_inline)) {
+    Offset ko = k_off;
+    if (!t.inside) ko = k_offset(t.org);
+    const char* kb = reinterpret_cast<const char*>(kbase + int64_t(t.row0) * kv_row);
 #pragma unroll
     for (int j = 0; j < KJ; ++j) {
-      if constexpr (PAD) t.k[j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (!PAD || 16 * j + 4 * g < p.head_dim) t.k[j] = *reinterpret_cast<const f32x4_t*>(kbase + ko + 16 * j + 4 * g);
+      if constexpr (PAD) kf[set][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (!PAD || 16 * j + 4 * g < p.head_dim) kf[set][j] = *reinterpret_cast<const f32x4_t*>(kb + ko + 64 * j);
     }
+  };
+  auto load_v = [&](int set, const Place& t) __attribute__((always_inline)) {
+    Offset vo[4] = {v_off[0], v_off[1], v_off[2], v_off[3]};
+    if (!t.inside) v_offsets(t.org, vo);
+    const char* vb = reinterpret_cast<const char*>(vbase + int64_t(t.row0) * kv_row);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
       for (int h = 0; h < NH; ++h) {
-        const int d = VEC * (16 * h + i16);
-        if constexpr (PAD) t.v[r][h] = fvec(0.f);
-        if (!PAD || d < p.head_dim) t.v[r][h] = *reinterpret_cast<const fvec*>(vbase + vo[r] + d);
+        if constexpr (PAD) vf[set][r][h] = fvec(0.f);
+        if (!PAD || VEC * (16 * h + i16) < p.head_dim) vf[set][r][h] = *reinterpret_cast<const fvec*>(vb + vo[r] + 64 * VEC * h);
       }
-    if (++it[2] == nblk[2]) {
-      it[2] = 0;
-      if (++it[1] == nblk[1]) {
-        it[1] = 0;
-        ++it[0];
-      }
-    }
   };
-  auto multiply = [&](const Block& t) {
+
+  auto block = [&](int n, int set) __attribute__((always_inline)) {
     f32x4_t S = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < KJ; ++j) {
       if (PAD && 16 * j >= p.head_dim) break;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) S = __builtin_amdgcn_mfma_f32_16x16x4f32(t.k[j][e], qf[j][e], S, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) S = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[set][j][e], qf[j][e], S, 0, 0, 0);
     }
-    if (!t.full) {
+    if (!((d_full >> (n - d_first)) & 1)) {
+      const Place here = place(n);
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
         if (a < p.dims) {
-          const int lo = ws[a] - t.org[a];
 #pragma unroll
-          for (int r = 0; r < 4; ++r) S[r] = uint32_t(vc[a][r] - lo) < uint32_t(width[a]) ? S[r] : -INFINITY;
+          for (int r = 0; r < 4; ++r) S[r] = uint32_t(v_rel[a][r] + here.org[a]) < uint32_t(width[a]) ? S[r] : -INFINITY;
         }
       }
     }
+    if (n + SETS - d_first >= 64) describe(n + 1);
+    const Place next = place(n + SETS);
+    load_k(set, next);
     const float mx_own = fmaxf(fmaxf(S[0], S[1]), fmaxf(S[2], S[3]));
     if (__ballot(mx_own > m_run + kLazyRescaleLog2) != 0) {
       float mx = fmaxf(mx_own, __shfl_xor(mx_own, 16));
@@ -481,22 +537,18 @@ __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32
 #pragma unroll
       for (int h = 0; h < NH; ++h)
 #pragma unroll
-        for (int c = 0; c < VEC; ++c) acc[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(t.v[r][h][c], S[r], acc[h][c], 0, 0, 0);
+        for (int c = 0; c < VEC; ++c) acc[h][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[set][r][h][c], S[r], acc[h][c], 0, 0, 0);
+    load_v(set, next);
   };
-
-  // Two blocks in registers: while one is multiplied the other is on its way.  The loads are not
-  // conditional (past the last block they fetch clamped rows that nothing reads): behind a branch the wait for
-  // a block becomes a wait for everything outstanding, the next block included (62.6 us instead of 54.0).
-  Block A, B;
-  const int total = nblk[0] * nblk[1] * nblk[2];
-  load(A);
-  for (int n = 0;; n += 2) {
-    load(B);
-    multiply(A);
-    if (n + 1 >= total) break;
-    load(A);
-    multiply(B);
-    if (n + 2 >= total) break;
+  describe(0);
+#pragma unroll
+  for (int i = 0; i < SETS; ++i) {
+    load_k(i, place(i));
+    load_v(i, place(i));
+  }
+  for (int n = 0; n < total; n += SETS) {
+    block(n, 0);
+    if (SETS > 1 && n + 1 < total) block(n + 1, SETS - 1);
   }
 
   float l = l_run + __shfl_xor(l_run, 16);

@@ -659,6 +659,24 @@ int natten_amd_fna_forward_fused(const void* q, const void* k, const void* v, vo
                                 k_scale, v_scale, anchor_kv_tiles, queues, stream);
 }
 
+extern "C++" {
+template <bool WIDE>
+static void launch_f32_direct(const FnaF32Params& p, dim3 grid, hipStream_t s) {
+  switch (p.head_dim) {
+    case 32: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, false, WIDE>), grid, dim3(256), 0, s, p); break;
+    case 64: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, false, WIDE>), grid, dim3(256), 0, s, p); break;
+    case 128: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, false, WIDE>), grid, dim3(256), 0, s, p); break;
+    default:
+      if (p.head_dim < 32)
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, true, WIDE>), grid, dim3(256), 0, s, p);
+      else if (p.head_dim < 64)
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, true, WIDE>), grid, dim3(256), 0, s, p);
+      else
+        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, true, WIDE>), grid, dim3(256), 0, s, p);
+  }
+}
+}  // extern "C++"
+
 int natten_amd_fna_forward_f32(const void* q, const void* k, const void* v, void* out, float* lse, int na_dim, int batch,
                                int heads_q, int heads_kv, int head_dim, const int32_t* qkv_shape,
                                const int32_t* kernel_size, const int32_t* stride, const int32_t* dilation,
@@ -730,18 +748,12 @@ int natten_amd_fna_forward_f32(const void* q, const void* k, const void* v, void
   p.d_num_groups = na_make_div(p.num_groups);
   const dim3 grid((unsigned)(wgs_per_xcd * kNumXcd));
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (head_dim) {
-    case 32: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, false>), grid, dim3(256), 0, s, p); break;
-    case 64: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, false>), grid, dim3(256), 0, s, p); break;
-    case 128: hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, false>), grid, dim3(256), 0, s, p); break;
-    default:
-      if (head_dim < 32)
-        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<32, true>), grid, dim3(256), 0, s, p);
-      else if (head_dim < 64)
-        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<64, true>), grid, dim3(256), 0, s, p);
-      else
-        hipLaunchKernelGGL((fna_fwd_f32_direct_kernel<128, true>), grid, dim3(256), 0, s, p);
-  }
+  // A block's rows lie within 32-bit byte offsets of its first one, or the launch takes the instances that form 64-bit ones
+  long long span = 0;
+  for (int a = 0; a < 3; ++a)
+    span += (long long)(na_min(1 << p.kv_lg[a], p.ext_base[a] + (p.ext_rem[a] > 0)) - 1) * p.dil[a] * p.tok_stride[a];
+  if ((span + 1) * heads_kv * head_dim * 4 < (1LL << 32)) launch_f32_direct<false>(p, grid, s);
+  else launch_f32_direct<true>(p, grid, s);
   return check_launch(what);
 }
 
