@@ -577,23 +577,19 @@ int natten_amd_merge_attention_parts(const void* parts, const float* lse_parts, 
  * three tensors [rows, part] (n = number x part; the others null): queries, keys and values as the attention
  * takes them.  k and part are multiples of 64 and at most 32768 columns are taken; tensors are 16-byte aligned, bias
  * and db 8-byte aligned.  Results do not differ from run to run.
- *   forward          y = x w^T + bias
- *   backward_input   dx = dy w
- *   backward_weight  dw = dy^T x and, unless db is null, db = column sums of dy; the workspace holds the float32 sums of
- *                    runs of rows (as many bytes as ..._workspace says, contents irrelevant)
+ *   forward   y = x w^T + bias
+ *   backward  dx = dy w, unless dx is null (w then may be); dw = dy^T x, unless dw is null (x and the workspace then may be);
+ *             db = column sums of dy, unless db is null.  One launch for both products; the workspace holds the float32
+ *             sums of runs of rows of dw and db (as many bytes as ..._workspace says, contents irrelevant)
  */
 int natten_amd_linear_forward(const void* x, const void* w, const void* bias, void* y0, void* y1,
                               void* y2, int dtype, int64_t rows, int n, int k, int part,
                               void* stream);
-int natten_amd_linear_backward_input(const void* dy0, const void* dy1, const void* dy2,
-                                     const void* w, void* dx, int dtype, int64_t rows, int n, int k,
-                                     int part, void* stream);
-int natten_amd_linear_backward_weight_workspace(int64_t rows, int n, int k, int part,
-                                                uint64_t* bytes);
-int natten_amd_linear_backward_weight(const void* dy0, const void* dy1, const void* dy2,
-                                      const void* x, void* dw, void* db, void* workspace,
-                                      uint64_t workspace_bytes, int dtype, int64_t rows, int n,
-                                      int k, int part, void* stream);
+int natten_amd_linear_backward_workspace(int64_t rows, int n, int k, int part, uint64_t* bytes);
+int natten_amd_linear_backward(const void* dy0, const void* dy1, const void* dy2, const void* x,
+                               const void* w, void* dx, void* dw, void* db, void* workspace,
+                               uint64_t workspace_bytes, int dtype, int64_t rows, int n, int k,
+                               int part, void* stream);
 
 /*
  * Diagnostic without a counterpart in the reference: sustained rate of the bf16 matrix

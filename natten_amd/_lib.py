@@ -136,14 +136,10 @@ _SIGNATURES = {
         ctypes.c_int,
         [ctypes.c_void_p] * 6 + [ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
     ),
-    "natten_amd_linear_backward_input": (
+    "natten_amd_linear_backward_workspace": (ctypes.c_int, [ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p]),
+    "natten_amd_linear_backward": (
         ctypes.c_int,
-        [ctypes.c_void_p] * 5 + [ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
-    ),
-    "natten_amd_linear_backward_weight_workspace": (ctypes.c_int, [ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p]),
-    "natten_amd_linear_backward_weight": (
-        ctypes.c_int,
-        [ctypes.c_void_p] * 7 + [ctypes.c_uint64, ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
+        [ctypes.c_void_p] * 9 + [ctypes.c_uint64, ctypes.c_int, ctypes.c_int64] + [ctypes.c_int] * 3 + [ctypes.c_void_p],
     ),
     "natten_amd_token_permute_widen": (
         ctypes.c_int,
@@ -730,40 +726,34 @@ def linear_forward(x: Tensor, weight: Tensor, bias: Optional[Tensor], parts: int
     return outs
 
 
-def linear_backward_input(d_outs, weight: Tensor, shape) -> Tensor:
-    """The gradient of a linear map's input, of `shape`, from those of its `len(d_outs)` outputs."""
-    n, k = weight.shape
-    _require_gpu(weight, *d_outs)
-    dx = torch.empty(shape, dtype=weight.dtype, device=weight.device)
-    with _on_device(weight):
-        _check(lib().natten_amd_linear_backward_input(
-            *_three(d_outs), weight.data_ptr(), dx.data_ptr(), DTYPE_CODES[weight.dtype], dx.numel() // k, n, k,
-            n // len(d_outs), _stream(weight)))
-    return dx
-
-
 @functools.lru_cache(maxsize=1024)
 def _linear_workspace(rows: int, n: int, k: int, part: int) -> int:
     nbytes = ctypes.c_uint64()
-    _check(lib().natten_amd_linear_backward_weight_workspace(rows, n, k, part, ctypes.byref(nbytes)))
+    _check(lib().natten_amd_linear_backward_workspace(rows, n, k, part, ctypes.byref(nbytes)))
     return nbytes.value
 
 
-def linear_backward_weight(d_outs, x: Tensor, shape, want_bias: bool) -> Tuple[Tensor, Optional[Tensor]]:
-    """The gradients of a linear map's weight [n, k] and bias (None unless wanted)."""
-    n, k = shape
-    L = lib()
-    _require_gpu(x, *d_outs)
-    rows = x.numel() // k
-    dw = torch.empty((n, k), dtype=x.dtype, device=x.device)
-    db = torch.empty((n,), dtype=x.dtype, device=x.device) if want_bias else None
-    nbytes = _linear_workspace(rows, n, k, n // len(d_outs))
-    workspace = torch.empty((nbytes // 4,), dtype=torch.float32, device=x.device)
+def linear_backward(d_outs, x: Tensor, weight: Tensor, need_x: bool, need_weight: bool,
+                    need_bias: bool) -> Tuple[Optional[Tensor], Optional[Tensor], Optional[Tensor]]:
+    """The gradients of a linear map's input (of x's shape), weight [n, k] and bias from those of its `len(d_outs)` outputs;
+    None where not needed.  (A bias gradient comes with the weight's.)"""
+    n, k = weight.shape
+    _require_gpu(x, weight, *d_outs)
+    rows, part = x.numel() // k, n // len(d_outs)
+    dx = torch.empty_like(x) if need_x else None
+    dw = db = workspace = None
+    nbytes = 0
+    if need_weight or need_bias:
+        dw = torch.empty_like(weight)
+        db = torch.empty((n,), dtype=x.dtype, device=x.device) if need_bias else None
+        nbytes = _linear_workspace(rows, n, k, part)
+        workspace = torch.empty((nbytes // 4,), dtype=torch.float32, device=x.device)
+    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     with _on_device(x):
-        _check(L.natten_amd_linear_backward_weight(
-            *_three(d_outs), x.data_ptr(), dw.data_ptr(), None if db is None else db.data_ptr(), workspace.data_ptr(), nbytes,
-            DTYPE_CODES[x.dtype], rows, n, k, n // len(d_outs), _stream(x)))
-    return dw, db
+        _check(lib().natten_amd_linear_backward(
+            *_three(d_outs), x.data_ptr(), weight.data_ptr(), ptr(dx), ptr(dw), ptr(db), ptr(workspace), nbytes,
+            DTYPE_CODES[x.dtype], rows, n, k, part, _stream(x)))
+    return dx, dw if need_weight else None, db
 
 
 def _head_major(lse: Tensor, delta: Tensor) -> Tuple[Tensor, Tensor]:

@@ -47,22 +47,25 @@ struct LinearTile {
   static constexpr int CHUNKS = ROWS * E / 8;
 };
 
-// RT, CT: row and column side of a workgroup's tile; four waves in a square
+// Two stages: a third keeps workgroups out of the compute unit (36864 tokens, 512 -> 1536: forward 80 us, 106 with three).
+constexpr int kLinearStep = 64;  // of the contraction
+constexpr int kLinearStages = 2;
+constexpr int linear_lds_bytes(int rt, int ct) { return kLinearStages * (rt + ct) * kLinearStep * 2; }
+
+// One tile of a result, RT rows by CT columns, four waves in a square; `block`: the workgroup's number in this part of a launch (which
+// has a multiple of the XCD count of them), `lds`: linear_lds_bytes(RT, CT).
 template <typename T, int MODE, int RT, int CT>
-__global__ void __launch_bounds__(256) linear_kernel(const LinearParams p) {
+static __device__ __forceinline__ void linear_tile(const LinearParams& p, const int block, char* lds) {
   using M = Mma<T>;
   using vec8 = typename M::vec8;
-  constexpr int STEP = 64;  // of the contraction
+  constexpr int STEP = kLinearStep;
   constexpr bool ROW_TR = MODE == kLinearWeight, COL_TR = MODE != kLinearForward;
   using RowTile = LinearTile<ROW_TR ? STEP : RT, ROW_TR ? RT : STEP>;
   using ColTile = LinearTile<COL_TR ? STEP : CT, COL_TR ? CT : STEP>;
   constexpr int MI = RT / 64, NI = CT / 64;  // 32 x 32 blocks of a wave
-  // Two stages: a third keeps workgroups out of the compute unit (36864 tokens, 512 -> 1536: forward 80 us, 106 with three).
-  constexpr int STAGES = 2;
   constexpr int PER_R = RowTile::CHUNKS / 256, PER_C = ColTile::CHUNKS / 256;
   static_assert(PER_R * 256 == RowTile::CHUNKS && PER_C * 256 == ColTile::CHUNKS, "a tile is a whole number of copies");
-  __shared__ __attribute__((aligned(1024))) char sR[STAGES * RowTile::BYTES];
-  __shared__ __attribute__((aligned(1024))) char sC[STAGES * ColTile::BYTES];
+  char *const sR = lds, *const sC = lds + kLinearStages * RowTile::BYTES;
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -72,8 +75,8 @@ __global__ void __launch_bounds__(256) linear_kernel(const LinearParams p) {
   // the tiles that read the same rows meet in its L2
   const int total = p.row_tiles * p.col_tiles * p.slices;
   const int chunk = (total + kNumXcd - 1) / kNumXcd;
-  const int lin = (int(blockIdx.x) % kNumXcd) * chunk + int(blockIdx.x) / kNumXcd;
-  if (int(blockIdx.x) / kNumXcd >= chunk || lin >= total) return;
+  const int lin = (block % kNumXcd) * chunk + block / kNumXcd;
+  if (block / kNumXcd >= chunk || lin >= total) return;
   const int rt = na_div(lin, p.d_col_tiles);
   const int col0 = (lin - rt * p.col_tiles) * CT;
   const int slice = MODE == kLinearWeight ? na_div(rt, p.d_row_tiles) : 0;
@@ -246,6 +249,28 @@ __global__ void __launch_bounds__(256) linear_kernel(const LinearParams p) {
       store_row_blocks<T, NI>(out, acc[i], 1.f, g, row < p.m, CT / 2);
     }
   }
+}
+
+template <typename T, int RT, int CT>
+__global__ void __launch_bounds__(256) linear_forward_kernel(const LinearParams p) {
+  __shared__ __attribute__((aligned(1024))) char lds[linear_lds_bytes(RT, CT)];
+  linear_tile<T, kLinearForward, RT, CT>(p, int(blockIdx.x), lds);
+}
+
+// Both products of the backward read dy, and at the sizes of layers neither fills the chip by itself: one launch, the
+// workgroups of the weight gradient (the longer ones) first.  In two launches / in one, tokens x in -> out: 12544, 256 -> 768
+// 31.0 / 28.1 us, 256 -> 256 23.0 / 19.0; 784, 64 -> 192 15.5 / 9.8; 36864, 512 -> 1536 177 / 134, the end of one product
+// filled by the other.  W: extents of its tiles; C: columns of the input gradient's.
+struct LinearBackwardParams {
+  LinearParams weight, input;
+  int weight_blocks, input_blocks;  // multiples of the XCD count, or 0
+};
+template <typename T, int W, int C>
+__global__ void __launch_bounds__(256) linear_backward_kernel(const LinearBackwardParams p) {
+  constexpr int BYTES = linear_lds_bytes(W, W) > linear_lds_bytes(128, C) ? linear_lds_bytes(W, W) : linear_lds_bytes(128, C);
+  __shared__ __attribute__((aligned(1024))) char lds[BYTES];
+  if (int(blockIdx.x) < p.weight_blocks) linear_tile<T, kLinearWeight, W, W>(p.weight, int(blockIdx.x), lds);
+  else linear_tile<T, kLinearInput, 128, C>(p.input, int(blockIdx.x) - p.weight_blocks, lds);
 }
 
 // dw and db: the float32 sums of the slices, added up in order and rounded once.  Four elements a thread; `elements` of dw

@@ -1626,7 +1626,7 @@ int fill_linear(const char* what, LinearParams& p, const void* const* outer, con
   if (m < 1 || m > 0x7fffffff - 128 || n < 1 || k < 1) return fail("%s: invalid sizes (%lld rows, %d and %d columns)", what, (long long)m, n, k);
   if (part < 1 || n % part != 0 || n / part > 3) return fail("%s: one to three tensors of %d columns do not make %d", what, part, n);
   if (k % 64 != 0 || part % 64 != 0) return fail("%s: columns must be multiples of 64, got %d and tensors of %d", what, k, part);
-  if (n > 32768 || k > 32768) return fail("%s: more than 32768 columns", what);
+  if (n > 32768 || k > 32768 || (long long)n * k > 0x3fffffffLL) return fail("%s: more than 32768 columns or 2^30 weights", what);
   uintptr_t bits = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w);
   for (int t = 0; t < n / part; ++t) {
     if (!outer[t]) return fail("%s: null pointer argument", what);
@@ -1642,34 +1642,21 @@ int fill_linear(const char* what, LinearParams& p, const void* const* outer, con
   return 0;
 }
 
-extern "C++" {
-template <int MODE, int RT, int CT>
-int launch_linear_tiles(LinearParams& p, int rows, int cols, int dtype, hipStream_t stream) {
-  p.row_tiles = na_ceil_div(rows, RT);
-  p.col_tiles = cols / CT;
+// Lays `rows` x `cols` of a result out in tiles of rt x ct; the workgroups that makes (a multiple of the XCD count)
+long long lay_out_linear(LinearParams& p, int rows, int cols, int rt, int ct) {
+  p.row_tiles = na_ceil_div(rows, rt);
+  p.col_tiles = cols / ct;
   p.d_row_tiles = na_make_div(p.row_tiles);
   p.d_col_tiles = na_make_div(p.col_tiles);
-  const long long total = (long long)p.row_tiles * p.col_tiles * p.slices;
-  const long long grid = (total + kNumXcd - 1) / kNumXcd * kNumXcd;
-  if (grid > 0x7fffffffLL) return fail("linear: problem needs more than 2^31 workgroups");
-  if (dtype == NATTEN_AMD_F16) {
-    hipLaunchKernelGGL((linear_kernel<_Float16, MODE, RT, CT>), dim3((unsigned)grid), dim3(256), 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((linear_kernel<__bf16, MODE, RT, CT>), dim3((unsigned)grid), dim3(256), 0, stream, p);
-  }
-  return check_launch("linear");
+  return ((long long)p.row_tiles * p.col_tiles * p.slices + kNumXcd - 1) / kNumXcd * kNumXcd;
 }
 
-// Result tiles of 128 x 128 where there are four for each compute unit and they divide the columns, else 128 x 64: forward, us, 128 x 128 /
-// 128 x 64: 36864 tokens, 512 -> 1536 (3456 wide tiles) 80 / 90, 256 -> 768 (1728) 26.6 / 28.9, 256 -> 256 (576) 13.9 / 12.3;
-// 12544, 256 -> 768 (588) 13.6 / 12.5.  Fewer workgroups than that leave compute units with one to wait on.
-template <int MODE>
-int launch_linear(LinearParams& p, int cols, int align, int dtype, hipStream_t stream) {
-  const long long wide = (long long)na_ceil_div(p.m, 128) * (cols / 128);
-  if (align % 128 == 0 && wide >= 1024) return launch_linear_tiles<MODE, 128, 128>(p, p.m, cols, dtype, stream);
-  return launch_linear_tiles<MODE, 128, 64>(p, p.m, cols, dtype, stream);
+// Result tiles of 128 x 128 where there are four for each compute unit and they divide the columns (`align`), else 128 x 64: forward, us,
+// 128 x 128 / 128 x 64: 36864 tokens, 512 -> 1536 (3456 wide tiles) 80 / 90, 256 -> 768 (1728) 26.6 / 28.9, 256 -> 256 (576) 13.9 /
+// 12.3; 12544, 256 -> 768 (588) 13.6 / 12.5.  Fewer workgroups than that leave compute units with one to wait on.
+bool wide_linear_tiles(int m, int cols, int align) {
+  return align % 128 == 0 && (long long)na_ceil_div(m, 128) * (cols / 128) >= 1024;
 }
-}  // extern "C++"
 
 // Tiles of a weight gradient (128 x 128, or 64 x 64 where that does not divide the tensors) and its slices: about one
 // workgroup per compute unit, of at least two steps.
@@ -1699,67 +1686,93 @@ int natten_amd_linear_forward(const void* x, const void* w, const void* bias, vo
   p.col = w;
   p.bias = bias;
   for (int t = 0; t < 3; ++t) p.out[t] = outs[t];
-  return launch_linear<kLinearForward>(p, n, part, dtype, static_cast<hipStream_t>(stream));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool wide = wide_linear_tiles(p.m, n, part);
+  const long long blocks = lay_out_linear(p, p.m, n, 128, wide ? 128 : 64);
+  if (blocks > 0x7fffffffLL) return fail("%s: problem needs more than 2^31 workgroups", what);
+  const dim3 grid((unsigned)blocks), threads(256);
+  if (dtype == NATTEN_AMD_F16) {
+    if (wide) hipLaunchKernelGGL((linear_forward_kernel<_Float16, 128, 128>), grid, threads, 0, s, p);
+    else hipLaunchKernelGGL((linear_forward_kernel<_Float16, 128, 64>), grid, threads, 0, s, p);
+  } else {
+    if (wide) hipLaunchKernelGGL((linear_forward_kernel<__bf16, 128, 128>), grid, threads, 0, s, p);
+    else hipLaunchKernelGGL((linear_forward_kernel<__bf16, 128, 64>), grid, threads, 0, s, p);
+  }
+  return check_launch(what);
 }
 
-int natten_amd_linear_backward_input(const void* dy0, const void* dy1, const void* dy2, const void* w, void* dx, int dtype,
-                                     int64_t rows, int n, int k, int part, void* stream) {
+int natten_amd_linear_backward_workspace(int64_t rows, int n, int k, int part, uint64_t* bytes) {
   g_error[0] = 0;
-  const char* what = "linear_backward_input";
-  if (!w || !dx) return fail("%s: null pointer argument", what);
-  LinearParams p;
-  const void* const outer[3] = {dy0, dy1, dy2};
-  if (int rc = fill_linear(what, p, outer, dx, w, dtype, rows, n, k, part)) return rc;
-  for (int t = 0; t < 3; ++t) p.row[t] = outer[t];
-  p.col = w;
-  p.out[0] = dx;
-  return launch_linear<kLinearInput>(p, k, k, dtype, static_cast<hipStream_t>(stream));
-}
-
-int natten_amd_linear_backward_weight_workspace(int64_t rows, int n, int k, int part, uint64_t* bytes) {
-  g_error[0] = 0;
-  if (!bytes) return fail("linear_backward_weight_workspace: null pointer argument");
+  if (!bytes) return fail("linear_backward_workspace: null pointer argument");
   if (rows < 1 || n < 64 || k < 64 || part < 64 || n % part != 0 || k % 64 != 0 || part % 64 != 0)
-    return fail("linear_backward_weight_workspace: %lld rows, %d columns in tensors of %d, and %d columns", (long long)rows, n, part, k);
+    return fail("linear_backward_workspace: %lld rows, %d columns in tensors of %d, and %d columns", (long long)rows, n, part, k);
   *bytes = uint64_t(linear_weight_slices(rows, n, k, part)) * uint64_t(n) * (uint64_t(k) + 1) * 4;
   return 0;
 }
 
-int natten_amd_linear_backward_weight(const void* dy0, const void* dy1, const void* dy2, const void* x, void* dw, void* db,
-                                      void* workspace, uint64_t workspace_bytes, int dtype, int64_t rows, int n, int k, int part,
-                                      void* stream) {
-  g_error[0] = 0;
-  const char* what = "linear_backward_weight";
-  if (!x || !dw || !workspace) return fail("%s: null pointer argument", what);
-  LinearParams p;
-  const void* const outer[3] = {dy0, dy1, dy2};
-  if (int rc = fill_linear(what, p, outer, x, dw, dtype, rows, n, k, part)) return rc;
-  if ((reinterpret_cast<uintptr_t>(db) & 7) || (reinterpret_cast<uintptr_t>(workspace) & 15))
-    return fail("%s: db must be 8-byte and the workspace 16-byte aligned", what);
-  if ((long long)n * k > 0x3fffffffLL) return fail("%s: weights of more than 2^30 elements", what);
-  p.slices = linear_weight_slices(rows, n, k, part);
-  const uint64_t need = uint64_t(p.slices) * uint64_t(n) * (uint64_t(k) + 1) * 4;
-  if (workspace_bytes < need)
-    return fail("%s: the workspace holds %llu bytes, %llu are needed", what, (unsigned long long)workspace_bytes, (unsigned long long)need);
-  const int blocks = int((rows + 63) / 64);
-  p.slice_rows = na_ceil_div(blocks, p.slices) * 64;
-  for (int t = 0; t < 3; ++t) p.row[t] = outer[t];
-  p.col = x;
-  p.partial = static_cast<float*>(workspace);
-  p.partial_bias = db ? p.partial + int64_t(p.slices) * n * k : nullptr;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (int rc = linear_weight_tile(k, part) == 128 ? launch_linear_tiles<kLinearWeight, 128, 128>(p, n, k, dtype, s)
-                                                  : launch_linear_tiles<kLinearWeight, 64, 64>(p, n, k, dtype, s))
-    return rc;
-  const unsigned grid = unsigned((n * k / 4 + n / 4 + 255) / 256);
-  if (dtype == NATTEN_AMD_F16) {
-    hipLaunchKernelGGL((linear_reduce_kernel<_Float16>), dim3(grid), dim3(256), 0, s, p.partial, p.partial_bias,
-                       static_cast<_Float16*>(dw), static_cast<_Float16*>(db), n * k, n, p.slices);
-  } else {
-    hipLaunchKernelGGL((linear_reduce_kernel<__bf16>), dim3(grid), dim3(256), 0, s, p.partial, p.partial_bias,
-                       static_cast<__bf16*>(dw), static_cast<__bf16*>(db), n * k, n, p.slices);
+namespace {
+extern "C++" {
+template <typename T>
+int launch_linear_backward(const char* what, const LinearBackwardParams& p, bool big, bool wide, void* dw, void* db, hipStream_t s) {
+  const dim3 grid((unsigned)(p.weight_blocks + p.input_blocks)), threads(256);
+  if (big && wide) hipLaunchKernelGGL((linear_backward_kernel<T, 128, 128>), grid, threads, 0, s, p);
+  else if (big) hipLaunchKernelGGL((linear_backward_kernel<T, 128, 64>), grid, threads, 0, s, p);
+  else if (wide) hipLaunchKernelGGL((linear_backward_kernel<T, 64, 128>), grid, threads, 0, s, p);
+  else hipLaunchKernelGGL((linear_backward_kernel<T, 64, 64>), grid, threads, 0, s, p);
+  if (int rc = check_launch(what)) return rc;
+  if (dw != nullptr) {
+    const int elements = p.weight.n * p.weight.k;
+    hipLaunchKernelGGL((linear_reduce_kernel<T>), dim3((unsigned)((elements / 4 + p.weight.n / 4 + 255) / 256)), threads, 0, s,
+                       p.weight.partial, p.weight.partial_bias, static_cast<T*>(dw), static_cast<T*>(db), elements, p.weight.n,
+                       p.weight.slices);
+    return check_launch(what);
   }
-  return check_launch(what);
+  return 0;
+}
+}  // extern "C++"
+}  // namespace
+
+int natten_amd_linear_backward(const void* dy0, const void* dy1, const void* dy2, const void* x, const void* w, void* dx, void* dw,
+                               void* db, void* workspace, uint64_t workspace_bytes, int dtype, int64_t rows, int n, int k, int part,
+                               void* stream) {
+  g_error[0] = 0;
+  const char* what = "linear_backward";
+  if ((!dx && !dw) || (dx && !w) || (dw && (!x || !workspace)) || (db && !dw)) return fail("%s: null pointer argument", what);
+  LinearBackwardParams p;
+  memset(&p, 0, sizeof(p));
+  const void* const outer[3] = {dy0, dy1, dy2};
+  bool wide = false;
+  if (dx) {
+    if (int rc = fill_linear(what, p.input, outer, dx, w, dtype, rows, n, k, part)) return rc;
+    for (int t = 0; t < 3; ++t) p.input.row[t] = outer[t];
+    p.input.col = w;
+    p.input.out[0] = dx;
+    wide = wide_linear_tiles(p.input.m, k, k);
+    const long long blocks = lay_out_linear(p.input, p.input.m, k, 128, wide ? 128 : 64);
+    if (blocks > 0x3fffffffLL) return fail("%s: problem needs more than 2^30 workgroups", what);
+    p.input_blocks = int(blocks);
+  }
+  const int tile = linear_weight_tile(k, part);
+  if (dw) {
+    if (int rc = fill_linear(what, p.weight, outer, x, dw, dtype, rows, n, k, part)) return rc;
+    if ((reinterpret_cast<uintptr_t>(db) & 7) || (reinterpret_cast<uintptr_t>(workspace) & 15))
+      return fail("%s: db must be 8-byte and the workspace 16-byte aligned", what);
+    p.weight.slices = linear_weight_slices(rows, n, k, part);
+    const uint64_t need = uint64_t(p.weight.slices) * uint64_t(n) * (uint64_t(k) + 1) * 4;
+    if (workspace_bytes < need)
+      return fail("%s: the workspace holds %llu bytes, %llu are needed", what, (unsigned long long)workspace_bytes, (unsigned long long)need);
+    p.weight.slice_rows = na_ceil_div(int((rows + 63) / 64), p.weight.slices) * 64;
+    for (int t = 0; t < 3; ++t) p.weight.row[t] = outer[t];
+    p.weight.col = x;
+    p.weight.partial = static_cast<float*>(workspace);
+    p.weight.partial_bias = db ? p.weight.partial + int64_t(p.weight.slices) * n * k : nullptr;
+    const long long blocks = lay_out_linear(p.weight, n, k, tile, tile);
+    if (blocks > 0x3fffffffLL) return fail("%s: problem needs more than 2^30 workgroups", what);
+    p.weight_blocks = int(blocks);
+  }
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  return dtype == NATTEN_AMD_F16 ? launch_linear_backward<_Float16>(what, p, tile == 128, wide, dw, db, s)
+                                 : launch_linear_backward<__bf16>(what, p, tile == 128, wide, dw, db, s);
 }
 
 int natten_amd_compute_delta(const void* out, const void* d_out, float* delta, int dtype, int64_t items, int head_dim,

@@ -5,7 +5,7 @@ of which 101 were the attention's kernels, the rest being library products that 
 (143 us for two weight gradients), reductions of the bias gradients (44), and nine strided copies of queries, keys,
 values and their gradients (47), each a launch that the host makes (some thirty a step).  Here the map writes queries, keys
 and values as the attention takes them, its backward reads their gradients as the attention returns them, bias gradients come with
-the weight gradients, and the step is one autograd node of eleven launches."""
+the weight gradients, and the step is one autograd node of nine launches."""
 
 from __future__ import annotations
 
@@ -87,12 +87,8 @@ class _Linear(torch.autograd.Function):
             db = dy.sum(0) if ctx.has_bias and ctx.needs_input_grad[2] else None
             return dx, dw, db, None, None
         d_outs = [_aligned(d) for d in d_outs]
-        want_bias = ctx.has_bias and ctx.needs_input_grad[2]
-        dx = _lib.linear_backward_input(d_outs, weight, x.shape) if ctx.needs_input_grad[0] else None
-        dw = db = None
-        if ctx.needs_input_grad[1] or want_bias:
-            dw, db = _lib.linear_backward_weight(d_outs, x, weight.shape, want_bias)
-        return dx, dw if ctx.needs_input_grad[1] else None, db, None, None
+        return (*_lib.linear_backward(d_outs, x, weight, *ctx.needs_input_grad[:2], ctx.has_bias and ctx.needs_input_grad[2]),
+                None, None)
 
 
 @functools.lru_cache(maxsize=1024)
@@ -119,7 +115,7 @@ def _layer_nodes(x, w_qkv, b_qkv, w_proj, b_proj, heads, problem, scale):
 
 class _Layer(torch.autograd.Function):
     """A layer's step as one node: between three of them the engine hands each gradient over from Python to Python
-    (4 x 56 x 56 tokens, H 8, D 32, 7 x 7: 373 us a step as three nodes, 267 as one, 178 of them on the device)."""
+    (4 x 56 x 56 tokens, H 8, D 32, 7 x 7: 373 us a step as three nodes, 267 as one)."""
 
     @staticmethod
     def forward(ctx, x, w_qkv, b_qkv, w_proj, b_proj, heads, problem, scale, plan):
@@ -140,17 +136,13 @@ class _Layer(torch.autograd.Function):
             grads = iter(torch.autograd.grad(_layer_nodes(*leaves, heads, problem, scale), wanted, d_out, create_graph=True))
             return (*(next(grads) if need else None for need in ctx.needs_input_grad[:5]), None, None, None, None)
         d_out = _aligned(d_out)
-        dx = dw1 = db1 = dw2 = db2 = None
-        if need_w2 or need_b2:
-            dw2, db2 = _lib.linear_backward_weight((d_out,), out, w_proj.shape, need_b2)
-        if need_x or need_w1 or need_b1:
-            d_attn = _lib.linear_backward_input((d_out,), w_proj, out.shape)
+        dx = dw1 = db1 = None
+        first = need_x or need_w1 or need_b1
+        d_attn, dw2, db2 = _lib.linear_backward((d_out,), out, w_proj, first, need_w2, need_b2)
+        if first:
             grads = _lib.fna_backward_fused(q, k, v, d_attn, lse, None, *problem, scale, *plan, out=out)
-            if need_x:
-                dx = _lib.linear_backward_input(grads, w_qkv, x.shape)
-            if need_w1 or need_b1:
-                dw1, db1 = _lib.linear_backward_weight(grads, x, w_qkv.shape, need_b1)
-        return dx, dw1 if need_w1 else None, db1, dw2 if need_w2 else None, db2, None, None, None, None
+            dx, dw1, db1 = _lib.linear_backward(grads, x, w_qkv, need_x, need_w1, need_b1)
+        return dx, dw1, db1, dw2, db2, None, None, None, None
 
 
 def layer_step(qkv: nn.Linear, proj: nn.Linear, x: Tensor, heads: int, problem, scale: float) -> Optional[Tensor]:

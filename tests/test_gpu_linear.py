@@ -30,11 +30,12 @@ def test_maps_against_float64(rows, k, part, parts, dtype):
                    (((rows, k), 1), ((n, k), k**-0.5), ((n,), 1), ((rows, n), 1)))
     ys = _lib.linear_forward(x, w, b, parts, (rows, part))
     dys = [d.contiguous() for d in dy.split(part, dim=1)]
-    dx = _lib.linear_backward_input(dys, w, (rows, k))
-    dw, db = _lib.linear_backward_weight(dys, x, (n, k), True)
-    again = _lib.linear_backward_weight(dys, x, (n, k), True)
-    assert torch.equal(dw, again[0]) and torch.equal(db, again[1])
-    assert torch.equal(dw, _lib.linear_backward_weight(dys, x, (n, k), False)[0])
+    dx, dw, db = grads = _lib.linear_backward(dys, x, w, True, True, True)
+    assert all(torch.equal(a, b) for a, b in zip(grads, _lib.linear_backward(dys, x, w, True, True, True)))
+    # parts of them, in launches of their own
+    for need in ((True, False, False), (False, True, False), (False, False, True), (True, False, True)):
+        for flag, got, ref in zip(need, _lib.linear_backward(dys, x, w, *need), grads):
+            assert torch.equal(got, ref) if flag else got is None
     X, W, B, DY = (t.double() for t in (x, w, b, dy))
     for got, ref, size, length in (
             (torch.cat(ys, dim=1), X @ W.t() + B, X.abs() @ W.abs().t() + B.abs(), k + 1),
@@ -51,7 +52,7 @@ def test_the_copies_behind_the_last_token_count_nowhere():
     # infinities in the last row reach the gradients once, through the products that hold them
     x, dy = torch.ones((70, 64), dtype=torch.float16, device="cuda"), torch.ones((70, 64), dtype=torch.float16, device="cuda")
     x[-1, 3] = float("inf")
-    dw, db = _lib.linear_backward_weight([dy], x, (64, 64), True)
+    _, dw, db = _lib.linear_backward([dy], x, torch.zeros((64, 64), dtype=torch.float16, device="cuda"), False, True, True)
     assert torch.isinf(dw[:, 3]).all() and (dw[:, :3] == 70).all() and (dw[:, 4:] == 70).all() and (db == 70).all()
 
 
@@ -60,8 +61,8 @@ def test_sizes_that_the_kernels_do_not_take_are_refused():
     with pytest.raises(RuntimeError, match="multiples of 64"):
         _lib.linear_forward(x, w, None, 1, (8, 96))
     with pytest.raises(RuntimeError, match="workspace"):
-        _lib._check(_lib.lib().natten_amd_linear_backward_weight(
-            x.data_ptr(), None, None, x.data_ptr(), w.data_ptr(), None, w.data_ptr(), 16, 1, 8, 64, 64, 64, None))
+        _lib._check(_lib.lib().natten_amd_linear_backward(
+            x.data_ptr(), None, None, x.data_ptr(), None, None, w.data_ptr(), None, w.data_ptr(), 16, 1, 8, 64, 64, 64, None))
 
 
 def _layer(**kwargs):
