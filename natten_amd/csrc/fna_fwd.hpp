@@ -490,6 +490,16 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   constexpr int NT = NWAVES * 64;
   constexpr int QT = NWAVES * 32;
   constexpr bool NARROW = DC != 0;
+  // Where most tiles need the mask (windows small enough for tiles of 64 queries, see choose_small_forward_tiles) or
+  // the vector units are the bound anyway (narrow rows, a context), the maxima are taken once, of the masked logits, and not
+  // in the slots as well: 16 instructions less for a tile with a mask, the same number, but outside the matrix
+  // products' shadow, for one without.  Us before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 64 17.3 / 16.7, D 96 26.6 / 25.5,
+  // D 96 with 128 context tokens 30.5 / 29.1; 96 x 96, 21 x 21, H 8, D 64 43.0 / 41.5.  The other instances meet long
+  // runs of tiles without a mask: 32768 tokens, window 2048, D 128 40.4 / 40.8; 16384 tokens, D 32 31.1 / 32.0.
+  constexpr bool LATE_MAX = !NOMASK && !RAGGED && (NWAVES == 2 || NARROW || CTX);
+  // The instances with registers to spare hold the query's window, and read the coming tile's description ahead of the
+  // mask: one of its three waits for LDS (16.7 -> 16.4 and 41.5 -> 40.9 us for the D 64 problems above).
+  constexpr bool HOLD_WINDOW = LATE_MAX && NWAVES == 2 && D <= 64;
   constexpr int KSTEPS = (NARROW ? DC : D) / 16;
   constexpr int DB = (NARROW ? DC : D) / 32;
   constexpr int NSB = KVT / 32;
@@ -1111,19 +1121,27 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // the tiling (the box origin plus a multiple of the tile extent): the keys up to there (`lead`)
   // belong to the tile before it.  All six rows are read at once (one register each), so that a
   // masked tile waits for LDS twice -- the windows, then the rows -- and not once per dimension.
+  typedef int i32x4 __attribute__((ext_vector_type(4)));
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  i32x4 w01, geo;  // the window and the tile extents
+  i32x2 w2;
+  i32x4 coming;    // HOLD_WINDOW: description of the coming tile
+  auto read_window = [&]() __attribute__((always_inline)) {
+    const int row = wave * 32 + l32;
+    w01 = *reinterpret_cast<const i32x4*>(&sWin[row][0]);
+    w2 = *reinterpret_cast<const i32x2*>(&sWin[row][4]);
+    geo = *reinterpret_cast<const i32x4*>(&sGeo[0]);
+  };
+  auto read_tile = [&](int l) __attribute__((always_inline)) { return *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]); };
   auto mask_bits = [&](const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
     uint32_t bits = ~uint32_t(0);
     if constexpr (!NOMASK) {
-      typedef int i32x4 __attribute__((ext_vector_type(4)));
-      typedef int i32x2 __attribute__((ext_vector_type(2)));
-      const int row = wave * 32 + l32;
-      const i32x4 w01 = *reinterpret_cast<const i32x4*>(&sWin[row][0]);
-      const i32x2 w2 = *reinterpret_cast<const i32x2*>(&sWin[row][4]);
+      if constexpr (!HOLD_WINDOW) read_window();
       const int ws[3] = {w01[0], w01[2], w2[0]}, we[3] = {w01[1], w01[3], w2[1]};
       int lo[3], hi[3];
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        const int kt = sGeo[a];
+        const int kt = geo[a];
         lo[a] = na_min(na_max(ws[a] - origin[a], lead[a]), kt);
         hi[a] = na_min(na_max(we[a] - origin[a], 0), kt);
       }
@@ -1207,8 +1225,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       } else {
         if (!full) {
           int origin[3], lead[3];
-          typedef int i32x4 __attribute__((ext_vector_type(4)));
-          const i32x4 tile = *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]);
+          const i32x4 tile = HOLD_WINDOW ? coming : read_tile(l);
 #pragma unroll
           for (int a = 0; a < 3; ++a) {
             origin[a] = tile[a];
@@ -1234,6 +1251,11 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   TileRows nxt = tile_rows(1);  // tile 1
   wait_vmcnt<0>();
   workgroup_sync();  // K(0), V(0), the mask tables and the queries' windows are in LDS
+  if constexpr (HOLD_WINDOW) {
+    read_window();
+    asm volatile("" : "+v"(w01), "+v"(w2), "+v"(geo));  // (or the compiler reads them once more where they are used)
+    coming = read_tile(0);
+  }
   at_tile(1, kbase, ld_koff, p.ctx_k, KLayout{});
   if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, 1, KLayout{});
 #pragma unroll
@@ -1335,6 +1357,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
 #pragma unroll
       for (int t = 0; t < PF_V; ++t) vf[t] = v_frag(sV_cur, t);
     }
+    if constexpr (HOLD_WINDOW) {
+      coming = read_tile((j + 1 - d_first) & 63);  // (past the last tile: a description that is not used)
+      asm volatile("" : "+v"(coming));
+    }
     float mx[2] = {-INFINITY, -INFINITY};
     auto pv_slot = [&](auto t_tag) __attribute__((always_inline)) {
       constexpr int t = decltype(t_tag)::value;
@@ -1354,7 +1380,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           pin(psum[1]);
         }
       }
-      if constexpr (NXT && t >= N_PV / 2 && (kAblate & kAblateMax) == 0) {
+      if constexpr (NXT && !LATE_MAX && t >= N_PV / 2 && (kAblate & kAblateMax) == 0) {
         // row maxima of the coming tile (as if unmasked), NSB * 16 values over N_PV / 2 slots
         constexpr int t3 = t - N_PV / 2;
         constexpr int NV = NSB * 16;
@@ -1374,7 +1400,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     if constexpr (CUR) l_run += psum[0] + psum[1];
 
     if ((kAblate & kAblateMax) == 0 && NXT && j + 1 < total_tiles) {
-      finish_logits(S_nxt, j + 1 - d_first, true, fmaxf(mx[0], mx[1]));
+      finish_logits(S_nxt, j + 1 - d_first, !LATE_MAX, fmaxf(mx[0], mx[1]));
     }
     nxt = t2;
   };
