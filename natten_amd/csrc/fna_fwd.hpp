@@ -263,6 +263,25 @@ static __device__ __forceinline__ void async_copy16_asm(const void* base, uint32
       : "memory", "m0");
 }
 
+// The copy for the lanes in `lanes` only (at least one): the mask is set around it, without a branch.
+template <int IMM>
+static __device__ __forceinline__ void async_copy16_lanes_asm(const void* base, uint32_t voff, uint32_t lds_addr, uint64_t lanes) {
+  const uint64_t b = reinterpret_cast<uint64_t>(base);
+  const uint64_t ub = (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(b >> 32)))) << 32) |
+                      uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(b))));
+  base = reinterpret_cast<const void*>(ub);
+  lds_addr = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_addr)));
+  uint64_t saved;
+  asm volatile(
+      "s_mov_b32 m0, %1\n\t"
+      "s_and_saveexec_b64 %0, %5\n\t"
+      "global_load_lds_dwordx4 %2, %3 offset:%4\n\t"
+      "s_mov_b64 exec, %0"
+      : "=&s"(saved)
+      : "s"(lds_addr), "v"(voff), "s"(base), "n"(IMM), "s"(lanes)
+      : "memory", "m0", "scc");
+}
+
 // The 4-byte-per-lane form: lane i's dword from `base + voff` lands at LDS address `lds_addr + 4 * i`.
 static __device__ __forceinline__ void async_copy4_asm(const void* base, uint32_t voff, uint32_t lds_addr) {
   const uint64_t b = reinterpret_cast<uint64_t>(base);
@@ -469,8 +488,12 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // multiple of 32) of the D columns that the tiles have room for are multiplied: head dims between
 // the native ones on the tensors as they are, where padded copies of q, k and v and a slice of the
 // result cost more than the attention itself (2x64x64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context
-// tokens: the call takes 76 us instead of 139 with its ten copies and fills).  The chunks past a row are not
-// fetched: their places in the tiles are zeroed once, before the first copy.
+// tokens: the call takes 76 us instead of 139 with its ten copies and fills).  The places of a key row's chunks past
+// row_dim are zeroed once, before the first copy, and not fetched (the query is zero there, but a key may be
+// infinite); the value columns there end in columns of the result that are not stored: the row's last chunk serves again.
+// A copy's lanes are a mask held in scalar registers: with a condition on them the loop fell into a block per copy,
+// forty register moves each turn between them.  Us before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 96 25.5 / 24.8;
+// with 128 context tokens 29.0 / 28.1; 2 x 2048 tokens, dense, D 96 34.8 / 32.8.
 // CTX: every query also attends to the ctx_len keys of its batch entry's context, whose tiles come behind those of the
 // window box, in the same walk.  Context as a launch of dense attention of its own and a merge write and read both
 // results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a
@@ -714,14 +737,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const char* kbase = static_cast<const char*>(p.k) + kv_base;
   const char* vbase = static_cast<const char*>(p.v) + kv_base;
   const int64_t ctx_base = CTX ? (int64_t(b_orig) * ctx_len * kv_row_stride + int64_t(head_kv) * row_dim) * 2 - kImmBias : 0;
-  if constexpr (NARROW) {
+  if (NARROW && row_dim < DC) {
     // (every copy leaves out the same places, so this is needed once)
     for (int i = tid; i < TILE_BYTES / 16; i += NT) {
       const u32x4_t zero = {0, 0, 0, 0};
       reinterpret_cast<u32x4_t*>(sK0)[i] = zero;
-      reinterpret_cast<u32x4_t*>(sV0)[i] = zero;
       reinterpret_cast<u32x4_t*>(sK1)[i] = zero;
-      reinterpret_cast<u32x4_t*>(sV1)[i] = zero;
     }
     workgroup_sync();
   }
@@ -755,7 +776,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const int P = (wave * PER + i) * 64 + lane;
     const int row = P / CPR, slot = P % CPR;
     // XOR swizzles are involutions: slot -> source chunk uses the same function
-    const int chunk = V_LAYOUT ? L::v_slot(row, slot) : L::k_slot(row, slot);
+    int chunk = V_LAYOUT ? L::v_slot(row, slot) : L::k_slot(row, slot);
+    if constexpr (NARROW) chunk = na_min(chunk, row_dim / 8 - 1);
     // the instruction adds its immediate i * 1024 to the global address as well (RAGGED: taken off the base): take it
     // off here, on top of a bias that keeps the offset non-negative and is taken off the tile base
     return uint32_t(pos_of(row)) * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16) + (RAGGED ? 0u : uint32_t(kImmBias - i * 1024));
@@ -765,6 +787,11 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     ld_row[i] = ((wave * PER + i) * 64 + lane) / CPR;
     ld_koff[i] = copy_offset(i, std::false_type{}, kv_tile_pos);
     ld_voff[i] = copy_offset(i, std::true_type{}, kv_tile_pos);
+  }
+  uint64_t k_lanes[NOFF];  // NARROW: the lanes of a copy of keys whose chunk the row holds (copies i and i + 4: the same)
+  if constexpr (NARROW) {
+#pragma unroll
+    for (int i = 0; i < NOFF; ++i) k_lanes[i] = __ballot(L::k_slot(ld_row[i], lane % CPR) * 8 < row_dim);
   }
   // CTX: from the first context tile on (number box_tiles) the copies are of consecutive rows of the context
   auto at_tile = [&](int tile, const char*& base, uint32_t (&off)[NOFF], const void* ctx, auto v_tag) __attribute__((always_inline)) {
@@ -912,7 +939,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
               t1 = na_min(t1, c.lim[1] - 1);
               t2 = na_min(t2, c.lim[2] - 1);
               const uint32_t pos = uint32_t(t0 * tok_step[0] + t1 * tok_step[1] + t2 * tok_step[2]);
-              voff = pos * uint32_t(kv_row_stride * 2) + uint32_t((V_LAYOUT ? L::v_slot(r, slot) : L::k_slot(r, slot)) * 16);
+              int chunk = V_LAYOUT ? L::v_slot(r, slot) : L::k_slot(r, slot);
+              if constexpr (NARROW) chunk = na_min(chunk, row_dim / 8 - 1);
+              voff = pos * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16);
               src = c.src;
             } else {
               // last, partial tile of an unpadded sequence: rows past the end are masked; read the
@@ -925,12 +954,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
           // off the uniform base instead
           src -= IMM;
         }
-        if constexpr (NARROW) {
+        if constexpr (NARROW && !V_LAYOUT) {
           // lanes whose chunk lies past the row sit out (a copy covers whole tile rows, so every wave
           // still issues it and the counted waits hold); a lane's place in LDS follows from its number
-          const int P = (wave * PER + I) * 64 + lane;
-          const int chunk = V_LAYOUT ? L::v_slot(P / CPR, P % CPR) : L::k_slot(P / CPR, P % CPR);
-          if (chunk * 8 < row_dim) async_copy16_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096));
+          async_copy16_lanes_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096), k_lanes[I % 4]);
         } else {
           async_copy16_asm<IMM>(src, voff, c.lds0 + uint32_t((I / 4) * 4096));
         }

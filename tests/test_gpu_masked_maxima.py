@@ -1,10 +1,11 @@
-"""GPU: the instances that take a tile's maxima from its masked logits, on walks of more tiles than are described at once."""
+"""GPU: the instances that take a tile's maxima from its masked logits, on walks of more tiles than are described at once;
+keys of minus infinity in rows between the native head dims, whose tiles hold places past the row."""
 
 import pytest
 import torch
 
 from natten_amd.fna import amd_fna_generic
-from tests.gpu_utils import make_qkv, sampled_check
+from tests.gpu_utils import assert_close, make_qkv, oracle_full, sampled_check, to_np
 
 pytestmark = pytest.mark.gpu
 
@@ -22,3 +23,15 @@ def test_walks_of_small_tiles(shape, kernel, stride, causal, tiles, head_dim):
         out, lse = amd_fna_generic(q, k, v, kernel, stride, ones, causal, return_lse=True, q_tile_shape=tiles[0],
                                    kv_tile_shape=tiles[1])
     sampled_check(q, k, v, out, lse, kernel, stride, ones, causal, 300, seed=1)
+
+
+@pytest.mark.parametrize("head_dim", [40, 64, 72, 96, 120])
+def test_keys_of_minus_infinity(head_dim):
+    q, k, v = make_qkv(1, (24, 29), 2, 2, head_dim, torch.float16, seed=5)
+    q[..., -1].abs_().add_(0.5)
+    k[:, ::3, 1::4, :, -1] = -float("inf")  # no weight, as by a mask
+    with torch.no_grad():
+        out, lse = amd_fna_generic(q, k, v, (7, 9), (1, 1), (1, 1), (False, False), return_lse=True)
+    ref_o, ref_l = oracle_full(q, k, v, (7, 9), (1, 1), (1, 1), (False, False))
+    assert_close("out", to_np(out), ref_o)
+    assert_close("lse", to_np(lse), ref_l)
