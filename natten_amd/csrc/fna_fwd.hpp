@@ -474,8 +474,8 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 }
 
 // One 32-row query block per wave, two or three waves per SIMD (fwd_max_waves).
-// RAGGED: seqlen_kv is not a multiple of KVT (dense attention on unpadded sequences); the tile
-// copies then clamp their rows and are issued at the top of an iteration instead of one per slot.
+// RAGGED: packed sequences, and key sequences and dilation groups that end inside a tile: the copies' offsets
+// follow the tile (see to_lim).
 // The work of one workgroup on one Q tile; `pid` is the position of that tile in the launch order
 // (what blockIdx.x is when every Q tile has a workgroup of its own).  `before_stores()` is called
 // once, after the last KV tile and before the results are stored: nothing of this wave is in flight
@@ -732,7 +732,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   const int64_t kv_row_base = p.fused ? int64_t(b_orig) * p.tokens + group_tok : kv_seq_row0;
   const T* qbase = reinterpret_cast<const T*>(p.q) + q_row_base * q_row_stride + int64_t(head) * row_dim;
   // (less the bias of the copies' per-lane offsets, see below)
-  constexpr int kImmBias = RAGGED ? 0 : 3 * 1024;  // largest immediate offset of a copy
+  constexpr int kImmBias = 3 * 1024;  // largest immediate offset of a copy
   const int64_t kv_base = (kv_row_base * kv_row_stride + int64_t(head_kv) * row_dim) * 2 - kImmBias;
   const char* kbase = static_cast<const char*>(p.k) + kv_base;
   const char* vbase = static_cast<const char*>(p.v) + kv_base;
@@ -769,29 +769,57 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // row (permuted) or token (fused) distance to copy i is the same for every lane.
   const int64_t bytes_per_4 = int64_t(kv_tile_pos(ROWS_PER_4 % KVT)) * (kv_row_stride * 2);
   static_assert(!CTX || PER <= 4, "the distance between the copies i and i + 4 is the window's");
-  int ld_row[NOFF];
   uint32_t ld_koff[NOFF], ld_voff[NOFF];
   auto copy_offset = [&](int i, auto v_tag, auto&& pos_of) __attribute__((always_inline)) {
     constexpr bool V_LAYOUT = decltype(v_tag)::value;
-    const int P = (wave * PER + i) * 64 + lane;
+    int at = lane;
+    if constexpr (RAGGED) asm volatile("" : "+v"(at));  // (or what the offsets of eight copies are formed from is kept through the loop)
+    const int P = (wave * PER + i) * 64 + at;
     const int row = P / CPR, slot = P % CPR;
     // XOR swizzles are involutions: slot -> source chunk uses the same function
     int chunk = V_LAYOUT ? L::v_slot(row, slot) : L::k_slot(row, slot);
     if constexpr (NARROW) chunk = na_min(chunk, row_dim / 8 - 1);
-    // the instruction adds its immediate i * 1024 to the global address as well (RAGGED: taken off the base): take it
-    // off here, on top of a bias that keeps the offset non-negative and is taken off the tile base
-    return uint32_t(pos_of(row)) * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16) + (RAGGED ? 0u : uint32_t(kImmBias - i * 1024));
+    // the instruction adds its immediate i * 1024 to the global address as well: take it off here, on top of a bias that
+    // keeps the offset non-negative and is taken off the tile base
+    return uint32_t(pos_of(row)) * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16 + kImmBias - i * 1024);
   };
+  // RAGGED: a tile may reach past the keys: past its dilation group (original layout), or past a sequence shorter
+  // than a tile.  The copies then read the last key along each dimension again, so that no address outside the tensor is formed
+  // (the places are masked, and the order of every sum stays that of the whole tile).  How many positions of a tile
+  // hold keys (`lim`, a byte per dimension: see describe) changes from tile to tile only at the end of a group, and
+  // never in a packed sequence: the offsets of each operand are formed anew where it does, and every other tile's
+  // copies are those of the other instances, one per slot.  With the clamp in each copy, behind a branch, all were issued at
+  // the top of an iteration, us before / after: packed, causal, 10 sequences of 1 .. 2048, H 16/4, D 128 88.6 / 78.1, D 64 not causal
+  // 73.6 / 67.4, H 8 D 96 84.1 / 78.9; 24 of 700, H 16/4, D 128 108.8 / 97.9; groups narrower than a tile (5 x 50 x 40) level.
+  int k_lim = -1, v_lim = -1;  // of the tile whose offsets ld_koff / ld_voff are
+  auto to_lim = [&](int lim, int& current, uint32_t (&off)[NOFF], auto v_tag) __attribute__((always_inline)) {
+    if constexpr (RAGGED) {
+      static_assert(PER <= 4, "a copy's row offset is one of the first four");
+      if (lim == current) return;
+      current = lim;
 #pragma unroll
-  for (int i = 0; i < NOFF; ++i) {
-    ld_row[i] = ((wave * PER + i) * 64 + lane) / CPR;
-    ld_koff[i] = copy_offset(i, std::false_type{}, kv_tile_pos);
-    ld_voff[i] = copy_offset(i, std::true_type{}, kv_tile_pos);
+      for (int i = 0; i < NOFF; ++i)
+        off[i] = copy_offset(i, v_tag, [&](int r) {
+          if (!p.fused) return na_min(r, lim - 1);
+          const int t0 = na_min(r & (p.kv_tile[0] - 1), (lim & 255) - 1);
+          r >>= p.kv_tile_lg[0];
+          const int t1 = na_min(r & (p.kv_tile[1] - 1), ((lim >> 8) & 255) - 1);
+          const int t2 = na_min(r >> p.kv_tile_lg[1], (lim >> 16) - 1);
+          return t0 * tok_step[0] + t1 * tok_step[1] + t2 * tok_step[2];
+        });
+    }
+  };
+  if constexpr (!RAGGED) {
+#pragma unroll
+    for (int i = 0; i < NOFF; ++i) {
+      ld_koff[i] = copy_offset(i, std::false_type{}, kv_tile_pos);
+      ld_voff[i] = copy_offset(i, std::true_type{}, kv_tile_pos);
+    }
   }
   uint64_t k_lanes[NOFF];  // NARROW: the lanes of a copy of keys whose chunk the row holds (copies i and i + 4: the same)
   if constexpr (NARROW) {
 #pragma unroll
-    for (int i = 0; i < NOFF; ++i) k_lanes[i] = __ballot(L::k_slot(ld_row[i], lane % CPR) * 8 < row_dim);
+    for (int i = 0; i < NOFF; ++i) k_lanes[i] = __ballot(L::k_slot(((wave * PER + i) * 64 + lane) / CPR, lane % CPR) * 8 < row_dim);
   }
   // CTX: from the first context tile on (number box_tiles) the copies are of consecutive rows of the context
   auto at_tile = [&](int tile, const char*& base, uint32_t (&off)[NOFF], const void* ctx, auto v_tag) __attribute__((always_inline)) {
@@ -825,7 +853,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // What only some tiles ask for, kept in LDS (in registers the instances of head dim 128 spill): the coordinate of
   // the tile's first token (a tile moved back from the group's edge: of the first one gathered), whose first
   // (lead >> 8 a) & 255 positions along dimension a belong to the tile before it.
-  int d_origin[3] = {0, 0, 0};  // (RAGGED instances, whose copies look at it)
+  int d_lim = 0;  // RAGGED: positions of the lane's tile that hold keys, (d_lim >> 8 a) & 255 along dimension a (whole rows: of rows)
   uint64_t d_plain = ~uint64_t(0);  // by lane: every key of the tile is attended by every query of this wave
   uint64_t d_skip = 0;              // ... no key of the tile is attended by any query of this wave
   auto describe = [&](int first) __attribute__((always_inline)) {
@@ -835,7 +863,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const int number = na_min(first + lane, total_tiles - 1);
     kv_tile_of_box(first_tile + (CTX ? na_min(number, box_tiles - 1) : number), box_n, t);
     bool full = true, skip = false;
-    int lead = 0;
+    int lead = 0, d_origin[3];
+    d_lim = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const int org = box_org[a] + (t[a] << p.kv_tile_lg[a]);
@@ -847,10 +876,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       if constexpr (RAGGED) d_origin[a] = a == 0 ? na_min(org, last_origin0) : org;
       else d_origin[a] = move_back ? na_min(org, extent[a] - p.kv_tile[a]) : org;
       lead |= (org - d_origin[a]) << (8 * a);
+      if constexpr (RAGGED) d_lim |= na_min(extent[a] - d_origin[a], p.kv_tile[a]) << (8 * a);
     }
     // (the clamping instances see no permuted rows, and hold tok_step anyway)
     const int* row_step = RAGGED ? tok_step : p.kv_row_step;
     d_row0 = d_origin[0] * row_step[0] + d_origin[1] * row_step[1] + d_origin[2] * row_step[2];
+    if constexpr (RAGGED) d_lim = p.fused ? d_lim : na_min(seqlen_kv - d_row0, KVT);
     if constexpr (CTX) {
       // the last context tile is moved back to end with the context; no coordinates: its first one is marked
       const int org = (number - box_tiles) * KVT;
@@ -875,11 +906,13 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   struct TileRows {
     int row0;
     uint64_t bytes;  // row0 in bytes
+    int lim;         // RAGGED: see describe
   };
   auto tile_rows = [&](int l) __attribute__((always_inline)) {
     TileRows t;
     t.row0 = __builtin_amdgcn_readlane(d_row0, l);
     t.bytes = uint64_t(uint32_t(t.row0)) * uint32_t(kv_row_stride * 2);
+    t.lim = RAGGED ? __builtin_amdgcn_readlane(d_lim, l) : 0;
     return t;
   };
 
@@ -887,31 +920,12 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   struct TileCopy {
     const char* src;  // first row of the tile (this head)
     uint32_t lds0;    // LDS byte address of this wave's first chunk
-    int row0;
-    int lim[3];       // original layout: positions of the tile that lie inside the dilation group, per dimension
-    bool inside;      // the whole tile lies inside the sequence / the dilation group
   };
   const uint32_t lds_wave = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sK0) + uint32_t(wave * PER * 1024))));
-  // `l`: place of the tile among the described ones (RAGGED instances, which look at its origin)
-  auto make_copy = [&](const char* base, char* dst, const TileRows& t, int l) {
+  auto make_copy = [&](const char* base, char* dst, const TileRows& t) {
     TileCopy c;
     c.src = base + t.bytes;
     c.lds0 = lds_wave + (lds_address(dst) - lds_address(sK0));
-    c.inside = true;
-    if constexpr (RAGGED) {
-      const int kv_row0 = t.row0;
-      c.row0 = kv_row0;
-      if (p.fused) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          const int origin = __builtin_amdgcn_readlane(d_origin[a], l);
-          c.lim[a] = na_min(extent[a] - origin, p.kv_tile[a]);
-          c.inside = c.inside && (c.lim[a] == p.kv_tile[a]);
-        }
-      } else {
-        c.inside = kv_row0 + KVT <= seqlen_kv;
-      }
-    }
     return c;
   };
   // issues copy I (0 <= I < PER) of a tile; V_LAYOUT selects the LDS swizzle of the operand
@@ -922,38 +936,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       if (CHUNKS % (NT * PER) == 0 || (wave * PER + I) * 64 < CHUNKS) {
         constexpr int IMM = (I % 4) * 1024;
         const char* src = c.src + int64_t(I / 4) * bytes_per_4;
-        uint32_t voff = off[I % 4];
-        if constexpr (RAGGED) {
-          if (!c.inside) {
-            if (p.fused) {
-              // a tile that reaches past its dilation group (original layout): positions beyond
-              // the group's extent are masked; gather the group's last row along that dimension
-              // instead, so that no address outside the tensor is formed.  The LDS placement
-              // (and with it the order of every sum) stays that of the whole tile.
-              const int P = (wave * PER + I) * 64 + lane;
-              const int r = P / CPR, slot = P % CPR;
-              int t0 = r & (p.kv_tile[0] - 1);
-              const int r1 = r >> p.kv_tile_lg[0];
-              int t1 = r1 & (p.kv_tile[1] - 1), t2 = r1 >> p.kv_tile_lg[1];
-              t0 = na_min(t0, c.lim[0] - 1);
-              t1 = na_min(t1, c.lim[1] - 1);
-              t2 = na_min(t2, c.lim[2] - 1);
-              const uint32_t pos = uint32_t(t0 * tok_step[0] + t1 * tok_step[1] + t2 * tok_step[2]);
-              int chunk = V_LAYOUT ? L::v_slot(r, slot) : L::k_slot(r, slot);
-              if constexpr (NARROW) chunk = na_min(chunk, row_dim / 8 - 1);
-              voff = pos * uint32_t(kv_row_stride * 2) + uint32_t(chunk * 16);
-              src = c.src;
-            } else {
-              // last, partial tile of an unpadded sequence: rows past the end are masked; read the
-              // last valid row instead so that no out-of-bounds address is formed
-              const int over = na_max(c.row0 + ld_row[I % 4] + (I / 4) * ROWS_PER_4 - (seqlen_kv - 1), 0);
-              voff -= uint32_t(over) * uint32_t(kv_row_stride * 2);
-            }
-          }
-          // the clamped per-lane offset may be smaller than the immediate: take the immediate
-          // off the uniform base instead
-          src -= IMM;
-        }
+        const uint32_t voff = off[I % 4];
         if constexpr (NARROW && !V_LAYOUT) {
           // lanes whose chunk lies past the row sit out (a copy covers whole tile rows, so every wave
           // still issues it and the counted waits hold); a lane's place in LDS follows from its number
@@ -965,8 +948,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
   };
   static_assert(PER <= 8, "tile copy is written for at most eight copies per thread");
-  auto issue_tile_load = [&](const char* base, const uint32_t (&off)[NOFF], char* dst, const TileRows& t, int l, auto v_tag) {
-    const TileCopy c = make_copy(base, dst, t, l);
+  auto issue_tile_load = [&](const char* base, const uint32_t (&off)[NOFF], char* dst, const TileRows& t, auto v_tag) {
+    const TileCopy c = make_copy(base, dst, t);
     copy_one(std::integral_constant<int, 0>{}, c, off, v_tag);
     copy_one(std::integral_constant<int, 1>{}, c, off, v_tag);
     copy_one(std::integral_constant<int, 2>{}, c, off, v_tag);
@@ -984,8 +967,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   describe(0);
   {
     const TileRows rows = tile_rows(0);
-    issue_tile_load(kbase, ld_koff, sK0, rows, 0, KLayout{});
-    issue_tile_load(vbase, ld_voff, sV0, rows, 0, VLayout{});
+    to_lim(rows.lim, k_lim, ld_koff, KLayout{});
+    to_lim(rows.lim, v_lim, ld_voff, VLayout{});
+    issue_tile_load(kbase, ld_koff, sK0, rows, KLayout{});
+    issue_tile_load(vbase, ld_voff, sV0, rows, VLayout{});
   }
 
   // ---- this lane's query row, on its way while the tables below are formed ---------------------------
@@ -1284,7 +1269,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     coming = read_tile(0);
   }
   at_tile(1, kbase, ld_koff, p.ctx_k, KLayout{});
-  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, 1, KLayout{});
+  to_lim(nxt.lim, k_lim, ld_koff, KLayout{});
+  if (1 < total_tiles) issue_tile_load(kbase, ld_koff, sK1, nxt, KLayout{});
 #pragma unroll
   for (int r = 0; r < 16; ++r) c_init[r] = 0.f;
   {
@@ -1305,7 +1291,6 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   auto iteration = [&](auto stage_tag, auto cur_tag, auto nxt_tag, int j) __attribute__((always_inline)) {
     constexpr int st = decltype(stage_tag)::value;
     constexpr bool CUR = decltype(cur_tag)::value, NXT = decltype(nxt_tag)::value;
-    constexpr bool SPREAD = !RAGGED;
     f32x16_t (&S_cur)[NSB] = st ? S_b : S_a;
     f32x16_t (&S_nxt)[NSB] = st ? S_a : S_b;
     char* sK_cur = st ? sK1 : sK0;  // held K(j): free, receives K(j+2)
@@ -1325,12 +1310,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const TileRows t2 = tile_rows(l2);
     at_tile(j + 2, kbase, ld_koff, p.ctx_k, KLayout{});
     at_tile(j + 1, vbase, ld_voff, p.ctx_v, VLayout{});
-    const TileCopy ck = make_copy(kbase, sK_cur, t2, l2);
-    const TileCopy cv = make_copy(vbase, sV_nxt, nxt, l2 - 1);
-    if constexpr (!SPREAD && (kAblate & kAblateCopies) == 0) {
-      if (j + 2 < total_tiles) issue_tile_load(kbase, ld_koff, sK_cur, t2, l2, KLayout{});
-      if (j + 1 < total_tiles) issue_tile_load(vbase, ld_voff, sV_nxt, nxt, l2 - 1, VLayout{});
-    }
+    to_lim(t2.lim, k_lim, ld_koff, KLayout{});
+    to_lim(nxt.lim, v_lim, ld_voff, VLayout{});
+    const TileCopy ck = make_copy(kbase, sK_cur, t2);
+    const TileCopy cv = make_copy(vbase, sV_nxt, nxt);
 
     // -- G1 ------------------------------------------------------------------------------------
     vec8 kf[N_QK];
@@ -1359,7 +1342,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
         pin(psum[0]);
         pin(psum[1]);
       }
-      if constexpr (SPREAD && (kAblate & kAblateCopies) == 0) {
+      if constexpr ((kAblate & kAblateCopies) == 0) {
         // 2 * PER copies spread over the first half of the slots, K first
         constexpr int c_lo = (s * 2 * PER * 2) / N_QK, c_hi = ((s + 1) * 2 * PER * 2) / N_QK;
         for_range<c_lo, c_hi - c_lo>([&](auto c_tag) {

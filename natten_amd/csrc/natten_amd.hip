@@ -197,9 +197,9 @@ int launch_fna_fp8(const FnaParams& p, hipStream_t stream, WorkQueue queues) {
 }
 
 // Key sequences that end inside a tile, where the tile cannot be moved back to end with them: packed
-// sequences, dense ones shorter than a tile, dilation groups narrower than a tile.  The instance that
-// clamps its rows issues its copies at the top of an iteration, behind a branch each, instead of one
-// per slot: 2 x 4097 tokens, H 16, D 64: 218 us there, 203 with the last tile moved back.
+// sequences, dense ones shorter than a tile, dilation groups narrower than a tile.  All others move it back: the
+// instance that clamps has the registers of each tile's end to hold (2 x 4097 tokens, H 16, D 64: 218 us there when it
+// also issued its copies at the top of an iteration, 203 with the last tile moved back).
 bool needs_clamped_rows(const FnaParams& p, int kvt) {
   return p.cu_q != nullptr || p.edge == 2 || (p.seqlen_kv % kvt != 0 && p.edge != 1);
 }
