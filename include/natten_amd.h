@@ -194,6 +194,20 @@ int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void*
                                        int anchor_kv_tiles, int kv_splits, void* stream);
 
 /*
+ * natten_amd_fna_forward_fused for launches of about as many Q tiles as the chip has compute units: a
+ * workgroup has two groups of waves, each on half of its Q tile's KV tiles, and adds up their results itself.
+ * fp16 / bf16 operands, head_dim 64 or 128, Q tiles of 128 and KV tiles of 64 tokens, no dilation group narrower than a
+ * KV tile, no dequantisation scales; other arguments as in natten_amd_fna_forward_fused.
+ */
+int natten_amd_fna_forward_fused_paired(const void* q, const void* k, const void* v, void* out, float* lse,
+                                        int dtype, int na_dim, int batch, int heads_q, int heads_kv,
+                                        int head_dim, const int32_t* qkv_shape, const int32_t* kernel_size,
+                                        const int32_t* stride, const int32_t* dilation,
+                                        const int32_t* is_causal, const int32_t* q_tile_shape,
+                                        const int32_t* kv_tile_shape, float scale, int anchor_kv_tiles,
+                                        void* stream);
+
+/*
  * natten_amd_fna_forward_fused (anchored KV tiles, fp16 / bf16) whose queries also
  * attend to context_len >= 64 more keys per batch entry, context_k / context_v [batch, context_len, heads_kv,
  * head_dim]: out and lse are those of attention over the window and the context together (the role of the

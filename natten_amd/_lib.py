@@ -71,6 +71,10 @@ _SIGNATURES = {
         [ctypes.c_void_p] * 5 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 7 + [ctypes.c_float]
         + [ctypes.c_int, ctypes.c_int, ctypes.c_void_p],
     ),
+    "natten_amd_fna_forward_fused_paired": (
+        ctypes.c_int,
+        [ctypes.c_void_p] * 5 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 7 + [ctypes.c_float, ctypes.c_int, ctypes.c_void_p],
+    ),
     "natten_amd_fna_forward_fused_static": (
         ctypes.c_int,
         [ctypes.c_void_p] * 5 + [ctypes.c_int] * 6 + [ctypes.c_void_p] * 7 + [ctypes.c_float] + [ctypes.c_void_p] * 4,
@@ -490,6 +494,28 @@ def fna_forward_fused_split(
             *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
                              tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
             float(scale), 1 if anchored_tiles else 0, int(kv_splits), _stream(q),
+        )
+    _check(rc)
+    return out, lse
+
+
+def fna_forward_fused_paired(
+    q: Tensor, k: Tensor, v: Tensor, kernel_size, stride, dilation, is_causal, scale: float, q_tile_shape, kv_tile_shape,
+) -> Tuple[Tensor, Tensor]:
+    """fna_forward_fused with two groups of waves in the workgroup of a Q tile, on half of its KV tiles each (fp16 / bf16, head
+    dims 64 and 128, tiles of 128 x 64 tokens)."""
+    L = lib()
+    _require_gpu(q, k, v)
+    na_dim = len(kernel_size)
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    lse = torch.empty(q.shape[:-1], dtype=torch.float32, device=q.device)
+    with _on_device(q):
+        rc = L.natten_amd_fna_forward_fused_paired(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
+            DTYPE_CODES[q.dtype], na_dim, q.shape[0], q.shape[-2], k.shape[-2], q.shape[-1],
+            *_problem_arrays(tuple(q.shape[1 : 1 + na_dim]), tuple(kernel_size), tuple(stride), tuple(dilation),
+                             tuple(is_causal), tuple(q_tile_shape), tuple(kv_tile_shape)),
+            float(scale), 1, _stream(q),
         )
     _check(rc)
     return out, lse

@@ -498,8 +498,11 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // window box, in the same walk.  Context as a launch of dense attention of its own and a merge write and read both
 // results once more: 2 x 64 x 64 tokens, H 8 / 2, D 96, 13 x 13 windows and 128 context tokens: 37 + 17 + 9 us, now 33 (a
 // call 62 -> 31; 4 x 96 x 96, 24 x 24, H 16, D 128, 256 tokens: 665 -> 476).
+// PAIRED: the workgroup has two groups of NWAVES waves, each on half of the Q tile's KV tiles with tiles in LDS of its own; they
+// meet at every tile's barrier, and at the end the first takes the second's sums through LDS.  For launches that
+// leave a SIMD one wave, with nothing to fill its waits (see fna_fwd_paired_kernel).
 template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
-          bool CTX = false, typename Hook>
+          bool CTX = false, bool PAIRED = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
   int split = 0, splits = 1, pid = pid_in;
@@ -510,6 +513,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       pid = pid_in - split * p.split_grid;
     }
   }
+  constexpr int GROUPS = PAIRED ? 2 : 1;
+  static_assert(!PAIRED || !(SPLIT || NOMASK || RAGGED || CTX || DC != 0), "pairs of groups: masked instances of whole tiles");
   constexpr int NT = NWAVES * 64;
   constexpr int QT = NWAVES * 32;
   constexpr bool NARROW = DC != 0;
@@ -541,10 +546,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // One LDS object per stage and operand: distinct objects let the compiler see that the
   // asynchronous fill of one stage does not alias the operand reads of the other, so those
   // reads do not wait for the fill.
-  __shared__ __attribute__((aligned(1024))) char sK0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sV0[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sK1[TILE_BYTES];
-  __shared__ __attribute__((aligned(1024))) char sV1[TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sK0[GROUPS * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sV0[GROUPS * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sK1[GROUPS * TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) char sV1[GROUPS * TILE_BYTES];
   // What the element mask of a PARTIAL tile needs (absent from NOMASK instances), kept in LDS and read
   // where such a tile is met -- in registers for the whole loop these values would push the loop's own
   // out to spill lanes:
@@ -555,14 +560,16 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   constexpr int MASK_ROWS = NOMASK ? 1 : KVT + 1;
   __shared__ __attribute__((aligned(16))) uint32_t sKeys[NOMASK ? 1 : 3][2][MASK_ROWS];
   __shared__ __attribute__((aligned(16))) int sWin[NOMASK ? 1 : NWAVES * 32][8];
-  //   sTile[wave * 64 + i]  the i-th described KV tile (see describe)
-  __shared__ __attribute__((aligned(16))) int sTile[NOMASK ? 1 : NWAVES * 64][4];
+  //   sTile[tile_slot0 + i]  the wave's i-th described KV tile (see describe)
+  __shared__ __attribute__((aligned(16))) int sTile[NOMASK ? 1 : GROUPS * NWAVES * 64][4];
   __shared__ __attribute__((aligned(16))) int sGeo[4];
   static_assert(NOMASK || KVT == 64, "the element mask holds one bit per key of a 64-key tile");
 
-  const int tid = threadIdx.x;
+  const int group_id = PAIRED ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) / NT) : 0;  // PAIRED: which group of waves
+  const int tid = int(threadIdx.x) - group_id * NT;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform by construction
+  const int tile_slot0 = (group_id * NWAVES + wave) * 64;     // the wave's rows of sTile
   const int l32 = lane & 31;
   const int g = lane >> 5;
 
@@ -691,7 +698,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       const int ws = na_window_start(c, ksz[a], p.stride[a], p.d_stride[a], extent[a], cs);
       const int we = na_window_end(c, ws, ksz[a], extent[a], cs);
       if constexpr (!NOMASK) {
-        if (g == 0) {
+        if (g == 0 && group_id == 0) {
           sWin[wave * 32 + l32][2 * a] = ws;
           sWin[wave * 32 + l32][2 * a + 1] = we;
         }
@@ -722,6 +729,14 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
       first_tile = 0;
       total_tiles = 1;
     }
+  }
+
+  // PAIRED: the second group's half; of an odd number the middle tile is described to both and skipped by the second
+  bool skip_first = false;
+  if constexpr (PAIRED) {
+    total_tiles = (box_tiles + 1) / 2;
+    first_tile = group_id * (box_tiles - total_tiles);
+    skip_first = group_id == 1 && (box_tiles & 1);
   }
 
   const int64_t q_row_stride = int64_t(p.heads_q) * row_dim;
@@ -895,8 +910,9 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
     if constexpr (!NOMASK) {
       typedef int i32x4 __attribute__((ext_vector_type(4)));
-      *reinterpret_cast<i32x4*>(&sTile[wave * 64 + lane][0]) = i32x4{d_origin[0], d_origin[1], d_origin[2], lead};
+      *reinterpret_cast<i32x4*>(&sTile[tile_slot0 + lane][0]) = i32x4{d_origin[0], d_origin[1], d_origin[2], lead};
     }
+    if constexpr (PAIRED) skip = skip || (skip_first && number == 0);
     if constexpr (!NOMASK && (kAblate & kAblateMask) == 0) {
       d_plain = __ballot(full && !skip);
       d_skip = __ballot(skip);
@@ -921,7 +937,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     const char* src;  // first row of the tile (this head)
     uint32_t lds0;    // LDS byte address of this wave's first chunk
   };
-  const uint32_t lds_wave = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sK0) + uint32_t(wave * PER * 1024))));
+  const uint32_t lds_wave = uint32_t(__builtin_amdgcn_readfirstlane(int(lds_address(sK0) + uint32_t(group_id * TILE_BYTES + wave * PER * 1024))));
   auto make_copy = [&](const char* base, char* dst, const TileRows& t) {
     TileCopy c;
     c.src = base + t.bytes;
@@ -1003,13 +1019,13 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   }
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (!NOMASK) {
-    if (tid < 3) sGeo[tid] = p.kv_tile[tid];
+    if (tid < 3 && group_id == 0) sGeo[tid] = p.kv_tile[tid];
     // one row per lane, a dimension per wave (the row past a tile of 64 keys along one dimension holds none):
     // keys are numbered with dimension 0 fastest
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const int lg_stride = a == 0 ? 0 : a == 1 ? p.kv_tile_lg[0] : p.kv_tile_lg[0] + p.kv_tile_lg[1];
-      if (wave == a % NWAVES) {
+      if (wave == a % NWAVES && group_id == 0) {
         const uint64_t keys = na_keys_at_or_after(na_min(lane, p.kv_tile[a]), lg_stride, p.kv_tile_lg[a]);
         sKeys[a][0][lane] = na_lane_half_bits(keys, 0);
         sKeys[a][1][lane] = na_lane_half_bits(keys, 1);
@@ -1039,7 +1055,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // lane-constant LDS read offsets
   int k_off[KSTEPS];  // K operand: row l32 (+32*sb), chunk 2*ks+g
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) k_off[ks] = l32 * ROWB + L::k_slot(l32, ks * 2 + g) * 16;
+  for (int ks = 0; ks < KSTEPS; ++ks) k_off[ks] = group_id * TILE_BYTES + l32 * ROWB + L::k_slot(l32, ks * 2 + g) * 16;
   // V operand: transpose read of rows (4g + e) [+8], 4 columns at 16*(l32/16) + 4*j4 of a 32-column block
   const int l16 = lane & 15;
   const int v_e = l16 >> 2, v_j4 = l16 & 3;
@@ -1049,7 +1065,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   uint32_t v_off[DB];  // (8 rows are a whole number of the V swizzle's periods)
   static_assert(8 % (L::RPL * CPR / 4) == 0, "the transpose reads of a fragment lie 8 rows apart");
 #pragma unroll
-  for (int db = 0; db < DB; ++db) v_off[db] = uint32_t(v_row * ROWB + v_sub + L::v_slot(v_row, db * 4 + v_chunk) * 16);
+  for (int db = 0; db < DB; ++db) v_off[db] = uint32_t(group_id * TILE_BYTES + v_row * ROWB + v_sub + L::v_slot(v_row, db * 4 + v_chunk) * 16);
 
   // ---- building blocks ---------------------------------------------------------------------------
   // The lane owns query row l32 of its wave's row block and, per 32-key sub-block,
@@ -1144,7 +1160,7 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     w2 = *reinterpret_cast<const i32x2*>(&sWin[row][4]);
     geo = *reinterpret_cast<const i32x4*>(&sGeo[0]);
   };
-  auto read_tile = [&](int l) __attribute__((always_inline)) { return *reinterpret_cast<const i32x4*>(&sTile[wave * 64 + l][0]); };
+  auto read_tile = [&](int l) __attribute__((always_inline)) { return *reinterpret_cast<const i32x4*>(&sTile[tile_slot0 + l][0]); };
   auto mask_bits = [&](const int (&origin)[3], const int (&lead)[3]) __attribute__((always_inline)) {
     uint32_t bits = ~uint32_t(0);
     if constexpr (!NOMASK) {
@@ -1424,6 +1440,38 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   wait_vmcnt<0>();  // the last iterations' copies into the unused stage must land before the LDS is released
   before_stores();
 
+  if constexpr (PAIRED) {
+    // The second group's O, row sums and maxima, by lane, in the place of the tiles (a wave's share of O is a tile's size:
+    // group 0's and 1's of sK0, then of sV0) and of the tiles' descriptions.
+    static_assert(NWAVES == 4 && DB * 4096 == TILE_BYTES, "a wave's share of O fills a tile's place");
+    f32x4_t* share = reinterpret_cast<f32x4_t*>((wave < 2 ? sK0 : sV0) + (wave & 1) * TILE_BYTES) + lane;
+    float* row = reinterpret_cast<float*>(&sTile[wave * 64 + lane][0]);
+    workgroup_sync();  // all waves are done with the tiles
+    if (group_id == 1) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) share[(db * 4 + j) * 64] = f32x4_t{acc[db][4 * j], acc[db][4 * j + 1], acc[db][4 * j + 2], acc[db][4 * j + 3]};
+      row[0] = m_run;
+      row[1] = l_run;
+    }
+    workgroup_sync();
+    if (group_id == 1) return;
+    const float m1 = row[0], l1 = row[1];
+    const float m = fmaxf(m_run, m1);
+    const float a0 = m_run == -INFINITY ? 0.f : fast_exp2(m_run - m), a1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - m);
+    l_run = l_run * a0 + l1 * a1;
+    m_run = m;
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t other = share[(db * 4 + j) * 64];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[db][4 * j + i] = acc[db][4 * j + i] * a0 + other[i] * a1;
+      }
+  }
+
   // ---- epilogue: O = acc / rowsum, LSE = ln(rowsum) + scale * rowmax -------------------------
   T* obase = reinterpret_cast<T*>(p.o) + q_row_base * q_row_stride + int64_t(head) * row_dim;
   float* lse_base = p.lse;
@@ -1548,6 +1596,18 @@ __global__ void __launch_bounds__(NWAVES * 64) __attribute__((amdgpu_waves_per_e
 fna_fwd_split_kernel(const FnaParams p) {
   touch_launch_params<sizeof(FnaParams)>();
   fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, true, false, DC>(p, int(blockIdx.x), []() {});
+}
+
+// Two groups of four waves per Q tile (PAIRED).  A launch of at most 256 Q tiles leaves each a compute unit of its own, and
+// a SIMD one wave, bound by its own waits: as pairs it has two, and the float32 sums meet in LDS instead of in memory (a split
+// launch and its merge).  One group / two, us, bf16: 32768 tokens, window 2048, H 1, D 128 41.9 / 40.5, D 64 27.8 / 24.2; 128 x
+// 128, 33 x 33, H 2, D 128 42.6 / 38.7; 16 x 32 x 32, 8 x 16 x 16, H 2, D 128 93.6 / 80.2; 96 x 96, 40 x 40, H 3, D 64 40.0 / 31.5.
+// Errors against float32 arithmetic (2-norm, seven problems): 2.68e-3 .. 2.89e-3 one group, 2.67e-3 .. 2.88e-3 two.
+template <typename T, int D>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
+fna_fwd_paired_kernel(const FnaParams p) {
+  touch_launch_params<sizeof(FnaParams)>();
+  fna_fwd_tile<T, D, 4, false, 64, false, false, 0, false, true>(p, int(blockIdx.x), []() {});
 }
 
 // Combines the partial results of a dense split launch, sixteen rows of a Q tile per workgroup, four columns per lane:

@@ -87,6 +87,7 @@ bool narrow_rows(int head_dim) { return head_dim > 32 && head_dim < 128 && head_
 struct WorkQueue {
   uint32_t* counters = nullptr;
   bool clear_first = true;
+  bool paired = false;  // no queue: a workgroup of two groups of waves for each Q tile
 };
 
 // DC != 0: rows of p.row_dim elements, DC columns multiplied (no work-queue launch)
@@ -141,6 +142,16 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
   hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)(wgs + clearing)),
                      dim3(NWAVES * 64), 0, stream, pk);
   return check_launch("fna_forward");
+}
+
+template <typename T, int D>
+int launch_paired(const FnaParams& p, hipStream_t stream) {
+  if (!fna_tiles_are_powers_of_two(p)) return fail("fna_forward: tile extents must be powers of two");
+  if ((p.seqlen_q + 127) / 128 != p.num_q_tiles) return fail("fna_forward: internal tile count mismatch");
+  const long long wgs = (long long)((p.total_groups + kNumXcd - 1) / kNumXcd) * kNumXcd * p.wg_group;
+  if (wgs > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
+  hipLaunchKernelGGL((fna_fwd_paired_kernel<T, D>), dim3((unsigned)wgs), dim3(512), 0, stream, p);
+  return check_launch("fna_forward (paired)");
 }
 
 // Whether the launch is fully block-sparse: every Q tile is whole (no padding queries), all its
@@ -221,6 +232,14 @@ int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, Work
   if (needs_clamped_rows(p, kvt)) {
     if (qt == 128 && kvt == 64) return launch_fna<T, D, 4, true, 64>(p, stream);
     return fail("fna_forward: seqlen_kv (%d) must be a multiple of the KV tile (%d tokens)", p.seqlen_kv, kvt);
+  }
+  // (A fully block-sparse launch of head dim 128 keeps its mask-free instance: 16 x 32 x 32, 8 x 16 x 16 blocked, H 2: 37.1 us
+  // there, 37.9 as pairs with masks.  Head dim 64: 32768 tokens, 2048 blocked by 128, H 1: 24.0 and 22.5.)
+  if (queues.paired && !(D == 128 && qt == 128 && kvt == 64 && fully_block_sparse(p))) {
+    if constexpr (D >= 64) {
+      if (qt == 128 && kvt == 64) return launch_paired<T, D>(p, stream);
+    }
+    return fail("fna_forward: pairs of groups exist for Q tiles of 128 and KV tiles of 64 tokens and head dims 64 and 128");
   }
   // the work-queue launch exists for the default tile pair; the others launch a workgroup per Q tile
   if (qt == 128 && kvt == 64) {
@@ -780,6 +799,23 @@ int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void*
   return fna_forward_fused_impl(q, k, v, out_parts, lse_parts, dtype, na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape,
                                 kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape, scale, nullptr,
                                 nullptr, nullptr, anchor_kv_tiles, WorkQueue{}, stream, kv_splits);
+}
+
+int natten_amd_fna_forward_fused_paired(const void* q, const void* k, const void* v, void* out, float* lse, int dtype,
+                                        int na_dim, int batch, int heads_q, int heads_kv, int head_dim,
+                                        const int32_t* qkv_shape, const int32_t* kernel_size, const int32_t* stride,
+                                        const int32_t* dilation, const int32_t* is_causal, const int32_t* q_tile_shape,
+                                        const int32_t* kv_tile_shape, float scale, int anchor_kv_tiles, void* stream) {
+  g_error[0] = 0;
+  const char* what = "fna_forward_fused_paired";
+  if (na_dim < 1 || na_dim > 3) return fail("%s: na_dim must be 1, 2 or 3, got %d", what, na_dim);
+  if (dtype != NATTEN_AMD_F16 && dtype != NATTEN_AMD_BF16) return fail("%s: fp16 / bf16 operands, got dtype code %d", what, dtype);
+  if (head_dim != 64 && head_dim != 128) return fail("%s: head_dim must be 64 or 128, got %d", what, head_dim);
+  WorkQueue launch;
+  launch.paired = true;
+  return fna_forward_fused_impl(q, k, v, out, lse, dtype, na_dim, batch, heads_q, heads_kv, head_dim, qkv_shape, kernel_size,
+                                stride, dilation, is_causal, q_tile_shape, kv_tile_shape, scale, nullptr, nullptr, nullptr,
+                                anchor_kv_tiles, launch, stream);
 }
 
 int natten_amd_fna_forward_fused_context(const void* q, const void* k, const void* v, const void* context_k,

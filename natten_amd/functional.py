@@ -10,6 +10,7 @@ accepted and ignored, except `q_tile_shape` / `kv_tile_shape`, which select the 
 from __future__ import annotations
 
 import functools
+import math
 from typing import Dict, Optional, Tuple, Union
 
 import torch
@@ -274,6 +275,24 @@ def narrow_kv_splits_default(batch: int, heads: int, token_layout, kernel_size, 
     if _kv_tiles_per_q_tile(token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape) < 24:
         return 1
     return kv_splits_default(batch, heads, token_layout, kernel_size, stride, dilation, is_causal, q_tile_shape, kv_tile_shape)
+
+
+def paired_groups_default(batch: int, heads: int, head_dim: int, token_layout, kernel_size, stride, dilation, is_causal,
+                          q_tile_shape, kv_tile_shape) -> bool:
+    """Whether a forward launch has two groups of waves in the workgroup of a Q tile: where every Q tile (128 x 64 tokens, not
+    split) has a compute unit of its own, and its KV tiles are enough to pay for the sums' way through LDS.  One group /
+    two, us, bf16, by KV tiles of a Q tile, 256 Q tiles each.  Head dim 128: 6 14.1 / 14.8, 10 17.8 / 18.0
+    (in two dimensions, most of them with a mask, 20.3 / 19.5), 18 25.4 / 25.2 (30.7 / 28.0), 34 41.9 / 40.5, 66 71.5 / 68.1; head
+    dim 64: 6 11.4 / 10.9, 10 12.8 / 12.0, 34 27.8 / 24.2."""
+    if head_dim not in (64, 128) or math.prod(q_tile_shape) != 128 or math.prod(kv_tile_shape) != 64:
+        return False
+    if any(x // d < t for x, d, t in zip(token_layout, dilation, kv_tile_shape)):
+        return False  # (groups narrower than a tile have an instance of their own)
+    tiles = batch * heads
+    for X, d, qt in zip(token_layout, dilation, q_tile_shape):
+        tiles *= -(-(-(-X // d)) // qt) * d
+    visits = _kv_tiles_per_q_tile(token_layout, kernel_size, stride, dilation, q_tile_shape, kv_tile_shape)
+    return tiles <= 256 and visits >= (8 if head_dim == 64 else 16)
 
 
 @functools.lru_cache(maxsize=1024)

@@ -1,0 +1,62 @@
+"""GPU: forward launches with two groups of waves per Q tile: even and odd numbers of KV tiles, one tile, walks longer than are
+described at once, tiles at the edges of groups; against the CPU oracle, and where the launch is chosen (CPU)."""
+
+import pytest
+import torch
+
+from natten_amd import _lib
+from natten_amd.fna import _open_call_plan
+from natten_amd.functional import na1d
+from tests.gpu_utils import make_qkv, sampled_check
+
+CASES = [
+    # shape, kernel, stride, dilation, causal, tiles
+    ((700,), (64,), (64,), (1,), (False,), ((128,), (64,))),                                  # two or three tiles
+    ((333,), (3,), (1,), (1,), (True,), ((128,), (64,))),                                     # a second group with one tile
+    ((300,), (2,), (2,), (2,), (False,), ((128,), (64,))),                                    # ... or none of its own
+    ((9000,), (8200,), (8,), (1,), (False,), ((128,), (64,))),                                # 65 and more each
+    ((41, 53), (17, 20), (1, 3), (1, 1), (False, True), ((8, 16), (8, 8))),
+    ((60, 47), (13, 9), (1, 1), (2, 3), (True, False), ((16, 8), (4, 16))),
+    ((9, 17, 21), (5, 7, 8), (1, 2, 1), (1, 1, 2), (True, False, False), ((2, 8, 8), (4, 4, 4))),
+    ((16, 32, 32), (8, 16, 16), (4, 8, 8), (1, 1, 1), (False, False, False), ((2, 8, 8), (1, 8, 8))),  # nearly no masks
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("case", CASES)
+def test_matches_oracle(case, head_dim, dtype):
+    shape, kernel, stride, dilation, causal, tiles = case
+    q, k, v = make_qkv(2, shape, 2, 1, head_dim, dtype, seed=11)
+    out, lse = _lib.fna_forward_fused_paired(q, k, v, kernel, stride, dilation, causal, head_dim**-0.5, *tiles)
+    sampled_check(q, k, v, out, lse, kernel, stride, dilation, causal, 300, seed=1)
+
+
+@pytest.mark.gpu
+def test_chosen_call_replays_in_a_graph():
+    q, k, v = make_qkv(1, (8192,), 4, 2, 64, torch.bfloat16, seed=2)
+    with torch.no_grad():
+        ref, ref_lse = na1d(q, k, v, 1024, return_lse=True)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out, lse = na1d(q, k, v, 1024, return_lse=True)
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, ref) and torch.equal(lse, ref_lse)
+    sampled_check(q, k, v, ref, ref_lse, (1024,), (1,), (1,), (False,), 300, seed=1)
+
+
+def test_where_it_is_chosen():
+    def kind(shape, heads, head_dim, kernel, launch=None, dtype=torch.bfloat16):
+        ones = (1,) * len(shape)
+        return _open_call_plan(dtype, (1, *shape, heads, head_dim), heads, kernel, ones, ones, (False,) * len(shape), launch)[2]
+
+    assert kind((32768,), 1, 128, (2048,)) == "paired" and kind((32768,), 1, 64, (512,)) == "paired"
+    assert kind((32768,), 2, 128, (2048,)) is False        # more Q tiles than compute units
+    assert kind((32768,), 1, 128, (512,)) is False         # few KV tiles
+    assert kind((8192,), 1, 128, (2048,)) is False         # a split launch
+    assert kind((32768,), 1, 96, (2048,)) is False
+    assert kind((32768,), 1, 128, (2048,), launch=False) is False and kind((32768,), 1, 128, (2048,), launch=True) is True
