@@ -15,6 +15,8 @@
  *                                  src/natten/backends/blackwell_fna.py:99-164, in one launch
  *   natten_amd_fna_forward_fused_split <- the same forward for small grids: several workgroups per
  *                                  Q tile, partial results merged by natten_amd_merge_attention_parts
+ *   natten_amd_fna_forward_fused_paired <- the same forward for about as many Q tiles as compute units:
+ *                                  two groups of waves per Q tile
  *   natten_amd_token_permute    <- token_permute_{1,2,3}d   csrc/include/natten/token_permute.h:34-52
  *   natten_amd_token_permute_widen <- the same, for e4m3 / e5m2 operands (writes bf16)
  *   natten_amd_token_unpermute  <- token_unpermute_{1,2,3}d csrc/include/natten/token_permute.h:54-74
@@ -27,6 +29,7 @@
  *                                  csrc/include/natten/blackwell_fna.h:92-160
  *   natten_amd_fna_backward_fused <- the reference driver's permutes + backward + unpermutes,
  *                                  src/natten/backends/blackwell_fna.py:205-297, without the copies
+ *   natten_amd_fna_backward_from_output <- the same, with the pass over out and d_out in the dQ launch
  *   natten_amd_attention_backward <- blackwell_fmha_backward csrc/include/natten/blackwell_fmha.h:52-73
  *                                  (fixed-length batches)
  *   natten_amd_attention_backward_varlen <- the same function with cumulative_seqlen_Q / _KV,
@@ -35,6 +38,8 @@
  *   natten_amd_merge_attentions <- the elementwise merge of src/natten/attn_merge.py:48-105
  *                                  (the reference runs it as framework ops; here it is one kernel)
  *   natten_amd_merge_attention_parts <- the same merge over any number of partial results at once
+ *   natten_amd_linear_forward, natten_amd_linear_backward <- the projections of the reference's layers
+ *                                  (torch.nn.Linear in src/natten/modules.py)
  */
 #ifndef NATTEN_AMD_H_
 #define NATTEN_AMD_H_
