@@ -94,6 +94,7 @@ struct FnaParams {
   // tile is a grid of such boxes, one per wave.  Chosen per launch (choose_wave_box) so
   // that as many (wave, KV tile) pairs as possible need no element mask.
   int wave_box_lg[3];
+  int mostly_masked;  // ... and whether more than half of those pairs that are attended at all do (problems of several dimensions)
   int ext_base[3], ext_rem[3];  // qkv_shape / dil and qkv_shape % dil: extent of dilation group g = base + (g < rem)
   NaDiv d_stride[3], d_dil[3], d_q_tiled[3];
   NaDiv d_wg_group, d_groups_per_bh, d_heads_q, d_q_per_kv, d_num_groups;
@@ -502,7 +503,7 @@ static __device__ __forceinline__ void kv_tile_of_box(int i, const int (&n)[3], 
 // meet at every tile's barrier, and at the end the first takes the second's sums through LDS.  For launches that
 // leave a SIMD one wave, with nothing to fill its waits (see fna_fwd_paired_kernel).
 template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool SPLIT = false, bool NOMASK = false, int DC = 0,
-          bool CTX = false, bool PAIRED = false, typename Hook>
+          bool CTX = false, bool PAIRED = false, bool LATE = false, typename Hook>
 static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const int pid_in, Hook&& before_stores) {
   // split launches: which run of the Q tile's KV tiles this workgroup takes
   int split = 0, splits = 1, pid = pid_in;
@@ -521,10 +522,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // Where most tiles need the mask (windows small enough for tiles of 64 queries, see choose_small_forward_tiles) or
   // the vector units are the bound anyway (narrow rows, a context), the maxima are taken once, of the masked logits, and not
   // in the slots as well: 16 instructions less for a tile with a mask, the same number, but outside the matrix
-  // products' shadow, for one without.  Us before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 64 17.3 / 16.7, D 96 26.6 / 25.5,
-  // D 96 with 128 context tokens 30.5 / 29.1; 96 x 96, 21 x 21, H 8, D 64 43.0 / 41.5.  The other instances meet long
-  // runs of tiles without a mask: 32768 tokens, window 2048, D 128 40.4 / 40.8; 16384 tokens, D 32 31.1 / 32.0.
-  constexpr bool LATE_MAX = !NOMASK && !RAGGED && (NWAVES == 2 || NARROW || CTX);
+  // products' shadow, for one without.  LATE: the launch's tiles mostly need the mask (FnaParams::mostly_masked).  Us before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 64 17.3 / 16.7, D 96 26.6 / 25.5,
+  // D 96 with 128 context tokens 30.5 / 29.1; 96 x 96, 21 x 21, H 8, D 64 43.0 / 41.5.  Where tiles without a mask
+  // prevail that costs: 32768 tokens, window 2048, D 128 40.4 / 40.8; 16384 tokens, D 32 31.1 / 32.0.
+  constexpr bool LATE_MAX = !NOMASK && !RAGGED && (NWAVES == 2 || NARROW || CTX || LATE);
   // The instances with registers to spare hold the query's window, and read the coming tile's description ahead of the
   // mask: one of its three waits for LDS (16.7 -> 16.4 and 41.5 -> 40.9 us for the D 64 problems above).
   constexpr bool HOLD_WINDOW = LATE_MAX && NWAVES == 2 && D <= 64;
@@ -1572,7 +1573,7 @@ static __device__ __forceinline__ void clear_uncovered_rows(const FnaParams& p, 
   }
 }
 
-template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false>
+template <typename T, int D, int NWAVES, bool RAGGED, int KVT, bool NOMASK = false, int DC = 0, bool CTX = false, bool LATE = false>
 __global__ void __launch_bounds__(NWAVES * 64)
     __attribute__((amdgpu_waves_per_eu(fwd_min_waves(D, NOMASK), fwd_max_waves(D, NOMASK))))
 fna_fwd_kernel(const FnaParams p) {
@@ -1583,7 +1584,7 @@ fna_fwd_kernel(const FnaParams p) {
       return;
     }
   }
-  fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, false, NOMASK, DC, CTX>(p, int(blockIdx.x), []() {});
+  fna_fwd_tile<T, D, NWAVES, RAGGED, KVT, false, NOMASK, DC, CTX, false, LATE>(p, int(blockIdx.x), []() {});
 }
 
 // Split launch: kv_splits workgroups per Q tile, each on a contiguous run of the tile's KV tiles,
@@ -1782,6 +1783,7 @@ inline void choose_wave_box(FnaParams& p) {
     left -= best[a];
   }
   for (int a = 0; a < 3; ++a) p.wave_box_lg[a] = best[a];
+  p.mostly_masked = 0;
   if (p.cu_q) return;
   // the boxes that fit the Q tile; with one (every 1-D problem) there is nothing to choose
   int cand[21][3], n_cand = 0;
@@ -1809,9 +1811,10 @@ inline void choose_wave_box(FnaParams& p) {
   }
   key.anchor = p.anchor;
   thread_local Key last_key;
-  thread_local int last_box[3] = {-1, -1, -1};
+  thread_local int last_box[3] = {-1, -1, -1}, last_masked = 0;
   if (last_box[0] >= 0 && key == last_key) {
     for (int a = 0; a < 3; ++a) p.wave_box_lg[a] = last_box[a];
+    p.mostly_masked = last_masked;
     return;
   }
   // per dimension and box extent: (wave box, KV tile) pairs attended in full / attended at all,
@@ -1859,7 +1862,10 @@ inline void choose_wave_box(FnaParams& p) {
       for (int a = 0; a < 3; ++a) p.wave_box_lg[a] = cand[c][a];
     }
   }
+  const int* box = p.wave_box_lg;
+  p.mostly_masked = best_masked > 0.5 * some[0][box[0]] * some[1][box[1]] * some[2][box[2]];
   last_key = key;
+  last_masked = p.mostly_masked;
   for (int a = 0; a < 3; ++a) last_box[a] = p.wave_box_lg[a];
 }
 

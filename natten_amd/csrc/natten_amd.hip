@@ -139,6 +139,15 @@ int launch_fna(const FnaParams& p, hipStream_t stream, WorkQueue queues = {}) {
     pk.split_first = int(wgs);
     if (wgs + clearing > 0x7fffffffLL) return fail("fna_forward: problem needs more than 2^31 workgroups");
   }
+  // Launches whose tiles mostly need the mask take the maxima late (LATE_MAX; the same bits).  A tile with a mask gains about twice
+  // what one without loses, hence the line at half of them.  Us before / after, bf16: 2 x 96 x 96, 7 x 7, H 8, D 128 48.0 / 46.7; 100
+  // x 90, 31 x 17, H 12 78.9 / 76.5; 16 x 32 x 32, 5 x 9 x 9, H 8 98.2 / 95.4; 96 x 96, 21 x 21, H 8, D 64 43.3 / 41.6.
+  if constexpr (NWAVES == 4 && D >= 64 && !RAGGED && !NOMASK && DC == 0 && !CTX) {
+    if (p.mostly_masked) {
+      hipLaunchKernelGGL((fna_fwd_kernel<T, D, 4, false, KVT, false, 0, false, true>), dim3((unsigned)wgs), dim3(256), 0, stream, pk);
+      return check_launch("fna_forward");
+    }
+  }
   hipLaunchKernelGGL((fna_fwd_kernel<T, D, NWAVES, RAGGED, KVT, NOMASK, DC, CTX>), dim3((unsigned)(wgs + clearing)),
                      dim3(NWAVES * 64), 0, stream, pk);
   return check_launch("fna_forward");

@@ -104,7 +104,7 @@ def _prod(t) -> int:
 def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
     """What amd_fna_generic comes to for a forward call on checked arguments that fixes neither tiles nor route
     nor splits and has no scales, where that runs on the operands as they are: its tile shapes,
-    launch kind (work queue, "paired" or neither) and KV splits, or "float32"; None for everything else.  A small call is bound by the time it
+    launch kind (work queue, "paired" or neither) and KV splits (paired: by the two groups of a workgroup), or "float32"; None for everything else.  A small call is bound by the time it
     takes to get to its launch (256 tokens, float32: 23 us a call for 5 us of kernel), and the choices are a
     third of that time.  Plain values in and out: nothing here knows a tensor."""
     if dtype == torch.float32:
@@ -128,7 +128,7 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
             tiles = choose_small_forward_tiles(*problem, *tiles) or tiles
         # (other sums of the same windows, like other tiles: for calls that leave the launch open)
         if splits == 1 and launch_left_open and not narrow and paired_groups_default(shape[0], shape[-2], head_dim, *problem, *tiles):
-            persistent = "paired"
+            persistent, splits = "paired", 2
     if not _lib.fused_layout_supported(layout, dilation, tiles[1], row_bytes=heads_kv * padded_head_dim(head_dim) * 2,
                                        q_tile_shape=tiles[0], dtype=dtype):
         return None
@@ -144,7 +144,7 @@ def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is
     plan = _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel)
     if plan is None:
         return None
-    layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2] is True, plan[3]
+    layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2] is True, 1 if plan[2] == "paired" else plan[3]
     if any(x // d < t for x, d, t in zip(layout, dilation, tiles[1])):
         tiles = choose_fitting_forward_tiles(layout, kernel_size, stride, dilation, is_causal)
         # (other tiles than the plan looked at: their rows have to lie within the kernels' 32-bit offsets as well)
@@ -272,9 +272,10 @@ def amd_fna_generic(
             if plan == "float32":
                 output, lse = _lib.fna_forward_f32(*operands)
             elif plan[3] > 1:
-                output, lse = _lib.merge_parts(*_lib.fna_forward_fused_split(*operands, plan[0], plan[1], plan[3]))
-            elif plan[2] == "paired":
-                output, lse = _lib.fna_forward_fused_paired(*operands, plan[0], plan[1])
+                if plan[2] == "paired":
+                    output, lse = _lib.fna_forward_fused_paired(*operands, plan[0], plan[1])
+                else:
+                    output, lse = _lib.merge_parts(*_lib.fna_forward_fused_split(*operands, plan[0], plan[1], plan[3]))
             else:
                 output, lse = _lib.fna_forward_fused(*operands, plan[0], plan[1], run_persistent=plan[2])
             if out_dtype is not None and out_dtype != output.dtype:

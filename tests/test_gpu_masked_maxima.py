@@ -25,6 +25,18 @@ def test_walks_of_small_tiles(shape, kernel, stride, causal, tiles, head_dim):
     sampled_check(q, k, v, out, lse, kernel, stride, ones, causal, 300, seed=1)
 
 
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("shape,kernel,stride", [((40, 33), (7, 9), (1, 1)), ((9, 20, 22), (3, 5, 7), (1, 1, 2)), ((48, 48), (24, 24), (8, 8))])
+def test_mostly_masked_launches_give_the_bits_of_the_work_queue(shape, kernel, stride, head_dim):
+    q, k, v = make_qkv(2, shape, 4, 2, head_dim, torch.float16, seed=9)
+    ones = (1,) * len(shape)
+    with torch.no_grad():
+        per_tile, queue = (amd_fna_generic(q, k, v, kernel, stride, ones, (False,) * len(shape), return_lse=True,
+                                           run_persistent_kernel=kind, kv_splits=1) for kind in (False, True))
+    assert all(torch.equal(a, b) for a, b in zip(per_tile, queue))
+    sampled_check(q, k, v, *per_tile, kernel, stride, ones, (False,) * len(shape), 300, seed=1)
+
+
 @pytest.mark.parametrize("head_dim", [40, 64, 72, 96, 120])
 def test_keys_of_minus_infinity(head_dim):
     q, k, v = make_qkv(1, (24, 29), 2, 2, head_dim, torch.float16, seed=5)
