@@ -104,9 +104,9 @@ def _prod(t) -> int:
 def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
     """What amd_fna_generic comes to for a forward call on checked arguments that fixes neither tiles nor route
     nor splits and has no scales, where that runs on the operands as they are: its tile shapes,
-    launch kind (work queue, "paired" or neither) and KV splits (paired: by the two groups of a workgroup), or "float32"; None for everything else.  A small call is bound by the time it
-    takes to get to its launch (256 tokens, float32: 23 us a call for 5 us of kernel), and the choices are a
-    third of that time.  Plain values in and out: nothing here knows a tensor."""
+    launch kind (work queue, "paired" or neither) and KV splits (paired: by the two groups of a workgroup), or
+    "float32"; None for everything else.  A small call is bound by the time it takes to get to its launch (256 tokens,
+    float32: 23 us a call for 5 us of kernel), and the choices are a third of that time.  Plain values in and out: nothing here knows a tensor."""
     if dtype == torch.float32:
         return "float32"
     head_dim, layout = shape[-1], shape[1:-2]
