@@ -101,7 +101,7 @@ def _prod(t) -> int:
 
 
 @functools.lru_cache(maxsize=1024)
-def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel):
+def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel, pairs: bool = True):
     """What amd_fna_generic comes to for a forward call on checked arguments that fixes neither tiles nor route
     nor splits and has no scales, where that runs on the operands as they are: its tile shapes,
     launch kind (work queue, "paired" or neither) and KV splits (paired: by the two groups of a workgroup), or
@@ -124,11 +124,13 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
     splits = 1
     if not persistent:
         splits = (narrow_kv_splits_default if narrow else kv_splits_default)(shape[0], shape[-2], *problem, *tiles)
-        if splits == 1 and launch_left_open and not narrow and head_dim <= 64:
-            tiles = choose_small_forward_tiles(*problem, *tiles) or tiles
-        # (other sums of the same windows, like other tiles: for calls that leave the launch open)
-        if splits == 1 and launch_left_open and not narrow and paired_groups_default(shape[0], shape[-2], head_dim, *problem, *tiles):
-            persistent, splits = "paired", 2
+        # (pairs: other sums of the same windows, like other tiles: for calls that leave the launch open)
+        if launch_left_open and not narrow:
+            small = choose_small_forward_tiles(*problem, *tiles) if splits == 1 and head_dim <= 64 else None
+            if pairs and paired_groups_default(shape[0], shape[-2], head_dim, *problem, *tiles, splits, small is not None):
+                persistent, splits = "paired", 2
+            elif small is not None:
+                tiles = small
     if not _lib.fused_layout_supported(layout, dilation, tiles[1], row_bytes=heads_kv * padded_head_dim(head_dim) * 2,
                                        q_tile_shape=tiles[0], dtype=dtype):
         return None
@@ -141,10 +143,10 @@ def _context_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is
     taken for up to 48 KV tiles a Q tile: a split launch, dense attention and two merges take the host 68 us and the device
     17 beside the split walk, the whole walk in one launch 1.05 us a tile (head dim 128; 2 x 30 x 40, 21 x 21, H 4 and 128
     context tokens: 68 us so, 23 in one launch).  `context`: its tokens (see _joint_walk_pays)."""
-    plan = _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel)
+    plan = _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_causal, run_persistent_kernel, False)
     if plan is None:
         return None
-    layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2] is True, 1 if plan[2] == "paired" else plan[3]
+    layout, tiles, persistent, splits = shape[1:-2], plan[:2], plan[2], plan[3]
     if any(x // d < t for x, d, t in zip(layout, dilation, tiles[1])):
         tiles = choose_fitting_forward_tiles(layout, kernel_size, stride, dilation, is_causal)
         # (other tiles than the plan looked at: their rows have to lie within the kernels' 32-bit offsets as well)

@@ -59,4 +59,6 @@ def test_where_it_is_chosen():
     assert kind((32768,), 1, 128, (512,)) is False         # few KV tiles
     assert kind((8192,), 1, 128, (2048,)) is False         # a split launch
     assert kind((32768,), 1, 96, (2048,)) is False
+    assert kind((128, 128), 2, 64, (13, 13)) == "paired" and kind((64, 64), 4, 64, (15, 15)) is False  # 64 x 64 tiles: 256 and fewer
+    assert kind((8192,), 2, 64, (600,)) == "paired" and kind((8192,), 2, 64, (3500,)) is False   # a two-way split's walks: short ones
     assert kind((32768,), 1, 128, (2048,), launch=False) is False and kind((32768,), 1, 128, (2048,), launch=True) is True
