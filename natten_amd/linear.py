@@ -45,7 +45,10 @@ def _nothing_watches() -> bool:
 def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
     """Whether the kernels stand for calling `module` on x (whose last dimensions hold its input columns) and
     splitting the result into `parts`: a plain nn.Linear that nothing is attached to, 16-bit operands on one device, columns that
-    the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear."""
+    the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is asked first: a
+    tracer cannot take a data pointer apart, a transform's tensors have none.)"""
+    if not _nothing_watches():
+        return False
     if type(module) is not nn.Linear or "forward" in module.__dict__:
         return False
     if module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or _has_any_global_hook():
@@ -59,7 +62,7 @@ def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
         return False
     w, b = module.weight, module.bias
     return (_plain(w, x.dtype, x.device, 16) and tuple(w.shape) == (n, k)
-            and (b is None or _plain(b, x.dtype, x.device, 8)) and _nothing_watches())
+            and (b is None or _plain(b, x.dtype, x.device, 8)))
 
 
 def _aligned(t: Tensor) -> Tensor:

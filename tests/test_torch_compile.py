@@ -97,3 +97,43 @@ def test_compiled_training_step_equals_eager(name):
         grads.append([a.grad for a in args])
     for a, b in zip(*grads):
         assert torch.equal(a, b)
+
+
+LAYERS = {
+    "1d": (natten_amd.NeighborhoodAttention1D, (128, 2, 7), (2, 40, 128)),
+    "2d": (natten_amd.NeighborhoodAttention2D, (128, 4, (5, 5)), (1, 12, 13, 128)),
+    "3d causal": (natten_amd.NeighborhoodAttention3D, (64, 2, (3, 3, 3), 1, 1, (True, False, False)), (1, 4, 6, 5, 64)),
+}
+
+
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("name", sorted(LAYERS))
+def test_layers_trace_into_one_graph_with_fake_tensors(name, train):
+    cls, args, shape = LAYERS[name]
+    torch._dynamo.reset()
+    with FakeTensorMode():
+        layer, width = cls(*args), args[0]  # (fake parameters cannot be moved: made where they belong)
+        layer.qkv = torch.nn.Linear(width, 3 * width, device="cuda", dtype=torch.bfloat16)
+        layer.proj = torch.nn.Linear(width, width, device="cuda", dtype=torch.bfloat16)
+        x = torch.empty(shape, device="cuda", dtype=torch.bfloat16, requires_grad=train)
+        with torch.set_grad_enabled(train):
+            out = torch.compile(layer, backend="eager", fullgraph=True)(x)
+    assert tuple(out.shape) == shape and out.dtype == torch.bfloat16 and out.requires_grad == train
+
+
+@pytest.mark.gpu
+def test_compiled_layer_step_agrees_with_eager():
+    torch._dynamo.reset()
+    torch.manual_seed(0)
+    cls, args, shape = LAYERS["2d"]
+    layer = cls(*args).to("cuda", torch.bfloat16)
+    x, d_out = (torch.randn(shape, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    results = []
+    for f in (layer, torch.compile(layer, backend="aot_eager", fullgraph=True)):
+        leaf = x.clone().requires_grad_(True)
+        out = f(leaf)
+        results.append([out.detach(), *torch.autograd.grad(out, [leaf, *layer.parameters()], d_out)])
+    # the eager layer's maps are kernels of their own: two roundings to bf16 of the same sums, carried through the attention
+    # and the second map
+    for a, b in zip(*results):
+        assert float((a.double() - b.double()).norm()) <= 2.0**-6 * float(b.double().norm())
