@@ -23,11 +23,11 @@ from .fna import amd_fna_generic, backward_route
 from .functional import neighborhood_attention_generic
 from .tile_config import BACKWARD_TILE_SIZE, choose_tile_shapes
 
-# Sizes of a map that these kernels are the faster way for: input and output columns up to which they were measured against
-# the library (us, here / there: 12544 tokens, 256 -> 768: y 13.7 / 21.7, dx 10.0 / 18.6, dw and db 20.5 / 90; 36864 tokens, 512 -> 1536:
+# Widest layer that takes these kernels: where measuring against the library ended, not where the library was found to be the faster
+# way (us, here / there: 12544 tokens, 256 -> 768: y 13.7 / 21.7, dx 10.0 / 18.6, dw and db 20.5 / 90; 36864 tokens, 512 -> 1536:
 # y 79.6 / 104, dx 64.3 / 60 to 65, dw and db 108 / 254; 196 tokens, 512 -> 1536: y 7.9 / 18.9, dx 12.6 / 18.2, dw and db 11.1 / 27;
 # below 20 us a call is the time the host takes to make it).
-MAX_COLUMNS_IN, MAX_COLUMNS_PART = 512, 512
+MAX_COLUMNS = 512
 
 
 def _plain(t: Optional[Tensor], dtype: torch.dtype, device: torch.device, align: int) -> bool:
@@ -43,9 +43,9 @@ def _nothing_watches() -> bool:
 
 
 def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
-    """Whether the kernels stand for calling `module` on x (whose last dimensions hold its input columns) and
-    splitting the result into `parts`: a plain nn.Linear that nothing is attached to, 16-bit operands on one device, columns that
-    the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is asked first: a
+    """Whether the kernels stand for calling `module` on x [.., columns] and splitting the result into `parts` of as
+    many columns each: a plain nn.Linear of these sizes that nothing is attached to, 16-bit operands on one device, columns
+    that the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is asked first: a
     tracer cannot take a data pointer apart, a transform's tensors have none.)"""
     if not _nothing_watches():
         return False
@@ -54,7 +54,9 @@ def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
     if module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or _has_any_global_hook():
         return False
     n, k = module.out_features, module.in_features
-    if k % 64 or n % (64 * parts) or k > MAX_COLUMNS_IN or n > MAX_COLUMNS_PART * parts:
+    if k != x.shape[-1] or n != parts * k:  # (another output width than the layer's, or a map that does not fit)
+        return False
+    if k % 64 or k > MAX_COLUMNS:
         return False
     if type(x) not in (Tensor, nn.Parameter) or not x.is_cuda or x.dtype not in (torch.float16, torch.bfloat16):
         return False
@@ -62,7 +64,7 @@ def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
         return False
     w, b = module.weight, module.bias
     return (_plain(w, x.dtype, x.device, 16) and tuple(w.shape) == (n, k)
-            and (b is None or _plain(b, x.dtype, x.device, 8)))
+            and (b is None or (_plain(b, x.dtype, x.device, 8) and tuple(b.shape) == (n,))))
 
 
 def _aligned(t: Tensor) -> Tensor:

@@ -137,6 +137,48 @@ def test_what_is_attached_to_a_map_is_kept():
     layer(x)
 
 
+@pytest.mark.parametrize("columns", [64, 192])
+def test_an_output_map_to_another_width_is_that_of_its_module(columns, monkeypatch):
+    layer, x = _layer(), torch.randn((2, 12, 13, 128), device="cuda", dtype=torch.bfloat16)
+    layer.proj = nn.Linear(128, columns).to("cuda", torch.bfloat16)
+    d = torch.randn((2, 12, 13, columns), device="cuda", dtype=torch.bfloat16)
+    got = _step(layer, x, d)
+    with torch.no_grad():
+        assert torch.equal(layer(x), got[0])
+    monkeypatch.setattr(linear, "takes_linear", lambda *a: False)
+    assert got[0].shape == d.shape and all(torch.equal(a, b) for a, b in zip(got, _step(layer, x, d)))
+
+
+@pytest.mark.parametrize("name,sizes", [("proj", (64, 64)), ("proj", (256, 128)), ("qkv", (64, 192)), ("qkv", (64, 384)),
+                                        ("qkv", (128, 192))])
+@pytest.mark.parametrize("grad", [False, True])
+def test_maps_that_do_not_fit_the_layer_are_refused(name, sizes, grad):
+    layer, x = _layer(), torch.randn((2, 12, 14, 128), device="cuda", dtype=torch.bfloat16)
+    setattr(layer, name, nn.Linear(*sizes).to("cuda", torch.bfloat16))
+    assert not linear.takes_linear(getattr(layer, name), x, 3 if name == "qkv" else 1)
+    with torch.set_grad_enabled(grad), pytest.raises(RuntimeError, match="shapes cannot be multiplied|is invalid for input of size"):
+        layer(x)
+
+
+def test_a_bias_of_one_element_is_left_to_its_module():
+    layer, x = _layer(), torch.randn((2, 12, 13, 128), device="cuda", dtype=torch.bfloat16)
+    layer.proj.bias = nn.Parameter(torch.ones((1,), device="cuda", dtype=torch.bfloat16))
+    assert not linear.takes_linear(layer.proj, x, 1)
+    with torch.no_grad():
+        assert layer(x).shape == x.shape
+
+
+def test_tensors_that_do_not_fit_a_map_are_refused():
+    x, w = torch.zeros((8, 128), dtype=torch.bfloat16, device="cuda"), torch.zeros((64, 64), dtype=torch.bfloat16, device="cuda")
+    for operand, shape in ((x, (8, 128)), (x, (16, 64)), (x.view(16, 64), (8, 64)), (x.view(16, 64), (8, 128))):
+        with pytest.raises(ValueError, match="columns|rows"):
+            _lib.linear_forward(operand, w, None, 1, shape)
+    with pytest.raises(ValueError, match="columns"):
+        _lib.linear_backward([x], x, w, True, True, False)
+    with pytest.raises(ValueError, match="rows"):
+        _lib.linear_backward([x.view(16, 64)[:8]], x.view(16, 64), w, True, True, False)
+
+
 def test_frozen_weights_and_saved_tensor_hooks():
     layer, x = _layer(), torch.randn((1, 8, 8, 128), device="cuda", dtype=torch.bfloat16)
     d = torch.randn_like(x)
