@@ -732,7 +732,8 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     }
   }
 
-  // PAIRED: the second group's half; of an odd number the middle tile is described to both and skipped by the second
+  // PAIRED: the second group's half; of an odd number the middle tile is described to both and skipped by the second,
+  // which multiplies zeros for its values
   bool skip_first = false;
   if constexpr (PAIRED) {
     total_tiles = (box_tiles + 1) / 2;
@@ -987,7 +988,16 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     to_lim(rows.lim, k_lim, ld_koff, KLayout{});
     to_lim(rows.lim, v_lim, ld_voff, VLayout{});
     issue_tile_load(kbase, ld_koff, sK0, rows, KLayout{});
-    issue_tile_load(vbase, ld_voff, sV0, rows, VLayout{});
+    if (PAIRED && skip_first) {
+      // the tile is the other group's; zeros as its values here: probabilities of 0 would make NaN of infinities
+#pragma unroll
+      for (int i = tid; i < TILE_BYTES / 16; i += NT) {
+        const u32x4_t zero = {0, 0, 0, 0};
+        reinterpret_cast<u32x4_t*>(sV0 + TILE_BYTES * group_id)[i] = zero;
+      }
+    } else {
+      issue_tile_load(vbase, ld_voff, sV0, rows, VLayout{});
+    }
   }
 
   // ---- this lane's query row, on its way while the tables below are formed ---------------------------

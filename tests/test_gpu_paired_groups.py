@@ -34,6 +34,26 @@ def test_matches_oracle(case, head_dim, dtype):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("head_dim", [64, 128])
+@pytest.mark.parametrize("case", CASES)
+def test_infinite_values_reach_the_queries_that_one_group_lets_them_reach(case, head_dim):
+    # (an odd walk's middle tile lies before both groups: the second multiplies its values by probabilities of zero)
+    shape, kernel, stride, dilation, causal, tiles = case
+    q, k, v = make_qkv(2, shape, 2, 2, head_dim, torch.bfloat16, seed=12)
+    tokens = v.view(2, -1, 2, head_dim)
+    gen = torch.Generator().manual_seed(3)
+    for b in range(2):
+        for h in range(2):
+            # every batch entry and head has infinities of its own: few, many
+            tokens[b, torch.randperm(tokens.shape[1], generator=gen)[: (2, 5, 20, 80)[2 * b + h]].cuda(), h, 7] = float("inf")
+    problem = (q, k, v, kernel, stride, dilation, causal, head_dim**-0.5, *tiles)
+    ref, ref_lse = _lib.fna_forward_fused(*problem)
+    out, lse = _lib.fna_forward_fused_paired(*problem)
+    assert torch.isinf(ref).any() and not torch.isnan(lse).any()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref)) and torch.equal(torch.isinf(out), torch.isinf(ref))
+
+
+@pytest.mark.gpu
 def test_chosen_call_replays_in_a_graph():
     q, k, v = make_qkv(1, (8192,), 4, 2, 64, torch.bfloat16, seed=2)
     with torch.no_grad():
