@@ -12,7 +12,6 @@ from __future__ import annotations
 import contextlib
 import ctypes
 import functools
-import math
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -739,29 +738,24 @@ def _three(tensors) -> Tuple[Optional[int], ...]:
     return tuple(t.data_ptr() for t in tensors) + (None,) * (3 - len(tensors))
 
 
-def _rows(shape, columns: int) -> int:
-    """Rows of a tensor whose last dimensions hold `columns` elements."""
-    held, i = 1, len(shape)
-    while i > 0 and held < columns:
-        i -= 1
-        held *= shape[i]
-    if held != columns:
-        raise ValueError(f"The last dimensions of {tuple(shape)} do not hold {columns} columns.")
-    return math.prod(shape[:i])
+def _holds_columns(shape, columns: int) -> bool:
+    """Whether the last dimension of a tensor, or its last two, hold `columns` elements."""
+    return shape[-1] == columns or (len(shape) > 1 and shape[-2] * shape[-1] == columns)
 
 
 def linear_forward(x: Tensor, weight: Tensor, bias: Optional[Tensor], parts: int, shape) -> Tuple[Tensor, ...]:
     """x (rows of weight.shape[1] elements) weight^T + bias, its columns split into `parts` tensors of `shape`."""
     n, k = weight.shape
     _require_gpu(x, weight)
-    rows = _rows(x.shape, k)
-    if n % parts or _rows(shape, n // parts) != rows:
-        raise ValueError(f"{parts} tensors of {tuple(shape)} do not hold {rows} rows of the {n} columns of a map of {tuple(x.shape)}.")
+    if not (_holds_columns(x.shape, k) and _holds_columns(shape, n // parts)):
+        raise ValueError(f"A map of {k} to {n} columns does not take {tuple(x.shape)} to {parts} tensors of {tuple(shape)}.")
     outs = tuple(torch.empty(shape, dtype=x.dtype, device=x.device) for _ in range(parts))
+    if outs[0].numel() * parts * k != x.numel() * n:
+        raise ValueError(f"{parts} tensors of {tuple(shape)} do not hold the {n} columns of a map of {tuple(x.shape)}.")
     with _on_device(x):
         _check(lib().natten_amd_linear_forward(
             x.data_ptr(), weight.data_ptr(), None if bias is None else bias.data_ptr(), *_three(outs), DTYPE_CODES[x.dtype],
-            rows, n, k, n // parts, _stream(x)))
+            x.numel() // k, n, k, n // parts, _stream(x)))
     return outs
 
 
@@ -778,8 +772,8 @@ def linear_backward(d_outs, x: Tensor, weight: Tensor, need_x: bool, need_weight
     None where not needed.  (A bias gradient comes with the weight's.)"""
     n, k = weight.shape
     _require_gpu(x, weight, *d_outs)
-    rows, part = _rows(x.shape, k), n // len(d_outs)
-    if any(_rows(d.shape, part) != rows for d in d_outs):
+    rows, part = x.numel() // k, n // len(d_outs)
+    if any(d.numel() != rows * part for d in d_outs):
         raise ValueError(f"Gradients of {[tuple(d.shape) for d in d_outs]} do not hold {rows} rows of {part} columns each.")
     dx = torch.empty_like(x) if need_x else None
     dw = db = workspace = None

@@ -47,8 +47,10 @@ def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
     many columns each: a plain nn.Linear of these sizes that nothing is attached to, 16-bit operands on one device, columns
     that the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is asked first: a
     tracer cannot take a data pointer apart, a transform's tensors have none.)"""
-    if not _nothing_watches():
-        return False
+    return _nothing_watches() and _fits(module, x, parts)
+
+
+def _fits(module: nn.Module, x: Tensor, parts: int) -> bool:
     if type(module) is not nn.Linear or "forward" in module.__dict__:
         return False
     if module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks or _has_any_global_hook():
@@ -153,7 +155,7 @@ class _Layer(torch.autograd.Function):
 def layer_step(qkv: nn.Linear, proj: nn.Linear, x: Tensor, heads: int, problem, scale: float) -> Optional[Tensor]:
     """proj(attention(qkv(x))), or None where the maps or their surroundings are not what takes_linear takes.  `problem`:
     kernel size, stride, dilation and causality per dimension."""
-    if not (takes_linear(qkv, x, 3) and takes_linear(proj, x, 1)):
+    if not (takes_linear(qkv, x, 3) and _fits(proj, x, 1)):
         return None
     params = (qkv.weight, qkv.bias, proj.weight, proj.bias)
     layout, head_dim = tuple(x.shape[1:-1]), x.shape[-1] // heads

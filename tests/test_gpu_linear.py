@@ -171,10 +171,8 @@ def test_a_bias_of_one_element_is_left_to_its_module():
 def test_tensors_that_do_not_fit_a_map_are_refused():
     x, w = torch.zeros((8, 128), dtype=torch.bfloat16, device="cuda"), torch.zeros((64, 64), dtype=torch.bfloat16, device="cuda")
     for operand, shape in ((x, (8, 128)), (x, (16, 64)), (x.view(16, 64), (8, 64)), (x.view(16, 64), (8, 128))):
-        with pytest.raises(ValueError, match="columns|rows"):
+        with pytest.raises(ValueError, match="columns"):
             _lib.linear_forward(operand, w, None, 1, shape)
-    with pytest.raises(ValueError, match="columns"):
-        _lib.linear_backward([x], x, w, True, True, False)
     with pytest.raises(ValueError, match="rows"):
         _lib.linear_backward([x.view(16, 64)[:8]], x.view(16, 64), w, True, True, False)
 
