@@ -203,6 +203,8 @@ int natten_amd_fna_forward_fused_split(const void* q, const void* k, const void*
  * workgroup has two groups of waves, each on half of its Q tile's KV tiles, and adds up their results itself.
  * fp16 / bf16 operands, head_dim 64 or 128, Q tiles of 128 and KV tiles of 64 tokens, no dilation group narrower than a
  * KV tile, no dequantisation scales; other arguments as in natten_amd_fna_forward_fused.
+ * At head_dim 128 a launch that natten_amd_fna_fully_block_sparse reports runs on its mask-free kernel, one group of
+ * waves per Q tile.
  */
 int natten_amd_fna_forward_fused_paired(const void* q, const void* k, const void* v, void* out, float* lse,
                                         int dtype, int na_dim, int batch, int heads_q, int heads_kv,

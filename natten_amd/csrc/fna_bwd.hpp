@@ -347,8 +347,9 @@ static __device__ __forceinline__ float dot8(typename Mma<T>::vec8 a, typename M
 }
 
 // Waves per SIMD the compiler makes room for (and, as the attribute's maximum, limits the kernel to).  Of the
-// SIMD's 512 registers a lane, the key-stationary and the dQ instance take 224 and 256 at head dim 128, 229 and
-// 210 at 64, 168 and 167 at 32; the dQ instance at 128 spills 9 more (11 where sequences end inside a tile).  One wave
+// SIMD's 512 registers a lane, the key-stationary and the dQ instance take 213 to 219 and 248 at head dim 128 (249
+// where it comes first and holds the output's fragments as well, 252 where sequences end inside a tile), 213 to 217
+// and 198 to 200 at 64, 158 to 162 and 159 or 160 at 32; none spills.  One wave
 // more for the dQ role at 64 and 32 needs its LSE and delta in a register each instead of sixteen copies that
 // the accumulators start from, and two additions a logit: dQ launch in us, copies / one wave more, D 64: 48 x 48
 // tokens, H 6, 11 x 11 18.5 / 20.3; 4 x 56 x 56, H 8, 7 x 7 39.5 / 41.9; 16 x 40 x 40, H 12, 7 x 15 x 15 409 / 424; D 32: 24 x
@@ -822,7 +823,8 @@ fna_bwd_kernel(const FnaBwdParams p) {
   // rows 4 g + e [+ 8], chunk 4 db + v_chunk.  The chunk numbers differ by exclusive or as the swizzle does, and stages begin at
   // multiples of a row of chunks, so that every fragment's address is one lane offset with a few bits turned over: an
   // instruction each where it is used, as an addition to the stage's base would be, and two registers instead of
-  // sixteen (head dim 128: the paired role 246 -> 216, the dQ role 256 and 9 spilled -> 244).
+  // sixteen (head dim 128: the paired role 246 -> 216, the dQ role 256 and 9 spilled -> 244, with three fragments read
+  // ahead 248).
   const uint32_t k_lane = uint32_t(l32 * ROWB + L::u_slot(l32, g) * 16);
   const int l16 = lane & 15;
   const int v_e = l16 >> 2, v_j4 = l16 & 3;

@@ -522,9 +522,10 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
   // Where most tiles need the mask (windows small enough for tiles of 64 queries, see choose_small_forward_tiles) or
   // the vector units are the bound anyway (narrow rows, a context), the maxima are taken once, of the masked logits, and not
   // in the slots as well: 16 instructions less for a tile with a mask, the same number, but outside the matrix
-  // products' shadow, for one without.  LATE: the launch's tiles mostly need the mask (FnaParams::mostly_masked).  Us before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 64 17.3 / 16.7, D 96 26.6 / 25.5,
-  // D 96 with 128 context tokens 30.5 / 29.1; 96 x 96, 21 x 21, H 8, D 64 43.0 / 41.5.  Where tiles without a mask
-  // prevail that costs: 32768 tokens, window 2048, D 128 40.4 / 40.8; 16384 tokens, D 32 31.1 / 32.0.
+  // products' shadow, for one without.  LATE: the launch's tiles mostly need the mask (FnaParams::mostly_masked).  Us of the
+  // launch before / after: 2 x 64 x 64 tokens, 13 x 13, H 8, D 64 17.3 / 16.7, D 96 26.6 / 25.5, D 96 with 128
+  // context tokens 30.5 / 29.1; 96 x 96, 21 x 21, H 8, D 64 43.0 / 41.5.  Where tiles without a mask prevail that
+  // costs: 32768 tokens, window 2048, D 128 40.4 / 40.8; 16384 tokens, D 32 31.1 / 32.0.
   constexpr bool LATE_MAX = !NOMASK && !RAGGED && (NWAVES == 2 || NARROW || CTX || LATE);
   // The instances with registers to spare hold the query's window, and read the coming tile's description ahead of the
   // mask: one of its three waits for LDS (16.7 -> 16.4 and 41.5 -> 40.9 us for the D 64 problems above).
@@ -990,7 +991,6 @@ static __device__ __forceinline__ void fna_fwd_tile(const FnaParams& p, const in
     issue_tile_load(kbase, ld_koff, sK0, rows, KLayout{});
     if (PAIRED && skip_first) {
       // the tile is the other group's; zeros as its values here: probabilities of 0 would make NaN of infinities
-#pragma unroll
       for (int i = tid; i < TILE_BYTES / 16; i += NT) {
         const u32x4_t zero = {0, 0, 0, 0};
         reinterpret_cast<u32x4_t*>(sV0 + TILE_BYTES * group_id)[i] = zero;

@@ -271,10 +271,14 @@ inline void choose_f32_boxes(FnaF32Params& p) {
 // V operands and results are VEC-wide loads and stores of whole rows.
 // Softmax in float32; a row's maximum is followed once it grew by more than 2^8 (exact: the sums are
 // normalised by the same maximum).
-// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 51 us (56 TFLOP/s of window pairs, 85 of pairs
-// multiplied; the card's float32 matrix products reach 154), 300 us as permutes, 128-query kernel and
-// unpermutes.  Of a wave's 81000 cycles there 63000 are its fifteen blocks, the matrix pipe full with four waves a SIMD,
-// and 16000 the set-up and the way of the first block; 256 tokens, H 2, D 32, window 7: 17 us, all of it the call, from 83.
+// 2 x 64 x 64 tokens, H 8, D 64, 13 x 13 windows: 50 us (57 TFLOP/s of window pairs, 83 of pairs
+// multiplied), 300 us as permutes, 128-query kernel and unpermutes; 256 tokens, H 2, D 32, window 7: 17 us, all of it the
+// call, from 83.  Where the first's time goes (all 4096 waves are resident at once, four a SIMD): the launch keeps the shader
+// engines busy for 110000 cycles (SQ_BUSY_CYCLES), of which the matrix pipe of a SIMD works 63000 (SQ_VALU_MFMA_BUSY_CYCLES), the
+// fifteen blocks of its four waves, nearly without a gap.  A wave lives 81000 to 85000 (SQ_WAVE_CYCLES), 16000 of them and more
+// set-up and the way of the first block; the 25000 others are the begin and end of the launch, when a SIMD does not have its
+// waves yet or no longer.  0.57 of the pipe's time, at 2.2 of the 2.35 GHz at which a large product reaches 154
+// TFLOP/s, are those 83.
 template <int D, bool PAD, bool WIDE = false, int SETS = (D == 32 ? 2 : 1)>
 __global__ void __launch_bounds__(256, 2) fna_fwd_f32_direct_kernel(const FnaF32Params p) {
   constexpr int KJ = D / 16;

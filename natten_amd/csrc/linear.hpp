@@ -52,8 +52,8 @@ constexpr int kLinearStep = 64;  // of the contraction
 constexpr int kLinearStages = 2;
 constexpr int linear_lds_bytes(int rt, int ct) { return kLinearStages * (rt + ct) * kLinearStep * 2; }
 
-// One tile of a result, RT rows by CT columns, four waves in a square; `block`: the workgroup's number in this part of a launch (which
-// has a multiple of the XCD count of them), `lds`: linear_lds_bytes(RT, CT).
+// One tile of a result, RT rows by CT columns, four waves in a square; `block`: the workgroup's number in this part of a
+// launch (which has a multiple of the XCD count of them), `lds`: linear_lds_bytes(RT, CT).
 template <typename T, int MODE, int RT, int CT>
 static __device__ __forceinline__ void linear_tile(const LinearParams& p, const int block, char* lds) {
   using M = Mma<T>;

@@ -242,8 +242,11 @@ int dispatch_tiles(const FnaParams& p, int qt, int kvt, hipStream_t stream, Work
     if (qt == 128 && kvt == 64) return launch_fna<T, D, 4, true, 64>(p, stream);
     return fail("fna_forward: seqlen_kv (%d) must be a multiple of the KV tile (%d tokens)", p.seqlen_kv, kvt);
   }
-  // (A fully block-sparse launch of head dim 128 keeps its mask-free instance: 16 x 32 x 32, 8 x 16 x 16 blocked, H 2: 37.1 us
-  // there, 37.9 as pairs with masks.  Head dim 64: 32768 tokens, 2048 blocked by 128, H 1: 24.0 and 22.5.)
+  // (A fully block-sparse launch of head dim 128 keeps its mask-free instance, one group a Q tile: 16 x 32 x 32, 8 x 16 x 16
+  // blocked, H 2: 37.1 us there, 37.9 as pairs with masks; 8192 tokens blocked by 128, windows of 8, 12 and 16 KV tiles, us in one
+  // group / split in two and merged / as pairs, 64 Q tiles 12.1 / 15.2 / 13.5, 15.0 / 16.6 / 16.0, 18.0 / 18.3 / 18.2, 128
+  // Q tiles 12.5 / 18.3 / 13.9, 15.3 / 20.2 / 16.4, 18.2 / 22.0 / 18.6.  Head dim 64: 32768 tokens, 2048 blocked by
+  // 128, H 1: 24.0 and 22.5; the 8192 tokens with 64 Q tiles 9.1 / 11.8 / 9.5, 11.4 / 13.0 / 11.1, 13.4 / 14.1 / 12.6.)
   if (queues.paired && !(D == 128 && qt == 128 && kvt == 64 && fully_block_sparse(p))) {
     if constexpr (D >= 64) {
       if (qt == 128 && kvt == 64) return launch_paired<T, D>(p, stream);

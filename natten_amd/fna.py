@@ -106,7 +106,8 @@ def _open_call_plan(dtype, shape, heads_kv, kernel_size, stride, dilation, is_ca
     nor splits and has no scales, where that runs on the operands as they are: its tile shapes,
     launch kind (work queue, "paired" or neither) and KV splits (paired: by the two groups of a workgroup), or
     "float32"; None for everything else.  A small call is bound by the time it takes to get to its launch (256 tokens,
-    float32: 23 us a call for 5 us of kernel), and the choices are a third of that time.  Plain values in and out: nothing here knows a tensor."""
+    float32: 23 us a call for 5 us of kernel), and the choices are a third of that time.  Plain values in and out:
+    nothing here knows a tensor."""
     if dtype == torch.float32:
         return "float32"
     head_dim, layout = shape[-1], shape[1:-2]
@@ -240,7 +241,10 @@ def amd_fna_generic(
     Q tiles from per-XCD queues) instead of a workgroup per Q tile; True gives the bits of an unsplit
     False.  None: whichever was measured faster for this kind of problem (`functional.work_queue_default`);
     the tiles are then open too (`choose_small_forward_tiles`, when `kv_splits` is None as well), and with
-    them the order of summation.
+    them the order of summation.  Calls without gradients that fix nothing may also run with two groups of waves a Q tile
+    (`functional.paired_groups_default`); so does the forward of a layer's training step in one node
+    (`linear._Layer`).  The forward of other calls that record gradients, and of compiled ones, does not, and sums in
+    another order there.
 
     `anchored_tiles` (one-launch path only): KV tiles are laid out from the first key of a Q tile's
     window instead of from multiples of the tile extent, so that no tile lies partly before the

@@ -285,8 +285,9 @@ def paired_groups_default(batch: int, heads: int, head_dim: int, token_layout, k
     (in two dimensions, most of them with a mask, 20.3 / 19.5), 18 25.4 / 25.2 (30.7 / 28.0), 34 41.9 / 40.5, 66 71.5 / 68.1; head
     dim 64: 6 11.4 / 10.9, 10 12.8 / 12.0, 34 27.8 / 24.2.  `splits`: what kv_splits_default says.  A walk that two workgroups
     would share is that of a pair up to 24 KV tiles at head dim 64 and 16 at 128: no merge launch, which also takes
-    the host 26 us a call (split and merged / paired, device: 12 tiles, 64 Q tiles 13.8 / 12.5 and 17.3 / 17.4, 128 Q tiles 15.0 / 12.7 and
-    20.6 / 17.8; 20 tiles 17.3 / 16.1 and 24.9 / 25.5; 34 tiles 21.4 / 21.8 and 30.0 / 30.9).  `small`: tiles of 64 x 64 tokens are
+    the host 26 us a call (split and merged / paired, device: 12 tiles, 64 Q tiles 13.8 / 12.5 and 17.3 / 17.4, 128 Q tiles
+    15.0 / 12.7 and 20.6 / 17.8; 20 tiles 17.3 / 16.1 and 24.9 / 25.5; 34 tiles 21.4 / 21.8 and 30.0 / 30.9).  (Without
+    masks at head dim 128 the entry point takes one group, faster still.)  `small`: tiles of 64 x 64 tokens are
     the alternative (choose_small_forward_tiles), which up to 128 Q tiles of 128 leave each a compute unit as well: 64 x 64, 15 x 15,
     H 4 13.0 / 13.9, 33 x 47, 19 x 19, H 6 18.0 / 18.6; 256 Q tiles: 128 x 128, 13 x 13, H 2 14.3 / 12.8, 21 x 21 22.3 / 17.9."""
     if splits > 2 or head_dim not in (64, 128) or math.prod(q_tile_shape) != 128 or math.prod(kv_tile_shape) != 64:

@@ -23,10 +23,10 @@ from .fna import amd_fna_generic, backward_route
 from .functional import neighborhood_attention_generic
 from .tile_config import BACKWARD_TILE_SIZE, choose_tile_shapes
 
-# Widest layer that takes these kernels: where measuring against the library ended, not where the library was found to be the faster
-# way (us, here / there: 12544 tokens, 256 -> 768: y 13.7 / 21.7, dx 10.0 / 18.6, dw and db 20.5 / 90; 36864 tokens, 512 -> 1536:
-# y 79.6 / 104, dx 64.3 / 60 to 65, dw and db 108 / 254; 196 tokens, 512 -> 1536: y 7.9 / 18.9, dx 12.6 / 18.2, dw and db 11.1 / 27;
-# below 20 us a call is the time the host takes to make it).
+# Widest layer that takes these kernels: where measuring against the library ended, not where the library was found to be the
+# faster way (us, here / there: 12544 tokens, 256 -> 768: y 13.7 / 21.7, dx 10.0 / 18.6, dw and db 20.5 / 90; 36864
+# tokens, 512 -> 1536: y 79.6 / 104, dx level (64.3 / 60 to 65), dw and db 108 / 254; 196 tokens, 512 -> 1536: y 7.9 / 18.9,
+# dx 12.6 / 18.2, dw and db 11.1 / 27; below 20 us a call is the time the host takes to make it).
 MAX_COLUMNS = 512
 
 
@@ -45,8 +45,8 @@ def _nothing_watches() -> bool:
 def takes_linear(module: nn.Module, x: Tensor, parts: int) -> bool:
     """Whether the kernels stand for calling `module` on x [.., columns] and splitting the result into `parts` of as
     many columns each: a plain nn.Linear of these sizes that nothing is attached to, 16-bit operands on one device, columns
-    that the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is asked first: a
-    tracer cannot take a data pointer apart, a transform's tensors have none.)"""
+    that the kernels take, and no one watching the call.  Everything else goes the way of nn.Linear.  (Who watches is
+    asked first: a tracer cannot take a data pointer apart, a transform's tensors have none.)"""
     return _nothing_watches() and _fits(module, x, parts)
 
 

@@ -6,6 +6,7 @@ from torch import nn
 
 import natten_amd
 from natten_amd import _lib, linear
+from natten_amd.fna import _open_call_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -111,6 +112,23 @@ def test_layer_steps_of_both_routes_agree(qkv_bias, monkeypatch):
     second = twice(layer)
     monkeypatch.setattr(linear, "takes_linear", lambda *a: False)
     assert _close(second, twice(layer))
+
+
+def test_a_step_whose_forward_runs_in_pairs_agrees_with_the_other_routes(monkeypatch):
+    # the one node's forward leaves the launch open (two groups of waves a Q tile here), those of three nodes and of the
+    # general route do not: other orders of summation
+    torch.manual_seed(0)
+    layer = natten_amd.NeighborhoodAttention2D(128, 2, (13, 13)).to("cuda", torch.bfloat16)
+    plan = _open_call_plan(torch.bfloat16, (1, 128, 128, 2, 64), 2, *((n, n) for n in (13, 1, 1)), (False, False), None)
+    assert plan[2] == "paired"
+    x, d = (torch.randn((1, 128, 128, 128), device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    own = _step(layer, x, d)
+    with torch.no_grad():
+        assert torch.equal(layer(x), own[0])
+    for name, stand_in in (("_layer_backward_plan", lambda *a: None), ("takes_linear", lambda *a: False)):
+        with monkeypatch.context() as m:
+            m.setattr(linear, name, stand_in)
+            assert _close(own, _step(layer, x, d))
 
 
 def test_what_is_attached_to_a_map_is_kept():

@@ -19,7 +19,14 @@ CASES = [
     ((60, 47), (13, 9), (1, 1), (2, 3), (True, False), ((16, 8), (4, 16))),
     ((9, 17, 21), (5, 7, 8), (1, 2, 1), (1, 1, 2), (True, False, False), ((2, 8, 8), (4, 4, 4))),
     ((16, 32, 32), (8, 16, 16), (4, 8, 8), (1, 1, 1), (False, False, False), ((2, 8, 8), (1, 8, 8))),  # nearly no masks
+    # the same with queries past the end (without, a launch of head dim 128 takes the kernel of one group)
+    ((16, 32, 30), (8, 16, 16), (4, 8, 8), (1, 1, 1), (False, False, False), ((2, 8, 8), (1, 8, 8))),
 ]
+
+
+def test_cases_that_need_no_mask():
+    # (at head dim 128 these run in one group)
+    assert [i for i, (*problem, tiles) in enumerate(CASES) if _lib.fully_block_sparse(*problem, *tiles)] == [7]
 
 
 @pytest.mark.gpu
