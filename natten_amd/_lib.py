@@ -859,14 +859,22 @@ def fna_backward_fused(
     problem = tuple(tuple(x) for x in (kernel_size, stride, dilation, is_causal))
     layout = tuple(q.shape[1 : 1 + na_dim])
     role = kv_role_q_tile_shape is not None
+    prepared, q_scaled = 0, None
     if out is not None:
+        try:
+            q_scaled = torch.empty_like(q)
+        except torch.OutOfMemoryError:
+            # no room for the scaled queries beside dq: the same gradients with dq as their place, behind a pass of its own
+            delta, lse = backward_prepare(q, out, d_out, lse, scale, dq)
+            prepared = 4
+    if q_scaled is not None:
         # the dq launch comes first and leaves what the dk / dv launch reads: the scaled queries, LSE and delta
         _require_gpu(q, k, v, out, d_out, lse)
         if out.dtype != q.dtype or d_out.dtype != q.dtype or out.shape != q.shape or d_out.shape != q.shape:
             raise ValueError("out and d_out must be of q's shape and dtype.")
         if lse.dtype != torch.float32 or lse.shape != q.shape[:-1]:
             raise ValueError("lse must be float32 of q's shape without the last dimension.")
-        q_scaled, rows = torch.empty_like(q), torch.empty((2, lse.numel()), dtype=torch.float32, device=q.device)
+        rows = torch.empty((2, lse.numel()), dtype=torch.float32, device=q.device)
         arrays = _problem_arrays(layout, *problem, tuple(q_tile_shape), tuple(kv_tile_shape),
                                  *((tuple(kv_role_q_tile_shape), tuple(kv_role_kv_tile_shape)) if role else ()))
         with _on_device(q):
@@ -876,7 +884,8 @@ def fna_backward_fused(
                 DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2], q.shape[-1], *arrays, *(() if role else (None, None)),
                 float(scale), _stream(q)))
         return dq, dk, dv
-    lse, delta = _head_major(lse, delta)
+    if not prepared:
+        lse, delta = _head_major(lse, delta)
     _require_gpu(q, k, v, d_out, lse, delta)
     same = not role or (
         tuple(kv_role_q_tile_shape) == tuple(q_tile_shape) and tuple(kv_role_kv_tile_shape) == tuple(kv_tile_shape))
@@ -890,8 +899,8 @@ def fna_backward_fused(
             rc = L.natten_amd_fna_backward_fused(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(), lse.data_ptr(), delta.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dq.data_ptr(), DTYPE_CODES[q.dtype], na_dim, B, H, k.shape[-2],
-                q.shape[-1], *_problem_arrays(layout, *problem, tuple(qt), tuple(kt)), float(scale), roles + (8 if role else 0),
-                _stream(q),
+                q.shape[-1], *_problem_arrays(layout, *problem, tuple(qt), tuple(kt)), float(scale),
+                roles + prepared + (8 if role else 0), _stream(q),
             )
             _check(rc)
     return dq, dk, dv

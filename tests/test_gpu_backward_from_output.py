@@ -42,6 +42,28 @@ def test_bits_of_the_prepared_launches(layout, heads, heads_kv, k, s, d, c, head
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
 
 
+@pytest.mark.parametrize("layout,heads,heads_kv,k,s,d,c", CASES[1:3])
+def test_without_room_for_the_scaled_queries(layout, heads, heads_kv, k, s, d, c, monkeypatch):
+    gen = torch.Generator().manual_seed(7)
+    q, kk, v, d_out = (torch.randn((2, *layout, h, 64), generator=gen).bfloat16().cuda() for h in (heads, heads_kv, heads_kv, heads))
+    q, kk, v = (t.requires_grad_(True) for t in (q, kk, v))
+    out = getattr(natten_amd, f"na{len(layout)}d")(q, kk, v, k, s, d, c)
+    ref = torch.autograd.grad(out, (q, kk, v), d_out, retain_graph=True)
+    empty_like, of_q = torch.empty_like, []
+
+    def full_memory(t, *args, **kwargs):
+        if t.shape == q.shape:
+            of_q.append(1)
+        if len(of_q) == (2 if heads != heads_kv else 4):  # dq (and dk, dv of q's shape) before it
+            raise torch.OutOfMemoryError("no room")
+        return empty_like(t, *args, **kwargs)
+
+    monkeypatch.setattr(torch, "empty_like", full_memory)
+    got = torch.autograd.grad(out, (q, kk, v), d_out)
+    assert len(of_q) == (2 if heads != heads_kv else 4)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
 def test_refusals():
     L, t = _lib.lib(), torch.zeros((1, 64, 1, 32), dtype=torch.float16, device="cuda")
     f = torch.zeros((1, 64, 1), device="cuda")
