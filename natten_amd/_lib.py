@@ -773,8 +773,9 @@ def linear_backward(d_outs, x: Tensor, weight: Tensor, need_x: bool, need_weight
     n, k = weight.shape
     _require_gpu(x, weight, *d_outs)
     rows, part = x.numel() // k, n // len(d_outs)
-    if any(d.numel() != rows * part for d in d_outs):
-        raise ValueError(f"Gradients of {[tuple(d.shape) for d in d_outs]} do not hold {rows} rows of {part} columns each.")
+    for d in d_outs:
+        if d.numel() != rows * part:
+            raise ValueError(f"Gradients of {[tuple(d.shape) for d in d_outs]} do not hold {rows} rows of {part} columns each.")
     dx = torch.empty_like(x) if need_x else None
     dw = db = workspace = None
     nbytes = 0
@@ -783,10 +784,11 @@ def linear_backward(d_outs, x: Tensor, weight: Tensor, need_x: bool, need_weight
         db = torch.empty((n,), dtype=x.dtype, device=x.device) if need_bias else None
         nbytes = _linear_workspace(rows, n, k, part)
         workspace = torch.empty((nbytes // 4,), dtype=torch.float32, device=x.device)
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
     with _on_device(x):
         _check(lib().natten_amd_linear_backward(
-            *_three(d_outs), x.data_ptr(), weight.data_ptr(), ptr(dx), ptr(dw), ptr(db), ptr(workspace), nbytes,
+            *_three(d_outs), x.data_ptr(), weight.data_ptr(), None if dx is None else dx.data_ptr(),
+            None if dw is None else dw.data_ptr(), None if db is None else db.data_ptr(),
+            None if workspace is None else workspace.data_ptr(), nbytes,
             DTYPE_CODES[x.dtype], rows, n, k, part, _stream(x)))
     return dx, dw if need_weight else None, db
 

@@ -65,8 +65,8 @@ def _fits(module: nn.Module, x: Tensor, parts: int) -> bool:
     if not 0 < x.numel() < 2**31 * 64 or x.numel() // k >= 2**31 - 128 or x.data_ptr() % 16:
         return False
     w, b = module.weight, module.bias
-    return (_plain(w, x.dtype, x.device, 16) and tuple(w.shape) == (n, k)
-            and (b is None or (_plain(b, x.dtype, x.device, 8) and tuple(b.shape) == (n,))))
+    return (_plain(w, x.dtype, x.device, 16) and w.shape == (n, k)
+            and (b is None or (_plain(b, x.dtype, x.device, 8) and b.shape == (n,))))
 
 
 def _aligned(t: Tensor) -> Tensor:
